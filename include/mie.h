@@ -838,6 +838,37 @@ int mie_events_to_frame_bf16(const double* events, int n_events, int kind, int n
                              double start_old, double start_new, double delta_t,
                              int delta, float* sums, void* out, uint8_t* pixmask, void* stream);
 
+/* ---- recorded call sequences ------------------------------------------------
+ * A step of a network is the same sequence of calls every time, with the same
+ * arguments but for the pointers of its inputs.  A host that has noted them once
+ * hands the whole sequence over in one call: no per-call binding, conversion or
+ * check on its side.
+ */
+typedef struct mie_call {
+  int32_t entry;            /* mie_call_index of the entry point */
+  int32_t n_args;           /* its arguments, the stream left out */
+  int32_t n_patches;
+  int32_t reserved;
+  const uint64_t* args;     /* one 8-byte word per argument: pointers and long long as they are, int32 sign-extended,
+                               float as its 32 bits, double as its 64; words and what they point to belong to the
+                               caller and are only read */
+  const int32_t* patches;   /* n_patches pairs (argument, input): that argument is inputs[input] instead of its word */
+} mie_call;
+
+/* Number of the entry point called `name` (MIE_ERR_UNSUPPORTED: none of that name can be part of a sequence). */
+int mie_call_index(const char* name);
+
+/* Argument types of an entry point, one letter each, the stream left out: r pointer that is read, w pointer that is
+ * written, t tile set, i int, l long long, f float, d double; NULL for a number that is none. */
+const char* mie_call_signature(int entry);
+
+/*
+ * The calls in order on `stream`; stops at the first that fails and returns its status.  `inputs`: what the patches
+ * refer to.  The sequence is only read: several threads may run one at the same time on buffers of their own
+ * choosing, as far as its entry points allow that.
+ */
+int mie_run_calls(const mie_call* calls, int n_calls, const uint64_t* inputs, int n_inputs, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

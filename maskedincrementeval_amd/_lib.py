@@ -38,6 +38,7 @@ EXPORTS = (
     "mie_conv_masked_ws", "mie_convgru_gates_incr", "mie_upsample2x_pair_incr", "mie_conv_masked_noalloc",
     "mie_convlstm_gates_refresh", "mie_convgru_gates_refresh", "mie_mul_dense", "mie_tconv2x_masked",
     "mie_tconv2x_refresh", "mie_conv_f32x3_takes", "mie_build_mask_plan", "mie_build_mask_plan_wgs",
+    "mie_call_index", "mie_call_signature", "mie_run_calls",
 )
 PLAN_MAX_STEPS = 40
 
@@ -58,6 +59,14 @@ class MiePlanOp(ctypes.Structure):
         ("h_in", ctypes.c_int32), ("w_in", ctypes.c_int32),
         ("foot", ctypes.c_int32), ("k", ctypes.c_int32), ("stride", ctypes.c_int32), ("pad", ctypes.c_int32),
         ("out", MieTileSet),
+    ]
+
+
+class MieCall(ctypes.Structure):
+    """struct mie_call of include/mie.h: one call of a recorded sequence."""
+    _fields_ = [
+        ("entry", ctypes.c_int32), ("n_args", ctypes.c_int32), ("n_patches", ctypes.c_int32), ("reserved", ctypes.c_int32),
+        ("args", ctypes.c_void_p), ("patches", ctypes.c_void_p),
     ]
 
 
@@ -91,6 +100,12 @@ def _declare(l):
     l.mie_build_mask_plan.argtypes = [ctypes.POINTER(MiePlanOp), ci, vp]
     l.mie_build_mask_plan_wgs.restype = ci
     l.mie_build_mask_plan_wgs.argtypes = [ctypes.POINTER(MiePlanOp), ci, ci, vp]
+    l.mie_call_index.restype = ci
+    l.mie_call_index.argtypes = [ctypes.c_char_p]
+    l.mie_call_signature.restype = ctypes.c_char_p
+    l.mie_call_signature.argtypes = [ci]
+    l.mie_run_calls.restype = ci
+    l.mie_run_calls.argtypes = [ctypes.POINTER(MieCall), ci, ctypes.POINTER(ctypes.c_uint64), ci, vp]
     l.mie_conv_masked.restype = ci
     l.mie_conv_masked.argtypes = [vp, vp, ci, vp, vp, ci, ci, ci, vp, vp, ci, ci, ci, ci, ci, tsp, vp,
                                   vp, vp, ci, cf, ci, ci, vp]

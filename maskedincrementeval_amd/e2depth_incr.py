@@ -17,13 +17,11 @@ are deliberate:
 * `BaseE2VID` (an un-vendored dependency of the reference, :4) is replaced
   by a plain config dict on `E2VIDRecurrentIncr`.
 """
-import contextlib
-
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _lib, ops
+from . import _lib, ops, replay
 from .masked_types import DenseT, Masked, TileMask
 from .mask_incr_functional import IncrementReserve, _unpack
 from .mask_incr_modules import (_IncrBuffers, nnAddIncr, nnBatchNorm2dIncr, nnConvIncr,
@@ -45,7 +43,7 @@ def _same_mask(a, b) -> bool:
     return pa.data_ptr() == pb.data_ptr() and pa.shape == pb.shape and pa.dtype == pb.dtype
 
 
-class ConvLayerIncr(nn.Module):
+class ConvLayerIncr(replay.Watched, nn.Module):
     """conv -> [BN] -> activation (reference :12-51)."""
 
     def __init__(self, in_channels, out_channels, kernel_size, stride=1, padding=0,
@@ -86,7 +84,7 @@ class ConvLayerIncr(nn.Module):
         return out
 
 
-class ConvLSTMIncr(nn.Module, _IncrBuffers):
+class ConvLSTMIncr(replay.Watched, nn.Module, _IncrBuffers):
     """Incremental ConvLSTM cell (reference :54-166).
 
     fused=True keeps three reservoirs -- gate pre-activations (4*hid channels),
@@ -234,7 +232,7 @@ class ConvLSTMIncr(nn.Module, _IncrBuffers):
         ts = self._gates_tile_set("gates" + sfx, x, pix, prev_h_incr, prev_c_incr, pix2)
         dh = self._delta_buf("h" + sfx, (n, hid, h, w), x.device, x.dtype)
         dc = self._delta_buf("c" + sfx, (n, hid, h, w), x.device, x.dtype)
-        self._own_slot(slot, dh, dc, ts)
+        replay.effect(self._own_slot, slot, dh, dc, ts)
         cp = cpm = None
         if prev_c_incr is not None:
             cp, cpm, _ = _unpack(prev_c_incr)
@@ -266,7 +264,7 @@ class ConvLSTMIncr(nn.Module, _IncrBuffers):
         ops.conv_masked(x, pix, x2, pix2, self.Gates.conv2d_weights, k, 1, k // 2, ts, gates, path=self.Gates.path)
         dh = self._delta_buf("h" + sfx, (n, hid, h, w), gates.device, gates.dtype)
         dc = self._delta_buf("c" + sfx, (n, hid, h, w), gates.device, gates.dtype)
-        self._own_slot(slot, dh, dc, ts)
+        replay.effect(self._own_slot, slot, dh, dc, ts)
         cp = cpm = None
         if prev_c_incr is not None:
             cp, cpm, _ = _unpack(prev_c_incr)
@@ -329,7 +327,7 @@ class ConvLSTMIncr(nn.Module, _IncrBuffers):
         self._reset_incr()
         # buffer ownership of the two state sets is told by raw addresses: forget them here, so that an address the
         # allocator has reused since (a shape or device change frees the old buffers) cannot be mistaken for one
-        self.__dict__.pop("_slot_ptrs", None)
+        replay.effect(self.__dict__.pop, "_slot_ptrs", None)
         if self.Gates.use_kf:
             self.Gates.kf.forward_refresh_reservoirs(input_)
         # the concat is never formed: two-pointer conv input, hidden half skipped when it is zero
@@ -337,7 +335,7 @@ class ConvLSTMIncr(nn.Module, _IncrBuffers):
             # the fp32 gate pre-activations go straight into their reservoir; the state is
             # computed from them in fp32 and handed on in the dtype of the input
             one_kernel = self._one_kernel_ok(input_, True)
-            self.__dict__["_gates_interleaved"] = one_kernel
+            replay.effect(self.__dict__.__setitem__, "_gates_interleaved", one_kernel)
             if one_kernel:
                 # reservoir in the gate-interleaved column order of the conv + gate chain kernel
                 filt, bias = self._gates_filter()
@@ -361,7 +359,7 @@ class ConvLSTMIncr(nn.Module, _IncrBuffers):
         return hidden, cell
 
 
-class RecurrentConvLayerIncr(nn.Module):
+class RecurrentConvLayerIncr(replay.Watched, nn.Module):
     """Reference :169-186."""
 
     def __init__(self, in_channels, out_channels, kernel_size=3, stride=1, padding=0,
@@ -386,7 +384,7 @@ class RecurrentConvLayerIncr(nn.Module):
         return x, state
 
 
-class ResidualBlockIncr(nn.Module):
+class ResidualBlockIncr(replay.Watched, nn.Module):
     """conv-relu-conv, + residual, relu (reference :189-240)."""
 
     def __init__(self, in_channels, out_channels, stride=1, downsample=None, norm=None, fuse=True):
@@ -450,7 +448,7 @@ class ResidualBlockIncr(nn.Module):
         return out
 
 
-class TransposedConvLayerIncr(nn.Module):
+class TransposedConvLayerIncr(replay.Watched, nn.Module):
     """Transposed conv (stride 2, output_padding 1) -> activation (reference :243-282)."""
 
     def __init__(self, in_channels, out_channels, kernel_size, stride=1, padding=0,
@@ -495,7 +493,7 @@ class TransposedConvLayerIncr(nn.Module):
         return out
 
 
-class UpsampleConvLayerIncr(nn.Module):
+class UpsampleConvLayerIncr(replay.Watched, nn.Module):
     """bilinear x2 -> conv -> activation (reference :284-322); the skip sum of the
     UNet is taken inside the up-sampling kernel."""
 
@@ -541,7 +539,7 @@ class UpsampleConvLayerIncr(nn.Module):
         return out
 
 
-class BaseUNetIncr(nn.Module):
+class BaseUNetIncr(replay.Watched, nn.Module):
     """Reference :325-377."""
 
     def __init__(self, num_input_channels, num_output_channels=1, skip_type='sum', activation='sigmoid',
@@ -726,7 +724,7 @@ E2DEPTH_DEFAULT_CONFIG = dict(num_bins=5, skip_type='sum', num_encoders=3, base_
                               recurrent_block_type='convlstm')
 
 
-class E2VIDRecurrentIncr(nn.Module, _IncrBuffers):
+class E2VIDRecurrentIncr(replay.Watched, nn.Module, _IncrBuffers):
     """E2Depth-incr / E2VID-incr (reference :471-498).
 
     `config` is a dict (keys of E2DEPTH_DEFAULT_CONFIG; missing keys take the
@@ -777,12 +775,9 @@ class E2VIDRecurrentIncr(nn.Module, _IncrBuffers):
         ops.require_no_lookahead(self)
         delta = ops.as_nhwc(event_tensor[0])
         mask = _mask_of(event_tensor)
-        if not self.async_masks and not self.plan_first:
-            if mask is None and self.derive_input_mask:
-                mask = self.input_mask(delta)
-            return self.unetrecurrent.forward([delta, mask], prev_states)
-        # (plan_first without async_masks: the planning pass runs on the compute stream, ahead of the compute pass)
-        with (ops.mask_planner(delta.device) if self.async_masks else contextlib.nullcontext()):
+        if not self.async_masks:
+            return self._step_planned([delta, mask], prev_states) if self.plan_first else self._step([delta, mask], prev_states)
+        with ops.mask_planner(delta.device):
             if mask is None and self.derive_input_mask:
                 mask = self.input_mask(delta)
             if self.plan_first:
@@ -793,6 +788,29 @@ class E2VIDRecurrentIncr(nn.Module, _IncrBuffers):
             else:
                 img_pred, states = self.unetrecurrent.forward([delta, mask], prev_states)
         return img_pred, states
+
+    # A recorded step builds its tile sets as one plan ahead of the compute calls, where the masks allow it, whatever
+    # plan_first says: the sets are the same, two launches instead of one or two per set.
+    @replay.replayed(record="_step_planned_pass", free_masks=False)
+    def _step(self, x_incr, prev_states):
+        delta, mask = x_incr
+        if mask is None and self.derive_input_mask:
+            mask = self.input_mask(delta)
+        return self.unetrecurrent.forward([delta, mask], prev_states)
+
+    @replay.replayed(free_masks=False)
+    def _step_planned(self, x_incr, prev_states):
+        return self._step_planned_pass(x_incr, prev_states)
+
+    def _step_planned_pass(self, x_incr, prev_states):
+        """The planning pass on the compute stream, ahead of the compute pass."""
+        delta, mask = x_incr
+        if mask is None and self.derive_input_mask:
+            mask = self.input_mask(delta)
+        with ops.network_pass("plan"):
+            self.unetrecurrent.forward([delta, mask], prev_states)
+        with ops.network_pass("compute"):
+            return self.unetrecurrent.forward([delta, mask], prev_states)
 
     def _lookahead_parts(self, delta):
         n, _, h, w = delta.shape
@@ -831,5 +849,9 @@ class E2VIDRecurrentIncr(nn.Module, _IncrBuffers):
 
     def forward_refresh_reservoirs(self, event_tensor: DenseT, prev_states):
         ops.drop_lookahead(self)
+        return self._refresh(event_tensor, prev_states)
+
+    @replay.replayed(dense=1, masked=0)
+    def _refresh(self, event_tensor, prev_states):
         img_pred, states = self.unetrecurrent.forward_refresh_reservoirs(event_tensor, prev_states)
         return img_pred, states

@@ -22,13 +22,11 @@ What differs on purpose:
 * Constructor arguments replace the literals of the reference class
   (`num_bins`, `base_num_channels`, decoder kind), defaults = the reference's.
 """
-import contextlib
-
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _lib, ops
+from . import _lib, ops, replay
 from .masked_types import DenseT, Masked, TileMask
 from .mask_incr_functional import _unpack
 from .mask_incr_modules import (_IncrBuffers, nnAddIncr, nnBatchNorm2dIncr, nnConvIncr,
@@ -49,7 +47,7 @@ def _mask_of(x_incr):
     return x_incr[1] if len(x_incr) > 1 else None
 
 
-class nnCatIncr(nn.Module, _IncrBuffers):
+class nnCatIncr(replay.Watched, nn.Module, _IncrBuffers):
     """Channel concat of deltas with the union of their masks (torch.cat on the clean delta
     buffers; used where a kernel takes one input pointer only)."""
 
@@ -58,6 +56,8 @@ class nnCatIncr(nn.Module, _IncrBuffers):
             # torch.cat / torch.maximum below run on the compute stream and would read pixel masks that the
             # planning stream is still writing
             raise NotImplementedError("nnCatIncr under asynchronous mask planning; use async_masks=False")
+        if ops._phase is not None:      # ... or that the plan of this pass has yet to write
+            raise replay.ValueDependentMask("nnCatIncr reads pixel masks: this network cannot be planned ahead; use plan_first=False")
         deltas = [ops.as_nhwc(p[0]) for p in parts]
         n, _, h, w = deltas[0].shape
         pix = [ops.pixel_mask_of(_mask_of(p), d) for p, d in zip(parts, deltas)]
@@ -72,7 +72,7 @@ class nnCatIncr(nn.Module, _IncrBuffers):
         return [out, ts]
 
 
-class ConvGRUIncr(nn.Module, _IncrBuffers):
+class ConvGRUIncr(replay.Watched, nn.Module, _IncrBuffers):
     """Incremental ConvGRU (reference :18-96)."""
 
     def __init__(self, input_size, hidden_size, kernel_size, activation=None, fuse=True, stacked=True):
@@ -138,7 +138,7 @@ class ConvGRUIncr(nn.Module, _IncrBuffers):
         if (self.fuse and self.stacked and prev_state is None and not self.update_gate.lossy
                 and not self.out_gate.lossy and self.sigmoid1.in_res.reservoir is not None):
             new_state = self._forward_stacked(input_incr)
-            self.__dict__["_mult_stale"] = True       # self.mult's reservoirs have missed this step
+            replay.effect(self.__dict__.__setitem__, "_mult_stale", True)       # self.mult's reservoirs have missed this step
             return new_state, new_state
         if self.__dict__.get("_mult_stale", False):
             raise RuntimeError("ConvGRUIncr: steps since the last refresh ran the one-conv form (no previous "
@@ -155,7 +155,7 @@ class ConvGRUIncr(nn.Module, _IncrBuffers):
 
     def forward_refresh_reservoirs(self, x, prev_state):
         self._reset_incr()
-        self.__dict__["_mult_stale"] = False
+        replay.effect(self.__dict__.__setitem__, "_mult_stale", False)
         zero_state = prev_state is None
         h_in = None if zero_state else ops.as_nhwc(prev_state)
         update = self.update_gate.forward_refresh_fused(x, self.sigmoid1, h_in)
@@ -181,7 +181,7 @@ class ConvGRUIncr(nn.Module, _IncrBuffers):
         return new_state, new_state
 
 
-class ConvLayerIncr(nn.Module):
+class ConvLayerIncr(replay.Watched, nn.Module):
     """conv -> [BN] -> activation (reference :99-156)."""
 
     def __init__(self, in_channels, out_channels, kernel_size, stride=1, activation="relu", norm=None,
@@ -225,7 +225,7 @@ class ConvLayerIncr(nn.Module):
         return out
 
 
-class RecurrentConvLayerIncr(nn.Module):
+class RecurrentConvLayerIncr(replay.Watched, nn.Module):
     """Reference :160-195."""
 
     def __init__(self, in_channels, out_channels, kernel_size=3, stride=1, activation_ff="relu",
@@ -247,7 +247,7 @@ class RecurrentConvLayerIncr(nn.Module):
         return x, state
 
 
-class ResidualBlockIncr(nn.Module):
+class ResidualBlockIncr(replay.Watched, nn.Module):
     """conv - act - conv, + residual, act; returns (out2, out1) (reference :198-289)."""
 
     def __init__(self, in_channels, out_channels, stride=1, activation="relu", downsample=None,
@@ -314,7 +314,7 @@ class ResidualBlockIncr(nn.Module):
         return out2, out1
 
 
-class UpsampleConvLayerIncr(nn.Module):
+class UpsampleConvLayerIncr(replay.Watched, nn.Module):
     """bilinear x2 -> conv -> activation over the parts of a concat (reference :294-343).
 
     forward / forward_refresh_reservoirs take the list of parts in concat order
@@ -444,7 +444,7 @@ class UpsampleConvLayerIncr(nn.Module):
         return out
 
 
-class TransposedConvLayerIncr(nn.Module):
+class TransposedConvLayerIncr(replay.Watched, nn.Module):
     """Transposed conv (stride 2, output_padding 1) -> activation over the concat of the parts:
     the decoder kind the benchmark configuration of this network names.  As in the up-sampling
     decoder the concat [previous flow (2 ch, optional), x, skip] is never formed: the two wide parts
@@ -525,7 +525,7 @@ class TransposedConvLayerIncr(nn.Module):
         return out
 
 
-class MultiResUNetRecurrentIncr(nn.Module, _IncrBuffers):
+class MultiResUNetRecurrentIncr(replay.Watched, nn.Module, _IncrBuffers):
     """EVFlowNet-incr (reference :346-495).  Defaults are the reference's literals
     (2 input bins, base 32, 4 encoders 64/128/256/512, 2 residual blocks, up-sampling
     decoders, tanh flow heads); `decoder="transposed"` swaps in transposed-conv decoders."""
@@ -607,13 +607,10 @@ class MultiResUNetRecurrentIncr(nn.Module, _IncrBuffers):
         ops.require_no_lookahead(self)
         delta = ops.as_nhwc(x_incr[0])
         mask = _mask_of(x_incr)
-        if not self.async_masks and not self.plan_first:
-            return self._forward(delta, mask)
-        # (plan_first without async_masks: the planning pass runs on the compute stream, ahead of the compute pass)
-        with (ops.mask_planner(delta.device) if self.async_masks else contextlib.nullcontext()):
-            if mask is None and self.derive_input_mask:
-                n, _, h, w = delta.shape
-                mask = ops.mask_from_delta(delta, self.mask_threshold, self._pix_buf("input", n, h, w, delta.device))
+        if not self.async_masks:
+            return self._step_planned([delta, mask]) if self.plan_first else self._step([delta, mask])
+        with ops.mask_planner(delta.device):
+            mask = self._input_mask(delta, mask)
             if self.plan_first:
                 with ops.network_pass("plan"):
                     self._forward(delta, mask)
@@ -621,10 +618,33 @@ class MultiResUNetRecurrentIncr(nn.Module, _IncrBuffers):
                     return self._forward(delta, mask)
             return self._forward(delta, mask)
 
+    # A recorded step builds its tile sets as one plan ahead of the compute calls, where the masks allow it, whatever
+    # plan_first says: the sets are the same, two launches instead of one or two per set.
+    @replay.replayed(record="_step_planned_pass", free_masks=False)
+    def _step(self, x_incr):
+        return self._forward(*x_incr)
+
+    @replay.replayed(free_masks=False)
+    def _step_planned(self, x_incr):
+        return self._step_planned_pass(x_incr)
+
+    def _step_planned_pass(self, x_incr):
+        """The planning pass on the compute stream, ahead of the compute pass."""
+        delta, mask = x_incr
+        mask = self._input_mask(delta, mask)
+        with ops.network_pass("plan"):
+            self._forward(delta, mask)
+        with ops.network_pass("compute"):
+            return self._forward(delta, mask)
+
+    def _input_mask(self, delta, mask):
+        if mask is not None or not self.derive_input_mask:
+            return mask
+        n, _, h, w = delta.shape
+        return ops.mask_from_delta(delta, self.mask_threshold, self._pix_buf("input", n, h, w, delta.device))
+
     def _forward(self, delta, mask):
-        if mask is None and self.derive_input_mask:
-            n, _, h, w = delta.shape
-            mask = ops.mask_from_delta(delta, self.mask_threshold, self._pix_buf("input", n, h, w, delta.device))
+        mask = self._input_mask(delta, mask)
         x_incr = [delta, mask]
         states_incr = [None] * self.num_states
         blocks = []
@@ -679,12 +699,19 @@ class MultiResUNetRecurrentIncr(nn.Module, _IncrBuffers):
 
     def forward_refresh_reservoirs(self, x):
         ops.drop_lookahead(self)
+        return self._refresh(x, list(self.states))
+
+    def _set_state(self, i, state):
+        self.states[i] = state
+
+    @replay.replayed(dense=1, masked=0)
+    def _refresh(self, x, prev_states):
         self._reset_incr()
         blocks = []
         for i, encoder in enumerate(self.encoders):
-            x, state = encoder.forward_refresh_reservoirs(x, self.states[i])
+            x, state = encoder.forward_refresh_reservoirs(x, prev_states[i])
             blocks.append(x)
-            self.states[i] = state
+            replay.effect(self._set_state, i, state)
         for resblock in self.resblocks:
             x, _ = resblock.forward_refresh_reservoirs(x)
         predictions = []

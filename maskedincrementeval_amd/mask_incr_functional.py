@@ -12,7 +12,7 @@ persistent buffers and are the ones to use in a loop).
 import torch
 import torch.nn as nn
 
-from . import _lib, ops
+from . import _lib, ops, replay
 from .masked_types import DenseT, Masked, TileMask
 
 
@@ -36,7 +36,7 @@ class AccumStreamManager:
         return torch.cuda.current_stream()
 
 
-class IncrementReserve:
+class IncrementReserve(replay.Watched):
     """Dense cached activation ("reservoir"), channels_last for 4-D tensors.
 
     Reference: mask_incr_functional.py:26-48.  `update_reservoir` copies into

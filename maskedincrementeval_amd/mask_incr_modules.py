@@ -19,7 +19,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _lib, ops
+from . import _lib, ops, replay
 from .masked_types import DenseT, Masked, TileMask
 from .mask_incr_functional import (IncrPointwiseMultiply, IncrementReserve, _square, _unpack,
                                    bn2d_from_module, bn_scale, conv2d_from_module)
@@ -112,7 +112,7 @@ class _IncrBuffers:
 
 
 # input output increments: interface for incremental modules
-class IncrementMaskModule(nn.Module, _IncrBuffers):
+class IncrementMaskModule(replay.Watched, nn.Module, _IncrBuffers):
 
     def forward_refresh_reservoirs(self, x: DenseT) -> DenseT:
         return x
@@ -276,11 +276,12 @@ class NonlinearPointOpIncr(IncrementMaskModule):
         self.refine_mask = refine_mask
 
     def forward(self, x_incr: Masked) -> Masked:
-        return self._nonlin(x_incr, keep_reservoir=True)
+        return self._nonlin(x_incr, True)
 
     def forward_refresh_reservoirs(self, x: DenseT):
         return self.op(x)
 
+    @replay.replayed()
     def _nonlin(self, x_incr: Masked, keep_reservoir: bool):
         kind, slope = activation_kind(self.op)
         d, _, _ = _unpack(x_incr)
@@ -303,7 +304,7 @@ class NonlinearPointOpIncr(IncrementMaskModule):
         return [out, ts]
 
 
-class nnLinearIncr(nn.Linear):
+class nnLinearIncr(replay.Watched, nn.Linear):
     """Fully connected layer on a delta: bias dropped (reference :106-116).  One kernel that reads only
     the weight rows of the features whose delta is non-zero; the transposed weight copy it walks is
     rebuilt when the weight changes."""
@@ -446,7 +447,7 @@ class _ConvIncrMixin(_IncrBuffers):
         return out
 
 
-class nnConvIncrBase(nn.Conv2d, _ConvIncrMixin):
+class nnConvIncrBase(replay.Watched, nn.Conv2d, _ConvIncrMixin):
     """Reference :122-142."""
 
     def forward(self, x_incr):
@@ -456,7 +457,7 @@ class nnConvIncrBase(nn.Conv2d, _ConvIncrMixin):
         return self._refresh_forward(x)
 
 
-class nnConvIncr(nn.Conv2d, _ConvIncrMixin):
+class nnConvIncr(replay.Watched, nn.Conv2d, _ConvIncrMixin):
     """Incremental conv: forward([d, m]) = [conv2d(d, W, bias=None), tile mask].
 
     Reference :146-196, where forward always falls back to a dense F.conv2d on
@@ -495,12 +496,17 @@ class nnConvIncr(nn.Conv2d, _ConvIncrMixin):
             x_incr = [x, pix]
         return x_incr
 
+    @replay.replayed(masked=2)
     def forward(self, x_incr, x2_incr=None):
         return self._incr_forward(self.lossy_input(x_incr), x2_incr, path=self.path)
 
     def forward_fused(self, x_incr, activation: "nnReservedActivation", x2_incr=None,
                       addend_incr=None, filt=None):
         """conv (+ addend) + activation increment in one kernel; updates activation.in_res in place."""
+        return self._forward_fused(x_incr, x2_incr, activation, addend_incr, filt)
+
+    @replay.replayed(masked=2, trees=(2,))
+    def _forward_fused(self, x_incr, x2_incr, activation, addend_incr, filt):
         x_incr = self.lossy_input(x_incr)
         kind, slope = activation_kind(activation.op)
         res = activation.in_res.reservoir
@@ -575,7 +581,7 @@ def set_input_threshold(net: nn.Module, thr: Optional[float]) -> int:
     return count
 
 
-class nnConvTranspose2dIncr(nn.ConvTranspose2d, _IncrBuffers):
+class nnConvTranspose2dIncr(replay.Watched, nn.ConvTranspose2d, _IncrBuffers):
     """Incremental transposed conv (named but not defined by the reference,
     incr_modules/e2depth_incr.py:248; semantics of transposed_conv2d_from_module,
     mask_incr_functional.py:64-66).  The decoder case -- stride 2, kernel 3 or 5, padding k // 2,
@@ -659,7 +665,7 @@ class nnConvTranspose2dIncr(nn.ConvTranspose2d, _IncrBuffers):
         return ops.tconv_refresh(x, filt, bias, k, s, p, ts, out, reservoir, act, slope)
 
 
-class nnBatchNorm2dIncr(nn.BatchNorm2d, _IncrBuffers):
+class nnBatchNorm2dIncr(replay.Watched, nn.BatchNorm2d, _IncrBuffers):
     """Reference :200-207: the linear part of the eval-mode batch norm on a delta, one masked kernel into a
     buffer the module keeps."""
 
@@ -677,7 +683,7 @@ class nnBatchNorm2dIncr(nn.BatchNorm2d, _IncrBuffers):
         return super().forward(x)
 
 
-class nnMaxPool2dIncr(nn.MaxPool2d, _IncrBuffers):
+class nnMaxPool2dIncr(replay.Watched, nn.MaxPool2d, _IncrBuffers):
     """pool(R + d) - pool(R), then R += d (reference :210-224): one kernel over the active output
     tiles and a masked accumulate of the reservoir (square windows, no dilation, floor mode)."""
 
@@ -714,7 +720,7 @@ class nnMaxPool2dIncr(nn.MaxPool2d, _IncrBuffers):
         return super().forward(x)
 
 
-class nnAdaptiveAvgPool2dIncr(nn.AdaptiveAvgPool2d):
+class nnAdaptiveAvgPool2dIncr(replay.Watched, nn.AdaptiveAvgPool2d):
     """Reference :228-233: adaptive average pooling of a delta; inactive pixels are not read.  The pooled
     delta is small and dense, so it carries no mask."""
 
@@ -750,7 +756,7 @@ class nnReservedActivation(NonlinearPointOpIncr):
         NonlinearPointOpIncr.__init__(self, self.in_res, op, refine_mask)
 
     def forward(self, x_incr: Masked):
-        return self._nonlin(x_incr, keep_reservoir=False)
+        return self._nonlin(x_incr, False)
 
     def forward_refresh_reservoirs(self, x: DenseT):
         out = NonlinearPointOpIncr.forward_refresh_reservoirs(self, x)

@@ -9,7 +9,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from . import _lib
+from . import _lib, replay
 from ._lib import check
 from .masked_types import TileMask
 
@@ -37,7 +37,7 @@ class _PhaseLib:
 
 
 def lib():
-    real = _lib.lib()
+    real = replay.lib()
     return real if _phase is None else _PhaseLib(real)
 
 
@@ -89,7 +89,7 @@ def _plan_ops(batch):
 def _launch_plan(batch):
     """Enqueue the collected builds: on the planning stream when one is active (with the waits and events a
     single build would get), else on the current stream."""
-    real = _lib.lib()
+    real = replay.lib()
     dev = batch[0][-1].device
     side = _planner[0] if (_planner is not None and _planner[1] == dev) else None
     if side is not None:
@@ -387,6 +387,7 @@ class mask_planner:
 
 def _ready(ts: TileMask):
     """Make the compute stream wait for the build of `ts` (once)."""
+    replay.keep(ts)
     if _phase == "plan":
         return
     root = ts.parent if ts.parent is not None else ts
@@ -399,7 +400,7 @@ def _ready(ts: TileMask):
 def _mark_pix(t: Optional[torch.Tensor], from_values: bool = False):
     """A pixel mask was written on the compute stream: builds that read it must wait."""
     if t is not None and from_values and _phase is not None:
-        raise RuntimeError("a mask that depends on values (a delta, refined or quantised deltas) cannot be "
+        raise replay.ValueDependentMask("a mask that depends on values (a delta, refined or quantised deltas) cannot be "
                            "planned ahead: run this network without the planning pass")
     if _phase == "compute":
         return
@@ -438,10 +439,11 @@ def nhwc_ptr(t: Optional[torch.Tensor], name: str, c: Optional[int] = None, dtyp
     _require_gpu(t, name)
     if t.dim() != 4 or t.dtype != dtype:
         raise ValueError("%s must be a 4-D %s tensor, got %s %s" % (name, dtype, tuple(t.shape), t.dtype))
-    if not t.permute(0, 2, 3, 1).is_contiguous():
+    if not t.is_contiguous(memory_format=torch.channels_last):
         raise ValueError("%s must be channels_last (NHWC in memory); strides %s" % (name, t.stride()))
     if c is not None and t.shape[1] != c:
         raise ValueError("%s has %d channels, expected %d" % (name, t.shape[1], c))
+    replay.keep(t)
     return t.data_ptr()
 
 
@@ -449,7 +451,7 @@ def as_nhwc(t: torch.Tensor) -> torch.Tensor:
     """Return t as channels_last fp32 (bf16 stays bf16); copies only if the layout / dtype differs."""
     if t.dtype not in _DTYPES:
         t = t.float()
-    if not t.permute(0, 2, 3, 1).is_contiguous():
+    if not t.is_contiguous(memory_format=torch.channels_last):
         t = t.contiguous(memory_format=torch.channels_last)
         if not t.permute(0, 2, 3, 1).is_contiguous():   # C == 1 corner: force the strides
             t = t.permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2)
@@ -472,6 +474,7 @@ def pix_ptr(m, n, h, w, name):
     _require_gpu(t, name)
     if _pending_thr:
         _force_threshold_mask(t)
+    replay.keep(t)
     return t.data_ptr()
 
 
@@ -553,6 +556,7 @@ def _thresholded_build(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, o
 
 def build_mask_tiles(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, out: TileMask):
     """in_mask / in_mask2: None | TileMask | uint8 (N,1,H,W)."""
+    replay.keep(out)
     if _pending_thr and _thresholded_build(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, out):
         return out
     p1 = pix_ptr(in_mask, n, h_in, w_in, "in_mask")
@@ -688,6 +692,7 @@ def _filter_args(filt, k, dtype=torch.float32, x3_shape=None, with_code=False):
             or filt.dtype != torch.float32:
         raise ValueError("filter must be contiguous fp32 [Cin,%d,%d,Cout], got %s" % (k, k, tuple(filt.shape)))
     _require_gpu(filt, "filter")
+    replay.keep((filt, mc))
     ptr = None if mc is None else mc.data_ptr()
     return (filt, ptr, code) if with_code else (filt, ptr)
 
@@ -719,6 +724,7 @@ def _workspace_args(workspace, small: bool, device):
         return None, 0
     if workspace.dtype != torch.float32 or not workspace.is_contiguous() or workspace.device != device:
         raise ValueError("workspace must be a contiguous fp32 tensor on the device of the operands")
+    replay.keep(workspace)
     return workspace.data_ptr(), workspace.numel() * 4
 
 
@@ -831,6 +837,7 @@ def upconv_pred_masked(a, amask, b, bmask, filt, out_ts: TileMask, reservoir, ac
     if pred_w.dtype != torch.float32 or tuple(pred_w.shape) != (2, cout) or not pred_w.is_contiguous():
         raise ValueError("pred_w must be contiguous fp32 (2, %d)" % cout)
     _require_gpu(pred_w, "pred_w")
+    replay.keep(pred_w)
     _ready(out_ts)
     check(lib().mie_upconv_pred_masked(
         nhwc_ptr(a, "a", dtype=dt), pix_ptr(amask, n, h, w, "amask"), nhwc_ptr(b, "b", dtype=dt),
@@ -854,6 +861,7 @@ def conv_refresh(x, x2, filt, bias, k, stride, pad, out_ts: TileMask, out_dense,
         raise ValueError("out_dense shape %s, expected %s" % (tuple(out_dense.shape), (n, cout, out_ts.h, out_ts.w)))
     if bias is not None and (bias.numel() != cout or bias.dtype != torch.float32 or not bias.is_contiguous()):
         raise ValueError("bias must be contiguous fp32 of %d elements" % cout)
+    replay.keep(bias)
     _ready(out_ts)
     check(lib().mie_conv_refresh(
         nhwc_ptr(x, "x", dtype=dt), c1, nhwc_ptr(x2, "x2", dtype=dt), c2, h, w, filt.data_ptr(), mc_ptr,
@@ -869,6 +877,7 @@ def tconv_masked(x, xmask, filt, k, stride, pad, out_ts: TileMask, out_delta, re
     n, cin, h, w = x.shape
     if isinstance(filt, ConvFilter):
         filt = filt.for_dtype(x.dtype)[0]
+    replay.keep(filt)
     if filt.dim() != 4 or filt.shape[0] != cin or filt.shape[1] != k or not filt.is_contiguous():
         raise ValueError("filter must be contiguous [Cin,%d,%d,Cout], got %s" % (k, k, tuple(filt.shape)))
     _require_gpu(filt, "filter")
@@ -889,6 +898,7 @@ def tconv_refresh(x, filt, bias, k, stride, pad, out_ts: TileMask, out_dense, re
     n, cin, h, w = x.shape
     if isinstance(filt, ConvFilter):
         filt = filt.for_dtype(x.dtype)[0]
+    replay.keep(filt)
     if filt.dim() != 4 or filt.shape[0] != cin or filt.shape[1] != k or not filt.is_contiguous():
         raise ValueError("filter must be contiguous [Cin,%d,%d,Cout], got %s" % (k, k, tuple(filt.shape)))
     _require_gpu(filt, "filter")
@@ -897,6 +907,7 @@ def tconv_refresh(x, filt, bias, k, stride, pad, out_ts: TileMask, out_dense, re
         raise ValueError("out_dense shape %s" % (tuple(out_dense.shape),))
     if bias is not None and (bias.numel() != cout or bias.dtype != torch.float32 or not bias.is_contiguous()):
         raise ValueError("bias must be contiguous fp32 of %d elements" % cout)
+    replay.keep(bias)
     _ready(out_ts)
     check(lib().mie_tconv_refresh(
         nhwc_ptr(x, "x", dtype=x.dtype), cin, h, w, filt.data_ptr(), k, stride, pad, cout,
@@ -924,7 +935,7 @@ def _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out, addend, reservoir):
           and c1 % 64 == 0 and c2 % 64 == 0 and filt.shape[3] % 32 == 0
           and filt.plain.is_cuda and filt.plain.shape[0] % 16 == 0)
     if x3:
-        plain, mc = filt.for_dtype(torch.float32, x3=True)
+        plain, mc = replay.keep(filt.for_dtype(torch.float32, x3=True))
         mc_ptr, code = mc.data_ptr(), _lib.DTYPE_F32_BF16X3
     else:
         plain, mc_ptr = _filter_args(filt, k, x.dtype)
@@ -954,6 +965,7 @@ def tconv2x_masked(x, xmask, x2, x2mask, filt, k, out_ts: TileMask, block_ts: Ti
     _ready(block_ts)
     if workspace is None:
         workspace = split_workspace(x.device) if (split_enabled and block_ts.capacity * (cout // 32) <= 128) else False
+    replay.keep(workspace)
     ws_ptr, ws_bytes = (None, 0) if workspace is False else (workspace.data_ptr(), workspace.numel() * 4)
     check(lib().mie_tconv2x_masked(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1, nhwc_ptr(x2, "x2", dtype=dt),
@@ -971,6 +983,7 @@ def tconv2x_refresh(x, x2, filt, bias, k, out_ts: TileMask, block_ts: TileMask, 
     dt = x.dtype
     if bias is not None and (bias.numel() != cout or bias.dtype != torch.float32 or not bias.is_contiguous()):
         raise ValueError("bias must be contiguous fp32 of %d elements" % cout)
+    replay.keep(bias)
     _ready(out_ts)
     _ready(block_ts)
     check(lib().mie_tconv2x_refresh(
@@ -1015,6 +1028,7 @@ def kfence_incr(in_delta, carry, k, out_delta, ts: TileMask, out_pixmask=None):
         if k.numel() != 1 or k.dtype != torch.float32:
             raise ValueError("k must be a float or a 1-element fp32 tensor")
         _require_gpu(k, "k")
+        replay.keep(k)
         k_dev, k_host = k.data_ptr(), 0.0
     else:
         k_dev, k_host = None, float(k)
@@ -1082,6 +1096,7 @@ def scale_incr(in_delta, scale, out_delta, ts: TileMask):
     _same_shape("out_delta", out_delta, in_delta)
     if scale.dtype != torch.float32 or scale.numel() != c or not scale.is_contiguous():
         raise ValueError("scale must be contiguous fp32 [%d]" % c)
+    replay.keep(scale)
     _require_gpu(scale, "scale")
     _ready(ts)
     dt = in_delta.dtype
@@ -1273,3 +1288,15 @@ def mfma_chunk(dtype) -> int:
 def conv_out_size(h, w, k, stride, pad) -> Tuple[int, int]:
     """Output size formula of the reference wrapper (ext/pointops/pointops_functional.py:25-26)."""
     return (h + 2 * pad - k) // stride + 1, (w + 2 * pad - k) // stride + 1
+
+
+# what a recorded pass (replay.py) depends on: it is not used while one of these functions is replaced, nor once one of
+# these settings has another value
+replay.bind_ops(globals(), (
+    "lib", "check", "mask_from_delta", "threshold_mask_lazy", "build_mask_tiles", "conv_masked", "upconv_masked",
+    "upconv_pred_masked", "conv_refresh", "tconv_masked", "tconv_refresh", "tconv2x_masked", "tconv2x_refresh", "act_incr",
+    "kfence_incr", "mul_incr", "add_incr", "maxpool_incr", "accumulate", "scale_incr", "avgpool_incr", "upsample2x_incr",
+    "upsample2x_pair_incr", "convlstm_gates_incr", "convgru_gates_incr", "convlstm_gates_refresh",
+    "convgru_gates_refresh", "mul_dense", "conv_gates_incr", "nhwc_ptr", "pix_ptr", "as_nhwc", "pixel_mask_of"), (
+    "f32_matmul", "split_enabled", "fused_plan", "fused_threshold_build", "upconv_max_tiles", "upconv_max_chunks",
+    "upconv_pred_enabled", "UPCONV_PRED_MIN_TILES", "UPCONV_PRED_MAX_TILES", "SPLIT_WORKSPACE_BYTES"))

@@ -1,0 +1,385 @@
+"""Recorded steps: the library calls of a module or a whole network, noted once and handed over as one sequence.
+
+A step makes the same calls every time: buffers, tile sets, filters and reservoirs stay where they are, only the input
+tensors move.  Walking the modules costs the host 15-25 us per call (shape checks, pointers, buffer look-ups, argument
+conversion) where the kernels behind it take 5-20 us, so the plain calls of small and medium frames were bound by Python:
+an E2Depth-incr step at 64x96 took 596 us for 230 us of kernels.  The third pass over an input of one shape is
+therefore recorded (`Recording`: every call of the library with its arguments), and later passes hand the sequence
+to mie_run_calls with the pointers of their inputs filled in -- about 3 us a call, the launch itself.
+
+A recording stands for the Python pass as long as everything that pass read is what it was:
+  * attributes of the package's modules and which reservoir tensor an IncrementReserve holds: any assignment bumps
+    `_epoch` (`Watched`);
+  * weights: the parameter objects, their addresses and version counters;
+  * the settings and functions of `ops` (a program or a test that replaces one gets its calls);
+  * forward hooks, and the members of module containers.
+Otherwise the pass runs in Python again and is recorded anew.  A pass that runs any torch operation of its own
+(a conversion, a concat, the allocation of a buffer) is never recorded, nor one on a planning stream or inside a
+planning pass.  Recordings hold references to every tensor whose address they use.
+"""
+import collections
+import ctypes
+import functools
+import operator
+import os
+import struct
+import threading
+
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from . import _lib
+from ._lib import check
+
+enabled = os.environ.get("MIE_REPLAY", "1") != "0"      # read once
+MAX_RECORDINGS = 8          # per module and method, least recently used first out
+_epoch = [0]
+_active = None              # the Recording being made, by the thread that makes it
+_SILENT = frozenset(("training", "states"))     # assignments no incremental pass depends on
+
+
+class Watched:
+    """First base of the package's modules and reservoirs: assignments to attributes outdate the recordings."""
+
+    def __setattr__(self, name, value):
+        if name not in _SILENT:
+            _epoch[0] += 1
+        super().__setattr__(name, value)
+
+    def __delattr__(self, name):
+        _epoch[0] += 1
+        super().__delattr__(name)
+
+
+class ValueDependentMask(RuntimeError):
+    """A mask that depends on values met inside a planning pass."""
+
+
+# ---- what the pass reads outside the modules -----------------------------------------------------------------
+_ops_globals = None
+_get_functions = _get_settings = None
+_functions = ()
+
+
+def bind_ops(namespace, functions, settings):
+    """Called once by ops: its namespace, and the names a pass goes through / depends on."""
+    global _ops_globals, _get_functions, _get_settings, _functions
+    _ops_globals = namespace
+    _get_functions, _get_settings = operator.itemgetter(*functions), operator.itemgetter(*settings)
+    _functions = _get_functions(namespace)
+
+
+def _idle() -> bool:
+    """Whether ops is in its ordinary state: no planning pass, no planning stream, no pending threshold mask."""
+    g = _ops_globals
+    return (g["_phase"] is None and g["_planner"] is None and not g["_pending_thr"] and g["buffer_parity"] == 0
+            and _get_functions(g) == _functions)
+
+
+# ---- recording ------------------------------------------------------------------------------------------------
+_PASS_THROUGH = frozenset(("mie_last_error_string", "mie_tile_capacity", "mie_version", "mie_conv_f32x3_takes"))
+_VIEWS = frozenset(("aten::permute", "aten::detach", "aten::view", "aten::slice", "aten::select", "aten::alias",
+                    "aten::as_strided", "aten::t", "aten::transpose", "aten::unsqueeze", "aten::squeeze",
+                    "aten::expand", "aten::_reshape_alias", "aten::_unsafe_view", "aten::split", "aten::unbind"))
+
+
+class _TorchWatch(TorchDispatchMode):
+    """Notes torch operations other than views."""
+
+    def __init__(self):
+        super().__init__()
+        self.seen = None
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if func._schema.name not in _VIEWS:
+            self.seen = func
+        return func(*args, **(kwargs or {}))
+
+
+class Recording:
+    """The library as a pass sees it while it is recorded: makes every call and notes the ones that succeed."""
+
+    def __init__(self, real):
+        self._real = real
+        self.thread = threading.get_ident()
+        self.calls, self.keep, self.effects = [], [], []
+
+    def __getattr__(self, name):
+        fn = getattr(self._real, name)
+        if name in _PASS_THROUGH or not name.startswith("mie_"):
+            return fn
+
+        def noted(*args):
+            rc = fn(*args)
+            if rc == 0:
+                self.calls.append((name, args))
+            return rc
+        return noted
+
+
+def lib():
+    """The library, or the recording of it this thread is making."""
+    r = _active
+    return r if r is not None and r.thread == threading.get_ident() else _lib.lib()
+
+
+def keep(obj):
+    """While a pass is recorded: its recording holds on to `obj`, whose address it uses."""
+    r = _active
+    if r is not None:
+        r.keep.append(obj)
+    return obj
+
+
+def effect(fn, *args):
+    """fn(*args), now and on every replay of the pass: for changes of host state the pass makes."""
+    r = _active
+    if r is not None and r.thread == threading.get_ident():
+        r.effects.append((fn, args))
+    return fn(*args)
+
+
+def _word(kind, value, held):
+    if kind in "rwt":
+        if value is None:
+            return 0
+        if isinstance(value, int):
+            return value
+        held.append(value)
+        return ctypes.addressof(getattr(value, "_obj", value))
+    if kind == "f":
+        return struct.unpack("<I", struct.pack("<f", value))[0]
+    if kind == "d":
+        return struct.unpack("<Q", struct.pack("<d", value))[0]
+    return int(value) & 0xFFFFFFFFFFFFFFFF
+
+
+_signatures = {}
+
+
+def _signature(name):
+    s = _signatures.get(name)
+    if s is None:
+        real = _lib.lib()
+        idx = real.mie_call_index(name.encode())
+        s = _signatures[name] = (idx, real.mie_call_signature(idx).decode()) if idx >= 0 else None
+    return s
+
+
+def _copy(v):
+    """A fresh list / tuple / dict structure around the same tensors and tile sets."""
+    t = type(v)
+    if t is list:
+        return [_copy(x) for x in v]
+    if t is tuple:
+        return tuple([_copy(x) for x in v])
+    if t is dict:
+        return {k: _copy(x) for k, x in v.items()}
+    return v
+
+
+class Program:
+    """A recorded pass that can be run again."""
+
+    def __init__(self, rec, pointers, result, tree, static):
+        self.effects, self.result = rec.effects, result
+        self.runs = 0
+        self.held = [rec.keep, static]
+        calls = (_lib.MieCall * len(rec.calls))()
+        for call, (name, args) in zip(calls, rec.calls):
+            idx, sig = _signature(name)
+            words = (ctypes.c_uint64 * max(1, len(sig)))()
+            patches = []
+            for i, kind in enumerate(sig):
+                words[i] = _word(kind, args[i], self.held)
+                if kind == "r" and words[i] and words[i] in pointers:
+                    patches += [i, pointers.index(words[i])]
+                elif kind == "w" and words[i] in pointers:
+                    raise _NotRecordable("an input is written")
+            pa = (ctypes.c_int32 * max(1, len(patches)))(*patches)
+            call.entry, call.n_args, call.n_patches = idx, len(sig), len(patches) // 2
+            call.args, call.patches = ctypes.addressof(words), ctypes.addressof(pa)
+            self.held += [words, pa]
+        self.calls, self.n = calls, len(rec.calls)
+        self.words_type = ctypes.c_uint64 * max(1, len(pointers))
+        self.n_inputs = len(pointers)
+        self.fn = _lib.lib().mie_run_calls
+        self._guards(tree)
+
+    # what the pass depended on
+    def _guards(self, tree):
+        mods = []
+        for m in tree:
+            mods.extend(m.modules())
+        mods = list({id(m): m for m in mods}.values())
+        self.epoch = _epoch[0]
+        self.settings = _get_settings(_ops_globals)
+        self.hooks = [d for m in mods for d in (m._forward_hooks, m._forward_pre_hooks)]
+        self.hooks += [torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks]
+        if any(self.hooks) or any("forward" in m.__dict__ for m in mods):
+            raise _NotRecordable("hooked")
+        self.classes = sorted({type(m) for m in mods}, key=lambda c: c.__qualname__)
+        for c in self.classes:
+            if c.__module__.split(".")[0] not in (__package__, "torch"):
+                raise _NotRecordable("a class of the caller's")
+        self.forwards = [c.forward for c in self.classes]
+        self.containers = [m._modules for m in mods if m._modules]
+        self.members = [list(d.values()) for d in self.containers]
+        self.param_dicts = [m._parameters for m in mods if m._parameters]
+        self.params = [p for d in self.param_dicts for p in d.values()]
+        self.tensors = [p for p in self.params if p is not None]
+        self.addresses = [p.data_ptr() for p in self.tensors]
+        self.versions = [p._version for p in self.tensors]
+
+    def valid(self) -> bool:
+        return (self.epoch == _epoch[0] and _get_settings(_ops_globals) == self.settings and not any(self.hooks)
+                and [p.data_ptr() for p in self.tensors] == self.addresses
+                and [p._version for p in self.tensors] == self.versions
+                and all(map(operator.is_, [p for d in self.param_dicts for p in d.values()], self.params))
+                and [list(d.values()) for d in self.containers] == self.members
+                and [c.forward for c in self.classes] == self.forwards)
+
+    def run(self, pointers, device):
+        self.runs += 1
+        check(self.fn(self.calls, self.n, self.words_type(*pointers), self.n_inputs,
+                      torch._C._cuda_getCurrentRawStream(device)))
+        for fn, args in self.effects:
+            fn(*args)
+        return _copy(self.result)
+
+
+class _NotRecordable(Exception):
+    pass
+
+
+class _Cache(collections.OrderedDict):
+    """Recordings of one module, by method and input.  Copies and pickles of a module start without any."""
+
+    def __deepcopy__(self, memo):
+        return _Cache()
+
+    def __reduce__(self):
+        return _Cache, ()
+
+
+class _Waiting:
+    """A pass that is not recorded (yet): how often it was seen, and when it is tried next."""
+    __slots__ = ("seen", "next", "step")
+
+    def __init__(self):
+        self.seen, self.next, self.step = 0, 3, 2
+
+
+def _record(owner, fns, pointers, tree, static):
+    """One pass, recorded if it can be: (result, Program or None)."""
+    global _active
+    for k, fn in enumerate(fns):
+        rec, watch = Recording(_lib.lib()), _TorchWatch()
+        _active = rec
+        try:
+            with watch:
+                result = fn()
+        except ValueDependentMask:
+            if k + 1 == len(fns):
+                raise
+            continue
+        finally:
+            _active = None
+        if watch.seen is not None or any(_signature(name) is None for name, _ in rec.calls):
+            return result, None
+        for name, args in rec.calls:        # a plan holds its input masks inside its own array
+            if name.startswith("mie_build_mask_plan") and any(
+                    op.in_mask in pointers or op.in_mask2 in pointers for op in args[0]):
+                return result, None
+        try:
+            return result, Program(rec, pointers, _copy(result), tree, static)
+        except _NotRecordable:
+            return result, None
+
+
+def _static_key(v, held):
+    if v is None or isinstance(v, (int, float, str, bool)):
+        return v
+    if torch.is_tensor(v):
+        return (v.data_ptr(), v.shape, v.stride(), v.dtype)
+    if isinstance(v, (list, tuple)):
+        return tuple([_static_key(x, held) for x in v])
+    held.append(v)
+    return id(v)
+
+
+def _is_nhwc(t) -> bool:
+    return (t.dim() == 4 and t.is_cuda and t.dtype in (torch.float32, torch.bfloat16)
+            and t.is_contiguous(memory_format=torch.channels_last))
+
+
+def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
+    """Decorator of a pass: method(self, *args).  The first `dense` arguments are dense tensors and the next `masked`
+    ones Masked pairs (or None); those may live anywhere, everything else has to be the same object or memory to be
+    the same pass.  free_masks: plain mask tensors of the pairs may live anywhere, too.  trees: positions of further
+    arguments that are modules the pass reads.  record: name of another method to record in place of this one, tried
+    first, with the same result (ValueDependentMask: it does not apply)."""
+    def decorate(method):
+        @functools.wraps(method)
+        def wrapped(self, *args, **kw):
+            if kw or not enabled or _active is not None or not _idle():
+                return method(self, *args, **kw)
+            key, pointers, held = [method.__name__], [], []
+            for i, a in enumerate(args):
+                if a is not None and i < dense + masked:
+                    x = a if i < dense else a[0]
+                    if not torch.is_tensor(x) or not _is_nhwc(x):
+                        return method(self, *args)
+                    pointers.append(x.data_ptr())
+                    key += (x.shape, x.dtype, x.device.index)
+                    m = None if i < dense or len(a) < 2 else a[1]
+                    if torch.is_tensor(m):
+                        n, _, h, w = x.shape
+                        if (m.dtype not in (torch.uint8, torch.bool) or m.shape != (n, 1, h, w) or not m.is_contiguous()
+                                or m.device != x.device):
+                            return method(self, *args)
+                        if free_masks:
+                            pointers.append(m.data_ptr())
+                            key.append("mask")
+                        else:
+                            key.append(m.data_ptr())
+                    else:
+                        key.append(_static_key(m, held))
+                else:
+                    key.append(_static_key(a, held))
+            if not pointers or len(set(pointers)) != len(pointers):
+                return method(self, *args)
+            key = tuple(key)
+            cache = self.__dict__.get("_replay")
+            if cache is None:
+                cache = self.__dict__["_replay"] = _Cache()
+            ent = cache.get(key)
+            if type(ent) is Program:
+                if ent.valid():
+                    cache.move_to_end(key)
+                    return ent.run(pointers, key[3])
+                # outdated: recorded anew at the next pass, or later and later if recordings here never last
+                w = cache[key] = _Waiting()
+                if ent.runs < 16:
+                    w.step = w.next = ent.step
+                ent = w
+            if ent is None:
+                while len(cache) >= MAX_RECORDINGS:
+                    cache.popitem(last=False)
+                ent = cache[key] = _Waiting()
+            ent.seen += 1
+            if ent.seen < ent.next:
+                return method(self, *args)
+            # tried again after twice as many passes each time, so that a pass that cannot be recorded, or whose
+            # surroundings change all the time, costs little more than it did
+            ent.step = min(2 * ent.step, 256)
+            ent.next = ent.seen + ent.step
+            fns = ([functools.partial(getattr(self, record), *args)] if record else []) + [
+                functools.partial(method, self, *args)]
+            result, program = _record(self, fns, pointers, (self,) + tuple(args[i] for i in trees), held)
+            if program is not None:
+                program.step = ent.step
+                cache[key] = program
+            return result
+        return wrapped
+    return decorate

@@ -368,3 +368,22 @@ def test_three_term_shape_query_needs_no_gpu(mie_lib):
     assert takes(3, 1, 64, 64, 256) == 1 and takes(5, 1, 256, 0, 128) == 1 and takes(5, 2, 32, 0, 64) == 1
     assert takes(3, 2, 64, 0, 64) == 0 and takes(7, 1, 64, 0, 64) == 0 and takes(1, 1, 64, 0, 64) == 0
     assert takes(3, 1, 48, 0, 64) == 0 and takes(3, 1, 64, 0, 48) == 0 and takes(5, 2, 24, 0, 64) == 0
+
+
+def test_call_sequences_check_what_they_are_given(mie_lib):
+    # every sequence below is rejected before a launch, or ends at a call whose own validation rejects it
+    idx = mie_lib.mie_call_index(b"mie_mask_from_delta")
+    assert idx >= 0 and mie_lib.mie_call_signature(idx) == b"riiiifwi"
+    assert mie_lib.mie_call_index(b"mie_version") == -2 and mie_lib.mie_call_signature(-1) is None
+    buf = (ctypes.c_uint64 * 64)()
+    words = (ctypes.c_uint64 * 8)(0, 1, 8, 8, 4, 0, ctypes.addressof(buf), 0)
+    patch = (ctypes.c_int32 * 2)(0, 0)
+    call = lambda **kw: (_lib.MieCall * 1)(_lib.MieCall(**dict(dict(entry=idx, n_args=8, n_patches=0, reserved=0, args=ctypes.addressof(words), patches=ctypes.addressof(patch)), **kw)))
+    inputs = (ctypes.c_uint64 * 1)(0)
+    run = lambda c, n_in=1: mie_lib.mie_run_calls(c, 1, inputs, n_in, None)
+    assert mie_lib.mie_run_calls(None, 0, None, 0, None) == 0
+    assert mie_lib.mie_run_calls(None, 1, None, 0, None) == -1
+    assert run(call(entry=10000)) == -1 and run(call(n_args=7)) == -1 and run(call(args=None)) == -1
+    assert run(call(n_patches=1), 0) == -1 and "patches argument 0 from input 0" in mie_lib.mie_last_error_string().decode()
+    assert run(call()) == -1                     # delta is NULL
+    assert run(call(n_patches=1)) == -1          # ... and so is the input that takes its place

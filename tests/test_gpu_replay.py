@@ -1,0 +1,149 @@
+"""Recorded passes (maskedincrementeval_amd/replay.py) against the same passes walked in Python."""
+import copy
+
+import pytest
+import torch
+
+from maskedincrementeval_amd import mask_incr_modules as mm
+from maskedincrementeval_amd import ops, replay
+from maskedincrementeval_amd.e2depth_incr import E2VIDRecurrentIncr
+from maskedincrementeval_amd.evflownet_incr import MultiResUNetRecurrentIncr
+from maskedincrementeval_amd.synthetic import event_voxel_delta, gaussian_delta, seed_module_
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _cl(t, dtype=torch.float32):
+    return t.to(DEV).to(dtype).contiguous(memory_format=torch.channels_last)
+
+
+def _walked(fn, *args):
+    replay.enabled = False
+    try:
+        return fn(*args)
+    finally:
+        replay.enabled = True
+
+
+def _programs(m):
+    return [p for p in m.__dict__.get("_replay", {}).values() if isinstance(p, replay.Program)]
+
+
+def _equal(a, b):
+    if torch.is_tensor(a):
+        assert torch.equal(a, b)
+    elif isinstance(a, (list, tuple)):
+        assert len(a) == len(b)
+        for x, y in zip(a, b):
+            _equal(x, y)
+    elif a is not None:
+        assert torch.equal(a.pixmask, b.pixmask) and torch.equal(a.active_tiles(), b.active_tiles())
+        assert torch.equal(a.stale_tiles(), b.stale_tiles())
+
+
+@pytest.mark.parametrize("net,dtype,feed,fuse", [
+    ("e2depth", torch.float32, False, True), ("e2depth", torch.float32, True, True), ("e2depth", torch.bfloat16, False, True),
+    ("e2depth", torch.float32, False, False), ("transposed", torch.float32, False, True), ("upsample", torch.bfloat16, False, True),
+    ("upsample", torch.float32, False, False)])
+def test_recorded_network_steps_equal_walked_steps(net, dtype, feed, fuse):
+    h, w, bins = (48, 80, 5) if net == "e2depth" else (64, 96, 4)
+    make = (lambda: E2VIDRecurrentIncr(fuse=fuse)) if net == "e2depth" else (
+        lambda: MultiResUNetRecurrentIncr(num_bins=4, decoder=net, fuse=fuse))
+    a, b = (seed_module_(make(), seed=3).to(DEV).eval() for _ in range(2))
+    x0 = _cl(torch.randn(1, bins, h, w, generator=torch.Generator().manual_seed(1)), dtype)
+    with torch.no_grad():
+        pa = pb = None
+        for i in range(12):
+            if i in (0, 7, 8, 9):
+                extra = (None,) if net == "e2depth" else ()
+                _equal(a.forward_refresh_reservoirs(x0, *extra), _walked(b.forward_refresh_reservoirs, x0, *extra))
+                pa = pb = None
+            d = _cl(event_voxel_delta(1, bins, h, w, 0.05, seed=40 + i)[0], dtype)       # a new address every step
+            if net == "e2depth":
+                ra, rb = a([d, None], pa), _walked(b, [d, None], pb)
+                _equal(ra, rb)
+                if feed:
+                    pa, pb = ra[1], rb[1]
+            else:
+                _equal(a([d, None]), _walked(b, [d, None]))
+    assert bool(_programs(a)) == fuse and not _programs(b)      # (un-fused: the pass copies slices and concats)
+    assert not _programs(copy.deepcopy(mm.nnConvIncr(32, 32, 3)))
+
+
+@pytest.mark.parametrize("change", ["weight", "in_place", "data", "reservoir", "threshold", "setting", "hook", "function", "member"])
+def test_a_recorded_step_notices_what_changed(change, monkeypatch):
+    h, w = 48, 80
+    a, b = (seed_module_(E2VIDRecurrentIncr(), seed=3).to(DEV).eval() for _ in range(2))
+    ds = [_cl(event_voxel_delta(1, 5, h, w, 0.05, seed=60 + i)[0]) for i in range(4)]
+    seen = []
+    with torch.no_grad():
+        for n in (a, b):
+            n.forward_refresh_reservoirs(_cl(torch.ones(1, 5, h, w)), None)
+        for i in range(8):
+            _equal(a([ds[i % 4], None], None)[0], _walked(b, [ds[i % 4], None], None)[0])
+        assert _programs(a)
+        for n in (a, b):
+            conv, act = n.unetrecurrent.head.conv2d, n.unetrecurrent.head.activation
+            if change == "weight":
+                conv.weight = torch.nn.Parameter(conv.weight * 0.5)
+            elif change == "in_place":
+                conv.weight.mul_(0.5)
+            elif change == "data":
+                conv.weight.data = conv.weight.data * 0.5
+            elif change == "reservoir":
+                act.in_res.reservoir = act.in_res.reservoir + 0.25
+            elif change == "threshold":
+                mm.set_input_threshold(n, 1e-3)
+            elif change == "hook":
+                conv_hook = n.unetrecurrent.encoders[0].register_forward_hook(lambda *_: seen.append(1))
+            elif change == "member":
+                n.unetrecurrent.resblocks[0] = seed_module_(type(n.unetrecurrent.resblocks[0])(256, 256), seed=9).to(DEV)
+                n.unetrecurrent.resblocks[0].relu1.in_res.reservoir = ops.new_nhwc(1, 256, h // 8, w // 8, DEV)
+                n.unetrecurrent.resblocks[0].relu2.in_res.reservoir = ops.new_nhwc(1, 256, h // 8, w // 8, DEV)
+        if change == "setting":
+            monkeypatch.setattr(ops, "f32_matmul", "native")
+            for n in (a, b):        # the gate reservoirs' column order is the same in both forms
+                n.forward_refresh_reservoirs(_cl(torch.ones(1, 5, h, w)), None)
+        if change == "function":
+            orig = ops.conv_masked
+            monkeypatch.setattr(ops, "conv_masked", lambda *args, **kw: (seen.append(1), orig(*args, **kw))[1])
+        for i in range(8):
+            before = len(seen)
+            ra = a([ds[i % 4], None], None)
+            if change in ("hook", "function"):
+                assert len(seen) > before
+            _equal(ra[0], _walked(b, [ds[i % 4], None], None)[0])
+        if change == "hook":
+            conv_hook.remove()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mask", ["tensor", "bool", "tile", None])
+def test_recorded_layers_equal_walked_layers(dtype, mask):
+    n, c, h, w = 2, 32, 19, 27
+    make = lambda: (seed_module_(mm.nnConvIncr(c, c, 3, 1, 1), seed=2).to(DEV).eval(), mm.nnReservedActivation(mm.leaky_relu_op(0.01), refine_mask=False), mm.nnReluIncr())
+    a, b = make(), make()
+    x0 = _cl(torch.randn(n, c, h, w, generator=torch.Generator().manual_seed(20)), dtype)
+    sets = {}
+
+    def step(layers, d, m):
+        conv, leaky, relu = layers
+        return relu(conv([conv.forward_fused([d, m], leaky)[0], m]))
+
+    with torch.no_grad():
+        for conv, leaky, relu in (a, b):
+            relu.forward_refresh_reservoirs(conv.forward_refresh_fused(x0, leaky))
+        for i in range(9):
+            d, m = gaussian_delta(n, c, h, w, 0.1, 0.2, seed=80 + i)
+            d, m = _cl(d, dtype), m.to(DEV)
+            masks = []
+            for key in "ab":
+                if mask == "tile":
+                    ts = sets.setdefault(key, mm.TileMask(n, h, w, DEV))
+                    ops.build_mask_tiles(m, None, n, h, w, 0, 1, 1, 0, ts)
+                    masks.append(ts)
+                else:
+                    masks.append(None if mask is None else m.bool() if mask == "bool" else m)
+            _equal(step(a, d, masks[0]), _walked(step, b, d, masks[1]))
+    assert all(_programs(m) for m in (a[0], a[2])) and not _programs(b[0])
