@@ -147,6 +147,10 @@ class LayerProbe:
             return dict(kind="conv", k=k, s=1, cin=c, cout=filt.shape[3], h=h, w=w, n=n, xmask=amask,
                         x2mask=bmask, ts=out_ts, fused=reservoir is not None, up=True, two=b_ is not None)
 
+        def upconv2x_desc(a_, amask, b_, bmask, filt, out_ts, out_delta, reservoir=None, *a, **kw):
+            # the same layer as four 4x4 convs at the resolution of its inputs: 16 taps an output, four filters
+            return dict(upconv_desc(a_, amask, b_, bmask, filt, 5, 2, out_ts, out_delta, reservoir), taps=16, filter_taps=64)
+
         def upconv_pred_desc(a_, amask, b_, bmask, filt, out_ts, reservoir, act, slope, skip, skip_mask, *a, **kw):
             n, c, h, w = a_.shape
             return dict(kind="conv", k=5, s=1, cin=c, cout=filt.shape[3], h=h, w=w, n=n, xmask=amask, x2mask=bmask,
@@ -167,6 +171,7 @@ class LayerProbe:
         self._wrap("tconv2x_masked", tconv2x_desc)
         self._wrap("tconv_masked", tconv_desc)
         self._wrap("upconv_masked", upconv_desc)
+        self._wrap("upconv2x_masked", upconv2x_desc)
         self._wrap("upconv_pred_masked", upconv_pred_desc)
         self._wrap("conv_gates_incr", conv_gates_desc)
         self._wrap("act_incr", pw_desc("act", 1, 1))
@@ -200,7 +205,7 @@ class LayerProbe:
                 a_out = int(ts.pixmask.sum().item())
                 cin, cout, k = d["cin"], d["cout"], d["k"]
                 es = self.es
-                byts = P + a_in * cin * es + cin * cout * k * k * es + ts.capacity * 4
+                byts = P + a_in * cin * es + cin * cout * d.get("filter_taps", k * k) * es + ts.capacity * 4
                 if d.get("gates"):
                     # gate reservoirs read + written, cell reservoir read + written, previous cell read,
                     # hidden and cell deltas written; the 4*hid-channel gate delta never reaches memory
@@ -215,7 +220,7 @@ class LayerProbe:
                     byts += a_out * cout * es
                     if d["fused"]:
                         byts += 2 * a_out * cout * 4
-                flops = 2 * a_out * cin * cout * k * k + (4 * a_out * cout if d.get("pred") else 0)
+                flops = 2 * a_out * cin * cout * d.get("taps", k * k) + (4 * a_out * cout if d.get("pred") else 0)
                 if d.get("tconv"):
                     # stride-s transposed conv: an output pixel meets (k/s)^2 taps on average
                     flops = 2 * a_out * cin * cout * k * k // (d["s"] * d["s"])
@@ -513,7 +518,8 @@ class NetBench:
         tile set, same buffers) launched `reps` times on the launch stream, each launch between two HIP events
         of its own; `us` is the mean of the pairs less what an empty pair reads."""
         torch = self.torch
-        convs = [l for l in layers if l["op"] in ("conv_masked", "conv_gates_incr", "upconv_masked", "upconv_pred_masked", "tconv2x_masked")]
+        convs = [l for l in layers if l["op"] in ("conv_masked", "conv_gates_incr", "upconv_masked", "upconv2x_masked", "upconv_pred_masked",
+                                            "tconv2x_masked")]
         dom = max(convs, key=lambda l: l["us"])
         orig, cargs, ckw = agg[layers.index(dom)]["call"]
         with torch.no_grad():

@@ -838,6 +838,38 @@ int mie_events_to_frame_bf16(const double* events, int n_events, int kind, int n
                              double start_old, double start_new, double delta_t,
                              int delta, float* sums, void* out, uint8_t* pixmask, void* stream);
 
+/*
+ * The decoder layer at the resolution of its inputs: out = 5x5 conv (pad 2) over up2x(a + b) as four 4x4 convs over
+ * a + b, one per output phase, with combined filters -- mie_upconv_masked's layer (interpolate_from_module +
+ * nnConvIncr.forward, incr_modules/e2depth_incr.py:306-313,429-431) in 16 instead of 25 products per weight.
+ *   filter_up : mie_pack_filter_up2x's copy for the dtype
+ *   dtype     : MIE_DTYPE_BF16, or MIE_DTYPE_F32_BF16X3 for fp32 deltas; c a multiple of 64 / 32, cout of 32;
+ *               planes of at least 2x2 pixels
+ *   the rest as in mie_upconv_masked.  The tile set's flags are read: it must be one of the library's builders'.
+ * bf16: what is rounded to bf16 is a + b and the combined weights, each once (mie_upconv_masked: the up-sampled sums and
+ * the plain weights).
+ */
+int mie_upconv2x_masked(const void* a, const uint8_t* amask, const void* b,
+                        const uint8_t* bmask, int c, int h_in, int w_in,
+                        const void* filter_up, int cout, const mie_tileset* out,
+                        void* out_delta, const void* addend, float* reservoir,
+                        int act_kind, float slope, int dtype, void* stream);
+
+/* Its dense twin (every tile of `out` active): bias, activation and reservoir fill as in mie_conv_refresh. */
+int mie_upconv2x_refresh(const void* a, const void* b, int c, int h_in, int w_in,
+                         const void* filter_up, int cout, const float* bias,
+                         const mie_tileset* out, void* out_dense, float* reservoir,
+                         int act_kind, float slope, int dtype, void* stream);
+
+/*
+ * Combined filters of mie_upconv2x_masked from a plain fp32 [cin][5][5][cout] filter (combined in double, rounded once):
+ * `packed` holds 4 * 80 * cin * cout bf16 values (16 taps, and the planes' four sides and corners,
+ * per phase) (MIE_DTYPE_BF16) or three times that (MIE_DTYPE_F32_BF16X3).
+ * cin a multiple of 16, cout of 32.
+ */
+int mie_pack_filter_up2x(const float* filter, int cin, int cout, void* packed, int dtype,
+                         void* stream);
+
 /* ---- recorded call sequences ------------------------------------------------
  * A step of a network is the same sequence of calls every time, with the same
  * arguments but for the pointers of its inputs.  A host that has noted them once

@@ -38,7 +38,7 @@ EXPORTS = (
     "mie_conv_masked_ws", "mie_convgru_gates_incr", "mie_upsample2x_pair_incr", "mie_conv_masked_noalloc",
     "mie_convlstm_gates_refresh", "mie_convgru_gates_refresh", "mie_mul_dense", "mie_tconv2x_masked",
     "mie_tconv2x_refresh", "mie_conv_f32x3_takes", "mie_build_mask_plan", "mie_build_mask_plan_wgs",
-    "mie_call_index", "mie_call_signature", "mie_run_calls",
+    "mie_upconv2x_masked", "mie_upconv2x_refresh", "mie_pack_filter_up2x", "mie_call_index", "mie_call_signature", "mie_run_calls",
 )
 PLAN_MAX_STEPS = 40
 
@@ -177,6 +177,12 @@ def _declare(l):
     l.mie_upconv_masked_ws.restype = ci
     l.mie_upconv_masked_ws.argtypes = [vp, vp, vp, vp, ci, ci, ci, vp, vp, ci, ci, ci, ci, tsp, vp, vp, vp, ci, cf, ci, vp,
                                        ctypes.c_longlong, vp]
+    l.mie_upconv2x_masked.restype = ci
+    l.mie_upconv2x_masked.argtypes = [vp, vp, vp, vp, ci, ci, ci, vp, ci, tsp, vp, vp, vp, ci, cf, ci, vp]
+    l.mie_upconv2x_refresh.restype = ci
+    l.mie_upconv2x_refresh.argtypes = [vp, vp, ci, ci, ci, vp, ci, vp, tsp, vp, vp, ci, cf, ci, vp]
+    l.mie_pack_filter_up2x.restype = ci
+    l.mie_pack_filter_up2x.argtypes = [vp, ci, ci, vp, ci, vp]
     l.mie_tconv_refresh.restype = ci
     l.mie_tconv_refresh.argtypes = [vp, ci, ci, ci, vp, ci, ci, ci, ci, vp, tsp, vp, vp, ci, cf, ci, vp]
     l.mie_tconv_masked.restype = ci

@@ -1,0 +1,636 @@
+// The decoder layer -- 5x5 conv, pad 2, over up2x(a + b), the bilinear x2 up-sampling of the sum of two deltas -- computed
+// at the resolution of its inputs (gfx950).
+//
+// Sub-pixel phases.  Along one axis output 2Y + q (q = 0, 1) of the conv over the up-sampled signal is a fixed combination
+// of four input samples, L[Y - 2 .. Y + 1] for q = 0 and L[Y - 1 .. Y + 2] for q = 1, with coefficients that are sums of the
+// five weights times 1/4 and 3/4.  In two dimensions each of the four output phases (py, px) is therefore an ordinary 4x4
+// conv over a + b: 16 taps where the conv over the up-sampled tile multiplies 25, nothing to blend, and a staged tile of
+// 11x11 input pixels for 64 outputs where the other form stages and blends 12x12 (k_conv_mfma<..., UP>, which
+// this replaces wherever a combined filter can be made: 0.64 of its matrix-core work and none of its blend).
+//
+// Border.  Up-sampled rows outside the image are the conv's zero padding and the bilinear taps are clamped, so the outputs of
+// input rows 0 and H - 1 and of columns 0 and W - 1 have filters of their own: three input rows deep across the border
+// instead of four.  Those positions go to workgroups of their own ("strips": 32 positions along one side, half an M block,
+// 12 taps; the columns' strips leave the corners to the rows', which subtract there what the column outside the image
+// would have given, a 3x1 filter on the corner lane only).  Everything else runs 16 taps and no special case.  (First built
+// as corrections inside ordinary blocks: a corner block then ran 25 taps' worth, and on the 33x44 plane, one round of
+// workgroups, every launch took as long as its corners.)
+//
+// Work decomposition: one workgroup (4 waves) = an 8x8 block of input positions (or a strip) x one phase x 32 * WN output
+// channels, M = 64, as in k_conv_mfma (same LDS layout, operand pairing, three-term form of fp32 deltas).  The filter runs
+// through a register ring three units ahead, across sub-chunks and chunks.
+// Work is found from the 8x8 tiles' flag words: a workgroup looks at the tiles its positions touch and leaves if none is
+// active (zeroing its pixels of stale ones).  There is no list to walk: behind the bottleneck these planes are active
+// throughout (every tile, at every density from 0.5 %), and a list of blocks would be one more tile set to build.
+// (Flag words are looked up where they are needed: kept in a small array indexed at run time they went to LDS, whose
+// promotion reads the workgroup size from the dispatch packet in host memory -- 7 us at the start of every workgroup.)
+#include "mie_conv_mfma_impl.h"
+
+namespace {
+
+// Units of a phase's filter: 16 of the interior, [row][column]; then 12 of each side, [depth across the border][tap along
+// it], the sides at the top and the bottom followed by two groups of their corners (three taps across and a zero).
+constexpr int UNITS = 80, U_TOP = 16, U_BOTTOM = 36, U_LEFT = 56, U_RIGHT = 68;
+constexpr int STRIP = 32;                 // positions of a border workgroup
+
+struct Up2xOrder {
+  const uint32_t* flags;                  // tile flags of the output tile set
+  int blocks_y, blocks_x;                 // 8x8 blocks of the positions 1 .. H - 2, 1 .. W - 2
+  int strips_x, strips_y;                 // strips of the top (and of the bottom), of the left (and of the right)
+  int items;                              // of a sample: the blocks, then the strips
+  int combos, groups;                     // (phase, slab) pairs, and how many parts of the launch order they are cut into
+  int total;                              // samples * items * combos
+  int nci;                                // blocks of 16 input channels in the filter
+};
+
+// 1-D coefficients of the five weights.  row 0..3: the 4-tap filter of phase q (window row 0 is Y - 2 + q); 4 / 5: what the
+// continued signal gives too much at the first / last position; 6..8 / 9..11: the whole filter of the first / last
+// position on the samples 0, 1, 2 steps inside.
+__device__ void up2x_coef(int q, int row, double (&c)[5]) {
+  for (int k = 0; k < 5; ++k) {
+    double v = 0.0;
+    if (row < 4) {
+      // up-sampled sample s = q - 2 + k relative to 2Y; even s = 2R: L[R - 1] / 4 + 3 L[R] / 4, odd: 3 L[R] / 4 + L[R + 1] / 4
+      const int s = q - 2 + k, r = (s - (s & 1)) / 2;           // (s & 1 is 0 or 1 for negative s, too)
+      const int lo = (s & 1) ? r : r - 1, want = row - 2 + q;
+      if (want == lo) v = (s & 1) ? 0.75 : 0.25;
+      else if (want == lo + 1) v = (s & 1) ? 0.25 : 0.75;
+    } else if (row == 4) {
+      v = (k < 2 - q) ? 1.0 : 0.0;
+    } else if (row == 5) {
+      v = (k > 3 - q) ? 1.0 : 0.0;
+    }
+    c[k] = v;
+  }
+  if (row < 6) return;
+  const bool first = row < 9;
+  const int depth = first ? row - 6 : row - 9;
+  double t[5];
+  for (int w = 0; w < 4; ++w) {
+    const int at = first ? w - 2 + q : 2 - q - w;               // steps inside of window row w (outside: the edge sample)
+    if ((at < 0 ? 0 : at) != depth) continue;
+    up2x_coef(q, w, t);
+    for (int k = 0; k < 5; ++k) c[k] += t[k];
+  }
+  if (depth == 0) {
+    up2x_coef(q, first ? 4 : 5, t);
+    for (int k = 0; k < 5; ++k) c[k] -= t[k];
+  }
+}
+
+// P[phase][ci/16][unit][term][(ci%16)/8][co][ci%8] in bf16: one term (bf16 deltas) or the three of an fp32 value.
+template <int PL>
+__global__ __launch_bounds__(256) void k_pack_up2x(const float* __restrict__ f, mie_bf16* __restrict__ p, int cin, int cout) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= 4LL * UNITS * cin * cout) return;
+  const int co = (int)(i % cout);
+  long long t = i / cout;
+  const int ci = (int)(t % cin);
+  t /= cin;
+  const int u = (int)(t % UNITS), ph = (int)(t / UNITS);
+  int vr, hr;
+  double sign = 1.0;
+  if (u < U_TOP) {
+    vr = u >> 2; hr = u & 3;
+  } else if (u < U_LEFT) {
+    const int side = u < U_BOTTOM ? 0 : 1, k = u - (side ? U_BOTTOM : U_TOP);
+    if (k < 12) { vr = 6 + 3 * side + (k >> 2); hr = k & 3; }
+    else { vr = 6 + 3 * side + (k & 3); hr = k < 16 ? 4 : 5; sign = (k & 3) < 3 ? -1.0 : 0.0; if ((k & 3) == 3) vr = 0; }
+  } else {
+    const int side = u < U_RIGHT ? 0 : 1, k = u - (side ? U_RIGHT : U_LEFT);
+    vr = k & 3; hr = 6 + 3 * side + (k >> 2);
+  }
+  double cv[5], ch[5], v = 0.0;
+  up2x_coef(ph >> 1, vr, cv);
+  up2x_coef(ph & 1, hr, ch);
+  for (int ky = 0; ky < 5; ++ky)
+    for (int kx = 0; kx < 5; ++kx) v += cv[ky] * ch[kx] * (double)f[((long long)ci * 25 + ky * 5 + kx) * cout + co];
+  const float w = (float)(sign * v);
+  const long long o = ((((((long long)ph * (cin / 16) + ci / 16) * UNITS + u) * PL) * 2 + (ci % 16) / 8) * cout + co) * 8 + ci % 8;
+  const long long term = 2LL * cout * 8;
+  const mie_bf16 hi = (mie_bf16)w;
+  p[o] = hi;
+  if (PL == 3) {
+    const float r1 = w - (float)hi;
+    const mie_bf16 mid = (mie_bf16)r1;
+    p[o + term] = mid;
+    p[o + 2 * term] = (mie_bf16)(r1 - (float)mid);
+  }
+}
+
+template <typename T, int WN>
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvArgsT<T> a, Up2xOrder od) {
+  constexpr bool X3 = sizeof(T) == 4;
+  typedef mie_bf16 TL;
+  constexpr int PL = X3 ? 3 : 1;
+  constexpr int GPS = X3 ? 2 : 1;                            // 16-byte global loads per staging slot
+  constexpr int NBUF = X3 ? 2 : 1;
+  constexpr int EPS = 8, SUB = 16;
+  constexpr int WK = 4 / WN;
+  constexpr int IT = 11;
+  constexpr int CC = X3 ? 32 : 64;
+  constexpr int LS = CC + EPS;
+  constexpr int Q4 = CC / EPS;
+  constexpr int NSLOT = IT * IT * Q4;
+  constexpr int NLD = (NSLOT + 255) / 256;
+  constexpr int RP = row_pitch_dw(IT, LS / 2, 1) * 2;
+  constexpr int ZOFF = IT * RP;                              // the zero pixel behind the tile
+  constexpr int STAGE = ZOFF + LS;
+  constexpr int SPX = STRIP + 3;                             // staged positions along a strip, three rows of them
+  constexpr int RPS = SPX * LS;
+  static_assert(3 * SPX <= IT * IT && 3 * RPS <= ZOFF, "a strip stages less than a block");
+  constexpr int NQ = CC / SUB;
+  constexpr int KS = NQ < WK ? NQ : WK;                      // the k-split: over sub-chunks, ...
+  constexpr int NQW = NQ / KS;                               // ... several of them per wave, ...
+  constexpr int RC = WK / KS;                                // ... or one of them and half of the tap rows
+  constexpr int NI = 4 / RC;                                 // tap rows of a wave
+  constexpr int UPC = 4 * NI * NQW;                          // units per chunk and wave
+  constexpr int CO_BLK = 32 * WN;
+  constexpr int RED = WK * 64 * CO_BLK;
+  constexpr int STAGE_F = NBUF * PL * STAGE / 2;
+  constexpr int SMEM = STAGE_F > RED ? STAGE_F : RED;
+  static_assert(SMEM * 4 <= 65536, "LDS budget");
+  __shared__ __attribute__((aligned(16))) float smem[SMEM];
+  TL* const sbuf = reinterpret_cast<TL*>(smem);
+
+  // ---- which positions, phase and slab: each XCD (workgroup index mod 8) takes a contiguous eighth of the order (group of
+  // (phase, slab) pairs, item, pair within the group)
+  const int bid = blockIdx.x + conv_args_entry_zero(a);
+  const int share = (od.total + 7) >> 3;
+  const int v = (bid & 7) * share + (bid >> 3);
+  if ((bid >> 3) >= share || v >= od.total) return;
+  const int cpg = od.combos / od.groups, per_group = a.ts.n * od.items * cpg;
+  const int cg = v / per_group, rem = v - cg * per_group;
+  const int it = rem / cpg, combo = cg * cpg + (rem - it * cpg);
+  const int phase = combo & 3, slab = combo >> 2;
+  const int n = it / od.items;
+  const int py = phase >> 1, px = phase & 1;
+  const int H = a.h_in, W = a.w_in, hout = a.ts.h, wout = a.ts.w;
+  // side: 0 a block at (y0, x0), rows x cols positions; 1 .. 4 a strip at the top, bottom, left, right
+  int side = 0, y0, x0, rows, cols;
+  {
+    int k = it - n * od.items;
+    const int nb = od.blocks_y * od.blocks_x;
+    if (k < nb) {
+      y0 = 1 + 8 * (k / od.blocks_x); x0 = 1 + 8 * (k % od.blocks_x);
+      rows = H - 1 - y0 < 8 ? H - 1 - y0 : 8; cols = W - 1 - x0 < 8 ? W - 1 - x0 : 8;
+    } else if ((k -= nb) < 2 * od.strips_x) {
+      side = 1 + (k >= od.strips_x ? 1 : 0);
+      x0 = STRIP * (k - (side - 1) * od.strips_x); y0 = side == 1 ? 0 : H - 1;
+      rows = 1; cols = W - x0 < STRIP ? W - x0 : STRIP;
+    } else {
+      k -= 2 * od.strips_x;
+      side = 3 + (k >= od.strips_y ? 1 : 0);
+      y0 = 1 + STRIP * (k - (side - 3) * od.strips_y); x0 = side == 3 ? 0 : W - 1;
+      rows = H - 1 - y0 < STRIP ? H - 1 - y0 : STRIP; cols = 1;
+    }
+  }
+  const bool lying = side == 1 || side == 2;                 // a strip along a row of the plane
+  // position p of the M block, relative to (y0, x0)
+  auto pos_y = [&](int p) { return side == 0 ? p >> 3 : (lying ? 0 : p); };
+  auto pos_x = [&](int p) { return side == 0 ? p & 7 : (lying ? p : 0); };
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l32 = lane & 31, half = lane >> 5;
+  const int wn = wave % WN, wk = wave / WN;
+  const int co0 = slab * CO_BLK, cout = a.cout;
+
+  // the tiles these positions touch (at most 3x3 or 1x9 of them), one per lane
+  const int tl_y = y0 >> 2, tl_x = x0 >> 2, tl_nx = ((2 * (x0 + cols) - 1) >> 3) - tl_x + 1, tl_ny = ((2 * (y0 + rows) - 1) >> 3) - tl_y + 1;
+  const int* const flags_n = reinterpret_cast<const int*>(od.flags) + (long long)n * a.ts.tiles_y * a.ts.tiles_x;
+  {
+    const bool in = lane < tl_nx * tl_ny;
+    const int f = flags_n[(tl_y + (in ? lane / tl_nx : 0)) * a.ts.tiles_x + tl_x + (in ? lane % tl_nx : 0)];
+    if (__ballot((f & 1) != 0) == 0ull) {
+      if (__ballot((f & 2) != 0) != 0ull)          // nothing active, something stale: zero this phase of it
+        for (int idx = tid; idx < 64 * (CO_BLK / 4); idx += 256) {
+          const int p = idx / (CO_BLK / 4), col = 4 * (idx - p * (CO_BLK / 4));
+          const int dy = pos_y(p), dx = pos_x(p);
+          if (dy >= rows || dx >= cols) continue;
+          const int oy = 2 * (y0 + dy) + py, ox = 2 * (x0 + dx) + px;
+          if ((flags_n[(oy >> 3) * a.ts.tiles_x + (ox >> 3)] & 2) != 0)
+            mie_st4(a.out, (((long long)n * hout + oy) * wout + ox) * cout + co0 + col, make_float4(0.f, 0.f, 0.f, 0.f));
+        }
+      return;
+    }
+  }
+
+  // ---- epilogue plan: a thread owns groups of four adjacent output channels of a pixel; the mask bytes are asked for now
+  constexpr int QPP = CO_BLK / 4;
+  constexpr int PER = 64 * QPP / 256;
+  constexpr int PB = PER > 4 ? 4 : PER;
+  unsigned live_bits = 0u;
+#pragma unroll
+  for (int g = 0; g < PER; ++g) {
+    const int p = (tid + 256 * g) / QPP;
+    const int dy = pos_y(p), dx = pos_x(p);
+    if (dy < rows && dx < cols &&
+        (a.refresh || a.ts.pixmask[((long long)n * hout + 2 * (y0 + dy) + py) * wout + 2 * (x0 + dx) + px] != 0))
+      live_bits |= 1u << g;
+  }
+
+  // ---- staging plan.  A block: its 11x11 window, rows from y0 - 2 + py on.  A strip: three rows of 35, row b the pixels b
+  // steps inside the border, from two (one) before the first position on.  Edge pixels continue the plane.
+  const bool m1 = a.xm != nullptr, has2 = a.x2 != nullptr, m2 = has2 && a.x2m != nullptr;
+  unsigned st_off[NLD];                                      // byte offset of the slot in chunk 0
+  int st_lds[NLD];
+  unsigned ok1 = 0u, ok2 = 0u;
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) {
+    const int slot = tid + 256 * i;
+    const int q4 = slot & (Q4 - 1);
+    int pix = slot / Q4, iy, ix;
+    if (side == 0) {
+      if (pix >= IT * IT) pix = 0;
+      const int r = pix / IT, c = pix - r * IT;
+      iy = y0 - 2 + py + r; ix = x0 - 2 + px + c;
+      st_lds[i] = r * RP + c * LS + EPS * q4;
+    } else {
+      if (pix >= 3 * SPX) pix = 0;
+      const int b = pix / SPX, c = pix - b * SPX;
+      const int in = (side & 1) ? b : -b, along = c - 2 + (lying ? px : py);
+      iy = y0 + (lying ? in : along); ix = x0 + (lying ? along : in);
+      st_lds[i] = b * RPS + c * LS + EPS * q4;
+    }
+    iy = iy < 0 ? 0 : (iy >= H ? H - 1 : iy);
+    ix = ix < 0 ? 0 : (ix >= W ? W - 1 : ix);
+    const int po = (n * H + iy) * W + ix;
+    st_off[i] = ((unsigned)po * (unsigned)a.c1 + (unsigned)(EPS * q4)) * (unsigned)sizeof(T);
+    const unsigned v1 = m1 ? (unsigned)(a.xm[po] != 0) : 1u;
+    const unsigned v2 = m2 ? (unsigned)(a.x2m[po] != 0) : (has2 ? 1u : 0u);
+    ok1 |= v1 << i;
+    ok2 |= v2 << i;
+  }
+  const int n_slots = (side == 0 ? IT * IT : 3 * SPX) * Q4;
+  const int nch = a.c1 / CC;
+
+  // Loads are for every pixel, active or not (these planes are dense): masked values are dropped when they are stored.
+  float4 ra[NLD][GPS], rb[NLD][GPS];
+  const T* x2p = has2 ? a.x2 : a.x;
+  auto stage_load = [&](int c) {
+    const char* xc = reinterpret_cast<const char*>(a.x + c * CC);
+    const char* x2c = reinterpret_cast<const char*>(x2p + c * CC);
+#pragma unroll
+    for (int i = 0; i < NLD; ++i)
+#pragma unroll
+      for (int g = 0; g < GPS; ++g) {
+        ra[i][g] = *reinterpret_cast<const float4*>(xc + st_off[i] + 16 * g);
+        rb[i][g] = *reinterpret_cast<const float4*>(x2c + st_off[i] + 16 * g);
+      }
+  };
+  auto stage_store = [&](int buf) {
+    TL* dst = sbuf + buf * (PL * STAGE);
+    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const bool k1 = (ok1 >> i) & 1u, k2 = (ok2 >> i) & 1u;
+      float fa[8], fb[8], f[8];
+      if constexpr (X3) {
+        const float4 a0 = k1 ? ra[i][0] : z4, a1 = k1 ? ra[i][1] : z4, b0 = k2 ? rb[i][0] : z4, b1 = k2 ? rb[i][1] : z4;
+        const float ta[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        const float tb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) fa[e] = ta[e], fb[e] = tb[e];
+      } else {
+        slot_to_f32(k1 ? ra[i][0] : z4, fa, T());
+        slot_to_f32(k2 ? rb[i][0] : z4, fb, T());
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = fa[e] + fb[e];
+      if (tid + 256 * i < n_slots) {
+        if constexpr (X3) {
+          float4 pl[3];
+          split3(f, pl);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
+        } else {
+          *reinterpret_cast<float4*>(dst + st_lds[i]) = f32_to_slot(f, T());
+        }
+      }
+    }
+  };
+
+  // ---- the units of this wave ---------------------------------------------------------------------------------------------
+  // A block: NI rows of four taps per sub-chunk.  A strip: groups of four units, packed in `strip`: codes 0..2 its rows, 3 / 4
+  // the corner groups of its first / last position (the two row classes of a k-split over rows share them out).
+  const int q0w = (RC > 1) ? wk % KS : wk * NQW;
+  const int cls = (RC > 1) ? wk / KS : 0;
+  unsigned strip = 0u;
+  int ng = 0;
+  {
+    auto add = [&](bool on, int code) {
+      strip |= on ? (unsigned)code << (4 * ng) : 0u;
+      ng += on ? 1 : 0;
+    };
+    if (cls == 0) { add(true, 0); add(true, 1); }
+    if (cls == RC - 1) { add(true, 2); add(lying && x0 == 0, 3); add(lying && x0 + cols == W, 4); }
+  }
+  const int u_side = side == 1 ? U_TOP : (side == 2 ? U_BOTTOM : (side == 3 ? U_LEFT : U_RIGHT));
+  const int jx = 2 - px;                                     // window column of the position itself
+  int a_lane[2];
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb) {
+    const int p = mb * 32 + l32;
+    a_lane[mb] = (side == 0 ? (p >> 3) * RP + (p & 7) * LS : l32 * LS) + SUB * q0w + EPS * half;
+  }
+  const bool at_first = l32 == 0, at_last = l32 == cols - 1;
+  const int b_lane = (half * cout + l32) * EPS;
+  const int unit_sz = PL * 2 * cout * EPS;                   // elements
+  const TL* const filt = reinterpret_cast<const TL*>(a.filt_mc) + (co0 + wn * 32) * EPS;
+  // the four units from `unit` on, of sub-chunk qi of this wave in chunk c
+  auto group_b = [&](int c, int qi, int unit) -> const TL* {
+    return filt + ((long long)(phase * od.nci + c * NQ + q0w + qi) * UNITS + unit) * unit_sz;
+  };
+  auto strip_unit = [&](int g) { return u_side + 4 * (int)((strip >> (4 * g)) & 15u); };
+  // the filter is read in order through one pointer per lane, set anew where a group does not follow the one before it
+  // (offsets from a base would all be kept in registers across the chunks)
+  const TL* bp;
+  auto seek_b = [&](const TL* gb) { bp = gb + b_lane; };
+  auto load_b = [&](float4 (&bv)[PL]) {
+#pragma unroll
+    for (int q = 0; q < PL; ++q) {
+      bv[q] = *reinterpret_cast<const float4*>(bp);
+      bp += 2 * cout * EPS;
+    }
+  };
+  auto first_b = [&](int c) { return group_b(c, 0, side == 0 ? 4 * NI * cls : strip_unit(0)); };
+
+  v16f acc[2], sm[X3 ? 2 : 1];
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      acc[mb][r] = 0.f;
+      if (X3) sm[mb][r] = 0.f;
+    }
+
+  float4 bring[4][PL];
+  seek_b(first_b(0));
+  stage_load(0);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) load_b(bring[i]);
+  // the zero pixels
+  for (int i = tid; i < NBUF * PL * (LS / EPS); i += 256) {
+    const int pl = i / (LS / EPS);
+    *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (i - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  stage_store(0);
+  __syncthreads();
+
+  // All loads of a chunk are unconditional (see k_conv_mfma); behind the last one "the next" is the chunk itself.
+  auto contract = [&](auto block) {
+    for (int c = 0; c < nch; ++c) {
+      const bool more = c + 1 < nch;
+      const int cn = more ? c + 1 : c;
+      const TL* const ub_next = first_b(cn);
+      stage_load(cn);
+      const TL* sin = sbuf + (c % NBUF) * (PL * STAGE);
+      if constexpr (decltype(block)::value) {
+        const TL* sa = sin + cls * NI * RP;
+        float4 av[2][2][PL];
+        auto load_a = [&](int u, float4 (&dst)[2][PL]) {
+          const int qi = u / (4 * NI), k = u % (4 * NI);
+#pragma unroll
+          for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+            for (int q = 0; q < PL; ++q)
+              dst[mb][q] = *reinterpret_cast<const float4*>(&sa[q * STAGE + a_lane[mb] + (k >> 2) * RP + (k & 3) * LS + SUB * qi]);
+        };
+        load_a(0, av[0]);
+#pragma unroll
+        for (int i = 0; i < UPC; ++i) {
+          const int ip = i + 3;
+          if (ip == UPC) seek_b(ub_next);
+          else if (ip % (4 * NI) == 0) seek_b(group_b(c, ip / (4 * NI), 4 * NI * cls));
+          load_b(bring[ip & 3]);
+          if (i + 1 < UPC) load_a(i + 1, av[(i + 1) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+          const auto& A = av[i & 1];
+          const auto& B = bring[i & 3];
+          if constexpr (X3) mma_unit2_x3(acc[0], acc[1], sm[0], sm[1], A[0], A[1], B);
+          else mma_unit2(acc[0], acc[1], A[0][0], A[1][0], B[0], mie_bf16());
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        // (lane's LDS offset, step from unit to unit) of group g of sub-chunk qi: rows for every lane, corners for theirs
+        auto lane_of = [&](int g, int qi, int& base, int& step) {
+          const int code = (int)((strip >> (4 * g)) & 15u);
+          const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
+          base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF;
+          step = on ? (corner ? RPS : LS) : 0;
+        };
+        float4 av[2][PL];
+        auto load_a = [&](int at, float4 (&dst)[PL]) {
+#pragma unroll
+          for (int q = 0; q < PL; ++q) dst[q] = *reinterpret_cast<const float4*>(&sin[q * STAGE + at]);
+        };
+        int base, step, qi = 0, g = 0;
+        lane_of(0, 0, base, step);
+        load_a(base, av[0]);
+        for (int left = NQW * ng; left > 0; --left) {
+          const bool end = g + 1 == ng;
+          const int gn = end ? 0 : g + 1, qn = left == 1 ? 0 : (end ? qi + 1 : qi);
+          const TL* const gb_next = left == 1 ? ub_next : group_b(c, qn, strip_unit(gn));
+          const bool corner = ((strip >> (4 * g)) & 15u) >= 3u;
+          int base_n, step_n;
+          lane_of(gn, qn, base_n, step_n);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            if (t == 1) seek_b(gb_next);
+            load_b(bring[(t + 3) & 3]);
+            // (a corner group has three units; its fourth A operand is read and not used)
+            load_a(t == 3 ? base_n : base + (t == 2 && corner ? 0 : (t + 1) * step), av[(t + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            const auto& A = av[t & 1];
+            const auto& B = bring[t];
+            if (t < 3 || !corner) {
+              if constexpr (X3) {
+                mma_unit(acc[0], A[0], B[0], mie_bf16()); mma_unit(sm[0], A[2], B[0], mie_bf16());
+                mma_unit(acc[0], A[1], B[0], mie_bf16()); mma_unit(sm[0], A[1], B[1], mie_bf16());
+                mma_unit(acc[0], A[0], B[1], mie_bf16()); mma_unit(sm[0], A[0], B[2], mie_bf16());
+              } else {
+                mma_unit(acc[0], A[0], B[0], mie_bf16());
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          base = base_n; step = step_n; g = gn; qi = qn;
+        }
+      }
+      if (NBUF == 1) __syncthreads();
+      if (more) stage_store((c + 1) % NBUF);
+      __syncthreads();
+    }
+  };
+  if (side == 0) contract(std::true_type());
+  else contract(std::false_type());
+
+  // ---- epilogue ----------------------------------------------------------------------------------------------------------
+  float* red = smem + wk * (64 * CO_BLK);
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int p = mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+      float s = acc[mb][r];
+      if (X3) s += sm[mb][r];
+      red[p * CO_BLK + wn * 32 + l32] = s;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int h0 = 0; h0 < PER; h0 += PB) {
+    long long off[PB];
+    int co[PB];
+    bool ok[PB], live[PB];
+    float4 r0[PB], add[PB], s[PB];
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int idx = tid + 256 * (h0 + i);
+      const int p = idx / QPP, col = 4 * (idx - p * QPP);
+      const int dy = pos_y(p), dx = pos_x(p);
+      ok[i] = dy < rows && dx < cols;
+      live[i] = ((live_bits >> (h0 + i)) & 1u) != 0;
+      off[i] = (((long long)n * hout + 2 * (y0 + dy) + py) * wout + 2 * (x0 + dx) + px) * cout + co0 + col;
+      co[i] = co0 + col;
+    }
+    conv_epilogue_load4<T, PB>(a, off, live, r0, add);
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int idx = tid + 256 * (h0 + i);
+      float4 sum = *reinterpret_cast<const float4*>(&smem[4 * idx]);
+#pragma unroll
+      for (int k2 = 1; k2 < WK; ++k2) {
+        const float4 part = *reinterpret_cast<const float4*>(&smem[k2 * (64 * CO_BLK) + 4 * idx]);
+        sum.x += part.x; sum.y += part.y; sum.z += part.z; sum.w += part.w;
+      }
+      s[i] = sum;
+    }
+    conv_epilogue_store4<T, PB>(a, off, co, ok, s, r0, add, live);
+  }
+}
+
+template <typename T, int WN>
+void launch_one(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
+  od.combos = 4 * (a.cout / (32 * WN));
+  od.total = a.ts.n * od.items * od.combos;
+  // Launch order: the (phase, slab) pairs in `groups` parts.  Every part of the filter then reaches 8 / groups of the eight
+  // L2s and the input all of them `groups` times; the split that moves the least is taken.
+  const double filt = 4.0 * 16 * a.c1 * a.cout * (sizeof(T) == 4 ? 6 : 2);
+  const double in = (double)a.ts.n * a.h_in * a.w_in * a.c1 * sizeof(T) * (a.x2 ? 2 : 1);
+  double best = 8 * filt + in;
+  od.groups = 1;
+  for (int g = 2; g <= 8 && od.combos % g == 0; g *= 2)
+    if (8 / g * filt + g * in < best) { best = 8 / g * filt + g * in; od.groups = g; }
+  hipLaunchKernelGGL((k_upconv2x<T, WN>), dim3(8 * ((od.total + 7) / 8)), dim3(256), 0, st, a, od);
+}
+
+// Slab width, by how many rounds of workgroups it takes.  A 64-column workgroup takes 1.75 times as long as a 32-column one.
+// fp32 (three-term): one workgroup fills a CU's matrix cores (two take twice as long), so a round is 256: 64 columns where they
+// need half the rounds or close to it, which leaves 32 columns up to one round (256->128 at 20x20: 26 us against 39) and in
+// the third (at 42x46, 608 of them: 68 against 78; at 33x44, 480: 48 against 45; at 60x80 134 against 122).  bf16: workgroups
+// are short and three of a CU hide each other's latencies, so 64 columns start where 32 no longer fit one round of
+// 768 (128->64 at 66x74, 656 of them: 15.7 against 17.2; at 66x88, 784: 20.4 against 17.7), 128 columns, which read the
+// input least, where they make more than a round themselves (256->128 at 8x60x80: 246 against 217; at 4x60x80, 1440: 126
+// against 116; at 3x60x80, 1080: 92 either way; at 8x30x40, 832: 76 against 83).
+template <typename T>
+void launch_up2x(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
+  const int cout = a.cout;
+  const long long wgs = (long long)a.ts.n * od.items * 4 * (cout / 32);
+  if constexpr (sizeof(T) == 4) {
+    if (cout % 64 == 0 && wgs > 256 && (wgs <= 512 || wgs > 768)) launch_one<T, 2>(a, od, st);
+    else launch_one<T, 1>(a, od, st);
+  } else {
+    if (cout % 128 == 0 && wgs / 4 >= 1024) launch_one<T, 4>(a, od, st);
+    else if (cout % 64 == 0 && wgs > 768) launch_one<T, 2>(a, od, st);
+    else launch_one<T, 1>(a, od, st);
+  }
+}
+
+template <typename T>
+int up2x_impl(const char* who, const void* x, const uint8_t* xm, const void* x2, const uint8_t* x2m, int c, int h, int w,
+              const void* filter_up, int cout, const float* bias, const mie_tileset* out, void* out_delta, const void* addend,
+              float* reservoir, int act_kind, float slope, bool refresh, void* stream) {
+  const int rc = mie_check_tileset(out, who);
+  if (rc != MIE_OK) return rc;
+  MIE_REQUIRE(x != nullptr && filter_up != nullptr && out_delta != nullptr, MIE_ERR_INVALID_ARG,
+              "%s: NULL pointer (a, filter_up and the output are required)", who);
+  MIE_REQUIRE(x2 != nullptr || x2m == nullptr, MIE_ERR_INVALID_ARG, "%s: mask of absent b", who);
+  MIE_REQUIRE(c > 0 && cout > 0 && h > 0 && w > 0, MIE_ERR_INVALID_ARG, "%s: sizes out of range (c=%d cout=%d h=%d w=%d)", who, c,
+              cout, h, w);
+  MIE_REQUIRE(c % (sizeof(T) == 4 ? 32 : 64) == 0 && cout % 32 == 0, MIE_ERR_UNSUPPORTED,
+              "%s: needs c %% %d == 0 and cout %% 32 == 0 (c=%d cout=%d)", who, sizeof(T) == 4 ? 32 : 64, c, cout);
+  MIE_REQUIRE(h >= 2 && w >= 2, MIE_ERR_UNSUPPORTED, "%s: planes of at least 2x2 pixels (%dx%d)", who, h, w);
+  MIE_REQUIRE(out->h == 2 * h && out->w == 2 * w, MIE_ERR_INVALID_ARG, "%s: the tile set is (%d,%d), twice the input is (%d,%d)", who,
+              out->h, out->w, 2 * h, 2 * w);
+  MIE_REQUIRE((long long)out->n * h * w * c * (long long)sizeof(T) < 0xffffff00LL && (long long)out->n * out->h * out->w < 0x7fffffffLL &&
+                  (long long)c * cout < (1LL << 24),
+              MIE_ERR_CAPACITY, "%s: tensor too large", who);
+  MIE_REQUIRE(mie_aligned(x, 16) && mie_aligned(x2, 16) && mie_aligned(filter_up, 16) && mie_aligned(out_delta, 16) &&
+                  mie_aligned(addend, 16) && mie_aligned(reservoir, 16) && mie_aligned(bias, 4),
+              MIE_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned (bias: 4)", who);
+  MIE_REQUIRE(act_kind >= MIE_ACT_NONE && act_kind <= MIE_ACT_TANH, MIE_ERR_UNSUPPORTED, "%s: unknown activation %d", who, act_kind);
+  MIE_REQUIRE(refresh || reservoir != nullptr || act_kind == MIE_ACT_NONE, MIE_ERR_INVALID_ARG, "%s: activation %d needs a reservoir",
+              who, act_kind);
+  MIE_REQUIRE(x != out_delta && x2 != out_delta && addend != out_delta, MIE_ERR_INVALID_ARG, "%s: inputs must not alias the output", who);
+  ConvArgsT<T> a = {};
+  a.x = (const T*)x; a.xm = xm; a.c1 = c; a.x2 = (const T*)x2; a.x2m = x2m; a.c2 = x2 ? c : 0;
+  a.h_in = h; a.w_in = w; a.cin_total = c; a.filt_mc = (const T*)filter_up; a.pad = 2; a.cout = cout;
+  a.out = (T*)out_delta; a.res = reservoir; a.act = act_kind; a.slope = slope; a.addend = (const T*)addend;
+  a.refresh = refresh ? 1 : 0; a.bias = bias;
+  a.ts = mie_dev_tileset(out);
+  Up2xOrder od = {};
+  od.flags = (const uint32_t*)out->flags;
+  od.blocks_y = (h - 2 + 7) / 8; od.blocks_x = (w - 2 + 7) / 8;
+  od.strips_x = mie_div_up(w, STRIP); od.strips_y = mie_div_up(h - 2, STRIP);
+  od.items = od.blocks_y * od.blocks_x + 2 * od.strips_x + 2 * od.strips_y;
+  od.nci = c / 16;
+  MIE_REQUIRE((long long)out->n * od.items * 4 * (cout / 32) < 0x7ffffff0LL, MIE_ERR_CAPACITY, "%s: tensor too large", who);
+  launch_up2x<T>(a, od, (hipStream_t)stream);
+  return mie_check_launch(who);
+}
+
+}  // namespace
+
+extern "C" int mie_pack_filter_up2x(const float* filter, int cin, int cout, void* packed, int dtype, void* stream) {
+  const char* who = "mie_pack_filter_up2x";
+  mie_clear_error();
+  MIE_REQUIRE(filter != nullptr && packed != nullptr && (const void*)filter != packed, MIE_ERR_INVALID_ARG,
+              "%s: filter and packed must be given and differ", who);
+  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3, MIE_ERR_UNSUPPORTED, "%s: no combined filter of dtype %d", who, dtype);
+  MIE_REQUIRE(cin > 0 && cout > 0 && cin % 16 == 0 && cout % 32 == 0 && (long long)cin * cout < (1LL << 24), MIE_ERR_UNSUPPORTED,
+              "%s: needs cin %% 16 == 0 and cout %% 32 == 0 (cin=%d cout=%d)", who, cin, cout);
+  MIE_REQUIRE(mie_aligned(filter, 4) && mie_aligned(packed, 16), MIE_ERR_INVALID_ARG, "%s: packed must be 16-byte aligned", who);
+  const dim3 grid((unsigned)((4LL * UNITS * cin * cout + 255) / 256));
+  if (dtype == MIE_DTYPE_BF16)
+    hipLaunchKernelGGL(k_pack_up2x<1>, grid, dim3(256), 0, (hipStream_t)stream, filter, (mie_bf16*)packed, cin, cout);
+  else
+    hipLaunchKernelGGL(k_pack_up2x<3>, grid, dim3(256), 0, (hipStream_t)stream, filter, (mie_bf16*)packed, cin, cout);
+  return mie_check_launch(who);
+}
+
+extern "C" int mie_upconv2x_masked(const void* a, const uint8_t* amask, const void* b, const uint8_t* bmask, int c, int h_in,
+                                   int w_in, const void* filter_up, int cout, const mie_tileset* out, void* out_delta,
+                                   const void* addend, float* reservoir, int act_kind, float slope, int dtype, void* stream) {
+  const char* who = "mie_upconv2x_masked";
+  mie_clear_error();
+  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3, MIE_ERR_UNSUPPORTED, "%s: dtype %d not implemented", who, dtype);
+  if (dtype == MIE_DTYPE_BF16)
+    return up2x_impl<mie_bf16>(who, a, amask, b, bmask, c, h_in, w_in, filter_up, cout, nullptr, out, out_delta, addend, reservoir,
+                               act_kind, slope, false, stream);
+  return up2x_impl<float>(who, a, amask, b, bmask, c, h_in, w_in, filter_up, cout, nullptr, out, out_delta, addend, reservoir,
+                          act_kind, slope, false, stream);
+}
+
+extern "C" int mie_upconv2x_refresh(const void* a, const void* b, int c, int h_in, int w_in, const void* filter_up, int cout,
+                                    const float* bias, const mie_tileset* out, void* out_dense, float* reservoir, int act_kind,
+                                    float slope, int dtype, void* stream) {
+  const char* who = "mie_upconv2x_refresh";
+  mie_clear_error();
+  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3, MIE_ERR_UNSUPPORTED, "%s: dtype %d not implemented", who, dtype);
+  if (dtype == MIE_DTYPE_BF16)
+    return up2x_impl<mie_bf16>(who, a, nullptr, b, nullptr, c, h_in, w_in, filter_up, cout, bias, out, out_dense, nullptr, reservoir,
+                               act_kind, slope, true, stream);
+  return up2x_impl<float>(who, a, nullptr, b, nullptr, c, h_in, w_in, filter_up, cout, bias, out, out_dense, nullptr, reservoir,
+                          act_kind, slope, true, stream);
+}

@@ -528,6 +528,11 @@ class UpsampleConvLayerIncr(replay.Watched, nn.Module):
         return out_incr
 
     def forward_refresh_reservoirs(self, x, skip=None):
+        if (self.fuse and self.activation is not None and self.norm not in ['BN', 'IN'] and not self.conv2d.lossy
+                and self.conv2d.path != _lib.PATH_VALU):
+            out = self.conv2d._upconv_refresh(self.upsample, x, skip, self.activation)
+            if out is not None:
+                return out
         x_upsampled = self.upsample.forward_refresh_reservoirs(x, skip)
         if self.fuse and self.activation is not None and self.norm not in ['BN', 'IN']:
             return self.conv2d.forward_refresh_fused(x_upsampled, self.activation)

@@ -330,6 +330,10 @@ class nnLinearIncr(replay.Watched, nn.Linear):
         return super().forward(x)
 
 
+def _is_gpu_delta(x) -> bool:
+    return x.is_cuda and x.dtype in (torch.float32, torch.bfloat16)
+
+
 class _ConvIncrMixin(_IncrBuffers):
     """Shared body of nnConvIncrBase / nnConvIncr."""
 
@@ -389,8 +393,32 @@ class _ConvIncrMixin(_IncrBuffers):
         ts = self._tile_set(out_name, n, 2 * h, 2 * w, a.device)
         ops.build_mask_tiles(ts_up, None, n, 2 * h, 2 * w, _lib.FOOT_CONV, k, s, p, ts)
         out = self._delta_buf(out_name, (n, self.out_channels, 2 * h, 2 * w), a.device, a.dtype)
+        if ops.upconv2x_takes(a, self.out_channels, k, s, p, self.conv2d_weights):
+            ops.upconv2x_masked(a, pa, b, pb, self.conv2d_weights, ts, out, reservoir, act, slope)
+            return [out, ts]
         ops.upconv_masked(a, pa, b, pb, self.conv2d_weights, k, p, ts, out, reservoir, act, slope)
         return [out, ts]
+
+    def _upconv_refresh(self, up: "nnUpsample2xIncr", x: DenseT, skip: DenseT, activation) -> DenseT:
+        """Dense twin of _upconv_forward where the layer runs at the resolution of its inputs; None where it does not."""
+        k, s, p = self._geometry()
+        if not _is_gpu_delta(x):
+            return None
+        x = ops.as_nhwc(x)
+        if not ops.upconv2x_takes(x, self.out_channels, k, s, p, self.conv2d_weights):
+            return None
+        up._reset_incr(), self._reset_incr(), activation._reset_incr()
+        n, _, h, w = x.shape
+        shape = (n, self.out_channels, 2 * h, 2 * w)
+        kind, slope = activation_kind(activation.op)
+        res = activation.in_res.reservoir
+        if res is None or tuple(res.shape) != shape or res.device != x.device:
+            res = activation.in_res.reservoir = ops.new_nhwc(*shape, x.device)
+        out = self._dense_buf("refresh_out", shape, x.device, x.dtype)
+        ops.upconv2x_refresh(x, None if skip is None else ops.as_nhwc(skip), self.conv2d_weights,
+                             None if self.bias is None else self.bias.detach(),
+                             self._dense_tile_set(n, 2 * h, 2 * w, x.device), out, res, kind, slope)
+        return out
 
     def _conv_tile_set(self, name, x, pix, x2, pix2, k, s, p) -> TileMask:
         """Tile set of the conv output for the (one or two) masked inputs, built for this step."""

@@ -29,7 +29,7 @@ class _PhaseLib:
     def __getattr__(self, name):
         fn = getattr(self._real, name)
         if name.startswith("mie_") and name not in ("mie_last_error_string", "mie_tile_capacity", "mie_version",
-                                                     "mie_pack_filter"):
+                                                     "mie_pack_filter", "mie_pack_filter_up2x"):
             runs = (name in _BUILD_ENTRIES) == (_phase == "plan")
             if not runs:
                 return lambda *args: 0
@@ -642,6 +642,7 @@ class ConvFilter:
         self._rows = {}
         self._bf16 = None
         self._x3 = None
+        self._up2x = {}
 
     def for_dtype(self, dtype, x3: bool = False):
         """(plain fp32 tensor, matrix-core copy | None) for deltas of `dtype`; x3: the three-term copy for fp32
@@ -657,6 +658,19 @@ class ConvFilter:
             mc = pack_filter(rounded, torch.bfloat16) if rounded.is_cuda and rounded.shape[0] % 16 == 0 else None
             self._bf16 = (rounded, mc)
         return self._bf16
+
+    def up2x(self, dtype) -> torch.Tensor:
+        """The combined filters of upconv2x_masked for deltas of `dtype` (a 5x5 filter, Cin % 16 == 0, Cout % 32 == 0), made
+        on first use from the fp32 weights."""
+        packed = self._up2x.get(dtype)
+        if packed is None:
+            cin, cout = self.plain.shape[0], self.plain.shape[3]
+            terms = 3 if dtype == torch.float32 else 1
+            packed = torch.empty((4, cin // 16, 80, terms, 2, cout, 8), dtype=torch.bfloat16, device=self.plain.device)
+            check(lib().mie_pack_filter_up2x(self.plain.contiguous().data_ptr(), cin, cout, packed.data_ptr(),
+                                             _lib.DTYPE_F32_BF16X3 if terms == 3 else _lib.DTYPE_BF16, _stream(self.plain)))
+            self._up2x[dtype] = packed
+        return packed
 
     @property
     def shape(self):
@@ -802,6 +816,71 @@ def upconv_masked(a, amask, b, bmask, filt, k, pad, out_ts: TileMask, out_delta,
         nhwc_ptr(out_delta, "out_delta", dtype=dt), nhwc_ptr(addend, "addend", cout, dtype=dt),
         nhwc_ptr(reservoir, "reservoir"), act, float(slope), code, ws_ptr, ws_bytes, _stream(a)))
     return out_delta
+
+
+# The decoder conv at the resolution of its inputs (four 4x4 convs with combined filters) for the layers it takes.
+upconv2x_enabled = os.environ.get("MIE_UPCONV2X", "1") != "0"      # tuning knob, read once
+
+
+def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt) -> bool:
+    """Whether a decoder layer over `a` runs at the resolution of its inputs: upconv2x_masked has a kernel for it and is the
+    faster form.  It is not on planes so small that upconv_masked splits the contraction (256->128 at 16x16: 25 us against
+    22, at 20x20 26 against 35), for bf16 layers of one staged chunk (64->32 at 8x240x320: 525 us against 417 in the
+    persistent kernel), and where border strips and blocks filled in part undo the fewer taps: 16 for each of the four
+    phases of an item against 25 for each tile, once that is more than a round of workgroups (256->128 at 8x19x23: 138
+    us against 123)."""
+    n, c, h, w = a.shape
+    chunk = mfma_chunk(a.dtype)
+    if not (upconv2x_enabled and isinstance(filt, ConvFilter) and filt.plain.is_cuda and k == 5 and stride == 1 and pad == 2
+            and (a.dtype == torch.bfloat16 or (a.dtype == torch.float32 and f32_matmul == "bf16x3")) and c == filt.shape[0]
+            and c % chunk == 0 and cout % 32 == 0 and h >= 2 and w >= 2 and c * cout < 1 << 24
+            and n * c * h * w * a.element_size() < 0xffffff00):
+        return False
+    tiles, slabs = _lib.tile_capacity(n, 2 * h, 2 * w), cout // 32
+    items = n * (-(-(h - 2) // 8) * -(-(w - 2) // 8) + 2 * -(-w // 32) + 2 * -(-(h - 2) // 32))
+    if (c >= 4 * chunk and tiles * slabs <= 64) or (4 * items * slabs > 256 and 4 * 16 * items > 25 * tiles):
+        return False
+    return not (a.dtype == torch.bfloat16 and c == chunk)
+
+
+def _upconv2x_args(a, b, filt, out_ts, out, reservoir, addend):
+    n, c, h, w = a.shape
+    if b is not None and (b.shape != a.shape or b.dtype != a.dtype):
+        raise ValueError("b %s %s does not match a %s %s" % (tuple(b.shape), b.dtype, tuple(a.shape), a.dtype))
+    cout = filt.shape[3]
+    if tuple(out.shape) != (n, cout, 2 * h, 2 * w) or (out_ts.n, out_ts.h, out_ts.w) != (n, 2 * h, 2 * w):
+        raise ValueError("output %s / tile set do not match twice the input %s" % (tuple(out.shape), tuple(a.shape)))
+    for name, t in (("reservoir", reservoir), ("addend", addend)):
+        if t is not None and t.shape != out.shape:
+            raise ValueError("%s shape %s != output %s" % (name, tuple(t.shape), tuple(out.shape)))
+    _ready(out_ts)
+    up = replay.keep(filt.up2x(a.dtype))
+    return n, c, h, w, cout, up.data_ptr(), _lib.DTYPE_BF16 if a.dtype == torch.bfloat16 else _lib.DTYPE_F32_BF16X3
+
+
+def upconv2x_masked(a, amask, b, bmask, filt: ConvFilter, out_ts: TileMask, out_delta, reservoir=None, act=_lib.ACT_NONE,
+                    slope=0.0, addend=None):
+    """5x5 conv (pad 2) over up2x(a + b) computed at the resolution of a and b; arguments as in upconv_masked."""
+    n, c, h, w, cout, up, code = _upconv2x_args(a, b, filt, out_ts, out_delta, reservoir, addend)
+    dt = a.dtype
+    check(lib().mie_upconv2x_masked(
+        nhwc_ptr(a, "a", dtype=dt), pix_ptr(amask, n, h, w, "amask"), nhwc_ptr(b, "b", dtype=dt), pix_ptr(bmask, n, h, w, "bmask"),
+        c, h, w, up, cout, out_ts.ref, nhwc_ptr(out_delta, "out_delta", dtype=dt), nhwc_ptr(addend, "addend", cout, dtype=dt),
+        nhwc_ptr(reservoir, "reservoir"), act, float(slope), code, _stream(a)))
+    return out_delta
+
+
+def upconv2x_refresh(a, b, filt: ConvFilter, bias, out_ts: TileMask, out_dense, reservoir=None, act=_lib.ACT_NONE, slope=0.0):
+    """Its dense twin (out_ts all active): bias, activation and reservoir fill fused."""
+    n, c, h, w, cout, up, code = _upconv2x_args(a, b, filt, out_ts, out_dense, reservoir, None)
+    dt = a.dtype
+    if bias is not None and (bias.numel() != cout or bias.dtype != torch.float32 or not bias.is_contiguous()):
+        raise ValueError("bias must be contiguous fp32 of %d elements" % cout)
+    replay.keep(bias)
+    check(lib().mie_upconv2x_refresh(
+        nhwc_ptr(a, "a", dtype=dt), nhwc_ptr(b, "b", dtype=dt), c, h, w, up, cout, None if bias is None else bias.data_ptr(),
+        out_ts.ref, nhwc_ptr(out_dense, "out_dense", dtype=dt), nhwc_ptr(reservoir, "reservoir"), act, float(slope), code, _stream(a)))
+    return out_dense
 
 
 # Planes the fused tail kernel takes (the persistent last-decoder kernel: tiles of the whole batch).
@@ -1294,9 +1373,9 @@ def conv_out_size(h, w, k, stride, pad) -> Tuple[int, int]:
 # these settings has another value
 replay.bind_ops(globals(), (
     "lib", "check", "mask_from_delta", "threshold_mask_lazy", "build_mask_tiles", "conv_masked", "upconv_masked",
-    "upconv_pred_masked", "conv_refresh", "tconv_masked", "tconv_refresh", "tconv2x_masked", "tconv2x_refresh", "act_incr",
+    "upconv_pred_masked", "upconv2x_masked", "upconv2x_refresh", "conv_refresh", "tconv_masked", "tconv_refresh", "tconv2x_masked", "tconv2x_refresh", "act_incr",
     "kfence_incr", "mul_incr", "add_incr", "maxpool_incr", "accumulate", "scale_incr", "avgpool_incr", "upsample2x_incr",
     "upsample2x_pair_incr", "convlstm_gates_incr", "convgru_gates_incr", "convlstm_gates_refresh",
     "convgru_gates_refresh", "mul_dense", "conv_gates_incr", "nhwc_ptr", "pix_ptr", "as_nhwc", "pixel_mask_of"), (
-    "f32_matmul", "split_enabled", "fused_plan", "fused_threshold_build", "upconv_max_tiles", "upconv_max_chunks",
+    "f32_matmul", "split_enabled", "fused_plan", "fused_threshold_build", "upconv2x_enabled", "upconv_max_tiles", "upconv_max_chunks",
     "upconv_pred_enabled", "UPCONV_PRED_MIN_TILES", "UPCONV_PRED_MAX_TILES", "SPLIT_WORKSPACE_BYTES"))

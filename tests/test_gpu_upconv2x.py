@@ -1,0 +1,74 @@
+"""The decoder conv at the resolution of its inputs (mie_upconv2x_masked / _refresh) against the oracle: 5x5 conv over the
+up-sampled sum.  Sizes: planes of border only, below / at / just above a block of 8 and a border strip of 32, several samples;
+borders are what the combined filters can get wrong, so every pixel is compared."""
+import pytest
+import torch
+
+from maskedincrementeval_amd import _lib, ops
+from maskedincrementeval_amd.masked_types import TileMask
+from maskedincrementeval_amd.synthetic import gaussian_delta, he_normal_conv_weight
+from oracle import incr_oracle as io
+from tolerances import BF16_RTOL, FP32_ATOL, FP32_RTOL, bf16_atol
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _dev(t, dtype=torch.float32):
+    return ops.as_nhwc(t.to(DEV).to(dtype).contiguous(memory_format=torch.channels_last))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,c,cout,h,w", [(1, 64, 32, 2, 2), (1, 64, 32, 2, 5), (2, 64, 64, 7, 2), (1, 64, 32, 3, 34), (1, 64, 64, 35, 3), (1, 64, 96, 8, 8), (1, 128, 64, 9, 16),
+                                          (1, 256, 128, 12, 20), (2, 64, 32, 33, 44), (1, 256, 128, 33, 44), (1, 128, 64, 66, 88),
+                                          (3, 64, 32, 80, 120), (1, 512, 32, 5, 3), (4, 256, 128, 60, 80)])
+def test_decoder_conv_at_input_resolution(n, c, cout, h, w, dtype):
+    bf = dtype == torch.bfloat16
+    q = (lambda t: t.to(torch.bfloat16).float()) if bf else (lambda t: t)
+    tol = (lambda ref: dict(rtol=BF16_RTOL, atol=bf16_atol(ref, 2.0))) if bf else (lambda ref: dict(rtol=FP32_RTOL, atol=FP32_ATOL))
+    wt = he_normal_conv_weight(cout, c, 5, 9)
+    filt = ops.ConvFilter(wt.permute(1, 2, 3, 0).contiguous().to(DEV))
+    assert ops.upconv2x_takes(torch.empty((n, c, h, w), dtype=dtype), cout, 5, 1, 2, filt) or c == 64 or h * w < 300
+    H, W = 2 * h, 2 * w
+    ts_up, ts = TileMask(n, H, W, DEV), TileMask(n, H, W, DEV)
+    out = ops.new_nhwc(n, cout, H, W, DEV, dtype)
+    r0 = gaussian_delta(n, cout, H, W, 1.0, 1.0, seed=3)[0]
+    res, res_ref = _dev(r0).clone(), r0.clone()
+    # dense, sparse (stale tiles), nothing at all, one input only, fused epilogue with an addend
+    for step, (da, db, two, act, add) in enumerate([(1.0, 1.0, True, _lib.ACT_NONE, False), (0.03, 0.05, True, _lib.ACT_RELU, False),
+                                                    (0.0, 0.0, True, _lib.ACT_NONE, False), (0.2, 0.0, False, _lib.ACT_LEAKY_RELU, True)]):
+        def one(d, seed):
+            if d == 0.0:
+                return torch.zeros(n, c, h, w), torch.zeros(n, 1, h, w, dtype=torch.uint8)
+            return gaussian_delta(n, c, h, w, d, 0.5, seed=seed)
+        (a, ma), (b, mb) = one(da, 100 + step), one(db, 200 + step)
+        a, b = q(a), q(b)
+        ref = io.conv_incr(io.interp_incr(a + b if two else a), wt, 1, 2)
+        dma, dmb = ma.to(DEV), mb.to(DEV)
+        ops.build_mask_tiles(dma, dmb if two else None, n, h, w, _lib.FOOT_UP2X, 0, 0, 0, ts_up)
+        ops.build_mask_tiles(ts_up, None, n, H, W, _lib.FOOT_CONV, 5, 1, 2, ts)
+        extra = q(gaussian_delta(n, cout, H, W, 1.0, 0.3, seed=7)[0] * ts.pixmask.cpu().float()) if add else None
+        poison = lambda t, m: torch.where(m.bool().expand_as(t), t, torch.full_like(t, float("nan")))
+        ops.upconv2x_masked(_dev(poison(a, ma), dtype), dma, _dev(poison(b, mb), dtype) if two else None, dmb if two else None, filt, ts,
+                            out, None if act == _lib.ACT_NONE else res, act, 0.1, addend=None if extra is None else _dev(extra, dtype))
+        got = out.float().cpu()
+        z = ref if extra is None else ref + extra
+        if act == _lib.ACT_NONE:
+            want = z
+        else:
+            op = torch.relu if act == _lib.ACT_RELU else (lambda t: torch.nn.functional.leaky_relu(t, 0.1))
+            want = op(res_ref + z) - op(res_ref)
+            res_ref = res_ref + z
+            assert torch.allclose(res.cpu(), res_ref, rtol=FP32_RTOL, atol=bf16_atol(ref, 2.0) if bf else FP32_ATOL)
+        assert torch.isfinite(got).all()
+        assert torch.allclose(got, want, **tol(want)), "step %d max|diff| %.3e of %.3e" % (step, (got - want).abs().max(), want.abs().max())
+        assert torch.count_nonzero(got * (1 - ts.pixmask.cpu().float())) == 0
+    # the dense twin
+    full, dense = TileMask(n, H, W, DEV), ops.new_nhwc(n, cout, H, W, DEV, dtype)
+    ops.build_mask_tiles(None, None, n, H, W, _lib.FOOT_CONV, 1, 1, 0, full)
+    a, b = q(gaussian_delta(n, c, h, w, 1.0, 0.5, seed=11)[0]), q(gaussian_delta(n, c, h, w, 1.0, 0.5, seed=12)[0])
+    bias = torch.linspace(-1, 1, cout)
+    ops.upconv2x_refresh(_dev(a, dtype), _dev(b, dtype), filt, bias.to(DEV), full, dense, res, _lib.ACT_RELU)
+    pre = io.conv_incr(io.interp_incr(a + b), wt, 1, 2) + bias.view(1, -1, 1, 1)
+    assert torch.allclose(res.cpu(), pre, rtol=FP32_RTOL, atol=bf16_atol(pre, 2.0) if bf else 2 * FP32_ATOL)
+    assert torch.allclose(dense.float().cpu(), torch.relu(pre), **tol(pre))
