@@ -337,7 +337,7 @@ def drop_lookahead(net):
 
 
 def _stream(t: torch.Tensor):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 # ---- mask planning on a side stream -------------------------------------------------------------
