@@ -1102,18 +1102,18 @@ void launch_split_finish(const ConvArgsT<T>& a, unsigned cap, int parts, hipStre
 
 template <typename T, int K, int S>
 bool launch_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
-  constexpr int CC = stage_channels(K, S, false) * (4 / (int)sizeof(T));
+  constexpr bool HAS_X3 = sizeof(T) == 4 && (K == 5 || (K == 3 && S == 1));
+  const bool x3 = HAS_X3 && a0.x3 != 0;
+  const int CC = x3 && S == 2 ? 16 : stage_channels(K, S, false) * (4 / (int)sizeof(T));
   if (a0.ws == nullptr || a0.refresh || a0.cout % 32 != 0 || a0.c1 % CC != 0 || a0.c2 % CC != 0) return false;
   ConvArgsT<T> a = a0;
   const int parts = split_parts(a, (long long)cap * (a0.cout / 32), (a0.c1 + a0.c2) / CC);
   if (parts == 0) return false;
-  bool x3 = false;
-  if constexpr (sizeof(T) == 4 && S == 1 && (K == 3 || K == 5)) x3 = a.x3 != 0;
+  const dim3 grid(cap, a.cout / 32, parts);
   if (x3) {
-    if constexpr (sizeof(T) == 4 && S == 1 && (K == 3 || K == 5))
-      hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true, true>), dim3(cap, a.cout / 32, parts), dim3(256), 0, st, a);
+    if constexpr (HAS_X3) hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true, true>), grid, dim3(256), 0, st, a);
   } else {
-    hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true>), dim3(cap, a.cout / 32, parts), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true>), grid, dim3(256), 0, st, a);
   }
   launch_split_finish(a, cap, parts, st);
   return true;
@@ -1379,7 +1379,9 @@ bool launch_any(const ConvArgsT<T>& a, int k, int s, unsigned cap, hipStream_t s
     if (a.x3) {
       if (k == 3 && s == 1) return launch_split<T, 3, 1>(a, cap, st) || launch_x3<3, false, false>(a, cap, st);
       if (k == 5 && s == 1) return launch_split<T, 5, 1>(a, cap, st) || launch_x3<5, false, false>(a, cap, st);
-      if (k == 5 && s == 2) return launch_x3<5, false, false, 2>(a, cap, st);     // (no split form at stride 2)
+      // (5x5 stride 2 on planes of few tiles, the fp32 instruction's split form -> this: 64->128 at 32x48 20.8 -> 12.1 us,
+      // 128->256 at 16x24 16.5 -> 13.1, at 32x32 16.8 -> 14.0; 32->64 at 64x96, two chunks and not split, 14.7 -> 12.3)
+      if (k == 5 && s == 2) return launch_split<T, 5, 2>(a, cap, st) || launch_x3<5, false, false, 2>(a, cap, st);
       return false;
     }
   }

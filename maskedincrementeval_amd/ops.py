@@ -751,11 +751,9 @@ def conv_masked(x, xmask, x2, x2mask, filt, k, stride, pad, out_ts: TileMask, ou
     if x2 is not None and (x2.shape[0] != n or x2.shape[2:] != x.shape[2:]):
         raise ValueError("x2 shape %s incompatible with x %s" % (tuple(x2.shape), tuple(x.shape)))
     dt = x.dtype
-    # launches the library would split over the contraction (k = 3 or 5, few tiles: see launch_split); at stride 2
-    # only the fp32-instruction kernels have that form, and it is worth more there than the three-term arithmetic
+    # launches the library would split over the contraction (k = 3 or 5, few tiles: see launch_split)
     small = k in (3, 5) and out_ts.capacity * (filt.shape[3] // 32) <= 128
-    want_split = small and split_enabled and workspace is not False
-    x3_shape = (stride, c1, c2, filt.shape[3]) if (path != _lib.PATH_VALU and not (stride == 2 and want_split)) else None
+    x3_shape = (stride, c1, c2, filt.shape[3]) if path != _lib.PATH_VALU else None
     filt, mc_ptr, code = _filter_args(filt, k, dt, x3_shape, with_code=True)
     cin_total, cout = filt.shape[0], filt.shape[3]
     if tuple(out_delta.shape) != (n, cout, out_ts.h, out_ts.w) or out_ts.n != n:
