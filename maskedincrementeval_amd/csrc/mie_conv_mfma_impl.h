@@ -717,6 +717,48 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
             ub + ((long long)(((qi * (K * K) + tap) * PL + q) * 2) * cout + nb * 32) * EPS + b_lane);
   };
 
+  // Three-term kernels with two buffers weave the staging of the next chunk into the MFMAs: a slot's split into terms (50
+  // VALU instructions) and its LDS writes go between the MFMAs of a unit, one slot to a unit, then the loads of the chunk
+  // after the next and its addresses between those of one more, all without a branch (a slot that does not exist is written
+  // behind row 0), and the barrier sits between the last two units as in PIPE.  An MFMA takes 32 cycles, of which a wave's
+  // own VALU instructions can use 28: measured, five of them between any two MFMAs cost nothing.  The slots of the next
+  // chunk are loaded a whole chunk before they are stored, and in the prologue in front of the first B loads, because the
+  // load counter is in order and takes the least of all paths: waiting for them must not mean waiting for the B loads
+  // behind them.  (3x3 256->256: a chunk 1.55 -> 1.2 us in a launch of 16 workgroups, 18.3 -> 16.2 us together; at 33x44,
+  // 240 workgroups, 20.0 -> 18.6; 512->512 at 8x12, unsplit, 30.7 -> 25.8.  On the full chip the matrix cores are held to
+  // 1.6 .. 2.0 GHz by their power, and a launch that wastes less time runs at a lower clock.)
+  constexpr bool WOVEN = X3 && NBUF == 2 && !UP && UPC >= NLD + 3;
+  constexpr int TRASH = IT * LS;                             // behind the pixels of row 0: where slots that do not exist go
+  static_assert(!WOVEN || RP - IT * LS >= EPS, "room for a slot in the row padding");
+  int st_at[NLD];
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) st_at[i] = tid + 256 * i < NSLOT ? st_lds[i] : TRASH;
+  unsigned ok_n = 0u;                                        // which slots of the chunk in st_reg count
+  auto load_raw = [&](int c, bool first = false) {
+    const bool second = c >= nch1;
+    const T* xin = second ? a.x2 : a.x;
+    const int cs = second ? a.c2 : a.c1;
+    const int ci0 = (second ? c - nch1 : c) * CC;
+    const T* dummy = a.filt_mc;
+    ok_n = second ? ok2 : ok1;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const T* p = xin + (long long)st_po[i] * cs + ci0 + st_c4[i];
+      p = (((first ? inb : ok_n) >> i) & 1u) ? p : dummy;
+#pragma unroll
+      for (int g = 0; g < GPS; ++g) st_reg[i][g] = *reinterpret_cast<const float4*>(p + 4 * g);
+    }
+  };
+  auto store_one = [&](int i, TL* dst) {
+    const bool k = (ok_n >> i) & 1u;
+    const float4 u = st_reg[i][0], v = st_reg[i][GPS - 1];
+    const float f[8] = {k ? u.x : 0.f, k ? u.y : 0.f, k ? u.z : 0.f, k ? u.w : 0.f, k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f};
+    float4 pl[3];
+    split3(f, pl);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<float4*>(dst + st_at[i] + q * STAGE) = pl[q];
+  };
+  float4 st_first[WOVEN ? NLD : 1][GPS];
   // All B loads below are unconditional: a conditional load would make the compiler's wait
   // counters conservative and collapse the prefetch distance.  After the last chunk the
   // "next chunk" pointer simply stays on the current one (a few redundant loads).
@@ -728,7 +770,9 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   const TL* ub_next = ub_cur;
   MIE_STAMP(2);
   const bool early = c_hi - c_lo >= 4;      // uniform over the workgroup
-  if (early) stage_load(c_lo, true);
+  if constexpr (WOVEN) {
+    if (early) load_slots(st_first, c_lo, true);
+  } else if (early) stage_load(c_lo, true);
   // the pixel-mask bytes, behind the first chunk's loads (pixel 0 stands in for slots outside the image, so that
   // these loads are unconditional too)
   {
@@ -753,7 +797,10 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       }
     }
   }
-  if (!early) stage_load(c_lo);
+  if constexpr (WOVEN) {
+    if (!early) load_slots(st_first, c_lo, false);
+    load_raw(c_lo + 1 < c_hi ? c_lo + 1 : c_lo, early);
+  } else if (!early) stage_load(c_lo);
 #pragma unroll
   for (int i = 0; i < (PD > 0 ? PD : 1); ++i) load_b(ub_cur, i, bring[i % RING]);
   // zero what the first chunk's loads fetched of masked pixels
@@ -772,9 +819,13 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     for (int i = 0; i < NLD; ++i)
 #pragma unroll
       for (int g = 0; g < GPS; ++g)
-        if (!((ok >> i) & 1u)) st_reg[i][g] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (!((ok >> i) & 1u)) {
+          if constexpr (WOVEN) st_first[i][g] = make_float4(0.f, 0.f, 0.f, 0.f);
+          else st_reg[i][g] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
   }
-  stage_store(0);
+  if constexpr (WOVEN) store_slots(st_first, 0);
+  else stage_store(0);
   __syncthreads();
   MIE_STAMP(3);
 
@@ -794,7 +845,8 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   };
   // the MFMAs of one unit position
   auto mma = [&](int unit, const float4 (&av)[2][PL], const float4 (&bv)[NB][PL]) {
-    if (TPAR && (unit * TP >= K * K || unit_tap(unit) >= K * K)) return;     // uniform over the wave
+    if (TPAR && unit * TP >= K * K) return;
+    if (TPAR && unit * TP + TP > K * K && unit_tap(unit) >= K * K) return;     // uniform over the wave
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       if constexpr (X3) mma_unit2_x3(acc[0][nb], acc[1][nb], accs[0][nb], accs[1][nb], av[0], av[1], bv[nb]);
@@ -814,7 +866,55 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // Measured on MI355X this ordering is worth under 1 % against "loads at the top of the chunk, stores and
   // barrier at its end": what a chunk loses against its MFMA time is not the hand-over (see the header).
   constexpr bool PIPE = MIE_PIPE && NBUF == 2 && !UP && UPC >= 8;
-  if constexpr (PIPE) {
+  if constexpr (WOVEN) {
+    float4 av[2][2][PL], av0[2][PL];
+    const TL* sin = sbuf;
+    TL* snext = sbuf + PL * STAGE;
+    load_a(sin, 0, av0);
+    for (int c = c_lo; c < c_hi; ++c) {
+#pragma unroll
+      for (int i = 0; i < UPC; ++i) {
+        const int ip = i + PD;
+        if (ip < UPC) load_b(ub_cur, ip, bring[ip % RING]);
+        else load_b(ub_next, ip - UPC, bring[ip % RING]);
+        if (i + 1 < UPC) load_a(sin, i + 1, av[(i + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (i == 0) mma(0, av0, bring[0]);
+        else mma(i, av[i & 1], bring[i % RING]);
+        if (i == 0) {
+          int cn = __builtin_amdgcn_readfirstlane(c + 1 < c_hi ? c + 1 : c);
+          asm volatile("" : "+s"(cn));
+          ub_next = chunk_b(cn);
+        }
+        if (i < NLD) {
+          store_one(i, snext);
+        } else if (i == NLD) {
+          int cn = __builtin_amdgcn_readfirstlane(c + 2 < c_hi ? c + 2 : c_hi - 1);
+          asm volatile("" : "+s"(cn));
+          load_raw(cn);
+        }
+        if (i <= NLD) {
+#pragma unroll
+          for (int j = 0; j < 12 * NB; ++j) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+            __builtin_amdgcn_sched_group_barrier(0x4, 3, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (i == UPC - 2) {
+          __syncthreads();
+          load_a(snext, 0, av0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      ub_cur = ub_next;
+      TL* const t = const_cast<TL*>(sin);
+      sin = snext;
+      snext = t;
+      MIE_STAMP(4 + (c - c_lo));
+    }
+  } else if constexpr (PIPE) {
     float4 av[2][2][PL], av0[2][PL];
     load_a(sbuf, 0, av0);
     for (int c = c_lo; c < c_hi; ++c) {
