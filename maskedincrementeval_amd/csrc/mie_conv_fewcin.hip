@@ -159,9 +159,276 @@ __global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
   conv_epilogue_store4<T, 2>(a, off, co, ok, v, r0, add, live);
 }
 
+// The same layers with bf16 deltas on planes of many tiles.  The kernel above pays for every tile what only the launch
+// needs: 25 kB of filter through registers into LDS, operands widened and read a word at a time, and the fp32 instruction
+// at a quarter of the bf16 one's rate for values that have eight bits.  Here
+//   * every weight is three bf16 terms whose sum is the fp32 weight (by truncation: exact, and no term overflows), so
+//     three v_mfma_f32_32x32x16_bf16 multiply what 16 of the deltas need, each product exact in fp32 as before;
+//   * a unit is two taps x 8 channels, so that an operand is 16 bytes of LDS: [pixel][8 channels] of the deltas and
+//     [unit][term][half][column][8 channels] of the filter, both read without bank conflicts;
+//   * the filter is split and staged once per workgroup, two workgroups of eight waves stay on a CU, and a wave walks
+//     the tile list by itself: it stages its tile, multiplies all 64 pixels (each filter operand serves two MFMAs) and
+//     writes them, with no barrier after the filter's.  Its reservoir loads are in flight during the MFMAs.
+// What is left is the traffic of the reservoir and the deltas (8x480x640, 5 -> 32 channels, 20 % of the pixels: 545 MB).
+// A delta that is not finite would make NaN of a zero among a weight's small terms: a wave that staged one multiplies the
+// finite ones first and then the others by the large terms alone, which decide what comes out.
+typedef __bf16 fc_bf16x8 __attribute__((ext_vector_type(8)));
+constexpr int FH_WAVES = 8;
+constexpr unsigned FH_GRID = 512;                 // two workgroups per CU
+
+// Between what lanes of one wave write to LDS and what others of it read: LDS requests of a wave are served in order, so
+// only the compiler has to keep it.
+__device__ __forceinline__ void fh_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ unsigned fh_finite(unsigned v) {            // two bf16 values, zero where not finite
+  const unsigned lo = (v & 0x7f80u) == 0x7f80u ? 0u : v & 0xffffu, hi = (v & 0x7f800000u) == 0x7f800000u ? 0u : v & 0xffff0000u;
+  return lo | hi;
+}
+
+__global__ __launch_bounds__(64 * FH_WAVES, 4) void k_conv_fewcin_bf16(ConvArgsT<mie_bf16> a) {
+  constexpr int K = 5, S = 1;
+  constexpr int IT = 7 * S + K, NPIX = IT * IT, KK = K * K, UN = (KK + 1) / 2;
+  constexpr int REGION = (NPIX + 1) * 16 > 4096 ? (NPIX + 1) * 16 : 4096;    // of a wave: its tile and a zero pixel; 32 rows of results
+  constexpr int NIN = (NPIX + 1 + 63) / 64;
+  __shared__ uint4 s_w[UN * 3 * 64];
+  __shared__ uint4 s_reg[FH_WAVES * REGION / 16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cout = a.cout, cin = a.c1, co0 = blockIdx.y * 32;
+  const int cap = a.ts.n * a.ts.tiles_y * a.ts.tiles_x;
+  const int n_active = a.ts.counts[MIE_CNT_ACTIVE], n_stale = a.ts.counts[MIE_CNT_STALE];
+  const int step = (int)gridDim.x * FH_WAVES;
+  int b = (int)blockIdx.x * FH_WAVES + wave;
+  int spec = a.ts.tiles[b < cap ? b : 0];
+
+#pragma unroll
+  for (int i = 0; i < (UN * 64 + 64 * FH_WAVES - 1) / (64 * FH_WAVES); ++i) {
+    const int idx = tid + 64 * FH_WAVES * i;
+    if (idx >= UN * 64) break;
+    const int tap = idx >> 5, col = idx & 31;
+    const float* wp = a.filt + (long long)tap * cout + co0 + col;
+    float w[8];
+#pragma unroll
+    for (int ch = 0; ch < 8; ++ch) w[ch] = (tap < KK && ch < cin) ? wp[(long long)ch * KK * cout] : 0.f;
+    unsigned t[3][4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      unsigned h[2][3];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float f = w[2 * p + e];
+        const unsigned u = __builtin_bit_cast(unsigned, f);
+        const bool finite = (u & 0x7f800000u) != 0x7f800000u;
+        // (a NaN whose payload lies in the lower half stays one)
+        const unsigned u0 = (u & 0xffff0000u) | (!finite && (u & 0x7fffffu) != 0u ? 0x400000u : 0u);
+        const float r1 = f - __builtin_bit_cast(float, u0);
+        const unsigned u1 = __builtin_bit_cast(unsigned, r1) & 0xffff0000u;
+        const float r2 = r1 - __builtin_bit_cast(float, u1);
+        h[e][0] = u0 >> 16;
+        h[e][1] = finite ? u1 >> 16 : 0u;
+        h[e][2] = finite ? __builtin_bit_cast(unsigned, r2) >> 16 : 0u;
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) t[q][p] = h[0][q] | (h[1][q] << 16);
+    }
+    uint4* dst = s_w + (tap >> 1) * 192 + (tap & 1) * 32 + col;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) dst[q * 64] = make_uint4(t[q][0], t[q][1], t[q][2], t[q][3]);
+  }
+  __syncthreads();
+
+  uint4* const s_in = s_reg + wave * (REGION / 16);
+  float* const s_out = reinterpret_cast<float*>(s_in);
+  const unsigned short* const x = reinterpret_cast<const unsigned short*>(a.x);
+  const int hout = a.ts.h, wout = a.ts.w;
+  const int l32 = lane & 31, half = lane >> 5;
+  // The ordinary epilogue -- reservoir, an activation of two straight pieces -- is branch-free and its reservoir is
+  // fetched ahead; any other takes the general code, a group of channels at a time.  (With the general code unrolled in
+  // its place the kernel had 8000 instructions, its branches on the activation among them.)
+  const bool relu = a.act == MIE_ACT_RELU;
+  const bool fast = a.res != nullptr && !a.refresh && (relu || a.act == MIE_ACT_NONE || a.act == MIE_ACT_LEAKY_RELU);
+  const float slope = a.act == MIE_ACT_LEAKY_RELU ? a.slope : 1.f;
+  const auto act = [&](float f) { return f > 0.f ? f : (relu ? 0.f : __fmul_rn(f, slope)); };
+  int py[NIN], px[NIN];                          // pixels of the staged tile this lane loads
+#pragma unroll
+  for (int i = 0; i < NIN; ++i) { py[i] = (lane + 64 * i) / IT; px[i] = (lane + 64 * i) - py[i] * IT; }
+  const int end = n_active + n_stale < cap ? n_active + n_stale : cap;
+  for (; b < end; b += step) {
+    int n, y0, x0;
+    const int tk = mie_pick_tile_loaded(a.ts, b, __builtin_amdgcn_readfirstlane(spec), n_active, n_stale, n, y0, x0);
+    spec = a.ts.tiles[b + step < cap ? b + step : 0];
+    if (tk == 0) continue;
+    // results of a lane: tile rows g = 0..7, column lane >> 3, four channels
+    const int ox = x0 + (lane >> 3), col = 4 * (lane & 7);
+    const long long obase = ((long long)n * hout + y0) * wout + ox;
+    const unsigned short* const xn = x + (long long)n * a.h_in * a.w_in * cin;      // (offsets in a sample fit 32 bits)
+    const uint8_t* const xmn = a.xm == nullptr ? nullptr : a.xm + (long long)n * a.h_in * a.w_in;
+    if (tk == 2) {
+#pragma unroll
+      for (int g = 0; g < 8; ++g)
+        if (y0 + g < hout && ox < wout)
+          mie_st4(a.out, (obase + (long long)g * wout) * cout + co0 + col, make_float4(0.f, 0.f, 0.f, 0.f));
+      continue;
+    }
+    uint8_t pm[8];
+#pragma unroll
+    for (int g = 0; g < 8; ++g) pm[g] = a.refresh ? (uint8_t)1 : a.ts.pixmask[y0 + g < hout && ox < wout ? obase + (long long)g * wout : 0];
+    // ---- stage the tile: a lane takes whole pixels; pixels outside the image or the input mask are loaded from a place
+    // that exists and cleared, so that all loads of the lane are in flight together
+    const int iy0 = y0 * S - a.pad, ix0 = x0 * S - a.pad;
+    unsigned short v[NIN][8];
+    bool use[NIN];
+#pragma unroll
+    for (int i = 0; i < NIN; ++i) {
+      const int pix = lane + 64 * i;
+      const int iy = iy0 + py[i], ix = ix0 + px[i];
+      use[i] = pix < NPIX && iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in;
+      const unsigned po = use[i] ? (unsigned)(iy * a.w_in + ix) : 0u;
+      if (xmn != nullptr) use[i] = use[i] && xmn[po] != 0;
+      const unsigned xo = po * (unsigned)cin;
+#pragma unroll
+      for (int ch = 0; ch < 8; ++ch) v[i][ch] = ch < cin ? xn[xo + ch] : (unsigned short)0;
+    }
+    unsigned odd = 0u;                           // a sign bit is set once an exponent was all ones
+#pragma unroll
+    for (int i = 0; i < NIN; ++i) {
+      const int pix = lane + 64 * i;
+      unsigned u[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        u[p] = use[i] ? (unsigned)v[i][2 * p] | ((unsigned)v[i][2 * p + 1] << 16) : 0u;
+        odd |= (u[p] & 0x7f807f80u) + 0x00800080u;
+      }
+      if (pix <= NPIX) s_in[pix] = make_uint4(u[0], u[1], u[2], u[3]);       // (pixel NPIX: the zero pixel)
+    }
+    unsigned live = 0u;                          // of the rows, which are inside the plane and its pixel mask
+#pragma unroll
+    for (int g = 0; g < 8; ++g) live |= pm[g] != 0 && y0 + g < hout && ox < wout ? 1u << g : 0u;
+    float4 r0[8];
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      r0[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (fast && ((live >> g) & 1u)) r0[g] = mie_ld4(a.res, (obase + (long long)g * wout) * cout + co0 + col);
+    }
+    fh_order();
+
+    // ---- contraction: 8 rows of 8 pixels as two blocks of 32
+    v16f acc[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
+    int p0 = (l32 >> 3) * S * IT + (l32 & 7) * S, hs = half;
+    asm volatile("" : "+v"(p0), "+v"(hs));       // (or the addresses of every unit are kept across tiles, and spilled)
+    const bool any_odd = __any((odd & 0x80008000u) != 0u);
+    if (any_odd) {                               // the contraction sees the finite values only ...
+#pragma unroll 1
+      for (int pix = lane; pix < NPIX; pix += 64) {
+        const uint4 u = s_in[pix];
+        s_in[pix] = make_uint4(fh_finite(u.x), fh_finite(u.y), fh_finite(u.z), fh_finite(u.w));
+      }
+      fh_order();
+    }
+    const auto mul = [](v16f& c, const uint4& d, const uint4& w) {
+      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fc_bf16x8, d), __builtin_bit_cast(fc_bf16x8, w), c, 0, 0, 0);
+    };
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int t0 = 2 * u, t1 = 2 * u + 1;
+      const int o0 = (t0 / K) * IT + t0 % K, o1 = t1 < KK ? (t1 / K) * IT + t1 % K : 0;
+      int pa = p0 + (hs ? o1 : o0), pb = pa + 4 * S * IT;
+      if (t1 >= KK && hs) pa = pb = NPIX;
+      const uint4 d0 = s_in[pa], d1 = s_in[pb];
+      const uint4* wp = s_w + u * 192 + lane;
+      const uint4 w0 = wp[0], w1 = wp[64], w2 = wp[128];
+      mul(acc[0], d0, w2); mul(acc[1], d1, w2);
+      mul(acc[0], d0, w1); mul(acc[1], d1, w1);
+      mul(acc[0], d0, w0); mul(acc[1], d1, w0);
+      __builtin_amdgcn_sched_barrier(0);         // (operands of several units ahead would not fit the registers)
+    }
+    if (any_odd) {                               // ... and the others follow with the large terms
+      fh_order();
+#pragma unroll 1
+      for (int pix = lane; pix < NPIX; pix += 64) {
+        const int iy = iy0 + pix / IT, ix = ix0 + pix % IT;
+        const bool in = iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in;
+        const unsigned po = in ? (unsigned)(iy * a.w_in + ix) : 0u;
+        const bool take = in && (xmn == nullptr || xmn[po] != 0);
+        unsigned short* dst = reinterpret_cast<unsigned short*>(s_in + pix);
+#pragma unroll 1
+        for (int ch = 0; ch < 8; ++ch) {
+          const unsigned short f = take && ch < cin ? xn[po * (unsigned)cin + ch] : (unsigned short)0;
+          dst[ch] = (f & 0x7f80) == 0x7f80 ? f : (unsigned short)0;
+        }
+      }
+      fh_order();
+#pragma unroll 1
+      for (int u = 0; u < UN; ++u) {
+        const int t = 2 * u + half;
+        const int pa = t < KK ? p0 + (t / K) * IT + t % K : NPIX, pb = t < KK ? pa + 4 * S * IT : NPIX;
+        const uint4 d0 = s_in[pa], d1 = s_in[pb], w0 = s_w[u * 192 + lane];
+        mul(acc[0], d0, w0); mul(acc[1], d1, w0);
+      }
+    }
+
+    // ---- epilogue: through LDS (over the staged tile, which is done with) to 16-byte groups of channels
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+      fh_order();
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s_out[(8 * (r >> 2) + 4 * half + (r & 3)) * 32 + l32] = acc[mb][r];
+      fh_order();
+      if (fast) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int g = 4 * mb + i;
+          const long long off = (obase + (long long)g * wout) * cout + co0 + col;
+          const float4 s4 = *reinterpret_cast<const float4*>(s_out + 4 * (lane + 64 * i));
+          const float4 q = r0[g], r1 = make_float4(q.x + s4.x, q.y + s4.y, q.z + s4.z, q.w + s4.w);
+          const bool l = (live >> g) & 1u;
+          if (l) mie_st4(a.res, off, r1);
+          if (y0 + g < hout && ox < wout)
+            mie_st4(a.out, off, make_float4(l ? act(r1.x) - act(q.x) : 0.f, l ? act(r1.y) - act(q.y) : 0.f,
+                                            l ? act(r1.z) - act(q.z) : 0.f, l ? act(r1.w) - act(q.w) : 0.f));
+        }
+      } else {
+#pragma unroll 1
+        for (int i = 0; i < 4; ++i) {
+          const int g = 4 * mb + i;
+          const long long off[1] = {(obase + (long long)g * wout) * cout + co0 + col};
+          const int co[1] = {co0 + col};
+          const bool ok[1] = {y0 + g < hout && ox < wout}, l[1] = {((live >> g) & 1u) != 0u};
+          const float4 s4[1] = {*reinterpret_cast<const float4*>(s_out + 4 * (lane + 64 * i))};
+          float4 r[1], add[1];
+          conv_epilogue_load4<mie_bf16, 1>(a, off, l, r, add);
+          conv_epilogue_store4<mie_bf16, 1>(a, off, co, ok, s4, r, add, l);
+        }
+      }
+    }
+    fh_order();
+  }
+}
+
+// 5x5, stride 1, from 2048 tiles on.  Below, a wave that does a whole tile by itself takes longer than four that share it
+// (5 -> 32 channels with a reservoir, graph of 20 calls, one workgroup a tile -> this: 1452 tiles, 409 active, 10.2 -> 12.8
+// us; 1750, 829 active, 14.0 -> 13.4; 2904, 1964 active, 25.4 -> 15.8; 38400, 3190 active, 39.7 -> 22.3, 26543 active, 256
+// -> 122, which is 4.5 TB/s).  3x3 stride 2 has so few products that the form above stays ahead at every size in use (4 ->
+// 64, 2400 tiles, 1026 active: 16.4 us against 19.6).
+constexpr unsigned FH_MIN_TILES = 2048;
+
+bool launch_fewcin_many(const ConvArgsT<float>&, int, int, unsigned, hipStream_t) { return false; }
+bool launch_fewcin_many(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st) {
+  if (k != 5 || s != 1 || cap < FH_MIN_TILES || a.addend != nullptr || (long long)a.h_in * a.w_in >= 1 << 27) return false;
+  const unsigned wgs = (cap + FH_WAVES - 1) / FH_WAVES;
+  hipLaunchKernelGGL(k_conv_fewcin_bf16, dim3(wgs < FH_GRID ? wgs : FH_GRID, a.cout / 32), dim3(64 * FH_WAVES), 0, st, a);
+  return true;
+}
+
 template <typename T>
 bool launch_fewcin(const ConvArgsT<T>& a, int k, int s, unsigned cap, hipStream_t st) {
   if (a.x2 != nullptr || a.c1 < 1 || a.c1 > FC_CH || a.cout % 32 != 0) return false;
+  if (launch_fewcin_many(a, k, s, cap, st)) return true;
   const dim3 grid(cap, a.cout / 32), block(256);
   switch (k * 10 + s) {
     case 31: hipLaunchKernelGGL((k_conv_fewcin<T, 3, 1>), grid, block, 0, st, a); return true;

@@ -623,6 +623,56 @@ def test_few_input_channels_matrix_core_kernel(cin, cout, k, s, dtype):
     assert torch.allclose(res.cpu(), res_ref, rtol=RTOL, atol=bf16_atol(ref, 2.0) if bf else ATOL)
 
 
+# bf16 5x5 layers of few input channels on planes of at least 2048 tiles: a batch of three ragged frames (2808 tiles) against
+# the same frames one by one (936 tiles each, one workgroup a tile), over three steps (stale tiles, an empty step) and a
+# refresh.  Both add exact products in fp32, so a sum of K = 25 Cin terms differs by at most 2 K 2^-24 of the terms' sizes.
+# An infinite delta (step 1) must leave the same Inf and NaN in both, weights with zeros among their small terms included.
+@pytest.mark.parametrize("cin,cout,act", [(1, 32, _lib.ACT_RELU), (5, 32, _lib.ACT_LEAKY_RELU), (8, 64, _lib.ACT_NONE), (5, 32, _lib.ACT_TANH), (3, 32, None)])
+def test_few_input_channels_of_many_tiles(cin, cout, act):
+    bf, n, h, w = torch.bfloat16, 3, 203, 283
+    assert 2048 > _lib.tile_capacity(1, h, w) and _lib.tile_capacity(n, h, w) >= 2048
+    wt = he_normal_conv_weight(cout, cin, 5, 3)
+    wt[0, 0] = 0.5
+    filt, absf = _filt(wt), wt.abs()
+    res0 = _dev(gaussian_delta(n, cout, h, w, 1.0, 1.0, seed=8)[0])
+    big = dict(ts=TileMask(n, h, w, DEV), out=ops.new_nhwc(n, cout, h, w, DEV, bf), res=res0.clone())
+    one = [dict(ts=TileMask(1, h, w, DEV), out=ops.new_nhwc(1, cout, h, w, DEV, bf), res=_dev(res0[i:i + 1]).clone()) for i in range(n)]
+    rbound = torch.zeros(())
+    for step, dens in enumerate([0.3, 0.05, 0.0]):
+        d, m = gaussian_delta(n, cin, h, w, dens, 0.5, seed=70 + step)
+        if step == 1:
+            y, x = m[1, 0].nonzero()[7].tolist()
+            d[1, 0, y, x] = float("inf")
+        d = d.to(bf)
+        bound = 2 * 25 * cin * 2.0 ** -24 * torch.nn.functional.conv2d(d.float().nan_to_num(0, 0, 0).abs(), absf, padding=2)
+        rbound = rbound + bound                                 # a reservoir carries what its steps differed by ...
+        for o, lo, hi in [(big, 0, n)] + [(one[i], i, i + 1) for i in range(n)]:
+            dm = m[lo:hi].contiguous().to(DEV)
+            ops.build_mask_tiles(dm, None, hi - lo, h, w, _lib.FOOT_CONV, 5, 1, 2, o["ts"])
+            xin = torch.where(m[lo:hi].bool().expand(-1, cin, -1, -1), d[lo:hi], torch.full_like(d[lo:hi], float("nan")))
+            ops.conv_masked(_dev(xin), dm, None, None, filt, 5, 1, 2, o["ts"], o["out"], None if act is None else o["res"],
+                            _lib.ACT_NONE if act is None else act, 0.1, _lib.PATH_AUTO)
+        torch.cuda.synchronize()
+        for key in ("res", "out"):
+            got, want = big[key].float().cpu(), torch.cat([o[key] for o in one]).float().cpu()
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf()), (step, key)
+            assert step == 0 or act is None or key == "out" or got.isinf().any()
+            f = torch.isfinite(want)
+            if key == "res":
+                rbound = rbound + torch.where(f, 2.0 ** -23 * want.abs(), 0.0)     # ... and a rounding of the sum, half an ulp a side
+                slack = rbound
+            else:                                               # the difference of two activations, rounded to bf16
+                slack = 2 * rbound + 2.0 ** -7 * want.abs()
+            assert ((got - want).abs() <= slack)[f].all(), (step, key, (got - want)[f].abs().max())
+    x0 = _dev(gaussian_delta(n, cin, h, w, 1.0, 1.0, seed=9)[0]).to(bf)
+    for o, lo, hi in [(big, 0, n)] + [(one[i], i, i + 1) for i in range(n)]:
+        ops.build_mask_tiles(torch.ones((hi - lo, 1, h, w), dtype=torch.uint8, device=DEV), None, hi - lo, h, w, _lib.FOOT_CONV, 5, 1, 2, o["ts"])
+        ops.conv_refresh(_dev(x0[lo:hi]).clone(), None, filt, torch.linspace(-1, 1, cout, device=DEV), 5, 1, 2, o["ts"], o["out"], o["res"],
+                         _lib.ACT_NONE if act is None else act, 0.1)
+    got, want = big["res"].cpu(), torch.cat([o["res"] for o in one]).cpu()
+    assert torch.isfinite(got).all() and torch.allclose(got, want, rtol=0, atol=2 * 25 * cin * 2.0 ** -24 * 200)
+
+
 # The persistent form of the 64 -> 32 bf16 up-sampling conv (the last decoder of the batched network) takes planes of
 # at least 2048 tiles.  Same inputs once as a batch of three ragged frames (2250 tiles: the persistent kernel) and once
 # frame by frame (750 tiles each: one workgroup per tile) must agree bit for bit -- deltas and reservoirs -- over three
