@@ -142,9 +142,10 @@ __global__ __launch_bounds__(64) void k_conv_smallco(ConvArgsT<T> a) {
 
 // ---------------------------------------------------------------------------------
 // 1x1 stride-1 conv with Cout <= 4 and Cin % 4 == 0 (prediction layer 32 -> 1, flow heads): pure
-// bandwidth work.  4 lanes share one pixel and walk its NHWC row in 16-byte (fp32) / 8-byte
+// bandwidth work.  LP lanes share one pixel and walk its NHWC row in 16-byte (fp32) / 8-byte
 // (bf16) pieces, so a wave reads whole 8-pixel tile rows as contiguous segments; the partial
-// sums meet through two lane exchanges.  Lane `sub` of a pixel stores output channel `sub`.
+// sums meet through lane exchanges.  Lane `sub` of a pixel stores output channel `sub`.  A tile of 64 pixels takes
+// LP / 4 workgroups (blockIdx.y).
 // ---------------------------------------------------------------------------------
 static __device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 static __device__ __forceinline__ float4 load4(const mie_bf16* p) {
@@ -152,12 +153,12 @@ static __device__ __forceinline__ float4 load4(const mie_bf16* p) {
   return make_float4((float)b[0], (float)b[1], (float)b[2], (float)b[3]);
 }
 
-template <typename T>
+template <typename T, int LP>
 __global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
   int n, y0, x0;
   const int tk = mie_pick_tile(a.ts, blockIdx.x + conv_args_entry_zero(a), n, y0, x0);
   if (tk == 0) return;
-  const int px = threadIdx.x >> 2, sub = threadIdx.x & 3;
+  const int px = blockIdx.y * (256 / LP) + threadIdx.x / LP, sub = threadIdx.x & (LP - 1);
   const int oy = y0 + (px >> 3), ox = x0 + (px & 7);
   const int hout = a.ts.h, wout = a.ts.w;
   const bool inb = oy < hout && ox < wout;
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
     if (xin == nullptr || !inb || (xm != nullptr && !xm[po])) continue;
     const T* xr = xin + po * cs;
     const float* wrow = a.filt + (long long)(src ? a.c1 : 0) * a.cout;
-    for (int v = sub; v < (cs >> 2); v += 4) {
+    for (int v = sub; v < (cs >> 2); v += LP) {
       const float4 x = load4(xr + 4 * v);
       const float* wp = wrow + (long long)(4 * v) * a.cout;
       for (int co = 0; co < a.cout; ++co)
@@ -183,8 +184,8 @@ __global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
   }
 #pragma unroll
   for (int co = 0; co < 4; ++co) {           // every lane of the wave takes part
-    acc[co] += __shfl_xor(acc[co], 1);
-    acc[co] += __shfl_xor(acc[co], 2);
+#pragma unroll
+    for (int d = 1; d < LP; d <<= 1) acc[co] += __shfl_xor(acc[co], d);
   }
   const float mine = sub == 0 ? acc[0] : (sub == 1 ? acc[1] : (sub == 2 ? acc[2] : acc[3]));
   if (inb && sub < a.cout) conv_store(a, po * a.cout + sub, sub, mine);
@@ -282,7 +283,10 @@ __global__ __launch_bounds__(256) void k_tconv2x_fewcin(ConvArgsT<T> a) {
 template <typename T, int K, int S>
 void launch_conv(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
   if (K == 1 && S == 1 && a.pad == 0 && a.cout <= 4 && (a.c1 & 3) == 0 && (a.c2 & 3) == 0) {
-    hipLaunchKernelGGL((k_conv1x1_smallco<T>), dim3(cap), dim3(256), 0, st, a);
+    // a pixel's row walked by 4 lanes is a chain of dependent rounds: 16 lanes from 128 channels on (256 at 32x32 11.4 -> 6.8 us,
+    // 128 at 64x64 7.1 -> 5.6; 64 at 128x128 5.3 -> 7.5, so not there)
+    if (a.c1 >= 128 || a.c2 >= 128) hipLaunchKernelGGL((k_conv1x1_smallco<T, 16>), dim3(cap, 4), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_conv1x1_smallco<T, 4>), dim3(cap), dim3(256), 0, st, a);
   } else if (a.cout <= 4) {
     hipLaunchKernelGGL((k_conv_smallco<T, K, S>), dim3(cap), dim3(64), 0, st, a);
   } else {
