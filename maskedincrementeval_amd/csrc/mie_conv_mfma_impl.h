@@ -1095,8 +1095,8 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
 
 // The partial sums of four channels (offset off), added in the order of the parts.  All of them are loaded before the first
 // is added, for the counts a split makes (split_parts: 2, 4, 8): in a loop over the parts each load waited for the one
-// before it, and these launches consist of little
-// but that wait (8 parts, 256 channels at 8x12: 5.3 -> 4.1 us; a gates conv of 4 parts there 7.1 -> 5.6).
+// before it, and these launches consist of little but that wait (8 parts, 256 channels at 8x12: 5.3 -> 4.1 us; a gates conv
+// of 4 parts there 7.1 -> 5.6).
 template <int PARTS>
 __device__ __forceinline__ float4 split_sum_of(const float* ws, long long plane) {
   float4 v[PARTS];
