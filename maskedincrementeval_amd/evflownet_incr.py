@@ -52,11 +52,11 @@ class nnCatIncr(replay.Watched, nn.Module, _IncrBuffers):
     buffers; used where a kernel takes one input pointer only)."""
 
     def forward(self, parts):
-        if ops._planner is not None:
+        if ops._pass.planner is not None:
             # torch.cat / torch.maximum below run on the compute stream and would read pixel masks that the
             # planning stream is still writing
             raise NotImplementedError("nnCatIncr under asynchronous mask planning; use async_masks=False")
-        if ops._phase is not None:      # ... or that the plan of this pass has yet to write
+        if ops._pass.phase is not None:      # ... or that the plan of this pass has yet to write
             raise replay.ValueDependentMask("nnCatIncr reads pixel masks: this network cannot be planned ahead; use plan_first=False")
         deltas = [ops.as_nhwc(p[0]) for p in parts]
         n, _, h, w = deltas[0].shape

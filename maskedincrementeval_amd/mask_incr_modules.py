@@ -43,7 +43,7 @@ class _IncrBuffers:
         return d
 
     def _delta_buf(self, name, shape, device, dtype=torch.float32) -> torch.Tensor:
-        key = ("d", name, tuple(shape), str(device), dtype, ops.buffer_parity)
+        key = ("d", name, tuple(shape), str(device), dtype, ops._pass.buffer_parity)
         b = self._ib().get(key)
         if b is None:
             b = ops.new_nhwc(*shape, device, dtype)
@@ -51,7 +51,7 @@ class _IncrBuffers:
         return b
 
     def _tile_set(self, name, n, h, w, device) -> TileMask:
-        key = ("t", name, (n, h, w), str(device), ops.buffer_parity)
+        key = ("t", name, (n, h, w), str(device), ops._pass.buffer_parity)
         b = self._ib().get(key)
         if b is None:
             b = TileMask(n, h, w, device)
@@ -59,7 +59,7 @@ class _IncrBuffers:
         return b
 
     def _pix_buf(self, name, n, h, w, device) -> torch.Tensor:
-        key = ("p", name, (n, h, w), str(device), ops.buffer_parity)
+        key = ("p", name, (n, h, w), str(device), ops._pass.buffer_parity)
         b = self._ib().get(key)
         if b is None:
             b = torch.zeros((n, 1, h, w), dtype=torch.uint8, device=device)

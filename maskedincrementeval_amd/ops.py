@@ -5,6 +5,7 @@ and the current HIP stream out of torch, and calls one entry point of
 include/mie.h.  torch is used for memory and streams only.
 """
 import os
+import threading
 from typing import Optional, Tuple
 
 import torch
@@ -17,8 +18,35 @@ from .masked_types import TileMask
 # A network whose masks depend on the input mask only can be walked twice per step: a planning pass in
 # which only the mask builds are launched (onto the planning stream), then a compute pass in which
 # only the other kernels are.  All builds are then enqueued -- and, in a captured graph, ordered --
-# ahead of the kernels that consume them.  `_phase` is None outside such a walk.
-_phase = None
+# ahead of the kernels that consume them.
+
+
+class _PassState(threading.local):
+    """What the pass under way is doing, for the thread that runs it: threads that step networks of their own see each
+    other's in nothing.  Readable as ops._phase, ops._planner, ... too (module __getattr__)."""
+    phase = None             # None | "plan" | "compute"
+    plan_batch = None        # [(p1, p2, h_in, w_in, foot, k, stride, pad, out TileMask)] while a planning pass collects
+    plan_wgs = 0             # workgroup limit of the plan being made (0: the library's own)
+    buffer_parity = 0        # generation of tile sets and delta buffers (planning one step ahead, below)
+    planner = None           # (side stream, device) inside a mask_planner block
+
+    def __init__(self):
+        self.pix_ready = {}      # data_ptr of a pixel mask written on the compute stream -> event
+        self.pending_thr = {}    # thresholded masks whose kernel is not launched yet (threshold_mask_lazy)
+        self.side_streams = {}           # device -> stream of the mask builds (mask_planner)
+        self.lookahead_streams = {}      # device -> stream of pipelined_step's plan
+
+
+_pass = _PassState()
+
+
+def __getattr__(name):
+    key = name[1:] if name.startswith("_") else name
+    if key in ("phase", "planner", "plan_batch", "plan_wgs", "pix_ready", "pending_thr", "buffer_parity"):
+        return getattr(_pass, key)
+    raise AttributeError("module %r has no attribute %r" % (__name__, name))
+
+
 _BUILD_ENTRIES = ("mie_build_mask_tiles",)
 
 
@@ -30,7 +58,7 @@ class _PhaseLib:
         fn = getattr(self._real, name)
         if name.startswith("mie_") and name not in ("mie_last_error_string", "mie_tile_capacity", "mie_version",
                                                      "mie_pack_filter", "mie_pack_filter_up2x"):
-            runs = (name in _BUILD_ENTRIES) == (_phase == "plan")
+            runs = (name in _BUILD_ENTRIES) == (_pass.phase == "plan")
             if not runs:
                 return lambda *args: 0
         return fn
@@ -38,7 +66,7 @@ class _PhaseLib:
 
 def lib():
     real = replay.lib()
-    return real if _phase is None else _PhaseLib(real)
+    return real if _pass.phase is None else _PhaseLib(real)
 
 
 # The builds of a planning pass are not launched one by one: they are collected and handed to the library as
@@ -49,7 +77,6 @@ def lib():
 # own with an event of their own, so that the first convs run beside the plan of the rest -- every extra dependency
 # between the two streams costs 5-10 us of idle time in the replayed graph, more than the overlap wins.)
 fused_plan = os.environ.get("MIE_FUSED_PLAN", "1") != "0"
-_plan_batch = None       # [(p1, p2, h_in, w_in, foot, k, stride, pad, out TileMask)] while a planning pass collects
 _plan_cache = {}         # signature of a batch -> [("plan", ctypes array, n) | ("single", index)] parts
 
 
@@ -60,20 +87,18 @@ class network_pass:
         self.phase = phase
 
     def __enter__(self):
-        global _phase, _plan_batch
-        self.prev, _phase = _phase, self.phase
+        self.prev, _pass.phase = _pass.phase, self.phase
         if self.phase == "plan" and fused_plan:
-            _plan_batch = []
+            _pass.plan_batch = []
         return self
 
     def __exit__(self, *exc):
-        global _phase, _plan_batch
-        batch, _plan_batch = _plan_batch, None
+        batch, _pass.plan_batch = _pass.plan_batch, None
         try:
             if self.phase == "plan" and batch and exc[0] is None:
                 _launch_plan(batch)
         finally:
-            _phase = self.prev
+            _pass.phase = self.prev
         return False
 
 
@@ -91,7 +116,8 @@ def _launch_plan(batch):
     single build would get), else on the current stream."""
     real = replay.lib()
     dev = batch[0][-1].device
-    side = _planner[0] if (_planner is not None and _planner[1] == dev) else None
+    planner, plan_wgs = _pass.planner, _pass.plan_wgs
+    side = planner[0] if (planner is not None and planner[1] == dev) else None
     if side is not None:
         fresh = False
         for b in batch:
@@ -104,16 +130,16 @@ def _launch_plan(batch):
             side.wait_event(ev0)
         for b in batch:
             for ptr in b[:2]:
-                ev = _pix_ready.get(ptr)
+                ev = _pass.pix_ready.get(ptr)
                 if ev is not None:
                     side.wait_event(ev)
         stream = side.cuda_stream
     else:
         stream = torch.cuda.current_stream(dev).cuda_stream
-    sig = tuple(b[:8] + (b[8].pixmask.data_ptr(), b[8].tiles.data_ptr()) for b in batch) + (_plan_wgs,)
+    sig = tuple(b[:8] + (b[8].pixmask.data_ptr(), b[8].tiles.data_ptr()) for b in batch) + (plan_wgs,)
     parts = _plan_cache.get(sig)
-    if _plan_wgs:
-        build_plan = lambda arr, n: real.mie_build_mask_plan_wgs(arr, n, _plan_wgs, stream)
+    if plan_wgs:
+        build_plan = lambda arr, n: real.mie_build_mask_plan_wgs(arr, n, plan_wgs, stream)
     else:
         build_plan = lambda arr, n: real.mie_build_mask_plan(arr, n, stream)
 
@@ -169,12 +195,9 @@ def _launch_plan(batch):
 # is not the one the plan of its parity was made for (same pointer and shape), and plan_step_ahead refuses sets whose
 # last plan was never run.  (Under graph capture these checks see the capture order only: replay the captured steps in the
 # cyclic order they were captured in.)
-buffer_parity = 0
-_lookahead_streams = {}
 # A plan made ahead runs beside the convs of the step before it and nothing waits for it: it is held to this many
 # workgroups (mie_build_mask_plan_wgs), so that the chip stays with the convs.  0: the library's own cap.
 LOOKAHEAD_PLAN_WGS = int(os.environ.get("MIE_LOOKAHEAD_PLAN_WGS", "64"))      # tuning knob, read once
-_plan_wgs = 0
 
 
 def _delta_key(t):
@@ -182,7 +205,7 @@ def _delta_key(t):
 
 
 def _check_lookahead_context(parity):
-    if _phase is not None or _planner is not None:
+    if _pass.phase is not None or _pass.planner is not None:
         raise RuntimeError("planning one step ahead: not inside a planning pass or a mask_planner block")
     if parity not in (0, 1):
         raise ValueError("parity must be 0 or 1")
@@ -197,20 +220,18 @@ def plan_step_ahead(state: dict, parity: int, delta: torch.Tensor, make_mask, wa
     the event recorded after that plan before step k + 1).
     state: a dict the caller keeps per network instance; make_mask(delta) -> the input pixel mask (or None: every
     pixel), written into the parity's buffer; walk(delta, mask) -> one walk of the network."""
-    global buffer_parity
     _check_lookahead_context(parity)
     pending = state.setdefault("planned", {})
     if pending.get(parity) is not None:
         raise RuntimeError("planning one step ahead: the step planned for parity %d was never run" % parity)
-    global _plan_wgs
     try:
-        buffer_parity, _plan_wgs = parity, LOOKAHEAD_PLAN_WGS
+        _pass.buffer_parity, _pass.plan_wgs = parity, LOOKAHEAD_PLAN_WGS
         mask = make_mask(delta)
         with network_pass("plan"):
             walk(delta, mask)
         pending[parity] = _delta_key(delta)
     finally:
-        buffer_parity = _plan_wgs = 0
+        _pass.buffer_parity = _pass.plan_wgs = 0
 
 
 def run_planned_step(state: dict, parity: int, delta: torch.Tensor, make_mask, mask_buffer, walk):
@@ -218,11 +239,10 @@ def run_planned_step(state: dict, parity: int, delta: torch.Tensor, make_mask, m
     planned for this parity (the first step of a sequence) the plan is made here first.  A plan for another delta
     (other pointer or shape) than the one passed is refused.  mask_buffer(delta) -> the parity's input-mask buffer
     without recomputing it."""
-    global buffer_parity
     _check_lookahead_context(parity)
     pending = state.setdefault("planned", {})
     try:
-        buffer_parity = parity
+        _pass.buffer_parity = parity
         if pending.get(parity) == _delta_key(delta):
             mask = mask_buffer(delta)
         elif pending.get(parity) is None:
@@ -236,7 +256,7 @@ def run_planned_step(state: dict, parity: int, delta: torch.Tensor, make_mask, m
         with network_pass("compute"):
             return walk(delta, mask)
     finally:
-        buffer_parity = 0
+        _pass.buffer_parity = 0
 
 
 def pipelined_step(state: dict, parity: int, delta: torch.Tensor, next_delta: Optional[torch.Tensor],
@@ -261,9 +281,9 @@ def pipelined_step(state: dict, parity: int, delta: torch.Tensor, next_delta: Op
     # this step's kernels are enqueued first: the look-ahead depends on none of them
     out = run_planned_step(state, parity, delta, make_mask, mask_buffer, walk)
     if fork is not None:
-        side = _lookahead_streams.get(dev)
+        side = _pass.lookahead_streams.get(dev)
         if side is None:
-            side = _lookahead_streams[dev] = torch.cuda.Stream(dev)
+            side = _pass.lookahead_streams[dev] = torch.cuda.Stream(dev)
         side.wait_event(fork)                          # fork (joins a graph capture, too)
         with torch.cuda.stream(side):
             plan_step_ahead(state, 1 - parity, next_delta, make_mask, walk)
@@ -347,9 +367,6 @@ def _stream(t: torch.Tensor):
 # event of its build and the first kernel that uses it makes the compute stream wait for it.
 # Pixel masks written on the compute stream (input mask, refined masks) carry an event the
 # other way.  Under HIP-graph capture these waits become edges of the graph.
-_planner = None          # (side stream, device) while active
-_side_streams = {}
-_pix_ready = {}          # data_ptr of a pixel mask written on the compute stream -> event
 
 
 class mask_planner:
@@ -357,28 +374,25 @@ class mask_planner:
         self.device = torch.device(device)
 
     def __enter__(self):
-        global _planner
-        if _planner is not None or self.device.type != "cuda":
+        if _pass.planner is not None or self.device.type != "cuda":
             self.nested = True
             return self
         self.nested = False
-        side = _side_streams.get(self.device)
+        side = _pass.side_streams.get(self.device)
         if side is None:
-            side = torch.cuda.Stream(self.device)
-            _side_streams[self.device] = side
+            side = _pass.side_streams[self.device] = torch.cuda.Stream(self.device)
         ev = torch.cuda.Event()
         ev.record(torch.cuda.current_stream(self.device))
         side.wait_event(ev)          # forks from the compute stream (also joins a graph capture)
-        _planner = (side, self.device)
+        _pass.planner = (side, self.device)
         return self
 
     def __exit__(self, *exc):
-        global _planner
         if self.nested:
             return False
-        side, dev = _planner
-        _planner = None
-        _pix_ready.clear()
+        side, dev = _pass.planner
+        _pass.planner = None
+        _pass.pix_ready.clear()
         ev = torch.cuda.Event()
         ev.record(side)
         torch.cuda.current_stream(dev).wait_event(ev)     # join
@@ -388,7 +402,7 @@ class mask_planner:
 def _ready(ts: TileMask):
     """Make the compute stream wait for the build of `ts` (once)."""
     replay.keep(ts)
-    if _phase == "plan":
+    if _pass.phase == "plan":
         return
     root = ts.parent if ts.parent is not None else ts
     ev = root.__dict__.get("ready")
@@ -399,15 +413,15 @@ def _ready(ts: TileMask):
 
 def _mark_pix(t: Optional[torch.Tensor], from_values: bool = False):
     """A pixel mask was written on the compute stream: builds that read it must wait."""
-    if t is not None and from_values and _phase is not None:
+    if t is not None and from_values and _pass.phase is not None:
         raise replay.ValueDependentMask("a mask that depends on values (a delta, refined or quantised deltas) cannot be "
                            "planned ahead: run this network without the planning pass")
-    if _phase == "compute":
+    if _pass.phase == "compute":
         return
-    if _planner is not None and t is not None:
+    if _pass.planner is not None and t is not None:
         ev = torch.cuda.Event()
         ev.record(torch.cuda.current_stream(t.device))
-        _pix_ready[t.data_ptr()] = ev
+        _pass.pix_ready[t.data_ptr()] = ev
 
 
 def _require_gpu(t: torch.Tensor, name: str):
@@ -472,7 +486,7 @@ def pix_ptr(m, n, h, w, name):
         raise ValueError("%s must be a contiguous uint8 (%d,1,%d,%d) mask, got %s %s"
                          % (name, n, h, w, tuple(t.shape), t.dtype))
     _require_gpu(t, name)
-    if _pending_thr:
+    if _pass.pending_thr:
         _force_threshold_mask(t)
     replay.keep(t)
     return t.data_ptr()
@@ -515,7 +529,6 @@ def mask_from_delta(delta: torch.Tensor, threshold: float, out: torch.Tensor):
 # buffer).  threshold_mask_lazy leaves the launch to the first reader of the buffer.  If that reader is the build of a
 # conv's tile set, threshold test, footprint and lists go out as one launch (mie_build_mask_tiles_thresholded); any
 # other reader (pix_ptr) launches mie_mask_from_delta first.
-_pending_thr = {}
 fused_threshold_build = os.environ.get("MIE_FUSED_THRESHOLD_BUILD", "1") != "0"      # tuning knob, read once
 
 
@@ -525,12 +538,12 @@ def threshold_mask_lazy(delta: torch.Tensor, threshold: float, out: torch.Tensor
     if not fused_threshold_build:
         return mask_from_delta(delta, threshold, out)
     _mark_pix(out, from_values=True)
-    _pending_thr[out.data_ptr()] = (delta, float(threshold), out)
+    _pass.pending_thr[out.data_ptr()] = (delta, float(threshold), out)
     return out
 
 
 def _force_threshold_mask(t: torch.Tensor):
-    ent = _pending_thr.pop(t.data_ptr(), None)
+    ent = _pass.pending_thr.pop(t.data_ptr(), None)
     if ent is not None:
         mask_from_delta(*ent)
 
@@ -538,15 +551,15 @@ def _force_threshold_mask(t: torch.Tensor):
 def _thresholded_build(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, out: TileMask) -> bool:
     """The one-launch form of a pending threshold mask + the build that reads it, where the library has one."""
     t = in_mask.pixmask if isinstance(in_mask, TileMask) else in_mask
-    ent = None if t is None else _pending_thr.get(t.data_ptr())
+    ent = None if t is None else _pass.pending_thr.get(t.data_ptr())
     if ent is None:
         return False
     delta, thr, buf = ent
     if (foot != _lib.FOOT_CONV or stride + pad > k or 7 * stride + k + max(0, stride - 1 - pad) > 24
-            or _phase is not None or (_planner is not None and _planner[1] == out.device)
+            or _pass.phase is not None or (_pass.planner is not None and _pass.planner[1] == out.device)
             or tuple(delta.shape) != (n, delta.shape[1], h_in, w_in)):
         return False
-    del _pending_thr[t.data_ptr()]
+    del _pass.pending_thr[t.data_ptr()]
     p2 = pix_ptr(in_mask2, n, h_in, w_in, "in_mask2")
     check(lib().mie_build_mask_tiles_thresholded(
         nhwc_ptr(delta, "delta", dtype=delta.dtype), delta.shape[1], delta_dtype(delta), thr,
@@ -557,22 +570,23 @@ def _thresholded_build(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, o
 def build_mask_tiles(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, out: TileMask):
     """in_mask / in_mask2: None | TileMask | uint8 (N,1,H,W)."""
     replay.keep(out)
-    if _pending_thr and _thresholded_build(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, out):
+    if _pass.pending_thr and _thresholded_build(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, out):
         return out
     p1 = pix_ptr(in_mask, n, h_in, w_in, "in_mask")
     p2 = pix_ptr(in_mask2, n, h_in, w_in, "in_mask2")
     if p1 is None and p2 is not None:   # "all active" OR anything = all active
         p2 = None
-    if _phase == "compute":             # built by the planning pass; its event is still attached
+    phase, planner = _pass.phase, _pass.planner
+    if phase == "compute":              # built by the planning pass; its event is still attached
         return out
-    if _phase == "plan" and _plan_batch is not None:
-        _plan_batch.append((p1, p2, h_in, w_in, foot, k, stride, pad, out))
+    if phase == "plan" and _pass.plan_batch is not None:
+        _pass.plan_batch.append((p1, p2, h_in, w_in, foot, k, stride, pad, out))
         return out
-    if _planner is None or _planner[1] != out.device:
+    if planner is None or planner[1] != out.device:
         st = torch.cuda.current_stream(out.device).cuda_stream
         check(lib().mie_build_mask_tiles(p1, p2, h_in, w_in, foot, k, stride, pad, out.ref, st))
         return out
-    side = _planner[0]
+    side = planner[0]
     root = out.parent if out.parent is not None else out
     if not root.__dict__.get("built_once"):
         # a freshly allocated tile set is zero-filled on the compute stream: its first build
@@ -582,7 +596,7 @@ def build_mask_tiles(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, out
         side.wait_event(ev0)
         root.built_once = True
     for ptr in (p1, p2):
-        ev = _pix_ready.get(ptr)
+        ev = _pass.pix_ready.get(ptr)
         if ev is not None:
             side.wait_event(ev)
     check(lib().mie_build_mask_tiles(p1, p2, h_in, w_in, foot, k, stride, pad, out.ref, side.cuda_stream))
@@ -1369,7 +1383,7 @@ def conv_out_size(h, w, k, stride, pad) -> Tuple[int, int]:
 
 # what a recorded pass (replay.py) depends on: it is not used while one of these functions is replaced, nor once one of
 # these settings has another value
-replay.bind_ops(globals(), (
+replay.bind_ops(globals(), _pass, (
     "lib", "check", "mask_from_delta", "threshold_mask_lazy", "build_mask_tiles", "conv_masked", "upconv_masked",
     "upconv_pred_masked", "upconv2x_masked", "upconv2x_refresh", "conv_refresh", "tconv_masked", "tconv_refresh", "tconv2x_masked", "tconv2x_refresh", "act_incr",
     "kfence_incr", "mul_incr", "add_incr", "maxpool_incr", "accumulate", "scale_incr", "avgpool_incr", "upsample2x_incr",

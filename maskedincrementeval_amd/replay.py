@@ -34,7 +34,7 @@ from ._lib import check
 enabled = os.environ.get("MIE_REPLAY", "1") != "0"      # read once
 MAX_RECORDINGS = 8          # per module and method, least recently used first out
 _epoch = [0]
-_active = None              # the Recording being made, by the thread that makes it
+_recording = {}             # thread identity -> the Recording that thread is making
 _SILENT = frozenset(("training", "states"))     # assignments no incremental pass depends on
 
 
@@ -56,24 +56,25 @@ class ValueDependentMask(RuntimeError):
 
 
 # ---- what the pass reads outside the modules -----------------------------------------------------------------
-_ops_globals = None
+_ops_globals = _ops_pass = None
 _get_functions = _get_settings = None
 _functions = ()
 
 
-def bind_ops(namespace, functions, settings):
-    """Called once by ops: its namespace, and the names a pass goes through / depends on."""
-    global _ops_globals, _get_functions, _get_settings, _functions
-    _ops_globals = namespace
+def bind_ops(namespace, pass_state, functions, settings):
+    """Called once by ops: its namespace, the state of a thread's pass, and the names a pass goes through / depends on."""
+    global _ops_globals, _ops_pass, _get_functions, _get_settings, _functions
+    _ops_globals, _ops_pass = namespace, pass_state
     _get_functions, _get_settings = operator.itemgetter(*functions), operator.itemgetter(*settings)
     _functions = _get_functions(namespace)
 
 
 def _idle() -> bool:
-    """Whether ops is in its ordinary state: no planning pass, no planning stream, no pending threshold mask."""
-    g = _ops_globals
-    return (g["_phase"] is None and g["_planner"] is None and not g["_pending_thr"] and g["buffer_parity"] == 0
-            and _get_functions(g) == _functions)
+    """Whether ops is in its ordinary state for this thread: no planning pass, no planning stream, no pending threshold
+    mask -- and its functions are its own."""
+    s = _ops_pass
+    return (s.phase is None and s.planner is None and not s.pending_thr and s.buffer_parity == 0
+            and _get_functions(_ops_globals) == _functions)
 
 
 # ---- recording ------------------------------------------------------------------------------------------------
@@ -101,7 +102,6 @@ class Recording:
 
     def __init__(self, real):
         self._real = real
-        self.thread = threading.get_ident()
         self.calls, self.keep, self.effects = [], [], []
 
     def __getattr__(self, name):
@@ -117,24 +117,33 @@ class Recording:
         return noted
 
 
+def current():
+    """The Recording this thread is making, or None."""
+    return _recording.get(threading.get_ident()) if _recording else None
+
+
 def lib():
     """The library, or the recording of it this thread is making."""
-    r = _active
-    return r if r is not None and r.thread == threading.get_ident() else _lib.lib()
+    if _recording:
+        r = _recording.get(threading.get_ident())
+        if r is not None:
+            return r
+    return _lib.lib()
 
 
 def keep(obj):
     """While a pass is recorded: its recording holds on to `obj`, whose address it uses."""
-    r = _active
-    if r is not None:
-        r.keep.append(obj)
+    if _recording:
+        r = _recording.get(threading.get_ident())
+        if r is not None:
+            r.keep.append(obj)
     return obj
 
 
 def effect(fn, *args):
     """fn(*args), now and on every replay of the pass: for changes of host state the pass makes."""
-    r = _active
-    if r is not None and r.thread == threading.get_ident():
+    r = current()
+    if r is not None:
         r.effects.append((fn, args))
     return fn(*args)
 
@@ -272,10 +281,10 @@ class _Waiting:
 
 def _record(owner, fns, pointers, tree, static):
     """One pass, recorded if it can be: (result, Program or None)."""
-    global _active
+    me = threading.get_ident()
     for k, fn in enumerate(fns):
         rec, watch = Recording(_lib.lib()), _TorchWatch()
-        _active = rec
+        _recording[me] = rec
         try:
             with watch:
                 result = fn()
@@ -284,7 +293,7 @@ def _record(owner, fns, pointers, tree, static):
                 raise
             continue
         finally:
-            _active = None
+            del _recording[me]
         if watch.seen is not None or any(_signature(name) is None for name, _ in rec.calls):
             return result, None
         for name, args in rec.calls:        # a plan holds its input masks inside its own array
@@ -322,7 +331,7 @@ def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
     def decorate(method):
         @functools.wraps(method)
         def wrapped(self, *args, **kw):
-            if kw or not enabled or _active is not None or not _idle():
+            if kw or not enabled or current() is not None or not _idle():
                 return method(self, *args, **kw)
             key, pointers, held = [method.__name__], [], []
             for i, a in enumerate(args):

@@ -1,0 +1,121 @@
+"""Recorded passes on the host side, without a GPU: the library is a stub that notes its calls and runs recorded sequences
+by reading their words, so what a recording holds and when it is used can be looked at call by call."""
+import ctypes
+import threading
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from maskedincrementeval_amd import _lib, ops, replay
+
+
+class StubLib:
+    """Answers every entry point with 0; `calls` holds (thread, name, arguments), recorded calls as their words."""
+
+    def __init__(self, real):
+        self._real = real
+        self.calls = []
+        self.mie_call_index, self.mie_call_signature = real.mie_call_index, real.mie_call_signature
+        self.mie_conv_f32x3_takes = lambda *a: 0
+
+    def __getattr__(self, name):
+        if not name.startswith("mie_"):
+            raise AttributeError(name)
+
+        def fn(*args):
+            self.calls.append((threading.get_ident(), name, args))
+            return 0
+        return fn
+
+    def mie_run_calls(self, calls, n, inputs, n_inputs, stream):
+        names = {self._real.mie_call_index(k.encode()): k for k in _lib.EXPORTS if self._real.mie_call_index(k.encode()) >= 0}
+        for c in calls[:n]:
+            words = list(ctypes.cast(c.args, ctypes.POINTER(ctypes.c_uint64))[:c.n_args])
+            patches = ctypes.cast(c.patches, ctypes.POINTER(ctypes.c_int32))
+            for p in range(c.n_patches):
+                words[patches[2 * p]] = inputs[patches[2 * p + 1]]
+            self.calls.append((threading.get_ident(), names[c.entry], words))
+        return 0
+
+    def named(self, name, thread=None):
+        return [a for t, n, a in self.calls if n == name and thread in (None, t)]
+
+
+@pytest.fixture
+def stub(mie_lib, monkeypatch):
+    """The package on CPU tensors over a StubLib."""
+    s = StubLib(mie_lib)
+    monkeypatch.setattr(_lib, "_lib", s)
+    monkeypatch.setattr(ops, "_require_gpu", lambda t, name: None)
+    monkeypatch.setattr(ops, "_stream", lambda t: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: SimpleNamespace(cuda_stream=0))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 0, raising=False)
+    monkeypatch.setattr(replay, "_is_nhwc", lambda t: t.dim() == 4 and t.is_contiguous(memory_format=torch.channels_last))
+    return s
+
+
+def in_thread(fn):
+    """fn() in another thread: its result, or its exception raised here."""
+    box = []
+
+    def body():
+        try:
+            box.append((fn(), None))
+        except BaseException as e:
+            box.append((None, e))
+    t = threading.Thread(target=body)
+    t.start()
+    t.join(60)
+    assert box, "the thread did not end"
+    if box[0][1] is not None:
+        raise box[0][1]
+    return box[0][0]
+
+
+def test_a_planning_pass_is_seen_by_its_own_thread_only(stub):
+    ts = SimpleNamespace(ref=None, device=torch.device("cpu"), parent=None)
+
+    def other():
+        assert ops._phase is None and ops._plan_batch is None and ops.buffer_parity == 0
+        assert ops.lib().mie_conv_masked_ws(1) == 0
+        ops.build_mask_tiles(None, None, 1, 8, 8, 0, 1, 1, 0, ts)
+        with ops.network_pass("compute"):
+            pass
+        return threading.get_ident()
+
+    with ops.network_pass("plan"):
+        ops.lib().mie_conv_masked_ws(0)                  # a planning pass: not made
+        me = in_thread(other)
+        assert not ops._plan_batch and ops._phase == "plan"
+        ops._plan_batch.clear()
+    assert stub.named("mie_conv_masked_ws") == stub.named("mie_conv_masked_ws", me) == [(1,)]
+    assert len(stub.named("mie_build_mask_tiles", me)) == 1
+
+
+def test_threads_record_side_by_side(stub):
+    """Two threads record at the same time: each recording holds its thread's calls, all of them and no other's."""
+    meet = threading.Barrier(2, timeout=30)
+
+    def one(tag):
+        def body():
+            meet.wait()
+            for i in range(20):
+                assert ops.lib().mie_mul_dense(0, 0, 0, 100 * tag + i, 0, 0) == 0
+                replay.keep(tag)
+                if i % 5 == 0:
+                    meet.wait()
+            return tag
+        result, program = replay._record(None, [body], [], (), [])
+        assert result == tag and program is not None and set(program.held[0]) == {tag}
+        return program
+
+    got = {}
+    threads = [threading.Thread(target=lambda t=t: got.__setitem__(t, one(t))) for t in (1, 2)]
+    [t.start() for t in threads]
+    [t.join(60) for t in threads]
+    for tag in (1, 2):
+        del stub.calls[:]
+        got[tag].run((), 0)
+        assert [w[3] for w in stub.named("mie_mul_dense")] == [100 * tag + i for i in range(20)]
