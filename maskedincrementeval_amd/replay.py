@@ -15,7 +15,8 @@ A recording stands for the Python pass as long as everything that pass read is w
   * forward hooks, and the members of module containers.
 Otherwise the pass runs in Python again and is recorded anew.  A pass that runs any torch operation of its own
 (a conversion, a concat, the allocation of a buffer) is never recorded, nor one on a planning stream or inside a
-planning pass.  Recordings hold references to every tensor whose address they use.
+planning pass, nor under graph capture.  It is recorded on copies of its inputs, so that what is an input is known by
+its address.  Recordings hold references to every tensor whose address they use.
 """
 import collections
 import ctypes
@@ -187,13 +188,63 @@ def _copy(v):
     return v
 
 
+class _Inputs:
+    """Copies of the inputs of a pass, which the pass is recorded on.  No other tensor lies where they lie, so an argument
+    with an address of theirs came from that input: the same argument given as anything else, too (a tensor that is the
+    delta in one place and the addend in another), has its own address there."""
+
+    def __init__(self, args, free):
+        self.args, self.copies = list(args), []
+        for i, j in free:
+            given = self.args[i] if j is None else self.args[i][j]
+            copy = given.detach().clone()
+            self.copies.append(copy)
+            if j is None:
+                self.args[i] = copy
+            else:
+                self.args[i] = list(self.args[i])
+                self.args[i][j] = copy
+        self.spans = [(c.data_ptr(), c.data_ptr() + c.numel() * c.element_size()) for c in self.copies]
+
+    def slot(self, address):
+        """Which input starts at `address`; None: it lies in none."""
+        for k, (lo, hi) in enumerate(self.spans):
+            if lo <= address < hi:
+                if address != lo:
+                    raise _NotRecordable("an address inside an input")
+                return k
+        return None
+
+    def holds(self, t):
+        return any(lo <= t.data_ptr() < hi for lo, hi in self.spans)
+
+    def refuse(self, what, *addresses):
+        if any(a and self.slot(a) is not None for a in addresses):
+            raise _NotRecordable(what)
+
+    def refuse_in(self, value):
+        """No part of a result or of a change of host state may be an input: the next pass has others."""
+        if torch.is_tensor(value):
+            self.refuse("an input is handed on", value.data_ptr())
+        elif isinstance(value, (list, tuple)):
+            for x in value:
+                self.refuse_in(x)
+        elif isinstance(value, dict):
+            self.refuse_in(list(value.values()))
+        elif hasattr(value, "c_struct"):
+            self.refuse_set(value.c_struct)
+
+    def refuse_set(self, ts):
+        self.refuse("a tile set over an input", ts.pixmask, ts.tiles, ts.stale, ts.counts, ts.flags)
+
+
 class Program:
     """A recorded pass that can be run again."""
 
-    def __init__(self, rec, pointers, result, tree, static):
+    def __init__(self, rec, inputs, result, tree, static):
         self.effects, self.result = rec.effects, result
         self.runs = 0
-        self.held = [rec.keep, static]
+        self.held = [[k for k in rec.keep if not (torch.is_tensor(k) and inputs.holds(k))], static]
         calls = (_lib.MieCall * len(rec.calls))()
         for call, (name, args) in zip(calls, rec.calls):
             idx, sig = _signature(name)
@@ -201,17 +252,25 @@ class Program:
             patches = []
             for i, kind in enumerate(sig):
                 words[i] = _word(kind, args[i], self.held)
-                if kind == "r" and words[i] and words[i] in pointers:
-                    patches += [i, pointers.index(words[i])]
-                elif kind == "w" and words[i] in pointers:
-                    raise _NotRecordable("an input is written")
+                if kind == "w":
+                    inputs.refuse("an input is written", words[i])
+                elif kind == "t" and args[i] is not None:
+                    inputs.refuse_set(args[i]._obj)
+                elif isinstance(args[i], ctypes.Array):          # the ops of a plan
+                    for op in args[i]:
+                        inputs.refuse("an input inside a plan", op.in_mask, op.in_mask2)
+                        inputs.refuse_set(op.out)
+                elif kind == "r" and words[i]:
+                    slot = inputs.slot(words[i])
+                    if slot is not None:
+                        patches += [i, slot]
             pa = (ctypes.c_int32 * max(1, len(patches)))(*patches)
             call.entry, call.n_args, call.n_patches = idx, len(sig), len(patches) // 2
             call.args, call.patches = ctypes.addressof(words), ctypes.addressof(pa)
             self.held += [words, pa]
         self.calls, self.n = calls, len(rec.calls)
-        self.words_type = ctypes.c_uint64 * max(1, len(pointers))
-        self.n_inputs = len(pointers)
+        self.n_inputs = len(inputs.copies)
+        self.words_type = ctypes.c_uint64 * max(1, self.n_inputs)
         self.fn = _lib.lib().mie_run_calls
         self._guards(tree)
 
@@ -279,15 +338,16 @@ class _Waiting:
         self.seen, self.next, self.step = 0, 3, 2
 
 
-def _record(owner, fns, pointers, tree, static):
-    """One pass, recorded if it can be: (result, Program or None)."""
+def _record(fns, args, free, tree, static):
+    """One pass, recorded if it can be: (result, Program or None).  free: positions (argument, index in it or None) of
+    the inputs that may lie elsewhere in the next pass."""
     me = threading.get_ident()
     for k, fn in enumerate(fns):
-        rec, watch = Recording(_lib.lib()), _TorchWatch()
+        inputs, rec, watch = _Inputs(args, free), Recording(_lib.lib()), _TorchWatch()
         _recording[me] = rec
         try:
             with watch:
-                result = fn()
+                result = fn(*inputs.args)
         except ValueDependentMask:
             if k + 1 == len(fns):
                 raise
@@ -296,12 +356,10 @@ def _record(owner, fns, pointers, tree, static):
             del _recording[me]
         if watch.seen is not None or any(_signature(name) is None for name, _ in rec.calls):
             return result, None
-        for name, args in rec.calls:        # a plan holds its input masks inside its own array
-            if name.startswith("mie_build_mask_plan") and any(
-                    op.in_mask in pointers or op.in_mask2 in pointers for op in args[0]):
-                return result, None
         try:
-            return result, Program(rec, pointers, _copy(result), tree, static)
+            inputs.refuse_in(result)
+            inputs.refuse_in([effect_args for _, effect_args in rec.effects])
+            return result, Program(rec, inputs, _copy(result), tree, static)
         except _NotRecordable:
             return result, None
 
@@ -333,13 +391,14 @@ def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
         def wrapped(self, *args, **kw):
             if kw or not enabled or current() is not None or not _idle():
                 return method(self, *args, **kw)
-            key, pointers, held = [method.__name__], [], []
+            key, pointers, free, held = [method.__name__], [], [], []
             for i, a in enumerate(args):
                 if a is not None and i < dense + masked:
                     x = a if i < dense else a[0]
                     if not torch.is_tensor(x) or not _is_nhwc(x):
                         return method(self, *args)
                     pointers.append(x.data_ptr())
+                    free.append((i, None if i < dense else 0))
                     key += (x.shape, x.dtype, x.device.index)
                     m = None if i < dense or len(a) < 2 else a[1]
                     if torch.is_tensor(m):
@@ -349,6 +408,7 @@ def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
                             return method(self, *args)
                         if free_masks:
                             pointers.append(m.data_ptr())
+                            free.append((i, 1))
                             key.append("mask")
                         else:
                             key.append(m.data_ptr())
@@ -356,7 +416,7 @@ def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
                         key.append(_static_key(m, held))
                 else:
                     key.append(_static_key(a, held))
-            if not pointers or len(set(pointers)) != len(pointers):
+            if not pointers or len(set(pointers)) != len(pointers) or 0 in pointers:
                 return method(self, *args)
             key = tuple(key)
             cache = self.__dict__.get("_replay")
@@ -377,15 +437,14 @@ def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
                     cache.popitem(last=False)
                 ent = cache[key] = _Waiting()
             ent.seen += 1
-            if ent.seen < ent.next:
+            if ent.seen < ent.next or torch.cuda.is_current_stream_capturing():
                 return method(self, *args)
             # tried again after twice as many passes each time, so that a pass that cannot be recorded, or whose
             # surroundings change all the time, costs little more than it did
             ent.step = min(2 * ent.step, 256)
             ent.next = ent.seen + ent.step
-            fns = ([functools.partial(getattr(self, record), *args)] if record else []) + [
-                functools.partial(method, self, *args)]
-            result, program = _record(self, fns, pointers, (self,) + tuple(args[i] for i in trees), held)
+            fns = ([getattr(self, record)] if record else []) + [functools.partial(method, self)]
+            result, program = _record(fns, args, free, (self,) + tuple(args[i] for i in trees), held)
             if program is not None:
                 program.step = ent.step
                 cache[key] = program

@@ -1,13 +1,16 @@
 """Recorded passes on the host side, without a GPU: the library is a stub that notes its calls and runs recorded sequences
 by reading their words, so what a recording holds and when it is used can be looked at call by call."""
 import ctypes
+import gc
 import threading
+import weakref
 from types import SimpleNamespace
 
 import pytest
 import torch
 
 from maskedincrementeval_amd import _lib, ops, replay
+from maskedincrementeval_amd import mask_incr_modules as mm
 
 
 class StubLib:
@@ -107,7 +110,7 @@ def test_threads_record_side_by_side(stub):
                 if i % 5 == 0:
                     meet.wait()
             return tag
-        result, program = replay._record(None, [body], [], (), [])
+        result, program = replay._record([body], (), [], (), [])
         assert result == tag and program is not None and set(program.held[0]) == {tag}
         return program
 
@@ -119,3 +122,56 @@ def test_threads_record_side_by_side(stub):
         del stub.calls[:]
         got[tag].run((), 0)
         assert [w[3] for w in stub.named("mie_mul_dense")] == [100 * tag + i for i in range(20)]
+
+
+def _cl(*shape):
+    return torch.randn(*shape).contiguous(memory_format=torch.channels_last)
+
+
+def _conv(c=8, k=3):
+    conv = mm.nnConvIncr(c, c, k, 1, k // 2)
+    act = mm.nnReservedActivation(mm.leaky_relu_op(0.01), refine_mask=False)
+    act.in_res.reservoir = _cl(1, c, 8, 8)
+    return conv, act
+
+
+def _programs(m):
+    return [p for p in m.__dict__.get("_replay", {}).values() if isinstance(p, replay.Program)]
+
+
+def _ptrs(words):
+    """(x, x mask, addend) of a recorded mie_conv_masked_ws."""
+    return words[0], words[1], words[17]
+
+
+def test_an_addend_that_was_the_delta_when_recorded(stub):
+    """The same tensor as the delta and as the addend in the recorded passes: later passes read each from where it is."""
+    conv, act = _conv()
+    c = _cl(1, 8, 8, 8)
+    m = torch.ones(1, 1, 8, 8, dtype=torch.uint8)
+    with torch.no_grad():
+        for _ in range(3):
+            conv.forward_fused([c, m], act, addend_incr=[c, m])
+        for x in (_cl(1, 8, 8, 8), c, _cl(1, 8, 8, 8)):
+            mask = m.clone()
+            del stub.calls[:]
+            conv.forward_fused([x, mask], act, addend_incr=[c, m])
+            (words,) = stub.named("mie_conv_masked_ws")
+            assert _ptrs(words) == (x.data_ptr(), mask.data_ptr(), c.data_ptr())
+    assert [p.runs for p in _programs(conv)] == [3]
+
+
+def test_a_recording_holds_no_input(stub):
+    conv, act = _conv()
+    gone = []
+    with torch.no_grad():
+        for _ in range(5):
+            x, m = _cl(1, 8, 8, 8), torch.ones(1, 1, 8, 8, dtype=torch.uint8)
+            gone += [weakref.ref(x), weakref.ref(m)]
+            conv.forward_fused([x, m], act)
+            del x, m
+    del stub.calls[:]
+    gc.collect()
+    assert [p.runs for p in _programs(conv)] == [2] and not any(r() is not None for r in gone)
+    sizes = [t for t in gc.get_objects() if type(t) is torch.Tensor and t.dtype == torch.uint8 and tuple(t.shape) == (1, 1, 8, 8)]
+    assert len(sizes) == 1          # the tile set's own pixel mask; no copy of an input's
