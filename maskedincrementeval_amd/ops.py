@@ -56,8 +56,7 @@ class _PhaseLib:
 
     def __getattr__(self, name):
         fn = getattr(self._real, name)
-        if name.startswith("mie_") and name not in ("mie_last_error_string", "mie_tile_capacity", "mie_version",
-                                                     "mie_pack_filter", "mie_pack_filter_up2x"):
+        if name.startswith("mie_") and name not in replay.PASS_THROUGH and not name.startswith("mie_pack_filter"):
             runs = (name in _BUILD_ENTRIES) == (_pass.phase == "plan")
             if not runs:
                 return lambda *args: 0

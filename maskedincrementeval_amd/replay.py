@@ -79,7 +79,8 @@ def _idle() -> bool:
 
 
 # ---- recording ------------------------------------------------------------------------------------------------
-_PASS_THROUGH = frozenset(("mie_last_error_string", "mie_tile_capacity", "mie_version", "mie_conv_f32x3_takes"))
+# questions to the library, answered in every phase and never recorded
+PASS_THROUGH = frozenset(("mie_last_error_string", "mie_tile_capacity", "mie_version", "mie_conv_f32x3_takes"))
 _VIEWS = frozenset(("aten::permute", "aten::detach", "aten::view", "aten::slice", "aten::select", "aten::alias",
                     "aten::as_strided", "aten::t", "aten::transpose", "aten::unsqueeze", "aten::squeeze",
                     "aten::expand", "aten::_reshape_alias", "aten::_unsafe_view", "aten::split", "aten::unbind"))
@@ -107,7 +108,7 @@ class Recording:
 
     def __getattr__(self, name):
         fn = getattr(self._real, name)
-        if name in _PASS_THROUGH or not name.startswith("mie_"):
+        if name in PASS_THROUGH or not name.startswith("mie_"):
             return fn
 
         def noted(*args):

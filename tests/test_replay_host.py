@@ -175,3 +175,11 @@ def test_a_recording_holds_no_input(stub):
     assert [p.runs for p in _programs(conv)] == [2] and not any(r() is not None for r in gone)
     sizes = [t for t in gc.get_objects() if type(t) is torch.Tensor and t.dtype == torch.uint8 and tuple(t.shape) == (1, 1, 8, 8)]
     assert len(sizes) == 1          # the tile set's own pixel mask; no copy of an input's
+
+
+def test_a_planning_pass_asks_the_library_for_its_shapes(stub):
+    """What decides a layer's kernels is asked in the planning pass as in the compute pass: both walk the same layers."""
+    stub.mie_conv_f32x3_takes = lambda *args: 1
+    for phase in (None, "plan", "compute"):
+        with ops.network_pass(phase):
+            assert ops.f32x3_takes(5, 1, 256, 0, 128), phase
