@@ -796,14 +796,14 @@ class E2VIDRecurrentIncr(replay.Watched, nn.Module, _IncrBuffers):
 
     # A recorded step builds its tile sets as one plan ahead of the compute calls, where the masks allow it, whatever
     # plan_first says: the sets are the same, two launches instead of one or two per set.
-    @replay.replayed(record="_step_planned_pass", free_masks=False)
+    @replay.replayed(record="_step_planned_pass")
     def _step(self, x_incr, prev_states):
         delta, mask = x_incr
         if mask is None and self.derive_input_mask:
             mask = self.input_mask(delta)
         return self.unetrecurrent.forward([delta, mask], prev_states)
 
-    @replay.replayed(free_masks=False)
+    @replay.replayed()
     def _step_planned(self, x_incr, prev_states):
         return self._step_planned_pass(x_incr, prev_states)
 

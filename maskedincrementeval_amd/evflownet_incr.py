@@ -620,11 +620,11 @@ class MultiResUNetRecurrentIncr(replay.Watched, nn.Module, _IncrBuffers):
 
     # A recorded step builds its tile sets as one plan ahead of the compute calls, where the masks allow it, whatever
     # plan_first says: the sets are the same, two launches instead of one or two per set.
-    @replay.replayed(record="_step_planned_pass", free_masks=False)
+    @replay.replayed(record="_step_planned_pass")
     def _step(self, x_incr):
         return self._forward(*x_incr)
 
-    @replay.replayed(free_masks=False)
+    @replay.replayed()
     def _step_planned(self, x_incr):
         return self._step_planned_pass(x_incr)
 

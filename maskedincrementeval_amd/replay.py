@@ -33,7 +33,7 @@ from . import _lib
 from ._lib import check
 
 enabled = os.environ.get("MIE_REPLAY", "1") != "0"      # read once
-MAX_RECORDINGS = 8          # per module and method, least recently used first out
+MAX_RECORDINGS = 8          # per module, least recently used first out
 _epoch = [0]
 _recording = {}             # thread identity -> the Recording that thread is making
 _SILENT = frozenset(("training", "states"))     # assignments no incremental pass depends on
@@ -245,6 +245,7 @@ class Program:
     def __init__(self, rec, inputs, result, tree, static):
         self.effects, self.result = rec.effects, result
         self.runs = 0
+        self.plan_masks = []         # (op of a plan, its field, input): set before each run
         self.held = [[k for k in rec.keep if not (torch.is_tensor(k) and inputs.holds(k))], static]
         calls = (_lib.MieCall * len(rec.calls))()
         for call, (name, args) in zip(calls, rec.calls):
@@ -257,10 +258,16 @@ class Program:
                     inputs.refuse("an input is written", words[i])
                 elif kind == "t" and args[i] is not None:
                     inputs.refuse_set(args[i]._obj)
-                elif isinstance(args[i], ctypes.Array):          # the ops of a plan
-                    for op in args[i]:
-                        inputs.refuse("an input inside a plan", op.in_mask, op.in_mask2)
+                elif isinstance(args[i], ctypes.Array):          # the ops of a plan: this program's own array of them
+                    plan = type(args[i]).from_buffer_copy(args[i])
+                    words[i] = _word(kind, plan, self.held)
+                    for op in plan:
                         inputs.refuse_set(op.out)
+                        for field in ("in_mask", "in_mask2"):
+                            address = getattr(op, field)
+                            slot = inputs.slot(address) if address else None
+                            if slot is not None:
+                                self.plan_masks.append((op, field, slot))
                 elif kind == "r" and words[i]:
                     slot = inputs.slot(words[i])
                     if slot is not None:
@@ -310,6 +317,8 @@ class Program:
 
     def run(self, pointers, device):
         self.runs += 1
+        for op, field, slot in self.plan_masks:
+            setattr(op, field, pointers[slot])
         check(self.fn(self.calls, self.n, self.words_type(*pointers), self.n_inputs,
                       torch._C._cuda_getCurrentRawStream(device)))
         for fn, args in self.effects:
@@ -322,7 +331,24 @@ class _NotRecordable(Exception):
 
 
 class _Cache(collections.OrderedDict):
-    """Recordings of one module, by method and input.  Copies and pickles of a module start without any."""
+    """Recordings of one module, by method and input.  Copies and pickles of a module start without any.  `waiting`: the
+    passes that have none (yet), apart, so that inputs that are never seen again push no recording out."""
+
+    def __init__(self):
+        super().__init__()
+        self.waiting = collections.OrderedDict()
+
+    def keep(self, key, entry):
+        if type(entry) is Program:
+            self.waiting.pop(key, None)
+            while len(self) >= MAX_RECORDINGS and key not in self:
+                self.popitem(last=False)
+            self[key] = entry
+        else:
+            self.pop(key, None)
+            while len(self.waiting) >= MAX_RECORDINGS:
+                self.waiting.popitem(last=False)
+            self.waiting[key] = entry
 
     def __deepcopy__(self, memo):
         return _Cache()
@@ -381,10 +407,10 @@ def _is_nhwc(t) -> bool:
             and t.is_contiguous(memory_format=torch.channels_last))
 
 
-def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
+def replayed(record=None, dense=0, masked=1, trees=()):
     """Decorator of a pass: method(self, *args).  The first `dense` arguments are dense tensors and the next `masked`
-    ones Masked pairs (or None); those may live anywhere, everything else has to be the same object or memory to be
-    the same pass.  free_masks: plain mask tensors of the pairs may live anywhere, too.  trees: positions of further
+    ones Masked pairs (or None); those and plain mask tensors of the pairs may live anywhere, everything else has to be
+    the same object or memory to be the same pass.  trees: positions of further
     arguments that are modules the pass reads.  record: name of another method to record in place of this one, tried
     first, with the same result (ValueDependentMask: it does not apply)."""
     def decorate(method):
@@ -407,12 +433,9 @@ def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
                         if (m.dtype not in (torch.uint8, torch.bool) or m.shape != (n, 1, h, w) or not m.is_contiguous()
                                 or m.device != x.device):
                             return method(self, *args)
-                        if free_masks:
-                            pointers.append(m.data_ptr())
-                            free.append((i, 1))
-                            key.append("mask")
-                        else:
-                            key.append(m.data_ptr())
+                        pointers.append(m.data_ptr())
+                        free.append((i, 1))
+                        key.append(m.dtype)
                     else:
                         key.append(_static_key(m, held))
                 else:
@@ -424,19 +447,21 @@ def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
             if cache is None:
                 cache = self.__dict__["_replay"] = _Cache()
             ent = cache.get(key)
-            if type(ent) is Program:
+            if ent is not None:
                 if ent.valid():
                     cache.move_to_end(key)
                     return ent.run(pointers, key[3])
                 # outdated: recorded anew at the next pass, or later and later if recordings here never last
-                w = cache[key] = _Waiting()
+                w = _Waiting()
                 if ent.runs < 16:
                     w.step = w.next = ent.step
+                cache.keep(key, w)
                 ent = w
-            if ent is None:
-                while len(cache) >= MAX_RECORDINGS:
-                    cache.popitem(last=False)
-                ent = cache[key] = _Waiting()
+            else:
+                ent = cache.waiting.get(key)
+                if ent is None:
+                    ent = _Waiting()
+                    cache.keep(key, ent)
             ent.seen += 1
             if ent.seen < ent.next or torch.cuda.is_current_stream_capturing():
                 return method(self, *args)
@@ -448,7 +473,7 @@ def replayed(record=None, dense=0, masked=1, free_masks=True, trees=()):
             result, program = _record(fns, args, free, (self,) + tuple(args[i] for i in trees), held)
             if program is not None:
                 program.step = ent.step
-                cache[key] = program
+                cache.keep(key, program)
             return result
         return wrapped
     return decorate

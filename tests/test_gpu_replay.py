@@ -147,3 +147,24 @@ def test_recorded_layers_equal_walked_layers(dtype, mask):
                     masks.append(None if mask is None else m.bool() if mask == "bool" else m)
             _equal(step(a, d, masks[0]), _walked(step, b, d, masks[1]))
     assert all(_programs(m) for m in (a[0], a[2])) and not _programs(b[0])
+
+
+@pytest.mark.parametrize("net,dtype", [("e2depth", torch.float32), ("e2depth", torch.bfloat16), ("transposed", torch.float32), ("upsample", torch.float32)])
+def test_recorded_steps_read_the_mask_of_the_pass_at_hand(net, dtype):
+    """A mask of the caller's in a new allocation each step, of changing kind and content: the plan of the recording builds
+    its sets from it."""
+    h, w, bins = (48, 80, 5) if net == "e2depth" else (64, 96, 4)
+    make = E2VIDRecurrentIncr if net == "e2depth" else (lambda: MultiResUNetRecurrentIncr(num_bins=4, decoder=net))
+    a, b = (seed_module_(make(), seed=3).to(DEV).eval() for _ in range(2))
+    extra = (None,) if net == "e2depth" else ()
+    alive = []
+    with torch.no_grad():
+        for n in (a, b):
+            n.forward_refresh_reservoirs(_cl(torch.ones(1, bins, h, w), dtype), *extra)
+        for i in range(9):
+            d, m = event_voxel_delta(1, bins, h, w, 0.02 + 0.04 * (i % 3), seed=140 + i)
+            d, m = _cl(d, dtype), m.to(DEV).view(1, 1, h, w)
+            m = m.bool() if i % 2 else m.to(torch.uint8)
+            alive.append((d, m))
+            _equal(a([d, m], *extra), _walked(b, [d, m], *extra))
+    assert sorted(p.runs for p in _programs(a)) == [1, 2] and not _programs(b)

@@ -11,6 +11,7 @@ import torch
 
 from maskedincrementeval_amd import _lib, ops, replay
 from maskedincrementeval_amd import mask_incr_modules as mm
+from maskedincrementeval_amd.e2depth_incr import E2VIDRecurrentIncr
 
 
 class StubLib:
@@ -183,3 +184,43 @@ def test_a_planning_pass_asks_the_library_for_its_shapes(stub):
     for phase in (None, "plan", "compute"):
         with ops.network_pass(phase):
             assert ops.f32x3_takes(5, 1, 256, 0, 128), phase
+
+
+def _network():
+    net = E2VIDRecurrentIncr().eval()
+    x = _cl(1, 5, 16, 16)
+    for _ in range(4):
+        net.forward_refresh_reservoirs(x, None)
+    return net, x
+
+
+def test_a_mask_of_the_callers_may_lie_anywhere(stub):
+    """Steps whose mask is a new tensor each time: recorded once, and the plan reads the mask of the pass at hand."""
+    with torch.no_grad():
+        net, _ = _network()
+        for i in range(8):
+            m = torch.ones(1, 1, 16, 16, dtype=torch.bool if i % 2 else torch.uint8)
+            x = _cl(1, 5, 16, 16)
+            del stub.calls[:]
+            net([x, m], None)
+            if i < 6:
+                continue
+            (plan,) = stub.named("mie_build_mask_plan")
+            arr = ctypes.cast(plan[0], ctypes.POINTER(_lib.MiePlanOp))
+            assert m.data_ptr() in [arr[k].in_mask for k in range(plan[1])]
+            assert stub.named("mie_conv_masked_ws")[0][:2] == [x.data_ptr(), m.data_ptr()]
+    assert sorted(p.runs for p in _programs(net)) == [1, 1, 1]      # two kinds of mask, and the refresh
+
+
+def test_inputs_never_seen_again_push_no_recording_out(stub):
+    with torch.no_grad():
+        net, x = _network()
+        assert [p.runs for p in _programs(net)] == [1]
+        alive = []
+        for _ in range(3 * replay.MAX_RECORDINGS):
+            states = [[_cl(1, c, s, s)] * 2 for c, s in ((64, 8), (128, 4), (256, 2))]
+            net([x, None], [[[h, None], [c, None]] for h, c in states])
+            alive.append(states)
+        net.forward_refresh_reservoirs(x, None)
+    assert [p.runs for p in _programs(net)] == [2]
+    assert len(net.__dict__["_replay"].waiting) <= replay.MAX_RECORDINGS
