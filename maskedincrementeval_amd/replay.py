@@ -8,8 +8,8 @@ therefore recorded (`Recording`: every call of the library with its arguments), 
 to mie_run_calls with the pointers of their inputs filled in -- about 3 us a call, the launch itself.
 
 A recording stands for the Python pass as long as everything that pass read is what it was:
-  * attributes of the package's modules and which reservoir tensor an IncrementReserve holds: any assignment bumps
-    `_epoch` (`Watched`);
+  * attributes of the package's modules it went through and which reservoir tensor an IncrementReserve of theirs holds:
+    an assignment ends the recordings that read the object, and what they hold is freed (`Watched`);
   * weights: the parameter objects, their addresses and version counters;
   * the settings and functions of `ops` (a program or a test that replaces one gets its calls);
   * forward hooks, and the members of module containers.
@@ -25,6 +25,7 @@ import operator
 import os
 import struct
 import threading
+import weakref
 
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -34,22 +35,50 @@ from ._lib import check
 
 enabled = os.environ.get("MIE_REPLAY", "1") != "0"      # read once
 MAX_RECORDINGS = 8          # per module, least recently used first out
-_epoch = [0]
 _recording = {}             # thread identity -> the Recording that thread is making
 _SILENT = frozenset(("training", "states"))     # assignments no incremental pass depends on
 
 
+class _Readers(list):
+    """Weak references to the programs that read an object.  Copies and pickles of the object start without any."""
+
+    def __deepcopy__(self, memo):
+        return _Readers()
+
+    def __reduce__(self):
+        return _Readers, ()
+
+
 class Watched:
-    """First base of the package's modules and reservoirs: assignments to attributes outdate the recordings."""
+    """First base of the package's modules and reservoirs: an assignment to an attribute ends the programs that read the
+    object, before the attribute changes."""
 
     def __setattr__(self, name, value):
         if name not in _SILENT:
-            _epoch[0] += 1
+            outdate(self)
         super().__setattr__(name, value)
 
     def __delattr__(self, name):
-        _epoch[0] += 1
+        outdate(self)
         super().__delattr__(name)
+
+
+def outdate(obj):
+    for ref in obj.__dict__.pop("_replay_readers", ()):
+        program = ref()
+        if program is not None:
+            program.end()
+
+
+def _watched_in(modules):
+    """The watched objects a pass over these modules reads: themselves, and the reservoirs they hold."""
+    found = {}
+    for m in modules:
+        for x in [m, *vars(m).values()]:
+            for y in (x if type(x) in (list, tuple) else (x,)):
+                if isinstance(y, Watched):
+                    found[id(y)] = y
+    return found.values()
 
 
 class ValueDependentMask(RuntimeError):
@@ -244,7 +273,7 @@ class Program:
 
     def __init__(self, rec, inputs, result, tree, static):
         self.effects, self.result = rec.effects, result
-        self.runs = 0
+        self.runs, self.alive = 0, True
         self.plan_masks = []         # (op of a plan, its field, input): set before each run
         self.held = [[k for k in rec.keep if not (torch.is_tensor(k) and inputs.holds(k))], static]
         calls = (_lib.MieCall * len(rec.calls))()
@@ -288,7 +317,6 @@ class Program:
         for m in tree:
             mods.extend(m.modules())
         mods = list({id(m): m for m in mods}.values())
-        self.epoch = _epoch[0]
         self.settings = _get_settings(_ops_globals)
         self.hooks = [d for m in mods for d in (m._forward_hooks, m._forward_pre_hooks)]
         self.hooks += [torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks]
@@ -306,9 +334,19 @@ class Program:
         self.tensors = [p for p in self.params if p is not None]
         self.addresses = [p.data_ptr() for p in self.tensors]
         self.versions = [p._version for p in self.tensors]
+        me = weakref.ref(self)
+        for w in _watched_in(mods):
+            readers = w.__dict__.setdefault("_replay_readers", _Readers())
+            readers[:] = [r for r in readers if r() is not None] + [me]
+
+    def end(self):
+        """Never valid again; lets go of everything it held."""
+        self.alive = False
+        self.held = self.effects = self.result = self.calls = None
+        self.plan_masks, self.tensors, self.params, self.param_dicts, self.members, self.containers = [], [], [], [], [], []
 
     def valid(self) -> bool:
-        return (self.epoch == _epoch[0] and _get_settings(_ops_globals) == self.settings and not any(self.hooks)
+        return (self.alive and _get_settings(_ops_globals) == self.settings and not any(self.hooks)
                 and [p.data_ptr() for p in self.tensors] == self.addresses
                 and [p._version for p in self.tensors] == self.versions
                 and all(map(operator.is_, [p for d in self.param_dicts for p in d.values()], self.params))
@@ -317,13 +355,13 @@ class Program:
 
     def run(self, pointers, device):
         self.runs += 1
+        calls, effects, result = self.calls, self.effects, self.result
         for op, field, slot in self.plan_masks:
             setattr(op, field, pointers[slot])
-        check(self.fn(self.calls, self.n, self.words_type(*pointers), self.n_inputs,
-                      torch._C._cuda_getCurrentRawStream(device)))
-        for fn, args in self.effects:
+        check(self.fn(calls, self.n, self.words_type(*pointers), self.n_inputs, torch._C._cuda_getCurrentRawStream(device)))
+        for fn, args in effects:
             fn(*args)
-        return _copy(self.result)
+        return _copy(result)
 
 
 class _NotRecordable(Exception):

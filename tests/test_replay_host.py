@@ -1,7 +1,9 @@
 """Recorded passes on the host side, without a GPU: the library is a stub that notes its calls and runs recorded sequences
 by reading their words, so what a recording holds and when it is used can be looked at call by call."""
+import copy
 import ctypes
 import gc
+import pickle
 import threading
 import weakref
 from types import SimpleNamespace
@@ -11,6 +13,7 @@ import torch
 
 from maskedincrementeval_amd import _lib, ops, replay
 from maskedincrementeval_amd import mask_incr_modules as mm
+from maskedincrementeval_amd.mask_incr_functional import IncrementReserve
 from maskedincrementeval_amd.e2depth_incr import E2VIDRecurrentIncr
 
 
@@ -224,3 +227,46 @@ def test_inputs_never_seen_again_push_no_recording_out(stub):
         net.forward_refresh_reservoirs(x, None)
     assert [p.runs for p in _programs(net)] == [2]
     assert len(net.__dict__["_replay"].waiting) <= replay.MAX_RECORDINGS
+
+
+def _step(net, size=16):
+    net([_cl(1, 5, size, size), None], None)
+
+
+def test_an_assignment_ends_the_recordings_that_read_the_object_and_no_other(stub):
+    with torch.no_grad():
+        a, b = (_network()[0] for _ in range(2))
+        layer, act = _conv()
+        for _ in range(4):
+            _step(a), _step(b)
+            layer.forward_fused([_cl(1, 8, 8, 8), None], act)
+        mm.set_input_threshold(b, None)
+        act.in_res.reservoir = _cl(1, 8, 8, 8)
+        assert [p.valid() for p in _programs(a)] == [True, True]
+        assert [p.valid() for p in _programs(b)] == [False, False]
+        assert [p.valid() for p in _programs(layer)] == [False]
+        for change in (lambda n: setattr(n.unetrecurrent.decoders[1].activation, "op", torch.tanh),
+                       lambda n: setattr(n.unetrecurrent.encoders[0].recurrent_block.cell_res, "reservoir", None),
+                       lambda n: delattr(n.unetrecurrent.head.conv2d, "path")):
+            net = _network()[0]
+            [_step(net) for _ in range(4)]
+            assert all(p.valid() for p in _programs(net)) and len(_programs(net)) == 2
+            change(net)
+            assert not any(p.valid() for p in _programs(net))
+
+
+def test_a_new_frame_size_frees_the_reservoirs_of_the_former_one(stub):
+    with torch.no_grad():
+        net, _ = _network()
+        [_step(net) for _ in range(5)]
+        reserves = [r for m in net.modules() for r in vars(m).values() if isinstance(r, IncrementReserve)]
+        old = [weakref.ref(r.reservoir) for r in reserves if r.reservoir is not None]
+        assert len(old) > 10
+        net.forward_refresh_reservoirs(_cl(1, 5, 32, 32), None)
+        assert not any(r() is not None for r in old)
+        [_step(net, 32) for _ in range(4)]
+    res = net.unetrecurrent.head.activation.in_res           # (what notes its readers stays copyable)
+    for twin in (copy.deepcopy(res), pickle.loads(pickle.dumps(res))):
+        assert torch.equal(twin.reservoir, res.reservoir)
+        twin.reservoir = None
+    assert all(p.valid() for p in _programs(net)[-1:])
