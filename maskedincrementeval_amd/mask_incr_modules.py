@@ -25,7 +25,7 @@ from .mask_incr_functional import (IncrPointwiseMultiply, IncrementReserve, _squ
                                    bn2d_from_module, bn_scale, conv2d_from_module)
 
 
-class _IncrBuffers:
+class _IncrBuffers(metaclass=replay.WatchedType):
     """Persistent per-module device buffers of the incremental path.
 
     Deltas written by the kernels live in fixed buffers (stable pointers, zero
@@ -765,7 +765,7 @@ class nnAdaptiveAvgPool2dIncr(replay.Watched, nn.AdaptiveAvgPool2d):
         return super().forward(x)
 
 
-class nnSequentialIncr(nn.Sequential):
+class nnSequentialIncr(replay.Watched, nn.Sequential):
     """Reference :236-240."""
 
     def forward_refresh_reservoirs(self, x):

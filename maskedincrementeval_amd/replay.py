@@ -12,12 +12,14 @@ A recording stands for the Python pass as long as everything that pass read is w
     an assignment ends the recordings that read the object, and what they hold is freed (`Watched`);
   * weights: the parameter objects, their addresses and version counters;
   * the settings and functions of `ops` (a program or a test that replaces one gets its calls);
-  * forward hooks, and the members of module containers.
+  * the package's module classes (a method replaced by an instrumented one gets its calls), forward hooks, and the
+    members of module containers.
 Otherwise the pass runs in Python again and is recorded anew.  A pass that runs any torch operation of its own
 (a conversion, a concat, the allocation of a buffer) is never recorded, nor one on a planning stream or inside a
 planning pass, nor under graph capture.  It is recorded on copies of its inputs, so that what is an input is known by
 its address.  Recordings hold references to every tensor whose address they use.
 """
+import abc
 import collections
 import ctypes
 import functools
@@ -49,7 +51,45 @@ class _Readers(list):
         return _Readers, ()
 
 
-class Watched:
+# attributes that Python itself puts on classes (copying an object adds __slotnames__)
+_NOT_CODE = frozenset(("__abstractmethods__", "__annotations__", "__doc__", "__dict__", "__weakref__", "__slotnames__"))
+
+
+class WatchedType(abc.ABCMeta):
+    """Class of the package's module classes and mixins: notes when an attribute of one is replaced, whoever does it.  (Of
+    ABCMeta, so that a caller's subclass may be an abstract one, too.)"""
+    changes = 0              # replacements so far, of all classes
+    defined = {}             # class -> its attributes as they were written
+
+    def __init__(cls, *args, **kw):
+        super().__init__(*args, **kw)
+        if cls.__module__.split(".")[0] == __package__:
+            WatchedType.defined[cls] = WatchedType.code_of(cls)
+
+    def code_of(cls):
+        return {k: v for k, v in vars(cls).items() if k not in _NOT_CODE and not k.startswith("_abc_")}
+
+    def __setattr__(cls, name, value):
+        if name not in _NOT_CODE:
+            WatchedType.changes += 1
+        super().__setattr__(name, value)
+
+    def __delattr__(cls, name):
+        WatchedType.changes += 1
+        super().__delattr__(name)
+
+    def as_written(cls):
+        """Whether this class and the package's classes it comes from are what their sources say."""
+        for c in cls.__mro__:
+            was = WatchedType.defined.get(c)
+            if was is not None:
+                now = WatchedType.code_of(c)
+                if now.keys() != was.keys() or any(now[k] is not was[k] for k in was):
+                    return False
+        return True
+
+
+class Watched(metaclass=WatchedType):
     """First base of the package's modules and reservoirs: an assignment to an attribute ends the programs that read the
     object, before the attribute changes."""
 
@@ -320,13 +360,17 @@ class Program:
         self.settings = _get_settings(_ops_globals)
         self.hooks = [d for m in mods for d in (m._forward_hooks, m._forward_pre_hooks)]
         self.hooks += [torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks]
-        if any(self.hooks) or any("forward" in m.__dict__ for m in mods):
-            raise _NotRecordable("hooked")
-        self.classes = sorted({type(m) for m in mods}, key=lambda c: c.__qualname__)
-        for c in self.classes:
+        if any(self.hooks) or any(callable(getattr(type(m), k, None)) for m in mods for k in m.__dict__):
+            raise _NotRecordable("hooked, or a method replaced in an object")
+        classes = {type(m) for m in mods}
+        for c in classes:
             if c.__module__.split(".")[0] not in (__package__, "torch"):
                 raise _NotRecordable("a class of the caller's")
-        self.forwards = [c.forward for c in self.classes]
+            if isinstance(c, WatchedType) and not c.as_written():
+                raise _NotRecordable("a class with something replaced")
+        self.changes = WatchedType.changes
+        self.torch_classes = [c for c in classes if not isinstance(c, WatchedType)]
+        self.forwards = [c.forward for c in self.torch_classes]
         self.containers = [m._modules for m in mods if m._modules]
         self.members = [list(d.values()) for d in self.containers]
         self.param_dicts = [m._parameters for m in mods if m._parameters]
@@ -346,12 +390,12 @@ class Program:
         self.plan_masks, self.tensors, self.params, self.param_dicts, self.members, self.containers = [], [], [], [], [], []
 
     def valid(self) -> bool:
-        return (self.alive and _get_settings(_ops_globals) == self.settings and not any(self.hooks)
+        return (self.alive and self.changes == WatchedType.changes and _get_settings(_ops_globals) == self.settings and not any(self.hooks)
                 and [p.data_ptr() for p in self.tensors] == self.addresses
                 and [p._version for p in self.tensors] == self.versions
                 and all(map(operator.is_, [p for d in self.param_dicts for p in d.values()], self.params))
                 and [list(d.values()) for d in self.containers] == self.members
-                and [c.forward for c in self.classes] == self.forwards)
+                and [c.forward for c in self.torch_classes] == self.forwards)
 
     def run(self, pointers, device):
         self.runs += 1

@@ -1,5 +1,6 @@
 """Recorded passes on the host side, without a GPU: the library is a stub that notes its calls and runs recorded sequences
 by reading their words, so what a recording holds and when it is used can be looked at call by call."""
+import abc
 import copy
 import ctypes
 import gc
@@ -270,3 +271,47 @@ def test_a_new_frame_size_frees_the_reservoirs_of_the_former_one(stub):
         assert torch.equal(twin.reservoir, res.reservoir)
         twin.reservoir = None
     assert all(p.valid() for p in _programs(net)[-1:])
+
+
+@pytest.mark.parametrize("cls,name", [(mm.nnConvIncr, "_incr_forward"), (mm.nnConvIncr, "lossy_input"), (mm._IncrBuffers, "_delta_buf"),
+                                      (mm._ConvIncrMixin, "_conv_tile_set"), (mm.nnReluIncr, "forward")])
+def test_a_replaced_method_gets_its_calls(stub, monkeypatch, cls, name):
+    """Also one that recordings do not go through by name, a mixin's, and one set on a class that inherited it."""
+    with torch.no_grad():
+        net, layer = _network()[0], mm.nnConvIncr(8, 8, 3, 1, 1)
+        one = lambda: (_step(net), layer([_cl(1, 8, 8, 8), None]))
+        [one() for _ in range(5)]
+        assert all(len(_programs(m)) and all(p.valid() for p in _programs(m)) for m in (net, layer))
+        seen, real = [], getattr(cls, name)
+        inherited = name not in vars(cls)
+        with monkeypatch.context() as patch:
+            patch.setattr(cls, name, lambda self, *args, **kw: (seen.append(1), real(self, *args, **kw))[1])
+            for _ in range(6):
+                del seen[:]
+                one()
+                assert seen or cls is mm.nnReluIncr
+            assert not any(p.valid() for p in _programs(net))
+        assert (name in vars(cls)) != inherited
+        before = len(stub.named("mie_conv_masked_ws"))
+        for _ in range(40):
+            one()
+        assert any(p.valid() for p in _programs(net)) and len(stub.named("mie_conv_masked_ws")) > before
+
+
+def test_a_method_replaced_in_an_object_gets_its_calls(stub):
+    with torch.no_grad():
+        net, _ = _network()
+        [_step(net) for _ in range(5)]
+        conv, seen = net.unetrecurrent.resblocks[0].conv1, []
+        real = conv._incr_forward
+        conv._incr_forward = lambda *args, **kw: (seen.append(1), real(*args, **kw))[1]
+        for _ in range(8):
+            del seen[:]
+            _step(net)
+            assert seen
+
+
+def test_a_subclass_of_a_module_may_be_abstract():
+    class Mine(mm.nnConvIncr, abc.ABC):
+        pass
+    assert Mine(4, 4, 3).weight.shape == (4, 4, 3, 3)
