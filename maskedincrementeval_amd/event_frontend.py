@@ -57,9 +57,7 @@ class EventFrames:
         self._sums = ops.new_nhwc(1, self.channels, self.out_h, self.out_w, self.device) if dtype != torch.float32 else None
         self._mask = torch.zeros((1, 1, self.out_h, self.out_w), dtype=torch.uint8, device=self.device)
         self._fmask = torch.zeros_like(self._mask)
-        self._at = None                               # device pointer of the events
         self._geometry = (self.kind, self.num_bins, self.height, self.width) + self.pad
-        self._pointers = None
 
     def set_events(self, events) -> int:
         """events: (n, 4) array-like of (t, x, y, p), float64, covering every window asked for
@@ -69,29 +67,29 @@ class EventFrames:
             raise ValueError("events must be float64 of shape (n, 4), got %s %s" % (tuple(ev.shape), ev.dtype))
         self._events = ev.contiguous().to(self.device)
         self._n = int(ev.shape[0])
-        self._at = self._events.data_ptr() if self._n else None
         return self._n
 
     def _run(self, start_old, start_new, delta, out, mask):
         if self._events is None:
             raise RuntimeError("EventFrames: call set_events first")
-        # (a call is as long on the host as its kernels are on the GPU: what stays the same between calls -- every buffer
-        # here is this object's own -- is looked up once)
-        if self._pointers is None:
-            self._pointers = {"_frame": ops.nhwc_ptr(self._frame, "frame", dtype=self.dtype), "_fmask": self._fmask.data_ptr(),
-                              "_delta": ops.nhwc_ptr(self._delta, "delta", dtype=self.dtype), "_mask": self._mask.data_ptr()}
-            self._to_frame = lib().mie_events_to_frame if self._sums is None else lib().mie_events_to_frame_bf16
-        at = (self._pointers[out], self._pointers[mask])
-        check(self._to_frame(self._at, self._n, *self._geometry, self.t_scale, float(start_old), float(start_new),
-                             self.window_size, 1 if delta else 0, *(at if self._sums is None else (self._sums.data_ptr(),) + at),
-                             torch._C._cuda_getCurrentRawStream(self._mask.device.index)))
+        # (a call is as long on the host as its kernels are on the GPU; the buffers are this object's own and were made in
+        # the layout the entry points take, so they are not checked again.  No address is kept: a copy of this object has
+        # buffers of its own.)
+        at = (out.data_ptr(), mask.data_ptr())
+        if self._sums is None:
+            to_frame = lib().mie_events_to_frame
+        else:
+            to_frame, at = lib().mie_events_to_frame_bf16, (self._sums.data_ptr(),) + at
+        check(to_frame(self._events.data_ptr() if self._n else None, self._n, *self._geometry, self.t_scale, float(start_old),
+                       float(start_new), self.window_size, 1 if delta else 0, *at,
+                       torch._C._cuda_getCurrentRawStream(mask.device.index)))
 
     def frame(self, start: float) -> torch.Tensor:
         """Dense (1, C, H', W') channels_last frame of the window (start, start + window_size)."""
-        self._run(0.0, start, False, "_frame", "_fmask")
+        self._run(0.0, start, False, self._frame, self._fmask)
         return self._frame
 
     def delta(self, start_old: float, start_new: float) -> Tuple[torch.Tensor, torch.Tensor]:
         """[frame(start_new) - frame(start_old), pixel mask of the touched pixels]."""
-        self._run(start_old, start_new, True, "_delta", "_mask")
+        self._run(start_old, start_new, True, self._delta, self._mask)
         return [self._delta, self._mask]

@@ -14,6 +14,7 @@ import torch
 
 from maskedincrementeval_amd import _lib, ops, replay
 from maskedincrementeval_amd import mask_incr_modules as mm
+from maskedincrementeval_amd.event_frontend import EventFrames
 from maskedincrementeval_amd.mask_incr_functional import IncrementReserve
 from maskedincrementeval_amd.e2depth_incr import E2VIDRecurrentIncr
 
@@ -315,3 +316,17 @@ def test_a_subclass_of_a_module_may_be_abstract():
     class Mine(mm.nnConvIncr, abc.ABC):
         pass
     assert Mine(4, 4, 3).weight.shape == (4, 4, 3, 3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_event_frames_are_copied_with_buffers_of_their_own(stub, dtype):
+    frames = EventFrames(20, 12, device="cpu", dtype=dtype)
+    frames.set_events(torch.zeros(3, 4, dtype=torch.float64))
+    entry = "mie_events_to_frame" if dtype == torch.float32 else "mie_events_to_frame_bf16"
+    frames.delta(0.0, 0.1)
+    for twin in (copy.deepcopy(frames), pickle.loads(pickle.dumps(frames))):
+        del stub.calls[:]
+        out, mask = twin.delta(0.0, 0.1)
+        (args,) = stub.named(entry)
+        assert args[0] == twin._events.data_ptr() != frames._events.data_ptr()
+        assert args[-3:-1] == (out.data_ptr(), mask.data_ptr()) and out.data_ptr() != frames._delta.data_ptr()
