@@ -304,7 +304,8 @@ int mie_conv_masked(const void* x, const uint8_t* xmask, int c1,
  *        least 2 planes of n*h*w*cout floats (8 MiB covers 8 planes of every
  *        shape that qualifies); otherwise the workspace is not touched.
  *        Its contents are scratch: undefined after the call, and calls that
- *        share one workspace must be ordered (same stream).
+ *        share one workspace must be ordered (same stream; several threads
+ *        may enqueue on it, the launches of a call stay together).
  * Has no counterpart in the reference, whose convs run as one launch of
  * whatever size (ext/pointops/_C_ext/pointops/ext_conv.cu:74-76).
  */

@@ -62,10 +62,12 @@ template <typename... A, int (*Fn)(A...)> struct Entry<Fn> {
   }
   static int call(const uint64_t* w, void* stream) { return run(w, stream, std::make_index_sequence<sizeof...(A)>{}); }
   static const char* sig() {
-    static const char s[] = {Word<A>::kind..., 0};
-    static char cut[kMaxArgs + 2];
-    memcpy(cut, s, n);
-    return cut;
+    struct Cut {
+      char s[kMaxArgs + 2] = {Word<A>::kind..., 0};
+      Cut() { s[n] = 0; }
+    };
+    static const Cut cut;
+    return cut.s;
   }
 };
 

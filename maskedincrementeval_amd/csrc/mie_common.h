@@ -5,6 +5,8 @@
 #include <stdio.h>
 #include <stdarg.h>
 
+#include <mutex>
+
 // The C ABI is the only thing exported from the library.
 #pragma GCC visibility push(default)
 #include "../../include/mie.h"
@@ -34,6 +36,14 @@ static __device__ __forceinline__ void mie_st4(mie_bf16* p, long long i, const f
   mie_bf16x4 b;
   b[0] = (mie_bf16)v.x; b[1] = (mie_bf16)v.y; b[2] = (mie_bf16)v.z; b[3] = (mie_bf16)v.w;
   *reinterpret_cast<mie_bf16x4*>(p + i) = b;
+}
+
+// ---- host side: launches that share a workspace ----------------------------
+// The two launches of a split form belong together: between them the workspace holds the partial sums.  Threads that
+// enqueue on one stream with one workspace take turns pair by pair (the lock is held while two launches are enqueued).
+inline std::mutex& mie_split_launches() {
+  static std::mutex m;
+  return m;
 }
 
 // ---- host side: error reporting -------------------------------------------

@@ -1226,6 +1226,7 @@ bool launch_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   const int parts = split_parts(a, (long long)cap * (a0.cout / 32), (a0.c1 + a0.c2) / CC);
   if (parts == 0) return false;
   const dim3 grid(cap, a.cout / 32, parts);
+  const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
     if constexpr (HAS_X3) hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true, true>), grid, dim3(256), 0, st, a);
   } else {
@@ -1246,6 +1247,7 @@ bool launch_up_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   if (parts == 0) return false;
   bool x3 = false;
   if constexpr (sizeof(T) == 4) x3 = a.x3 != 0;
+  const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
     if constexpr (sizeof(T) == 4)
       hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true, true>), dim3(cap, a.cout / 32, parts), dim3(256), 0, st, a);
@@ -1269,6 +1271,7 @@ bool launch_gates_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   if (parts < 4) return false;
   bool x3 = false;
   if constexpr (sizeof(T) == 4) x3 = a.x3 != 0;
+  const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
     if constexpr (sizeof(T) == 4)
       hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true, true>), dim3(cap, a.cout / 32, parts), dim3(256), 0, st, a);

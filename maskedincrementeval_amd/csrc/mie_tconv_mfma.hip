@@ -326,6 +326,7 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
     while (2 * parts <= 8 && 2 * parts <= nch && groups * (2 * parts) <= 256 && (long long)(2 * parts) * a.ws_plane <= a.ws_floats)
       parts *= 2;
     if (parts >= 2) {
+      const std::lock_guard<std::mutex> pair(mie_split_launches());
       hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, true, X3>), dim3(cap_p, cout / 32, parts), dim3(256), 0, st, a, pts);
       unsigned ny = (unsigned)((1024 + cap_out - 1) / cap_out);
       if (ny > (unsigned)(cout / 4)) ny = (unsigned)(cout / 4);

@@ -29,6 +29,7 @@ class _PassState(threading.local):
     plan_wgs = 0             # workgroup limit of the plan being made (0: the library's own)
     buffer_parity = 0        # generation of tile sets and delta buffers (planning one step ahead, below)
     planner = None           # (side stream, device) inside a mask_planner block
+    workspace = None         # the shared split workspace used last
 
     def __init__(self):
         self.pix_ready = {}      # data_ptr of a pixel mask written on the compute stream -> event
@@ -727,26 +728,51 @@ def _filter_args(filt, k, dtype=torch.float32, x3_shape=None, with_code=False):
 # Workspace of the matrix-core conv for planes of very few tiles (a 16x16 plane is 4 tiles, 64 workgroups
 # for 512 channels): the library then splits the contraction over up to 8 workgroups per (tile, slab) and
 # needs room for their partial sums.  A launch is split only up to 128 workgroups, i.e. up to 4096
-# tile-channels, so 8 planes of 4096 * 64 floats (8 MiB) cover every case.  One buffer per device: the
-# convs of a device are taken to run on one stream at a time; callers that run convs concurrently on
-# several streams pass buffers of their own (`workspace=`), or False for none.
+# tile-channels, so 8 planes of 4096 * 64 floats (8 MiB) cover every case.  One buffer per stream: launches of one stream
+# run in order and the two launches of a split form stay together (mie_split_launches), so threads may share a stream.  The
+# SPLIT_WORKSPACES newest are kept (a thread holds on to the one it is using); one that goes back to the allocator is
+# handed out again in the order of its stream.  Launches under graph capture have a buffer of their own, one per device and kept for good, since
+# graphs hold its address: graphs with split launches are taken to replay one at a time; a caller that replays them on
+# several streams at once passes buffers of its own while capturing (`workspace=`), or False for none.
 SPLIT_WORKSPACE_BYTES = 8 * 4096 * 64 * 4
+SPLIT_WORKSPACES = 16
 split_enabled = True
-_split_ws = {}
+_split_ws = {}              # (device index, raw stream) -> buffer, oldest first
+_captured_ws = {}           # device index -> buffer
+_split_ws_lock = threading.Lock()
 
 
 def split_workspace(device):
-    ws = _split_ws.get(device)
-    if ws is None:
-        ws = _split_ws[device] = torch.empty(SPLIT_WORKSPACE_BYTES // 4, dtype=torch.float32, device=device)
-    return ws
+    """The split workspace of the current stream of `device` (a torch.device or an index)."""
+    dev = device if isinstance(device, int) else device.index
+    if dev is None:
+        dev = torch.cuda.current_device()
+    capturing = torch.cuda.is_current_stream_capturing()
+    ws = _captured_ws.get(dev) if capturing else _split_ws.get((dev, torch._C._cuda_getCurrentRawStream(dev)))
+    return ws if ws is not None else _new_split_workspace(dev, capturing)
+
+
+def _new_split_workspace(dev, capturing):
+    new = lambda: torch.empty(SPLIT_WORKSPACE_BYTES // 4, dtype=torch.float32, device=torch.device("cuda", dev))
+    with _split_ws_lock:
+        if dev not in _captured_ws:          # made with the first of the device, so that a capture allocates nothing
+            _captured_ws[dev] = new()
+        if capturing:
+            return _captured_ws[dev]
+        while len(_split_ws) >= SPLIT_WORKSPACES:
+            del _split_ws[next(iter(_split_ws))]
+        ws = _split_ws[(dev, torch._C._cuda_getCurrentRawStream(dev))] = new()
+        return ws
 
 
 def _workspace_args(workspace, small: bool, device):
-    """(pointer, bytes) of the split form's workspace: None -> the device's shared buffer where the launch is small
+    """(pointer, bytes) of the split form's workspace: None -> the stream's shared buffer where the launch is small
     enough to be split, False -> none."""
     if workspace is None:
-        workspace = split_workspace(device) if (split_enabled and small) else False
+        if not (split_enabled and small):
+            return None, 0
+        workspace = _pass.workspace = replay.shared_workspace(split_workspace(device))
+        return workspace.data_ptr(), workspace.numel() * 4
     if workspace is False:
         return None, 0
     if workspace.dtype != torch.float32 or not workspace.is_contiguous() or workspace.device != device:
@@ -758,7 +784,7 @@ def _workspace_args(workspace, small: bool, device):
 def conv_masked(x, xmask, x2, x2mask, filt, k, stride, pad, out_ts: TileMask, out_delta,
                 reservoir=None, act=_lib.ACT_NONE, slope=0.0, path=_lib.PATH_AUTO, addend=None, workspace=None):
     """filt: ConvFilter, or a contiguous fp32 [Cin_total, K, K, Cout] tensor (VALU kernels only).
-    workspace: fp32 tensor for the split form of small launches (None: the device's shared one, False: none)."""
+    workspace: fp32 tensor for the split form of small launches (None: the stream's shared one, False: none)."""
     n, c1, h, w = x.shape
     c2 = 0 if x2 is None else x2.shape[1]
     if x2 is not None and (x2.shape[0] != n or x2.shape[2:] != x.shape[2:]):
@@ -1047,16 +1073,13 @@ def tconv2x_masked(x, xmask, x2, x2mask, filt, k, out_ts: TileMask, block_ts: Ti
     """Stride-2 transposed conv (k in {3, 5}, pad k // 2, output twice the input) of x ++ x2 on the matrix
     cores.  out_ts: MIE_FOOT_TCONV tile set of the output; block_ts: tile set of the 16x16 output blocks at
     input resolution (build_mask_tiles(out_ts, None, ..., FOOT_CONV, 2, 2, 0, block_ts)).
-    workspace: as in conv_masked (None: the device's shared one when the plane is small, False: none)."""
+    workspace: as in conv_masked (None: the stream's shared one when the plane is small, False: none)."""
     n, c1, c2, h, w, plain, mc_ptr, cin_total, cout, code = _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out_delta,
                                                                     addend, reservoir)
     dt = x.dtype
     _ready(out_ts)
     _ready(block_ts)
-    if workspace is None:
-        workspace = split_workspace(x.device) if (split_enabled and block_ts.capacity * (cout // 32) <= 128) else False
-    replay.keep(workspace)
-    ws_ptr, ws_bytes = (None, 0) if workspace is False else (workspace.data_ptr(), workspace.numel() * 4)
+    ws_ptr, ws_bytes = _workspace_args(workspace, block_ts.capacity * (cout // 32) <= 128, x.device)
     check(lib().mie_tconv2x_masked(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1, nhwc_ptr(x2, "x2", dtype=dt),
         pix_ptr(x2mask, n, h, w, "x2mask"), c2, h, w, plain.data_ptr(), mc_ptr, cin_total, k, cout, out_ts.ref,

@@ -174,6 +174,7 @@ class Recording:
     def __init__(self, real):
         self._real = real
         self.calls, self.keep, self.effects = [], [], []
+        self.workspace = None
 
     def __getattr__(self, name):
         fn = getattr(self._real, name)
@@ -209,6 +210,14 @@ def keep(obj):
         if r is not None:
             r.keep.append(obj)
     return obj
+
+
+def shared_workspace(ws):
+    """While a pass is recorded: notes that `ws` is the workspace of the stream at hand; a replay takes its own stream's."""
+    r = current()
+    if r is not None:
+        r.workspace = ws
+    return ws
 
 
 def effect(fn, *args):
@@ -316,6 +325,7 @@ class Program:
         self.runs, self.alive = 0, True
         self.plan_masks = []         # (op of a plan, its field, input): set before each run
         self.held = [[k for k in rec.keep if not (torch.is_tensor(k) and inputs.holds(k))], static]
+        workspace = None if rec.workspace is None else rec.workspace.data_ptr()
         calls = (_lib.MieCall * len(rec.calls))()
         for call, (name, args) in zip(calls, rec.calls):
             idx, sig = _signature(name)
@@ -323,7 +333,9 @@ class Program:
             patches = []
             for i, kind in enumerate(sig):
                 words[i] = _word(kind, args[i], self.held)
-                if kind == "w":
+                if kind == "w" and workspace is not None and words[i] == workspace:
+                    patches += [i, len(inputs.copies)]          # one input more: the workspace of the stream it runs on
+                elif kind == "w":
                     inputs.refuse("an input is written", words[i])
                 elif kind == "t" and args[i] is not None:
                     inputs.refuse_set(args[i]._obj)
@@ -346,7 +358,8 @@ class Program:
             call.args, call.patches = ctypes.addressof(words), ctypes.addressof(pa)
             self.held += [words, pa]
         self.calls, self.n = calls, len(rec.calls)
-        self.n_inputs = len(inputs.copies)
+        self.uses_workspace = workspace is not None
+        self.n_inputs = len(inputs.copies) + (1 if self.uses_workspace else 0)
         self.words_type = ctypes.c_uint64 * max(1, self.n_inputs)
         self.fn = _lib.lib().mie_run_calls
         self._guards(tree)
@@ -402,6 +415,9 @@ class Program:
         calls, effects, result = self.calls, self.effects, self.result
         for op, field, slot in self.plan_masks:
             setattr(op, field, pointers[slot])
+        if self.uses_workspace:
+            ws = _ops_globals["split_workspace"](device)
+            pointers = [*pointers, ws.data_ptr()]
         check(self.fn(calls, self.n, self.words_type(*pointers), self.n_inputs, torch._C._cuda_getCurrentRawStream(device)))
         for fn, args in effects:
             fn(*args)

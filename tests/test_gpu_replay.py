@@ -1,5 +1,6 @@
 """Recorded passes (maskedincrementeval_amd/replay.py) against the same passes walked in Python."""
 import copy
+import threading
 
 import pytest
 import torch
@@ -168,3 +169,49 @@ def test_recorded_steps_read_the_mask_of_the_pass_at_hand(net, dtype):
             alive.append((d, m))
             _equal(a([d, m], *extra), _walked(b, [d, m], *extra))
     assert sorted(p.runs for p in _programs(a)) == [1, 2] and not _programs(b)
+
+
+@pytest.mark.parametrize("own_stream", [False, True], ids=["one_stream", "a_stream_each"])
+def test_threads_step_networks_of_their_own(own_stream):
+    """Two threads, each with networks of its own on a plane whose convs are split, walk and record their first ten passes
+    side by side -- on one stream, and on a stream each: outputs as in one thread alone."""
+    kinds = [("e2depth", 5, (48, 80)), ("transposed", 4, (64, 96))]
+
+    def make(kind):
+        net = E2VIDRecurrentIncr() if kind == "e2depth" else MultiResUNetRecurrentIncr(num_bins=4, decoder=kind)
+        return seed_module_(net, seed=3).to(DEV).eval()
+
+    def passes(kind, bins, size, meet=None):
+        net, extra, got = make(kind), (None,) if kind == "e2depth" else (), []
+        x0 = _cl(torch.randn(1, bins, *size, generator=torch.Generator().manual_seed(1)))
+        ds = [_cl(event_voxel_delta(1, bins, *size, 0.05, seed=160 + i)[0]) for i in range(10)]
+        stream = torch.cuda.Stream() if own_stream and meet is not None else torch.cuda.current_stream()
+        stream.wait_stream(torch.cuda.default_stream())
+        with torch.no_grad(), torch.cuda.stream(stream):
+            net.forward_refresh_reservoirs(x0, *extra)
+            for d in ds:
+                if meet is not None:
+                    meet.wait()
+                out = net([d, None], *extra)
+                got.append([p[0].clone() for p in ([out[0]] if extra else out)])
+        stream.synchronize()
+        assert sorted(p.runs for p in _programs(net)) == [7]
+        return got
+
+    want = [passes(*k) for k in kinds]
+    torch.cuda.synchronize()
+    meet, box = threading.Barrier(2, timeout=60), [None, None]
+
+    def body(i):
+        try:
+            box[i] = passes(*kinds[i], meet=meet)
+        except BaseException as e:
+            meet.abort()
+            box[i] = e
+    threads = [threading.Thread(target=body, args=(i,)) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join(100) for t in threads]
+    for got, ref in zip(box, want):
+        if isinstance(got, BaseException):
+            raise got
+        _equal(got, ref)

@@ -330,3 +330,45 @@ def test_event_frames_are_copied_with_buffers_of_their_own(stub, dtype):
         (args,) = stub.named(entry)
         assert args[0] == twin._events.data_ptr() != frames._events.data_ptr()
         assert args[-3:-1] == (out.data_ptr(), mask.data_ptr()) and out.data_ptr() != frames._delta.data_ptr()
+
+
+def test_a_workspace_per_stream(stub, monkeypatch):
+    """Two streams never share a split workspace, whoever recorded what where; captured launches have one of their own."""
+    at = [1]
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: at[0], raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, device=None, **kw: empty(*a, **kw))
+    monkeypatch.setattr(ops, "_split_ws", {})
+    monkeypatch.setattr(ops, "_captured_ws", {})
+    monkeypatch.setattr(ops, "SPLIT_WORKSPACE_BYTES", 4096)
+    dev = torch.device("cpu")
+    got = {}
+    for stream in (1, 2, 1, 2):
+        at[0] = stream
+        got.setdefault(stream, ops.split_workspace(dev))
+        assert got[stream] is ops.split_workspace(dev)
+    assert got[1] is not got[2]
+    with monkeypatch.context() as patch:
+        patch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        captured = ops.split_workspace(dev)
+        at[0] = 1
+        assert captured is ops.split_workspace(dev) and captured is not got[1] and captured is not got[2]
+
+    def body(x):
+        ptr, size = ops._workspace_args(None, True, dev)
+        ops.lib().mie_upconv_masked_ws(x.data_ptr(), None, None, None, 64, 4, 4, 0, 0, 64, 5, 2, 32, None, 0, None, None, 0, 0.0, 0, ptr, size, 0)
+        return None
+
+    x = _cl(1, 64, 4, 4)
+    at[0] = 1
+    _, program = replay._record([body], (x,), [(0, None)], (), [])
+    for stream in (1, 2, 3, 1):
+        at[0] = stream
+        del stub.calls[:]
+        program.run([x.data_ptr()], dev)
+        assert stub.named("mie_upconv_masked_ws")[0][20] == ops.split_workspace(dev).data_ptr()
+    for stream in range(10, 60):
+        at[0] = stream
+        ops.split_workspace(dev)
+    assert len(ops._split_ws) <= ops.SPLIT_WORKSPACES
