@@ -4,6 +4,7 @@ Each function checks shapes / layouts on the host, pulls raw device pointers
 and the current HIP stream out of torch, and calls one entry point of
 include/mie.h.  torch is used for memory and streams only.
 """
+import collections
 import os
 import threading
 from typing import Optional, Tuple
@@ -77,7 +78,9 @@ def lib():
 # own with an event of their own, so that the first convs run beside the plan of the rest -- every extra dependency
 # between the two streams costs 5-10 us of idle time in the replayed graph, more than the overlap wins.)
 fused_plan = os.environ.get("MIE_FUSED_PLAN", "1") != "0"
-_plan_cache = {}         # signature of a batch -> [("plan", ctypes array, n) | ("single", index)] parts
+# everything a batch says -> [("plan", ctypes array, n, first) | ("single", None, 1, index)] parts, newest last
+_plan_cache = collections.OrderedDict()
+PLAN_CACHE = 64
 
 
 class network_pass:
@@ -136,7 +139,7 @@ def _launch_plan(batch):
         stream = side.cuda_stream
     else:
         stream = torch.cuda.current_stream(dev).cuda_stream
-    sig = tuple(b[:8] + (b[8].pixmask.data_ptr(), b[8].tiles.data_ptr()) for b in batch) + (plan_wgs,)
+    sig = tuple(b[:8] + (bytes(b[8].c_struct),) for b in batch) + (plan_wgs,)
     parts = _plan_cache.get(sig)
     if plan_wgs:
         build_plan = lambda arr, n: real.mie_build_mask_plan_wgs(arr, n, plan_wgs, stream)
@@ -169,6 +172,8 @@ def _launch_plan(batch):
             else:
                 check(rc)
         _plan_cache[sig] = parts
+        while len(_plan_cache) > PLAN_CACHE:
+            _plan_cache.popitem(last=False)
     else:
         for kind, arr, n_ops, lo in parts:
             if kind == "plan":

@@ -16,6 +16,7 @@ from maskedincrementeval_amd import _lib, ops, replay
 from maskedincrementeval_amd import mask_incr_modules as mm
 from maskedincrementeval_amd.event_frontend import EventFrames
 from maskedincrementeval_amd.mask_incr_functional import IncrementReserve
+from maskedincrementeval_amd.masked_types import TileMask
 from maskedincrementeval_amd.e2depth_incr import E2VIDRecurrentIncr
 
 
@@ -372,3 +373,24 @@ def test_a_workspace_per_stream(stub, monkeypatch):
         at[0] = stream
         ops.split_workspace(dev)
     assert len(ops._split_ws) <= ops.SPLIT_WORKSPACES
+
+
+def test_a_plan_is_for_the_tile_sets_at_hand(stub):
+    """A tile set that shares some of its addresses with a former one is not planned as that one; plans made for buffers
+    that are gone do not pile up."""
+    def planned(*sets):
+        with ops.network_pass("plan"):
+            for ts in sets:
+                ops.build_mask_tiles(None, None, 1, 16, 16, _lib.FOOT_CONV, 3, 1, 1, ts)
+        arr, n, _ = stub.named("mie_build_mask_plan")[-1]
+        return [bytes(op.out) for op in arr[:n]]
+
+    a, b = (TileMask(1, 16, 16, "cpu") for _ in range(2))
+    assert planned(a, b) == planned(a, b) == [bytes(a.c_struct), bytes(b.c_struct)]
+    other = torch.zeros_like(a.flags)
+    a.c_struct.flags = other.data_ptr()
+    assert planned(a, b) == [bytes(a.c_struct), bytes(b.c_struct)]
+    for _ in range(3 * ops.PLAN_CACHE):
+        a.c_struct.flags += 64
+        planned(a)
+    assert len(ops._plan_cache) <= ops.PLAN_CACHE
