@@ -266,6 +266,50 @@ __device__ __forceinline__ void conv_gates_item(const ConvArgsT<T>& a, long long
   mie_st4(a.g_dc, ho, make_float4(dc[0], dc[1], dc[2], dc[3]));
 }
 
+// The arguments of the running kernel, whose first and largest is a ConvArgsT<T>, where the launch put them.  To be inlined
+// into the kernel itself: in a function that is called there is no such place.
+template <typename T>
+__device__ __forceinline__ const ConvArgsT<T>& conv_args_again() {
+  uint64_t at = (uint64_t)(const void*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm("" : "+s"(at));
+  return *(const ConvArgsT<T>*)at;
+}
+
+__device__ __forceinline__ bool finite4(const float4& v) {
+  return isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w);
+}
+
+// Four output channels of a conv in plain fp32, straight from the inputs and the plain filter, with the epilogue: what is
+// done instead where a sum of the three-term form is not finite.  That form makes NaN of an infinite delta and of a finite
+// one that rounds to an infinite bf16 term (3.39e38 and more); either leaves no finite sum, so the test of the sum finds all
+// of them, and finite sums cost that test only.  For the 5x5 stride-2 convs, whose launches of few tiles ran on the fp32
+// instruction before and carried such values (the forms at stride 1 do not: mie.h, MIE_DTYPE_F32_BF16X3).  It runs behind
+// the ordinary stores, over the groups these left out: inside them the loops cost registers (1-2 us a launch).
+// (The arguments are read from memory anew, through conv_args_again: taken from the kernel's `a`, a dozen fields more stayed
+// in registers through the contraction, whose scalar spills cost 0.5-1.1 us a launch.)
+template <typename T, int K, int S>
+__device__ void conv_quad_again(const ConvArgsT<T>& a, int n, int oy, int ox, int co) {
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int t = 0; t < K * K; ++t) {
+    const int iy = oy * S - a.pad + t / K, ix = ox * S - a.pad + t % K;
+    if (iy < 0 || iy >= a.h_in || ix < 0 || ix >= a.w_in) continue;
+    const long long pix = ((long long)n * a.h_in + iy) * a.w_in + ix;
+    for (int in = 0; in < 2; ++in) {
+      const T* x = in ? a.x2 : a.x;
+      const uint8_t* m = in ? a.x2m : a.xm;
+      const int c = in ? a.c2 : a.c1, ci0 = in ? a.c1 : 0;
+      if (x == nullptr || (m != nullptr && m[pix] == 0)) continue;
+      for (int ci = 0; ci < c; ++ci) {
+        const float v = mie_ld(x, pix * c + ci);
+        const float* w = a.filt + ((long long)(ci0 + ci) * (K * K) + t) * a.cout + co;
+        s.x = fmaf(v, w[0], s.x); s.y = fmaf(v, w[1], s.y); s.z = fmaf(v, w[2], s.z); s.w = fmaf(v, w[3], s.w);
+      }
+    }
+  }
+  const long long off = (((long long)n * a.ts.h + oy) * a.ts.w + ox) * a.cout + co;
+  conv_store(a, off, co, s.x); conv_store(a, off + 1, co + 1, s.y); conv_store(a, off + 2, co + 2, s.z); conv_store(a, off + 3, co + 3, s.w);
+}
+
 // UP: the conv input is up2x(x + x2), the bilinear x2 up-sampling of the sum of two deltas given at
 // half resolution (x2 optional), and is never formed in memory: per chunk the 8x8 block of source
 // pixels a tile's 12x12 input window blends is summed into LDS (fp32), and the staged tile is expanded
@@ -1065,6 +1109,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
           red[p * CO_BLK + wn * (32 * NB) + nb * 32 + l32] = acc[mb][nb][r];
       }
     __syncthreads();
+    unsigned bad_bits = 0u;                      // groups whose sums are not finite (conv_quad_again)
 #pragma unroll
     for (int h0 = 0; h0 < PER; h0 += PB) {       // the 128-column slabs in two passes of four groups per thread
       if (!EARLY || SPLIT) epilogue_fetch(h0);
@@ -1086,8 +1131,23 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         for (int i = 0; i < PB; ++i)
           if (e_ok[i]) *reinterpret_cast<float4*>(plane + e_off[i]) = v[i];
       } else {
+        if constexpr (X3 && S == 2) {
+#pragma unroll
+          for (int i = 0; i < PB; ++i)
+            if (e_ok[i] && !finite4(v[i])) {
+              e_ok[i] = false;
+              bad_bits |= 1u << (h0 + i);
+            }
+        }
         conv_epilogue_store4<T, PB>(a, e_off, e_co, e_ok, v, e_r0, e_add, e_live);
       }
+    }
+    if constexpr (X3 && S == 2 && !SPLIT) {
+      if (__builtin_expect(__ballot(bad_bits != 0u) != 0ull, 0))
+        for (int g = 0; g < PER; ++g) {
+          const int idx = tid + 256 * g, p = idx / QPP, co = co0 + 4 * (idx - p * QPP);
+          if ((bad_bits >> g) & 1u) conv_quad_again<T, K, S>(conv_args_again<T>(), n, y0 + (p >> 3), x0 + (p & 7), co);
+        }
     }
   }
   MIE_STAMP(14);
@@ -1123,7 +1183,8 @@ __device__ __forceinline__ float4 split_sum(const float* ws, long long plane, in
 // Second half of a SPLIT launch: per active tile the `parts` partial planes are added in order and
 // the ordinary epilogue (addend, reservoir, activation) runs; stale tiles are zeroed.  One thread per
 // (pixel, channel), channels fastest.
-template <typename T>
+// K, S != 0: sums that are not finite are computed again in fp32 (conv_quad_again).
+template <typename T, int K = 0, int S = 0>
 __global__ __launch_bounds__(256) void k_conv_split_finish(ConvArgsT<T> a, int parts) {
   int n, y0, x0;
   const int tk = mie_pick_tile(a.ts, blockIdx.x + conv_args_entry_zero(a), n, y0, x0);
@@ -1133,6 +1194,7 @@ __global__ __launch_bounds__(256) void k_conv_split_finish(ConvArgsT<T> a, int p
   const int c0 = (int)blockIdx.y * cb;
   const int cn = (cout - c0 < cb) ? cout - c0 : cb;
   const int qn = cn >> 2;                                             // groups of four adjacent channels
+  bool bad = false;
   for (int idx = threadIdx.x; idx < 64 * qn; idx += 256) {
     const int p = idx / qn, co = c0 + 4 * (idx - p * qn);
     const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
@@ -1148,7 +1210,22 @@ __global__ __launch_bounds__(256) void k_conv_split_finish(ConvArgsT<T> a, int p
     float4 r0[1], add[1];
     conv_epilogue_load4<T, 1>(a, offs, oks, r0, add);
     const float4 accs[1] = {split_sum(a.ws + off, a.ws_plane, parts)};
+    if constexpr (K != 0) {
+      if (!finite4(accs[0])) {
+        bad = true;
+        continue;
+      }
+    }
     conv_epilogue_store4<T, 1>(a, offs, cos, oks, accs, r0, add);
+  }
+  if constexpr (K != 0) {
+    if (__builtin_expect(__ballot(bad) != 0ull, 0))
+      for (int idx = threadIdx.x; idx < 64 * qn; idx += 256) {
+        const int p = idx / qn, co = c0 + 4 * (idx - p * qn);
+        const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
+        if (oy < hout && ox < wout && !finite4(split_sum(a.ws + (((long long)n * hout + oy) * wout + ox) * cout + co, a.ws_plane, parts)))
+          conv_quad_again<T, K, S>(conv_args_again<T>(), n, oy, ox, co);
+      }
   }
 }
 
@@ -1208,12 +1285,12 @@ int split_parts(ConvArgsT<T>& a, long long groups, int nch) {
   return parts < 2 ? 0 : parts;
 }
 
-template <typename T>
+template <typename T, int K = 0, int S = 0>
 void launch_split_finish(const ConvArgsT<T>& a, unsigned cap, int parts, hipStream_t st) {
   unsigned ny = (unsigned)((1024 + cap - 1) / cap);
   if (ny > (unsigned)(a.cout / 4)) ny = (unsigned)(a.cout / 4);
   if (ny < 1) ny = 1;
-  hipLaunchKernelGGL(k_conv_split_finish<T>, dim3(cap, ny), dim3(256), 0, st, a, parts);
+  hipLaunchKernelGGL((k_conv_split_finish<T, K, S>), dim3(cap, ny), dim3(256), 0, st, a, parts);
 }
 
 template <typename T, int K, int S>
@@ -1231,6 +1308,12 @@ bool launch_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
     if constexpr (HAS_X3) hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true, true>), grid, dim3(256), 0, st, a);
   } else {
     hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true>), grid, dim3(256), 0, st, a);
+  }
+  if constexpr (HAS_X3 && S == 2) {
+    if (x3) {
+      launch_split_finish<T, K, S>(a, cap, parts, st);
+      return true;
+    }
   }
   launch_split_finish(a, cap, parts, st);
   return true;

@@ -211,3 +211,60 @@ def test_non_finite_deltas_never_come_out_as_finite_numbers():
     near_big[0, 0, 20, 20] = 1
     near_big = (F.max_pool2d(near_big, k, 1, k // 2) > 0).expand(1, cout, h, w)
     assert (~torch.isfinite(x3[near_big])).all()
+
+
+def _stride2_split(x, wt, mode, mask=None, second=0):
+    """5x5 stride-2 conv given a workspace, `second` of the input channels from a second tensor."""
+    n, cin, h, w = x.shape
+    cout, c1 = wt.shape[0], cin - second
+    ho, wo = ops.conv_out_size(h, w, 5, 2, 2)
+    ts = TileMask(n, ho, wo, DEV)
+    dm = None if mask is None else mask.to(DEV)
+    ops.build_mask_tiles(dm, None, n, h, w, _lib.FOOT_CONV, 5, 2, 2, ts)
+    out = ops.new_nhwc(n, cout, ho, wo, DEV)
+    ws = torch.full((ops.SPLIT_WORKSPACE_BYTES // 4,), -1.0, device=DEV)
+    old = ops.f32_matmul
+    try:
+        ops.f32_matmul = mode
+        ops.conv_masked(_dev(x[:, :c1]), dm, _dev(x[:, c1:]) if second else None, dm if second else None, _filt(wt), 5, 2, 2, ts, out,
+                        path=_lib.PATH_MFMA, workspace=ws)
+    finally:
+        ops.f32_matmul = old
+    if mode == "bf16x3":        # the split form: few tiles, at least four chunks of 16 channels
+        split = ts.capacity * (cout // 32) <= 128 and cin >= 64
+        assert bool((ws[:2 * out.numel()] != -1.0).any()) == split
+    return out.cpu(), ts.pixmask.cpu().bool()
+
+
+@pytest.mark.parametrize("cin,cout,h,w,second", [(64, 128, 32, 48, 0), (128, 256, 16, 24, 0), (64, 64, 33, 29, 32), (64, 32, 7, 5, 0),
+                                                     (32, 64, 64, 96, 0), (32, 64, 132, 176, 0), (128, 256, 66, 88, 0)])
+def test_stride_2_convs_against_fp64_and_with_non_finite_deltas(cin, cout, h, w, second):
+    """Error of the three-term form (split, unsplit on few tiles, unsplit on many) against fp64 next to the fp32 instruction's (both bounded like the unsplit forms,
+    4e-7 of sum |x||w|: three fp32 roundings), then the same conv over infinite, NaN and huge deltas: what an fp32 conv
+    gives, in both forms.  A masked pixel's value is not read."""
+    g = torch.Generator().manual_seed(cin + h)
+    x, wt = torch.randn(1, cin, h, w, generator=g), he_normal_conv_weight(cout, cin, 5, 7)
+    ref = F.conv2d(x.double(), wt.double(), stride=2, padding=2)
+    bound = F.conv2d(x.double().abs(), wt.double().abs(), stride=2, padding=2)
+    err = {}
+    for mode in ("native", "bf16x3"):
+        got, _ = _stride2_split(x, wt, mode, second=second)
+        e = (got.double() - ref).abs()
+        err[mode] = (e / bound).max().item(), (e.norm() / ref.norm()).item()
+    assert max(err["bf16x3"][0], err["native"][0]) < 4e-7 and err["bf16x3"][1] <= err["native"][1], err
+    bad, mask = x.clone(), torch.ones(1, 1, h, w, dtype=torch.uint8)
+    spots = {(1, 2, 1): float("inf"), (5, h - 1, w - 1): float("-inf"), (cin - 1, h // 2, 0): 3.4e38, (cin // 2, 0, w // 2): float("nan")}
+    for (c, y, x_), v in spots.items():
+        bad[0, c, y, x_] = v
+    bad[0, 0, h // 2, w // 2], mask[0, 0, h // 2, w // 2] = float("inf"), 0
+    seen = torch.where(mask.bool(), bad, torch.zeros(()))
+    want = F.conv2d(seen, wt, stride=2, padding=2)
+    # values of 3.4e38 times small weights: fp32 sums of 1600 .. 3200 terms in another order
+    scale = F.conv2d(torch.nan_to_num(seen, posinf=0.0, neginf=0.0).double().abs(), wt.double().abs(), stride=2, padding=2)
+    for mode in ("native", "bf16x3"):
+        got, live = _stride2_split(bad, wt, mode, mask, second)
+        live = live.expand_as(got)
+        fine = torch.isfinite(want) & live
+        assert torch.equal(torch.isnan(got) & live, torch.isnan(want) & live) and torch.equal(torch.isinf(got) & live, torch.isinf(want) & live), mode
+        assert torch.equal(got[torch.isinf(want) & live], want[torch.isinf(want) & live])
+        assert ((got.double() - want.double()).abs() <= 2e-6 * scale)[fine].all(), mode
