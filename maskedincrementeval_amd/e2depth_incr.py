@@ -497,6 +497,8 @@ class UpsampleConvLayerIncr(replay.Watched, nn.Module):
     """bilinear x2 -> conv -> activation (reference :284-322); the skip sum of the
     UNet is taken inside the up-sampling kernel."""
 
+    dense_plane = False      # nnConvIncr.forward_fused_upsampled: what is known of the masks of x and skip
+
     def __init__(self, in_channels, out_channels, kernel_size, stride=1, padding=0,
                  activation='relu', norm=None, fuse=True):
         super().__init__()
@@ -518,7 +520,7 @@ class UpsampleConvLayerIncr(replay.Watched, nn.Module):
     def forward(self, x_incr: Masked, skip_incr: Masked = None) -> Masked:
         if self.fuse and self.activation is not None and self.norm not in ['BN', 'IN']:
             # up-sampling, skip sum, conv and activation in one kernel where the shape allows it
-            return self.conv2d.forward_fused_upsampled(self.upsample, x_incr, skip_incr, self.activation)
+            return self.conv2d.forward_fused_upsampled(self.upsample, x_incr, skip_incr, self.activation, self.dense_plane)
         x_upsampled_incr = self.upsample(x_incr, skip_incr)
         out_incr = self.conv2d(x_upsampled_incr)
         if self.norm in ['BN', 'IN']:
@@ -583,6 +585,9 @@ class BaseUNetIncr(replay.Watched, nn.Module):
         for input_size in decoder_input_sizes:
             self.decoders.append(self.UpsampleLayer(input_size, input_size // 2, kernel_size=5,
                                                     padding=2, norm=self.norm, fuse=self.fuse))
+            # behind three encoders and two residual blocks the footprint of one input pixel is 15 pixels wide and more at the
+            # decoders' resolutions (measured: every tile active from 0.5 % of the input on)
+            self.decoders[-1].dense_plane = True
 
     def build_prediction_layer(self):
         self.pred = ConvLayerIncr(self.base_num_channels, self.num_output_channels, 1,

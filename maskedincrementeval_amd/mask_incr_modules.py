@@ -385,15 +385,21 @@ class _ConvIncrMixin(_IncrBuffers):
 
 
     def _upconv_forward(self, up: "nnUpsample2xIncr", x_incr: Masked, skip_incr: Masked, reservoir, act, slope,
-                        out_name="out_act") -> Masked:
-        """conv over up2x(x + skip) without forming the up-sampled delta (ops.upconv_masked)."""
+                        out_name="out_act", dense_plane=False) -> Masked:
+        """conv over up2x(x + skip) without forming the up-sampled delta (ops.upconv_masked / upconv2x_masked)."""
         k, s, p = self._geometry()
         a, pa, b, pb, ts_up = up.plan(x_incr, skip_incr)
         n, _, h, w = a.shape
         ts = self._tile_set(out_name, n, 2 * h, 2 * w, a.device)
         ops.build_mask_tiles(ts_up, None, n, 2 * h, 2 * w, _lib.FOOT_CONV, k, s, p, ts)
         out = self._delta_buf(out_name, (n, self.out_channels, 2 * h, 2 * w), a.device, a.dtype)
-        if ops.upconv2x_takes(a, self.out_channels, k, s, p, self.conv2d_weights):
+        # The form at the resolution of the inputs has no list of active tiles: it computes whole 8x8 blocks of positions for
+        # each tile they touch.  Where every tile is active, or the active ones lie together, it is the faster one; single
+        # active pixels spread over the plane make up to 2.4 times the work of the list (bf16 128->64 at 8x120x160: all
+        # tiles 254 us against 340, a blob of 10 % 46 against 48, 12 % of the tiles around single pixels 100 against 42).
+        # So: for planes known to be active as a whole (no mask), or said to be (dense_plane).
+        dense = dense_plane or pa is None or (b is not None and pb is None)
+        if dense and ops.upconv2x_takes(a, self.out_channels, k, s, p, self.conv2d_weights):
             ops.upconv2x_masked(a, pa, b, pb, self.conv2d_weights, ts, out, reservoir, act, slope)
             return [out, ts]
         ops.upconv_masked(a, pa, b, pb, self.conv2d_weights, k, p, ts, out, reservoir, act, slope)
@@ -543,9 +549,11 @@ class nnConvIncr(replay.Watched, nn.Conv2d, _ConvIncrMixin):
         return self._incr_forward(x_incr, x2_incr, reservoir=res, act=kind, slope=slope,
                                   path=self.path, out_name="out_act", addend_incr=addend_incr, filt=filt)
 
-    def forward_fused_upsampled(self, up: "nnUpsample2xIncr", x_incr, skip_incr, activation: "nnReservedActivation"):
+    def forward_fused_upsampled(self, up: "nnUpsample2xIncr", x_incr, skip_incr, activation: "nnReservedActivation",
+                                dense_plane: bool = False):
         """bilinear x2 of (x + skip) + conv + activation increment; one kernel when the shape allows it,
-        else the up-sampling kernel followed by forward_fused."""
+        else the up-sampling kernel followed by forward_fused.  dense_plane: the active pixels of x and skip come in
+        regions of a dozen pixels and more, or are all of them (see _upconv_forward)."""
         k, s, p = self._geometry()
         x = x_incr[0]
         # Measured on MI355X.  bf16: the one-kernel form wins at every size (264x352 frame -3 %, 8x480x640
@@ -568,7 +576,7 @@ class nnConvIncr(replay.Watched, nn.Conv2d, _ConvIncrMixin):
         res = activation.in_res.reservoir
         if res is None:
             raise RuntimeError("fused conv+activation: call forward_refresh_reservoirs first")
-        return self._upconv_forward(up, x_incr, skip_incr, res, kind, slope)
+        return self._upconv_forward(up, x_incr, skip_incr, res, kind, slope, dense_plane=dense_plane)
 
     def forward_refresh_reservoirs(self, x):
         # The reference refreshes self.kf here unconditionally (:193): a norm and a zero clone

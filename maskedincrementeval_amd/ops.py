@@ -866,7 +866,7 @@ upconv2x_enabled = os.environ.get("MIE_UPCONV2X", "1") != "0"      # tuning knob
 
 def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt) -> bool:
     """Whether a decoder layer over `a` runs at the resolution of its inputs: upconv2x_masked has a kernel for it and is the
-    faster form.  It is not on planes so small that upconv_masked splits the contraction (256->128 at 16x16: 25 us against
+    faster form where all tiles are active (nnConvIncr._upconv_forward asks for that first).  It is not on planes so small that upconv_masked splits the contraction (256->128 at 16x16: 25 us against
     22, at 20x20 26 against 35), for bf16 layers of one staged chunk (64->32 at 8x240x320: 525 us against 417 in the
     persistent kernel), and where border strips and blocks filled in part undo the fewer taps: 16 for each of the four
     phases of an item against 25 for each tile, once that is more than a round of workgroups (256->128 at 8x19x23: 138

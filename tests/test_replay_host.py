@@ -17,7 +17,7 @@ from maskedincrementeval_amd import mask_incr_modules as mm
 from maskedincrementeval_amd.event_frontend import EventFrames
 from maskedincrementeval_amd.mask_incr_functional import IncrementReserve
 from maskedincrementeval_amd.masked_types import TileMask
-from maskedincrementeval_amd.e2depth_incr import E2VIDRecurrentIncr
+from maskedincrementeval_amd.e2depth_incr import E2VIDRecurrentIncr, UpsampleConvLayerIncr
 
 
 class StubLib:
@@ -394,3 +394,25 @@ def test_a_plan_is_for_the_tile_sets_at_hand(stub):
         a.c_struct.flags += 64
         planned(a)
     assert len(ops._plan_cache) <= ops.PLAN_CACHE
+
+
+def test_decoder_layers_take_the_form_without_lists_where_the_plane_is_dense(stub, monkeypatch):
+    monkeypatch.setattr(ops, "upconv2x_takes", lambda *args: True)
+    monkeypatch.setattr(ops, "upconv_takes", lambda *args: True)
+
+    def taken(layer, x_mask, skip_mask, skip=True):
+        x, y = _cl(1, 64, 8, 8), _cl(1, 64, 8, 8)
+        layer.activation.in_res.reservoir = _cl(1, 32, 16, 16)
+        del stub.calls[:]
+        layer([x, x_mask], [y, skip_mask] if skip else None)
+        return [n for _, n, _ in stub.calls if n.startswith("mie_upconv")]
+
+    mask = torch.ones(1, 1, 8, 8, dtype=torch.uint8)
+    with torch.no_grad():
+        layer = UpsampleConvLayerIncr(64, 32, 5, padding=2)
+        lists, dense = ["mie_upconv_masked_ws"], ["mie_upconv2x_masked"]
+        assert taken(layer, mask, mask) == taken(layer, mask, None, skip=False) == lists
+        assert taken(layer, None, mask) == taken(layer, mask, None) == taken(layer, None, None, skip=False) == dense
+        layer.dense_plane = True
+        assert taken(layer, mask, mask) == dense
+        assert all(d.dense_plane for d in E2VIDRecurrentIncr().unetrecurrent.decoders)
