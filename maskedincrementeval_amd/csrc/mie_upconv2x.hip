@@ -118,6 +118,22 @@ __global__ __launch_bounds__(256) void k_pack_up2x(const float* __restrict__ f, 
   }
 }
 
+// A unit of two M blocks in the three-term form, only the product of the leading terms into `acc` and the five smaller ones
+// into `sm` (mma_unit2_x3 has two of them, 2^-9 of the leading one, in `acc`): a third of the roundings at the size of the
+// sum.  The four phases' chains are longer than the list-driven form's, which splits the channels over more waves; with
+// mma_unit2_x3 the error against fp64 was up to 1.13 times that form's at some layers of the networks (128->64 at 66x88:
+// 3.5e-7 of the output against 3.1e-7), this way it is below it at all of them (1.9e-7).  Same time: an MFMA waits for the
+// one before the last at most.
+__device__ __forceinline__ void mma_up2x_x3(v16f& acc0, v16f& acc1, v16f& sm0, v16f& sm1, const float4 (&a0)[3],
+                                            const float4 (&a1)[3], const float4 (&b)[3]) {
+  mma_unit(sm0, a0[2], b[0], mie_bf16()); mma_unit(sm1, a1[2], b[0], mie_bf16());
+  mma_unit(acc0, a0[0], b[0], mie_bf16()); mma_unit(acc1, a1[0], b[0], mie_bf16());
+  mma_unit(sm0, a0[1], b[1], mie_bf16()); mma_unit(sm1, a1[1], b[1], mie_bf16());
+  mma_unit(sm0, a0[0], b[2], mie_bf16()); mma_unit(sm1, a1[0], b[2], mie_bf16());
+  mma_unit(sm0, a0[1], b[0], mie_bf16()); mma_unit(sm1, a1[1], b[0], mie_bf16());
+  mma_unit(sm0, a0[0], b[1], mie_bf16()); mma_unit(sm1, a1[0], b[1], mie_bf16());
+}
+
 template <typename T, int WN>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvArgsT<T> a, Up2xOrder od) {
   constexpr bool X3 = sizeof(T) == 4;
@@ -408,7 +424,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
           __builtin_amdgcn_sched_barrier(0);
           const auto& A = av[i & 1];
           const auto& B = bring[i & 3];
-          if constexpr (X3) mma_unit2_x3(acc[0], acc[1], sm[0], sm[1], A[0], A[1], B);
+          if constexpr (X3) mma_up2x_x3(acc[0], acc[1], sm[0], sm[1], A[0], A[1], B);
           else mma_unit2(acc[0], acc[1], A[0][0], A[1][0], B[0], mie_bf16());
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -446,9 +462,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
             const auto& B = bring[t];
             if (t < 3 || !corner) {
               if constexpr (X3) {
-                mma_unit(acc[0], A[0], B[0], mie_bf16()); mma_unit(sm[0], A[2], B[0], mie_bf16());
-                mma_unit(acc[0], A[1], B[0], mie_bf16()); mma_unit(sm[0], A[1], B[1], mie_bf16());
-                mma_unit(acc[0], A[0], B[1], mie_bf16()); mma_unit(sm[0], A[0], B[2], mie_bf16());
+                mma_unit(sm[0], A[2], B[0], mie_bf16()); mma_unit(sm[0], A[1], B[1], mie_bf16());
+                mma_unit(acc[0], A[0], B[0], mie_bf16()); mma_unit(sm[0], A[0], B[2], mie_bf16());
+                mma_unit(sm[0], A[1], B[0], mie_bf16()); mma_unit(sm[0], A[0], B[1], mie_bf16());
               } else {
                 mma_unit(acc[0], A[0], B[0], mie_bf16());
               }

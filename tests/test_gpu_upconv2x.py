@@ -72,3 +72,42 @@ def test_decoder_conv_at_input_resolution(n, c, cout, h, w, dtype):
     pre = io.conv_incr(io.interp_incr(a + b), wt, 1, 2) + bias.view(1, -1, 1, 1)
     assert torch.allclose(res.cpu(), pre, rtol=FP32_RTOL, atol=bf16_atol(pre, 2.0) if bf else 2 * FP32_ATOL)
     assert torch.allclose(dense.float().cpu(), torch.relu(pre), **tol(pre))
+
+
+@pytest.mark.parametrize("kind", ["white", "smooth"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,c,cout,h,w", [(1, 256, 128, 33, 44), (1, 128, 64, 66, 88), (2, 128, 64, 25, 35), (1, 64, 32, 132, 176), (4, 256, 128, 30, 40)])
+def test_error_against_fp64_beside_the_list_driven_form(n, c, cout, h, w, dtype, kind):
+    """The two forms of a decoder layer next to the layer in fp64, over the fp32 weights.
+    bf16: each rounds the sum of its inputs (up-sampled or not), its weights (combined or not) and its output to 8 bits, a
+    relative error of 1.66e-3 rms each (a mantissa spread evenly over its octave), sqrt(3) of that = 2.87e-3 where the
+    products are independent: 3.0e-3 allowed, and 4 % more than the list-driven form on white inputs (whose blend of
+    independent pixels spreads the mantissas more evenly: 2.5-3 % measured).  On smooth inputs this form is the closer one:
+    its taps' combined weights share less of their roundings (the list-driven form's then add up: 2.75-3.34e-3 measured).
+    fp32: the order of the sums and the accumulators are what differs; no more error than the list-driven form's."""
+    g = torch.Generator().manual_seed(c + h)
+    a, b = (torch.randn(n, c, h, w, generator=g) for _ in range(2))
+    if kind == "smooth":
+        a, b = (torch.nn.functional.avg_pool2d(t, 5, 1, 2) * 4.0 + 1.0 for t in (a, b))
+    wt = he_normal_conv_weight(cout, c, 5, 9)
+    filt = ops.ConvFilter(wt.permute(1, 2, 3, 0).contiguous().to(DEV))
+    da, db = _dev(a, dtype), _dev(b, dtype)
+    # fp64 on the GPU as 25 matrix products over shifted planes of the up-sampled sum
+    up = torch.nn.functional.interpolate(da.double() + db.double(), scale_factor=2, mode="bilinear", align_corners=False)
+    up = torch.nn.functional.pad(up, (2, 2, 2, 2)).permute(0, 2, 3, 1).contiguous()
+    H, W = 2 * h, 2 * w
+    ref = sum(up[:, y:y + H, x:x + W].reshape(-1, c) @ filt.plain[:, y, x].double() for y in range(5) for x in range(5))
+    ref = ref.view(n, H, W, cout).permute(0, 3, 1, 2)
+    ts = TileMask(n, H, W, DEV)
+    ops.build_mask_tiles(None, None, n, H, W, _lib.FOOT_CONV, 1, 1, 0, ts)
+    err = []
+    for form in (lambda out: ops.upconv_masked(da, None, db, None, filt, 5, 2, ts, out),
+                 lambda out: ops.upconv2x_masked(da, None, db, None, filt, ts, out)):
+        out = ops.new_nhwc(n, cout, H, W, DEV, dtype)
+        form(out)
+        err.append(((out.double() - ref).norm() / ref.norm()).item())
+    print("%s %s %dx%dx%d %d->%d: list-driven %.3e, here %.3e" % (dtype, kind, n, h, w, c, cout, *err))
+    if dtype == torch.bfloat16:
+        assert err[1] < 3.0e-3 and err[1] <= (1.04 if kind == "white" else 1.0) * err[0], err
+    else:
+        assert err[1] <= err[0], err
