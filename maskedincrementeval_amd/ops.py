@@ -31,6 +31,7 @@ class _PassState(threading.local):
     buffer_parity = 0        # generation of tile sets and delta buffers (planning one step ahead, below)
     planner = None           # (side stream, device) inside a mask_planner block
     workspace = None         # the shared split workspace used last
+    walking = False          # a pass is walked (or recorded) as a whole: its layers are not replayed one by one
 
     def __init__(self):
         self.pix_ready = {}      # data_ptr of a pixel mask written on the compute stream -> event

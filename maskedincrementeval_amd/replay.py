@@ -37,6 +37,9 @@ from ._lib import check
 
 enabled = os.environ.get("MIE_REPLAY", "1") != "0"      # read once
 MAX_RECORDINGS = 8          # per module, least recently used first out
+# While a pass waits to be recorded, the passes inside it (its layers') do not look for recordings of their own; once this
+# many passes in a row were walked it is one that is not recorded, and its layers are.
+WALKS = 4
 _recording = {}             # thread identity -> the Recording that thread is making
 _SILENT = frozenset(("training", "states"))     # assignments no incremental pass depends on
 
@@ -60,6 +63,7 @@ class WatchedType(abc.ABCMeta):
     ABCMeta, so that a caller's subclass may be an abstract one, too.)"""
     changes = 0              # replacements so far, of all classes
     defined = {}             # class -> its attributes as they were written
+    looked_at = {}           # class -> (changes, as_written) when last looked at
 
     def __init__(cls, *args, **kw):
         super().__init__(*args, **kw)
@@ -80,13 +84,27 @@ class WatchedType(abc.ABCMeta):
 
     def as_written(cls):
         """Whether this class and the package's classes it comes from are what their sources say."""
-        for c in cls.__mro__:
-            was = WatchedType.defined.get(c)
-            if was is not None:
-                now = WatchedType.code_of(c)
-                if now.keys() != was.keys() or any(now[k] is not was[k] for k in was):
-                    return False
-        return True
+        seen = WatchedType.looked_at.get(cls)
+        if seen is None or seen[0] != WatchedType.changes:
+            same = True
+            for c in cls.__mro__:
+                was = WatchedType.defined.get(c)
+                if was is not None:
+                    now = WatchedType.code_of(c)
+                    same = same and now.keys() == was.keys() and all(now[k] is was[k] for k in was)
+            seen = WatchedType.looked_at[cls] = (WatchedType.changes, same)
+        return seen[1]
+
+
+_methods = {}                # class -> (changes, names of what can be called on it)
+
+
+def _methods_of(cls):
+    seen = _methods.get(cls)
+    if seen is None or seen[0] != WatchedType.changes:
+        names = frozenset(k for c in cls.__mro__ for k, v in vars(c).items() if callable(v))
+        seen = _methods[cls] = (WatchedType.changes, names)
+    return seen[1]
 
 
 class Watched(metaclass=WatchedType):
@@ -116,7 +134,7 @@ def _watched_in(modules):
     for m in modules:
         for x in [m, *vars(m).values()]:
             for y in (x if type(x) in (list, tuple) else (x,)):
-                if isinstance(y, Watched):
+                if isinstance(type(y), WatchedType):
                     found[id(y)] = y
     return found.values()
 
@@ -228,19 +246,9 @@ def effect(fn, *args):
     return fn(*args)
 
 
-def _word(kind, value, held):
-    if kind in "rwt":
-        if value is None:
-            return 0
-        if isinstance(value, int):
-            return value
-        held.append(value)
-        return ctypes.addressof(getattr(value, "_obj", value))
-    if kind == "f":
-        return struct.unpack("<I", struct.pack("<f", value))[0]
-    if kind == "d":
-        return struct.unpack("<Q", struct.pack("<d", value))[0]
-    return int(value) & 0xFFFFFFFFFFFFFFFF
+def _bits(kind, value):
+    """The word of a floating-point argument."""
+    return struct.unpack("<I", struct.pack("<f", value))[0] if kind == "f" else struct.unpack("<Q", struct.pack("<d", value))[0]
 
 
 _signatures = {}
@@ -284,9 +292,12 @@ class _Inputs:
                 self.args[i] = list(self.args[i])
                 self.args[i][j] = copy
         self.spans = [(c.data_ptr(), c.data_ptr() + c.numel() * c.element_size()) for c in self.copies]
+        self.lo, self.hi = min([lo for lo, _ in self.spans], default=0), max([hi for _, hi in self.spans], default=0)
 
     def slot(self, address):
         """Which input starts at `address`; None: it lies in none."""
+        if not address or not self.lo <= address < self.hi:
+            return None
         for k, (lo, hi) in enumerate(self.spans):
             if lo <= address < hi:
                 if address != lo:
@@ -298,7 +309,7 @@ class _Inputs:
         return any(lo <= t.data_ptr() < hi for lo, hi in self.spans)
 
     def refuse(self, what, *addresses):
-        if any(a and self.slot(a) is not None for a in addresses):
+        if any(self.slot(a) is not None for a in addresses):
             raise _NotRecordable(what)
 
     def refuse_in(self, value):
@@ -331,28 +342,35 @@ class Program:
             idx, sig = _signature(name)
             words = (ctypes.c_uint64 * max(1, len(sig)))()
             patches = []
-            for i, kind in enumerate(sig):
-                words[i] = _word(kind, args[i], self.held)
-                if kind == "w" and workspace is not None and words[i] == workspace:
-                    patches += [i, len(inputs.copies)]          # one input more: the workspace of the stream it runs on
-                elif kind == "w":
-                    inputs.refuse("an input is written", words[i])
-                elif kind == "t" and args[i] is not None:
-                    inputs.refuse_set(args[i]._obj)
-                elif isinstance(args[i], ctypes.Array):          # the ops of a plan: this program's own array of them
-                    plan = type(args[i]).from_buffer_copy(args[i])
-                    words[i] = _word(kind, plan, self.held)
-                    for op in plan:
+            for i, (kind, value) in enumerate(zip(sig, args)):
+                if kind == "i" or kind == "l":
+                    words[i] = value & 0xFFFFFFFFFFFFFFFF
+                    continue
+                if value is None or kind == "f" or kind == "d":
+                    words[i] = 0 if value is None else _bits(kind, value)
+                    continue
+                if kind == "t":
+                    inputs.refuse_set(value._obj)
+                elif isinstance(value, ctypes.Array):       # the ops of a plan: this program's own array of them
+                    value = type(value).from_buffer_copy(value)
+                    for op in value:
                         inputs.refuse_set(op.out)
                         for field in ("in_mask", "in_mask2"):
-                            address = getattr(op, field)
-                            slot = inputs.slot(address) if address else None
+                            slot = inputs.slot(getattr(op, field))
                             if slot is not None:
                                 self.plan_masks.append((op, field, slot))
-                elif kind == "r" and words[i]:
-                    slot = inputs.slot(words[i])
-                    if slot is not None:
-                        patches += [i, slot]
+                if not isinstance(value, int):
+                    self.held.append(value)
+                    words[i] = ctypes.addressof(getattr(value, "_obj", value))
+                    continue
+                words[i] = value
+                slot = inputs.slot(value)
+                if slot is not None:
+                    if kind == "w":
+                        raise _NotRecordable("an input is written")
+                    patches += [i, slot]
+                elif kind == "w" and value == workspace:
+                    patches += [i, len(inputs.copies)]          # one input more: the workspace of the stream it runs on
             pa = (ctypes.c_int32 * max(1, len(patches)))(*patches)
             call.entry, call.n_args, call.n_patches = idx, len(sig), len(patches) // 2
             call.args, call.patches = ctypes.addressof(words), ctypes.addressof(pa)
@@ -373,7 +391,7 @@ class Program:
         self.settings = _get_settings(_ops_globals)
         self.hooks = [d for m in mods for d in (m._forward_hooks, m._forward_pre_hooks)]
         self.hooks += [torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks]
-        if any(self.hooks) or any(callable(getattr(type(m), k, None)) for m in mods for k in m.__dict__):
+        if any(self.hooks) or not all(_methods_of(type(m)).isdisjoint(vars(m)) for m in mods):
             raise _NotRecordable("hooked, or a method replaced in an object")
         classes = {type(m) for m in mods}
         for c in classes:
@@ -435,6 +453,7 @@ class _Cache(collections.OrderedDict):
     def __init__(self):
         super().__init__()
         self.waiting = collections.OrderedDict()
+        self.walks = 0           # passes walked since the last one that ran from a recording
 
     def keep(self, key, entry):
         if type(entry) is Program:
@@ -469,7 +488,7 @@ def _record(fns, args, free, tree, static):
     me = threading.get_ident()
     for k, fn in enumerate(fns):
         inputs, rec, watch = _Inputs(args, free), Recording(_lib.lib()), _TorchWatch()
-        _recording[me] = rec
+        _recording[me], _ops_pass.walking = rec, True
         try:
             with watch:
                 result = fn(*inputs.args)
@@ -479,6 +498,7 @@ def _record(fns, args, free, tree, static):
             continue
         finally:
             del _recording[me]
+            _ops_pass.walking = False
         if watch.seen is not None or any(_signature(name) is None for name, _ in rec.calls):
             return result, None
         try:
@@ -514,7 +534,7 @@ def replayed(record=None, dense=0, masked=1, trees=()):
     def decorate(method):
         @functools.wraps(method)
         def wrapped(self, *args, **kw):
-            if kw or not enabled or current() is not None or not _idle():
+            if kw or not enabled or _ops_pass.walking or not _idle():
                 return method(self, *args, **kw)
             key, pointers, free, held = [method.__name__], [], [], []
             for i, a in enumerate(args):
@@ -548,6 +568,7 @@ def replayed(record=None, dense=0, masked=1, trees=()):
             if ent is not None:
                 if ent.valid():
                     cache.move_to_end(key)
+                    cache.walks = 0
                     return ent.run(pointers, key[3])
                 # outdated: recorded anew at the next pass, or later and later if recordings here never last
                 w = _Waiting()
@@ -562,7 +583,14 @@ def replayed(record=None, dense=0, masked=1, trees=()):
                     cache.keep(key, ent)
             ent.seen += 1
             if ent.seen < ent.next or torch.cuda.is_current_stream_capturing():
-                return method(self, *args)
+                cache.walks += 1
+                if cache.walks > WALKS:
+                    return method(self, *args)
+                _ops_pass.walking = True
+                try:
+                    return method(self, *args)
+                finally:
+                    _ops_pass.walking = False
             # tried again after twice as many passes each time, so that a pass that cannot be recorded, or whose
             # surroundings change all the time, costs little more than it did
             ent.step = min(2 * ent.step, 256)

@@ -416,3 +416,19 @@ def test_decoder_layers_take_the_form_without_lists_where_the_plane_is_dense(stu
         layer.dense_plane = True
         assert taken(layer, mask, mask) == dense
         assert all(d.dense_plane for d in E2VIDRecurrentIncr().unetrecurrent.decoders)
+
+
+def test_layers_are_recorded_one_by_one_only_where_their_network_is_not(stub):
+    inner = lambda net: [m for m in net.modules() if m is not net and m.__dict__.get("_replay") is not None]
+    with torch.no_grad():
+        net, _ = _network()
+        for _ in range(6):
+            _step(net)
+            assert not inner(net)
+        alive = []
+        for i in range(replay.WALKS + 8):        # (states at new addresses each time: passes that are never recorded)
+            alive.append([[_cl(1, c, s, s), _cl(1, c, s, s)] for c, s in ((64, 8), (128, 4), (256, 2))])
+            net([_cl(1, 5, 16, 16), None], [[[h, None], [c, None]] for h, c in alive[-1]])
+            assert bool(inner(net)) == (i >= replay.WALKS)
+        assert any(p.runs for m in inner(net) for p in _programs(m))
+        assert not ops._pass.walking
