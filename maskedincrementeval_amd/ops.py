@@ -759,7 +759,7 @@ def split_workspace(device):
 
 
 def _new_split_workspace(dev, capturing):
-    new = lambda: torch.empty(SPLIT_WORKSPACE_BYTES // 4, dtype=torch.float32, device=torch.device("cuda", dev))
+    new = lambda: replay.apart(lambda: torch.empty(SPLIT_WORKSPACE_BYTES // 4, dtype=torch.float32, device=torch.device("cuda", dev)))
     with _split_ws_lock:
         if dev not in _captured_ws:          # made with the first of the device, so that a capture allocates nothing
             _captured_ws[dev] = new()

@@ -61,8 +61,8 @@ _NOT_CODE = frozenset(("__abstractmethods__", "__annotations__", "__doc__", "__d
 class WatchedType(abc.ABCMeta):
     """Class of the package's module classes and mixins: notes when an attribute of one is replaced, whoever does it.  (Of
     ABCMeta, so that a caller's subclass may be an abstract one, too.)"""
-    changes = 0              # replacements so far, of all classes
-    defined = {}             # class -> its attributes as they were written
+    changes = 0              # replacements so far, in all classes of the package
+    defined = {}             # class of the package -> its attributes as they were written
     looked_at = {}           # class -> (changes, as_written) when last looked at
 
     def __init__(cls, *args, **kw):
@@ -74,12 +74,13 @@ class WatchedType(abc.ABCMeta):
         return {k: v for k, v in vars(cls).items() if k not in _NOT_CODE and not k.startswith("_abc_")}
 
     def __setattr__(cls, name, value):
-        if name not in _NOT_CODE:
+        if cls in WatchedType.defined and name not in _NOT_CODE:
             WatchedType.changes += 1
         super().__setattr__(name, value)
 
     def __delattr__(cls, name):
-        WatchedType.changes += 1
+        if cls in WatchedType.defined:
+            WatchedType.changes += 1
         super().__delattr__(name)
 
     def as_written(cls):
@@ -189,8 +190,8 @@ class _TorchWatch(TorchDispatchMode):
 class Recording:
     """The library as a pass sees it while it is recorded: makes every call and notes the ones that succeed."""
 
-    def __init__(self, real):
-        self._real = real
+    def __init__(self, real, watch):
+        self._real, self.watch = real, watch
         self.calls, self.keep, self.effects = [], [], []
         self.workspace = None
 
@@ -228,6 +229,17 @@ def keep(obj):
         if r is not None:
             r.keep.append(obj)
     return obj
+
+
+def apart(fn):
+    """fn(), which runs torch operations that are no part of a pass being recorded."""
+    r = current()
+    if r is None:
+        return fn()
+    seen = r.watch.seen
+    result = fn()
+    r.watch.seen = seen
+    return result
 
 
 def shared_workspace(ws):
@@ -487,7 +499,8 @@ def _record(fns, args, free, tree, static):
     the inputs that may lie elsewhere in the next pass."""
     me = threading.get_ident()
     for k, fn in enumerate(fns):
-        inputs, rec, watch = _Inputs(args, free), Recording(_lib.lib()), _TorchWatch()
+        inputs, watch = _Inputs(args, free), _TorchWatch()
+        rec = Recording(_lib.lib(), watch)
         _recording[me], _ops_pass.walking = rec, True
         try:
             with watch:
@@ -570,7 +583,7 @@ def replayed(record=None, dense=0, masked=1, trees=()):
                     cache.move_to_end(key)
                     cache.walks = 0
                     return ent.run(pointers, key[3])
-                # outdated: recorded anew at the next pass, or later and later if recordings here never last
+                # outdated: recorded anew like a new one, or later and later if recordings here never last
                 w = _Waiting()
                 if ent.runs < 16:
                     w.step = w.next = ent.step

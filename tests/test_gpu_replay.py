@@ -215,3 +215,47 @@ def test_threads_step_networks_of_their_own(own_stream):
         if isinstance(got, BaseException):
             raise got
         _equal(got, ref)
+
+
+def test_recordings_run_for_new_inputs_on_other_streams_and_after_other_frame_sizes():
+    """One network over two frame sizes in turn, each step on another stream and at a new address: the passes run from
+    recordings, and equal the walked ones."""
+    a, b = (seed_module_(E2VIDRecurrentIncr(), seed=3).to(DEV).eval() for _ in range(2))
+    streams = [torch.cuda.current_stream()] + [torch.cuda.Stream() for _ in range(2)]
+    alive, last = [], streams[0]
+    with torch.no_grad():
+        # (from the third pass of a size on; a recording that a change of size ended is made anew one pass later)
+        for (h, w), runs in (((48, 80), 4), ((40, 56), 4), ((48, 80), 3)):
+            for n in (a, b):
+                streams[0].wait_stream(last)
+                n.forward_refresh_reservoirs(_cl(torch.ones(1, 5, h, w)), None)
+            last = streams[0]
+            for i in range(7):
+                d = _cl(event_voxel_delta(1, 5, h, w, 0.05, seed=200 + i)[0])
+                alive.append(d)
+                s = streams[i % 3]
+                s.wait_stream(last)
+                s.wait_stream(streams[0])
+                with torch.cuda.stream(s):
+                    _equal(a([d, None], None), _walked(b, [d, None], None))
+                last = s
+            assert [p.runs for p in _programs(a) if p.valid()] == [runs]
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_an_addend_that_was_the_delta_once(dtype):
+    """A layer whose addend was the same tensor as its delta while it was recorded, and is not any more."""
+    n, c, h, w = 1, 32, 19, 27
+    make = lambda: (seed_module_(mm.nnConvIncr(c, c, 3, 1, 1), seed=2).to(DEV).eval(), mm.nnReservedActivation(mm.leaky_relu_op(0.01), refine_mask=False))
+    (a, act_a), (b, act_b) = make(), make()
+    d0, m0 = gaussian_delta(n, c, h, w, 0.1, 0.2, seed=90)
+    d0, m0 = _cl(d0, dtype), m0.to(DEV)
+    with torch.no_grad():
+        for conv, act in ((a, act_a), (b, act_b)):
+            conv.forward_refresh_fused(_cl(torch.zeros(n, c, h, w), dtype), act)
+        for i in range(8):
+            # (the addend's active pixels are the delta's, in every pass)
+            d = d0 if i < 4 else _cl(gaussian_delta(n, c, h, w, 0.1, 0.2, seed=90)[0] * (1.0 + i), dtype)
+            _equal(a.forward_fused([d, m0], act_a, addend_incr=[d0, m0]), _walked(b.forward_fused, [d, m0], act_b, None, [d0, m0]))
+    assert torch.equal(act_a.in_res.reservoir, act_b.in_res.reservoir) and [p.runs for p in _programs(a)] == [5]

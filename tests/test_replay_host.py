@@ -313,10 +313,12 @@ def test_a_method_replaced_in_an_object_gets_its_calls(stub):
             assert seen
 
 
-def test_a_subclass_of_a_module_may_be_abstract():
+def test_a_subclass_of_a_module_may_be_abstract_and_changes_nothing_for_others():
     class Mine(mm.nnConvIncr, abc.ABC):
-        pass
-    assert Mine(4, 4, 3).weight.shape == (4, 4, 3, 3)
+        count = 0
+    before = replay.WatchedType.changes
+    Mine.count += 1
+    assert Mine(4, 4, 3).weight.shape == (4, 4, 3, 3) and replay.WatchedType.changes == before
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
