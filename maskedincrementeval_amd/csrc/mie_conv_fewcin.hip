@@ -410,9 +410,10 @@ __global__ __launch_bounds__(64 * FH_WAVES, 4) void k_conv_fewcin_bf16(ConvArgsT
   }
 }
 
-// 5x5, stride 1, from 2048 tiles on.  Below, a wave that does a whole tile by itself takes longer than four that share it
-// (5 -> 32 channels with a reservoir, graph of 20 calls, one workgroup a tile -> this: 1452 tiles, 409 active, 10.2 -> 12.8
-// us; 1750, 829 active, 14.0 -> 13.4; 2904, 1964 active, 25.4 -> 15.8; 38400, 3190 active, 39.7 -> 22.3, 26543 active, 256
+// 5x5, stride 1, from 2048 tiles on.  On few tiles a wave that does a whole tile by itself takes longer than four that
+// share it; the times cross between 1500 and 1750 tiles, and near the crossing the number of active ones decides, which the
+// host does not know: the line lies where this form is ahead by a clear margin (5 -> 32 channels with a reservoir, graph of
+// 20 calls, one workgroup a tile -> this: 1452 tiles, 409 active, 10.2 -> 12.8 us; 1750, 829 active, 14.0 -> 13.4; 2904, 1964 active, 25.4 -> 15.8; 38400, 3190 active, 39.7 -> 22.3, 26543 active, 256
 // -> 122, which is 4.5 TB/s).  3x3 stride 2 has so few products that the form above stays ahead at every size in use (4 ->
 // 64, 2400 tiles, 1026 active: 16.4 us against 19.6).
 constexpr unsigned FH_MIN_TILES = 2048;

@@ -58,6 +58,7 @@ class EventFrames:
         self._mask = torch.zeros((1, 1, self.out_h, self.out_w), dtype=torch.uint8, device=self.device)
         self._fmask = torch.zeros_like(self._mask)
         self._geometry = (self.kind, self.num_bins, self.height, self.width) + self.pad
+        self._index = self._mask.device.index
 
     def set_events(self, events) -> int:
         """events: (n, 4) array-like of (t, x, y, p), float64, covering every window asked for
@@ -75,21 +76,22 @@ class EventFrames:
         # (a call is as long on the host as its kernels are on the GPU; the buffers are this object's own and were made in
         # the layout the entry points take, so they are not checked again.  No address is kept: a copy of this object has
         # buffers of its own.)
-        at = (out.data_ptr(), mask.data_ptr())
+        events = self._events.data_ptr() if self._n else None
+        at, stream = (out.data_ptr(), mask.data_ptr()), torch._C._cuda_getCurrentRawStream(self._index)
         if self._sums is None:
             to_frame = lib().mie_events_to_frame
         else:
-            to_frame, at = lib().mie_events_to_frame_bf16, (self._sums.data_ptr(),) + at
-        check(to_frame(self._events.data_ptr() if self._n else None, self._n, *self._geometry, self.t_scale, float(start_old),
-                       float(start_new), self.window_size, 1 if delta else 0, *at,
-                       torch._C._cuda_getCurrentRawStream(mask.device.index)))
+            to_frame, at = lib().mie_events_to_frame_bf16, (self._sums.data_ptr(), *at)
+        status = to_frame(events, self._n, *self._geometry, self.t_scale, start_old, start_new, self.window_size, delta, *at, stream)
+        if status != 0:
+            check(status)
 
     def frame(self, start: float) -> torch.Tensor:
         """Dense (1, C, H', W') channels_last frame of the window (start, start + window_size)."""
-        self._run(0.0, start, False, self._frame, self._fmask)
+        self._run(0.0, float(start), 0, self._frame, self._fmask)
         return self._frame
 
     def delta(self, start_old: float, start_new: float) -> Tuple[torch.Tensor, torch.Tensor]:
         """[frame(start_new) - frame(start_old), pixel mask of the touched pixels]."""
-        self._run(start_old, start_new, True, self._delta, self._mask)
+        self._run(float(start_old), float(start_new), 1, self._delta, self._mask)
         return [self._delta, self._mask]
