@@ -129,14 +129,18 @@ def outdate(obj):
             program.end()
 
 
+_PLAIN = frozenset((dict, collections.OrderedDict, set, bool, int, float, str, type(None), torch.Tensor))
+
+
 def _watched_in(modules):
     """The watched objects a pass over these modules reads: themselves, and the reservoirs they hold."""
-    found = {}
+    found = {id(m): m for m in modules if isinstance(type(m), WatchedType)}
     for m in modules:
-        for x in [m, *vars(m).values()]:
-            for y in (x if type(x) in (list, tuple) else (x,)):
-                if isinstance(type(y), WatchedType):
-                    found[id(y)] = y
+        for x in vars(m).values():
+            if type(x) not in _PLAIN:
+                for y in (x if type(x) in (list, tuple) else (x,)):
+                    if isinstance(type(y), WatchedType):
+                        found[id(y)] = y
     return found.values()
 
 
@@ -318,11 +322,13 @@ class _Inputs:
         return None
 
     def holds(self, t):
-        return any(lo <= t.data_ptr() < hi for lo, hi in self.spans)
+        at = t.data_ptr()
+        return self.lo <= at < self.hi and any(lo <= at < hi for lo, hi in self.spans)
 
     def refuse(self, what, *addresses):
-        if any(self.slot(a) is not None for a in addresses):
-            raise _NotRecordable(what)
+        for a in addresses:
+            if a and self.lo <= a < self.hi and self.slot(a) is not None:
+                raise _NotRecordable(what)
 
     def refuse_in(self, value):
         """No part of a result or of a change of host state may be an input: the next pass has others."""
