@@ -297,10 +297,11 @@ class _Inputs:
     delta in one place and the addend in another), has its own address there."""
 
     def __init__(self, args, free):
-        self.args, self.copies = list(args), []
+        self.args, self.given, self.copies = list(args), [], []
         for i, j in free:
             given = self.args[i] if j is None else self.args[i][j]
             copy = given.detach().clone()
+            self.given.append(given)
             self.copies.append(copy)
             if j is None:
                 self.args[i] = copy
@@ -341,6 +342,17 @@ class _Inputs:
             self.refuse_in(list(value.values()))
         elif hasattr(value, "c_struct"):
             self.refuse_set(value.c_struct)
+
+    def give_back(self, value):
+        """A result with the inputs it hands on, in place of their copies."""
+        if type(value) in (list, tuple):
+            return type(value)([self.give_back(x) for x in value])
+        if type(value) is dict:
+            return {k: self.give_back(x) for k, x in value.items()}
+        for given, copy in zip(self.given, self.copies):
+            if value is copy:
+                return given
+        return value
 
     def refuse_set(self, ts):
         self.refuse("a tile set over an input", ts.pixmask, ts.tiles, ts.stale, ts.counts, ts.flags)
@@ -448,7 +460,8 @@ class Program:
 
     def run(self, pointers, device):
         self.runs += 1
-        calls, effects, result = self.calls, self.effects, self.result
+        # (an effect, or another thread, may end this program meanwhile)
+        calls, held, effects, result = self.calls, self.held, self.effects, self.result
         for op, field, slot in self.plan_masks:
             setattr(op, field, pointers[slot])
         if self.uses_workspace:
@@ -519,13 +532,13 @@ def _record(fns, args, free, tree, static):
             del _recording[me]
             _ops_pass.walking = False
         if watch.seen is not None or any(_signature(name) is None for name, _ in rec.calls):
-            return result, None
+            return inputs.give_back(result), None
         try:
             inputs.refuse_in(result)
             inputs.refuse_in([effect_args for _, effect_args in rec.effects])
             return result, Program(rec, inputs, _copy(result), tree, static)
         except _NotRecordable:
-            return result, None
+            return inputs.give_back(result), None
 
 
 def _static_key(v, held):
@@ -555,7 +568,7 @@ def replayed(record=None, dense=0, masked=1, trees=()):
         def wrapped(self, *args, **kw):
             if kw or not enabled or _ops_pass.walking or not _idle():
                 return method(self, *args, **kw)
-            key, pointers, free, held = [method.__name__], [], [], []
+            key, pointers, free, held, device = [method.__name__], [], [], [], None
             for i, a in enumerate(args):
                 if a is not None and i < dense + masked:
                     x = a if i < dense else a[0]
@@ -563,7 +576,8 @@ def replayed(record=None, dense=0, masked=1, trees=()):
                         return method(self, *args)
                     pointers.append(x.data_ptr())
                     free.append((i, None if i < dense else 0))
-                    key += (x.shape, x.dtype, x.device.index)
+                    device = x.device.index
+                    key += (x.shape, x.dtype, device)
                     m = None if i < dense or len(a) < 2 else a[1]
                     if torch.is_tensor(m):
                         n, _, h, w = x.shape
@@ -588,7 +602,7 @@ def replayed(record=None, dense=0, masked=1, trees=()):
                 if ent.valid():
                     cache.move_to_end(key)
                     cache.walks = 0
-                    return ent.run(pointers, key[3])
+                    return ent.run(pointers, device)
                 # outdated: recorded anew like a new one, or later and later if recordings here never last
                 w = _Waiting()
                 if ent.runs < 16:

@@ -184,6 +184,16 @@ def test_a_recording_holds_no_input(stub):
     assert len(sizes) == 1          # the tile set's own pixel mask; no copy of an input's
 
 
+def test_a_pass_that_hands_an_input_on_is_walked_and_hands_on_the_callers(stub):
+    x, m = _cl(1, 8, 8, 8), torch.ones(1, 1, 8, 8, dtype=torch.uint8)
+
+    def body(pair):
+        ops.lib().mie_mul_dense(pair[0].data_ptr(), 0, 0, 1, 0, 0)
+        return [pair[0], (pair[1], {"mask": pair[1]})]
+    result, program = replay._record([body], ([x, m],), [(0, 0), (0, 1)], (), [])
+    assert program is None and result[0] is x and result[1][0] is m and result[1][1]["mask"] is m
+
+
 def test_a_planning_pass_asks_the_library_for_its_shapes(stub):
     """What decides a layer's kernels is asked in the planning pass as in the compute pass: both walk the same layers."""
     stub.mie_conv_f32x3_takes = lambda *args: 1
