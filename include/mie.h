@@ -83,8 +83,9 @@ extern "C" {
  * mie_conv_f32x3_takes) and mie_tconv2x_masked / mie_tconv2x_refresh (c1, c2 multiples of 64), with filter_mc
  * packed for it; every buffer is what it is for MIE_DTYPE_F32.  Values must be finite and below the bf16
  * maximum (3.39e38): an infinity, or a value that rounds to one in bf16, splits into inf - inf and gives
- * NaN where the fp32 instruction would give an infinity -- except in convs at stride 2, which compute the
- * outputs concerned again in fp32 and give what the fp32 instruction gives. */
+ * NaN where the fp32 instruction would give an infinity -- except in convs at stride 2 on few tiles with a
+ * workspace (mie_conv_masked_ws: tiles x cout/32 <= 128), which compute the outputs concerned again in fp32
+ * and give what the fp32 instruction gives. */
 #define MIE_DTYPE_F32_BF16X3 2
 
 /* frame kinds of mie_events_to_frame */

@@ -282,9 +282,11 @@ __device__ __forceinline__ bool finite4(const float4& v) {
 // Four output channels of a conv in plain fp32, straight from the inputs and the plain filter, with the epilogue: what is
 // done instead where a sum of the three-term form is not finite.  That form makes NaN of an infinite delta and of a finite
 // one that rounds to an infinite bf16 term (3.39e38 and more); either leaves no finite sum, so the test of the sum finds all
-// of them, and finite sums cost that test only.  For the 5x5 stride-2 convs, whose launches of few tiles ran on the fp32
-// instruction before and carried such values (the forms at stride 1 do not: mie.h, MIE_DTYPE_F32_BF16X3).  It runs behind
-// the ordinary stores, over the groups these left out: inside them the loops cost registers (1-2 us a launch).
+// of them, and finite sums cost that test only.  For the 5x5 stride-2 convs of few tiles with a workspace, which ran on the
+// fp32 instruction before and carried such values (the others do not: mie.h, MIE_DTYPE_F32_BF16X3).  It runs behind the
+// ordinary stores, over the groups these left out: inside them the loops cost registers (1-2 us a launch).  Alone, without
+// -> with: 32->64 at 64x96 10.9 -> 11.1 us, split 64->128 at 32x48 11.2 -> 11.3; on planes of many tiles it would be
+// 24.4 -> 24.7 (64->128 at 132x176) and 25.8 -> 26.5 (128->256 at 66x88).
 // (The arguments are read from memory anew, through conv_args_again: taken from the kernel's `a`, a dozen fields more stayed
 // in registers through the contraction, whose scalar spills cost 0.5-1.1 us a launch.)
 template <typename T, int K, int S>
@@ -328,8 +330,10 @@ __device__ void conv_quad_again(const ConvArgsT<T>& a, int n, int oy, int ox, in
 // eight v_mfma_f32_32x32x2_f32 take 8 x 64 cycles to do.  Chunks of 32 channels (two units per tap; stride 2, whose
 // staged tile is four times the size: 16 channels, one unit per tap); where the k-split has more waves than a tap
 // has units it is over (sub-chunk, tap class).  Global loads, masks, epilogue: fp32.
+//
+// AGAIN (X3 only): outputs whose sum is not finite are computed again in fp32 (conv_quad_again).
 template <typename T, int K, int S, int WN, int NB, bool HALF, bool GATES = false, bool UP = false, bool SPLIT = false,
-          bool X3 = false>
+          bool X3 = false, bool AGAIN = false>
 // (Build with -mllvm -pragma-unroll-threshold=65536: the unit loop of the 128-column 5x5 / 7x7 kernels is 100 / 196
 // positions long, and where the compiler refuses to unroll it the operand ring is indexed at run time and lands in
 // scratch memory -- a factor of three in time.)
@@ -1131,7 +1135,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         for (int i = 0; i < PB; ++i)
           if (e_ok[i]) *reinterpret_cast<float4*>(plane + e_off[i]) = v[i];
       } else {
-        if constexpr (X3 && S == 2) {
+        if constexpr (AGAIN) {
 #pragma unroll
           for (int i = 0; i < PB; ++i)
             if (e_ok[i] && !finite4(v[i])) {
@@ -1142,7 +1146,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         conv_epilogue_store4<T, PB>(a, e_off, e_co, e_ok, v, e_r0, e_add, e_live);
       }
     }
-    if constexpr (X3 && S == 2 && !SPLIT) {
+    if constexpr (AGAIN) {
       if (__builtin_expect(__ballot(bad_bits != 0u) != 0ull, 0))
         for (int g = 0; g < PER; ++g) {
           const int idx = tid + 256 * g, p = idx / QPP, co = co0 + 4 * (idx - p * QPP);
@@ -1464,6 +1468,13 @@ bool launch_x3(const ConvArgsT<float>& a0, unsigned cap, hipStream_t st) {
   ConvArgsT<float> a = a0;
   const int cout = a.cout;
   if (!x3_takes(K, S, a.c1, UP ? 0 : a.c2, cout)) return false;
+  if constexpr (S == 2) {
+    // few tiles and a workspace, but too few chunks to split (32->64 at 64x96): the same outputs as from the split form
+    if (a.ws != nullptr && !a.refresh && (long long)cap * (cout / 32) <= 128) {
+      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 1, 1, false, GATES, UP, false, true, true>), dim3(xcd_plan(a, cap, cout / 32, K, UP), cout / 32), dim3(256), 0, st, a);
+      return true;
+    }
+  }
   switch (pick_slab_x3(cout, cap, S)) {
     case 128:
       hipLaunchKernelGGL((k_conv_mfma<float, K, S, 4, 1, false, GATES, UP, false, true>), dim3(xcd_plan(a, cap, cout / 128, K, UP), cout / 128), dim3(256), 0, st, a);

@@ -239,9 +239,9 @@ def _stride2_split(x, wt, mode, mask=None, second=0):
 @pytest.mark.parametrize("cin,cout,h,w,second", [(64, 128, 32, 48, 0), (128, 256, 16, 24, 0), (64, 64, 33, 29, 32), (64, 32, 7, 5, 0),
                                                      (32, 64, 64, 96, 0), (32, 64, 132, 176, 0), (128, 256, 66, 88, 0)])
 def test_stride_2_convs_against_fp64_and_with_non_finite_deltas(cin, cout, h, w, second):
-    """Error of the three-term form (split, unsplit on few tiles, unsplit on many) against fp64 next to the fp32 instruction's (both bounded like the unsplit forms,
-    4e-7 of sum |x||w|: three fp32 roundings), then the same conv over infinite, NaN and huge deltas: what an fp32 conv
-    gives, in both forms.  A masked pixel's value is not read."""
+    """Error of the three-term form (split, unsplit on few tiles, unsplit on many) against fp64 next to the fp32 instruction's
+    (both bounded like the unsplit forms, 4e-7 of sum |x||w|: three fp32 roundings), then, on few tiles, the same conv over
+    infinite, NaN and huge deltas: what an fp32 conv gives, in both forms.  A masked pixel's value is not read."""
     g = torch.Generator().manual_seed(cin + h)
     x, wt = torch.randn(1, cin, h, w, generator=g), he_normal_conv_weight(cout, cin, 5, 7)
     ref = F.conv2d(x.double(), wt.double(), stride=2, padding=2)
@@ -252,6 +252,8 @@ def test_stride_2_convs_against_fp64_and_with_non_finite_deltas(cin, cout, h, w,
         e = (got.double() - ref).abs()
         err[mode] = (e / bound).max().item(), (e.norm() / ref.norm()).item()
     assert max(err["bf16x3"][0], err["native"][0]) < 4e-7 and err["bf16x3"][1] <= err["native"][1], err
+    if -(-((h + 1) // 2) // 8) * -(-((w + 1) // 2) // 8) * (cout // 32) > 128:
+        return              # (many tiles: the three-term form's own rule, as at stride 1)
     bad, mask = x.clone(), torch.ones(1, 1, h, w, dtype=torch.uint8)
     spots = {(1, 2, 1): float("inf"), (5, h - 1, w - 1): float("-inf"), (cin - 1, h // 2, 0): 3.4e38, (cin // 2, 0, w // 2): float("nan")}
     for (c, y, x_), v in spots.items():
