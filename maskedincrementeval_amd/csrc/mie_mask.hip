@@ -720,68 +720,90 @@ extern "C" int mie_build_mask_tiles_thresholded(const void* delta, int c, int dt
   return mie_check_launch(who);
 }
 
-// ---- every tile set of a network in two launches ------------------------------------------------
+// ---- every tile set of a network in one or two launches ------------------------------------------
 // mie_build_mask_plan runs a sequence of mie_build_mask_tiles calls -- every structural mask of a network is a chain
-// of footprints of the input pixel mask -- as two kernels.  In the first, a workgroup keeps the pixel masks of one
-// sample's chain as BITMAPS in LDS (a 264x352 plane is 11.6 KB): a footprint is then a handful of word operations
-// per 32 pixels -- the window of a conv is the OR of the rows it covers, shifted left and right (stride 2: the even
-// bits of that, compressed); bilinear x2 and the stride-2 transposed conv interleave two such ORs bit by bit --
-// instead of k*k byte loads per pixel, and no launch or memory round trip separates one mask of the chain from the
-// next.  That part is so cheap that several workgroups per sample each walk the whole chain on their own and share
-// only what goes to memory: of every set's pixel mask (bytes, 16 per store where the rows allow it) and tile flags a
-// workgroup writes its slice, so the stores of a large plane do not queue up behind one CU.  The second kernel
-// ranks the lists of all sets, one block per 4096 tiles of each (as k_compact_tiles).  Slots of LDS are handed out
-// on the host by lifetime (a mask is dropped after its last reader).
+// of footprints of the input pixel mask.  A workgroup keeps the pixel masks of one sample's chain as BITMAPS in LDS (a
+// 264x352 plane is 11.6 KB): a footprint is then a handful of word operations per 32 pixels -- the window of a conv is
+// the OR of the rows it covers, shifted left and right (stride 2: the even bits of that, compressed); bilinear x2 and
+// the stride-2 transposed conv interleave two such ORs bit by bit -- instead of k*k byte loads per pixel, and no launch
+// or memory round trip separates one mask of the chain from the next.  Several workgroups per sample each walk the whole
+// chain on their own and share only what goes to memory.
+//
+// What bounds it is the chain: one step after the other, a barrier between them, next to no work in the small planes.
+// A step costs the latency of the instructions of one wave (some 1100 clocks, hardly fewer for a plane of 16 words than
+// for one of 700), so there are few of them and each does little:
+//  * a same-size conv window over the result of another is one wider window over what that one read (both padded by half
+//    their size: every pixel between two pixels of the plane is in the plane), so the host lets a step read its input's
+//    input where the wider window has a form below: the four convs of a bottleneck are one level, and so are a conv and
+//    the stride-2 conv behind it;
+//  * steps that do not depend on each other share a level (a barrier interval), each on waves of its own;
+//  * a wave finds its step's parameters in one register, a word per lane, asked for a level ahead; a wave without a
+//    step goes straight to the barrier;
+//  * rows outside the plane are read from words of zeros, by address, instead of being masked after the load;
+//  * where all bitmaps fit the LDS together nothing is written between the levels: the pixel masks of all sets go to
+//    memory at the end, 16 pixels a thread, a slice per workgroup.  Where they do not, a bitmap is dropped after its last
+//    reader and waves of their own write the masks of a level beside the next one's bitmaps.
+// With one sample (all bitmaps resident, sets of at most 4096 tiles) a workgroup OWNS sets: it alone reads and writes their
+// flags, and ranks their lists itself at the end, so the plan is one launch.  With a batch the lists run over all samples:
+// a workgroup writes the flags of its slice of every set and k_plan_compact ranks the lists behind it, one block per 4096
+// tiles.
 namespace {
 
-constexpr int PLAN_THREADS = COMPACT_THREADS;
+constexpr int PLAN_THREADS = 1024;
+constexpr int PLAN_WAVES = PLAN_THREADS / 64;
+constexpr int PLAN_COMPUTE_WAVES = 12;                 // of a level's bitmaps where the others write the level before it
+constexpr int PLAN_WRITE_WAVES = PLAN_WAVES - PLAN_COMPUTE_WAVES;
+constexpr int PLAN_LEVEL_STEPS = 8;                    // steps of a level (not resident: at least one writing wave each)
 constexpr int PLAN_MAX_SHARES = 64;                    // workgroups per sample
-constexpr int PLAN_PIXELS_PER_SHARE = 8192;            // of the plan's largest plane: 128 tiles, so a thread owns at most one
-constexpr int PLAN_STEP_LOAD = 0, PLAN_STEP_FOOT = 1;
-constexpr int PLAN_IN_NONE = -1, PLAN_IN_ALL = -2;
+constexpr int PLAN_PIXELS_PER_SHARE = 8192;            // of the plan's largest plane
+constexpr int PLAN_OWNED_TILES = 4096;                 // largest set a workgroup ranks by itself
+constexpr int PLAN_KIND_LOAD = 0, PLAN_KIND_FOOT = 1;
+constexpr unsigned PLAN_IN_NONE = 0xffffu;             // instead of an LDS word offset (at most 40960)
+constexpr int PLAN_IDLE = 255;                         // task table: nothing to do for this wave in this level
 
-struct PlanStep {
-  int kind;                 // PLAN_STEP_LOAD: bytes -> bitmap; PLAN_STEP_FOOT: footprint of one or two bitmaps
-  int in1, in2;             // LDS word offsets of the input bitmaps (PLAN_IN_*)
-  int out;                  // LDS word offset of the bitmap this step makes
-  int h_in, w_in, h_out, w_out;
-  int geom;                 // foot | k << 8 | stride << 16 | pad << 24
-  int flag_off, flag_cnt;   // this step's part of the workgroup's flag area in LDS: first word, words
-  int key;                  // which specialised form of the footprint runs (PLAN_KEY_*), chosen on the host
-  unsigned m_words, m_units, m_tiles;   // plan_magic of the words per row, the 16-pixel units per row, the tiles per row
-  int pad_;
-  const uint8_t* ext;       // LOAD: the mask in memory, [n, h_out, w_out]
-  uint8_t* pixmask;
-  uint32_t* flags;
+// A step's words (lane l of a wave that works on it holds word l).
+enum {
+  PS_IN,            // LDS word offsets of the input bitmaps: in1 | in2 << 16
+  PS_OUT_WIN,       // LDS word offset of the bitmap it makes | input width << 16
+  PS_HIN, PS_HOUT,
+  PS_WOUT_KEY,      // output width | PLAN_KEY_* << 16 | kind << 24 | size of its accesses to the mask in memory << 28 (2: 16 bytes, 1: 4, 0: 1)
+  PS_GEOM,          // foot | k << 8 | stride << 16 | pad << 24
+  PS_MWORDS,        // plan_magic of the words per row
+  PS_MUNITS,        // plan_magic of the 16-pixel units per row
+  PS_WAVES,         // computing waves: first | number << 8; writing waves: first << 16 | number << 24
+  PS_UBASE,         // 16-pixel units of the sets before it
+  PS_FL,            // byte offset of its tiles in the workgroup's flag area
+  PS_OWN,           // sets owned: the next set of the same owner, or PLAN_IDLE; else tiles of the set per share
+  PS_MTILES,        // plan_magic of the tiles per row
+  PS_PIX, PS_PIX_HI,          // pixel mask in memory (LOAD: the mask to read)
+  PS_FLAGS, PS_FLAGS_HI, PS_TILES, PS_TILES_HI, PS_STALE, PS_STALE_HI, PS_COUNTS, PS_COUNTS_HI,
+  PS_WORDS
 };
 
 struct PlanArgs {
-  int n_steps, n, flag_words, pad1_;
-#ifdef MIE_PLAN_PROFILE
-  int* dbg;                // measurement builds only: 2 ticks per step
-#endif
-  PlanStep st[MIE_PLAN_MAX_STEPS];
+  int n_steps, n_levels, n_loads;         // steps are in level order; the first n_loads are the masks from memory of level 0
+  int first_last;                         // the first step of the last level
+  int resident;                           // all bitmaps stay: everything is written at the end
+  int owned;                              // a workgroup owns sets and ranks them (resident only); 0: slices, lists by k_plan_compact
+  int units, pad_;                        // 16-pixel units of all sets
+  int zero_off, flag_off;                 // LDS: words of zeros; a byte per tile (owned: old state; not resident: new state)
+  uint32_t st[MIE_PLAN_MAX_STEPS * PS_WORDS];
+  uint8_t task[(MIE_PLAN_MAX_STEPS + 3) * PLAN_WAVES];     // [level][wave] -> step
+  uint8_t head[PLAN_MAX_SHARES];          // the first set each share owns, or PLAN_IDLE
 };
-constexpr int PLAN_HEAD = MIE_PLAN_MAX_STEPS * (int)(sizeof(PlanStep) / 4);     // words of LDS in front of the bitmaps: the steps
+constexpr int PLAN_ZERO_WORDS = 8;
 
-// a step's fields, read from LDS (the same address in every lane), as scalars
-__device__ __forceinline__ int plan_uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// (To be called where every lane of the wave is active: a load that feeds it may move down to it, and the lanes that a
+// branch around both has switched off would not have loaded their word.)
+__device__ __forceinline__ uint32_t plan_word(uint32_t pw, int i) { return (uint32_t)__builtin_amdgcn_readlane((int)pw, i); }
 template <typename P>
-__device__ __forceinline__ P* plan_uni(P* p) {
-  const unsigned long long v = reinterpret_cast<unsigned long long>(p);
-  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-  return reinterpret_cast<P*>(((unsigned long long)hi << 32) | lo);
+__device__ __forceinline__ P* plan_ptr(uint32_t pw, int i) {
+  const unsigned long long v = ((unsigned long long)plan_word(pw, i + 1) << 32) | plan_word(pw, i);
+  return reinterpret_cast<P*>(v);
 }
-__device__ __forceinline__ PlanStep plan_uni(const PlanStep& s) {
-  PlanStep u;
-  u.kind = plan_uni(s.kind); u.in1 = plan_uni(s.in1); u.in2 = plan_uni(s.in2); u.out = plan_uni(s.out);
-  u.h_in = plan_uni(s.h_in); u.w_in = plan_uni(s.w_in); u.h_out = plan_uni(s.h_out); u.w_out = plan_uni(s.w_out);
-  u.geom = plan_uni(s.geom); u.flag_off = plan_uni(s.flag_off); u.flag_cnt = plan_uni(s.flag_cnt); u.key = plan_uni(s.key);
-  u.m_words = (unsigned)plan_uni((int)s.m_words); u.m_units = (unsigned)plan_uni((int)s.m_units);
-  u.m_tiles = (unsigned)plan_uni((int)s.m_tiles); u.pad_ = 0;
-  u.ext = plan_uni(s.ext); u.pixmask = plan_uni(s.pixmask); u.flags = plan_uni(s.flags);
-  return u;
-}
+__device__ __forceinline__ int plan_kind(uint32_t pw) { return (int)((plan_word(pw, PS_WOUT_KEY) >> 24) & 15u); }
+
+__device__ __forceinline__ uint32_t plan_dot4(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_udot4(a, b, c, false); }
 
 // bit x of the result = bit (x + t) of the row whose words around the current one are prev, cur, next (|t| < 32):
 // 32 bits out of the middle of two adjacent words (v_alignbit_b32), no branch on the sign of t
@@ -807,128 +829,19 @@ __device__ __forceinline__ uint32_t plan_spread(uint32_t x) {
   x = (x | (x << 1)) & 0x55555555u;
   return x;
 }
-// four mask bytes -> four bits (a byte counts when it is not zero)
-__device__ __forceinline__ uint32_t plan_nibble(uint32_t v) {
-  const uint32_t t = (v | ((v | 0x80808080u) - 0x01010101u)) & 0x80808080u;     // bit 7 of every non-zero byte
-  return ((t >> 7) & 1u) | ((t >> 14) & 2u) | ((t >> 21) & 4u) | ((t >> 28) & 8u);
+// eight mask bytes -> eight bits (a byte counts when it is not zero): 0 / 1 in every byte, then the dot product with the
+// bits' places
+__device__ __forceinline__ uint32_t plan_ones(uint32_t v) {
+  return ((((v & 0x7f7f7f7fu) + 0x7f7f7f7fu) | v) >> 7) & 0x01010101u;
 }
-// four bits -> four bytes of 0 / 1
+__device__ __forceinline__ uint32_t plan_octet(uint32_t a, uint32_t b) {
+  return plan_dot4(plan_ones(a), 0x08040201u, plan_dot4(plan_ones(b), 0x80402010u, 0u));
+}
+// four mask bytes, or the four bytes of a word of a bitmap -> four bits
+__device__ __forceinline__ uint32_t plan_nibble(uint32_t v) { return plan_dot4(plan_ones(v), 0x08040201u, 0u); }
+// four bits -> four bytes of 0 / 1 (bit i to bit 8 i: a copy shifted by 7 i each, then the one bit of each byte)
 __device__ __forceinline__ uint32_t plan_bytes(uint32_t nib) {
-  return (nib & 1u) | ((nib & 2u) << 7) | ((nib & 4u) << 14) | ((nib & 8u) << 21);
-}
-
-// The input of a step: one bitmap, or (TWO) the OR of two.  Every load below goes out unconditionally from a clamped
-// address and is masked afterwards, so that the loads of a whole window are in flight together instead of one row
-// after the other.
-template <bool TWO>
-struct PlanRowAcc {
-  const uint32_t* b1;
-  const uint32_t* b2;
-  int ww, h;
-  __device__ __forceinline__ uint32_t at(int y, int j) const {
-    return TWO ? (b1[y * ww + j] | b2[y * ww + j]) : b1[y * ww + j];
-  }
-  // row y if it exists, else all zeros: (clamped row, mask)
-  __device__ __forceinline__ int row(int y, uint32_t& m) const {
-    const bool ok = y >= 0 && y < h;
-    m = ok ? 0xffffffffu : 0u;
-    return ok ? y : 0;
-  }
-};
-
-// One output word of a footprint step: pixels 32*j .. 32*j+31 of row oy.  K = 0: kernel size read at run time.
-struct PlanGeom { int k, p; };
-template <int FOOT, int K, int S, bool TWO>
-__device__ __forceinline__ uint32_t plan_foot_word(const PlanGeom& g, const PlanRowAcc<TWO>& in, int oy, int j) {
-  // kernel size and padding: compile-time constants for the common footprints (K > 0: "same" padding K / 2)
-  const PlanGeom s = {K > 0 ? K : g.k, K > 0 ? K / 2 : g.p};
-  const int k = s.k;
-  const int ww = in.ww, h = in.h;
-  if (FOOT == MIE_FOOT_CONV && S == 1) {
-    const int lo = -s.p;
-    const bool okp = j > 0, okc = j < ww, okn = j + 1 < ww;
-    const int jp = okp ? j - 1 : 0, jc = okc ? j : 0, jn = okn ? j + 1 : 0;
-    uint32_t vp = 0u, vc = 0u, vn = 0u;
-#pragma unroll
-    for (int ky = 0; ky < k; ++ky) {
-      uint32_t m;
-      const int iy = in.row(oy - s.p + ky, m);
-      vp |= in.at(iy, jp) & m;
-      vc |= in.at(iy, jc) & m;
-      vn |= in.at(iy, jn) & m;
-    }
-    vp = okp ? vp : 0u; vc = okc ? vc : 0u; vn = okn ? vn : 0u;
-    uint32_t r = 0u;
-#pragma unroll
-    for (int t = 0; t < k; ++t) r |= plan_shift(vp, vc, vn, lo + t);
-    return r;
-  }
-  if (FOOT == MIE_FOOT_CONV) {
-    // stride 2: the window OR at input positions 64*j .. 64*j+63, of which the even ones are the outputs
-    const int lo = -s.p;
-    const int j0 = 2 * j - 1;
-    bool ok[4];
-    int jj[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      ok[q] = j0 + q >= 0 && j0 + q < ww;
-      jj[q] = ok[q] ? j0 + q : 0;
-    }
-    uint32_t v[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int ky = 0; ky < k; ++ky) {
-      uint32_t m;
-      const int iy = in.row(2 * oy - s.p + ky, m);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] |= in.at(iy, jj[q]) & m;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = ok[q] ? v[q] : 0u;
-    uint32_t d0 = 0u, d1 = 0u;
-#pragma unroll
-    for (int t = 0; t < k; ++t) {
-      d0 |= plan_shift(v[0], v[1], v[2], lo + t);
-      d1 |= plan_shift(v[1], v[2], v[3], lo + t);
-    }
-    return plan_even_bits(d0) | (plan_even_bits(d1) << 16);
-  }
-  const int js = j >> 1, sh = 16 * (j & 1);
-  const bool okp = js > 0, okc = js < ww, okn = js + 1 < ww;
-  const int jp = okp ? js - 1 : 0, jc = okc ? js : 0, jn = okn ? js + 1 : 0;
-  uint32_t vp = 0u, vc = 0u, vn = 0u;
-  if (FOOT == MIE_FOOT_UP2X) {
-    // out[2m] = in[m-1] | in[m], out[2m+1] = in[m] | in[m+1], rows and columns alike (clamping at the border adds
-    // nothing: the clamped neighbour is the pixel itself)
-    int r0, r1;
-    up2x_src(oy, h, r0, r1);
-    vp = in.at(r0, jp) | in.at(r1, jp);
-    vc = in.at(r0, jc) | in.at(r1, jc);
-    vn = in.at(r0, jn) | in.at(r1, jn);
-    vp = okp ? vp : 0u; vc = okc ? vc : 0u; vn = okn ? vn : 0u;
-    const uint32_t ev = vc | plan_shift(vp, vc, vn, -1), od = vc | plan_shift(vp, vc, vn, 1);
-    return plan_spread(ev >> sh) | (plan_spread(od >> sh) << 1);
-  }
-  // MIE_FOOT_TCONV, stride 2: output 2m + e sees input m + (e + p - kk) / 2 for the taps kk with e + p - kk even
-  const int e = oy & 1, m_ = oy >> 1;
-#pragma unroll
-  for (int ky = 0; ky < k; ++ky) {
-    const int d2 = e + s.p - ky;
-    uint32_t m;
-    const int iy = in.row(m_ + (d2 >> 1), m);
-    m = (d2 & 1) ? 0u : m;
-    vp |= in.at(iy, jp) & m;
-    vc |= in.at(iy, jc) & m;
-    vn |= in.at(iy, jn) & m;
-  }
-  vp = okp ? vp : 0u; vc = okc ? vc : 0u; vn = okn ? vn : 0u;
-  uint32_t ev = 0u, od = 0u;
-#pragma unroll
-  for (int kx = 0; kx < k; ++kx) {
-    const int d2 = s.p - kx;
-    if (d2 & 1) od |= plan_shift(vp, vc, vn, (d2 + 1) >> 1);
-    else ev |= plan_shift(vp, vc, vn, d2 >> 1);
-  }
-  return plan_spread(ev >> sh) | (plan_spread(od >> sh) << 1);
+  return __umul24(nib, 0x204081u) & 0x01010101u;
 }
 
 // floor(a / d) with m = plan_magic(d) = ceil(2^32 / d) worked out on the host: one multiply instead of a division by a
@@ -940,209 +853,556 @@ __device__ __forceinline__ int plan_div(int a, unsigned m) {
   const int q = (int)__umulhi((unsigned)a, m);
   return m == 0u ? a : q;
 }
-
-// Threads of a workgroup by role: the first PLAN_COMPUTE make the bitmap of a step while PLAN_PIX others write the
-// pixel mask of the step before it and the last PLAN_FLG its tile flags, so that none waits for another's
-// instruction stream: a step is a few hundred instructions of each kind and nothing else to hide them behind.
-constexpr int PLAN_COMPUTE = 640;
-constexpr int PLAN_PIX = 192;
-constexpr int PLAN_FLG = PLAN_THREADS - PLAN_COMPUTE - PLAN_PIX;
+// the bits of word j of a row of w pixels that are pixels
+__device__ __forceinline__ uint32_t plan_valid(int w, int j) {
+  const int left = w - 32 * j;
+  return left >= 32 ? 0xffffffffu : ((1u << left) - 1u);
+}
 
 // specialised forms of the footprint (kernel size, stride and "same" padding K / 2 at compile time)
-enum { PLAN_KEY_GENERIC = 0, PLAN_KEY_C11, PLAN_KEY_C31, PLAN_KEY_C51, PLAN_KEY_C32, PLAN_KEY_C52, PLAN_KEY_UP, PLAN_KEY_T32, PLAN_KEY_T52 };
+enum { PLAN_KEY_GENERIC = 0, PLAN_KEY_C11, PLAN_KEY_C31, PLAN_KEY_C51, PLAN_KEY_C71, PLAN_KEY_C91, PLAN_KEY_C111, PLAN_KEY_C32, PLAN_KEY_C52,
+       PLAN_KEY_C72, PLAN_KEY_C92, PLAN_KEY_UP, PLAN_KEY_T32, PLAN_KEY_T52, PLAN_KEY_ALL };
+constexpr int PLAN_MAX_K1 = 11, PLAN_MAX_K2 = 9;       // widest windows of stride 1 and 2 among them
+constexpr int plan_key_size(int key) {
+  return key == PLAN_KEY_C31 || key == PLAN_KEY_C32 || key == PLAN_KEY_T32 ? 3 : key == PLAN_KEY_C51 || key == PLAN_KEY_C52 || key == PLAN_KEY_T52 ? 5
+         : key == PLAN_KEY_C71 || key == PLAN_KEY_C72 ? 7 : key == PLAN_KEY_C91 || key == PLAN_KEY_C92 ? 9 : key == PLAN_KEY_C111 ? 11 : 1;
+}
 
-// the bitmap of a footprint step: compute thread r of nthr takes words r, r + nthr, ...
-template <int FOOT, int K, int S, bool TWO>
-__device__ __forceinline__ void plan_foot_all(const PlanStep& s, const uint32_t* bm, uint32_t* out, int r, int nthr) {
-  PlanRowAcc<TWO> in;
-  in.b1 = bm + s.in1;
-  in.b2 = bm + ((TWO && s.in2 >= 0) ? s.in2 : s.in1);
-  in.ww = (s.w_in + 31) >> 5;
-  in.h = s.h_in;
-  const int ho = s.h_out, wo = s.w_out, wwo = (wo + 31) >> 5;
-  PlanGeom g;
-  g.k = (s.geom >> 8) & 255; g.p = (s.geom >> 24) & 255;
-  for (int wd = r; wd < ho * wwo; wd += nthr) {
-    const int y = plan_div(wd, s.m_words), j = wd - y * wwo;
-    const int left = wo - 32 * j;
-    const uint32_t valid = left >= 32 ? 0xffffffffu : ((1u << left) - 1u);
-    out[wd] = plan_foot_word<FOOT, K, S, TWO>(g, in, y, j) & valid;
+// What the computing waves of a step know of it.
+struct PlanIn {
+  const uint32_t* lds;
+  int in1, in2;             // LDS word offsets (in2: that of in1 where there is one input)
+  int zero;                 // LDS word offset of the words of zeros
+  int ww, h;                // words per row and rows of the input
+};
+
+// The K rows of a window, and of the windows of the R - 1 output rows below it (R = 1 or 2, S input rows apart): v[r][q] is
+// the OR of word j0 + q of the rows first + r * S ... first + r * S + K - 1.  Rows that both windows hold are read once.
+// Rows outside the plane come from the words of zeros.  A word left or right of the row is a word of a neighbouring row
+// (or of the header): the caller drops those.
+template <int K, int N, int S, int R, bool TWO>
+__device__ __forceinline__ void plan_rows(const PlanIn& in, int first, int j0, uint32_t (&v)[R][N]) {
+  int off = first * in.ww + j0;
+  uint32_t both[N];
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    both[q] = 0u;
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r][q] = 0u;
+  }
+#pragma unroll
+  for (int ky = 0; ky < K + (R - 1) * S; ++ky) {
+    const bool ok = (unsigned)(first + ky) < (unsigned)in.h;
+    const uint32_t* p1 = in.lds + (ok ? in.in1 + off : in.zero);
+    const uint32_t* p2 = in.lds + (ok ? in.in2 + off : in.zero);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      const uint32_t x = TWO ? p1[q] | p2[q] : p1[q];
+      if (R == 2 && ky < S) v[0][q] |= x;
+      else if (R == 2 && ky >= K) v[R - 1][q] |= x;
+      else both[q] |= x;
+    }
+    off += in.ww;
+  }
+#pragma unroll
+  for (int q = 0; q < N; ++q)
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r][q] |= both[q];
+}
+
+// Output words j of rows y .. y + R - 1 of a specialised footprint (pixels 32*j .. 32*j+31; R = 2: y is even).
+template <int KEY, bool TWO, int R>
+__device__ __forceinline__ void plan_foot_words(const PlanIn& in, int y, int j, uint32_t (&r)[R]) {
+  constexpr int K = plan_key_size(KEY);
+  constexpr int P = K / 2;
+  if constexpr (KEY == PLAN_KEY_C11) {
+    uint32_t v[R][1];
+    plan_rows<1, 1, 1, R, TWO>(in, y, j, v);
+#pragma unroll
+    for (int i = 0; i < R; ++i) r[i] = v[i][0];
+  } else if constexpr (KEY >= PLAN_KEY_C31 && KEY <= PLAN_KEY_C111) {
+    uint32_t v[R][3];
+    plan_rows<K, 3, 1, R, TWO>(in, y - P, j - 1, v);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const uint32_t vp = j > 0 ? v[i][0] : 0u, vn = j + 1 < in.ww ? v[i][2] : 0u;
+      r[i] = 0u;
+#pragma unroll
+      for (int t = 0; t < K; ++t) r[i] |= plan_shift(vp, v[i][1], vn, t - P);
+    }
+  } else if constexpr (KEY >= PLAN_KEY_C32 && KEY <= PLAN_KEY_C92) {
+    // the window OR at input positions 64*j .. 64*j+63, of which the even ones are the outputs
+    uint32_t v[R][4];
+    plan_rows<K, 4, 2, R, TWO>(in, 2 * y - P, 2 * j - 1, v);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const uint32_t v0 = j > 0 ? v[i][0] : 0u, v2 = 2 * j + 1 < in.ww ? v[i][2] : 0u, v3 = 2 * j + 2 < in.ww ? v[i][3] : 0u;
+      uint32_t d0 = 0u, d1 = 0u;
+#pragma unroll
+      for (int t = 0; t < K; ++t) {
+        d0 |= plan_shift(v0, v[i][1], v2, t - P);
+        d1 |= plan_shift(v[i][1], v2, v3, t - P);
+      }
+      r[i] = plan_even_bits(d0) | (plan_even_bits(d1) << 16);
+    }
+  } else {
+    const int js = j >> 1, sh = 16 * (j & 1), e = y & 1, m = y >> 1;
+    const bool okp = js > 0, okn = js + 1 < in.ww;
+    uint32_t v[R][3];
+    if constexpr (KEY == PLAN_KEY_UP) {
+      // out[2m] = in[m-1] | in[m], out[2m+1] = in[m] | in[m+1], rows and columns alike (clamping at the border adds
+      // nothing: the clamped neighbour is the pixel itself)
+      plan_rows<2, 3, 1, R, TWO>(in, m - 1 + e, js - 1, v);
+    } else {
+      // transposed conv, stride 2: output 2m + e sees input m + (e + P - kk) / 2 for the taps kk with e + P - kk even:
+      // K = 3: {m} for e = 0, {m, m+1} for e = 1;  K = 5: {m-1, m, m+1}, {m, m+1}
+      uint32_t w[1][3];
+      if constexpr (K == 3) {
+        plan_rows<1, 3, 1, 1, TWO>(in, m, js - 1, v);
+        plan_rows<1, 3, 1, 1, TWO>(in, e ? m + 1 : -1, js - 1, w);
+      } else {
+        plan_rows<2, 3, 1, 1, TWO>(in, m, js - 1, v);
+        plan_rows<1, 3, 1, 1, TWO>(in, e ? -1 : m - 1, js - 1, w);
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) v[0][q] |= w[0][q];
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const uint32_t vp = okp ? v[i][0] : 0u, vn = okn ? v[i][2] : 0u;
+      uint32_t ev = 0u, od = 0u;
+      if constexpr (KEY == PLAN_KEY_UP) {
+        ev = v[i][1] | plan_shift(vp, v[i][1], vn, -1);
+        od = v[i][1] | plan_shift(vp, v[i][1], vn, 1);
+      } else {
+#pragma unroll
+        for (int kx = 0; kx < K; ++kx) {
+          const int d2 = P - kx;
+          if (d2 & 1) od |= plan_shift(vp, v[i][1], vn, (d2 + 1) >> 1);
+          else ev |= plan_shift(vp, v[i][1], vn, d2 >> 1);
+        }
+      }
+      r[i] = plan_spread(ev >> sh) | (plan_spread(od >> sh) << 1);
+    }
   }
 }
-template <int FOOT, int K, int S>
-__device__ __forceinline__ void plan_foot_any(const PlanStep& s, const uint32_t* bm, uint32_t* out, int r, int nthr) {
-  if (s.in2 >= 0) plan_foot_all<FOOT, K, S, true>(s, bm, out, r, nthr);
-  else plan_foot_all<FOOT, K, S, false>(s, bm, out, r, nthr);
+
+// The general form: any kernel size and padding, conv of stride 1 or 2, transposed conv of stride 2.  Output word j of
+// row oy; words and rows outside the input count as zero.
+__device__ uint32_t plan_foot_general(const PlanIn& in, int geom, int oy, int j) {
+  const int foot = geom & 255, k = (geom >> 8) & 255, s = (geom >> 16) & 255, p = (geom >> 24) & 255;
+  auto word = [&](int y, int jj) -> uint32_t {
+    const bool ok = (unsigned)y < (unsigned)in.h && (unsigned)jj < (unsigned)in.ww;
+    const int o = y * in.ww + jj;
+    return in.lds[ok ? in.in1 + o : in.zero] | in.lds[ok ? in.in2 + o : in.zero];
+  };
+  if (foot == MIE_FOOT_CONV && s == 1) {
+    uint32_t vp = 0u, vc = 0u, vn = 0u, r = 0u;
+    for (int ky = 0; ky < k; ++ky) {
+      vp |= word(oy - p + ky, j - 1);
+      vc |= word(oy - p + ky, j);
+      vn |= word(oy - p + ky, j + 1);
+    }
+    for (int t = 0; t < k; ++t) r |= plan_shift(vp, vc, vn, t - p);
+    return r;
+  }
+  if (foot == MIE_FOOT_CONV) {
+    uint32_t v[4] = {0u, 0u, 0u, 0u}, d0 = 0u, d1 = 0u;
+    for (int ky = 0; ky < k; ++ky)
+      for (int q = 0; q < 4; ++q) v[q] |= word(2 * oy - p + ky, 2 * j - 1 + q);
+    for (int t = 0; t < k; ++t) {
+      d0 |= plan_shift(v[0], v[1], v[2], t - p);
+      d1 |= plan_shift(v[1], v[2], v[3], t - p);
+    }
+    return plan_even_bits(d0) | (plan_even_bits(d1) << 16);
+  }
+  const int js = j >> 1, sh = 16 * (j & 1), e = oy & 1, m = oy >> 1;
+  uint32_t vp = 0u, vc = 0u, vn = 0u, ev = 0u, od = 0u;
+  for (int ky = 0; ky < k; ++ky) {
+    const int d2 = e + p - ky;
+    if (d2 & 1) continue;
+    vp |= word(m + (d2 >> 1), js - 1);
+    vc |= word(m + (d2 >> 1), js);
+    vn |= word(m + (d2 >> 1), js + 1);
+  }
+  for (int kx = 0; kx < k; ++kx) {
+    const int d2 = p - kx;
+    if (d2 & 1) od |= plan_shift(vp, vc, vn, (d2 + 1) >> 1);
+    else ev |= plan_shift(vp, vc, vn, d2 >> 1);
+  }
+  return plan_spread(ev >> sh) | (plan_spread(od >> sh) << 1);
 }
 
-__device__ void plan_compute(const PlanStep& s, const uint32_t* bm, uint32_t* out, int r, int nthr) {
-  const int ho = s.h_out, wo = s.w_out, wwo = (wo + 31) >> 5;
-  if (s.in1 == PLAN_IN_ALL) {
-    for (int wd = r; wd < ho * wwo; wd += nthr) {
-      const int j = wd - plan_div(wd, s.m_words) * wwo;
-      const int left = wo - 32 * j;
-      out[wd] = left >= 32 ? 0xffffffffu : ((1u << left) - 1u);
+// R = 2: a thread makes the words of two rows, where there are more words than threads (fewer reads a word, a longer step).
+template <int KEY, bool TWO, int R>
+__device__ __forceinline__ void plan_foot_all(const PlanIn& in, uint32_t* out, int ho, int wo, uint32_t m_words, int geom, int r,
+                                              int nthr) {
+  const int wwo = (wo + 31) >> 5, total = (R == 2 ? (ho + 1) >> 1 : ho) * wwo;
+  for (int wd = r; wd < total; wd += nthr) {
+    const int y = R * plan_div(wd, m_words), j = wd - (R == 2 ? y >> 1 : y) * wwo;
+    uint32_t v[R];
+    if constexpr (KEY == PLAN_KEY_ALL) v[0] = 0xffffffffu;
+    else if constexpr (KEY == PLAN_KEY_GENERIC) v[0] = plan_foot_general(in, geom, y, j);
+    else plan_foot_words<KEY, TWO, R>(in, y, j, v);
+    const uint32_t valid = plan_valid(wo, j);
+    out[y * wwo + j] = v[0] & valid;
+    if (R == 2 && y + 1 < ho) out[(y + 1) * wwo + j] = v[R - 1] & valid;
+  }
+}
+
+// The bitmap of a footprint step: thread r of nthr takes words r, r + nthr, ...
+__device__ void plan_compute(uint32_t pw, uint32_t* lds, int zero, int r, int nthr) {
+  const uint32_t io = plan_word(pw, PS_IN), ow = plan_word(pw, PS_OUT_WIN), wk = plan_word(pw, PS_WOUT_KEY);
+  const int ho = (int)plan_word(pw, PS_HOUT), wo = (int)(wk & 0xffffu), key = (int)((wk >> 16) & 0xffu);
+  const uint32_t mw = plan_word(pw, PS_MWORDS);
+  const int geom = (int)plan_word(pw, PS_GEOM);
+  uint32_t* out = lds + (ow & 0xffffu);
+  PlanIn in;
+  in.lds = lds;
+  in.zero = zero;
+  in.in1 = (int)(io & 0xffffu);
+  const bool two = (io >> 16) != PLAN_IN_NONE;
+  in.in2 = two ? (int)(io >> 16) : in.in1;
+  in.ww = ((int)(ow >> 16) + 31) >> 5;
+  in.h = (int)plan_word(pw, PS_HIN);
+  const bool many = ho * ((wo + 31) >> 5) > nthr;
+  switch (key) {       // uniform over the wave
+#define PLAN_CASE(KEY)                                                                          \
+    case KEY:                                                                                   \
+      if (two) plan_foot_all<KEY, true, 1>(in, out, ho, wo, mw, geom, r, nthr);                 \
+      else plan_foot_all<KEY, false, 1>(in, out, ho, wo, mw, geom, r, nthr);                    \
+      break
+#define PLAN_CASE_R(KEY)                                                                        \
+    case KEY:                                                                                   \
+      if (two) plan_foot_all<KEY, true, 1>(in, out, ho, wo, mw, geom, r, nthr);                 \
+      else if (many) plan_foot_all<KEY, false, 2>(in, out, ho, wo, mw, geom, r, nthr);          \
+      else plan_foot_all<KEY, false, 1>(in, out, ho, wo, mw, geom, r, nthr);                    \
+      break
+    PLAN_CASE(PLAN_KEY_C11);
+    PLAN_CASE_R(PLAN_KEY_C31);
+    PLAN_CASE_R(PLAN_KEY_C51);
+    PLAN_CASE(PLAN_KEY_C71);
+    PLAN_CASE(PLAN_KEY_C91);
+    PLAN_CASE(PLAN_KEY_C111);
+    PLAN_CASE_R(PLAN_KEY_C32);
+    PLAN_CASE_R(PLAN_KEY_C52);
+    PLAN_CASE_R(PLAN_KEY_C72);
+    PLAN_CASE_R(PLAN_KEY_C92);
+    case PLAN_KEY_UP:
+      if (two && many) plan_foot_all<PLAN_KEY_UP, true, 2>(in, out, ho, wo, mw, geom, r, nthr);
+      else if (many) plan_foot_all<PLAN_KEY_UP, false, 2>(in, out, ho, wo, mw, geom, r, nthr);
+      else if (two) plan_foot_all<PLAN_KEY_UP, true, 1>(in, out, ho, wo, mw, geom, r, nthr);
+      else plan_foot_all<PLAN_KEY_UP, false, 1>(in, out, ho, wo, mw, geom, r, nthr);
+      break;
+    PLAN_CASE(PLAN_KEY_T32);
+    PLAN_CASE(PLAN_KEY_T52);
+#undef PLAN_CASE_R
+#undef PLAN_CASE
+    case PLAN_KEY_ALL: plan_foot_all<PLAN_KEY_ALL, false, 1>(in, out, ho, wo, mw, geom, r, nthr); break;
+    default: plan_foot_all<PLAN_KEY_GENERIC, true, 1>(in, out, ho, wo, mw, geom, r, nthr);
+  }
+}
+
+// A mask in memory -> bitmap: two words a thread asked for together where rows allow 16-byte loads.
+__device__ __forceinline__ void plan_load(uint32_t pw, uint32_t* lds, int n, int r, int nthr) {
+  const uint32_t ow = plan_word(pw, PS_OUT_WIN), wk = plan_word(pw, PS_WOUT_KEY);
+  const int ho = (int)plan_word(pw, PS_HOUT), wo = (int)(wk & 0xffffu), wwo = (wo + 31) >> 5, total = ho * wwo;
+  const uint32_t mw = plan_word(pw, PS_MWORDS);
+  const uint8_t* src = plan_ptr<const uint8_t>(pw, PS_PIX) + (long long)n * ho * wo;
+  uint32_t* out = lds + (ow & 0xffffu);
+  const int unit = (int)(wk >> 28);
+  if (unit == 2) {
+    constexpr int U = 2;
+    for (int w0 = r; w0 < total; w0 += U * nthr) {
+      uint4 v[U][2];
+      bool half[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int wd = w0 + u * nthr < total ? w0 + u * nthr : w0;
+        const int y = plan_div(wd, mw), j = wd - y * wwo;
+        const uint4* p = reinterpret_cast<const uint4*>(src + (long long)y * wo + 32 * j);
+        half[u] = wo - 32 * j <= 16;
+        v[u][0] = p[0];
+        v[u][1] = p[half[u] ? 0 : 1];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        uint32_t b[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          b[q] = plan_octet(v[u][q].x, v[u][q].y) | (plan_octet(v[u][q].z, v[u][q].w) << 8);
+        if (w0 + u * nthr < total) out[w0 + u * nthr] = b[0] | (half[u] ? 0u : b[1] << 16);
+      }
     }
     return;
   }
-  switch (s.key) {       // uniform over the workgroup
-    case PLAN_KEY_C11: plan_foot_any<MIE_FOOT_CONV, 1, 1>(s, bm, out, r, nthr); break;
-    case PLAN_KEY_C31: plan_foot_any<MIE_FOOT_CONV, 3, 1>(s, bm, out, r, nthr); break;
-    case PLAN_KEY_C51: plan_foot_any<MIE_FOOT_CONV, 5, 1>(s, bm, out, r, nthr); break;
-    case PLAN_KEY_C32: plan_foot_any<MIE_FOOT_CONV, 3, 2>(s, bm, out, r, nthr); break;
-    case PLAN_KEY_C52: plan_foot_any<MIE_FOOT_CONV, 5, 2>(s, bm, out, r, nthr); break;
-    case PLAN_KEY_UP: plan_foot_any<MIE_FOOT_UP2X, 1, 1>(s, bm, out, r, nthr); break;
-    case PLAN_KEY_T32: plan_foot_any<MIE_FOOT_TCONV, 3, 2>(s, bm, out, r, nthr); break;
-    case PLAN_KEY_T52: plan_foot_any<MIE_FOOT_TCONV, 5, 2>(s, bm, out, r, nthr); break;
-    default: {
-      const int foot = s.geom & 255, ss = (s.geom >> 16) & 255;
-      if (foot == MIE_FOOT_TCONV) plan_foot_all<MIE_FOOT_TCONV, 0, 2, true>(s, bm, out, r, nthr);
-      else if (ss == 1) plan_foot_all<MIE_FOOT_CONV, 0, 1, true>(s, bm, out, r, nthr);
-      else plan_foot_all<MIE_FOOT_CONV, 0, 2, true>(s, bm, out, r, nthr);
-    }
-  }
-}
-
-// What a step leaves in memory, from its bitmap `out`.  The pixel mask, as bytes: this workgroup's slice (share of
-// shares), by threads r of nthr.
-__device__ void plan_write_pixels(const PlanStep& s, const uint32_t* out, int n, int share, int shares, int r, int nthr) {
-  const int ho = s.h_out, wo = s.w_out, wwo = (wo + 31) >> 5;
-  const int first = share * nthr + r, stride = shares * nthr;
-  uint8_t* pm = s.pixmask + (long long)n * ho * wo;
-  if ((wo & 15) == 0) {
-    const int per_row = wo >> 4, units = ho * per_row;
-    for (int u = first; u < units; u += stride) {
-      const int y = plan_div(u, s.m_units), q = u - y * per_row;
-      const uint32_t b16 = out[y * wwo + (q >> 1)] >> (16 * (q & 1));
-      const uint4 v = make_uint4(plan_bytes(b16 & 15u), plan_bytes((b16 >> 4) & 15u), plan_bytes((b16 >> 8) & 15u),
-                                 plan_bytes((b16 >> 12) & 15u));
-      *reinterpret_cast<uint4*>(pm + (long long)y * wo + 16 * q) = v;
-    }
-  } else if ((wo & 3) == 0) {
-    const int per_row = wo >> 2, units = ho * per_row;
-    for (int u = first; u < units; u += stride) {
-      const int y = plan_div(u, s.m_units), q = u - y * per_row;
-      const uint32_t nib = (out[y * wwo + (q >> 3)] >> (4 * (q & 7))) & 15u;
-      *reinterpret_cast<uint32_t*>(pm + (long long)y * wo + 4 * q) = plan_bytes(nib);
-    }
-  } else {
-    for (int u = first; u < ho * wo; u += stride) {
-      const int y = plan_div(u, s.m_units), x = u - y * wo;
-      pm[u] = (uint8_t)((out[y * wwo + (x >> 5)] >> (x & 31)) & 1u);
-    }
-  }
-}
-
-// The tile flags: tile (ty, tx) is byte tx % 4 of word tx / 4 in rows 8*ty .. 8*ty+7.  A flag word is written by the one
-// thread that owns its tile -- word f of this step's flag area is tile f * shares + share -- from the old value fetched
-// at the start.
-__device__ void plan_write_flags(const PlanStep& s, const uint32_t* out, const uint32_t* s_old, int n, int share, int shares,
-                                 int r, int nthr) {
-  const int ho = s.h_out, wo = s.w_out, wwo = (wo + 31) >> 5;
-  const int tiles_y = (ho + MIE_TILE - 1) / MIE_TILE, tiles_x = (wo + MIE_TILE - 1) / MIE_TILE;
-  const int tpp = tiles_y * tiles_x;
-  for (int f = r; f < s.flag_cnt; f += nthr) {
-    const int t = f * shares + share;
-    if (t >= tpp) break;
-    const int ty = plan_div(t, s.m_tiles), tx = t - ty * tiles_x;
-    uint32_t any = 0u;
+  for (int wd = r; wd < total; wd += nthr) {
+    const int y = plan_div(wd, mw), j = wd - y * wwo;
+    const int x0 = 32 * j, nb = (wo - x0 < 32) ? wo - x0 : 32;
+    const uint8_t* row = src + (long long)y * wo + x0;
+    uint32_t bits = 0u;
+    if (unit == 1) {
+      const uint32_t* r4 = reinterpret_cast<const uint32_t*>(row);
+      const int nq = nb >> 2;
+      uint32_t v[8];
 #pragma unroll
-    for (int q = 0; q < MIE_TILE; ++q) {
-      const int y = ty * MIE_TILE + q;
-      any |= out[(y < ho ? y : ho - 1) * wwo + (tx >> 2)] & (y < ho ? 0xffffffffu : 0u);
+      for (int q = 0; q < 8; ++q) v[q] = r4[q < nq ? q : 0];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) bits |= q < nq ? plan_nibble(v[q]) << (4 * q) : 0u;
+    } else {
+      for (int b0 = 0; b0 < nb; b0 += 8) {
+        uint8_t v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = row[b0 + q < nb ? b0 + q : 0];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) bits |= (b0 + q < nb && v[q] != 0) ? 1u << (b0 + q) : 0u;
+      }
     }
-    s.flags[n * tpp + t] = next_flag(s_old[s.flag_off + f], ((any >> (8 * (tx & 3))) & 0xffu) != 0u);
+    out[wd] = bits;
   }
 }
 
-__global__ __launch_bounds__(PLAN_THREADS) void k_plan_bits(PlanArgs a) {
+// 16 pixels of a row of a mask: bits -> bytes, as wide as the rows allow.
+__device__ __forceinline__ void plan_put16(uint8_t* p, uint32_t b16, int left, int unit) {
+  const uint4 v = make_uint4(plan_bytes(b16 & 15u), plan_bytes((b16 >> 4) & 15u), plan_bytes((b16 >> 8) & 15u), plan_bytes((b16 >> 12) & 15u));
+  if (unit == 2) {
+    *reinterpret_cast<uint4*>(p) = v;
+  } else if (unit == 1) {
+    uint32_t* p4 = reinterpret_cast<uint32_t*>(p);
+    p4[0] = v.x;
+    if (left > 4) p4[1] = v.y;
+    if (left > 8) p4[2] = v.z;
+    if (left > 12) p4[3] = v.w;
+  } else {
+    for (int q = 0; q < 16 && q < left; ++q) p[q] = (uint8_t)((b16 >> q) & 1u);
+  }
+}
+
+__device__ __forceinline__ int plan_tiles(uint32_t pw) {
+  const int ho = (int)plan_word(pw, PS_HOUT), wo = (int)(plan_word(pw, PS_WOUT_KEY) & 0xffffu);
+  return ((ho + MIE_TILE - 1) / MIE_TILE) * ((wo + MIE_TILE - 1) / MIE_TILE);
+}
+// The tiles of a set whose flags a workgroup writes where it does not own sets: [lo, hi).
+__device__ __forceinline__ void plan_slice(uint32_t pw, int share, int& lo, int& hi) {
+  const int tiles = plan_tiles(pw), own = (int)plan_word(pw, PS_OWN);
+  lo = share * own;
+  hi = lo + own < tiles ? lo + own : tiles;
+}
+// Whether tile t of a set holds an active pixel.
+__device__ __forceinline__ bool plan_tile_any(const uint32_t* bitmap, int t, int ho, int wo, uint32_t mt) {
+  const int wwo = (wo + 31) >> 5, tiles_x = (wo + MIE_TILE - 1) / MIE_TILE, ty = plan_div(t, mt), tx = t - ty * tiles_x;
+  uint32_t any = 0u;
+#pragma unroll
+  for (int q = 0; q < MIE_TILE; ++q) {
+    const int y = ty * MIE_TILE + q;
+    any |= bitmap[(y < ho ? y : ho - 1) * wwo + (tx >> 2)];       // the last row again where a tile ends below the plane
+  }
+  return ((any >> (8 * (tx & 3))) & 0xffu) != 0u;
+}
+
+// Not resident: what a step leaves in memory, from its bitmap, by threads r of nthr.  The pixel mask, this workgroup's
+// slice (share of shares), and, in LDS, the state of the tiles it writes the flags of: byte t - lo of the step's part of
+// the flag area.
+__device__ void plan_write(uint32_t pw, const uint32_t* lds, uint8_t* fl, int n, int share, int shares, int r, int nthr) {
+  const int ho = (int)plan_word(pw, PS_HOUT), wo = (int)(plan_word(pw, PS_WOUT_KEY) & 0xffffu), wwo = (wo + 31) >> 5;
+  const uint32_t* out = lds + (plan_word(pw, PS_OUT_WIN) & 0xffffu);
+  const uint32_t mu = plan_word(pw, PS_MUNITS), mt = plan_word(pw, PS_MTILES);
+  const int unit = (int)(plan_word(pw, PS_WOUT_KEY) >> 28), per_row = (wo + 15) >> 4, units = ho * per_row;
+  uint8_t* pm = plan_ptr<uint8_t>(pw, PS_PIX) + (long long)n * ho * wo;
+  for (int u = share * nthr + r; u < units; u += shares * nthr) {
+    const int y = plan_div(u, mu), q = u - y * per_row;
+    plan_put16(pm + (long long)y * wo + 16 * q, out[y * wwo + (q >> 1)] >> (16 * (q & 1)), wo - 16 * q, unit);
+  }
+  int lo, hi;
+  plan_slice(pw, share, lo, hi);
+  uint8_t* bits = fl + plan_word(pw, PS_FL);
+  for (int t = lo + r; t < hi; t += nthr) bits[t - lo] = plan_tile_any(out, t, ho, wo, mt) ? 1 : 0;
+}
+
+// Resident: a thread's 16-pixel unit u of all sets' units -- its set is the last step whose units start at or below it --
+// as the place of its bits in LDS and of its bytes in memory.
+// (bits: LDS word | upper half << 16 | pixels of it that the row has << 17 | width of the stores << 22)
+struct PlanPut { uint8_t* dst; uint32_t bits; };
+__device__ __forceinline__ PlanPut plan_find(const uint32_t* lds, int n_steps, int n, int u) {
+  int i = 0;
+#pragma unroll
+  for (int b = 32; b > 0; b >>= 1) {
+    const int at = i + b < n_steps ? i + b : i;
+    i = (int)lds[at * PS_WORDS + PS_UBASE] <= u ? at : i;
+  }
+  const uint32_t* p = lds + i * PS_WORDS;
+  const int ho = (int)p[PS_HOUT], wo = (int)(p[PS_WOUT_KEY] & 0xffffu), wwo = (wo + 31) >> 5, per_row = (wo + 15) >> 4;
+  const int q0 = u - (int)p[PS_UBASE], y = plan_div(q0, p[PS_MUNITS]), q = q0 - y * per_row;
+  PlanPut r;
+  r.dst = reinterpret_cast<uint8_t*>(((unsigned long long)p[PS_PIX_HI] << 32) | p[PS_PIX]) + ((long long)n * ho + y) * wo + 16 * q;
+  const int left = wo - 16 * q < 16 ? wo - 16 * q : 16;
+  r.bits = ((p[PS_OUT_WIN] & 0xffffu) + (uint32_t)(y * wwo + (q >> 1))) | (uint32_t)(q & 1) << 16 | (uint32_t)left << 17 | (p[PS_WOUT_KEY] >> 28) << 22;
+  return r;
+}
+__device__ __forceinline__ void plan_put(const uint32_t* lds, const PlanPut& p) {
+  plan_put16(p.dst, lds[p.bits & 0xffffu] >> ((p.bits >> 12) & 16u), (int)((p.bits >> 17) & 31u), (int)(p.bits >> 22));
+}
+
+// The lists, counts and flags of a set the workgroup owns, from its bitmap and its tiles' old state: by all threads.
+// `par` alternates from set to set (and chunk to chunk) so that one barrier a chunk is enough.
+__device__ __forceinline__ void plan_rank(uint32_t pw, const uint32_t* lds, const uint8_t* old, int* s_tot, int& par, int tid) {
+  const int ho = (int)plan_word(pw, PS_HOUT), wo = (int)(plan_word(pw, PS_WOUT_KEY) & 0xffffu), tiles = plan_tiles(pw);
+  const uint32_t mt = plan_word(pw, PS_MTILES);
+  const uint8_t* o_tiles = old + plan_word(pw, PS_FL);
+  const uint32_t* bitmap = lds + (plan_word(pw, PS_OUT_WIN) & 0xffffu);
+  uint32_t* flags = plan_ptr<uint32_t>(pw, PS_FLAGS);
+  int32_t* act = plan_ptr<int32_t>(pw, PS_TILES);
+  int32_t* stale = plan_ptr<int32_t>(pw, PS_STALE);
+  int32_t* counts = plan_ptr<int32_t>(pw, PS_COUNTS);
+  const int wave = tid >> 6;
+  int run_a = 0, run_s = 0;
+  for (int t0 = 0; t0 < tiles; t0 += PLAN_THREADS) {
+    const int t = t0 + tid;
+    bool a = false, s = false;
+    if (t < tiles) {
+      a = plan_tile_any(bitmap, t, ho, wo, mt);
+      const uint32_t o = o_tiles[t];
+      s = !a && (o & 1u) != 0u;
+      flags[t] = next_flag(o, a);
+    }
+    const unsigned long long ba = __ballot(a), bs = __ballot(s);
+    int* tot = s_tot + par * PLAN_WAVES;
+    par ^= 1;
+    if ((tid & 63) == 0) tot[wave] = __popcll(ba) | (__popcll(bs) << 16);        // at most 64 each
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < PLAN_WAVES; ++w) {
+      const int v = tot[w];
+      before += w < wave ? v : 0;
+      all += v;                                              // at most 1024 in either half
+    }
+    const int ra = run_a + (before & 0xffff), rs = run_s + (before >> 16);
+    if (a) act[__builtin_amdgcn_mbcnt_hi((uint32_t)(ba >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ba, (uint32_t)ra))] = t;
+    if (s) stale[__builtin_amdgcn_mbcnt_hi((uint32_t)(bs >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bs, (uint32_t)rs))] = t;
+    run_a += all & 0xffff;
+    run_s += all >> 16;
+  }
+  if (tid == 0) {
+    counts[MIE_CNT_ACTIVE] = run_a;
+    counts[MIE_CNT_STALE] = run_s;
+  }
+}
+
+// (64 registers: beside a plan made ahead there is room for a conv's workgroup on the same CU)
+__global__ __launch_bounds__(PLAN_THREADS, 8) void k_plan_bits(PlanArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint32_t plan_lds[];
-  // The steps first go from the argument block to LDS in one batch: read where they are used, every step's fields
-  // would be a cache miss of their own in a chain where nothing else hides it.
-  PlanStep* steps = reinterpret_cast<PlanStep*>(plan_lds);
-  uint32_t* bm = plan_lds + PLAN_HEAD;
-  const int n = blockIdx.y, tid = threadIdx.x;
+  uint32_t* lds = plan_lds;
+  const int n = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int share = blockIdx.x, shares = gridDim.x;
+  const int step_words = a.n_steps * PS_WORDS, lw = lane < PS_WORDS ? lane : 0;
+  uint8_t* task = reinterpret_cast<uint8_t*>(lds + step_words);
+  uint8_t* fl = reinterpret_cast<uint8_t*>(lds + a.flag_off);
+  int* s_tot = reinterpret_cast<int*>(lds + a.zero_off + PLAN_ZERO_WORDS);        // 2 * PLAN_WAVES
   {
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(&a.st[0]);
-    const int nw = a.n_steps * (int)(sizeof(PlanStep) / 4);
-    for (int i = tid; i < nw; i += PLAN_THREADS) plan_lds[i] = src[i];
+    // The steps and the task table go from the argument block to LDS in one batch: read where they are used, every
+    // step's words would be a cache miss of their own in a chain where nothing else hides it.
+    const uint32_t* tsrc = reinterpret_cast<const uint32_t*>(a.task);
+    const int tw = (a.n_levels + 2) * (PLAN_WAVES / 4);
+    for (int i = tid; i < step_words + tw; i += PLAN_THREADS) lds[i] = i < step_words ? a.st[i] : tsrc[i - step_words];
+    if (tid < PLAN_ZERO_WORDS) lds[a.zero_off + tid] = 0u;
+  }
+  const int first = a.owned ? a.head[share] : PLAN_IDLE;
+  __syncthreads();
+  // The old state of the tiles of the first set this workgroup owns is asked for, then the masks that level 0 loads; while
+  // those are on their way a thread finds the place of its first unit of the pixel masks.
+  uint32_t f0 = 0u, fl0 = 0u;
+  int tiles0 = 0;
+  if (first != PLAN_IDLE) {
+    const uint32_t q = lds[first * PS_WORDS + lw];
+    tiles0 = plan_tiles(q);
+    fl0 = plan_word(q, PS_FL);
+    f0 = plan_ptr<const uint32_t>(q, PS_FLAGS)[tid < tiles0 ? tid : 0];
+  }
+  const int load = __builtin_amdgcn_readfirstlane((int)task[wave]);       // level 0: masks from memory, by all waves
+  if (load < a.n_loads) {
+    const uint32_t q = lds[load * PS_WORDS + lw], wv = plan_word(q, PS_WAVES);
+    plan_load(q, lds, n, (wave - (int)(wv & 255u)) * 64 + lane, (int)((wv >> 8) & 255u) * 64);
+  }
+  PlanPut put = {nullptr, 0u};
+  const int u0 = share * PLAN_THREADS + tid;
+  if (a.resident) put = plan_find(lds, a.n_steps, n, u0 < a.units ? u0 : 0);
+  if (first != PLAN_IDLE) {
+    if (tid < tiles0) fl[fl0 + tid] = (uint8_t)(f0 & 1u);
+    // what is left: tiles beyond the first 1024, further sets
+    for (int i = first; i != PLAN_IDLE;) {
+      const uint32_t p = lds[i * PS_WORDS + lw];
+      const int tiles = plan_tiles(p);
+      const uint32_t* flags = plan_ptr<const uint32_t>(p, PS_FLAGS);
+      uint8_t* o = fl + plan_word(p, PS_FL);
+      for (int t = tid + (i == first ? PLAN_THREADS : 0); t < tiles; t += PLAN_THREADS) o[t] = (uint8_t)(flags[t] & 1u);
+      i = (int)plan_word(p, PS_OWN);
+    }
   }
   __syncthreads();
-  // sample blockIdx.y; share blockIdx.x of gridDim.x of everything that is written to memory
-  const int share = blockIdx.x, shares = gridDim.x;
-  // The tile flags this workgroup owns -- tiles share, share + shares, ... of every set -- hold the previous build's
-  // state and are needed when a step is written out.  Asked for step by step, each would be a memory round trip that
-  // nothing hides; so all of them are fetched now, in one batch behind which the first mask's loads queue up, into the
-  // LDS area in front of the bitmaps (word flag_off + f of a step = tile f * shares + share).
-  uint32_t* s_old = bm;
-  bm += a.flag_words;
-  for (int u = tid; u < a.flag_words; u += PLAN_THREADS) {
-    int q = 0;
-    for (int i = 1; i < a.n_steps; ++i)
-      if (steps[i].flag_off <= u) q = i;            // the last step whose area starts at or below u (areas are in step order)
-    const PlanStep& sq = steps[q];
-    const int tpp = ((sq.h_out + MIE_TILE - 1) / MIE_TILE) * ((sq.w_out + MIE_TILE - 1) / MIE_TILE);
-    const int t = (u - sq.flag_off) * shares + share;
-    s_old[u] = (sq.kind == PLAN_STEP_FOOT && t < tpp) ? sq.flags[n * tpp + t] : 0u;
-  }
-  // role of this wave: 0 = bitmaps, 1 = pixel masks, 2 = tile flags (uniform over a wave: the limits are multiples of 64)
-  const int role = tid < PLAN_COMPUTE ? 0 : (tid < PLAN_COMPUTE + PLAN_PIX ? 1 : 2);
-  int pending = -1;                                    // the footprint step that is not written out yet
-  for (int i = 0; i < a.n_steps; ++i) {
-#ifdef MIE_PLAN_PROFILE
-    const long long t_step = wall_clock64();
-#endif
-    const PlanStep s = plan_uni(steps[i]);
-    uint32_t* out = bm + s.out;
-    const int ho = s.h_out, wo = s.w_out, wwo = (wo + 31) >> 5;
-    if (s.kind == PLAN_STEP_LOAD) {
-      const uint8_t* src = s.ext + (long long)n * ho * wo;
-      for (int wd = tid; wd < ho * wwo; wd += PLAN_THREADS) {
-        const int y = plan_div(wd, s.m_words), j = wd - y * wwo;
-        const int x0 = 32 * j, nb = (wo - x0 < 32) ? wo - x0 : 32;
-        const uint8_t* row = src + (long long)y * wo + x0;
-        uint32_t bits = 0u;
-        if ((wo & 15) == 0) {           // rows start on 16-byte boundaries and hold whole groups of 16 pixels
-          const uint4* r16 = reinterpret_cast<const uint4*>(row);
-          const uint4 v0 = r16[0];
-          bits = plan_nibble(v0.x) | (plan_nibble(v0.y) << 4) | (plan_nibble(v0.z) << 8) | (plan_nibble(v0.w) << 12);
-          if (nb > 16) {
-            const uint4 v1 = r16[1];
-            bits |= (plan_nibble(v1.x) | (plan_nibble(v1.y) << 4) | (plan_nibble(v1.z) << 8) | (plan_nibble(v1.w) << 12)) << 16;
-          }
-        } else if ((wo & 3) == 0) {     // 4-byte boundaries
-          const uint32_t* r4 = reinterpret_cast<const uint32_t*>(row);
-          for (int q = 0; q < (nb >> 2); ++q) bits |= plan_nibble(r4[q]) << (4 * q);
-        } else {
-          for (int b = 0; b < nb; ++b) bits |= (row[b] != 0 ? 1u : 0u) << b;
-        }
-        out[wd] = bits;
+  const int compute_waves = a.resident ? PLAN_WAVES : PLAN_COMPUTE_WAVES;
+  int idx = __builtin_amdgcn_readfirstlane((int)task[PLAN_WAVES + wave]);
+  int next = task[2 * PLAN_WAVES + wave];
+  uint32_t pw = lds[(idx == PLAN_IDLE ? 0 : idx) * PS_WORDS + lw];
+  for (int lv = 1; lv < a.n_levels; ++lv) {
+    // the step of the next level and the number of the one after it
+    const int nidx = __builtin_amdgcn_readfirstlane(next);
+    const uint32_t npw = lds[(nidx == PLAN_IDLE ? 0 : nidx) * PS_WORDS + lw];
+    next = task[(lv + 2 <= a.n_levels ? lv + 2 : 0) * PLAN_WAVES + wave];
+    if (idx != PLAN_IDLE) {
+      const uint32_t wv = plan_word(pw, PS_WAVES);
+      if (wave < compute_waves) {
+        int r = (wave - (int)(wv & 255u)) * 64 + lane;
+        const int nthr = (int)((wv >> 8) & 255u) * 64;
+        asm volatile("" : "+v"(r));        // or a dozen multiples of it are kept in registers through the whole chain
+        if (plan_kind(pw) == PLAN_KIND_LOAD) plan_load(pw, lds, n, r, nthr);
+        else plan_compute(pw, lds, a.zero_off, r, nthr);
+      } else {
+        // (the writing waves read the slots of the level before while this level's are written: the host keeps them
+        // apart -- a slot is handed on one level after its last reader)
+        plan_write(pw, lds, fl, n, share, shares, (wave - (int)((wv >> 16) & 255u)) * 64 + lane, (int)(wv >> 24) * 64);
       }
-      __syncthreads();
-      continue;
     }
-    // The compute waves make this step's bitmap while the others put the step before it into memory.  (They read that
-    // step's slot while this step's is written, and the step after this one writes its own one barrier later: the host
-    // keeps all three apart -- a slot is handed on one step after its last reader.)
-    if (role == 0) {
-      plan_compute(s, bm, out, tid, PLAN_COMPUTE);
-    } else if (pending >= 0) {
-      const PlanStep sp = plan_uni(steps[pending]);
-      if (role == 1) plan_write_pixels(sp, bm + sp.out, n, share, shares, tid - PLAN_COMPUTE, PLAN_PIX);
-      else plan_write_flags(sp, bm + sp.out, s_old, n, share, shares, tid - PLAN_COMPUTE - PLAN_PIX, PLAN_FLG);
-    }
-#ifdef MIE_PLAN_PROFILE
-    // measurement builds only: ticks of the 100 MHz clock of this step in workgroup (0, 0), first thread of each role
-    if (blockIdx.x == 0 && n == 0 && (tid == 0 || tid == PLAN_COMPUTE || tid == PLAN_COMPUTE + PLAN_PIX))
-      reinterpret_cast<int32_t*>(a.dbg)[3 * i + role] = (int)(wall_clock64() - t_step);
-#endif
     __syncthreads();
-    pending = i;
+    idx = nidx;
+    pw = npw;
   }
-  if (pending >= 0) {       // the last step, by everybody
-    const PlanStep sp = plan_uni(steps[pending]);
-    plan_write_pixels(sp, bm + sp.out, n, share, shares, tid, PLAN_THREADS);
-    plan_write_flags(sp, bm + sp.out, s_old, n, share, shares, tid, PLAN_THREADS);
+  if (a.resident) {
+    // the pixel masks of all sets: this workgroup's slice of their units
+    for (int u = u0; u < a.units; u += shares * PLAN_THREADS) {
+      if (u != u0) put = plan_find(lds, a.n_steps, n, u);
+      plan_put(lds, put);
+    }
+  } else {
+    for (int i = a.first_last; i < a.n_steps; ++i)       // the last level, by everybody
+      plan_write(lds[i * PS_WORDS + lw], lds, fl, n, share, shares, tid, PLAN_THREADS);
+    __syncthreads();
+  }
+  if (a.owned) {
+    int par = 0;
+    for (int i = first; i != PLAN_IDLE;) {
+      const uint32_t q = lds[i * PS_WORDS + lw];
+      plan_rank(q, lds, fl, s_tot, par, tid);
+      i = (int)plan_word(q, PS_OWN);
+    }
+    return;
+  }
+  // one wave a set: the flags of this workgroup's slice, old state asked for here
+  for (int i = wave; i < a.n_steps; i += PLAN_WAVES) {
+    const uint32_t q = lds[i * PS_WORDS + lw];
+    if (plan_kind(q) != PLAN_KIND_FOOT) continue;
+    int lo, hi;
+    plan_slice(q, share, lo, hi);
+    const int ho = (int)plan_word(q, PS_HOUT), wo = (int)(plan_word(q, PS_WOUT_KEY) & 0xffffu);
+    const uint32_t mt = plan_word(q, PS_MTILES);
+    const uint8_t* now = fl + plan_word(q, PS_FL);
+    const uint32_t* bitmap = lds + (plan_word(q, PS_OUT_WIN) & 0xffffu);
+    uint32_t* flags = plan_ptr<uint32_t>(q, PS_FLAGS) + (long long)n * plan_tiles(q);
+    for (int t = lo + lane; t < hi; t += 64) {
+      const uint32_t o = flags[t];
+      flags[t] = next_flag(o, a.resident ? plan_tile_any(bitmap, t, ho, wo, mt) : now[t - lo] != 0);
+    }
   }
 }
 
@@ -1177,61 +1437,9 @@ __global__ __launch_bounds__(COMPACT_THREADS) void k_plan_compact(PlanCompactArg
   compact_chunk(ba, b - a.first_chunk[i], a.first_chunk[i + 1] - a.first_chunk[i], s_tot, s_base);
 }
 
-// Host side: LDS words of a plane's bitmap.
-inline long long plan_words(int h, int w) { return (long long)h * ((w + 31) / 32); }
-
-// First-fit allocator over the bitmap area (word offsets), free blocks kept sorted and coalesced.
-struct PlanArena {
-  struct Blk { long long off, size; };
-  Blk free_[2 * MIE_PLAN_MAX_STEPS + 2];
-  int nfree = 0;
-  long long top = 0;          // high-water mark
-  long long alloc(long long size) {
-    for (int i = 0; i < nfree; ++i)
-      if (free_[i].size >= size) {
-        const long long off = free_[i].off;
-        free_[i].off += size;
-        free_[i].size -= size;
-        if (free_[i].size == 0) {
-          for (int j = i; j + 1 < nfree; ++j) free_[j] = free_[j + 1];
-          --nfree;
-        }
-        return off;
-      }
-    // grow: extend a free block that ends at the top, else start a new one there
-    if (nfree > 0 && free_[nfree - 1].off + free_[nfree - 1].size == top) {
-      const long long off = free_[nfree - 1].off;
-      top = off + size;
-      --nfree;
-      return off;
-    }
-    const long long off = top;
-    top += size;
-    return off;
-  }
-  void release(long long off, long long size) {
-    int i = 0;
-    while (i < nfree && free_[i].off < off) ++i;
-    for (int j = nfree; j > i; --j) free_[j] = free_[j - 1];
-    free_[i] = {off, size};
-    ++nfree;
-    if (i + 1 < nfree && free_[i].off + free_[i].size == free_[i + 1].off) {
-      free_[i].size += free_[i + 1].size;
-      for (int j = i + 1; j + 1 < nfree; ++j) free_[j] = free_[j + 1];
-      --nfree;
-    }
-    if (i > 0 && free_[i - 1].off + free_[i - 1].size == free_[i].off) {
-      free_[i - 1].size += free_[i].size;
-      for (int j = i; j + 1 < nfree; ++j) free_[j] = free_[j + 1];
-      --nfree;
-    }
-  }
-};
-
-// LDS a workgroup may use on the current device, and the opt-in for more than 64 KB of it (once per process).
-int plan_lds_limit(long long need_bytes, const char* who) {
+// LDS a workgroup may use on the current device.
+int plan_lds_limit(int* bytes, const char* who) {
   static int limit[64];
-  static long long opted[64];
   int dev = -1;
   hipError_t e = hipGetDevice(&dev);
   MIE_REQUIRE(e == hipSuccess && dev >= 0 && dev < 64, MIE_ERR_LAUNCH, "%s: no current device (%s)", who, hipGetErrorString(e));
@@ -1241,16 +1449,207 @@ int plan_lds_limit(long long need_bytes, const char* who) {
     MIE_REQUIRE(e == hipSuccess && v > 0, MIE_ERR_LAUNCH, "%s: cannot read the LDS size of device %d (%s)", who, dev, hipGetErrorString(e));
     limit[dev] = v;
   }
-  MIE_REQUIRE(need_bytes <= limit[dev], MIE_ERR_CAPACITY,
+  *bytes = limit[dev];
+  return MIE_OK;
+}
+
+// Whether a plan's LDS is there, and the opt-in for more than 64 KB of it (once per process).
+int plan_lds_take(long long need_bytes, int limit, const char* who) {
+  static long long opted[64];
+  int dev = -1;
+  hipError_t e = hipGetDevice(&dev);
+  MIE_REQUIRE(e == hipSuccess && dev >= 0 && dev < 64, MIE_ERR_LAUNCH, "%s: no current device (%s)", who, hipGetErrorString(e));
+  MIE_REQUIRE(need_bytes <= limit, MIE_ERR_CAPACITY,
               "%s: the masks of this plan need %lld bytes of LDS at once, the device offers %d per workgroup; "
-              "build the plan in parts, or with mie_build_mask_tiles", who, need_bytes, limit[dev]);
+              "build the plan in parts, or with mie_build_mask_tiles", who, need_bytes, limit);
   if (need_bytes > 65536 && need_bytes > opted[dev]) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_plan_bits), hipFuncAttributeMaxDynamicSharedMemorySize, limit[dev]);
-    MIE_REQUIRE(e == hipSuccess, MIE_ERR_CAPACITY, "%s: the device refuses %d bytes of dynamic LDS (%s)", who, limit[dev],
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_plan_bits), hipFuncAttributeMaxDynamicSharedMemorySize, limit);
+    MIE_REQUIRE(e == hipSuccess, MIE_ERR_CAPACITY, "%s: the device refuses %d bytes of dynamic LDS (%s)", who, limit,
                 hipGetErrorString(e));
-    opted[dev] = limit[dev];
+    opted[dev] = limit;
   }
   return MIE_OK;
+}
+
+// Host side of a plan: its steps (masks loaded from memory and ops), the level each runs in and the LDS its bitmap takes.
+struct PlanHost {
+  static constexpr int MAX = MIE_PLAN_MAX_STEPS;
+  struct Step {
+    int op;                     // the op, or -1: a mask loaded from memory
+    int in[2];                  // steps whose bitmaps it reads, -1: none
+    int k;                      // its window over them (conv windows of stride 1 and 2 that may have been widened)
+    int src[2];                 // as in[], as the op says it
+    const uint8_t* ptr;         // its mask in memory
+    int h, w;
+    long long words;
+    int level, last;            // when its bitmap is made, and the last level that reads it (writing waves included)
+    int rec;                    // the allocation its bitmap lies in
+  };
+  struct Alloc { long long words, off; int born, rel; };
+  Step st[MAX];
+  int n_steps = 0, n_levels = 0;
+  Alloc rec[MAX];
+  int n_rec = 0;
+  long long top = 0;            // words of LDS of all bitmaps
+
+  // A conv window with "same" padding over the result of a stride-1 window with "same" padding is one wider window over
+  // that one's input: read that, where the wide window has a form of its own.
+  void widen(const mie_plan_op* ops) {
+    auto same = [&](const Step& s, int stride) {
+      if (s.op < 0 || s.src[0] < 0) return false;
+      const mie_plan_op& op = ops[s.op];
+      return op.foot == MIE_FOOT_CONV && op.stride == stride && (op.k & 1) && op.pad == op.k / 2;
+    };
+    for (int i = 0; i < n_steps; ++i) {
+      Step& s = st[i];
+      const bool one = same(s, 1);
+      if (!(one || same(s, 2)) || s.src[1] >= 0) continue;
+      const Step& m = st[s.src[0]];
+      const int k = s.k + m.k - 1;
+      if (!same(m, 1) || k > (one ? PLAN_MAX_K1 : PLAN_MAX_K2)) continue;
+      s.in[0] = m.in[0];
+      s.in[1] = m.in[1];
+      s.k = k;
+    }
+  }
+  void as_given(const mie_plan_op* ops) {
+    for (int i = 0; i < n_steps; ++i) {
+      st[i].in[0] = st[i].src[0];
+      st[i].in[1] = st[i].src[1];
+      st[i].k = st[i].op >= 0 ? ops[st[i].op].k : 0;
+    }
+  }
+
+  // What a word of a step costs, roughly: the words it reads (R = 1) and some twenty instructions more.
+  long long cost(int i, const mie_plan_op* ops) const {
+    if (st[i].op < 0) return 20;
+    const mie_plan_op& op = ops[st[i].op];
+    const int rows = op.foot == MIE_FOOT_CONV ? st[i].k : 2, words = op.foot == MIE_FOOT_CONV && op.stride == 2 ? 4 : 3;
+    return rows * words * (st[i].in[1] >= 0 ? 2 : 1) + 20;
+  }
+
+  // Level 0 holds masks from memory only; they are there before the chain starts.  serial: one step after the other, a mask from memory right before the op that reads it first (the form
+  // that needs least LDS).  Otherwise a step runs as soon as what it reads is there, at most so many a level.
+  // resident: every bitmap is held to the end.
+  void schedule(bool serial, bool resident, const mie_plan_op* ops) {
+    int count[MAX + 2] = {0};
+    n_levels = 1;
+    for (int i = 0; i < n_steps; ++i) {
+      int lv = st[i].op >= 0 ? 1 : 0;
+      for (int q = 0; q < 2; ++q)
+        if (st[i].in[q] >= 0 && st[st[i].in[q]].level + 1 > lv) lv = st[st[i].in[q]].level + 1;
+      // a set or a mask that is written twice: in the order of the ops, and after it was loaded
+      for (int j = 0; j < i && st[i].op >= 0; ++j)
+        if (st[j].ptr == st[i].ptr || (st[j].op >= 0 && ops[st[j].op].out.flags == ops[st[i].op].out.flags))
+          if (st[j].level + 1 > lv) lv = st[j].level + 1;
+      if (serial) lv = i + (i > 0 || st[i].op >= 0 ? 1 : 0);
+      else
+        while (count[lv] >= (resident ? PLAN_LEVEL_STEPS : PLAN_WRITE_WAVES)) ++lv;
+      ++count[lv];
+      st[i].level = lv;
+      if (lv + 1 > n_levels) n_levels = lv + 1;
+    }
+    for (int i = 0; i < n_steps; ++i) st[i].last = st[i].op < 0 ? st[i].level : resident ? n_levels : st[i].level + 1;
+    for (int i = 0; i < n_steps; ++i)
+      for (int q = 0; q < 2; ++q)
+        if (st[i].in[q] >= 0 && st[i].level > st[st[i].in[q]].last) st[st[i].in[q]].last = st[i].level;
+  }
+
+  // LDS: an allocation per bitmap, held from its level to its last reader's (both included).  A union (the 1x1
+  // footprint of two masks) is a word-by-word OR and may overwrite an input that nothing else reads in its level or
+  // later -- the writing waves of the level before are through with it if it is at least two levels old.
+  void place(const mie_plan_op* ops) {
+    n_rec = 0;
+    int order[MAX];              // steps by level
+    int no = 0;
+    for (int lv = 0; lv < n_levels; ++lv)
+      for (int i = 0; i < n_steps; ++i)
+        if (st[i].level == lv) order[no++] = i;
+    for (int oi = 0; oi < no; ++oi) {
+      Step& s = st[order[oi]];
+      s.rec = -1;
+      if (s.op >= 0 && s.in[0] >= 0 && s.in[1] >= 0) {
+        const mie_plan_op& op = ops[s.op];
+        if (op.foot == MIE_FOOT_CONV && s.k == 1 && op.stride == 1 && op.pad == 0) {
+          for (int q = 1; q >= 0 && s.rec < 0; --q) {
+            const Step& m = st[s.in[q]];
+            bool alone = m.words == s.words && m.last == s.level && m.level <= s.level - 2 && s.in[0] != s.in[1];
+            for (int j = 0; j < n_steps && alone; ++j)
+              if (&st[j] != &s && st[j].level == s.level && (st[j].in[0] == s.in[q] || st[j].in[1] == s.in[q])) alone = false;
+            if (!alone || rec[m.rec].rel != s.level) continue;      // (rel: the memory was handed to another union already)
+            s.rec = m.rec;
+            rec[s.rec].rel = s.last;
+          }
+        }
+      }
+      if (s.rec < 0) {
+        s.rec = n_rec;
+        rec[n_rec++] = {s.words, 0, s.level, s.last};
+      }
+    }
+    // two ways of packing, the tighter one counts: in order of birth, and largest first; each allocation at the lowest
+    // offset where it meets none whose lifetime overlaps
+    long long best[MAX];
+    top = -1;
+    for (int way = 0; way < 2; ++way) {
+      int by[MAX];
+      for (int i = 0; i < n_rec; ++i) by[i] = i;
+      for (int i = 1; way == 1 && i < n_rec; ++i)
+        for (int j = i; j > 0 && rec[by[j]].words > rec[by[j - 1]].words; --j) {
+          const int t = by[j]; by[j] = by[j - 1]; by[j - 1] = t;
+        }
+      long long t = 0;
+      for (int oi = 0; oi < n_rec; ++oi) {
+        Alloc& r = rec[by[oi]];
+        long long off = 0;
+        for (bool moved = true; moved;) {
+          moved = false;
+          for (int oj = 0; oj < oi; ++oj) {
+            const Alloc& q = rec[by[oj]];
+            if (r.born <= q.rel && q.born <= r.rel && off < q.off + q.words && q.off < off + r.words) {
+              off = q.off + q.words;
+              moved = true;
+            }
+          }
+        }
+        r.off = off;
+        if (off + r.words > t) t = off + r.words;
+      }
+      if (top < 0 || t < top) {
+        top = t;
+        for (int i = 0; i < n_rec; ++i) best[i] = rec[i].off;
+      }
+    }
+    for (int i = 0; i < n_rec; ++i) rec[i].off = best[i];
+  }
+};
+
+// `total` waves for the steps of a level by their weights: at least one each, none more than it has work for.
+void plan_deal(int total, int n, const long long* weight, const int* most, int* first, int* count) {
+  long long sum = 0;
+  for (int i = 0; i < n; ++i) sum += weight[i];
+  int used = 0;
+  for (int i = 0; i < n; ++i) {
+    int c = (int)(weight[i] * total / (sum > 0 ? sum : 1));
+    c = c < 1 ? 1 : c;
+    c = c > most[i] ? most[i] : c;
+    count[i] = c;
+    used += c;
+  }
+  while (used > total) {          // the minimum of one each went beyond: from the largest
+    int b = 0;
+    for (int i = 1; i < n; ++i) b = count[i] > count[b] ? i : b;
+    --count[b];
+    --used;
+  }
+  for (bool more = true; more && used < total;) {
+    more = false;
+    int b = -1;
+    for (int i = 0; i < n; ++i)
+      if (count[i] < most[i] && (b < 0 || weight[i] * count[b] > weight[b] * count[i])) b = i;
+    if (b >= 0) { ++count[b]; ++used; more = true; }
+  }
+  for (int i = 0, at = 0; i < n; ++i) { first[i] = at; at += count[i]; }
 }
 
 }  // namespace
@@ -1275,55 +1674,20 @@ int build_mask_plan(const char* who, const mie_plan_op* ops, int n_ops, int wg_c
   mie_clear_error();
   MIE_REQUIRE(ops != nullptr && n_ops > 0, MIE_ERR_INVALID_ARG, "%s: no ops", who);
   MIE_REQUIRE(n_ops <= MIE_PLAN_MAX_STEPS, MIE_ERR_CAPACITY, "%s: %d ops, at most %d per call", who, n_ops, MIE_PLAN_MAX_STEPS);
-  PlanArgs a;
-  memset(&a, 0, sizeof(a));
-  a.n = ops[0].out.n;
-  // masks in LDS: pointer -> (slot offset, words, step index of the last reader)
-  struct Slot { const uint8_t* ptr; long long off, words; int h, w, last, born, rec; };
-  // Every allocation of the walk below, with the ops during which it is held (born .. rel, both included): the walk
-  // runs twice -- first with a first-fit allocator, which fragments (the short-lived input mask of a UNet leaves a hole
-  // that small masks then chop up, and the two full-resolution masks at the end of the chain no longer fit into it);
-  // then, if that is tighter, with offsets packed off line from the recorded lifetimes, largest masks first.
-  struct AllocRec { long long words, off; int born, rel; };
-  AllocRec recs[2 * MIE_PLAN_MAX_STEPS];
-  int nrec = 0;
-  bool replay = false;
-  Slot slots[2 * MIE_PLAN_MAX_STEPS];
-  int nslots = 0;
-  // which op reads a mask last (by pointer), so that its slot can be handed on afterwards
-  auto last_reader = [&](const uint8_t* p, int from) {
-    int last = from;
-    for (int j = from; j < n_ops; ++j)
-      if (ops[j].in_mask == p || ops[j].in_mask2 == p) last = j;
-    return last;
-  };
-  auto find_slot = [&](const uint8_t* p) -> Slot* {
-    for (int i = nslots - 1; i >= 0; --i)      // the latest mask at this address
-      if (slots[i].ptr == p) return &slots[i];
-    return nullptr;
-  };
-  PlanArena arena;
-  long long total_chunks = 0, max_pixels = 0, max_tiles = 0;
-  int alloc_no = 0;
-  auto slot_alloc = [&](long long words, int born) -> int {      // returns the record index; recs[..].off is the offset
-    const int id = alloc_no++;
-    if (!replay) {
-      recs[id].words = words; recs[id].born = born; recs[id].rel = n_ops;
-      recs[id].off = arena.alloc(words);
-      nrec = alloc_no;
-    }
-    return id;
-  };
-  auto walk = [&]() -> int {
+  const int n = ops[0].out.n;
+  PlanHost ph;
+  long long total_chunks = 0, max_pixels = 0;
+  bool owned = n == 1;            // one launch: no set with more tiles than a workgroup ranks, none twice
+  bool reread = false;            // an op overwrites a mask that the plan also loads from memory
   for (int i = 0; i < n_ops; ++i) {
     const mie_plan_op& op = ops[i];
     int rc = mie_check_tileset(&op.out, who);
     if (rc != MIE_OK) return rc;
-    MIE_REQUIRE(op.out.n == a.n, MIE_ERR_INVALID_ARG, "%s: op %d has batch size %d, op 0 has %d", who, i, op.out.n, a.n);
+    MIE_REQUIRE(op.out.n == n, MIE_ERR_INVALID_ARG, "%s: op %d has batch size %d, op 0 has %d", who, i, op.out.n, n);
     MIE_REQUIRE(op.h_in > 0 && op.w_in > 0, MIE_ERR_INVALID_ARG, "%s: op %d: input size (%d,%d) must be positive", who, i,
                 op.h_in, op.w_in);
     MIE_REQUIRE(op.in_mask != nullptr || op.in_mask2 == nullptr, MIE_ERR_INVALID_ARG, "%s: op %d: in_mask2 given without in_mask", who, i);
-    MIE_REQUIRE((long long)a.n * op.h_in * op.w_in < 0x7fffffffLL, MIE_ERR_CAPACITY, "%s: op %d: more than 2^31 input pixels", who, i);
+    MIE_REQUIRE((long long)n * op.h_in * op.w_in < 0x7fffffffLL, MIE_ERR_CAPACITY, "%s: op %d: more than 2^31 input pixels", who, i);
     MIE_REQUIRE(op.w_in <= 2048 && op.out.w <= 2048 && (long long)op.h_in * op.w_in <= (1 << 20) &&
                     (long long)op.out.h * op.out.w <= (1 << 20),
                 MIE_ERR_CAPACITY, "%s: op %d: planes of up to 2048 pixels per row and 2^20 pixels per sample (use mie_build_mask_tiles)", who, i);
@@ -1351,184 +1715,188 @@ int build_mask_plan(const char* who, const mie_plan_op* ops, int n_ops, int wg_c
     const bool identity = op.foot == MIE_FOOT_CONV && k == 1 && st == 1 && pad == 0;
     MIE_REQUIRE(identity || ((const uint8_t*)op.out.pixmask != op.in_mask && (const uint8_t*)op.out.pixmask != op.in_mask2),
                 MIE_ERR_INVALID_ARG, "%s: op %d: out.pixmask aliases an input mask (allowed for the 1x1 stride-1 footprint only)", who, i);
-    // inputs: a mask an earlier op of this plan wrote is still in LDS; any other is loaded from memory first
-    int in_off[2] = {PLAN_IN_NONE, PLAN_IN_NONE};
+    // inputs: the mask an earlier op of this plan left at this address last; any other is loaded from memory, once
+    int in[2] = {-1, -1};
     const uint8_t* ins[2] = {op.in_mask, op.in_mask2};
-    if (op.in_mask == nullptr) in_off[0] = PLAN_IN_ALL;
-    for (int q = 0; q < 2 && op.in_mask != nullptr; ++q) {
+    for (int q = 0; q < 2; ++q) {
       if (ins[q] == nullptr) continue;
-      Slot* sl = find_slot(ins[q]);
-      if (sl == nullptr || sl->last < i) {
-        // not in LDS (never was, or its slot has been handed on): load it
-        MIE_REQUIRE(a.n_steps < MIE_PLAN_MAX_STEPS && nslots < 2 * MIE_PLAN_MAX_STEPS, MIE_ERR_CAPACITY,
+      for (int j = ph.n_steps - 1; j >= 0 && in[q] < 0; --j)
+        if (ph.st[j].ptr == ins[q]) in[q] = j;
+      if (in[q] < 0) {
+        MIE_REQUIRE(ph.n_steps < MIE_PLAN_MAX_STEPS, MIE_ERR_CAPACITY,
                     "%s: more than %d steps (ops plus masks loaded from memory); build the plan in parts", who, MIE_PLAN_MAX_STEPS);
-        Slot ns;
-        ns.ptr = ins[q]; ns.h = op.h_in; ns.w = op.w_in; ns.words = plan_words(op.h_in, op.w_in);
-        ns.born = i;
-        ns.last = last_reader(ins[q], i);
-        // (a later op of the plan may overwrite this address: then the mask in LDS is the old one from there on)
-        for (int j = i; j < ns.last; ++j)
-          if (ops[j].out.pixmask == ins[q]) { ns.last = j; break; }
-        ns.rec = slot_alloc(ns.words, i);
-        ns.off = recs[ns.rec].off;
-        PlanStep& ld = a.st[a.n_steps++];
-        ld.kind = PLAN_STEP_LOAD;
-        ld.in1 = ld.in2 = PLAN_IN_NONE;
-        ld.out = (int)ns.off;
-        ld.h_in = ld.h_out = op.h_in; ld.w_in = ld.w_out = op.w_in;
-        ld.m_words = plan_magic((op.w_in + 31) / 32);
-        ld.ext = ins[q];
-        slots[nslots++] = ns;
-        sl = &slots[nslots - 1];
+        PlanHost::Step& ld = ph.st[ph.n_steps];
+        ld = {-1, {-1, -1}, 0, {-1, -1}, ins[q], op.h_in, op.w_in, (long long)op.h_in * ((op.w_in + 31) / 32), 0, 0, -1};
+        in[q] = ph.n_steps++;
+        for (int j = i; j < n_ops; ++j) reread |= (const uint8_t*)ops[j].out.pixmask == ins[q];
       }
-      MIE_REQUIRE(sl->h == op.h_in && sl->w == op.w_in, MIE_ERR_INVALID_ARG,
-                  "%s: op %d reads a mask of (%d,%d) as (%d,%d)", who, i, sl->h, sl->w, op.h_in, op.w_in);
-      in_off[q] = (int)sl->off;
+      const PlanHost::Step& m = ph.st[in[q]];
+      MIE_REQUIRE(m.h == op.h_in && m.w == op.w_in, MIE_ERR_INVALID_ARG,
+                  "%s: op %d reads a mask of (%d,%d) as (%d,%d)", who, i, m.h, m.w, op.h_in, op.w_in);
     }
-    if (in_off[0] == PLAN_IN_ALL) in_off[1] = PLAN_IN_NONE;
-    MIE_REQUIRE(a.n_steps < MIE_PLAN_MAX_STEPS && nslots < 2 * MIE_PLAN_MAX_STEPS, MIE_ERR_CAPACITY,
+    MIE_REQUIRE(ph.n_steps < MIE_PLAN_MAX_STEPS, MIE_ERR_CAPACITY,
                 "%s: more than %d steps (ops plus masks loaded from memory); build the plan in parts", who, MIE_PLAN_MAX_STEPS);
-    // the output's slot: every input of this op is still alive, so it cannot land on one of them
-    Slot os;
-    os.ptr = op.out.pixmask; os.h = op.out.h; os.w = op.out.w; os.words = plan_words(op.out.h, op.out.w);
-    os.last = last_reader(op.out.pixmask, i);
-    for (int j = i + 1; j < os.last; ++j)
-      if (ops[j].out.pixmask == op.out.pixmask) { os.last = j; break; }      // rewritten before its last reader
-    os.born = i;
-    // A union (the 1x1 footprint of two masks) is a word-by-word OR: it may overwrite an input that nobody reads after
-    // this op -- provided that input is at least two ops old, so that the writer waves of the op before this one, which
-    // still read THEIR op's output while this op computes, are not looking at it.  Saves a slot of the plane's size
-    // (the full-resolution union at the end of a UNet is what decides whether the chain fits the LDS in one plan).
-    os.off = -1;
-    if (identity && op.in_mask != nullptr && op.in_mask2 != nullptr) {
-      for (int q = 1; q >= 0 && os.off < 0; --q) {
-        Slot* sl = find_slot(ins[q]);
-        if (sl != nullptr && sl->off == in_off[q] && sl->words == os.words && sl->last == i && sl->born <= i - 2 &&
-            ins[q] != (const uint8_t*)op.out.pixmask) {
-          os.off = sl->off;
-          os.rec = sl->rec;       // the memory is the output's now: one allocation, held on
-          sl->words = 0;
-          sl->last = -1;
-        }
-      }
-    }
-    if (os.off < 0) {
-      os.rec = slot_alloc(os.words, i);
-      os.off = recs[os.rec].off;
-    }
-    PlanStep& ft = a.st[a.n_steps++];
-    ft.kind = PLAN_STEP_FOOT;
-    ft.in1 = in_off[0]; ft.in2 = in_off[1];
-    ft.out = (int)os.off;
-    ft.h_in = op.h_in; ft.w_in = op.w_in; ft.h_out = op.out.h; ft.w_out = op.out.w;
-    ft.geom = op.foot | (k << 8) | (st << 16) | (pad << 24);
-    ft.pixmask = op.out.pixmask;
-    ft.flags = op.out.flags;
-    ft.m_words = plan_magic((op.out.w + 31) / 32);
-    ft.m_units = plan_magic(op.out.w % 16 == 0 ? op.out.w / 16 : (op.out.w % 4 == 0 ? op.out.w / 4 : op.out.w));
-    ft.m_tiles = plan_magic(mie_div_up(op.out.w, MIE_TILE));
-    // the specialised forms have kernel size, stride and the padding k / 2 built in
-    ft.key = PLAN_KEY_GENERIC;
-    if (op.foot == MIE_FOOT_UP2X) ft.key = PLAN_KEY_UP;
-    else if (pad == k / 2) {
-      if (op.foot == MIE_FOOT_CONV && st == 1) ft.key = k == 1 ? PLAN_KEY_C11 : k == 3 ? PLAN_KEY_C31 : k == 5 ? PLAN_KEY_C51 : PLAN_KEY_GENERIC;
-      if (op.foot == MIE_FOOT_CONV && st == 2) ft.key = k == 3 ? PLAN_KEY_C32 : k == 5 ? PLAN_KEY_C52 : PLAN_KEY_GENERIC;
-      if (op.foot == MIE_FOOT_TCONV) ft.key = k == 3 ? PLAN_KEY_T32 : k == 5 ? PLAN_KEY_T52 : PLAN_KEY_GENERIC;
-    }
-    slots[nslots++] = os;
-    // Slots whose last reader was the PREVIOUS op are free from here on: one op late, because the kernel has no
-    // barrier between the end of a step (threads still reading its output slot while they write the pixel mask and
-    // the flags) and the compute phase of the next step, which writes that step's output slot.  With the release
-    // delayed, the slot a step writes was last read at least one whole step -- and its barrier -- earlier.
-    for (int q = 0; q < nslots; ++q)
-      if (slots[q].last >= 0 && slots[q].last < i && slots[q].words > 0) {
-        if (!replay) {
-          arena.release(slots[q].off, slots[q].words);
-          recs[slots[q].rec].rel = i;
-        }
-        slots[q].words = 0;
-        slots[q].last = -1;
-      }
-    const int cap = mie_tile_capacity(op.out.n, op.out.h, op.out.w);
+    PlanHost::Step& ft = ph.st[ph.n_steps++];
+    ft = {i, {in[0], in[1]}, k, {in[0], in[1]}, op.out.pixmask, op.out.h, op.out.w, (long long)op.out.h * ((op.out.w + 31) / 32), 0, 0, -1};
+    const int cap = mie_tile_capacity(n, op.out.h, op.out.w);
     total_chunks += mie_div_up(cap, COMPACT_CHUNK);
     if ((long long)op.out.h * op.out.w > max_pixels) max_pixels = (long long)op.out.h * op.out.w;
-    if (cap / op.out.n > max_tiles) max_tiles = cap / op.out.n;
+    owned = owned && cap <= PLAN_OWNED_TILES;
+    for (int j = 0; j < i; ++j) owned = owned && ops[j].out.flags != op.out.flags;
   }
-  return MIE_OK;
-  };
-  int rc = walk();
-  if (rc != MIE_OK) return rc;
-  {
-    // off-line packing: largest first, each at the lowest offset where it meets no allocation whose lifetime overlaps
-    int order[2 * MIE_PLAN_MAX_STEPS];
-    long long packed[2 * MIE_PLAN_MAX_STEPS];
-    for (int i = 0; i < nrec; ++i) order[i] = i;
-    for (int i = 1; i < nrec; ++i)
-      for (int j = i; j > 0 && (recs[order[j]].words > recs[order[j - 1]].words ||
-                                (recs[order[j]].words == recs[order[j - 1]].words && recs[order[j]].born < recs[order[j - 1]].born)); --j) {
-        const int t = order[j]; order[j] = order[j - 1]; order[j - 1] = t;
-      }
-    long long top = 0;
-    for (int oi = 0; oi < nrec; ++oi) {
-      const AllocRec& r = recs[order[oi]];
-      long long off = 0;
-      for (bool moved = true; moved;) {
-        moved = false;
-        for (int oj = 0; oj < oi; ++oj) {
-          const AllocRec& q = recs[order[oj]];
-          const long long qo = packed[order[oj]];
-          if (r.born <= q.rel && q.born <= r.rel && off < qo + q.words && qo < off + r.words) {
-            off = qo + q.words;
-            moved = true;
-          }
-        }
-      }
-      packed[order[oi]] = off;
-      if (off + r.words > top) top = off + r.words;
-    }
-    if (top < arena.top) {
-      for (int i = 0; i < nrec; ++i) recs[i].off = packed[i];
-      arena.top = top;
-      replay = true;
-      memset(&a, 0, sizeof(a));
-      a.n = ops[0].out.n;
-      nslots = 0; alloc_no = 0; total_chunks = 0; max_pixels = 0; max_tiles = 0;
-      rc = walk();
-      if (rc != MIE_OK) return rc;
-    }
-  }
-  // workgroups per sample: a slice of the largest plane's stores each, and never more than one tile flag per thread
+  // workgroups per sample: a slice of the largest plane's stores each, and with one sample a set or two to rank
   long long shares = (max_pixels + PLAN_PIXELS_PER_SHARE - 1) / PLAN_PIXELS_PER_SHARE;
   // Every workgroup walks the whole chain of its sample (and loads every mask that comes from memory): with a batch of
   // samples there are workgroups enough without many per sample, and more than one per CU would only queue (a
   // workgroup of a large plane takes most of a CU's LDS).
   static const int max_wgs = [] { const char* e = getenv("MIE_PLAN_WGS"); return e ? atoi(e) : 256; }();      // tuning knob
   const int wgs = (wg_cap > 0 && wg_cap < max_wgs) ? wg_cap : max_wgs;     // a caller's cap: the plan runs beside other kernels
-  if (shares * a.n > wgs) shares = wgs / a.n > 0 ? wgs / a.n : 1;
-  if (shares * PLAN_THREADS < max_tiles) shares = (max_tiles + PLAN_THREADS - 1) / PLAN_THREADS;
-  // the flag area of a workgroup: per set, the tiles it owns (every shares-th one)
-  for (int i = 0; i < a.n_steps; ++i) {
-    PlanStep& stp = a.st[i];
-    stp.flag_off = a.flag_words;
-    stp.flag_cnt = 0;
-    if (stp.kind != PLAN_STEP_FOOT) continue;
-    const long long tpp = (long long)mie_div_up(stp.h_out, MIE_TILE) * mie_div_up(stp.w_out, MIE_TILE);
-    stp.flag_cnt = (int)((tpp + shares - 1) / shares);
-    a.flag_words += stp.flag_cnt;
-  }
+  if (shares * n > wgs) shares = wgs / n > 0 ? wgs / n : 1;
   MIE_REQUIRE(shares <= PLAN_MAX_SHARES, MIE_ERR_CAPACITY,
-              "%s: a plane of %lld pixels (%lld tiles) per sample is beyond the plan's %d workgroups per sample; use "
-              "mie_build_mask_tiles", who, max_pixels, max_tiles, PLAN_MAX_SHARES);
-  const long long lds_bytes = (PLAN_HEAD + a.flag_words + arena.top) * 4;
-  rc = plan_lds_limit(lds_bytes, who);
+              "%s: a plane of %lld pixels per sample is beyond the plan's %d workgroups per sample; use "
+              "mie_build_mask_tiles", who, max_pixels, PLAN_MAX_SHARES);
+  if (reread) shares = 1;         // a workgroup that lags must not load what another has already overwritten
+  const long long shares_in_slices = shares;
+  // (a plan held to some workgroups runs beside other kernels: no more of them than its stores need)
+  if (owned && !reread && wg_cap == 0 && shares < n_ops) shares = n_ops < wgs ? n_ops : wgs;
+  if (shares > PLAN_MAX_SHARES) shares = PLAN_MAX_SHARES;
+  int limit = 0;
+  int rc = plan_lds_limit(&limit, who);
   if (rc != MIE_OK) return rc;
-#ifdef MIE_PLAN_PROFILE
-  a.dbg = reinterpret_cast<int*>(ops[n_ops - 1].out.stale) + (mie_tile_capacity(a.n, ops[n_ops - 1].out.h, ops[n_ops - 1].out.w) - 3 * MIE_PLAN_MAX_STEPS);
-#endif
-  hipLaunchKernelGGL(k_plan_bits, dim3((unsigned)shares, (unsigned)a.n), dim3(PLAN_THREADS), (size_t)lds_bytes,
+  PlanArgs a;
+  long long lds_words = 0;
+  // The first form that fits: everything resident; bitmaps dropped after their last reader; step by step.
+  for (int form = 0; form < 3; ++form) {
+    const bool resident = form == 0, serial = form == 2;
+    owned = owned && resident;
+    if (!owned) shares = shares_in_slices;
+    ph.as_given(ops);
+    if (!serial) ph.widen(ops);
+    ph.schedule(serial, resident, ops);
+    ph.place(ops);
+    memset(&a, 0, sizeof(a));
+    memset(a.task, PLAN_IDLE, sizeof(a.task));
+    memset(a.head, PLAN_IDLE, sizeof(a.head));
+    a.n_steps = ph.n_steps;
+    a.n_levels = ph.n_levels;
+    a.resident = resident ? 1 : 0;
+    a.owned = owned ? 1 : 0;
+    const int compute_waves = resident ? PLAN_WAVES : PLAN_COMPUTE_WAVES;
+    // flags: who owns which set (largest first, to whoever has least), or how much of each a workgroup writes
+    int own[PlanHost::MAX];
+    long long fl[PlanHost::MAX], flag_bytes = 0;
+    auto set_tiles = [&](int i) { return (long long)mie_div_up(ph.st[i].h, MIE_TILE) * mie_div_up(ph.st[i].w, MIE_TILE); };
+    int owner[PlanHost::MAX];
+    for (int i = 0; i < ph.n_steps; ++i) {
+      if (ph.st[i].op < 0) continue;
+      own[i] = (int)((set_tiles(i) + shares - 1) / shares);
+      fl[i] = flag_bytes;
+      if (!resident) flag_bytes += own[i];
+    }
+    if (owned) {
+      long long load[PLAN_MAX_SHARES] = {0};
+      bool done[PlanHost::MAX] = {false};
+      for (int c = 0; c < n_ops; ++c) {
+        int b = -1, to = 0;
+        for (int i = 0; i < ph.n_steps; ++i)
+          if (ph.st[i].op >= 0 && !done[i] && (b < 0 || set_tiles(i) > set_tiles(b))) b = i;
+        for (int s = 1; s < shares; ++s) to = load[s] < load[to] ? s : to;
+        owner[b] = to;
+        fl[b] = load[to];
+        load[to] += set_tiles(b);
+        done[b] = true;
+        flag_bytes = load[to] > flag_bytes ? load[to] : flag_bytes;
+      }
+    }
+    flag_bytes = (flag_bytes + 15) / 16 * 16;
+    // LDS: steps, task table, zeros and wave totals, tile bits, bitmaps, and the words a load right of the last row reaches
+    a.zero_off = ph.n_steps * PS_WORDS + (ph.n_levels + 2) * (PLAN_WAVES / 4);
+    a.flag_off = a.zero_off + PLAN_ZERO_WORDS + 2 * PLAN_WAVES;
+    const long long base = a.flag_off + flag_bytes / 4;
+    lds_words = base + ph.top + 4;
+    int at = 0;                   // a step's place in the level order
+    for (int lv = 0; lv < ph.n_levels; ++lv) {
+      int id[PLAN_LEVEL_STEPS], ns = 0, most[PLAN_LEVEL_STEPS], cf[PLAN_LEVEL_STEPS], cn[PLAN_LEVEL_STEPS], wf[PLAN_LEVEL_STEPS], wn[PLAN_LEVEL_STEPS];
+      long long weight[PLAN_LEVEL_STEPS];
+      if (lv == ph.n_levels - 1) a.first_last = at;
+      for (int i = 0; i < ph.n_steps; ++i)
+        if (ph.st[i].level == lv) id[ns++] = i;
+      for (int q = 0; q < ns; ++q) {
+        weight[q] = ph.st[id[q]].words * ph.cost(id[q], ops);
+        most[q] = (int)(ph.st[id[q]].words + 63) / 64;
+        if (most[q] > (lv == 0 ? PLAN_WAVES : compute_waves)) most[q] = lv == 0 ? PLAN_WAVES : compute_waves;
+      }
+      // level 0 holds masks from memory only: by all waves, before the chain starts
+      if (lv == 0) a.n_loads = ns;
+      plan_deal(lv == 0 ? PLAN_WAVES : compute_waves, ns, weight, most, cf, cn);
+      for (int q = 0; q < ns; ++q) most[q] = PLAN_WRITE_WAVES, wf[q] = wn[q] = 0;
+      if (!resident) plan_deal(PLAN_WRITE_WAVES, ns, weight, most, wf, wn);
+      for (int q = 0; q < ns; ++q) {
+        const int i = id[q];
+        const PlanHost::Step& s = ph.st[i];
+        if (owned && s.op >= 0) {        // in front of its owner's list
+          own[i] = a.head[owner[i]];
+          a.head[owner[i]] = (uint8_t)at;
+        }
+        wf[q] += PLAN_COMPUTE_WAVES;
+        for (int w = cf[q]; w < cf[q] + cn[q]; ++w) a.task[lv * PLAN_WAVES + w] = (uint8_t)at;
+        if (!resident && s.op >= 0 && lv + 1 < ph.n_levels)
+          for (int w = wf[q]; w < wf[q] + wn[q]; ++w) a.task[(lv + 1) * PLAN_WAVES + w] = (uint8_t)at;
+        uint32_t* p = a.st + at * PS_WORDS;
+        ++at;
+        auto offset = [&](int j) { return (uint32_t)(base + ph.rec[ph.st[j].rec].off); };
+        auto pointer = [&](int word, const void* v) {
+          const unsigned long long b = reinterpret_cast<unsigned long long>(v);
+          p[word] = (uint32_t)b;
+          p[word + 1] = (uint32_t)(b >> 32);
+        };
+        if (lds_words > 0xfff0) continue;       // refused below; the offsets would not fit their fields
+        int key = PLAN_KEY_GENERIC, unit = 0, h_in = s.h, w_in = s.w;
+        if (mie_aligned(s.ptr, 16) && s.w % 16 == 0) unit = 2;        // rows of whole 16-byte (4-byte) groups, on such boundaries
+        else if (mie_aligned(s.ptr, 4) && s.w % 4 == 0) unit = 1;
+        p[PS_IN] = (s.in[0] < 0 ? PLAN_IN_NONE : offset(s.in[0])) | (s.in[1] < 0 ? PLAN_IN_NONE : offset(s.in[1])) << 16;
+        if (s.op >= 0) {
+          const mie_plan_op& op = ops[s.op];
+          h_in = op.h_in;
+          w_in = op.w_in;
+          // the specialised forms have kernel size, stride and the padding k / 2 built in
+          if (op.in_mask == nullptr) key = PLAN_KEY_ALL;
+          else if (op.foot == MIE_FOOT_UP2X) key = PLAN_KEY_UP;
+          else if (op.pad == op.k / 2) {
+            const int k = s.k;
+            if (op.foot == MIE_FOOT_CONV && op.stride == 1 && (k & 1) && k <= PLAN_MAX_K1) key = PLAN_KEY_C11 + k / 2;
+            if (op.foot == MIE_FOOT_CONV && op.stride == 2 && (k & 1) && k >= 3 && k <= PLAN_MAX_K2) key = PLAN_KEY_C32 + k / 2 - 1;
+            if (op.foot == MIE_FOOT_TCONV) key = k == 3 ? PLAN_KEY_T32 : k == 5 ? PLAN_KEY_T52 : PLAN_KEY_GENERIC;
+          }
+          p[PS_GEOM] = (uint32_t)op.foot | (uint32_t)op.k << 8 | (uint32_t)op.stride << 16 | (uint32_t)op.pad << 24;
+          p[PS_FL] = (uint32_t)fl[i];
+          p[PS_OWN] = (uint32_t)own[i];
+          pointer(PS_FLAGS, op.out.flags);
+          pointer(PS_TILES, op.out.tiles);
+          pointer(PS_STALE, op.out.stale);
+          pointer(PS_COUNTS, op.out.counts);
+        }
+        p[PS_OUT_WIN] = offset(i) | (uint32_t)w_in << 16;
+        p[PS_HIN] = (uint32_t)h_in;
+        p[PS_HOUT] = (uint32_t)s.h;
+        p[PS_WOUT_KEY] = (uint32_t)s.w | (uint32_t)key << 16 | (uint32_t)(s.op < 0 ? PLAN_KIND_LOAD : PLAN_KIND_FOOT) << 24 | (uint32_t)unit << 28;
+        p[PS_MWORDS] = plan_magic(mie_div_up(s.w, 32));
+        p[PS_MUNITS] = plan_magic(mie_div_up(s.w, 16));
+        p[PS_MTILES] = plan_magic(mie_div_up(s.w, MIE_TILE));
+        p[PS_UBASE] = (uint32_t)a.units;
+        if (s.op >= 0) a.units += s.h * mie_div_up(s.w, 16);
+        p[PS_WAVES] = (uint32_t)cf[q] | (uint32_t)cn[q] << 8 | (uint32_t)wf[q] << 16 | (uint32_t)wn[q] << 24;
+        pointer(PS_PIX, s.ptr);
+      }
+    }
+    if (lds_words * 4 <= limit) break;
+  }
+  rc = plan_lds_take(lds_words * 4, limit, who);
+  if (rc != MIE_OK) return rc;
+  hipLaunchKernelGGL(k_plan_bits, dim3((unsigned)shares, (unsigned)n), dim3(PLAN_THREADS), (size_t)lds_words * 4,
                      (hipStream_t)stream, a);
   rc = mie_check_launch(who);
-  if (rc != MIE_OK) return rc;
+  if (rc != MIE_OK || owned) return rc;
   PlanCompactArgs c;
   memset(&c, 0, sizeof(c));
   for (int i = 0; i < n_ops; ++i) {

@@ -325,6 +325,62 @@ def test_mask_plan_equals_the_builds_it_replaces(n, h, w):
             prev[name] = _check_tileset(b, m, prev.get(name))
 
 
+@pytest.mark.parametrize("n,h,w", [
+    (1, 264, 352),      # everything in LDS, sets of 1452 tiles: two rounds of the workgroup that ranks them
+    (1, 61, 67), (1, 8, 8), (2, 45, 100),
+    (1, 304, 512),      # bitmaps of 19 KB: not all at once, dropped after their last reader
+    (2, 352, 640),      # bitmaps of 28 KB: only one step after the other
+])
+def test_mask_plan_with_windows_over_windows(n, h, w):
+    # a plan reads a same-size conv window over another's result as one wider window over that one's input, up to 11
+    # pixels (9 at stride 2), unions in between included; chains longer than that, windows without "same" padding, and
+    # steps side by side.  Against one build per set, bit for bit, sparse / empty / dense.
+    c2 = lambda v, k, p: (v + 2 * p - k) // 2 + 1
+    half = lambda k, p: (c2(h, k, p), c2(w, k, p))
+    C = _lib.FOOT_CONV
+    chain = [
+        ("a", ("x",), C, 3, 1, 1, (h, w)), ("t", ("a", "y"), C, 1, 1, 0, (h, w)), ("tt", ("t",), C, 5, 1, 2, (h, w)),
+        ("p", ("a",), C, 5, 1, 1, (h - 2, w - 2)), ("q", ("p",), C, 3, 1, 1, (h - 2, w - 2)),
+        ("b", ("a",), C, 3, 1, 1, (h, w)), ("s3", ("b",), C, 3, 2, 1, half(3, 1)), ("s5", ("b",), C, 5, 2, 2, half(5, 2)),
+        ("s1", ("b",), C, 1, 2, 0, half(1, 0)), ("c", ("b",), C, 3, 1, 1, (h, w)), ("s", ("c",), C, 5, 2, 2, half(5, 2)),
+        ("d", ("c",), C, 3, 1, 1, (h, w)), ("e", ("d",), C, 3, 1, 1, (h, w)), ("f", ("e",), C, 3, 1, 1, (h, w)),
+    ]
+    mk = lambda: {name: TileMask(n, plane[0], plane[1], DEV) for name, _, _, _, _, _, plane in chain}
+    seq, plan = mk(), mk()
+    for step, dens in enumerate((0.01, 0.0, 0.1)):
+        m = lambda seed: np.stack([blob_mask(h, w, dens, seed=seed + b) if dens > 0 else np.zeros((h, w), np.uint8) for b in range(n)])
+        dev = {"x": _to_dev_mask(m(50 * step + 1)), "y": _to_dev_mask(m(50 * step + 31))}
+        _run_chain(chain, seq, dev, n, planned=False)
+        _run_chain(chain, plan, dev, n, planned=True)
+        torch.cuda.synchronize()
+        for name, *_ in chain:
+            a, b = seq[name], plan[name]
+            na, ns = int(a.counts[0].item()), int(a.counts[1].item())
+            tag = "step %d set %s" % (step, name)
+            assert torch.equal(a.pixmask, b.pixmask), tag + ": pixel mask"
+            assert torch.equal(a.counts, b.counts), tag + ": counts"
+            assert torch.equal(a.flags, b.flags), tag + ": flags"
+            assert torch.equal(a.tiles[:na], b.tiles[:na]), tag + ": active list"
+            assert torch.equal(a.stale[:ns], b.stale[:ns]), tag + ": stale list"
+
+
+def test_mask_plan_that_overwrites_a_mask_it_loads():
+    # The union goes in place over a mask that the plan also loads from memory for another op: one workgroup walks such a
+    # plan, so that none can load what another has overwritten already.
+    h, w = 264, 352
+    x, y = (_to_dev_mask(blob_mask(h, w, 0.02, seed=s)[None]) for s in (3, 4))
+    want_a = mo.footprint_conv(y.cpu().numpy()[:, 0], 3, 1, 1)
+    want_u = x.cpu().numpy()[:, 0] | y.cpu().numpy()[:, 0]
+    a, u = TileMask(1, h, w, DEV), TileMask(1, h, w, DEV)
+    u.pixmask.copy_(y)
+    batch = [(u.pixmask.data_ptr(), None, h, w, _lib.FOOT_CONV, 3, 1, 1, a),
+             (x.data_ptr(), u.pixmask.data_ptr(), h, w, _lib.FOOT_CONV, 1, 1, 0, u)]
+    _lib.check(_lib.lib().mie_build_mask_plan(ops._plan_ops(batch), 2, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    _check_tileset(a, want_a)
+    _check_tileset(u, want_u)
+
+
 @pytest.mark.parametrize("n,h,w,wgs", [(1, 264, 352, 1), (1, 264, 352, 3), (4, 240, 320, 4), (4, 240, 320, 9),
                                        (3, 37, 53, 64), (2, 128, 160, 100000)])
 def test_mask_plan_held_to_few_workgroups_builds_the_same_sets(n, h, w, wgs):
