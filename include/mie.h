@@ -183,8 +183,8 @@ int mie_build_mask_tiles_thresholded(const void* delta, int c, int dtype, float 
  * the result -- every out[i].pixmask, flags, tiles, stale, counts -- is what the n_ops calls would leave when
  * issued in order on the stream.  An in_mask / in_mask2 that is the pixmask of an earlier op's `out` is taken
  * from that op (the chain never goes through memory); any other is read from memory once.  All ops share one
- * batch size out.n.  One workgroup per sample walks the chain on bitmaps in LDS; with one sample and at most 4096
- * tiles per set that is the only launch, otherwise a second kernel ranks all the lists.
+ * batch size out.n.  A workgroup walks the chain of its sample on bitmaps in LDS; with one sample, all bitmaps in LDS
+ * together and at most 4096 tiles per set that is the only launch, otherwise a second kernel ranks all the lists.
  * Limits: conv footprints of stride 1 or 2, transposed-conv footprints of stride 2 (MIE_ERR_UNSUPPORTED
  * otherwise); ops plus masks read from memory <= MIE_PLAN_MAX_STEPS, and the masks alive at one time must fit the
  * LDS of a workgroup as bitmaps (MIE_ERR_CAPACITY: split the plan, or fall back to mie_build_mask_tiles).  ops is

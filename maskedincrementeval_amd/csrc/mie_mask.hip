@@ -746,7 +746,10 @@ extern "C" int mie_build_mask_tiles_thresholded(const void* delta, int c, int dt
 // With one sample (all bitmaps resident, sets of at most 4096 tiles) a workgroup OWNS sets: it alone reads and writes their
 // flags, and ranks their lists itself at the end, so the plan is one launch.  With a batch the lists run over all samples:
 // a workgroup writes the flags of its slice of every set and k_plan_compact ranks the lists behind it, one block per 4096
-// tiles.
+// tiles.  Slots of LDS are handed out on the host by lifetime in levels.
+// Measured, both kernels together (before: one step a level, 28 words of parameters read by all 16 waves in every step, the
+// masks written between the steps, two launches): E2Depth-incr 64x96 25.8 -> 17.0 us, 264x352 37.2 -> 24.5, EVFlowNet-incr
+// 256x256 45.1 -> 23.7, 8x480x640 75.8 -> 58.6.
 namespace {
 
 constexpr int PLAN_THREADS = 1024;

@@ -72,7 +72,7 @@ def lib():
 
 
 # The builds of a planning pass are not launched one by one: they are collected and handed to the library as
-# plans (mie_build_mask_plan: the whole chain of footprints on bitmaps in LDS, two kernels per plan).  A plan the
+# plans (mie_build_mask_plan: the whole chain of footprints on bitmaps in LDS, one or two kernels a plan).  A plan the
 # library says is too long goes out in halves; a part the library does not take as a plan (a footprint it has no
 # bitmap form for, masks too large for LDS) is built set by set as before.  `fused_plan = False` restores one
 # mie_build_mask_tiles launch pair per set.  (Measured and not kept: the first one or two builds as a plan of their
