@@ -717,6 +717,21 @@ int mie_upconv_pred_masked(const void* a, const uint8_t* amask, const void* b,
                            void* pred_delta, int dtype, void* stream);
 
 /*
+ * mie_upconv_pred_masked with the tiles away from the plane's border computed at the resolution of a and b, as four 4x4
+ * convs over a + b, one per output phase (mie_upconv2x_masked): filter_up is mie_pack_filter_up2x's combined filter of
+ * `filter` in MIE_DTYPE_BF16, 16-byte aligned; a + b and the combined filter are rounded to bf16 (there: the blended
+ * up-sampled values and the filter).  Two launches.  Planes of at least 3 x 3 tiles; all else as there.
+ */
+int mie_upconv2x_pred_masked(const void* a, const uint8_t* amask, const void* b,
+                             const uint8_t* bmask, int c, int h_in, int w_in,
+                             const float* filter, const void* filter_mc, const void* filter_up,
+                             int cin_total, int cout, const mie_tileset* out, float* reservoir,
+                             int act_kind, float slope, const void* skip,
+                             const uint8_t* skip_mask, const float* pred_filter,
+                             float* pred_reservoir, int pred_act, float pred_slope,
+                             void* pred_delta, int dtype, void* stream);
+
+/*
  * Masked transposed convolution of a delta (stride s, padding p; the output
  * size out->h/w fixes output_padding): out(oy,ox,co) = sum x(iy,ix,ci) *
  * filter[ci][ky][kx][co] over oy = iy*s - p + ky, ox = ix*s - p + kx, with

@@ -200,6 +200,10 @@ bool mie_launch_upconv_persist(const ConvArgsT<mie_bf16>& a, unsigned cap, hipSt
 // ... with the network's tail fused in: the layer's activation increment is not stored; the 1x1 prediction conv over it
 // and over `skip` (32 channels, same resolution), the prediction's reservoir update and its activation increment
 // (one channel, pred_out) run in the epilogue.  pred_w: [2][32] fp32 (weights of the layer's output, of skip).
+constexpr int UP2X_UNITS = 80;      // units of a phase's combined filter (mie_upconv2x.hip)
+bool mie_launch_upconv2x_pred_persist(const ConvArgsT<mie_bf16>& a, const mie_bf16* filter_up, const uint32_t* flags,
+                                      const mie_bf16* skip, const uint8_t* skip_mask, const float* pred_w, float* pred_res,
+                                      mie_bf16* pred_out, int pred_act, float pred_slope, unsigned cap, hipStream_t st);
 bool mie_launch_upconv_pred_persist(const ConvArgsT<mie_bf16>& a, const mie_bf16* skip, const uint8_t* skip_mask,
                                     const float* pred_w, float* pred_res, mie_bf16* pred_out, int pred_act,
                                     float pred_slope, unsigned cap, hipStream_t st);

@@ -849,14 +849,13 @@ extern "C" int mie_upconv_masked(const void* a, const uint8_t* amask, const void
                               out_delta, addend, reservoir, act_kind, slope, dtype, nullptr, 0, stream);
 }
 
-extern "C" int mie_upconv_pred_masked(const void* a_lo, const uint8_t* amask, const void* b_lo, const uint8_t* bmask,
+static int upconv_pred_entry(const char* who, const void* filter_up, const void* a_lo, const uint8_t* amask, const void* b_lo, const uint8_t* bmask,
                                       int c, int h_in, int w_in, const float* filter, const void* filter_mc,
                                       int cin_total, int cout, const mie_tileset* out, float* reservoir, int act_kind,
                                       float slope, const void* skip, const uint8_t* skip_mask, const float* pred_filter,
                                       float* pred_reservoir, int pred_act, float pred_slope, void* pred_delta,
                                       int dtype, void* stream) {
   mie_clear_error();
-  const char* who = "mie_upconv_pred_masked";
   int rc = mie_check_tileset(out, who);
   if (rc != MIE_OK) return rc;
   MIE_REQUIRE(dtype == MIE_DTYPE_BF16 && c == 64 && cout == 32, MIE_ERR_UNSUPPORTED,
@@ -888,10 +887,42 @@ extern "C" int mie_upconv_pred_masked(const void* a_lo, const uint8_t* amask, co
   a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.x3 = 0;
   a.ts = mie_dev_tileset(out);
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
+  if (filter_up != nullptr) {
+    MIE_REQUIRE(mie_aligned(filter_up, 16), MIE_ERR_INVALID_ARG, "%s: misaligned operand", who);
+    MIE_REQUIRE(mie_launch_upconv2x_pred_persist(a, (const mie_bf16*)filter_up, (const uint32_t*)out->flags, (const mie_bf16*)skip,
+                                                 skip_mask, pred_filter, pred_reservoir, (mie_bf16*)pred_delta, pred_act,
+                                                 pred_slope, cap, (hipStream_t)stream),
+                MIE_ERR_UNSUPPORTED, "%s: planes of fewer than 2048 tiles (or more than 2^20), or of fewer than 3 rows or columns of "
+                "them, take the separate kernels", who);
+    return mie_check_launch(who);
+  }
   MIE_REQUIRE(mie_launch_upconv_pred_persist(a, (const mie_bf16*)skip, skip_mask, pred_filter, pred_reservoir,
                                              (mie_bf16*)pred_delta, pred_act, pred_slope, cap, (hipStream_t)stream),
               MIE_ERR_UNSUPPORTED, "%s: planes of fewer than 2048 tiles (or more than 2^20) take the separate kernels", who);
   return mie_check_launch(who);
+}
+
+extern "C" int mie_upconv_pred_masked(const void* a_lo, const uint8_t* amask, const void* b_lo, const uint8_t* bmask,
+                                      int c, int h_in, int w_in, const float* filter, const void* filter_mc,
+                                      int cin_total, int cout, const mie_tileset* out, float* reservoir, int act_kind,
+                                      float slope, const void* skip, const uint8_t* skip_mask, const float* pred_filter,
+                                      float* pred_reservoir, int pred_act, float pred_slope, void* pred_delta,
+                                      int dtype, void* stream) {
+  return upconv_pred_entry("mie_upconv_pred_masked", nullptr, a_lo, amask, b_lo, bmask, c, h_in, w_in, filter, filter_mc, cin_total, cout, out, reservoir, act_kind, slope, skip, skip_mask, pred_filter,
+                           pred_reservoir, pred_act, pred_slope, pred_delta, dtype, stream);
+}
+
+extern "C" int mie_upconv2x_pred_masked(const void* a_lo, const uint8_t* amask, const void* b_lo, const uint8_t* bmask,
+                                      int c, int h_in, int w_in, const float* filter, const void* filter_mc, const void* filter_up,
+                                      int cin_total, int cout, const mie_tileset* out, float* reservoir, int act_kind,
+                                      float slope, const void* skip, const uint8_t* skip_mask, const float* pred_filter,
+                                      float* pred_reservoir, int pred_act, float pred_slope, void* pred_delta,
+                                      int dtype, void* stream) {
+  const char* who = "mie_upconv2x_pred_masked";
+  mie_clear_error();
+  MIE_REQUIRE(filter_up != nullptr, MIE_ERR_INVALID_ARG, "%s: NULL pointer", who);
+  return upconv_pred_entry(who, filter_up, a_lo, amask, b_lo, bmask, c, h_in, w_in, filter, filter_mc, cin_total, cout, out, reservoir, act_kind, slope, skip, skip_mask, pred_filter,
+                           pred_reservoir, pred_act, pred_slope, pred_delta, dtype, stream);
 }
 
 extern "C" int mie_conv_gates_masked_ws(const void* x, const uint8_t* xmask, int c1, const void* x2,

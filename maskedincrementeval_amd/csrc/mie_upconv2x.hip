@@ -30,7 +30,7 @@ namespace {
 
 // Units of a phase's filter: 16 of the interior, [row][column]; then 12 of each side, [depth across the border][tap along
 // it], the sides at the top and the bottom followed by two groups of their corners (three taps across and a zero).
-constexpr int UNITS = 80, U_TOP = 16, U_BOTTOM = 36, U_LEFT = 56, U_RIGHT = 68;
+constexpr int UNITS = UP2X_UNITS, U_TOP = 16, U_BOTTOM = 36, U_LEFT = 56, U_RIGHT = 68;
 constexpr int STRIP = 32;                 // positions of a border workgroup
 
 struct Up2xOrder {

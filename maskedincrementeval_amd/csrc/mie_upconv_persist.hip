@@ -25,6 +25,8 @@
 
 #include <stdlib.h>
 
+#include <type_traits>
+
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -114,11 +116,15 @@ struct PredTail {
   mie_bf16* out;               // [n, h, w] prediction delta
   int act;
   float slope;
+  const uint32_t* flags;       // tile flags of the output tile set (BORDER, k_upconv2x_pred)
 };
 
-template <bool RES, int ACT, bool PRED = false>
+// BORDER: of the active tiles only those along the border of the plane (k_upconv2x_pred makes the others), found by their
+// flags instead of through the list; the stale tiles are all zeroed here.
+template <bool RES, int ACT, bool PRED = false, bool BORDER = false>
 __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16> a, PredTail pt) {
   static_assert(!PRED || RES, "the fused tail needs the layer's reservoir");
+  static_assert(!BORDER || PRED, "the border's tiles belong to the fused tail");
   __shared__ __attribute__((aligned(16))) mie_bf16 s_stage[STAGE];
   __shared__ __attribute__((aligned(16))) float s_lo[LO_F];
   __shared__ __attribute__((aligned(16))) float s_red[RED_F];
@@ -157,11 +163,21 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
 
   // ---- this workgroup's walk over the active list ------------------------------------------------------------------
   const int xcd = bid & 7, per = GRID >> 3;
-  const int c_act = (n_act + 7) >> 3;
-  const int t_hi = (xcd + 1) * c_act < n_act ? (xcd + 1) * c_act : n_act;
+  const int edge = 2 * grid.tiles_x + 2 * (grid.tiles_y - 2);        // BORDER: border tiles of a sample
+  const int n_walk = BORDER ? a.ts.n * edge : n_act;
+  const int c_act = (n_walk + 7) >> 3;
+  const int t_hi = (xcd + 1) * c_act < n_walk ? (xcd + 1) * c_act : n_walk;
   int t = xcd * c_act + (bid >> 3);
   if (t >= t_hi) return;
-  auto list_entry = [&](int pos) -> int {     // tile id at list position pos of this walk, -1 past its end
+  auto list_entry = [&](int pos) -> int {     // tile id at position pos of this walk, -1 past its end, -2: nothing to do there
+    if constexpr (BORDER) {
+      if (pos >= t_hi) return -1;
+      const int n = pos / edge, k = pos - n * edge, s = k - 2 * grid.tiles_x;
+      const int ty = k < grid.tiles_x ? 0 : (s < 0 ? grid.tiles_y - 1 : 1 + (s >> 1));
+      const int tx = s < 0 ? (k < grid.tiles_x ? k : k - grid.tiles_x) : ((s & 1) ? grid.tiles_x - 1 : 0);
+      const int v = (n * grid.tiles_y + ty) * grid.tiles_x + tx;
+      return (pt.flags[v] & 1u) != 0u ? v : -2;
+    }
     const int v = a.ts.tiles[pos < t_hi ? pos : t_hi - 1];
     return (pos < t_hi && v >= 0 && v < cap) ? v : -1;
   };
@@ -222,7 +238,14 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
   unsigned ok_a, ok_b;
   load_src(tile, ra, rb, ok_a, ok_b);
 
-  while (tile >= 0) {
+  while (BORDER ? tile != -1 : tile >= 0) {
+    if (BORDER && tile < 0) {
+      t += per;
+      tile = tile_next;
+      tile_next = list_entry(t + per);
+      load_src(tile, ra, rb, ok_a, ok_b);
+      continue;
+    }
     const TilePos tp = tile_pos(grid, tile);
     const int n = tp.n, y0 = tp.y0, x0 = tp.x0;
     const int iy0 = y0 - 2, ix0 = x0 - 2;
@@ -409,6 +432,297 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
   }
 }
 
+// ---- the same tail at the resolution of its inputs ---------------------------------------------------------------------
+// The conv over the up-sampled image is four 4x4 convs over a + b, one per output phase (py, px), away from the image's
+// border (mie_upconv2x.hip): 16 taps instead of 25, nothing to blend, and an input pixel is staged once for the four
+// outputs it stands for.  What bounds the one-tile form above is instruction issue (1900 slots a wave and tile, the blend
+// first among them); what is left here is the traffic of the reservoirs, and the wait for it.
+//   * An item is 8 x 16 input positions = 16 x 32 outputs = 2 x 4 tiles.  A workgroup (8 waves, one per CU) makes the output
+//     rows of one parity py; a wave takes one column parity px, half of the 32 output channels and half of the 64 input
+//     channels.  Its filter -- 16 taps x 32 x 16 -- stays in 64 registers for good, which leaves room for everything the
+//     next item needs.  (Four waves with 128 registers of filter each, two workgroups a CU: 370 us at 8x480x640, three
+//     quarters of them waiting, for what was asked for too late.)
+//   * 16x16x32 MFMAs with the filter as the first operand: a lane then holds four adjacent channels of one position, so
+//     reservoirs, the other delta and the prediction's products go from the accumulators to memory and back without LDS.
+//     A fragment of input row r serves the output rows r - 3 .. r: 44 fragments are read for 128 MFMAs.  The two waves
+//     that share their outputs exchange half of their sums: each finishes four of the eight rows.
+//   * Nothing is waited for where it is asked for, and loads are spread over an item: a slot of the window after next and a
+//     row of the next item's reservoir are asked for between the MFMAs of this item's sums.  (A CU keeps about 32 KB of misses
+//     on their way; asked for in one go, what an item needs -- 115 KB -- held its waves at the issue of their loads for 7400
+//     of 16000 clocks.)
+//   * One barrier an item, so that some waves make sums while others are at the reservoirs.
+//   * Tiles along the border are left to k_upconv64_persist<..., BORDER>, in a launch of its own before this one (45 us of
+//     the 268 below).
+// Sums of a wave run over K = 16 x 32 in one accumulator.  Measured against the one-tile form, all tiles active: 8x480x640
+// 570 -> 268 us (2.8 TB/s of reservoirs and deltas), 1x480x640 66 -> 49, 2x264x352 44 -> 39, 1x360x500 44 -> 38.  Error of the layer's sums
+// against fp64 in networks of 1 .. 20 % input density 0.88 - 0.91 of that form's, of the prediction's 0.91 - 0.95 (white
+// noise, which no layer sees: 1.04).
+constexpr int PR = 8, PC = 16;                     // positions of an item
+constexpr int SR = PR + 3, SC = PC + 4;            // its staged window
+constexpr int PSTG = (SR * SC + 1) * LS;           // bf16 elements; the last pixel takes what lies behind the window
+constexpr int PTHR = 512, PGRID = 256, PITEMS = 2048;      // threads, workgroups, items of a walk at most
+constexpr int PSLOT = SR * SC * Q4;                // 1760
+constexpr int PLD = (PSLOT + PTHR - 1) / PTHR;     // 4
+static_assert(PSTG * 2 * 2 + 2 * 8 * (PR / 2) * 64 * 16 + 2 * 4 * PR * PC * 4 + 512 + PITEMS * 4 + 32 + 8 * COUT <= 160 * 1024, "LDS of a CU");
+
+struct PhaseItems {
+  const mie_bf16* filter;       // the combined filter of mie_pack_filter_up2x
+  int iy, ix, total;            // items of a sample along y and x, items of all samples (at most 2^18: cap <= 2^20 tiles)
+  unsigned my, mx;              // ceil(2^32 / iy), ceil(2^32 / ix)
+};
+
+__device__ __forceinline__ v4f mma16(const v4f& w, const v4f& x, const v4f& acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mie_bf16x8, w), __builtin_bit_cast(mie_bf16x8, x), acc, 0, 0, 0);
+}
+
+template <int ACT>
+__global__ __launch_bounds__(PTHR, 2) void k_upconv2x_pred(ConvArgsT<mie_bf16> a, PredTail pt, PhaseItems g) {
+  __shared__ __attribute__((aligned(16))) mie_bf16 s_stage[2][PSTG];
+  __shared__ v4f s_sum[2][8][PR / 2][64];          // [parity of the item][wave that finishes them][row][lane]
+  __shared__ float s_z[2][2][2][PR][PC];           // [parity of the item][half of the output channels][px][row][position]
+  __shared__ unsigned char s_m[2][256];            // [parity][pixel of the window]: bit 0 a's mask, bit 1 b's
+  __shared__ unsigned s_list[PITEMS];
+  __shared__ int s_count[PTHR / 64];
+  __shared__ __attribute__((aligned(16))) float s_w[2 * COUT];
+  const int bid = blockIdx.x + conv_args_entry_zero(a);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int pos = lane & 15, cg = lane >> 4, px = wave & 1, nh = (wave >> 1) & 1, ks = wave >> 2;
+  const int xcd = bid & 7, py = (bid >> 3) & 1, step = PGRID >> 4;
+  const int H = a.h_in >> 1, W = a.w_in >> 1, hout = a.ts.h, wout = a.ts.w, tiles_x = a.ts.tiles_x, tiles_y = a.ts.tiles_y;
+  const int chunk = (g.total + 7) >> 3;
+  const int hi = (xcd + 1) * chunk < g.total ? (xcd + 1) * chunk : g.total;
+  const int first = xcd * chunk + (bid >> 4);
+  if (first >= hi) return;
+
+  // ---- the items of this walk with an active tile: place in the walk, and which of the 2 x 4 tiles (bit 4 * row + column)
+  // in the upper half
+  int n_items = 0;
+  {
+    const int n_walk = (hi - first + step - 1) / step;       // at most 2048: see the launcher
+    for (int k0 = 0; k0 < n_walk; k0 += PTHR / 8) {
+      const int k = k0 + (tid >> 3), it = first + step * k;
+      const int t2 = div_magic(it, g.ix, g.mx), n = div_magic(t2, g.iy, g.my);
+      const int ty = 1 + 2 * (t2 - n * g.iy) + ((tid >> 2) & 1), tx = 1 + 4 * (it - t2 * g.ix) + (tid & 3);
+      const bool in = k < n_walk && ty < tiles_y - 1 && tx < tiles_x - 1;
+      const unsigned f = in ? pt.flags[(n * tiles_y + ty) * tiles_x + tx] : 0u;
+      const unsigned act = (unsigned)(__ballot((f & 1u) != 0u) >> (lane & 56)) & 0xffu;
+      const bool has = (lane & 7) == 0 && act != 0u;
+      const unsigned long long b = __ballot(has);
+      if (lane == 0) s_count[wave] = __popcll(b);
+      __syncthreads();
+      int at = n_items, all = 0;
+#pragma unroll
+      for (int w = 0; w < PTHR / 64; ++w) {
+        at += w < wave ? s_count[w] : 0;
+        all += s_count[w];
+      }
+      if (has) s_list[at + __popcll(b & ((1ull << lane) - 1ull))] = (unsigned)k | act << 16;
+      n_items += all;
+      __syncthreads();
+    }
+    if (n_items == 0) return;
+  }
+  struct Item { int n, ty, tx; unsigned act; };
+  auto item_at = [&](int i) -> Item {            // past the end: the last one with nothing active
+    const unsigned e = __builtin_amdgcn_readfirstlane(s_list[i < n_items ? i : n_items - 1]);
+    const int it = first + step * (int)(e & 0xffffu);
+    const int t2 = div_magic(it, g.ix, g.mx), n = div_magic(t2, g.iy, g.my);
+    return {n, 1 + 2 * (t2 - n * g.iy), 1 + 4 * (it - t2 * g.ix), i < n_items ? e >> 16 : 0u};
+  };
+
+  // ---- this wave's filter: taps x 32 input channels x 16 output channels
+  v4f wt[16];
+  {
+    const int phase = 2 * py + px;
+    const mie_bf16* f = g.filter + ((long long)(phase * (C / 16) + 2 * ks + (cg >> 1)) * UP2X_UNITS * 2 + (cg & 1)) * COUT * EPS + (16 * nh + pos) * EPS;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) wt[t] = *reinterpret_cast<const v4f*>(f + (long long)t * 2 * COUT * EPS);
+  }
+  if (tid < 2 * COUT) s_w[tid] = pt.w[tid];
+
+  // ---- staging: slot tid + 512 i = 16 bytes (eight channels) of pixel (tid >> 3) + 64 i of the window
+  int sid = tid;         // (opaque in every item, below: the places of all slots, kept from item to item, would be spilled)
+  const bool has2 = a.x2 != nullptr;
+  const mie_bf16* x2p = has2 ? a.x2 : a.x;
+  // A mask that is not there: bytes of the tensor itself are read in its place (a branch around a load is a place where it
+  // is waited for) and `all` makes a one of them.
+  const uint8_t* m1p = a.xm != nullptr ? a.xm : reinterpret_cast<const uint8_t*>(a.x);
+  const uint8_t* m2p = has2 && a.x2m != nullptr ? a.x2m : reinterpret_cast<const uint8_t*>(x2p);
+  const unsigned m_all = (a.xm == nullptr ? 1u : 0u) | (has2 && a.x2m == nullptr ? 2u : 0u), m_use = has2 ? 3u : 1u;
+  typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;      // (said, or the selected pointer is read with flat loads)
+  const GlobalBytes skm = (GlobalBytes)(pt.skip_mask != nullptr ? pt.skip_mask : reinterpret_cast<const uint8_t*>(pt.skip));
+  const unsigned sk_all = pt.skip_mask == nullptr ? 1u : 0u;
+  // pixel p of an item's window (beyond the last inner tile, and beyond the window: read, not used)
+  auto window_pixel = [&](const Item& q, int p) -> unsigned {
+    const int r = p / SC, c = p - r * SC;
+    int y = 4 * q.ty - 2 + py + r, x = 4 * q.tx - 2 + c;
+    y = y < H ? y : H - 1;
+    x = x < W ? x : W - 1;
+    return (unsigned)((q.n * H + y) * W + x);
+  };
+  auto load_slot = [&](const Item& q, int i, float4& va, float4& vb) {
+    const unsigned eo = (window_pixel(q, (sid >> 3) + 64 * i) * C + EPS * (sid & 7)) * 2u;      // bytes: below 2^31
+    va = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.x) + eo);
+    vb = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(x2p) + eo);
+  };
+  // (masks go through LDS: two bytes a thread on their way instead of two for each slot)
+  struct MaskBytes { unsigned a, b; };
+  auto load_masks = [&](const Item& q) -> MaskBytes {
+    const unsigned po = window_pixel(q, sid < SR * SC ? sid : 0);
+    return {m1p[po], m2p[po]};
+  };
+  auto store_masks = [&](int buf, const MaskBytes& m) {
+    if (tid < 256) s_m[buf][tid] = (unsigned char)(((m.a != 0u ? 1u : 0u) | (m.b != 0u ? 2u : 0u) | m_all) & m_use);
+  };
+  auto store_slot = [&](int buf, int mbuf, int i, const float4& va, const float4& vb) {
+    const int p = (tid >> 3) + 64 * i, at = p < SR * SC ? p : SR * SC;
+    const unsigned ok = s_m[mbuf][p];
+    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float fa[8], fb[8], f[8];
+    bf16x8_to_f32((ok & 1u) ? va : z4, fa);
+    bf16x8_to_f32((ok & 2u) ? vb : z4, fb);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = fa[e] + fb[e];
+    *reinterpret_cast<float4*>(&s_stage[buf][at * LS + EPS * (tid & 7)]) = f32_to_bf16x8(f);
+  };
+
+  // ---- the rows this wave finishes: 4 ks .. 4 ks + 3 of the item, position pos, channels 16 nh + 4 cg ..
+  const unsigned row = 2u * (unsigned)wout;
+  unsigned l_pix = (unsigned)(2 * pos + px), l_ch = (unsigned)(16 * nh + 4 * cg);
+  auto item_pix = [&](const Item& q) -> long long { return ((long long)q.n * hout + 8 * q.ty + py) * wout + 8 * q.tx; };
+  auto row_live = [&](unsigned act) -> bool { return ((act >> (4 * ks + (pos >> 2))) & 1u) != 0u; };
+  struct Rows { float4 r0[PR / 2]; mie_bf16x4 sk[PR / 2]; unsigned on[PR / 2]; float p0; };
+  // the prediction: thread tid < 256 owns pixel (row tid >> 5, column tid & 31) of the item's outputs
+  const int p_r = (tid >> 5) & 7, p_x = tid & 31;
+  const unsigned p_off = p_r * row + p_x;
+  auto pred_live = [&](unsigned act) -> bool { return tid < 256 && ((act >> (4 * (p_r >> 2) + (p_x >> 3))) & 1u) != 0u; };
+  // (no branch around the loads, or what they fetch would be waited for in it: lanes of inactive tiles read the item's first
+  // pixel)
+  auto load_row = [&](Rows& rows, long long pix0, bool live, int r) {
+    const unsigned p = live ? (4 * ks + r) * row + l_pix : 0u, off = p * COUT + l_ch;       // bytes below 2^32: w < 2^20
+    rows.r0[r] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.res + pix0 * COUT) + 4u * off);
+    rows.sk[r] = *reinterpret_cast<const mie_bf16x4*>(reinterpret_cast<const char*>(pt.skip + pix0 * COUT) + 2u * off);
+    rows.on[r] = (skm + pix0)[p];
+  };
+  auto load_pred = [&](Rows& rows, long long pix0, unsigned act) { rows.p0 = (pt.res + pix0)[pred_live(act) ? p_off : 0u]; };
+
+  // ---- before the first item: its window and its rows, the second item's window and masks, the third's masks
+  Item cur = item_at(0), nxt = item_at(1), after = item_at(2);
+  float4 va[PLD], vb[PLD];
+  Rows rows_a, rows_b;
+#pragma unroll
+  for (int i = 0; i < PLD; ++i) load_slot(cur, i, va[i], vb[i]);
+  store_masks(0, load_masks(cur));
+  store_masks(1, load_masks(nxt));
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PLD; ++i) store_slot(0, 0, i, va[i], vb[i]);
+#pragma unroll
+  for (int i = 0; i < PLD; ++i) load_slot(nxt, i, va[i], vb[i]);
+  MaskBytes masks = load_masks(after);
+#pragma unroll
+  for (int r = 0; r < PR / 2; ++r) load_row(rows_a, item_pix(cur), row_live(cur.act), r);
+  load_pred(rows_a, item_pix(cur), cur.act);
+  __syncthreads();
+
+  int par = 0;
+  // the predictions of an item, once its products are in LDS: behind the next item's barrier
+  long long z_pix = 0;
+  unsigned z_act = 0u;
+  float z_p0 = 0.f;
+  auto predict = [&]() {
+    if (pred_live(z_act)) {
+      const float p1 = z_p0 + (s_z[par ^ 1][0][p_x & 1][p_r][p_x >> 1] + s_z[par ^ 1][1][p_x & 1][p_r][p_x >> 1]);
+      (pt.res + z_pix)[p_off] = p1;
+      (pt.out + z_pix)[p_off] = (mie_bf16)(mie_act(pt.act, pt.slope, p1) - mie_act(pt.act, pt.slope, z_p0));
+    }
+  };
+  auto one_item = [&](int i, const Rows& rows, Rows& rows_next) {
+    asm volatile("" : "+v"(sid), "+v"(l_pix), "+v"(l_ch));
+    const long long pix_next = item_pix(nxt);
+    const bool live_next = row_live(nxt.act);
+    // ---- sums
+    v4f acc[PR];
+    {
+#pragma unroll
+      for (int r = 0; r < PR; ++r) acc[r] = v4f{0.f, 0.f, 0.f, 0.f};
+      const mie_bf16* s = &s_stage[par][(pos + px) * LS + 32 * ks + EPS * cg];
+      constexpr int NF = 4 * SR, AHEAD = 3;          // fragments: window column j, row r; asked for three ahead
+      v4f x[AHEAD + 1];
+      auto fetch = [&](int f) { x[f % (AHEAD + 1)] = *reinterpret_cast<const v4f*>(s + ((f % SR) * SC + f / SR) * LS); };
+#pragma unroll
+      for (int f = 0; f < AHEAD; ++f) fetch(f);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        if (f + AHEAD < NF) fetch(f + AHEAD);
+        // the next item's window, a slot per window column: its conversions fill the time between MFMAs
+        // and a slot of the window behind that is asked for in its place
+        if (f % SR == 2) store_slot(par ^ 1, par ^ 1, f / SR, va[f / SR], vb[f / SR]);
+        if (f % SR == 6) load_slot(after, f / SR, va[f / SR], vb[f / SR]);
+        if (f % SR == 10) load_row(rows_next, pix_next, live_next, f / SR);
+        __builtin_amdgcn_sched_barrier(0);
+        const int j = f / SR, r = f % SR;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (r - i >= 0 && r - i < PR) acc[r - i] = mma16(wt[4 * i + j], x[f % (AHEAD + 1)], acc[r - i]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      load_pred(rows_next, pix_next, nxt.act);
+      // the rows the other wave finishes
+#pragma unroll
+      for (int r = 0; r < PR / 2; ++r) s_sum[par][wave ^ 4][r][lane] = ks == 0 ? acc[PR / 2 + r] : acc[r];
+    }
+    store_masks(par, masks);
+    // Sums exchanged; the next window is there, this one has been read; the products of the item before this are there.  (The
+    // one barrier of an item: a wave may finish this item while another makes the next one's sums.)
+    __syncthreads();
+    const Item later = item_at(i + 3);
+    masks = load_masks(later);
+    predict();
+    // ---- reservoirs and increments
+    const long long pix0 = item_pix(cur);
+    const bool live = row_live(cur.act);
+    const float4 pw_y = *reinterpret_cast<const float4*>(&s_w[16 * nh + 4 * cg]);
+    const float4 pw_s = *reinterpret_cast<const float4*>(&s_w[COUT + 16 * nh + 4 * cg]);
+    z_pix = pix0;
+    z_act = cur.act;
+    asm volatile("v_mov_b32 %0, %1" : "=v"(z_p0) : "v"(rows.p0));      // here: a copy left to the loop's end waits for the load below
+#pragma unroll
+    for (int r = 0; r < PR / 2; ++r) {
+      {
+        const v4f mine = ks == 0 ? acc[r] : acc[PR / 2 + r], other = s_sum[par][wave][r][lane];
+        const float4 q0 = rows.r0[r], q1 = make_float4(q0.x + (mine[0] + other[0]), q0.y + (mine[1] + other[1]),
+                                                       q0.z + (mine[2] + other[2]), q0.w + (mine[3] + other[3]));
+        // the increment as the bf16 delta it would be stored as
+        const float y0 = (float)(mie_bf16)(mie_act(ACT, a.slope, q1.x) - mie_act(ACT, a.slope, q0.x));
+        const float y1 = (float)(mie_bf16)(mie_act(ACT, a.slope, q1.y) - mie_act(ACT, a.slope, q0.y));
+        const float y2 = (float)(mie_bf16)(mie_act(ACT, a.slope, q1.z) - mie_act(ACT, a.slope, q0.z));
+        const float y3 = (float)(mie_bf16)(mie_act(ACT, a.slope, q1.w) - mie_act(ACT, a.slope, q0.w));
+        float z = pw_y.x * y0 + pw_y.y * y1 + pw_y.z * y2 + pw_y.w * y3;
+        const mie_bf16x4 v = rows.sk[r];
+        const float zs = pw_s.x * (float)v[0] + pw_s.y * (float)v[1] + pw_s.z * (float)v[2] + pw_s.w * (float)v[3];
+        z += (rows.on[r] | sk_all) != 0u ? zs : 0.f;
+        if (live) *reinterpret_cast<float4*>(reinterpret_cast<char*>(a.res + pix0 * COUT) + 4u * (((4 * ks + r) * row + l_pix) * COUT + l_ch)) = q1;
+        z += __shfl_xor(z, 16);
+        z += __shfl_xor(z, 32);
+        if (cg == 0) s_z[par][nh][px][4 * ks + r][pos] = z;
+      }
+    }
+    cur = nxt;
+    nxt = after;
+    after = later;
+    par ^= 1;
+  };
+  // Two items a round: the two sets of rows change places without copies, which would wait for their loads (the second may
+  // lie past the end)
+  for (int i = 0; i < n_items; i += 2) {
+    one_item(i, rows_a, rows_b);
+    one_item(i + 1, rows_b, rows_a);
+  }
+  __syncthreads();
+  predict();
+}
+
 }  // namespace
 
 // Takes the shape of the batched bf16 network's last decoder on planes large enough to keep the resident grid busy
@@ -447,11 +761,41 @@ bool mie_launch_upconv_pred_persist(const ConvArgsT<mie_bf16>& a, const mie_bf16
   PredTail pt;
   pt.skip = skip; pt.skip_mask = skip_mask; pt.w = pred_w; pt.res = pred_res; pt.out = pred_out; pt.act = pred_act;
   pt.slope = pred_slope;
+  pt.flags = nullptr;
   const dim3 g(GRID), b(256);
   switch (a.act) {
     case MIE_ACT_NONE: hipLaunchKernelGGL((k_upconv64_persist<true, MIE_ACT_NONE, true>), g, b, 0, st, a, pt); return true;
     case MIE_ACT_RELU: hipLaunchKernelGGL((k_upconv64_persist<true, MIE_ACT_RELU, true>), g, b, 0, st, a, pt); return true;
     case MIE_ACT_LEAKY_RELU: hipLaunchKernelGGL((k_upconv64_persist<true, MIE_ACT_LEAKY_RELU, true>), g, b, 0, st, a, pt); return true;
+    default: return false;
+  }
+}
+
+// The same with the inner tiles at the resolution of the inputs (filter_up: mie_pack_filter_up2x's, bf16).
+template <int ACT>
+static void launch_up2x_pred(const ConvArgsT<mie_bf16>& a, const PredTail& pt, const PhaseItems& g, hipStream_t st) {
+  hipLaunchKernelGGL((k_upconv64_persist<true, ACT, true, true>), dim3(GRID), dim3(256), 0, st, a, pt);
+  hipLaunchKernelGGL((k_upconv2x_pred<ACT>), dim3(PGRID), dim3(PTHR), 0, st, a, pt, g);
+}
+bool mie_launch_upconv2x_pred_persist(const ConvArgsT<mie_bf16>& a, const mie_bf16* filter_up, const uint32_t* flags,
+                                      const mie_bf16* skip, const uint8_t* skip_mask, const float* pred_w, float* pred_res,
+                                      mie_bf16* pred_out, int pred_act, float pred_slope, unsigned cap, hipStream_t st) {
+  if (!persist_takes(a, cap) || a.res == nullptr || a.ts.tiles_y < 3 || a.ts.tiles_x < 3 || a.ts.w >= (1 << 20)) return false;
+  PredTail pt;
+  pt.skip = skip; pt.skip_mask = skip_mask; pt.w = pred_w; pt.res = pred_res; pt.out = pred_out; pt.act = pred_act;
+  pt.slope = pred_slope; pt.flags = flags;
+  PhaseItems g;
+  g.filter = filter_up;
+  g.iy = (a.ts.tiles_y - 2 + 1) / 2;
+  g.ix = (a.ts.tiles_x - 2 + 3) / 4;
+  g.total = a.ts.n * g.iy * g.ix;
+  if (((g.total + 7) / 8 + PGRID / 16 - 1) / (PGRID / 16) > PITEMS) return false;      // (no plane of 2^20 tiles has as many)
+  g.my = 0xffffffffu / (unsigned)g.iy + 1u;
+  g.mx = 0xffffffffu / (unsigned)g.ix + 1u;
+  switch (a.act) {
+    case MIE_ACT_NONE: launch_up2x_pred<MIE_ACT_NONE>(a, pt, g, st); return true;
+    case MIE_ACT_RELU: launch_up2x_pred<MIE_ACT_RELU>(a, pt, g, st); return true;
+    case MIE_ACT_LEAKY_RELU: launch_up2x_pred<MIE_ACT_LEAKY_RELU>(a, pt, g, st); return true;
     default: return false;
   }
 }

@@ -682,7 +682,7 @@ class UNetRecurrentIncr(BaseUNetIncr):
         pkind, pslope = activation_kind(self.activation.op)
         out = pconv._delta_buf("out_act", (n, 1, H, W), a.device, a.dtype)
         ops.upconv_pred_masked(a, pa, b, pb, conv.conv2d_weights, ts_pred, res, kind, slope, ops.as_nhwc(head[0]), head[1],
-                               self._pred_tail_weights(), pres, pkind, pslope, out)
+                               self._pred_tail_weights(), pres, pkind, pslope, out, decoder.dense_plane)
         return [out, ts_pred]
 
     def _pred_tail_weights(self):

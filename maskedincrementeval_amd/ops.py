@@ -940,11 +940,12 @@ def upconv_pred_takes(c: int, cout: int, k: int, stride: int, pad: int, filt, dt
 
 
 def upconv_pred_masked(a, amask, b, bmask, filt, out_ts: TileMask, reservoir, act, slope, skip, skip_mask, pred_w,
-                       pred_res, pred_act, pred_slope, pred_out):
+                       pred_res, pred_act, pred_slope, pred_out, dense_plane=False):
     """Last decoder (5x5 conv over up2x(a + b), 64 -> 32 bf16 channels, reservoir + activation) with the 1x1
     prediction conv over (its increment + skip), the prediction's reservoir and activation increment in its epilogue.
     out_ts: the prediction's tile set; pred_w: fp32 [2, 32] (weights of the increment, of skip); pred_res fp32 and
-    pred_out bf16, both (N, 1, 2H, 2W)."""
+    pred_out bf16, both (N, 1, 2H, 2W).  dense_plane: the active pixels lie together or are all of them: the tiles away from
+    the border are then computed at the resolution of a and b, in items of 2 x 4 tiles (upconv2x_masked says why only then)."""
     n, c, h, w = a.shape
     dt = a.dtype
     if b is not None and (b.shape != a.shape or b.dtype != dt):
@@ -961,9 +962,12 @@ def upconv_pred_masked(a, amask, b, bmask, filt, out_ts: TileMask, reservoir, ac
     _require_gpu(pred_w, "pred_w")
     replay.keep(pred_w)
     _ready(out_ts)
-    check(lib().mie_upconv_pred_masked(
+    entry, up = lib().mie_upconv_pred_masked, ()
+    if dense_plane and upconv2x_enabled and cin_total == c and isinstance(filt, ConvFilter) and min(h, w) > 8:
+        entry, up = lib().mie_upconv2x_pred_masked, (replay.keep(filt.up2x(dt)).data_ptr(),)
+    check(entry(
         nhwc_ptr(a, "a", dtype=dt), pix_ptr(amask, n, h, w, "amask"), nhwc_ptr(b, "b", dtype=dt),
-        pix_ptr(bmask, n, h, w, "bmask"), c, h, w, plain.data_ptr(), mc_ptr, cin_total, cout, out_ts.ref,
+        pix_ptr(bmask, n, h, w, "bmask"), c, h, w, plain.data_ptr(), mc_ptr, *up, cin_total, cout, out_ts.ref,
         nhwc_ptr(reservoir, "reservoir"), act, float(slope), nhwc_ptr(skip, "skip", dtype=dt),
         pix_ptr(skip_mask, n, 2 * h, 2 * w, "skip_mask"), pred_w.data_ptr(), nhwc_ptr(pred_res, "pred_res"), pred_act,
         float(pred_slope), nhwc_ptr(pred_out, "pred_out", dtype=dt), code, _stream(a)))

@@ -111,3 +111,52 @@ def test_error_against_fp64_beside_the_list_driven_form(n, c, cout, h, w, dtype,
         assert err[1] < 3.0e-3 and err[1] <= (1.04 if kind == "white" else 1.0) * err[0], err
     else:
         assert err[1] <= err[0], err
+
+
+@pytest.mark.parametrize("n,h,w", [(3, 100, 118), (1, 182, 183), (2, 129, 145), (2, 10, 2100), (5, 80, 84)])
+def test_fused_tail_at_input_resolution(n, h, w):
+    # mie_upconv2x_pred_masked: the last decoder (64 -> 32, bf16) with the 1x1 prediction over its increment and a second
+    # delta.  Away from the border the conv runs at the resolution of its inputs, in items of 2 x 4 tiles: tile grids whose
+    # inner part is and is not a multiple of an item, last tiles of 2 .. 8 rows, two rows of inner tiles only; NaN in every
+    # inactive input pixel; dense, sparse, empty and one-input steps (stale tiles).
+    bf = torch.bfloat16
+    c, cout, H, W = 64, 32, 2 * h, 2 * w
+    q = lambda t: t.to(bf).float()
+    wt = he_normal_conv_weight(cout, c, 5, 9)
+    filt = ops.ConvFilter(wt.permute(1, 2, 3, 0).contiguous().to(DEV))
+    pw = q(torch.randn(cout, generator=torch.Generator().manual_seed(4)) * 0.3)
+    pred_w = torch.stack((pw, -0.5 * pw)).contiguous().to(DEV)
+    assert ops.upconv_pred_takes(c, cout, 5, 1, 2, filt, bf, _lib.tile_capacity(n, H, W), _lib.ACT_RELU)
+    ts_up, ts_dec, ts = (TileMask(n, H, W, DEV) for _ in range(3))
+    out = ops.new_nhwc(n, 1, H, W, DEV, bf)
+    res_ref, pres_ref = gaussian_delta(n, cout, H, W, 1.0, 1.0, seed=3)[0], gaussian_delta(n, 1, H, W, 1.0, 1.0, seed=5)[0]
+    res, pres = _dev(res_ref).clone(), _dev(pres_ref).clone()
+    poison = lambda t, m: torch.where(m.bool().expand_as(t), t, torch.full_like(t, float("nan")))
+    for step, (da, db, ds, two) in enumerate([(1.0, 1.0, 1.0, True), (0.02, 0.01, 0.1, True), (0.0, 0.0, 0.0, True), (0.05, 0.0, 0.3, False)]):
+        def one(ch, hh, ww, d, seed):
+            if d == 0.0:
+                return torch.zeros(n, ch, hh, ww), torch.zeros(n, 1, hh, ww, dtype=torch.uint8)
+            return gaussian_delta(n, ch, hh, ww, d, 0.5, seed=seed)
+        (a, ma), (b, mb), (sk, ms) = one(c, h, w, da, 100 + step), one(c, h, w, db, 200 + step), one(cout, H, W, ds, 300 + step)
+        a, b, sk = q(a), q(b), q(sk)
+        dma, dmb, dms = ma.to(DEV), mb.to(DEV), ms.to(DEV)
+        ops.build_mask_tiles(dma, dmb if two else None, n, h, w, _lib.FOOT_UP2X, 0, 0, 0, ts_up)
+        ops.build_mask_tiles(ts_up, None, n, H, W, _lib.FOOT_CONV, 5, 1, 2, ts_dec)
+        ops.build_mask_tiles(ts_dec, dms, n, H, W, _lib.FOOT_CONV, 1, 1, 0, ts)
+        ops.upconv_pred_masked(_dev(poison(a, ma), bf), dma, _dev(poison(b, mb), bf) if two else None, dmb if two else None, filt, ts,
+                               res, _lib.ACT_RELU, 0.0, _dev(poison(sk, ms), bf), dms, pred_w, pres, _lib.ACT_SIGMOID, 0.0, out,
+                               dense_plane=True)
+        conv = io.conv_incr(io.interp_incr(a + b if two else a), wt, 1, 2)
+        got_res = res.cpu()
+        assert torch.allclose(got_res, res_ref + conv, rtol=BF16_RTOL, atol=bf16_atol(conv, 2.0)), "step %d reservoir %.3e" % (
+            step, (got_res - res_ref - conv).abs().max())
+        # the tail from the decoder's own sums: what is left is fp32 rounding and y's rounding to bf16, which the kernel does
+        y = q(torch.relu(got_res) - torch.relu(res_ref))
+        z = (y * pw.view(1, -1, 1, 1) - 0.5 * sk * pw.view(1, -1, 1, 1)).sum(1, keepdim=True)
+        want = torch.sigmoid(pres_ref + z) - torch.sigmoid(pres_ref)
+        live = ts.pixmask.cpu().float()
+        assert torch.allclose(pres.cpu(), pres_ref + z, rtol=1e-5, atol=1e-5), "step %d: %.3e" % (step, (pres.cpu() - pres_ref - z).abs().max())
+        assert torch.allclose(out.float().cpu(), want * live, rtol=2 ** -8, atol=1e-5), "step %d: %.3e" % (
+            step, (out.float().cpu() - want * live).abs().max())
+        assert torch.count_nonzero(out.float().cpu() * (1 - live)) == 0
+        res_ref, pres_ref = got_res, pres.cpu()
