@@ -20,7 +20,9 @@ SOURCES = ["mie_mask.hip", "mie_pointwise.hip", "mie_conv.hip", "mie_conv_mfma_f
 # without the higher threshold the compiler gives up on the longest ones (the 128-column 5x5 / 7x7 kernels), their
 # operand ring is then indexed at run time and ends up in scratch memory (measured: 5.7 instead of 2.0 ms on the
 # 8x120x160 5x5 conv).  The other sources are faster with the default.
-EXTRA_FLAGS = {"mie_conv_mfma_f32.hip": ["-mllvm", "-pragma-unroll-threshold=65536"]}
+EXTRA_FLAGS = {"mie_conv_mfma_f32.hip": ["-mllvm", "-pragma-unroll-threshold=65536"],
+               # (k_upconv2x_rows: 88 fragments, 256 MFMAs)
+               "mie_upconv_persist.hip": ["-mllvm", "-pragma-unroll-threshold=65536"]}
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",

@@ -204,6 +204,9 @@ constexpr int UP2X_UNITS = 80;      // units of a phase's combined filter (mie_u
 bool mie_launch_upconv2x_pred_persist(const ConvArgsT<mie_bf16>& a, const mie_bf16* filter_up, const uint32_t* flags,
                                       const mie_bf16* skip, const uint8_t* skip_mask, const float* pred_w, float* pred_res,
                                       mie_bf16* pred_out, int pred_act, float pred_slope, unsigned cap, hipStream_t st);
+// The inner positions of a decoder layer at the resolution of its inputs (mie_upconv_persist.hip); returns false, launching
+// nothing, where k_upconv2x takes them.
+bool mie_launch_upconv2x_rows(const ConvArgsT<mie_bf16>& a, const uint32_t* flags, hipStream_t st);
 bool mie_launch_upconv_pred_persist(const ConvArgsT<mie_bf16>& a, const mie_bf16* skip, const uint8_t* skip_mask,
                                     const float* pred_w, float* pred_res, mie_bf16* pred_out, int pred_act,
                                     float pred_slope, unsigned cap, hipStream_t st);

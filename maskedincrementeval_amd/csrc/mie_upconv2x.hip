@@ -602,6 +602,13 @@ int up2x_impl(const char* who, const void* x, const uint8_t* xm, const void* x2,
   od.items = od.blocks_y * od.blocks_x + 2 * od.strips_x + 2 * od.strips_y;
   od.nci = c / 16;
   MIE_REQUIRE((long long)out->n * od.items * 4 * (cout / 32) < 0x7ffffff0LL, MIE_ERR_CAPACITY, "%s: tensor too large", who);
+  if constexpr (sizeof(T) == 2) {
+    // many items of 128 -> 64 channels: the inner positions in a persistent kernel, the strips here
+    if (mie_launch_upconv2x_rows(a, od.flags, (hipStream_t)stream)) {
+      od.blocks_y = od.blocks_x = 0;
+      od.items = 2 * od.strips_x + 2 * od.strips_y;
+    }
+  }
   launch_up2x<T>(a, od, (hipStream_t)stream);
   return mie_check_launch(who);
 }

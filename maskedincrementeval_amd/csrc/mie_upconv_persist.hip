@@ -723,6 +723,232 @@ __global__ __launch_bounds__(PTHR, 2) void k_upconv2x_pred(ConvArgsT<mie_bf16> a
   predict();
 }
 
+
+// ---- the decoder before it, 128 -> 64 channels ---------------------------------------------------------------------------
+// The inner positions of mie_upconv2x_masked's layer on planes of many items, in the same manner: an item of 8 x 16 input
+// positions, one output phase a workgroup, a wave = 16 of the 64 output channels and half of the 128 input channels, its
+// filter (16 taps x 64 x 16) in 128 registers for good, sums exchanged between the two waves that share their outputs.
+// Against k_upconv2x's blocks of 8 x 8, which read the filter (256 KB a phase) anew for each: one workgroup of eight waves a
+// CU instead of three of four, no filter traffic, and every load between MFMAs, ahead of its use: the window's slots, four at
+// a time, a slot of the window after next as one of the next window's is stored; the reservoir's rows at the beginning of
+// the sums that go with them.  A second barrier behind the exchange stands for a second buffer (32 KB that the LDS does not
+// have).  The positions along the border stay with k_upconv2x's strips.
+// Measured, all tiles active, the strips' launch included: 8x120x160 265 -> 192 us (the matrix instructions alone 144 at the
+// rate of a large product), 4x120x160 124 -> 99; in a masked 8x480x640 pass 281 -> 156 + 22.  An item takes 15500 cycles:
+// 8000 to 10500 for its 512 matrix instructions a SIMD of 16 cycles, 2000 to 4000 for the exchange and the reservoir's rows,
+// the rest at the two barriers.  The terms and their rounding are k_upconv2x's: against 64 bits the same 0.0020 from each.
+constexpr int DC = 128, DCO = 64;
+constexpr int DSC = PC + 3, DLS = DC + EPS, DQ4 = DC / EPS;
+constexpr int DPIX = SR * DSC;                     // 209 pixels of the window
+constexpr int DSTG = (DPIX + 1) * DLS;             // the last pixel takes what lies behind the window
+constexpr int DLD = (DPIX * DQ4 + PTHR - 1) / PTHR, DRING = 4;      // slots of a thread, and of them on their way at a time
+constexpr int DITEMS = 1024;
+static_assert(DSTG * 2 * 2 + 8 * (PR / 2) * 64 * 16 + 512 + DITEMS * 4 + 32 <= 160 * 1024, "LDS of a CU");
+
+template <bool RES, int ACT>
+__global__ __launch_bounds__(PTHR, 2) void k_upconv2x_rows(ConvArgsT<mie_bf16> a, const uint32_t* flags, PhaseItems g) {
+  __shared__ __attribute__((aligned(16))) mie_bf16 s_stage[2][DSTG];
+  __shared__ v4f s_sum[8][PR / 2][64];             // [wave that finishes them][row][lane]
+  __shared__ unsigned char s_m[2][256];            // [parity][pixel of the window]: bit 0 a's mask, bit 1 b's
+  __shared__ unsigned s_list[DITEMS];
+  __shared__ int s_count[PTHR / 64];
+  const int bid = blockIdx.x + conv_args_entry_zero(a);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int pos = lane & 15, cg = lane >> 4, q = wave & 3, ks = wave >> 2;
+  const int xcd = bid & 7, phase = (bid >> 3) & 3, py = phase >> 1, px = phase & 1, step = PGRID >> 5;
+  const int H = a.h_in, W = a.w_in, hout = a.ts.h, wout = a.ts.w, tiles_x = a.ts.tiles_x, tiles_y = a.ts.tiles_y;
+  const int chunk = (g.total + 7) >> 3;
+  const int hi = (xcd + 1) * chunk < g.total ? (xcd + 1) * chunk : g.total;
+  const int first = xcd * chunk + (bid >> 5);
+  if (first >= hi) return;
+
+  // ---- the items of this walk with an active or a stale tile: place in the walk (16 bits), active tiles, stale tiles (8 each;
+  // bit 4 * row + column of the 2 x 4)
+  int n_items = 0;
+  {
+    const int n_walk = (hi - first + step - 1) / step;       // at most DITEMS: see the launcher
+    for (int k0 = 0; k0 < n_walk; k0 += PTHR / 8) {
+      const int k = k0 + (tid >> 3), it = first + step * k;
+      const int t2 = div_magic(it, g.ix, g.mx), n = div_magic(t2, g.iy, g.my);
+      const int ty = 2 * (t2 - n * g.iy) + ((tid >> 2) & 1), tx = 4 * (it - t2 * g.ix) + (tid & 3);
+      const bool in = k < n_walk && ty < tiles_y && tx < tiles_x;
+      const unsigned f = in ? flags[(n * tiles_y + ty) * tiles_x + tx] : 0u;
+      const unsigned act = (unsigned)(__ballot((f & 1u) != 0u) >> (lane & 56)) & 0xffu;
+      const unsigned old = (unsigned)(__ballot((f & 3u) == 2u) >> (lane & 56)) & 0xffu;
+      const bool has = (lane & 7) == 0 && (act | old) != 0u;
+      const unsigned long long b = __ballot(has);
+      if (lane == 0) s_count[wave] = __popcll(b);
+      __syncthreads();
+      int at = n_items, all = 0;
+#pragma unroll
+      for (int w = 0; w < PTHR / 64; ++w) {
+        at += w < wave ? s_count[w] : 0;
+        all += s_count[w];
+      }
+      if (has) s_list[at + __popcll(b & ((1ull << lane) - 1ull))] = (unsigned)k | act << 16 | old << 24;
+      n_items += all;
+      __syncthreads();
+    }
+    if (n_items == 0) return;
+  }
+  struct Item { int n, y0, x0; unsigned act, old; };      // sample, first position
+  auto item_at = [&](int i) -> Item {            // past the end: the last one (looked at, not used)
+    const unsigned e = __builtin_amdgcn_readfirstlane(s_list[i < n_items ? i : n_items - 1]);
+    const int it = first + step * (int)(e & 0xffffu);
+    const int t2 = div_magic(it, g.ix, g.mx), n = div_magic(t2, g.iy, g.my);
+    return {n, PR * (t2 - n * g.iy), PC * (it - t2 * g.ix), (e >> 16) & 0xffu, e >> 24};
+  };
+
+  // ---- this wave's filter: taps x two blocks of 32 input channels x 16 output channels
+  v4f wt[16][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const mie_bf16* f = g.filter + ((long long)(phase * (DC / 16) + 4 * ks + 2 * h + (cg >> 1)) * UP2X_UNITS * 2 + (cg & 1)) * DCO * EPS + (16 * q + pos) * EPS;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) wt[t][h] = *reinterpret_cast<const v4f*>(f + (long long)t * 2 * DCO * EPS);
+  }
+
+  // ---- staging: slot tid + 512 i = 16 bytes (eight channels) of pixel (tid >> 4) + 32 i of the window
+  int sid = tid;         // (opaque in every item, below: the places of all slots, kept from item to item, would be spilled)
+  const bool has2 = a.x2 != nullptr;
+  const mie_bf16* x2p = has2 ? a.x2 : a.x;
+  // (masks that are not there: see k_upconv2x_pred)
+  const uint8_t* m1p = a.xm != nullptr ? a.xm : reinterpret_cast<const uint8_t*>(a.x);
+  const uint8_t* m2p = has2 && a.x2m != nullptr ? a.x2m : reinterpret_cast<const uint8_t*>(x2p);
+  const unsigned m_all = (a.xm == nullptr ? 1u : 0u) | (has2 && a.x2m == nullptr ? 2u : 0u), m_use = has2 ? 3u : 1u;
+  // pixel p of an item's window; edge pixels continue the plane
+  auto window_pixel = [&](const Item& o, int p) -> unsigned {
+    const int r = p / DSC, c = p - r * DSC;
+    int y = o.y0 - 2 + py + r, x = o.x0 - 2 + px + c;
+    y = y < 0 ? 0 : (y < H ? y : H - 1);
+    x = x < 0 ? 0 : (x < W ? x : W - 1);
+    return (unsigned)((o.n * H + y) * W + x);
+  };
+  auto load_slot = [&](const Item& o, int i, float4& va, float4& vb) {
+    const unsigned eo = (window_pixel(o, (sid >> 4) + 32 * i) * DC + EPS * (sid & 15)) * 2u;      // bytes: below 2^32
+    va = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.x) + eo);
+    vb = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(x2p) + eo);
+  };
+  struct MaskBytes { unsigned a, b; };
+  auto load_masks = [&](const Item& o) -> MaskBytes {
+    const unsigned po = window_pixel(o, sid < DPIX ? sid : 0);
+    return {m1p[po], m2p[po]};
+  };
+  auto store_masks = [&](int buf, const MaskBytes& m) {
+    if (tid < 256) s_m[buf][tid] = (unsigned char)(((m.a != 0u ? 1u : 0u) | (m.b != 0u ? 2u : 0u) | m_all) & m_use);
+  };
+  auto store_slot = [&](int buf, int i, const float4& va, const float4& vb) {
+    const int p = (sid >> 4) + 32 * i, at = p < DPIX ? p : DPIX;
+    const unsigned ok = s_m[buf][p];
+    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float fa[8], fb[8], f[8];
+    bf16x8_to_f32((ok & 1u) ? va : z4, fa);
+    bf16x8_to_f32((ok & 2u) ? vb : z4, fb);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = fa[e] + fb[e];
+    *reinterpret_cast<float4*>(&s_stage[buf][at * DLS + EPS * (sid & 15)]) = f32_to_bf16x8(f);
+  };
+
+  // ---- the rows this wave finishes: 4 ks .. 4 ks + 3 of the item, position pos, channels 16 q + 4 cg ..
+  const unsigned row = 2u * (unsigned)wout;
+  unsigned l_pix = (unsigned)(2 * pos + px), l_ch = (unsigned)(16 * q + 4 * cg);
+  auto item_pix = [&](const Item& o) -> long long { return ((long long)o.n * hout + 2 * o.y0 + py) * wout + 2 * o.x0; };
+  // (the first and the last row and column of positions belong to the strips)
+  auto inner = [&](const Item& o, int r) -> bool {
+    const int y = o.y0 + 4 * ks + r, x = o.x0 + pos;
+    return (y > 0) & (y < H - 1) & (x > 0) & (x < W - 1);
+  };
+  auto tile_bit = [&](unsigned bits) -> bool { return ((bits >> (4 * ks + (pos >> 2))) & 1u) != 0u; };
+  float4 r0[PR / 2];
+  auto load_row = [&](const Item& o, int r) {      // (no branch around the load; lanes without a pixel read the item's first)
+    const unsigned off = (tile_bit(o.act) & inner(o, r)) ? ((4 * ks + r) * row + l_pix) * DCO + l_ch : l_ch;
+    r0[r] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.res + item_pix(o) * DCO) + 4u * off);
+  };
+
+  // ---- before the first item: its window, the first slots of the second item's, the masks of the first three
+  Item cur = item_at(0), nxt = item_at(1), after = item_at(2);
+  float4 va[DRING], vb[DRING];
+  store_masks(0, load_masks(cur));
+  store_masks(1, load_masks(nxt));
+  __syncthreads();
+#pragma unroll
+  for (int i0 = 0; i0 < DLD; i0 += DRING) {
+#pragma unroll
+    for (int i = i0; i < i0 + DRING && i < DLD; ++i) load_slot(cur, i, va[i - i0], vb[i - i0]);
+#pragma unroll
+    for (int i = i0; i < i0 + DRING && i < DLD; ++i) store_slot(0, i, va[i - i0], vb[i - i0]);
+  }
+#pragma unroll
+  for (int i = 0; i < DRING; ++i) load_slot(nxt, i, va[i], vb[i]);
+  MaskBytes masks = load_masks(after);
+  __syncthreads();
+
+  int par = 0;
+  for (int i = 0; i < n_items; ++i, par ^= 1) {
+    asm volatile("" : "+v"(sid), "+v"(l_pix), "+v"(l_ch));
+    // ---- sums
+    v4f acc[PR];
+#pragma unroll
+    for (int r = 0; r < PR; ++r) acc[r] = v4f{0.f, 0.f, 0.f, 0.f};
+    {
+      const mie_bf16* s = &s_stage[par][pos * DLS + 64 * ks + EPS * cg];
+      constexpr int NF = 8 * SR, AHEAD = 2;          // fragments: block of channels, window column j, row r; two ahead
+      v4f x[AHEAD + 1];
+      auto fetch = [&](int f) { x[f % (AHEAD + 1)] = *reinterpret_cast<const v4f*>(s + (f % SR) * DSC * DLS + (f / SR % 4) * DLS + f / (4 * SR) * 32); };
+#pragma unroll
+      for (int f = 0; f < AHEAD; ++f) fetch(f);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        if (f + AHEAD < NF) fetch(f + AHEAD);
+        const int u = f / SR;                        // the next window's slot u; then slot u + 4, of it or of the one after it
+        if (f % SR == 2 && u < DLD) store_slot(par ^ 1, u, va[u % DRING], vb[u % DRING]);
+        if (f % SR == 6 && (u + DRING) % 8 < DLD) load_slot(u + DRING < 8 ? nxt : after, (u + DRING) % 8, va[u % DRING], vb[u % DRING]);
+        if (RES && f % SR == 9 && u < PR / 2) load_row(cur, u);
+        __builtin_amdgcn_sched_barrier(0);
+        const int h = f / (4 * SR), j = u % 4, r = f % SR;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (r - t >= 0 && r - t < PR) acc[r - t] = mma16(wt[4 * t + j][h], x[f % (AHEAD + 1)], acc[r - t]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // the rows the other wave finishes
+#pragma unroll
+      for (int r = 0; r < PR / 2; ++r) s_sum[wave ^ 4][r][lane] = ks == 0 ? acc[PR / 2 + r] : acc[r];
+    }
+    store_masks(par, masks);
+    __syncthreads();      // sums exchanged; the next window is there, this one has been read
+    v4f sum[PR / 2];
+#pragma unroll
+    for (int r = 0; r < PR / 2; ++r) {
+      const v4f mine = ks == 0 ? acc[r] : acc[PR / 2 + r];
+      sum[r] = mine + s_sum[wave][r][lane];
+    }
+    __syncthreads();      // the exchanged sums have been read
+    const Item later = item_at(i + 3);
+    masks = load_masks(later);
+    const long long pix0 = item_pix(cur);
+    const bool on = tile_bit(cur.act), zero = tile_bit(cur.old);
+#pragma unroll
+    for (int r = 0; r < PR / 2; ++r) {
+      const unsigned off = ((4 * ks + r) * row + l_pix) * DCO + l_ch;
+      mie_bf16* out = reinterpret_cast<mie_bf16*>(reinterpret_cast<char*>(a.out + pix0 * DCO) + 2u * off);
+      float4 d = make_float4(sum[r][0], sum[r][1], sum[r][2], sum[r][3]);
+      const bool in = inner(cur, r);
+      if (RES) {
+        const float4 q0 = r0[r], q1 = make_float4(q0.x + d.x, q0.y + d.y, q0.z + d.z, q0.w + d.w);
+        if (on & in) *reinterpret_cast<float4*>(reinterpret_cast<char*>(a.res + pix0 * DCO) + 4u * off) = q1;
+        d = make_float4(mie_act(ACT, a.slope, q1.x) - mie_act(ACT, a.slope, q0.x), mie_act(ACT, a.slope, q1.y) - mie_act(ACT, a.slope, q0.y),
+                        mie_act(ACT, a.slope, q1.z) - mie_act(ACT, a.slope, q0.z), mie_act(ACT, a.slope, q1.w) - mie_act(ACT, a.slope, q0.w));
+      }
+      if (!on) d = make_float4(0.f, 0.f, 0.f, 0.f);
+      if ((on | zero) & in) mie_st4(out, 0, d);
+    }
+    cur = nxt;
+    nxt = after;
+    after = later;
+  }
+}
+
 }  // namespace
 
 // Takes the shape of the batched bf16 network's last decoder on planes large enough to keep the resident grid busy
@@ -796,6 +1022,36 @@ bool mie_launch_upconv2x_pred_persist(const ConvArgsT<mie_bf16>& a, const mie_bf
     case MIE_ACT_NONE: launch_up2x_pred<MIE_ACT_NONE>(a, pt, g, st); return true;
     case MIE_ACT_RELU: launch_up2x_pred<MIE_ACT_RELU>(a, pt, g, st); return true;
     case MIE_ACT_LEAKY_RELU: launch_up2x_pred<MIE_ACT_LEAKY_RELU>(a, pt, g, st); return true;
+    default: return false;
+  }
+}
+
+// The inner positions of mie_upconv2x_masked's layer, 128 -> 64 channels in bf16 without an addend (a.h_in, a.w_in: the input
+// plane).  From three items a workgroup on (192 in all): there both forms take as long (1x120x160, 150 items, 38.1 us with
+// k_upconv2x against 36.8; 3x54x76, 210: 32.0 against 31.2; 4x66x88, 216: 48.2 against 48.3), below it the fill of 128
+// registers with the filter weighs more, and above it this one wins (2x120x160, 300: 67.8 against 58.2).  False, launching
+// nothing, for other calls.
+bool mie_launch_upconv2x_rows(const ConvArgsT<mie_bf16>& a, const uint32_t* flags, hipStream_t st) {
+  if (a.c1 != DC || a.cout != DCO || a.refresh || a.addend != nullptr || a.ts.w >= (1 << 20) || a.h_in < 3 || a.w_in < 3) return false;
+  PhaseItems g;
+  g.filter = a.filt_mc;
+  g.iy = (a.ts.tiles_y + 1) / 2;
+  g.ix = (a.ts.tiles_x + 3) / 4;
+  const long long total = (long long)a.ts.n * g.iy * g.ix;
+  if (total > (long long)DITEMS * (PGRID / 32) * 8 - 64 || 4 * total < 3 * PGRID) return false;
+  g.total = (int)total;
+  g.my = 0xffffffffu / (unsigned)g.iy + 1u;
+  g.mx = 0xffffffffu / (unsigned)g.ix + 1u;
+  const dim3 grid(PGRID), block(PTHR);
+  if (a.res == nullptr) {
+    if (a.act != MIE_ACT_NONE) return false;
+    hipLaunchKernelGGL((k_upconv2x_rows<false, MIE_ACT_NONE>), grid, block, 0, st, a, flags, g);
+    return true;
+  }
+  switch (a.act) {
+    case MIE_ACT_NONE: hipLaunchKernelGGL((k_upconv2x_rows<true, MIE_ACT_NONE>), grid, block, 0, st, a, flags, g); return true;
+    case MIE_ACT_RELU: hipLaunchKernelGGL((k_upconv2x_rows<true, MIE_ACT_RELU>), grid, block, 0, st, a, flags, g); return true;
+    case MIE_ACT_LEAKY_RELU: hipLaunchKernelGGL((k_upconv2x_rows<true, MIE_ACT_LEAKY_RELU>), grid, block, 0, st, a, flags, g); return true;
     default: return false;
   }
 }

@@ -160,3 +160,11 @@ def test_fused_tail_at_input_resolution(n, h, w):
             step, (out.float().cpu() - want * live).abs().max())
         assert torch.count_nonzero(out.float().cpu() * (1 - live)) == 0
         res_ref, pres_ref = got_res, pres.cpu()
+
+
+@pytest.mark.parametrize("n,h,w", [(3, 100, 118), (1, 150, 170), (8, 35, 67), (2, 20, 801)])
+def test_decoder_conv_of_many_items(n, h, w):
+    # 128 -> 64 channels in bf16 from three items of 8 x 16 positions a workgroup on: the persistent kernel makes all but the
+    # border's positions (the step with an addend stays with the other form).  Planes whose last item is and is not
+    # filled.
+    test_decoder_conv_at_input_resolution(n, 128, 64, h, w, torch.bfloat16)
