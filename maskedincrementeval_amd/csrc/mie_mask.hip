@@ -415,7 +415,9 @@ __device__ __forceinline__ void store_flag(uint32_t* flags, int tile, uint32_t f
 
 // true in exactly one workgroup of the grid: the one whose ticket is the last
 __device__ __forceinline__ bool last_workgroup(int32_t* counts, int* s_last) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");      // this thread's flag stores have completed
+  // This thread's flag stores have completed.  (A release fence of the workgroup does not say so: the caches a workgroup
+  // shares need no such wait, and the compiler leaves it out.)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) {
     const int t = __hip_atomic_fetch_add(&counts[MIE_CNT_TICKET], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
