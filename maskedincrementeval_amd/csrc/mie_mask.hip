@@ -407,7 +407,6 @@ __global__ __launch_bounds__(COMPACT_THREADS) void k_build_small(BuildArgs a) {
 // are ordinary stores: nothing in the kernel reads another workgroup's.
 constexpr int TICKET_CAP = 4096;
 constexpr int TICKET_THREADS = 256;
-constexpr int TICKET_ITEMS = TICKET_CAP / TICKET_THREADS;      // consecutive flags per thread
 
 __device__ __forceinline__ void store_flag(uint32_t* flags, int tile, uint32_t f) {
   __hip_atomic_store(flags + tile, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -430,50 +429,60 @@ __device__ __forceinline__ bool last_workgroup(int32_t* counts, int* s_last) {
 }
 
 // the two lists of a set of at most TICKET_CAP tiles, by the first TICKET_THREADS threads of one workgroup (all of its
-// threads call)
-__device__ void compact_by_one(const BuildArgs& a, int* s_w) {
+// threads call): flag j * TICKET_THREADS + tid in round j, ranked by ballots -- a wave's round is 64 tiles in a row, and the
+// rounds' counts, active and stale in the halves of a word, meet in LDS for one scan.  (With sixteen consecutive flags
+// per thread and two scans over the threads by shuffles, the mask and lists of 374 tiles took 1.0 us more.)
+template <int ROUNDS>
+__device__ __forceinline__ void compact_rounds(const BuildArgs& a, int* s_w) {
+  constexpr int WAVES = TICKET_THREADS / 64, WORDS = ROUNDS * WAVES;
+  static_assert(WORDS <= 64, "a wave scans the words");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  uint32_t f[TICKET_ITEMS];
-  int na = 0, ns = 0;
+  uint32_t f[ROUNDS];
+  if (wave < WAVES) {
 #pragma unroll
-  for (int j = 0; j < TICKET_ITEMS; ++j) {
-    const int t = tid * TICKET_ITEMS + j;
-    f[j] = (tid < TICKET_THREADS && t < a.cap) ? __hip_atomic_load(a.flags + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-    na += (int)(f[j] & 1u);
-    ns += (int)((f[j] & 3u) == 2u);
-  }
-  // exclusive prefix over the threads: inside the wave by shuffles, wave totals through LDS
-  int ia = na, is = ns;
+    for (int j = 0; j < ROUNDS; ++j) {      // every load goes out, from a clamped address
+      const int t = j * TICKET_THREADS + tid;
+      f[j] = __hip_atomic_load(a.flags + (t < a.cap ? t : a.cap - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int ua = __shfl_up(ia, o), us = __shfl_up(is, o);
-    if (lane >= o) ia += ua, is += us;
+    for (int j = 0; j < ROUNDS; ++j) {
+      if (j * TICKET_THREADS + tid >= a.cap) f[j] = 0u;
+      const int na = __popcll(__ballot(f[j] & 1u)), ns = __popcll(__ballot((f[j] & 3u) == 2u));
+      if (lane == 0) s_w[j * WAVES + wave] = na | ns << 16;
+    }
   }
-  if (lane == 63 && wave < TICKET_THREADS / 64) s_w[wave] = ia, s_w[4 + wave] = is;
   __syncthreads();
-  if (tid >= TICKET_THREADS) return;      // a wider workgroup: its other waves only meet the barrier
-  int pa = ia - na, ps = is - ns, ta = 0, tst = 0;
+  if (wave >= WAVES) return;      // a wider workgroup: its other waves only meet the barrier
+  int sum = lane < WORDS ? s_w[lane] : 0;
+  const int own = sum;
 #pragma unroll
-  for (int wv = 0; wv < TICKET_THREADS / 64; ++wv) {
-    if (wv < wave) pa += s_w[wv], ps += s_w[4 + wv];
-    ta += s_w[wv];
-    tst += s_w[4 + wv];
+  for (int o = 1; o < WORDS; o <<= 1) {
+    const int u = __shfl_up(sum, o);
+    if (lane >= o) sum += u;
   }
+  const int before = sum - own, all = __builtin_amdgcn_readlane(sum, WORDS - 1);
 #pragma unroll
-  for (int j = 0; j < TICKET_ITEMS; ++j) {
-    const int t = tid * TICKET_ITEMS + j;
-    if (f[j] & 1u) a.tiles[pa++] = t;
-    if ((f[j] & 3u) == 2u) a.stale[ps++] = t;
+  for (int j = 0; j < ROUNDS; ++j) {
+    const unsigned long long ba = __ballot(f[j] & 1u), bs = __ballot((f[j] & 3u) == 2u);
+    const int at = __builtin_amdgcn_readlane(before, j * WAVES + __builtin_amdgcn_readfirstlane(wave));
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const int t = j * TICKET_THREADS + tid;
+    if (f[j] & 1u) a.tiles[(at & 0xffff) + __popcll(ba & below)] = t;
+    if ((f[j] & 3u) == 2u) a.stale[(at >> 16) + __popcll(bs & below)] = t;
   }
   if (tid == 0) {
-    a.counts[MIE_CNT_ACTIVE] = ta;
-    a.counts[MIE_CNT_STALE] = tst;
+    a.counts[MIE_CNT_ACTIVE] = all & 0xffff;
+    a.counts[MIE_CNT_STALE] = all >> 16;
   }
+}
+__device__ __forceinline__ void compact_by_one(const BuildArgs& a, int* s_w) {
+  if (a.cap <= 2 * TICKET_THREADS) compact_rounds<2>(a, s_w);
+  else compact_rounds<TICKET_CAP / TICKET_THREADS>(a, s_w);
 }
 
 // k_mask_footprint + k_compact_tiles for sets of up to TICKET_CAP tiles
 __global__ __launch_bounds__(TICKET_THREADS) void k_mask_footprint_lists(BuildArgs a) {
-  __shared__ int s_w[8];
+  __shared__ int s_w[64];
   __shared__ int s_last;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tile = blockIdx.x * 4 + wave;
@@ -509,7 +518,7 @@ constexpr int TICKET_MAX_WGS = 128;      // more workgroups than this queue up a
 template <typename T>
 __global__ __launch_bounds__(1024) void k_build_thresholded(ThrArgs a) {
   __shared__ uint8_t s_in[THR_EDGE * THR_EDGE];
-  __shared__ int s_w[8];
+  __shared__ int s_w[64];
   __shared__ int s_last;
   const BuildArgs& b = a.b;
   const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63;

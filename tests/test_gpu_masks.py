@@ -66,6 +66,18 @@ def test_conv_footprint_tiles_and_stale(k, s, p, n, h, w, dens):
         prev = _check_tileset(ts, mo.footprint_conv(m, k, s, p), prev)
 
 
+@pytest.mark.parametrize("tiles", [33, 64, 255, 256, 257, 511, 512, 513, 1100])
+def test_lists_at_the_edges_of_their_rounds(tiles):
+    # one row of tiles, the last of them ragged: lists of a launch that ranks them by ballots, 256 tiles a round
+    h, w = 5, 8 * tiles - 3
+    ts, prev = TileMask(1, h, w, DEV), np.zeros(0, np.int32)
+    g = np.random.default_rng(tiles)
+    for step, dens in enumerate((0.5, 1.0, 0.0, 0.3, 0.03)):
+        m = np.repeat(g.random((1, 1, tiles)) < dens, 8, axis=2)[:, :, :w].repeat(h, axis=1).astype(np.uint8)
+        ops.build_mask_tiles(_to_dev_mask(m), None, 1, h, w, _lib.FOOT_CONV, 1, 1, 0, ts)
+        prev = _check_tileset(ts, m, prev)
+
+
 @pytest.mark.parametrize("k,s,p", [(1, 1, 0), (3, 1, 1), (3, 2, 1), (5, 1, 2), (5, 2, 2), (7, 1, 3), (3, 1, 0), (5, 2, 1), (3, 1, 2)])
 @pytest.mark.parametrize("n,h,w,c,dt,second", [(1, 33, 44, 256, torch.float32, False), (2, 45, 61, 5, torch.float32, True),
                                                (1, 132, 176, 64, torch.bfloat16, True), (4, 264, 352, 4, torch.float32, False),
