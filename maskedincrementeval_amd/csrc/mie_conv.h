@@ -51,17 +51,16 @@ static __device__ __forceinline__ int conv_args_entry_zero(const ConvArgsT<T>& a
 template <typename T>
 static __device__ __forceinline__ void conv_store(const ConvArgsT<T>& a, long long off, int co, float acc) {
   if (a.addend) acc += mie_ld(a.addend, off);
-  if (a.refresh) {
-    const float v = a.bias ? acc + a.bias[co] : acc;
-    if (a.res) a.res[off] = v;
-    mie_st(a.out, off, mie_act(a.act, a.slope, v));
-  } else if (a.res) {
-    const float r0 = a.res[off], r1 = r0 + acc;
-    a.res[off] = r1;
-    mie_st(a.out, off, mie_act(a.act, a.slope, r1) - mie_act(a.act, a.slope, r0));
-  } else {
+  if (!a.refresh && !a.res) {
     mie_st(a.out, off, acc);
+    return;
   }
+  if (a.refresh && a.bias) acc += a.bias[co];
+  const float r0 = a.refresh ? 0.f : a.res[off];
+  float r[2] = {a.refresh ? acc : r0 + acc, r0};
+  if (a.res) a.res[off] = r[0];
+  mie_act_n(a.act, a.slope, r);
+  mie_st(a.out, off, a.refresh ? r[0] : r[0] - r[1]);
 }
 
 // The same epilogue for N elements of one thread, in two halves.  conv_epilogue_load issues every
@@ -94,17 +93,15 @@ static __device__ __forceinline__ void conv_epilogue_store(const ConvArgsT<T>& a
   for (int i = 0; i < N; ++i) {
     if (!ok[i]) continue;
     float v = acc[i] + add[i];
-    if (a.refresh) {
-      if (a.bias) v += a.bias[co[i]];
-      if (a.res) a.res[off[i]] = v;
-      mie_st(a.out, off[i], mie_act(a.act, a.slope, v));
-    } else if (a.res) {
-      const float r1 = r0[i] + v;
-      a.res[off[i]] = r1;
-      mie_st(a.out, off[i], mie_act(a.act, a.slope, r1) - mie_act(a.act, a.slope, r0[i]));
-    } else {
+    if (!a.refresh && !a.res) {
       mie_st(a.out, off[i], v);
+      continue;
     }
+    if (a.refresh && a.bias) v += a.bias[co[i]];
+    float r[2] = {a.refresh ? v : r0[i] + v, r0[i]};
+    if (a.res) a.res[off[i]] = r[0];
+    mie_act_n(a.act, a.slope, r);
+    mie_st(a.out, off[i], a.refresh ? r[0] : r[0] - r[1]);
   }
 }
 
@@ -142,24 +139,19 @@ static __device__ __forceinline__ void conv_epilogue_store4(const ConvArgsT<T>& 
       continue;
     }
     float4 v = make_float4(acc[i].x + add[i].x, acc[i].y + add[i].y, acc[i].z + add[i].z, acc[i].w + add[i].w);
-    if (a.refresh) {
-      if (a.bias) {
-        v.x += a.bias[co[i]]; v.y += a.bias[co[i] + 1]; v.z += a.bias[co[i] + 2]; v.w += a.bias[co[i] + 3];
-      }
-      if (a.res) mie_st4(a.res, off[i], v);
-      mie_st4(a.out, off[i], make_float4(mie_act(a.act, a.slope, v.x), mie_act(a.act, a.slope, v.y),
-                                         mie_act(a.act, a.slope, v.z), mie_act(a.act, a.slope, v.w)));
-    } else if (a.res) {
-      const float4 r1 = make_float4(r0[i].x + v.x, r0[i].y + v.y, r0[i].z + v.z, r0[i].w + v.w);
-      mie_st4(a.res, off[i], r1);
-      mie_st4(a.out, off[i],
-              make_float4(mie_act(a.act, a.slope, r1.x) - mie_act(a.act, a.slope, r0[i].x),
-                          mie_act(a.act, a.slope, r1.y) - mie_act(a.act, a.slope, r0[i].y),
-                          mie_act(a.act, a.slope, r1.z) - mie_act(a.act, a.slope, r0[i].z),
-                          mie_act(a.act, a.slope, r1.w) - mie_act(a.act, a.slope, r0[i].w)));
-    } else {
+    if (!a.refresh && !a.res) {
       mie_st4(a.out, off[i], v);
+      continue;
     }
+    if (a.refresh && a.bias) {
+      v.x += a.bias[co[i]]; v.y += a.bias[co[i] + 1]; v.z += a.bias[co[i] + 2]; v.w += a.bias[co[i] + 3];
+    }
+    float r[8] = {a.refresh ? v.x : r0[i].x + v.x, a.refresh ? v.y : r0[i].y + v.y, a.refresh ? v.z : r0[i].z + v.z,
+                  a.refresh ? v.w : r0[i].w + v.w, r0[i].x, r0[i].y, r0[i].z, r0[i].w};
+    if (a.res) mie_st4(a.res, off[i], make_float4(r[0], r[1], r[2], r[3]));
+    mie_act_n(a.act, a.slope, r);
+    mie_st4(a.out, off[i], a.refresh ? make_float4(r[0], r[1], r[2], r[3])
+                                     : make_float4(r[0] - r[4], r[1] - r[5], r[2] - r[6], r[3] - r[7]));
   }
 }
 

@@ -786,3 +786,34 @@ def test_fused_tail_equals_decoder_then_prediction():
             step, (outs[1].float().cpu() - want).abs().max())
         # clean delta: zero outside the pixels of the prediction's tile set
         assert torch.count_nonzero(outs[1].float() * (1 - sets[1]["pred"].pixmask.float())) == 0
+
+
+# The epilogue's activations (selects for three kinds, one loop over a thread's values for the other two): the increment is
+# act(new reservoir) - act(old reservoir) of the reservoirs the conv leaves, for values on both sides of zero, far out, and
+# not finite.  Exact but for the transcendental kinds (4 ulp of a value of at most 1 in each term) and bf16's last rounding.
+@pytest.mark.parametrize("act", [_lib.ACT_NONE, _lib.ACT_RELU, _lib.ACT_LEAKY_RELU, _lib.ACT_SIGMOID, _lib.ACT_TANH])
+@pytest.mark.parametrize("cin,cout,k,path,dtype", [(32, 64, 3, _lib.PATH_MFMA, torch.float32), (64, 128, 3, _lib.PATH_MFMA, torch.bfloat16),
+                                                   (5, 32, 5, _lib.PATH_VALU, torch.float32), (32, 1, 1, _lib.PATH_VALU, torch.float32),
+                                                   (12, 20, 3, _lib.PATH_VALU, torch.float32)])
+def test_increment_of_every_activation(act, cin, cout, k, path, dtype):
+    n, h, w, slope = 2, 19, 21, 0.125
+    x, m = gaussian_delta(n, cin, h, w, 0.4, 1.0, seed=70 + act)
+    filt = _filt(he_normal_conv_weight(cout, cin, k, 71))
+    ts, out = TileMask(n, h, w, DEV), ops.new_nhwc(n, cout, h, w, DEV, dtype)
+    r0 = torch.randn(n, cout, h, w, generator=torch.Generator().manual_seed(72)) * 3
+    r0[0, 0, 3, 3], r0[0, 0, 4, 4], r0[1, 0, 5, 5], r0[1, 0, 6, 6] = float("inf"), float("-inf"), float("nan"), -90.0
+    res = _dev(r0).clone()
+    ops.build_mask_tiles(m.to(DEV), None, n, h, w, _lib.FOOT_CONV, k, 1, k // 2, ts)
+    ops.conv_masked(_dev(x).to(dtype), m.to(DEV), None, None, filt if path == _lib.PATH_MFMA else filt.plain, k, 1, k // 2, ts, out, res, act,
+                    slope, path)
+    torch.cuda.synchronize()
+    f = {_lib.ACT_NONE: lambda v: v, _lib.ACT_RELU: lambda v: torch.where(v > 0, v, torch.zeros_like(v)),
+         _lib.ACT_LEAKY_RELU: lambda v: torch.where(v > 0, v, v * slope), _lib.ACT_SIGMOID: lambda v: torch.sigmoid(v.double()).float(),
+         _lib.ACT_TANH: lambda v: torch.tanh(v.double()).float()}[act]
+    live = ts.pixmask.cpu().bool().expand_as(r0)
+    got, want = out.float().cpu()[live], (f(res.cpu()) - f(r0)).to(dtype).float()[live]
+    bits = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    tol = 8 * 2.0 ** -24 + bits if act >= _lib.ACT_SIGMOID else 0.0
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    fin = ~torch.isnan(want)
+    assert torch.allclose(got[fin], want[fin], rtol=0.0, atol=tol)
