@@ -160,7 +160,7 @@ __device__ __forceinline__ float mie_act(int kind, float slope, float v) {
 // fp32 1x64x96 201 -> 196 us, 1x264x352 461 -> 449; bf16 2x200x280 320 -> 314, 8x480x640 2740 -> 2590.
 template <int N>
 __device__ __forceinline__ void mie_act_n(int kind, float slope, float (&v)[N]) {
-  if (kind <= MIE_ACT_LEAKY_RELU) {
+  if (__builtin_expect(kind <= MIE_ACT_LEAKY_RELU, 1)) {
     const bool none = kind == MIE_ACT_NONE, leaky = kind == MIE_ACT_LEAKY_RELU;
 #pragma unroll
     for (int i = 0; i < N; ++i) {

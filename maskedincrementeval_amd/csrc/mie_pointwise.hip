@@ -119,13 +119,18 @@ __global__ __launch_bounds__(256) void k_act_incr(TileSetDev ts, int kind, float
       Vec<VEC> d = Vec<VEC>::load(din + off);
       Vec<VEC> r = Vec<VEC>::load(res + off);
       unsigned nz = 0u;
+      float v[2 * VEC];
 #pragma unroll
       for (int i = 0; i < VEC; ++i) {
-        const float r0 = r[i], r1 = r0 + d[i];
-        const float v = mie_act(kind, slope, r1) - mie_act(kind, slope, r0);
-        o[i] = v;
-        r[i] = r1;
-        nz |= (v != 0.f) ? 1u : 0u;
+        v[VEC + i] = r[i];
+        r[i] += d[i];
+        v[i] = r[i];
+      }
+      mie_act_n(kind, slope, v);
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        o[i] = v[i] - v[VEC + i];
+        nz |= (o[i] != 0.f) ? 1u : 0u;
       }
       if (!keep) r.store(res + off);
       if (out_mask && nz) atomicOr(&s_any[px], 1u);
