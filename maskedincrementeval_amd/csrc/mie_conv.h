@@ -114,15 +114,16 @@ static __device__ __forceinline__ void conv_epilogue_store(const ConvArgsT<T>& a
 template <typename T, int N>
 static __device__ __forceinline__ void conv_epilogue_load4(const ConvArgsT<T>& a, const long long (&off)[N],
                                                            const bool (&ok)[N], float4 (&r0)[N], float4 (&add)[N]) {
-  const bool want_res = a.res != nullptr && !a.refresh;
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    r0[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    add[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (ok[i]) {
-      if (a.addend) add[i] = mie_ld4(a.addend, off[i]);
-      if (want_res) r0[i] = mie_ld4(a.res, off[i]);
-    }
+  for (int i = 0; i < N; ++i) r0[i] = add[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  // (groups that are not ok read the first one's place: a branch around a load would wait for the one before it)
+  if (a.addend) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) add[i] = mie_ld4(a.addend, ok[i] ? off[i] : 0);
+  }
+  if (a.res != nullptr && !a.refresh) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) r0[i] = mie_ld4(a.res, ok[i] ? off[i] : 0);
   }
 }
 

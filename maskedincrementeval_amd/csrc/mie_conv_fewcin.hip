@@ -56,13 +56,19 @@ __global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
 
   // pixels of this thread's two epilogue groups that lie in the output pixel mask (elsewhere the sums are exactly
   // zero: no reservoir access, a zero delta); the bytes are asked for before the staging loads
-  bool live[2];
+  int live_at[2];
+  unsigned live_in = 0u;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int p = (tid + 256 * i) >> 3;
     const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
-    live[i] = oy < hout && ox < wout && (a.refresh || a.ts.pixmask[((long long)n * hout + oy) * wout + ox] != 0);
+    const bool k = oy < hout && ox < wout;
+    live_at[i] = k ? (n * hout + oy) * wout + ox : 0;
+    live_in |= (k ? 1u : 0u) << i;
   }
+  const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
+  unsigned live_b[2];
+  mie_mask_ask(live_m, a.filt, live_at, live_b);
 
   // ---- stage the input tile (fp32, 8 channels per pixel) and the filter slab ---------------------
   // Every global load of the thread is issued before the first LDS store (compile-time trip counts, fully
@@ -76,28 +82,49 @@ __global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
 #pragma unroll
     for (int tap = 0; tap < K * K; ++tap) vw[tap] = (ch < cin) ? wp[(long long)tap * cout] : 0.f;
   }
+  // (the values of masked pixels too, which the mask bytes, loaded beside them, drop)
+  constexpr int TAPS = UP ? 4 : 1;                 // source pixels of a staged one
+  const int ch = tid & 7, h_src = UP ? a.h_in >> 1 : a.h_in, w_src = UP ? a.w_in >> 1 : a.w_in;
+  int src[NIN * TAPS];
+  unsigned in = 0u;
+  float lw[UP ? NIN * TAPS : 1];
 #pragma unroll
   for (int i = 0; i < NIN; ++i) {
-    const int idx = tid + 256 * i;
-    const int pix = idx >> 3, ch = idx & 7;
+    const int pix = (tid + 256 * i) >> 3;
     const int iy = iy0 + pix / IT, ix = ix0 + pix % IT;
-    float v = 0.f;
-    if (pix < NPIX && ch < cin && iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in) {
-      if constexpr (UP) {
-        const int h_lo = a.h_in >> 1, w_lo = a.w_in >> 1;
-        int r[2], q[2];
-        float lr[2], lq[2];
-        conv_up2x_coef(iy, h_lo, r[0], r[1], lr[0], lr[1]);
-        conv_up2x_coef(ix, w_lo, q[0], q[1], lq[0], lq[1]);
+    const bool k = pix < NPIX && ch < cin && iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in;
+    if constexpr (UP) {
+      int r[2], q[2];
+      float lr[2], lq[2];
+      conv_up2x_coef(k ? iy : 0, h_src, r[0], r[1], lr[0], lr[1]);
+      conv_up2x_coef(k ? ix : 0, w_src, q[0], q[1], lq[0], lq[1]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const long long po = ((long long)n * h_lo + r[j >> 1]) * w_lo + q[j & 1];
-          if (a.xm == nullptr || a.xm[po]) v += lr[j >> 1] * lq[j & 1] * mie_ld(a.x, po * cin + ch);
-        }
-      } else {
-        const long long po = ((long long)n * a.h_in + iy) * a.w_in + ix;
-        if (a.xm == nullptr || a.xm[po]) v = mie_ld(a.x, po * cin + ch);
+      for (int j = 0; j < 4; ++j) {
+        src[4 * i + j] = k ? (n * h_src + r[j >> 1]) * w_src + q[j & 1] : 0;
+        lw[4 * i + j] = lr[j >> 1] * lq[j & 1];
+        in |= (k ? 1u : 0u) << (4 * i + j);
       }
+    } else {
+      src[i] = k ? (n * h_src + iy) * w_src + ix : 0;
+      in |= (k ? 1u : 0u) << i;
+    }
+  }
+  static_assert(NIN * TAPS <= 32, "a bit for each");
+  float raw[NIN * TAPS];
+#pragma unroll
+  for (int i = 0; i < NIN * TAPS; ++i) raw[i] = mie_ld(a.x, (long long)src[i] * cin + (ch < cin ? ch : 0));
+  unsigned b[NIN * TAPS];
+  mie_mask_ask(a.xm, a.filt, src, b);
+  mie_mask_asked();
+  const unsigned on = mie_mask_take(a.xm, b, in), live_bits = mie_mask_take(live_m, live_b, live_in);
+  const bool live[2] = {(live_bits & 1u) != 0u, (live_bits & 2u) != 0u};
+#pragma unroll
+  for (int i = 0; i < NIN; ++i) {
+    float v = 0.f;
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+      const float x = ((on >> (TAPS * i + j)) & 1u) ? raw[TAPS * i + j] : 0.f;
+      v = UP ? v + lw[UP ? TAPS * i + j : 0] * x : x;
     }
     vin[i] = v;
   }

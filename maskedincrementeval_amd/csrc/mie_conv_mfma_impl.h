@@ -466,7 +466,8 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // Epilogue (all but the gate chain): every wave parks its accumulators in LDS, and a thread then owns groups of
   // four adjacent output channels of a pixel -- 16-byte reads of the k-split partial sums, 16-byte reservoir
   // accesses, 16- / 8-byte delta accesses.  A thread's share of the output is fixed by its index, so in the k-split
-  // fp32 kernels the reservoir / addend values are fetched right away and have the whole contraction to arrive.
+  // fp32 kernels the reservoir / addend values are fetched once the mask bytes are there and have the whole contraction to
+  // arrive.
   constexpr int QPP = CO_BLK / 4;                            // groups of four channels per pixel
   constexpr int PER = GATES ? 1 : 64 * QPP / 256;            // groups per thread
   constexpr int PB = PER > 4 ? 4 : PER;                      // groups per pass of the epilogue (registers)
@@ -475,16 +476,8 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   bool e_ok[PB], e_live[PB];
   float4 e_r0[PB], e_add[PB];
   // bit g: group g of this thread lies on a pixel of the output pixel mask.  Elsewhere in an active tile the sums are
-  // exactly zero: no reservoir access, a zero delta.  (The bytes are asked for here, long before the epilogue needs them.)
+  // exactly zero: no reservoir access, a zero delta.
   unsigned live_bits = 0u;
-  if (!GATES && !SPLIT) {
-#pragma unroll
-    for (int g = 0; g < PER; ++g) {
-      const int p = (tid + 256 * g) / QPP;
-      const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
-      if (oy < hout && ox < wout && (a.refresh || a.ts.pixmask[((long long)n * hout + oy) * wout + ox] != 0)) live_bits |= 1u << g;
-    }
-  }
   // (bf16: a workgroup's contraction is too short to be worth the registers that hold these values
   // through it -- they cost a resident workgroup per CU -- so they are fetched after it instead; the same
   // holds for the 128-column slabs, whose threads own 8 groups.)
@@ -503,7 +496,6 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     }
     if (!SPLIT) conv_epilogue_load4<T, PB>(a, e_off, e_live, e_r0, e_add);
   };
-  if (!GATES && EARLY && !SPLIT) epilogue_fetch(0);
 
   v16f acc[2][NB];
   v16f accs[X3 ? 2 : 1][X3 ? NB : 1];      // X3: the small term products
@@ -569,7 +561,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // The pixel-mask bytes a workgroup needs are one more dependent round trip at its start (tile id -> mask
   // bytes -> input loads).  Where the contraction has at least four chunks, the loads of the FIRST chunk
   // therefore go out for every pixel inside the image, before the mask bytes are there (`first`), and the
-  // masked pixels are zeroed when the bytes have arrived; from the second chunk on -- and in layers of fewer
+  // masked pixels are zeroed when they are stored; from the second chunk on -- and in layers of fewer
   // chunks, where that would be a large share of the reads -- a masked pixel is not fetched at all.
   float4 st_reg[NLD][GPS];
   auto load_slots = [&](float4 (&regs)[NLD][GPS], int c, bool first) {
@@ -581,7 +573,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     // The loads are unconditional in control flow (a branch around a load makes the compiler's
     // wait counters conservative: the first MFMAs of a chunk would then wait for the whole
     // global-memory latency of these loads).  Lanes whose pixel is masked or outside the image
-    // all read one fixed, cache-resident address instead and get zeros selected afterwards,
+    // all read one fixed, cache-resident address instead, and zeros are selected when the slot is stored,
     // so inactive pixels still cost no HBM traffic.
     const T* dummy = a.filt_mc;
 #pragma unroll
@@ -591,9 +583,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       p = okb ? p : dummy;
 #pragma unroll
       for (int g = 0; g < GPS; ++g) {
-        float4 v = *reinterpret_cast<const float4*>(p + 4 * g);
-        v.x = okb ? v.x : 0.f; v.y = okb ? v.y : 0.f; v.z = okb ? v.z : 0.f; v.w = okb ? v.w : 0.f;
-        regs[i][g] = v;
+        regs[i][g] = *reinterpret_cast<const float4*>(p + 4 * g);
       }
     }
   };
@@ -608,12 +598,8 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         const bool k2 = first ? (a.x2 != nullptr && ((lo_inb >> i) & 1u)) : ((lo_ok2 >> i) & 1u);
 #pragma unroll
         for (int g = 0; g < GPS; ++g) {
-          float4 v = *reinterpret_cast<const float4*>(k1 ? a.x + eo + 4 * g : dummy);
-          float4 u = *reinterpret_cast<const float4*>(k2 ? a.x2 + eo + 4 * g : dummy);
-          v.x = k1 ? v.x : 0.f; v.y = k1 ? v.y : 0.f; v.z = k1 ? v.z : 0.f; v.w = k1 ? v.w : 0.f;
-          u.x = k2 ? u.x : 0.f; u.y = k2 ? u.y : 0.f; u.z = k2 ? u.z : 0.f; u.w = k2 ? u.w : 0.f;
-          lo_a[i][g] = v;
-          lo_b[i][g] = u;
+          lo_a[i][g] = *reinterpret_cast<const float4*>(k1 ? a.x + eo + 4 * g : dummy);
+          lo_b[i][g] = *reinterpret_cast<const float4*>(k2 ? a.x2 + eo + 4 * g : dummy);
         }
       }
       return;
@@ -632,13 +618,20 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       *reinterpret_cast<float4*>(dst) = raw[0];
     }
   };
-  auto store_slots = [&](const float4 (&regs)[NLD][GPS], int buf) {
+  auto kept = [](const float4& v, bool k) { return make_float4(k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f); };
+  auto store_slots = [&](const float4 (&regs)[NLD][GPS], int buf, unsigned ok) {
     TL* dst = sbuf + buf * (PL * STAGE);
 #pragma unroll
     for (int i = 0; i < NLD; ++i)
-      if (tid + 256 * i < NSLOT) store_slot(dst + st_lds[i], regs[i]);
+      if (tid + 256 * i < NSLOT) {
+        float4 r[GPS];
+#pragma unroll
+        for (int g = 0; g < GPS; ++g) r[g] = kept(regs[i][g], (ok >> i) & 1u);
+        store_slot(dst + st_lds[i], r);
+      }
   };
-  auto stage_store = [&](int buf) {
+  // (c: the chunk in the registers)
+  auto stage_store = [&](int buf, int c) {
     TL* dst = sbuf + buf * (PL * STAGE);
     if constexpr (UP) {
       // x + x2 of the source block to LDS in fp32 (bit pattern zero = 0 in both element types) ...
@@ -647,14 +640,17 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         const int slot = tid + 256 * i;
         const int lpix = slot / Q4, q4 = slot - lpix * Q4;
         float fa[EPS], fb[EPS];
+        const bool k1 = (lo_ok1 >> i) & 1u, k2 = (lo_ok2 >> i) & 1u;
+        const float4 a0 = kept(lo_a[i][0], k1), b0 = kept(lo_b[i][0], k2);
         if constexpr (X3) {
-          const float ta[8] = {lo_a[i][0].x, lo_a[i][0].y, lo_a[i][0].z, lo_a[i][0].w, lo_a[i][1].x, lo_a[i][1].y, lo_a[i][1].z, lo_a[i][1].w};
-          const float tb[8] = {lo_b[i][0].x, lo_b[i][0].y, lo_b[i][0].z, lo_b[i][0].w, lo_b[i][1].x, lo_b[i][1].y, lo_b[i][1].z, lo_b[i][1].w};
+          const float4 a1 = kept(lo_a[i][1], k1), b1 = kept(lo_b[i][1], k2);
+          const float ta[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+          const float tb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
 #pragma unroll
           for (int e = 0; e < 8; ++e) fa[e] = ta[e], fb[e] = tb[e];
         } else {
-          slot_to_f32(lo_a[i][0], fa, T());
-          slot_to_f32(lo_b[i][0], fb, T());
+          slot_to_f32(a0, fa, T());
+          slot_to_f32(b0, fb, T());
         }
         if (lpix < 64) {
 #pragma unroll
@@ -714,7 +710,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       }
       return;
     }
-    store_slots(st_reg, buf);
+    store_slots(st_reg, buf, c >= nch1 ? ok2 : ok1);
   };
 
   // ---- operand addressing ------------------------------------------------------------------------
@@ -824,26 +820,26 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // the pixel-mask bytes, behind the first chunk's loads (pixel 0 stands in for slots outside the image, so that
   // these loads are unconditional too)
   {
-    const bool m1 = a.xm != nullptr, has2 = a.x2 != nullptr, m2 = has2 && a.x2m != nullptr;
-    if constexpr (UP) {
-#pragma unroll
-      for (int i = 0; i < NLO; ++i) {
-        const unsigned b = (lo_inb >> i) & 1u;
-        const unsigned v1 = m1 ? (unsigned)(a.xm[lo_po[i]] != 0) : 1u;
-        const unsigned v2 = m2 ? (unsigned)(a.x2m[lo_po[i]] != 0) : (has2 ? 1u : 0u);
-        lo_ok1 |= (b & v1) << i;
-        lo_ok2 |= (b & v2) << i;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < NLD; ++i) {
-        const unsigned b = (inb >> i) & 1u;
-        const unsigned v1 = m1 ? (unsigned)(a.xm[st_po[i]] != 0) : 1u;
-        const unsigned v2 = m2 ? (unsigned)(a.x2m[st_po[i]] != 0) : (has2 ? 1u : 0u);
-        ok1 |= (b & v1) << i;
-        ok2 |= (b & v2) << i;
-      }
+    constexpr int NM = UP ? NLO : NLD;
+    constexpr bool BOTH = NM <= 8;               // (with more slots the bytes of both cost registers: x2's follow, if there are any)
+    const uint8_t* const x2m = a.x2 != nullptr ? a.x2m : nullptr;
+    unsigned b1[NM], b2[NM];
+    const auto& at = [&]() -> const int (&)[NM] { if constexpr (UP) return lo_po; else return st_po; }();
+    const unsigned in = UP ? lo_inb : inb;
+    unsigned k1, k2 = 0u;
+    mie_mask_ask(a.xm, a.filt_mc, at, b1);
+    if (BOTH) mie_mask_ask(x2m, a.filt_mc, at, b2);
+    mie_mask_asked();
+    k1 = mie_mask_take(a.xm, b1, in);
+    if (BOTH) {
+      k2 = mie_mask_take(x2m, b2, a.x2 != nullptr ? in : 0u);
+    } else if (a.x2 != nullptr) {
+      mie_mask_ask(x2m, a.filt_mc, at, b2);
+      mie_mask_asked();
+      k2 = mie_mask_take(x2m, b2, in);
     }
+    if (UP) lo_ok1 = k1, lo_ok2 = k2;
+    else ok1 = k1, ok2 = k2;
   }
   if constexpr (WOVEN) {
     if (!early) load_slots(st_first, c_lo, false);
@@ -851,30 +847,30 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   } else if (!early) stage_load(c_lo);
 #pragma unroll
   for (int i = 0; i < (PD > 0 ? PD : 1); ++i) load_b(ub_cur, i, bring[i % RING]);
-  // zero what the first chunk's loads fetched of masked pixels
-  if (!early) {
-  } else if constexpr (UP) {
+  // the output pixel mask of this thread's groups: asked for behind the first loads, taken behind their barrier
+  const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
+  unsigned live_in = 0u, live_b[PER];
+  if (!GATES && !SPLIT) {
+    int at[PER];
 #pragma unroll
-    for (int i = 0; i < NLO; ++i)
-#pragma unroll
-      for (int g = 0; g < GPS; ++g) {
-        if (!((lo_ok1 >> i) & 1u)) lo_a[i][g] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (!((lo_ok2 >> i) & 1u)) lo_b[i][g] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-  } else {
-    const unsigned ok = (c_lo >= nch1) ? ok2 : ok1;
-#pragma unroll
-    for (int i = 0; i < NLD; ++i)
-#pragma unroll
-      for (int g = 0; g < GPS; ++g)
-        if (!((ok >> i) & 1u)) {
-          if constexpr (WOVEN) st_first[i][g] = make_float4(0.f, 0.f, 0.f, 0.f);
-          else st_reg[i][g] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+    for (int g = 0; g < PER; ++g) {
+      const int p = (tid + 256 * g) / QPP;
+      const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
+      const bool k = oy < hout && ox < wout;
+      at[g] = k ? (n * hout + oy) * wout + ox : 0;
+      live_in |= (k ? 1u : 0u) << g;
+    }
+    mie_mask_ask(live_m, a.filt_mc, at, live_b);
+    mie_mask_asked();
   }
-  if constexpr (WOVEN) store_slots(st_first, 0);
-  else stage_store(0);
+  // (masked pixels that the first chunk's loads fetched are zeroed here)
+  if constexpr (WOVEN) store_slots(st_first, 0, c_lo >= nch1 ? ok2 : ok1);
+  else stage_store(0, c_lo);
   __syncthreads();
+  if (!GATES && !SPLIT) {
+    live_bits = mie_mask_take(live_m, live_b, live_in);
+    if (EARLY) epilogue_fetch(0);
+  }
   MIE_STAMP(3);
 
   // A operand of unit `unit` from the staged chunk at `sin` (one 16-byte LDS read per pixel block).
@@ -989,7 +985,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
           __builtin_amdgcn_sched_barrier(0);
         }
         if (i == UPC - 3) {
-          if (more) stage_store((c - c_lo + 1) & 1);    // the other buffer: nobody reads it during this chunk
+          if (more) stage_store((c - c_lo + 1) & 1, c + 1);    // the other buffer: nobody reads it during this chunk
           __builtin_amdgcn_sched_barrier(0);
         }
         if (i == UPC - 2) {
@@ -1031,7 +1027,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         if (PD == 0) load_b(ub_next, 0, bring[0]);   // ring of one: reload right after use
       }
       if (NBUF == 1 && !UP) __syncthreads();   // every wave is done reading the only buffer (UP: stage_store syncs)
-      if (more) stage_store((c - c_lo + 1) % NBUF);
+      if (more) stage_store((c - c_lo + 1) % NBUF, c + 1);
       __syncthreads();
       ub_cur = ub_next;
       MIE_STAMP(4 + (c - c_lo));

@@ -32,7 +32,7 @@ __host__ __device__ constexpr int tc_shift(int k, int pad) { return (tc_phase(k,
 // single-buffered.  With the accumulators of four phases it needs 140-176 registers beside them: one workgroup per CU
 // (forcing two makes it spill and costs 1 % of the EVFlowNet frame; as it is the form gains 1-2 % there).
 template <typename T, int K, int WN, bool SPLIT, bool X3 = false>
-__global__ __launch_bounds__(256) void k_tconv_mfma(ConvArgsT<T> a, TileSetDev pts) {
+__global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(ConvArgsT<T> a, TileSetDev pts) {
   static_assert(!X3 || sizeof(T) == 4, "X3: fp32 deltas");
   using TL = std::conditional_t<X3, mie_bf16, T>;            // element type in LDS and on the matrix cores
   constexpr int PL = X3 ? 3 : 1;                             // operand planes (terms per value)
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void k_tconv_mfma(ConvArgsT<T> a, TileSetDev p
   // ---- staging plan (as in k_conv_mfma, stride 1) ------------------------------------------------------
   const int iy0 = y0 - LO, ix0 = x0 - LO;
   int st_po[NLD], st_lds[NLD], st_c4[NLD];
-  unsigned ok1 = 0u, ok2 = 0u;
+  unsigned inb = 0u;
 #pragma unroll
   for (int i = 0; i < NLD; ++i) {
     const int slot = tid + 256 * i;
@@ -113,13 +113,17 @@ __global__ __launch_bounds__(256) void k_tconv_mfma(ConvArgsT<T> a, TileSetDev p
     if (slot < NSLOT) {
       const int iy = iy0 + lrow, ix = ix0 + (pix - lrow * IT);
       if (iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in) {
-        const int po = (n * a.h_in + iy) * a.w_in + ix;
-        st_po[i] = po;
-        if (a.xm == nullptr || a.xm[po]) ok1 |= 1u << i;
-        if (a.x2 != nullptr && (a.x2m == nullptr || a.x2m[po])) ok2 |= 1u << i;
+        st_po[i] = (n * a.h_in + iy) * a.w_in + ix;
+        inb |= 1u << i;
       }
     }
   }
+  const uint8_t* const x2m = a.x2 != nullptr ? a.x2m : nullptr;
+  unsigned b1[NLD], b2[NLD];
+  mie_mask_ask(a.xm, a.filt_mc, st_po, b1);
+  mie_mask_ask(x2m, a.filt_mc, st_po, b2);
+  mie_mask_asked();
+  const unsigned ok1 = mie_mask_take(a.xm, b1, inb), ok2 = mie_mask_take(x2m, b2, a.x2 != nullptr ? inb : 0u);
   const int nch1 = a.c1 / CC;
   const int nch = nch1 + (a.x2 != nullptr ? a.c2 / CC : 0);
 

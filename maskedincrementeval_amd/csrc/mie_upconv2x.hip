@@ -236,22 +236,25 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   constexpr int QPP = CO_BLK / 4;
   constexpr int PER = 64 * QPP / 256;
   constexpr int PB = PER > 4 ? 4 : PER;
-  unsigned live_bits = 0u;
+  int at[PER];
+  unsigned in = 0u;
 #pragma unroll
   for (int g = 0; g < PER; ++g) {
     const int p = (tid + 256 * g) / QPP;
     const int dy = pos_y(p), dx = pos_x(p);
-    if (dy < rows && dx < cols &&
-        (a.refresh || a.ts.pixmask[((long long)n * hout + 2 * (y0 + dy) + py) * wout + 2 * (x0 + dx) + px] != 0))
-      live_bits |= 1u << g;
+    const bool k = dy < rows && dx < cols;
+    at[g] = k ? (n * hout + 2 * (y0 + dy) + py) * wout + 2 * (x0 + dx) + px : 0;
+    in |= (k ? 1u : 0u) << g;
   }
+  const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
+  unsigned live_b[PER];
+  mie_mask_ask(live_m, a.filt_mc, at, live_b);
 
   // ---- staging plan.  A block: its 11x11 window, rows from y0 - 2 + py on.  A strip: three rows of 35, row b the pixels b
   // steps inside the border, from two (one) before the first position on.  Edge pixels continue the plane.
-  const bool m1 = a.xm != nullptr, has2 = a.x2 != nullptr, m2 = has2 && a.x2m != nullptr;
+  const bool has2 = a.x2 != nullptr;
   unsigned st_off[NLD];                                      // byte offset of the slot in chunk 0
-  int st_lds[NLD];
-  unsigned ok1 = 0u, ok2 = 0u;
+  int st_lds[NLD], st_po[NLD];
 #pragma unroll
   for (int i = 0; i < NLD; ++i) {
     const int slot = tid + 256 * i;
@@ -273,11 +276,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
     ix = ix < 0 ? 0 : (ix >= W ? W - 1 : ix);
     const int po = (n * H + iy) * W + ix;
     st_off[i] = ((unsigned)po * (unsigned)a.c1 + (unsigned)(EPS * q4)) * (unsigned)sizeof(T);
-    const unsigned v1 = m1 ? (unsigned)(a.xm[po] != 0) : 1u;
-    const unsigned v2 = m2 ? (unsigned)(a.x2m[po] != 0) : (has2 ? 1u : 0u);
-    ok1 |= v1 << i;
-    ok2 |= v2 << i;
+    st_po[i] = po;
   }
+  const uint8_t* const x2m = has2 ? a.x2m : nullptr;
+  unsigned b1[NLD], b2[NLD], ok1 = 0u, ok2 = 0u, live_bits = 0u;      // (taken behind the first chunk's loads)
+  mie_mask_ask(a.xm, a.filt_mc, st_po, b1);
+  mie_mask_ask(x2m, a.filt_mc, st_po, b2);
   const int n_slots = (side == 0 ? IT * IT : 3 * SPX) * Q4;
   const int nch = a.c1 / CC;
 
@@ -386,6 +390,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   stage_load(0);
 #pragma unroll
   for (int i = 0; i < 3; ++i) load_b(bring[i]);
+  mie_mask_asked();
+  ok1 = mie_mask_take(a.xm, b1, ~0u);
+  ok2 = mie_mask_take(x2m, b2, has2 ? ~0u : 0u);
+  live_bits = mie_mask_take(live_m, live_b, in);
   // the zero pixels
   for (int i = tid; i < NBUF * PL * (LS / EPS); i += 256) {
     const int pl = i / (LS / EPS);
