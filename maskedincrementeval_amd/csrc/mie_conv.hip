@@ -153,7 +153,7 @@ static __device__ __forceinline__ float4 load4(const mie_bf16* p) {
   return make_float4((float)b[0], (float)b[1], (float)b[2], (float)b[3]);
 }
 
-template <typename T, int LP>
+template <typename T, int LP, int CO>
 __global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
   int n, y0, x0;
   const int tk = mie_pick_tile(a.ts, blockIdx.x + conv_args_entry_zero(a), n, y0, x0);
@@ -167,28 +167,62 @@ __global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
     if (inb && sub < a.cout) mie_st(a.out, po * a.cout + sub, 0.f);
     return;
   }
+  // Everything is asked for at once: the mask bytes, the channels of both inputs (of a masked pixel too: they are dropped),
+  // their filter rows (x feeds rows [0, c1), x2 rows [c1, c1 + c2)) and what the epilogue reads.  One after the other, behind
+  // conditions, those were seven trips to memory of a kernel that does little else (with this, the transposed form below and
+  // the few-channel convs' epilogue loads ahead of their contraction: 1x64x96 pass 186.9 -> 185.3 us, optical flow with
+  // transposed convs 399.6 -> 384.5, with up-sampling 497.1 -> 488.4).
+  const bool mine_ok = inb && sub < a.cout;
+  const int pix = inb ? (int)po : 0;
+  const int at[1] = {pix};
+  const uint8_t* const x2m = a.x2 != nullptr ? a.x2m : nullptr;
+  unsigned b1[1], b2[1];
+  mie_mask_ask(a.xm, a.filt, at, b1);
+  mie_mask_ask(x2m, a.filt, at, b2);
+  const long long off = mine_ok ? po * a.cout + sub : 0;
+  const float e_add = a.addend ? mie_ld(a.addend, off) : 0.f, e_r0 = a.res && !a.refresh ? a.res[off] : 0.f;
+  const int v1 = a.c1 >> 2, vt = v1 + (a.x2 != nullptr ? a.c2 >> 2 : 0);
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int src = 0; src < 2; ++src) {        // x feeds filter rows [0, c1), x2 rows [c1, c1 + c2)
-    const T* xin = src ? a.x2 : a.x;
-    const uint8_t* xm = src ? a.x2m : a.xm;
-    const int cs = src ? a.c2 : a.c1;
-    if (xin == nullptr || !inb || (xm != nullptr && !xm[po])) continue;
-    const T* xr = xin + po * cs;
-    const float* wrow = a.filt + (long long)(src ? a.c1 : 0) * a.cout;
-    for (int v = sub; v < (cs >> 2); v += LP) {
-      const float4 x = load4(xr + 4 * v);
-      const float* wp = wrow + (long long)(4 * v) * a.cout;
-      for (int co = 0; co < a.cout; ++co)
-        acc[co] += x.x * wp[co] + x.y * wp[a.cout + co] + x.z * wp[2 * a.cout + co] + x.w * wp[3 * a.cout + co];
+  unsigned on = 0u;
+  for (int v0 = sub; v0 < vt; v0 += 4 * LP) {
+    float4 x[4], w[4][CO];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int v = v0 + u * LP, vc = v < vt ? v : sub;
+      const T* xr = vc < v1 ? a.x + ((long long)pix * a.c1 + 4 * vc) : a.x2 + ((long long)pix * a.c2 + 4 * (vc - v1));
+      x[u] = load4(xr);
+#pragma unroll
+      for (int j = 0; j < CO; ++j) w[u][j] = *reinterpret_cast<const float4*>(a.filt + 4 * (long long)(vc * CO + j));
+    }
+    if (v0 == sub) {
+      mie_mask_asked();
+      on = mie_mask_take(a.xm, b1, inb ? 1u : 0u) | mie_mask_take(x2m, b2, inb && a.x2 != nullptr ? 1u : 0u) << 1;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int v = v0 + u * LP;
+      const bool k = v < vt && ((v < v1 ? on : on >> 1) & 1u) != 0u;
+      const float xe[4] = {k ? x[u].x : 0.f, k ? x[u].y : 0.f, k ? x[u].z : 0.f, k ? x[u].w : 0.f};
+      auto row = [&](int e, int co) {      // the filter's row 4 * v + e, column co
+        const int f = e * CO + co;
+        const float4& q = w[u][f >> 2];
+        return (f & 3) == 0 ? q.x : (f & 3) == 1 ? q.y : (f & 3) == 2 ? q.z : q.w;
+      };
+#pragma unroll
+      for (int co = 0; co < CO; ++co) acc[co] += xe[0] * row(0, co) + xe[1] * row(1, co) + xe[2] * row(2, co) + xe[3] * row(3, co);
     }
   }
 #pragma unroll
-  for (int co = 0; co < 4; ++co) {           // every lane of the wave takes part
+  for (int co = 0; co < CO; ++co) {           // every lane of the wave takes part
 #pragma unroll
     for (int d = 1; d < LP; d <<= 1) acc[co] += __shfl_xor(acc[co], d);
   }
   const float mine = sub == 0 ? acc[0] : (sub == 1 ? acc[1] : (sub == 2 ? acc[2] : acc[3]));
-  if (inb && sub < a.cout) conv_store(a, po * a.cout + sub, sub, mine);
+  const long long offs[1] = {off};
+  const int cos[1] = {sub};
+  const bool oks[1] = {mine_ok};
+  const float accs[1] = {mine}, r0s[1] = {e_r0}, adds[1] = {e_add};
+  conv_epilogue_store<T, 1>(a, offs, cos, oks, accs, r0s, adds);
 }
 
 // ---------------------------------------------------------------------------------
@@ -254,30 +288,57 @@ __global__ __launch_bounds__(256) void k_tconv2x_fewcin(ConvArgsT<T> a) {
       for (int e = 0; e < 4; ++e) mie_st(a.out, off + e, 0.f);
       continue;
     }
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    const int nky = (oy & 1) ? 2 : 1, nkx = (ox & 1) ? 2 : 1;
-    for (int iky = 0; iky < nky; ++iky) {
-      const int ky = (oy & 1) ? 2 * iky : 1;
-      const int iy = (oy + 1 - ky) >> 1;
-      if (iy >= a.h_in) continue;
-      for (int ikx = 0; ikx < nkx; ++ikx) {
-        const int kx = (ox & 1) ? 2 * ikx : 1;
-        const int ix = (ox + 1 - kx) >> 1;
-        if (ix >= a.w_in) continue;
-        const long long po = ((long long)n * a.h_in + iy) * a.w_in + ix;
-        if (a.xm != nullptr && !a.xm[po]) continue;
-        const T* xr = a.x + po * c1;
-        const float* wp = a.filt + (long long)(ky * 3 + kx) * cout + 4 * g;
-        for (int ci = 0; ci < c1; ++ci) {
-          const float xv = mie_ld(xr, ci);
-          const float4 w4 = *reinterpret_cast<const float4*>(wp + (long long)ci * 9 * cout);
-          acc[0] += xv * w4.x; acc[1] += xv * w4.y; acc[2] += xv * w4.z; acc[3] += xv * w4.w;
-        }
-      }
-    }
+    // taps 2 * dy + dx, of the four those that the pixel's phase has; all their loads go out together (figures above)
+    int at[4];
+    const float* wp[4];
+    unsigned in = 0u, b1[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) conv_store(a, off + e, 4 * g + e, acc[e]);
+    for (int t = 0; t < 4; ++t) {
+      const int ky = (oy & 1) ? 2 * (t >> 1) : 1, kx = (ox & 1) ? 2 * (t & 1) : 1;
+      const int iy = (oy + 1 - ky) >> 1, ix = (ox + 1 - kx) >> 1;
+      const bool k = iy < a.h_in && ix < a.w_in && ((oy & 1) || t < 2) && ((ox & 1) || (t & 1) == 0);
+      at[t] = k ? (n * a.h_in + iy) * a.w_in + ix : 0;
+      wp[t] = a.filt + (long long)(ky * 3 + kx) * cout + 4 * g;
+      in |= (k ? 1u : 0u) << t;
+    }
+    mie_mask_ask(a.xm, a.filt, at, b1);
+    const long long offs[1] = {off};
+    const int cos[1] = {4 * g};
+    const bool oks[1] = {true};
+    float4 r0[1], add[1], acc[1] = {make_float4(0.f, 0.f, 0.f, 0.f)};
+    conv_epilogue_load4<T, 1>(a, offs, oks, r0, add);
+    unsigned on = 0u;
+    for (int ci = 0; ci < c1; ci += 2) {
+      const int c2 = ci + 1 < c1 ? ci + 1 : ci;
+      float x[4][2];
+      float4 w[4][2];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        x[t][0] = mie_ld(a.x, (long long)at[t] * c1 + ci);
+        x[t][1] = mie_ld(a.x, (long long)at[t] * c1 + c2);
+        w[t][0] = *reinterpret_cast<const float4*>(wp[t] + (long long)ci * 9 * cout);
+        w[t][1] = *reinterpret_cast<const float4*>(wp[t] + (long long)c2 * 9 * cout);
+      }
+      if (ci == 0) {
+        mie_mask_asked();
+        on = mie_mask_take(a.xm, b1, in);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float xv = ((on >> t) & 1u) != 0u && ci + e < c1 ? x[t][e] : 0.f;
+          acc[0].x += xv * w[t][e].x; acc[0].y += xv * w[t][e].y; acc[0].z += xv * w[t][e].z; acc[0].w += xv * w[t][e].w;
+        }
+    }
+    conv_epilogue_store4<T, 1>(a, offs, cos, oks, acc, r0, add);
   }
+}
+
+template <typename T, int CO>
+void launch_conv1x1(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  if (a.c1 >= 128 || a.c2 >= 128) hipLaunchKernelGGL((k_conv1x1_smallco<T, 16, CO>), dim3(cap, 4), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((k_conv1x1_smallco<T, 4, CO>), dim3(cap), dim3(256), 0, st, a);
 }
 
 template <typename T, int K, int S>
@@ -285,8 +346,12 @@ void launch_conv(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
   if (K == 1 && S == 1 && a.pad == 0 && a.cout <= 4 && (a.c1 & 3) == 0 && (a.c2 & 3) == 0) {
     // a pixel's row walked by 4 lanes is a chain of dependent rounds: 16 lanes from 128 channels on (256 at 32x32 11.4 -> 6.8 us,
     // 128 at 64x64 7.1 -> 5.6; 64 at 128x128 5.3 -> 7.5, so not there)
-    if (a.c1 >= 128 || a.c2 >= 128) hipLaunchKernelGGL((k_conv1x1_smallco<T, 16>), dim3(cap, 4), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((k_conv1x1_smallco<T, 4>), dim3(cap), dim3(256), 0, st, a);
+    switch (a.cout) {
+      case 1: launch_conv1x1<T, 1>(a, cap, st); break;
+      case 2: launch_conv1x1<T, 2>(a, cap, st); break;
+      case 3: launch_conv1x1<T, 3>(a, cap, st); break;
+      default: launch_conv1x1<T, 4>(a, cap, st);
+    }
   } else if (a.cout <= 4) {
     hipLaunchKernelGGL((k_conv_smallco<T, K, S>), dim3(cap), dim3(64), 0, st, a);
   } else {

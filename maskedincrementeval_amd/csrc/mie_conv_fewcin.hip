@@ -118,6 +118,21 @@ __global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
   mie_mask_asked();
   const unsigned on = mie_mask_take(a.xm, b, in), live_bits = mie_mask_take(live_m, live_b, live_in);
   const bool live[2] = {(live_bits & 1u) != 0u, (live_bits & 2u) != 0u};
+  // the reservoir and addend values of the epilogue have the contraction to arrive
+  long long off[2];
+  int co[2];
+  bool ok[2];
+  float4 r0[2], add[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int idx = tid + 256 * i;
+    const int p = idx >> 3, col = 4 * (idx & 7);
+    const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
+    ok[i] = oy < hout && ox < wout;
+    off[i] = (((long long)n * hout + oy) * wout + ox) * cout + co0 + col;
+    co[i] = co0 + col;
+  }
+  conv_epilogue_load4<T, 2>(a, off, live, r0, add);
 #pragma unroll
   for (int i = 0; i < NIN; ++i) {
     float v = 0.f;
@@ -166,23 +181,14 @@ __global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
     red[p * 32 + l32] = acc[r];
   }
   __syncthreads();
-  long long off[2];
-  int co[2];
-  bool ok[2];
-  float4 v[2], r0[2], add[2];
+  float4 v[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int idx = tid + 256 * i;
-    const int p = idx >> 3, col = 4 * (idx & 7);
-    const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
-    ok[i] = oy < hout && ox < wout;
-    off[i] = (((long long)n * hout + oy) * wout + ox) * cout + co0 + col;
-    co[i] = co0 + col;
     const float4 s0 = *reinterpret_cast<const float4*>(&smem[4 * idx]);
     const float4 s1 = *reinterpret_cast<const float4*>(&smem[64 * 32 + 4 * idx]);
     v[i] = make_float4(s0.x + s1.x, s0.y + s1.y, s0.z + s1.z, s0.w + s1.w);
   }
-  conv_epilogue_load4<T, 2>(a, off, live, r0, add);
   conv_epilogue_store4<T, 2>(a, off, co, ok, v, r0, add, live);
 }
 

@@ -95,6 +95,32 @@ def test_odd_channel_counts_auto_path(cin, cout, k, s, p):
     _close(conv.run(d, m), io.conv_incr(d, conv.w, s, p))
 
 
+# 1x1 convs to a few channels over two inputs: every count of output channels, inputs whose channel vectors end between two
+# rounds of a pixel's lanes, a mask that is absent, an addend.  Bound: fp32 sums of c products of rounded inputs.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("c1,c2,cout,masked2", [(20, 12, 1, True), (32, 32, 2, False), (4, 136, 3, True), (132, 4, 4, True), (8, 60, 4, False)])
+def test_two_inputs_to_a_few_channels(c1, c2, cout, masked2, dtype):
+    n, h, w = 2, 13, 21
+    x, m = gaussian_delta(n, c1, h, w, 0.3, 0.5, seed=c1)
+    x2, m2 = gaussian_delta(n, c2, h, w, 0.3, 0.5, seed=c2)
+    poison = lambda t, k: torch.where(k.bool().expand_as(t), t, torch.full_like(t, float("nan")))
+    wt = he_normal_conv_weight(cout, c1 + c2, 1, 3).to(dtype).float()      # (bf16 deltas: the filter is rounded too)
+    ts, out = TileMask(n, h, w, DEV), ops.new_nhwc(n, cout, h, w, DEV, dtype)
+    r0 = torch.randn(n, cout, h, w, generator=torch.Generator().manual_seed(4))
+    res, add = _dev(r0).clone(), torch.randn(n, cout, h, w, generator=torch.Generator().manual_seed(5)).to(dtype)
+    ops.build_mask_tiles((m | m2).to(DEV) if masked2 else None, None, n, h, w, _lib.FOOT_CONV, 1, 1, 0, ts)
+    live = ts.pixmask.cpu()
+    ops.conv_masked(_dev(poison(x, m)).to(dtype), m.to(DEV), _dev(poison(x2, m2) if masked2 else x2).to(dtype), m2.to(DEV) if masked2 else None,
+                    _filt(wt), 1, 1, 0, ts, out, res, _lib.ACT_RELU, 0.0, _lib.PATH_AUTO, _dev(add.float() * live).to(dtype))
+    torch.cuda.synchronize()
+    both = torch.cat([x, x2], 1).to(dtype).double()
+    want = (F.conv2d(both, wt.double()) + add.double()) * live.double()
+    scale = F.conv2d(both.abs(), wt.abs().double()).max().item() + 8
+    assert ((res.cpu().double() - r0.double() - want).abs().max().item()) <= (c1 + c2 + 4) * 2.0 ** -24 * scale
+    inc = torch.relu(res.cpu()) - torch.relu(r0)
+    assert torch.equal(out.cpu(), (inc * live).to(dtype))
+
+
 @pytest.mark.parametrize("pname,path", PATHS)
 def test_all_ones_mask_equals_dense_conv(pname, path):
     # reference tests/test_pointops.py:25-35, at a shape both paths take
