@@ -312,17 +312,19 @@ __device__ __forceinline__ void up2x_tile(const TileSetDev& ts, const T* __restr
     for (int idx = threadIdx.x; idx < 36 * cvb; idx += 256) {
       const int sp = idx / cvb, cq = idx - sp * cvb;
       const int sy = ry0 + sp / 6, sx = rx0 + sp % 6;
-      Vec<VEC> t = Vec<VEC>::zero();
-      if (sy >= 0 && sy < h_in && sx >= 0 && sx < w_in) {
-        const long long so = ((long long)n * h_in + sy) * w_in + sx;
-        const long long eo = so * c + (long long)(cq0 + cq) * VEC;
-        if (ma == nullptr || ma[so]) t = Vec<VEC>::load(a + eo);
-        if (b != nullptr && (mb == nullptr || mb[so])) {
-          Vec<VEC> u = Vec<VEC>::load(b + eo);
+      const bool in = sy >= 0 && sy < h_in && sx >= 0 && sx < w_in;
+      // masks and values go out together
+      const int at[1] = {in ? (n * h_in + sy) * w_in + sx : 0};
+      const long long eo = (long long)at[0] * c + (long long)(cq0 + cq) * VEC;
+      const uint8_t* const m1 = b != nullptr ? mb : nullptr;
+      unsigned b0[1], b1[1];
+      mie_mask_ask(ma, a, at, b0);
+      mie_mask_ask(m1, a, at, b1);
+      Vec<VEC> t = Vec<VEC>::load(a + eo), u = Vec<VEC>::load((b != nullptr ? b : a) + eo);
+      mie_mask_asked();
+      const bool k0 = mie_mask_take(ma, b0, in ? 1u : 0u) != 0u, k1 = mie_mask_take(m1, b1, in && b != nullptr ? 1u : 0u) != 0u;
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) t[e] += u[e];
-        }
-      }
+      for (int e = 0; e < VEC; ++e) t[e] = (k0 ? t[e] : 0.f) + (k1 ? u[e] : 0.f);
       t.store(s_src + sp * cw + cq * VEC);
     }
     __syncthreads();
