@@ -1116,6 +1116,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     }
   } else {
     // the last barrier of the main loop has retired every read of the staging buffers that is used
+    if (!EARLY && !SPLIT) epilogue_fetch(0);      // (ahead of the exchange: bf16 2x200x280 pass 298.8 -> 294.7 us with k_upconv2x's)
     float* red = smem + wk * (64 * CO_BLK);
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
@@ -1130,7 +1131,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     unsigned bad_bits = 0u;                      // groups whose sums are not finite (conv_quad_again)
 #pragma unroll
     for (int h0 = 0; h0 < PER; h0 += PB) {       // the 128-column slabs in two passes of four groups per thread
-      if (!EARLY || SPLIT) epilogue_fetch(h0);
+      if (SPLIT || h0 > 0) epilogue_fetch(h0);
       float4 v[PB];
 #pragma unroll
       for (int i = 0; i < PB; ++i) {

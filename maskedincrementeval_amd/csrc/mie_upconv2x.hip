@@ -491,6 +491,24 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   else contract(std::false_type());
 
   // ---- epilogue ----------------------------------------------------------------------------------------------------------
+  long long off[PB];
+  int co[PB];
+  bool ok[PB], live[PB];
+  float4 r0[PB], add[PB];
+  auto fetch = [&](int h0) {
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int idx = tid + 256 * (h0 + i);
+      const int p = idx / QPP, col = 4 * (idx - p * QPP);
+      const int dy = pos_y(p), dx = pos_x(p);
+      ok[i] = dy < rows && dx < cols;
+      live[i] = ((live_bits >> (h0 + i)) & 1u) != 0;
+      off[i] = (((long long)n * hout + 2 * (y0 + dy) + py) * wout + 2 * (x0 + dx) + px) * cout + co0 + col;
+      co[i] = co0 + col;
+    }
+    conv_epilogue_load4<T, PB>(a, off, live, r0, add);
+  };
+  fetch(0);      // (ahead of the exchange)
   float* red = smem + wk * (64 * CO_BLK);
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
@@ -504,21 +522,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   __syncthreads();
 #pragma unroll
   for (int h0 = 0; h0 < PER; h0 += PB) {
-    long long off[PB];
-    int co[PB];
-    bool ok[PB], live[PB];
-    float4 r0[PB], add[PB], s[PB];
-#pragma unroll
-    for (int i = 0; i < PB; ++i) {
-      const int idx = tid + 256 * (h0 + i);
-      const int p = idx / QPP, col = 4 * (idx - p * QPP);
-      const int dy = pos_y(p), dx = pos_x(p);
-      ok[i] = dy < rows && dx < cols;
-      live[i] = ((live_bits >> (h0 + i)) & 1u) != 0;
-      off[i] = (((long long)n * hout + 2 * (y0 + dy) + py) * wout + 2 * (x0 + dx) + px) * cout + co0 + col;
-      co[i] = co0 + col;
-    }
-    conv_epilogue_load4<T, PB>(a, off, live, r0, add);
+    if (h0 > 0) fetch(h0);
+    float4 s[PB];
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
       const int idx = tid + 256 * (h0 + i);
