@@ -14,7 +14,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmie_hip.so")
 SOURCES = ["mie_mask.hip", "mie_pointwise.hip", "mie_conv.hip", "mie_conv_mfma_f32.hip",
-           "mie_conv_mfma_bf16.hip", "mie_upconv_persist.hip", "mie_conv_fewcin.hip", "mie_events.hip", "mie_tail.hip", "mie_refresh.hip", "mie_tconv_mfma.hip", "mie_calls.hip", "mie_upconv2x.hip"]
+           "mie_conv_mfma_bf16.hip", "mie_upconv_persist.hip", "mie_conv_fewcin.hip", "mie_events.hip", "mie_tail.hip", "mie_refresh.hip", "mie_tconv_mfma.hip", "mie_calls.hip", "mie_upconv2x.hip", "mie_gates_pairs.hip"]
 
 # Per-source additions.  The fp32 matrix-core kernels unroll their unit loops completely (up to 196 positions);
 # without the higher threshold the compiler gives up on the longest ones (the 128-column 5x5 / 7x7 kernels), their
@@ -22,7 +22,8 @@ SOURCES = ["mie_mask.hip", "mie_pointwise.hip", "mie_conv.hip", "mie_conv_mfma_f
 # 8x120x160 5x5 conv).  The other sources are faster with the default.
 EXTRA_FLAGS = {"mie_conv_mfma_f32.hip": ["-mllvm", "-pragma-unroll-threshold=65536"],
                # (k_upconv2x_rows: 88 fragments, 256 MFMAs)
-               "mie_upconv_persist.hip": ["-mllvm", "-pragma-unroll-threshold=65536"]}
+               "mie_upconv_persist.hip": ["-mllvm", "-pragma-unroll-threshold=65536"],
+               "mie_gates_pairs.hip": ["-mllvm", "-pragma-unroll-threshold=65536"]}
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",

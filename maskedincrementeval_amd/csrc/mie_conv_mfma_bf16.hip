@@ -5,7 +5,7 @@ bool mie_launch_conv_mfma(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned c
   return launch_any<mie_bf16>(a, k, s, cap, st);
 }
 bool mie_launch_conv_gates_mfma(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) {
-  return launch_gates<mie_bf16>(a, cap, st);
+  return mie_launch_gates_pairs(a, cap, st) || launch_gates<mie_bf16>(a, cap, st);
 }
 bool mie_launch_conv_up_mfma(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) {
   // 64 -> 32 channels on a large plane: the persistent kernel (mie_upconv_persist.hip)

@@ -843,3 +843,58 @@ def test_increment_of_every_activation(act, cin, cout, k, path, dtype):
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     fin = ~torch.isnan(want)
     assert torch.allclose(got[fin], want[fin], rtol=0.0, atol=tol)
+
+
+# The bf16 gates conv of a ConvLSTM on planes of many tiles: two tiles a workgroup.  Odd numbers of active and of stale tiles,
+# ragged planes, one and two inputs, two to eight chunks, absent masks, previous-cell deltas with and without a mask.  Against
+# fp64: a gate's sum is one of K products of bf16 values added in fp32 (K * 2^-24 of sum |x||w|, a twentieth of that in
+# practice), the chain's factors are at most 1 in slope, a few fp32 roundings each, and the deltas are rounded to bf16 at the end.
+@pytest.mark.parametrize("n,h,w,c1,c2,hid,masks,prev", [(1, 128, 128, 64, 64, 64, "both", None), (4, 75, 101, 64, 64, 32, "both", "masked"),
+                                                        (1, 100, 117, 128, 128, 128, "first", "all"), (2, 61, 67, 256, 256, 128, "both", None),
+                                                        (1, 90, 190, 64, 0, 64, "both", None), (1, 130, 125, 64, 64, 64, "none", None)])
+def test_gates_conv_with_two_tiles_a_workgroup(n, h, w, c1, c2, hid, masks, prev):
+    bf = torch.bfloat16
+    cols, cin = 4 * hid, c1 + c2
+    wt = (he_normal_conv_weight(cols, cin, 3, 31) * 0.5).to(bf).float()      # columns in the gate-interleaved order
+    filt, ts = _filt(wt), TileMask(n, h, w, DEV)
+    assert (ts.capacity // 2 + 1) * (cols // 128) >= 256
+    rnd = lambda ch, seed, s=1.0: torch.randn(n, ch, h, w, generator=torch.Generator().manual_seed(seed)) * s
+    gr, cp, cell = rnd(cols, 1), rnd(hid, 2), rnd(hid, 3)
+    dgr, dcp, dcell = _dev(gr).clone(), _dev(cp).clone(), _dev(cell).clone()
+    dh, dc = (ops.new_nhwc(n, hid, h, w, DEV, bf) for _ in range(2))
+    poison = lambda t, m: torch.where(m.bool().expand_as(t), t, torch.full_like(t, float("nan")))
+    for step, dens in enumerate((0.3, 0.02, 0.0005, 0.2)):
+        x, m = gaussian_delta(n, c1, h, w, dens, 0.5, seed=90 + step)
+        x2, m2 = gaussian_delta(n, c2 or 1, h, w, dens, 0.5, seed=95 + step)
+        x, x2 = x.to(bf).float(), x2.to(bf).float()
+        both = x if c2 == 0 else torch.cat([x, x2], 1)
+        use = [m if masks != "none" else None, m2 if masks == "both" and c2 else None]
+        dm, dm2 = (None if k is None else k.to(DEV) for k in use)
+        whole = dm is None or (c2 and dm2 is None)
+        ops.build_mask_tiles(None if whole else dm, None if whole or not c2 else dm2, n, h, w, _lib.FOOT_CONV, 3, 1, 1, ts)
+        live = ts.pixmask.cpu().bool()
+        pd, pm = gaussian_delta(n, hid, h, w, 0.3, 0.3, seed=70 + step)
+        pd = pd.to(bf).float() if prev == "masked" else rnd(hid, 70 + step, 0.3).to(bf).float()
+        ops.conv_gates_incr(_dev(poison(x, m) if dm is not None else x).to(bf), dm,
+                            None if not c2 else _dev(poison(x2, m2) if dm2 is not None else x2).to(bf), dm2, filt, ts, dgr,
+                            None if prev is None else _dev(pd).to(bf), pm.to(DEV) if prev == "masked" else None, dcp, dcell, dh, dc)
+        torch.cuda.synchronize()
+        d = F.conv2d(both.double(), wt.double(), padding=1) * live.double()
+        bound = F.conv2d(both.abs().double(), wt.abs().double(), padding=1).amax().item() * 9 * cin * 2.0 ** -24
+        g0 = gr.double().view(n, hid, 4, h, w)
+        g1 = g0 + d.view(n, hid, 4, h, w)
+        p0 = cp.double()
+        pdl = (pd if prev else torch.zeros_like(pd)).double() * live.double() * (pm.double() if prev == "masked" else 1.0)
+        sg, th = torch.sigmoid, torch.tanh
+        dcw = sg(g1[:, :, 0]) * th(g1[:, :, 3]) - sg(g0[:, :, 0]) * th(g0[:, :, 3]) + sg(g1[:, :, 1]) * (p0 + pdl) - sg(g0[:, :, 1]) * p0
+        c0 = cell.double()
+        dhw = sg(g1[:, :, 2]) * th(c0 + dcw) - sg(g0[:, :, 2]) * th(c0)
+        gr, cp, cell = dgr.cpu(), dcp.cpu(), dcell.cpu()
+        scale = 4.0 + p0.abs().amax().item()
+        tol = bound * scale + 64 * 2.0 ** -24 * scale
+        assert (gr.double() - g1.reshape(n, cols, h, w)).abs().max().item() <= bound + 8 * 2.0 ** -24
+        assert (cell.double() - (c0 + dcw)).abs().max().item() <= tol and (cp.double() - (p0 + pdl)).abs().max().item() <= 8 * 2.0 ** -24
+        for got, want in ((dh, dhw), (dc, dcw)):
+            got = got.float().cpu().double()
+            assert (got - want).abs().max().item() <= tol + want.abs().max().item() * 2.0 ** -8
+            assert not got[~live.expand_as(got)].any()
