@@ -208,42 +208,47 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
     const int p = mb * 32 + l32;
     a_lane[mb] = (p >> 3) * RP + (p & 7) * LS + 16 * wave + EPS * half;
   }
-  const bool m1 = a.xm != nullptr, has2 = a.x2 != nullptr, m2 = has2 && a.x2m != nullptr;
-  const mie_bf16* dummy = a.filt_mc;      // masked lanes read one cache-resident address
+  const bool has2 = a.x2 != nullptr;
+  const uint8_t* const x2m = has2 ? a.x2m : nullptr;
+  const mie_bf16* dummy = a.filt_mc;      // lanes outside the plane read one cache-resident address
 
   // source pixels and mask bits of a tile, into registers (loads unconditional in control flow)
-  auto load_src = [&](int tile, float4 (&ra)[2], float4 (&rb)[2], unsigned& ok_a, unsigned& ok_b) {
-    ok_a = ok_b = 0u;
+  // (values and mask bytes go out together and are looked at when the tile's turn comes: with the reservoirs, the other delta
+  // and its mask likewise, the tail at 8x480x640 takes 262 us instead of 270, both launches)
+  struct Src {
+    float4 a[2], b[2];
+    unsigned ma[2], mb[2], in;
+  } src;
+  auto load_src = [&](int tile) {
     const TilePos tp = tile_pos(grid, tile < 0 ? 0 : tile);
     const int lo_y0 = ((tp.y0 - 2) >> 1) - 1, lo_x0 = ((tp.x0 - 2) >> 1) - 1;
+    int po[2];
+    src.in = 0u;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int lp = lp0 + 32 * i;
       const int ly = lo_y0 + (lp >> 3), lx = lo_x0 + (lp & 7);
       const bool inb = tile >= 0 && ly >= 0 && ly < h_lo && lx >= 0 && lx < w_lo;
-      const long long po = inb ? ((long long)tp.n * h_lo + ly) * w_lo + lx : 0;
-      const long long eo = po * C + EPS * q4;
-      const unsigned v1 = m1 ? (unsigned)(a.xm[po] != 0) : 1u;
-      const unsigned v2 = m2 ? (unsigned)(a.x2m[po] != 0) : (has2 ? 1u : 0u);
-      ra[i] = *reinterpret_cast<const float4*>(inb ? a.x + eo : dummy);
-      rb[i] = *reinterpret_cast<const float4*>((inb && has2) ? a.x2 + eo : dummy);
-      ok_a |= (inb ? v1 : 0u) << i;
-      ok_b |= (inb ? v2 : 0u) << i;
+      po[i] = inb ? (tp.n * h_lo + ly) * w_lo + lx : 0;
+      const long long eo = (long long)po[i] * C + EPS * q4;
+      src.a[i] = *reinterpret_cast<const float4*>(inb ? a.x + eo : dummy);
+      src.b[i] = *reinterpret_cast<const float4*>((inb && has2) ? a.x2 + eo : dummy);
+      src.in |= (inb ? 1u : 0u) << i;
     }
+    mie_mask_ask(a.xm, dummy, po, src.ma);
+    mie_mask_ask(x2m, dummy, po, src.mb);
   };
 
   int tile = list_entry(t);
   int tile_next = list_entry(t + per);
-  float4 ra[2], rb[2];
-  unsigned ok_a, ok_b;
-  load_src(tile, ra, rb, ok_a, ok_b);
+  load_src(tile);
 
   while (BORDER ? tile != -1 : tile >= 0) {
     if (BORDER && tile < 0) {
       t += per;
       tile = tile_next;
       tile_next = list_entry(t + per);
-      load_src(tile, ra, rb, ok_a, ok_b);
+      load_src(tile);
       continue;
     }
     const TilePos tp = tile_pos(grid, tile);
@@ -252,10 +257,13 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
     const int lo_y0 = (iy0 >> 1) - 1, lo_x0 = (ix0 >> 1) - 1;
 
     // A. a + b of the source block to LDS, fp32 (masked pixels: the raw registers are zeroed, bit pattern 0 = 0.0)
+    const unsigned ok_a = mie_mask_take(a.xm, src.ma, src.in), ok_b = mie_mask_take(x2m, src.mb, has2 ? src.in : 0u);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const bool ka = (ok_a >> i) & 1u, kb = (ok_b >> i) & 1u;
-      const float4 za = ka ? ra[i] : make_float4(0.f, 0.f, 0.f, 0.f), zb = kb ? rb[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 ra = src.a[i], rb = src.b[i];
+      const float4 za = make_float4(ka ? ra.x : 0.f, ka ? ra.y : 0.f, ka ? ra.z : 0.f, ka ? ra.w : 0.f);
+      const float4 zb = make_float4(kb ? rb.x : 0.f, kb ? rb.y : 0.f, kb ? rb.z : 0.f, kb ? rb.w : 0.f);
       float fa[8], fb[8];
       bf16x8_to_f32(za, fa);
       bf16x8_to_f32(zb, fb);
@@ -268,36 +276,34 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
     long long e_off[2];
     bool e_ok[2];
     float4 e_r0[2];
-    long long t_pix[2];          // PRED: pixel index, the second delta's four channels, the prediction's reservoir value
-    float4 t_skip[2];
+    long long t_pix[2];          // PRED: pixel index, the second delta's four channels and mask, the prediction's reservoir value
+    mie_bf16x4 t_skip[2];
     float t_p0[2];
+    int t_at[2];
+    unsigned t_in = 0u, t_m[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int idx = tid + 256 * i;
       const int p = idx >> 3, col = 4 * (idx & 7);
       const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
       e_ok[i] = oy < hout && ox < wout;
-      e_off[i] = (((long long)n * hout + oy) * wout + ox) * COUT + col;
+      const int pix = e_ok[i] ? (n * hout + oy) * wout + ox : 0;
+      e_off[i] = (long long)pix * COUT + col;
       e_r0[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (RES && e_ok[i]) e_r0[i] = *reinterpret_cast<const float4*>(a.res + e_off[i]);
+      if (RES) e_r0[i] = *reinterpret_cast<const float4*>(a.res + e_off[i]);
       if (PRED) {
-        const long long pix = ((long long)n * hout + oy) * wout + ox;
-        t_pix[i] = pix;
-        t_skip[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        t_p0[i] = 0.f;
-        if (e_ok[i]) {
-          const bool on = pt.skip_mask == nullptr || pt.skip_mask[pix] != 0;
-          const mie_bf16x4 sv = *reinterpret_cast<const mie_bf16x4*>(pt.skip + pix * COUT + col);
-          if (on) t_skip[i] = make_float4((float)sv[0], (float)sv[1], (float)sv[2], (float)sv[3]);
-          if ((tid & 7) == 0) t_p0[i] = pt.res[pix];
-        }
+        t_pix[i] = t_at[i] = pix;
+        t_in |= (e_ok[i] ? 1u : 0u) << i;
+        t_skip[i] = *reinterpret_cast<const mie_bf16x4*>(pt.skip + e_off[i]);
+        t_p0[i] = pt.res[pix];
       }
     }
+    if (PRED) mie_mask_ask(pt.skip_mask, dummy, t_at, t_m);
 
     // C. the next tile's source pixels and the list entry after it
     t += per;
     const int tile_nn = list_entry(t + per);
-    load_src(tile_next, ra, rb, ok_a, ok_b);
+    load_src(tile_next);
     __syncthreads();                                   // (1) the source block is in LDS
 
     // D. the staged tile, blended from the source block.  Thread u < 192 owns column pcol, channels 8 * sq .. and rows
@@ -394,8 +400,11 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
         v[i] = sum;
       }
       if constexpr (PRED) {
+        const unsigned t_on = mie_mask_take(pt.skip_mask, t_m, t_in);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
+          const bool on = (t_on >> i) & 1u;
+          const float4 sk = make_float4(on ? (float)t_skip[i][0] : 0.f, on ? (float)t_skip[i][1] : 0.f, on ? (float)t_skip[i][2] : 0.f, on ? (float)t_skip[i][3] : 0.f);
           const float4 r0 = e_r0[i];
           const float4 r1 = make_float4(r0.x + v[i].x, r0.y + v[i].y, r0.z + v[i].z, r0.w + v[i].w);
           if (e_ok[i]) mie_st4(a.res, e_off[i], r1);
@@ -405,7 +414,7 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
           const float y2_ = (float)(mie_bf16)(mie_act(ACT, a.slope, r1.z) - mie_act(ACT, a.slope, r0.z));
           const float y3_ = (float)(mie_bf16)(mie_act(ACT, a.slope, r1.w) - mie_act(ACT, a.slope, r0.w));
           float z = pw_y.x * y0_ + pw_y.y * y1_ + pw_y.z * y2_ + pw_y.w * y3_;
-          z += pw_s.x * t_skip[i].x + pw_s.y * t_skip[i].y + pw_s.z * t_skip[i].z + pw_s.w * t_skip[i].w;
+          z += pw_s.x * sk.x + pw_s.y * sk.y + pw_s.z * sk.z + pw_s.w * sk.w;
           if (!e_ok[i]) z = 0.f;
           // the eight lanes of a pixel, by data-parallel moves inside the wave's rows of 16 (no LDS round trip):
           // neighbours within quads, then the quad four lanes up -- complete in the lanes 0 and 8 of a row, the ones
@@ -414,9 +423,10 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
           z += dpp_f32<0x4E>(z);               // quad_perm [2,3,0,1]
           z += dpp_f32<0x104>(z);              // row_shl:4 (lane l reads lane l + 4)
           if (e_ok[i] && (tid & 7) == 0) {
-            const float p1 = t_p0[i] + z;
-            pt.res[t_pix[i]] = p1;
-            pt.out[t_pix[i]] = (mie_bf16)(mie_act(pt.act, pt.slope, p1) - mie_act(pt.act, pt.slope, t_p0[i]));
+            float r[2] = {t_p0[i] + z, t_p0[i]};
+            pt.res[t_pix[i]] = r[0];
+            mie_act_n(pt.act, pt.slope, r);
+            pt.out[t_pix[i]] = (mie_bf16)(r[0] - r[1]);
           }
         }
       } else {
@@ -632,9 +642,10 @@ __global__ __launch_bounds__(PTHR, 2) void k_upconv2x_pred(ConvArgsT<mie_bf16> a
   float z_p0 = 0.f;
   auto predict = [&]() {
     if (pred_live(z_act)) {
-      const float p1 = z_p0 + (s_z[par ^ 1][0][p_x & 1][p_r][p_x >> 1] + s_z[par ^ 1][1][p_x & 1][p_r][p_x >> 1]);
-      (pt.res + z_pix)[p_off] = p1;
-      (pt.out + z_pix)[p_off] = (mie_bf16)(mie_act(pt.act, pt.slope, p1) - mie_act(pt.act, pt.slope, z_p0));
+      float r[2] = {z_p0 + (s_z[par ^ 1][0][p_x & 1][p_r][p_x >> 1] + s_z[par ^ 1][1][p_x & 1][p_r][p_x >> 1]), z_p0};
+      (pt.res + z_pix)[p_off] = r[0];
+      mie_act_n(pt.act, pt.slope, r);
+      (pt.out + z_pix)[p_off] = (mie_bf16)(r[0] - r[1]);
     }
   };
   auto one_item = [&](int i, const Rows& rows, Rows& rows_next) {
