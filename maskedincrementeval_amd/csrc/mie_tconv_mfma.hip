@@ -333,7 +333,7 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
       const std::lock_guard<std::mutex> pair(mie_split_launches());
       hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, true, X3>), dim3(cap_p, cout / 32, parts), dim3(256), 0, st, a, pts);
       unsigned ny = (unsigned)((1024 + cap_out - 1) / cap_out);
-      if (ny > (unsigned)(cout / 4)) ny = (unsigned)(cout / 4);
+      if (ny > (unsigned)(cout / 16)) ny = (unsigned)(cout / 16);
       if (ny < 1) ny = 1;
       hipLaunchKernelGGL(k_conv_split_finish<T>, dim3(cap_out, ny), dim3(256), 0, st, a, parts);
       return true;
