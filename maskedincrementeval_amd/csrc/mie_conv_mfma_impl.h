@@ -328,6 +328,22 @@ __device__ void conv_quad_again(const ConvArgsT<T>& a, int n, int oy, int ox, in
   conv_store(a, off, co, s.x); conv_store(a, off + 1, co + 1, s.y); conv_store(a, off + 2, co + 2, s.z); conv_store(a, off + 3, co + 3, s.w);
 }
 
+// (tile, slab, part) of a workgroup of a split launch (x, y, z of the grid).  Such a launch is bound by the way of its filter
+// into the L2s: in launch order the tiles of a (slab, part) -- a filter slice -- lie on different XCDs (4 tiles, two slabs:
+// all 8), and each of them fetches the slice.  Here every tile of a slice is on one XCD, an eighth of the slices on each.
+// Grids whose slices do not divide by 8 keep the launch order.  Whole passes, launch order -> this: optical flow 1x256x256
+// 366.7 -> 361.7 us (transposed convs), 467.9 -> 459.5 (up-sampling), e2depth 1x128x128 246.4 -> 243.8, 1x64x96 181.1 ->
+// 180.6 (two tiles: a slice was on two XCDs).
+__device__ __forceinline__ void split_order(int& bx, int& by, int& bz) {
+  const int gx = (int)gridDim.x, gy = (int)gridDim.y, slices = gy * (int)gridDim.z;
+  if ((slices & 7) != 0) return;
+  const int id = (bz * gy + by) * gx + bx, at = id >> 3, q = at / gx;
+  const int c = (id & 7) * (slices >> 3) + q;
+  bx = at - q * gx;
+  bz = c / gy;
+  by = c - bz * gy;
+}
+
 // UP: the conv input is up2x(x + x2), the bilinear x2 up-sampling of the sum of two deltas given at
 // half resolution (x2 optional), and is never formed in memory: per chunk the 8x8 block of source
 // pixels a tile's 12x12 input window blends is summed into LDS (fp32), and the staged tile is expanded
@@ -406,11 +422,11 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // (a stale tile costs next to nothing); the shares depend on their numbers, read from the tile set
   // (one more dependent load at the start of a workgroup: measured, it costs nothing even on launches
   // of a few dozen workgroups), and idle positions of the capacity-sized grid fall off the end.
-  // (For the SPLIT launches the same idea, one filter slice per XCD, was measured: no gain.)
   const int entry_zero = conv_args_entry_zero(a);      // every line of the argument block, fetched in one batch
   MIE_STAMP(0);
   int bx = blockIdx.x + entry_zero, by = blockIdx.y;
-  const int bz = SPLIT ? (int)blockIdx.z : 0;
+  int bz = SPLIT ? (int)blockIdx.z : 0;
+  if constexpr (SPLIT) split_order(bx, by, bz);
   int n, y0, x0, tk;
   if (!SPLIT && a.xcd_fs > 0) {
     const int cap = a.ts.n * a.ts.tiles_y * a.ts.tiles_x;

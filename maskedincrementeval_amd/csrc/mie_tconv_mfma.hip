@@ -68,9 +68,10 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
   TL* const sbuf = reinterpret_cast<TL*>(smem);
 
   int n, y0, x0;                                             // block origin in INPUT coordinates
-  const int tk = mie_pick_tile(pts, blockIdx.x + conv_args_entry_zero(a), n, y0, x0);
+  int bx = blockIdx.x + conv_args_entry_zero(a), by = blockIdx.y, bz = SPLIT ? (int)blockIdx.z : 0;
+  if constexpr (SPLIT) split_order(bx, by, bz);
+  const int tk = mie_pick_tile(pts, bx, n, y0, x0);
   if (tk == 0) return;
-  const int by = blockIdx.y, bz = SPLIT ? (int)blockIdx.z : 0;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l32 = lane & 31, half = lane >> 5;
