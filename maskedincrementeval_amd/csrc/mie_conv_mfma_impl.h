@@ -328,7 +328,7 @@ __device__ void conv_quad_again(const ConvArgsT<T>& a, int n, int oy, int ox, in
   conv_store(a, off, co, s.x); conv_store(a, off + 1, co + 1, s.y); conv_store(a, off + 2, co + 2, s.z); conv_store(a, off + 3, co + 3, s.w);
 }
 
-// (tile, slab, part) of a workgroup of a split launch (x, y, z of the grid).  Such a launch is bound by the way of its filter
+// (tile, slab, part) of a workgroup of a split launch (x, y, z of the grid).  A few per cent of such a launch are its filter's way
 // into the L2s: in launch order the tiles of a (slab, part) -- a filter slice -- lie on different XCDs (4 tiles, two slabs:
 // all 8), and each of them fetches the slice.  Here every tile of a slice is on one XCD, an eighth of the slices on each.
 // Grids whose slices do not divide by 8 keep the launch order.  Whole passes, launch order -> this: optical flow 1x256x256
