@@ -1252,6 +1252,7 @@ __global__ __launch_bounds__(256) void k_conv_split_finish(ConvArgsT<T> a, int p
   const int c0 = (int)blockIdx.y * cb;
   const int cn = (cout - c0 < cb) ? cout - c0 : cb;
   const int qn = cn >> 2;                                             // groups of four adjacent channels
+  const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
   bool bad = false;
   for (int idx = threadIdx.x; idx < 64 * qn; idx += 256) {
     const int p = idx / qn, co = c0 + 4 * (idx - p * qn);
@@ -1263,9 +1264,11 @@ __global__ __launch_bounds__(256) void k_conv_split_finish(ConvArgsT<T> a, int p
       continue;
     }
     const long long offs[1] = {off};
-    const int cos[1] = {co};
+    const int cos[1] = {co}, at[1] = {(n * hout + oy) * wout + ox};
     const bool oks[1] = {true};
     float4 r0[1], add[1];
+    unsigned live_b[1];
+    mie_mask_ask(live_m, a.ws, at, live_b);
     conv_epilogue_load4<T, 1>(a, offs, oks, r0, add);
     const float4 accs[1] = {split_sum(a.ws + off, a.ws_plane, parts)};
     if constexpr (K != 0) {
@@ -1274,7 +1277,8 @@ __global__ __launch_bounds__(256) void k_conv_split_finish(ConvArgsT<T> a, int p
         continue;
       }
     }
-    conv_epilogue_store4<T, 1>(a, offs, cos, oks, accs, r0, add);
+    const bool live[1] = {mie_mask_take(live_m, live_b, 1u) != 0u};
+    conv_epilogue_store4<T, 1>(a, offs, cos, oks, accs, r0, add, live);
   }
   if constexpr (K != 0) {
     if (__builtin_expect(__ballot(bad) != 0ull, 0))

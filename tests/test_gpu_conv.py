@@ -898,3 +898,32 @@ def test_gates_conv_with_two_tiles_a_workgroup(n, h, w, c1, c2, hid, masks, prev
             got = got.float().cpu().double()
             assert (got - want).abs().max().item() <= tol + want.abs().max().item() * 2.0 ** -8
             assert not got[~live.expand_as(got)].any()
+
+
+# At a pixel of an active tile outside the output pixel mask every matrix-core conv writes a zero delta and leaves the reservoir
+# alone, also where it holds an infinity or a NaN: one launch, split launches with their finish, and the transposed conv's blocks
+# (which reach over their active tiles), both forms.
+@pytest.mark.parametrize("kind,cin,cout,k,s,n,h,w", [("conv", 64, 64, 3, 1, 2, 70, 90), ("conv", 256, 256, 3, 1, 1, 16, 19), ("conv", 128, 256, 5, 2, 1, 24, 28),
+                                                     ("conv", 128, 256, 5, 2, 4, 60, 80), ("tconv", 256, 64, 3, 2, 1, 16, 18)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_pixels_outside_the_mask_keep_their_reservoir(kind, cin, cout, k, s, n, h, w, dtype):
+    x, m = gaussian_delta(n, cin, h, w, 0.02, 0.5, seed=21)
+    filt = _filt(he_normal_conv_weight(cout, cin, k, 22))
+    ho, wo = (2 * h, 2 * w) if kind == "tconv" else ops.conv_out_size(h, w, k, s, k // 2)
+    ts, out, dm = TileMask(n, ho, wo, DEV), ops.new_nhwc(n, cout, ho, wo, DEV, dtype), m.to(DEV)
+    ops.build_mask_tiles(dm, None, n, h, w, _lib.FOOT_TCONV if kind == "tconv" else _lib.FOOT_CONV, k, s, k // 2, ts)
+    off = ~ts.pixmask.cpu().bool().expand(n, cout, ho, wo)
+    r0 = torch.randn(n, cout, ho, wo, generator=torch.Generator().manual_seed(23))
+    r0[off] = torch.tensor([float("inf"), float("-inf"), float("nan")])[torch.arange(int(off.sum())) % 3]
+    for act in (_lib.ACT_NONE, _lib.ACT_LEAKY_RELU):
+        res = _dev(r0).clone()
+        if kind == "tconv":
+            assert ops.tconv2x_takes(cin, 0, cout, k, s, k // 2, 1, filt, dtype)
+            blocks = TileMask(n, h, w, DEV)
+            ops.build_mask_tiles(ts, None, n, ho, wo, _lib.FOOT_CONV, 2, 2, 0, blocks)
+            ops.tconv2x_masked(_dev(x).to(dtype), dm, None, None, filt, k, ts, blocks, out, res, act, 0.1)
+        else:
+            ops.conv_masked(_dev(x).to(dtype), dm, None, None, filt, k, s, k // 2, ts, out, res, act, 0.1, _lib.PATH_MFMA)
+        got = out.float().cpu()
+        assert torch.isfinite(got).all() and torch.count_nonzero(got[off]) == 0 and torch.count_nonzero(got[~off]) > 0
+        assert torch.equal(res.cpu().contiguous().view(torch.int32)[off], r0.contiguous().view(torch.int32)[off])
