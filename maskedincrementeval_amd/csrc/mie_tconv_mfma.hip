@@ -15,7 +15,8 @@
 // Tile sets.  `a.ts` is the output tile set (8x8 output tiles, MIE_FOOT_TCONV); the workgroups walk `pts`,
 // the tile set of the 16x16 output blocks at input resolution (built from the output pixel mask with a 2x2
 // stride-2 OR): a block is live when any of its four output tiles is.  A live block writes all its 256
-// pixels (zeros where no input reaches), a stale block is zeroed, which covers every stale output tile.
+// pixels (zeros where no input reaches, their reservoirs left alone), a stale block is zeroed, which covers every stale
+// output tile.
 // On planes of very few blocks the chunks are split over gridDim.z workgroups that write partial sums to the
 // workspace, and k_conv_split_finish (walking the OUTPUT tile set) adds them and runs the epilogue.
 #include "mie_conv_mfma_impl.h"
@@ -267,6 +268,18 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
     // of a pixel (16-byte reads of the k-split partial sums, 16-byte reservoir accesses, 16- / 8-byte delta accesses)
     constexpr int QPP = CO_BLK / 4;
     constexpr int PER = 64 * QPP / 256;
+    // (the output pixel mask of these groups is asked for before, and taken when the sums and the reservoir are there)
+    const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
+    unsigned live_b[PER];
+    if constexpr (!SPLIT) {
+      int at[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int p = (tid + 256 * i) / QPP, iy = y0 + (p >> 3), ix = x0 + (p & 7);
+        at[i] = iy < a.h_in && ix < a.w_in ? (n * hout + 2 * iy + py) * wout + 2 * ix + px : 0;
+      }
+      mie_mask_ask(live_m, a.filt_mc, at, live_b);
+    }
     float* red = smem + wk * (64 * CO_BLK);
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
@@ -304,7 +317,11 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
     } else {
       float4 r0[PER], add[PER];
       conv_epilogue_load4<T, PER>(a, off, ok, r0, add);
-      conv_epilogue_store4<T, PER>(a, off, co, ok, v, r0, add);
+      const unsigned live_bits = mie_mask_take(live_m, live_b, ~0u);
+      bool live[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) live[i] = ((live_bits >> i) & 1u) != 0u;
+      conv_epilogue_store4<T, PER>(a, off, co, ok, v, r0, add, live);
     }
     __syncthreads();                   // the next phase overwrites the parked accumulators
   };

@@ -904,7 +904,7 @@ def test_gates_conv_with_two_tiles_a_workgroup(n, h, w, c1, c2, hid, masks, prev
 # alone, also where it holds an infinity or a NaN: one launch, split launches with their finish, and the transposed conv's blocks
 # (which reach over their active tiles), both forms.
 @pytest.mark.parametrize("kind,cin,cout,k,s,n,h,w", [("conv", 64, 64, 3, 1, 2, 70, 90), ("conv", 256, 256, 3, 1, 1, 16, 19), ("conv", 128, 256, 5, 2, 1, 24, 28),
-                                                     ("conv", 128, 256, 5, 2, 4, 60, 80), ("tconv", 256, 64, 3, 2, 1, 16, 18)])
+                                                     ("conv", 128, 256, 5, 2, 4, 60, 80), ("tconv", 256, 64, 3, 2, 1, 16, 18), ("tconv", 128, 32, 5, 2, 2, 50, 60)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_pixels_outside_the_mask_keep_their_reservoir(kind, cin, cout, k, s, n, h, w, dtype):
     x, m = gaussian_delta(n, cin, h, w, 0.02, 0.5, seed=21)
