@@ -90,7 +90,11 @@ __device__ __forceinline__ float dpp_f32(float v) {
 
 // epilogue of one group of four adjacent channels, its cases fixed at compile time
 template <bool RES, int ACT>
-__device__ __forceinline__ void epilogue4(const ConvArgsT<mie_bf16>& a, long long off, const float4& v, const float4& r0) {
+__device__ __forceinline__ void epilogue4(const ConvArgsT<mie_bf16>& a, long long off, const float4& v, const float4& r0, bool live) {
+  if (!live) {      // outside the output pixel mask: the reservoir stays as it is
+    mie_st4(a.out, off, make_float4(0.f, 0.f, 0.f, 0.f));
+    return;
+  }
   if (!RES) {
     mie_st4(a.out, off, v);
     return;
@@ -280,7 +284,7 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
     mie_bf16x4 t_skip[2];
     float t_p0[2];
     int t_at[2];
-    unsigned t_in = 0u, t_m[2];
+    unsigned t_in = 0u, t_m[2];  // mask bytes: of the second delta (PRED), of the output pixel mask otherwise
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int idx = tid + 256 * i;
@@ -291,14 +295,16 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
       e_off[i] = (long long)pix * COUT + col;
       e_r0[i] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (RES) e_r0[i] = *reinterpret_cast<const float4*>(a.res + e_off[i]);
+      t_at[i] = pix;
+      t_in |= (e_ok[i] ? 1u : 0u) << i;
       if (PRED) {
-        t_pix[i] = t_at[i] = pix;
-        t_in |= (e_ok[i] ? 1u : 0u) << i;
+        t_pix[i] = pix;
         t_skip[i] = *reinterpret_cast<const mie_bf16x4*>(pt.skip + e_off[i]);
         t_p0[i] = pt.res[pix];
       }
     }
-    if (PRED) mie_mask_ask(pt.skip_mask, dummy, t_at, t_m);
+    const uint8_t* const t_mask = PRED ? pt.skip_mask : a.ts.pixmask;
+    mie_mask_ask(t_mask, dummy, t_at, t_m);
 
     // C. the next tile's source pixels and the list entry after it
     t += per;
@@ -399,8 +405,8 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
         }
         v[i] = sum;
       }
+      const unsigned t_on = mie_mask_take(t_mask, t_m, t_in);
       if constexpr (PRED) {
-        const unsigned t_on = mie_mask_take(pt.skip_mask, t_m, t_in);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const bool on = (t_on >> i) & 1u;
@@ -432,7 +438,7 @@ __global__ __launch_bounds__(256, 2) void k_upconv64_persist(ConvArgsT<mie_bf16>
       } else {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          if (e_ok[i]) epilogue4<RES, ACT>(a, e_off[i], v[i], e_r0[i]);
+          if (e_ok[i]) epilogue4<RES, ACT>(a, e_off[i], v[i], e_r0[i], ((t_on >> i) & 1u) != 0u);
       }
     }
     // (the next tile's barriers (1) and (2) stand between these reads of s_red and its next writes, barrier (3) between
@@ -748,6 +754,8 @@ __global__ __launch_bounds__(PTHR, 2) void k_upconv2x_pred(ConvArgsT<mie_bf16> a
 // rate of a large product), 4x120x160 124 -> 99; in a masked 8x480x640 pass 281 -> 156 + 22.  An item takes 15500 cycles:
 // 8000 to 10500 for its 512 matrix instructions a SIMD of 16 cycles, 2000 to 4000 for the exchange and the reservoir's rows,
 // the rest at the two barriers.  The terms and their rounding are k_upconv2x's: against 64 bits the same 0.0020 from each.
+// Like there, a pixel of an active tile outside the output pixel mask gets a zero delta and keeps its reservoir (its sum is
+// zero, but an infinity or a NaN in the reservoir has no increment of zero).  The byte of each costs a pass 0 to 0.4 %.
 constexpr int DC = 128, DCO = 64;
 constexpr int DSC = PC + 3, DLS = DC + EPS, DQ4 = DC / EPS;
 constexpr int DPIX = SR * DSC;                     // 209 pixels of the window
@@ -876,6 +884,13 @@ __global__ __launch_bounds__(PTHR, 2) void k_upconv2x_rows(ConvArgsT<mie_bf16> a
     r0[r] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.res + item_pix(o) * DCO) + 4u * off);
   };
 
+  // The output pixel mask of the four rows, a byte a lane: of row cg, position pos.  (Outside it the delta is zero and the
+  // reservoir stays as it is; a ballot hands the bits round.)
+  auto load_live = [&](const Item& o) -> unsigned {
+    const unsigned p = (tile_bit(o.act) & inner(o, cg)) ? (4 * ks + cg) * row + 2 * pos + px : 0u;
+    return (a.ts.pixmask + item_pix(o))[p];
+  };
+
   // ---- before the first item: its window, the first slots of the second item's, the masks of the first three
   Item cur = item_at(0), nxt = item_at(1), after = item_at(2);
   float4 va[DRING], vb[DRING];
@@ -899,6 +914,8 @@ __global__ __launch_bounds__(PTHR, 2) void k_upconv2x_rows(ConvArgsT<mie_bf16> a
     asm volatile("" : "+v"(sid), "+v"(l_pix), "+v"(l_ch));
     // ---- sums
     v4f acc[PR];
+    unsigned live_b = 0u;
+    unsigned long long live = 0ull;      // bit 16 * row + position
 #pragma unroll
     for (int r = 0; r < PR; ++r) acc[r] = v4f{0.f, 0.f, 0.f, 0.f};
     {
@@ -914,6 +931,8 @@ __global__ __launch_bounds__(PTHR, 2) void k_upconv2x_rows(ConvArgsT<mie_bf16> a
         const int u = f / SR;                        // the next window's slot u; then slot u + 4, of it or of the one after it
         if (f % SR == 2 && u < DLD) store_slot(par ^ 1, u, va[u % DRING], vb[u % DRING]);
         if (f % SR == 6 && (u + DRING) % 8 < DLD) load_slot(u + DRING < 8 ? nxt : after, (u + DRING) % 8, va[u % DRING], vb[u % DRING]);
+        if (f == 0) live_b = load_live(cur);
+        if (f == 3 * SR) live = __ballot(live_b != 0u);      // (two scalars from here on: what the sums leave of the registers is the rows')
         if (RES && f % SR == 9 && u < PR / 2) load_row(cur, u);
         __builtin_amdgcn_sched_barrier(0);
         const int h = f / (4 * SR), j = u % 4, r = f % SR;
@@ -944,14 +963,14 @@ __global__ __launch_bounds__(PTHR, 2) void k_upconv2x_rows(ConvArgsT<mie_bf16> a
       const unsigned off = ((4 * ks + r) * row + l_pix) * DCO + l_ch;
       mie_bf16* out = reinterpret_cast<mie_bf16*>(reinterpret_cast<char*>(a.out + pix0 * DCO) + 2u * off);
       float4 d = make_float4(sum[r][0], sum[r][1], sum[r][2], sum[r][3]);
-      const bool in = inner(cur, r);
+      const bool in = inner(cur, r), keep = on & (((live >> (16 * r + pos)) & 1ull) != 0ull);
       if (RES) {
         const float4 q0 = r0[r], q1 = make_float4(q0.x + d.x, q0.y + d.y, q0.z + d.z, q0.w + d.w);
-        if (on & in) *reinterpret_cast<float4*>(reinterpret_cast<char*>(a.res + pix0 * DCO) + 4u * off) = q1;
+        if (keep & in) *reinterpret_cast<float4*>(reinterpret_cast<char*>(a.res + pix0 * DCO) + 4u * off) = q1;
         d = make_float4(mie_act(ACT, a.slope, q1.x) - mie_act(ACT, a.slope, q0.x), mie_act(ACT, a.slope, q1.y) - mie_act(ACT, a.slope, q0.y),
                         mie_act(ACT, a.slope, q1.z) - mie_act(ACT, a.slope, q0.z), mie_act(ACT, a.slope, q1.w) - mie_act(ACT, a.slope, q0.w));
       }
-      if (!on) d = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (!keep) d = make_float4(0.f, 0.f, 0.f, 0.f);
       if ((on | zero) & in) mie_st4(out, 0, d);
     }
     cur = nxt;

@@ -168,3 +168,37 @@ def test_decoder_conv_of_many_items(n, h, w):
     # border's positions (the step with an addend stays with the other form).  Planes whose last item is and is not
     # filled.
     test_decoder_conv_at_input_resolution(n, 128, 64, h, w, torch.bfloat16)
+
+
+@pytest.mark.parametrize("form", ["blocks", "list"])
+@pytest.mark.parametrize("n,c,cout,h,w,dtype", [(1, 128, 64, 9, 16, torch.bfloat16), (1, 128, 64, 150, 170, torch.bfloat16), (8, 128, 64, 35, 67, torch.bfloat16),
+                                                (1, 64, 32, 20, 24, torch.bfloat16), (1, 64, 32, 182, 183, torch.bfloat16), (1, 128, 64, 33, 20, torch.float32)])
+def test_pixels_outside_the_mask_keep_their_reservoir(n, c, cout, h, w, dtype, form):
+    # The contract of every matrix-core conv: at a pixel of an active tile that lies outside the output pixel mask the delta is
+    # zero and the reservoir is not touched -- also where it holds an infinity or a NaN, whose increment would be NaN.  Planes
+    # that the blocks, the persistent kernel of 128 -> 64 channels and the one of 64 -> 32 (list-driven, from 2048 tiles) take.
+    H, W = 2 * h, 2 * w
+    filt = ops.ConvFilter(he_normal_conv_weight(cout, c, 5, 9).permute(1, 2, 3, 0).contiguous().to(DEV))
+    ts_up, ts = TileMask(n, H, W, DEV), TileMask(n, H, W, DEV)
+    out = ops.new_nhwc(n, cout, H, W, DEV, dtype)
+    odd = torch.tensor([float("inf"), float("-inf"), float("nan")])
+    for step, act in enumerate((None, _lib.ACT_NONE, _lib.ACT_RELU, _lib.ACT_LEAKY_RELU)):
+        (a, ma), (b, mb) = (gaussian_delta(n, c, h, w, d, 0.5, seed=40 + 10 * k + step) for k, d in enumerate((0.02, 0.05)))
+        dma, dmb = ma.to(DEV), mb.to(DEV)
+        ops.build_mask_tiles(dma, dmb, n, h, w, _lib.FOOT_UP2X, 0, 0, 0, ts_up)
+        ops.build_mask_tiles(ts_up, None, n, H, W, _lib.FOOT_CONV, 5, 1, 2, ts)
+        off = ~ts.pixmask.cpu().bool().expand(n, cout, H, W)
+        r0 = gaussian_delta(n, cout, H, W, 1.0, 1.0, seed=3)[0]
+        r0[off] = odd[torch.arange(int(off.sum())) % 3]
+        res = None if act is None else _dev(r0).clone()
+        args = (_dev(a, dtype), dma, _dev(b, dtype), dmb, filt)
+        if form == "blocks":
+            ops.upconv2x_masked(*args, ts, out, res, act or _lib.ACT_NONE, 0.1)
+        else:
+            ops.upconv_masked(*args, 5, 2, ts, out, res, act or _lib.ACT_NONE, 0.1)
+        got = out.float().cpu()
+        assert torch.isfinite(got).all() and torch.count_nonzero(got[off]) == 0, "step %d: %d not finite" % (step, (~torch.isfinite(got)).sum())
+        assert torch.count_nonzero(got[~off]) > 0
+        if res is not None:
+            bits = lambda t: t.contiguous().view(torch.int32)
+            assert torch.equal(bits(res.cpu())[off], bits(r0)[off])
