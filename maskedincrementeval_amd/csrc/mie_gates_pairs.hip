@@ -10,6 +10,11 @@
 // 2x66x88 51.2 -> 45.6, at 2x50x70 32.0 -> 30.1.  Whole passes: 8x480x640 2487 -> 2451 us (20 % active), 1669 -> 1646 (1 %),
 // 2x200x280 293 -> 290.  The plain convs of 256 channels lose by it (8x60x80 65 -> 74 us: 640 workgroups are one round and a
 // quarter), so they keep one tile.
+// The second tile costs a workgroup half as long again as one alone takes, which pays where it saves a round of workgroups:
+// while the active tiles alone are at most one workgroup a CU, each has its own (a sparse step on a large plane; the sums are
+// in the same order either way).  64+64->256 at 240x320, two -> one: 13 tiles 13.1 -> 8.6 us, 81 tiles 16.1 -> 10.1;
+// 128+128->512 at 120x160, 57 tiles 21.7 -> 14.5; 256+256->1024 at 60x80, 26 tiles 32.1 -> 21.3.  Just above the line (274,
+// 280 workgroups of one tile) both forms take as long (16.1 and 15.7 us; 34.5 and 35.1).
 #include "mie_conv_mfma_impl.h"
 
 namespace {
@@ -17,71 +22,29 @@ namespace {
 typedef mie_bf16 T;
 constexpr int K = 3, EPS = 8, SUB = 16, IT = 10, CC = 64, Q4 = CC / EPS;
 constexpr int LS = CC + EPS, RP = row_pitch_dw(IT, LS / 2, 1) * 2, STAGE = IT * RP;      // elements: pixel, row, tile
-constexpr int NSLOT = 2 * IT * IT * Q4, NLD = (NSLOT + 255) / 256;                       // 1600, 7
 constexpr int NQ = CC / SUB, UPC = K * K * NQ;                                           // units of a chunk: 36
 constexpr int RING = 6, PD = RING - 1;
 constexpr int COLS = 128;
 static_assert(UPC % RING == 0, "a ring slot means the same registers in every chunk");
-static_assert(NSLOT / 2 % Q4 == 0 && 256 % Q4 == 0, "a thread's channels are the same in all of its slots");
+static_assert(256 % Q4 == 0, "a thread's channels are the same in all of its slots");
+constexpr int ONE_MOST = 256;                                                            // workgroups of one tile, at most
 constexpr int SMEM = (2 * STAGE * 2 > 64 * COLS * 4 ? 2 * STAGE * 2 : 64 * COLS * 4) / 4;
 
-__global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
-  __shared__ __attribute__((aligned(16))) float smem[SMEM];
-  T* const sbuf = reinterpret_cast<T*>(smem);
-  const int bx = blockIdx.x + conv_args_entry_zero(a);
-  // ---- which pair of list positions and which slab: the order of k_conv_mfma with pairs for tiles -------------------------
-  const int cap = a.ts.n * a.ts.tiles_y * a.ts.tiles_x;
-  const int n_act = a.ts.counts[MIE_CNT_ACTIVE], n_st = a.ts.counts[MIE_CNT_STALE];
-  if (n_act < 0 || n_st < 0 || n_act > cap || n_st > cap) return;
-  const int ns = (int)gridDim.y, p_act = (n_act + 1) >> 1, p_st = (n_st + 1) >> 1;
-  const int w_act = p_act * ns, w_st = p_st * ns;
-  const int c_act = (w_act + 7) >> 3, c_st = (w_st + 7) >> 3;
-  const int xcd = bx & 7, slot = (int)blockIdx.y * ((int)gridDim.x >> 3) + (bx >> 3);
-  const int spg = ns / a.xcd_fs;
-  const bool active = slot < c_act;
-  const int v = active ? xcd * c_act + slot : xcd * c_st + (slot - c_act);
-  if (v >= (active ? w_act : w_st) || (!active && slot - c_act >= c_st)) return;
-  const int per_group = (active ? p_act : p_st) * spg;
-  const int sg = v / per_group, r0 = v - sg * per_group, pair = r0 / spg;
-  const int co0 = (sg * spg + (r0 - pair * spg)) * COLS;
-  const int count = active ? n_act : n_st, at = 2 * pair;
-  const int32_t* const list = active ? a.ts.tiles : a.ts.stale;
-  const int tiles[2] = {list[at], list[at + 1 < count ? at + 1 : at]};
-  const bool second = at + 1 < count;
-  int n[2], y0[2], x0[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (tiles[t] < 0 || tiles[t] >= cap) return;      // corrupt list entry: skip rather than touch memory
-    const int ty = tiles[t] / a.ts.tiles_x;
-    x0[t] = (tiles[t] - ty * a.ts.tiles_x) * MIE_TILE;
-    n[t] = ty / a.ts.tiles_y;
-    y0[t] = (ty - n[t] * a.ts.tiles_y) * MIE_TILE;
-  }
+// The workgroup's NT tiles (the second of two may be none: `second`).
+template <int NT>
+__device__ __forceinline__ void gates_tiles(const ConvArgsT<T>& a, T* const sbuf, float* const smem, const int (&n)[2], const int (&y0)[2], const int (&x0)[2],
+                                            const bool second, const int co0) {
+  constexpr int NSLOT = NT * IT * IT * Q4, NLD = (NSLOT + 255) / 256;                    // 800 or 1600, 4 or 7
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, half = lane >> 5;
   const int hout = a.ts.h, wout = a.ts.w, cout = a.cout;
 
-  if (!active) {
-    auto zero = [&](int n, int y0, int x0) {
-      for (int idx = tid; idx < 64 * (COLS / 16); idx += 256) {
-        const int p = idx >> 3, g4 = idx & 7, oy = y0 + (p >> 3), ox = x0 + (p & 7);
-        if (oy >= hout || ox >= wout) continue;
-        const long long o = (((long long)n * hout + oy) * wout + ox) * a.hid + co0 / 4 + 4 * g4;
-        mie_st4(a.g_dh, o, make_float4(0.f, 0.f, 0.f, 0.f));
-        mie_st4(a.g_dc, o, make_float4(0.f, 0.f, 0.f, 0.f));
-      }
-    };
-    zero(n[0], y0[0], x0[0]);
-    if (second) zero(n[1], y0[1], x0[1]);
-    return;
-  }
-
   // which of this thread's outputs lie on a pixel of the mask: bit 8 * t + i, item i of tile t
   constexpr int PER = 2;
-  int live_at[2 * PER];
+  int live_at[NT * PER];
   unsigned live_in = 0u;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int p = (tid + 256 * i) >> 3;
@@ -97,11 +60,11 @@ __global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
   unsigned inb = 0u, ok1 = 0u, ok2 = 0u;
 #pragma unroll
   for (int i = 0; i < NLD; ++i) {
-    const int s = (tid + 256 * i) >> 3, t = s >= IT * IT ? 1 : 0, pix = s - t * (IT * IT);
+    const int s = (tid + 256 * i) >> 3, t = NT == 2 && s >= IT * IT ? 1 : 0, pix = s - t * (IT * IT);
     const int row = pix / IT, col = pix - row * IT;
     st_lds[i] = t * STAGE + row * RP + col * LS + q8;
     const int iy = (t ? y0[1] : y0[0]) - a.pad + row, ix = (t ? x0[1] : x0[0]) - a.pad + col;
-    const bool in = s < 2 * IT * IT && iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in && (t == 0 || second);
+    const bool in = s < NT * IT * IT && iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in && (t == 0 || second);
     st_po[i] = in ? ((t ? n[1] : n[0]) * a.h_in + iy) * a.w_in + ix : 0;
     inb |= (in ? 1u : 0u) << i;
   }
@@ -128,15 +91,15 @@ __global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
   unsigned unit_b = (unsigned)cout * (2 * 2 * EPS);          // bytes of one
   auto load_b = [&](const char* ub, int u) { return *reinterpret_cast<const float4*>(ub + u * unit_b + b_lane); };
   const T* const a0 = sbuf + ((l32 >> 3) * RP + (l32 & 7) * LS + EPS * half);
-  auto load_a = [&](int u, float4 (&x)[4]) {
+  auto load_a = [&](int u, float4 (&x)[2 * NT]) {
     const int tap = u % (K * K), q = u / (K * K);
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
+    for (int mb = 0; mb < 2 * NT; ++mb)
       x[mb] = *reinterpret_cast<const float4*>(a0 + (mb >> 1) * STAGE + (4 * (mb & 1) + tap / K) * RP + tap % K * LS + SUB * q);
   };
-  v16f acc[4];
+  v16f acc[2 * NT];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+  for (int mb = 0; mb < 2 * NT; ++mb)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[mb][r] = 0.f;
 
@@ -166,7 +129,7 @@ __global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
 #pragma unroll
   for (int u = 0; u < PD; ++u) ring[u] = load_b(ub, u);
   const uint8_t* const cp_m = a.g_cpd != nullptr ? a.g_cpm : nullptr;
-  unsigned live_b[2 * PER], cp_b[2 * PER];
+  unsigned live_b[NT * PER], cp_b[NT * PER];
   mie_mask_ask(a.ts.pixmask, a.filt_mc, live_at, live_b);
   mie_mask_ask(cp_m, a.filt_mc, live_at, cp_b);
   mie_mask_asked();
@@ -190,7 +153,7 @@ __global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
   // one chunk; with the next one's slots, or (LAST) the first tile's reservoirs, asked for between its first units
   auto chunk = [&](const char* ub_next, const T* xin, unsigned cs, unsigned ci, auto LAST) {
     constexpr bool last = decltype(LAST)::value;
-    float4 av[2][4];
+    float4 av[2][2 * NT];
     load_a(0, av[0]);
 #pragma unroll
     for (int u = 0; u < UPC; ++u) {
@@ -202,7 +165,7 @@ __global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
       if (u + 1 < UPC) load_a(u + 1, av[(u + 1) & 1]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) mma_unit(acc[mb], av[u & 1][mb], ring[u % RING], T());
+      for (int mb = 0; mb < 2 * NT; ++mb) mma_unit(acc[mb], av[u & 1][mb], ring[u % RING], T());
       __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
@@ -237,15 +200,70 @@ __global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
       long long ho, go;
       item_at(t, i, ho, go);
       GateItem g = item[i];
-      if (t == 0) item_load(1, i);      // (this item's registers are free)
+      if constexpr (NT == 2 && t == 0) item_load(1, i);      // (this item's registers are free)
       if ((live_in >> (t * PER + i)) & 1u)
         conv_gates_item<T>(a, (live >> (t * PER + i)) & 1u, (cp_live >> (t * PER + i)) & 1u, ho, go, dg[i], g);
     }
   };
   epilogue(std::integral_constant<int, 0>{});
-  if (!second) return;
-  __syncthreads();
-  epilogue(std::integral_constant<int, 1>{});
+  if constexpr (NT == 2) {
+    if (!second) return;
+    __syncthreads();
+    epilogue(std::integral_constant<int, 1>{});
+  }
+}
+
+__global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
+  __shared__ __attribute__((aligned(16))) float smem[SMEM];
+  T* const sbuf = reinterpret_cast<T*>(smem);
+  const int bx = blockIdx.x + conv_args_entry_zero(a);
+  // ---- which pair of list positions and which slab: the order of k_conv_mfma with pairs for tiles -------------------------
+  const int cap = a.ts.n * a.ts.tiles_y * a.ts.tiles_x;
+  const int n_act = a.ts.counts[MIE_CNT_ACTIVE], n_st = a.ts.counts[MIE_CNT_STALE];
+  if (n_act < 0 || n_st < 0 || n_act > cap || n_st > cap) return;
+  // few active tiles: one a workgroup (the launcher's grid has room for them)
+  const int ns = (int)gridDim.y;
+  const bool one = n_act * ns <= ONE_MOST;
+  const int p_act = one ? n_act : (n_act + 1) >> 1, p_st = (n_st + 1) >> 1;
+  const int w_act = p_act * ns, w_st = p_st * ns;
+  const int c_act = (w_act + 7) >> 3, c_st = (w_st + 7) >> 3;
+  const int xcd = bx & 7, slot = (int)blockIdx.y * ((int)gridDim.x >> 3) + (bx >> 3);
+  const int spg = ns / a.xcd_fs;
+  const bool active = slot < c_act;
+  const int v = active ? xcd * c_act + slot : xcd * c_st + (slot - c_act);
+  if (v >= (active ? w_act : w_st) || (!active && slot - c_act >= c_st)) return;
+  const int per_group = (active ? p_act : p_st) * spg;
+  const int sg = v / per_group, r0 = v - sg * per_group, pair = r0 / spg;
+  const int co0 = (sg * spg + (r0 - pair * spg)) * COLS;
+  const int count = active ? n_act : n_st, at = one && active ? pair : 2 * pair;
+  const int32_t* const list = active ? a.ts.tiles : a.ts.stale;
+  const int tiles[2] = {list[at], list[at + 1 < count ? at + 1 : at]};
+  const bool second = at + 1 < count && !(one && active);
+  int n[2], y0[2], x0[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (tiles[t] < 0 || tiles[t] >= cap) return;      // corrupt list entry: skip rather than touch memory
+    const int ty = tiles[t] / a.ts.tiles_x;
+    x0[t] = (tiles[t] - ty * a.ts.tiles_x) * MIE_TILE;
+    n[t] = ty / a.ts.tiles_y;
+    y0[t] = (ty - n[t] * a.ts.tiles_y) * MIE_TILE;
+  }
+  if (!active) {
+    auto zero = [&](int n, int y0, int x0) {
+      for (int idx = threadIdx.x; idx < 64 * (COLS / 16); idx += 256) {
+        const int p = idx >> 3, g4 = idx & 7, oy = y0 + (p >> 3), ox = x0 + (p & 7);
+        if (oy >= a.ts.h || ox >= a.ts.w) continue;
+        const long long o = (((long long)n * a.ts.h + oy) * a.ts.w + ox) * a.hid + co0 / 4 + 4 * g4;
+        mie_st4(a.g_dh, o, make_float4(0.f, 0.f, 0.f, 0.f));
+        mie_st4(a.g_dc, o, make_float4(0.f, 0.f, 0.f, 0.f));
+      }
+    };
+    zero(n[0], y0[0], x0[0]);
+    if (second) zero(n[1], y0[1], x0[1]);
+    return;
+  }
+  if (one) gates_tiles<1>(a, sbuf, smem, n, y0, x0, false, co0);
+  else gates_tiles<2>(a, sbuf, smem, n, y0, x0, second, co0);
 }
 
 }  // namespace
@@ -259,7 +277,8 @@ bool mie_launch_gates_pairs(const ConvArgsT<mie_bf16>& a0, unsigned cap, hipStre
   if ((long long)a.ts.n * a.h_in * a.w_in * (a.c1 > a.c2 ? a.c1 : a.c2) >= 1LL << 31) return false;      // 32-bit offsets
   const unsigned pairs = cap / 2 + 1;
   if (least == 0 || (long long)pairs * (a.cout / COLS) < least) return false;
-  const unsigned gx = xcd_plan(a, pairs, a.cout / COLS, K);
+  // (of at most ONE_MOST workgroups of one tile half are more than the pairs have)
+  const unsigned gx = xcd_plan(a, pairs + ONE_MOST / 2 / (a.cout / COLS) + 1, a.cout / COLS, K);
   if (a.xcd_fs == 0) return false;
   hipLaunchKernelGGL(k_gates_pairs, dim3(gx, a.cout / COLS), dim3(256), 0, st, a);
   return true;

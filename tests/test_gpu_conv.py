@@ -927,3 +927,41 @@ def test_pixels_outside_the_mask_keep_their_reservoir(kind, cin, cout, k, s, n, 
         got = out.float().cpu()
         assert torch.isfinite(got).all() and torch.count_nonzero(got[off]) == 0 and torch.count_nonzero(got[~off]) > 0
         assert torch.equal(res.cpu().contiguous().view(torch.int32)[off], r0.contiguous().view(torch.int32)[off])
+
+
+# The same kernel where few tiles are active: up to 256 workgroups of one tile each, pairs from there on, with the stale tiles
+# of the step before behind them.  Counts at both sides of the line (two slabs of 128 columns: 128 tiles) and planes whose grid
+# just holds them; reservoirs of zero, so that a step is sigmoid(in) * tanh(cell) and sigmoid(out) * tanh of that.
+@pytest.mark.parametrize("h,w,c2,hid", [(128, 128, 64, 64), (61, 250, 0, 64), (64, 64, 256, 256)])
+def test_gates_conv_of_few_active_tiles(h, w, c2, hid):
+    bf, c1, cols = torch.bfloat16, 64, 4 * hid
+    wt = (he_normal_conv_weight(cols, c1 + c2, 3, 31) * 0.5).to(bf).float()
+    filt, ts = _filt(wt), TileMask(1, h, w, DEV)
+    ns = cols // 128
+    assert 256 <= (ts.capacity // 2 + 1) * ns <= 270
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(1, c1, h, w, generator=g).to(bf).float()
+    x2 = torch.randn(1, c2, h, w, generator=g).to(bf).float() if c2 else None
+    dh, dc = (ops.new_nhwc(1, hid, h, w, DEV, bf) for _ in range(2))
+    order = torch.randperm(ts.capacity, generator=g)
+    tx = (w + 7) // 8
+    for step, count in enumerate((1, 256 // ns, 256 // ns + 1, 3, ts.capacity, 0, 256 // ns - 1)):
+        tiles = order[:count] if step % 2 else order[ts.capacity - count:]
+        m = torch.zeros(1, 1, h, w, dtype=torch.uint8)
+        m[0, 0, (tiles // tx * 8 + 1).clamp(max=h - 2), (tiles % tx * 8 + 1).clamp(max=w - 1)] = 1      # a pixel whose 3x3 stays in its tile
+        dm = m.to(DEV)
+        ops.build_mask_tiles(dm, None, 1, h, w, _lib.FOOT_CONV, 3, 1, 1, ts)
+        res = [ops.new_nhwc(1, c, h, w, DEV).zero_() for c in (cols, hid, hid)]
+        both = (x if x2 is None else torch.cat([x, x2], 1)) * m.float()
+        ops.conv_gates_incr(_dev(x).to(bf), dm, None if x2 is None else _dev(x2).to(bf), None if x2 is None else dm, filt, ts, res[0], None, None, res[1], res[2], dh, dc)
+        d = F.conv2d(both.double(), wt.double(), padding=1)
+        bound = F.conv2d(both.abs().double(), wt.abs().double(), padding=1).amax().item() * 9 * (c1 + c2) * 2.0 ** -24 + 8 * 2.0 ** -24
+        q = d.view(1, hid, 4, h, w)
+        want_c = torch.sigmoid(q[:, :, 0]) * torch.tanh(q[:, :, 3])
+        want_h = torch.sigmoid(q[:, :, 2]) * torch.tanh(want_c)
+        assert int(ts.counts[0]) == count
+        assert (res[0].cpu().double() - d).abs().max().item() <= bound
+        for got, want in ((dh, want_h), (dc, want_c)):
+            got = got.float().cpu().double()
+            assert (got - want).abs().max().item() <= 4 * bound + want.abs().max().item() * 2.0 ** -8, (count, step)
+            assert not got[(m == 0).expand_as(got) & (torch.nn.functional.max_pool2d(m.float(), 3, 1, 1) == 0).expand_as(got)].any()
