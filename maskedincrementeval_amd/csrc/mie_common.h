@@ -186,14 +186,18 @@ __device__ __forceinline__ float mie_act(int kind, float slope, float v) {
 // and those two are one loop over the values, which move up a place each time round (19 KB).  Measured over whole passes:
 // fp32 1x64x96 201 -> 196 us, 1x264x352 461 -> 449; bf16 2x200x280 320 -> 314, 8x480x640 2740 -> 2590.
 template <int N>
+__device__ __forceinline__ void mie_act_select(int kind, float slope, float (&v)[N]) {      // none, ReLU, leaky ReLU
+  const bool none = kind == MIE_ACT_NONE, leaky = kind == MIE_ACT_LEAKY_RELU;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float low = none ? v[i] : leaky ? __fmul_rn(v[i], slope) : 0.f;
+    v[i] = v[i] > 0.f ? v[i] : low;
+  }
+}
+template <int N>
 __device__ __forceinline__ void mie_act_n(int kind, float slope, float (&v)[N]) {
   if (__builtin_expect(kind <= MIE_ACT_LEAKY_RELU, 1)) {
-    const bool none = kind == MIE_ACT_NONE, leaky = kind == MIE_ACT_LEAKY_RELU;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const float low = none ? v[i] : leaky ? __fmul_rn(v[i], slope) : 0.f;
-      v[i] = v[i] > 0.f ? v[i] : low;
-    }
+    mie_act_select(kind, slope, v);
     return;
   }
 #pragma unroll 1
