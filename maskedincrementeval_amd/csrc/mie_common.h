@@ -180,11 +180,6 @@ __device__ __forceinline__ float mie_act(int kind, float slope, float v) {
   }
 }
 
-// mie_act of N values, for a kind that is not known at compile time.  Inlined once per value, the two transcendental
-// kinds made 55 of the 70 KB of a kernel with 64 values a thread, and a workgroup that took neither still had to fetch the
-// lines it jumped between; the instruction cache holds 64 KB for two CUs, and starts cold.  So the other kinds are selects,
-// and those two are one loop over the values, which move up a place each time round (19 KB).  Measured over whole passes:
-// fp32 1x64x96 201 -> 196 us, 1x264x352 461 -> 449; bf16 2x200x280 320 -> 314, 8x480x640 2740 -> 2590.
 template <int N>
 __device__ __forceinline__ void mie_act_select(int kind, float slope, float (&v)[N]) {      // none, ReLU, leaky ReLU
   const bool none = kind == MIE_ACT_NONE, leaky = kind == MIE_ACT_LEAKY_RELU;
@@ -194,6 +189,12 @@ __device__ __forceinline__ void mie_act_select(int kind, float slope, float (&v)
     v[i] = v[i] > 0.f ? v[i] : low;
   }
 }
+
+// mie_act of N values, for a kind that is not known at compile time.  Inlined once per value, the two transcendental
+// kinds made 55 of the 70 KB of a kernel with 64 values a thread, and a workgroup that took neither still had to fetch the
+// lines it jumped between; the instruction cache holds 64 KB for two CUs, and starts cold.  So the other kinds are selects,
+// and those two are one loop over the values, which move up a place each time round (19 KB).  Measured over whole passes:
+// fp32 1x64x96 201 -> 196 us, 1x264x352 461 -> 449; bf16 2x200x280 320 -> 314, 8x480x640 2740 -> 2590.
 template <int N>
 __device__ __forceinline__ void mie_act_n(int kind, float slope, float (&v)[N]) {
   if (__builtin_expect(kind <= MIE_ACT_LEAKY_RELU, 1)) {

@@ -4,8 +4,8 @@
 // and on the VALU path they run at a tenth of the vector peak.  Here the whole problem of a workgroup
 // fits LDS at once:
 //   * one 256-thread workgroup = one active 8x8 output tile x 32 output channels;
-//   * the input tile plus halo is staged in fp32, channels padded to 8 (pixel stride 9 floats), inactive
-//     pixels zero-filled without being read; bf16 deltas are widened while staging, so one kernel body
+//   * the input tile plus halo is staged in fp32, channels padded to 8 (pixel stride 9 floats), zeros for inactive
+//     pixels (what is fetched of them is dropped); bf16 deltas are widened while staging, so one kernel body
 //     (v_mfma_f32_32x32x2_f32) serves both element types -- products of bf16 values are exact in fp32;
 //   * the filter slab [tap][8 channels][32 columns] is staged from the plain fp32 filter, zero rows for
 //     the padding channels;
@@ -14,8 +14,8 @@
 //     LDS and are added in a fixed order; epilogue as everywhere (addend, reservoir, activation, refresh).
 // One input only (x2 unsupported), stride 1 or 2, K = 3 or 5, Cout % 32 == 0.
 // UP: the input is up2x(x), the bilinear x2 up-sampling of a delta given at half resolution (a.h_in / a.w_in are
-// the up-sampled size): every staged pixel is blended from its four source pixels while staging, the up-sampled
-// tensor is never formed (the 2-channel flow estimate in front of an EVFlowNet decoder).  Stride 1 only.
+// the up-sampled size): the source pixels are staged first and every staged pixel is blended from four of them, the
+// up-sampled tensor is never formed (the 2-channel flow estimate in front of an EVFlowNet decoder).  Stride 1 only.
 #include "mie_conv.h"
 
 namespace {
@@ -25,15 +25,27 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int FC_CH = 8;     // staged channels per pixel
 constexpr int FC_PS = 9;     // LDS floats per staged pixel (odd: the 32 pixels of a block fall on distinct banks)
 
+// Waves a SIMD: as many workgroups a CU as the LDS has room for (3x3 at stride 2: as many as without spills).  Without a bound the
+// compiler gives the accumulators registers of their own and a CU holds one to four fewer: 8x480x640, every pixel active, 4->64
+// 3x3 stride 2 139 -> 128 us, 5->32 5x5 stride 2 125 -> 115, 4->32 3x3 205 -> 189.
+constexpr int fc_waves(int k, int s, bool up) { return k == 3 ? (s == 2 ? 5 : 8) : s == 2 ? 4 : up ? 5 : 1; }
+
 template <typename T, int K, int S, bool UP = false>
-__global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
+__global__ __launch_bounds__(256, fc_waves(K, S, UP)) void k_conv_fewcin(ConvArgsT<T> a) {
   static_assert(!UP || S == 1, "the up-sampling form is stride 1");
   constexpr int IT = 7 * S + K;                  // input tile edge incl. halo
   constexpr int NPIX = IT * IT;
   constexpr int IN_F = NPIX * FC_PS;
   constexpr int W_F = K * K * FC_CH * 32;
   constexpr int RED_F = 2 * 64 * 32;             // the accumulators of the two tap halves, parked for the epilogue
+  constexpr int NIN = (NPIX * FC_CH + 255) / 256;
+  constexpr int LO = UP ? (K == 5 ? 8 : 6) : IT; // edge of what is loaded: source pixels, or the staged ones themselves
+  constexpr int NLD = (LO * LO * FC_CH + 255) / 256;
   constexpr int SMEM_F = (IN_F + W_F > RED_F) ? IN_F + W_F : RED_F;      // (they reuse the staging area)
+  // the source pixels lie behind the filter, or (5x5, five workgroups a CU) where its last taps go afterwards
+  constexpr int LATE = UP && IN_F + W_F + LO * LO * FC_PS > SMEM_F ? 3 : 0;
+  constexpr int LO_AT = IN_F + W_F - LATE * FC_CH * 32;
+  static_assert(!UP || LO_AT + LO * LO * FC_PS <= SMEM_F, "room for the source pixels");
   __shared__ float smem[SMEM_F];
   float* const s_in = smem;
   float* const s_w = smem + IN_F;
@@ -74,8 +86,7 @@ __global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
   // Every global load of the thread is issued before the first LDS store (compile-time trip counts, fully
   // unrolled): one memory round trip for the whole staging instead of one per loop iteration.
   const int iy0 = y0 * S - a.pad, ix0 = x0 * S - a.pad;
-  constexpr int NIN = (NPIX * FC_CH + 255) / 256;
-  float vin[NIN], vw[K * K];
+  float vw[K * K];
   {
     const int col = tid & 31, ch = (tid >> 5) & 7;           // filter: thread = (channel, column), one load per tap
     const float* wp = a.filt + (long long)ch * (K * K) * cout + co0 + col;
@@ -83,37 +94,26 @@ __global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
     for (int tap = 0; tap < K * K; ++tap) vw[tap] = (ch < cin) ? wp[(long long)tap * cout] : 0.f;
   }
   // (the values of masked pixels too, which the mask bytes, loaded beside them, drop)
-  constexpr int TAPS = UP ? 4 : 1;                 // source pixels of a staged one
+  // UP: what is loaded are the LO x LO source pixels under the staged tile; the staged pixels are blended from LDS.  (Four loads
+  // and four mask bytes for each staged pixel took 156 registers and two workgroups a CU instead of five: 2->32 5x5, every pixel
+  // active, 1x256x256 21.1 us, this way 13.9; 8x240x320 159 -> 76; 2->256 at 1x32x32 9.4 -> 8.6.)
   const int ch = tid & 7, h_src = UP ? a.h_in >> 1 : a.h_in, w_src = UP ? a.w_in >> 1 : a.w_in;
-  int src[NIN * TAPS];
+  const int sy0 = UP ? ((iy0 + 1) >> 1) - 1 : iy0, sx0 = UP ? ((ix0 + 1) >> 1) - 1 : ix0;
+  int src[NLD];
   unsigned in = 0u;
-  float lw[UP ? NIN * TAPS : 1];
 #pragma unroll
-  for (int i = 0; i < NIN; ++i) {
+  for (int i = 0; i < NLD; ++i) {
     const int pix = (tid + 256 * i) >> 3;
-    const int iy = iy0 + pix / IT, ix = ix0 + pix % IT;
-    const bool k = pix < NPIX && ch < cin && iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in;
-    if constexpr (UP) {
-      int r[2], q[2];
-      float lr[2], lq[2];
-      conv_up2x_coef(k ? iy : 0, h_src, r[0], r[1], lr[0], lr[1]);
-      conv_up2x_coef(k ? ix : 0, w_src, q[0], q[1], lq[0], lq[1]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        src[4 * i + j] = k ? (n * h_src + r[j >> 1]) * w_src + q[j & 1] : 0;
-        lw[4 * i + j] = lr[j >> 1] * lq[j & 1];
-        in |= (k ? 1u : 0u) << (4 * i + j);
-      }
-    } else {
-      src[i] = k ? (n * h_src + iy) * w_src + ix : 0;
-      in |= (k ? 1u : 0u) << i;
-    }
+    const int sy = sy0 + pix / LO, sx = sx0 + pix % LO;
+    const bool k = pix < LO * LO && ch < cin && sy >= 0 && sy < h_src && sx >= 0 && sx < w_src;
+    src[i] = k ? (n * h_src + sy) * w_src + sx : 0;
+    in |= (k ? 1u : 0u) << i;
   }
-  static_assert(NIN * TAPS <= 32, "a bit for each");
-  float raw[NIN * TAPS];
+  static_assert(NLD <= 32, "a bit for each");
+  float vin[NLD];
 #pragma unroll
-  for (int i = 0; i < NIN * TAPS; ++i) raw[i] = mie_ld(a.x, (long long)src[i] * cin + (ch < cin ? ch : 0));
-  unsigned b[NIN * TAPS];
+  for (int i = 0; i < NLD; ++i) vin[i] = mie_ld(a.x, (long long)src[i] * cin + (ch < cin ? ch : 0));
+  unsigned b[NLD];
   mie_mask_ask(a.xm, a.filt, src, b);
   mie_mask_asked();
   const unsigned on = mie_mask_take(a.xm, b, in), live_bits = mie_mask_take(live_m, live_b, live_in);
@@ -133,24 +133,39 @@ __global__ __launch_bounds__(256) void k_conv_fewcin(ConvArgsT<T> a) {
     co[i] = co0 + col;
   }
   conv_epilogue_load4<T, 2>(a, off, live, r0, add);
+  float* const s_src = UP ? smem + LO_AT : s_in;
 #pragma unroll
-  for (int i = 0; i < NIN; ++i) {
-    float v = 0.f;
+  for (int tap = 0; tap < K * K - LATE; ++tap) s_w[tap * 256 + tid] = vw[tap];
 #pragma unroll
-    for (int j = 0; j < TAPS; ++j) {
-      const float x = ((on >> (TAPS * i + j)) & 1u) ? raw[TAPS * i + j] : 0.f;
-      v = UP ? v + lw[UP ? TAPS * i + j : 0] * x : x;
-    }
-    vin[i] = v;
-  }
-#pragma unroll
-  for (int tap = 0; tap < K * K; ++tap) s_w[tap * 256 + tid] = vw[tap];
-#pragma unroll
-  for (int i = 0; i < NIN; ++i) {
+  for (int i = 0; i < NLD; ++i) {
     const int idx = tid + 256 * i;
-    if ((idx >> 3) < NPIX) s_in[(idx >> 3) * FC_PS + (idx & 7)] = vin[i];
+    if ((idx >> 3) < LO * LO) s_src[(idx >> 3) * FC_PS + (idx & 7)] = ((on >> i) & 1u) ? vin[i] : 0.f;
   }
   __syncthreads();
+  if constexpr (UP) {
+#pragma unroll
+    for (int i = 0; i < NIN; ++i) {
+      const int pix = (tid + 256 * i) >> 3;
+      const int iy = iy0 + pix / IT, ix = ix0 + pix % IT;
+      float v = 0.f;
+      if (iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in) {
+        int r[2], q[2];
+        float lr[2], lq[2];
+        conv_up2x_coef(iy, h_src, r[0], r[1], lr[0], lr[1]);
+        conv_up2x_coef(ix, w_src, q[0], q[1], lq[0], lq[1]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (pix < NPIX) v += lr[j >> 1] * lq[j & 1] * s_src[((r[j >> 1] - sy0) * LO + (q[j & 1] - sx0)) * FC_PS + ch];
+      }
+      if (pix < NPIX) s_in[pix * FC_PS + ch] = v;
+    }
+    __syncthreads();
+    if (LATE > 0) {
+#pragma unroll
+      for (int tap = K * K - LATE; tap < K * K; ++tap) s_w[tap * 256 + tid] = vw[tap];
+      __syncthreads();
+    }
+  }
 
   // ---- contraction ---------------------------------------------------------------------------------
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;

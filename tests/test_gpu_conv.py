@@ -504,6 +504,14 @@ def test_upsampled_conv_few_channels(c, cout, k, h, w, dtype):
         assert torch.allclose(got, ref, **tol(ref)), "step %d max|diff| = %.3e" % (step, (got - ref).abs().max())
 
 
+# Planes below, at and just above the block of source pixels that a tile's staged pixels are blended from (6x6, 8x8), down to one
+# pixel, and every channel count's padding.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("c,cout,k,h,w", [(1, 32, 5, 1, 1), (2, 32, 3, 1, 1), (3, 32, 5, 1, 9), (8, 32, 5, 2, 2), (4, 64, 5, 8, 8), (7, 32, 5, 5, 33), (6, 32, 3, 4, 6)])
+def test_upsampled_conv_few_channels_small_planes(c, cout, k, h, w, dtype):
+    test_upsampled_conv_few_channels(c, cout, k, h, w, dtype)
+
+
 def _random_cases(count, seed):
     rng = np.random.RandomState(seed)
     cases = []
