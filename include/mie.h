@@ -248,8 +248,10 @@ int mie_conv_f32x3_takes(int k, int stride, int c1, int c2, int cout);
  *                                         reservoir = r1;
  *                                         out_delta = act(r1) - act(r0)
  * (the fused form of nnConvIncr followed by nnReservedActivation).
- * Stale tiles of `out` are zeroed in out_delta.  Inactive input pixels are
- * never read.  out->pixmask must hold every output pixel whose window contains
+ * Stale tiles of `out` are zeroed in out_delta.  The values of inactive input
+ * pixels have no part in any result, whatever they are (NaN, infinities); a
+ * kernel may fetch them beside their mask bytes (all of x and x2 must be
+ * readable).  out->pixmask must hold every output pixel whose window contains
  * an active input pixel (mie_build_mask_tiles / mie_build_mask_plan make exactly
  * that set; a superset is fine): at the other pixels of an active tile acc is
  * zero by construction, and the matrix-core kernels write out_delta = 0 there

@@ -168,6 +168,22 @@ __device__ __forceinline__ int mie_pick_tile(const TileSetDev& ts, int b,
   return mie_pick_tile_loaded(ts, b, spec, n_active, n_stale, n, y0, x0);
 }
 
+// Whether block `b` of a capacity-sized grid is beyond the active and the stale tiles.
+__device__ __forceinline__ bool mie_no_tile(const TileSetDev& ts, int b) {
+  return b >= ts.counts[MIE_CNT_ACTIVE] + ts.counts[MIE_CNT_STALE];
+}
+
+// Masks first: whether a kernel of little else than loads waits for its mask bytes before it asks for values, so that masked
+// pixels are not fetched.  It is a trip to memory more.  That pays where what could be fetched is more than the L2s keep from one
+// layer to the next -- known to the launcher, which then takes a kernel with both forms: where there is nothing to gain, the
+// branch alone costs 4 to 6 % of a small plane's few microseconds -- and where the step is in between: 4 MB and more
+// (`per_tile` bytes each) in active tiles, or latency is all there is, and fewer than 7 of 8 tiles active, or the masks of the
+// active ones tend to be full.  Figures stand beside the launchers.
+__device__ __forceinline__ bool mie_masks_first(const TileSetDev& ts, int per_tile) {
+  const long long n_act = ts.counts[MIE_CNT_ACTIVE];
+  return n_act * per_tile >= 4LL << 20 && 8 * n_act < 7LL * ts.n * ts.tiles_y * ts.tiles_x;
+}
+
 __device__ __forceinline__ float mie_act(int kind, float slope, float v) {
   switch (kind) {
     case MIE_ACT_RELU: return v > 0.f ? v : 0.f;

@@ -153,11 +153,9 @@ static __device__ __forceinline__ float4 load4(const mie_bf16* p) {
   return make_float4((float)b[0], (float)b[1], (float)b[2], (float)b[3]);
 }
 
-template <typename T, int LP, int CO>
-__global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
-  int n, y0, x0;
-  const int tk = mie_pick_tile(a.ts, blockIdx.x + conv_args_entry_zero(a), n, y0, x0);
-  if (tk == 0) return;
+// MF: masks first (mie_masks_first).
+template <typename T, int LP, int CO, bool MF>
+__device__ __forceinline__ void conv1x1_smallco_tile(const ConvArgsT<T>& a, int tk, int n, int y0, int x0) {
   const int px = blockIdx.y * (256 / LP) + threadIdx.x / LP, sub = threadIdx.x & (LP - 1);
   const int oy = y0 + (px >> 3), ox = x0 + (px & 7);
   const int hout = a.ts.h, wout = a.ts.w;
@@ -167,7 +165,8 @@ __global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
     if (inb && sub < a.cout) mie_st(a.out, po * a.cout + sub, 0.f);
     return;
   }
-  // Everything is asked for at once: the mask bytes, the channels of both inputs (of a masked pixel too: they are dropped),
+  // Everything is asked for at once: the mask bytes, the channels of both inputs (of a masked pixel too, but for large
+  // planes -- mie_masks_first --: they are dropped),
   // their filter rows (x feeds rows [0, c1), x2 rows [c1, c1 + c2)) and what the epilogue reads.  One after the other, behind
   // conditions, those were seven trips to memory of a kernel that does little else (with this, the transposed form below and
   // the few-channel convs' epilogue loads ahead of their contraction: 1x64x96 pass 186.9 -> 185.3 us, optical flow with
@@ -181,20 +180,28 @@ __global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
   mie_mask_ask(x2m, a.filt, at, b2);
   const long long off = mine_ok ? po * a.cout + sub : 0;
   const float e_add = a.addend ? mie_ld(a.addend, off) : 0.f, e_r0 = a.res && !a.refresh ? a.res[off] : 0.f;
-  const int v1 = a.c1 >> 2, vt = v1 + (a.x2 != nullptr ? a.c2 >> 2 : 0);
+  const int v1 = a.c1 >> 2;
+  int vt = v1 + (a.x2 != nullptr ? a.c2 >> 2 : 0);
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   unsigned on = 0u;
+  int pix1 = pix, pix2 = pix;
+  if constexpr (MF) {
+    on = mie_mask_take(a.xm, b1, inb ? 1u : 0u) | mie_mask_take(x2m, b2, inb && a.x2 != nullptr ? 1u : 0u) << 1;
+    pix1 = (on & 1u) != 0u ? pix : 0;
+    pix2 = (on & 2u) != 0u ? pix : 0;
+    if (__ballot(on != 0u) == 0ull) vt = 0;
+  }
   for (int v0 = sub; v0 < vt; v0 += 4 * LP) {
     float4 x[4], w[4][CO];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int v = v0 + u * LP, vc = v < vt ? v : sub;
-      const T* xr = vc < v1 ? a.x + ((long long)pix * a.c1 + 4 * vc) : a.x2 + ((long long)pix * a.c2 + 4 * (vc - v1));
+      const T* xr = vc < v1 ? a.x + ((long long)pix1 * a.c1 + 4 * vc) : a.x2 + ((long long)pix2 * a.c2 + 4 * (vc - v1));
       x[u] = load4(xr);
 #pragma unroll
       for (int j = 0; j < CO; ++j) w[u][j] = *reinterpret_cast<const float4*>(a.filt + 4 * (long long)(vc * CO + j));
     }
-    if (v0 == sub) {
+    if (!MF && v0 == sub) {
       mie_mask_asked();
       on = mie_mask_take(a.xm, b1, inb ? 1u : 0u) | mie_mask_take(x2m, b2, inb && a.x2 != nullptr ? 1u : 0u) << 1;
     }
@@ -223,6 +230,15 @@ __global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
   const bool oks[1] = {mine_ok};
   const float accs[1] = {mine}, r0s[1] = {e_r0}, adds[1] = {e_add};
   conv_epilogue_store<T, 1>(a, offs, cos, oks, accs, r0s, adds);
+}
+
+template <typename T, int LP, int CO, bool LARGE>
+__global__ __launch_bounds__(256) void k_conv1x1_smallco(ConvArgsT<T> a) {
+  int n, y0, x0;
+  const int tk = mie_pick_tile(a.ts, blockIdx.x + conv_args_entry_zero(a), n, y0, x0);
+  if (tk == 0) return;
+  if (LARGE && mie_masks_first(a.ts, 64 * (a.c1 + a.c2) * (int)sizeof(T))) conv1x1_smallco_tile<T, LP, CO, true>(a, tk, n, y0, x0);
+  else conv1x1_smallco_tile<T, LP, CO, false>(a, tk, n, y0, x0);
 }
 
 // ---------------------------------------------------------------------------------
@@ -269,11 +285,8 @@ __global__ __launch_bounds__(256) void k_tconv_valu(ConvArgsT<T> a, int K, int S
 // so 1, 2 or 4 taps -- no division, no modulo.  A thread owns 4 adjacent output channels of one pixel
 // (16-byte filter loads, the input values are broadcast loads); the workgroups of grid row x share one
 // 8x8 output tile.
-template <typename T>
-__global__ __launch_bounds__(256) void k_tconv2x_fewcin(ConvArgsT<T> a) {
-  int n, y0, x0;
-  const int tk = mie_pick_tile(a.ts, blockIdx.x + conv_args_entry_zero(a), n, y0, x0);
-  if (tk == 0) return;
+template <typename T, bool MF>
+__device__ __forceinline__ void tconv2x_fewcin_tile(const ConvArgsT<T>& a, int tk, int n, int y0, int x0) {
   const int hout = a.ts.h, wout = a.ts.w, cout = a.cout, c1 = a.c1;
   const int G = cout >> 2;
   // one (pixel, channel group) per thread: grid y covers the 64 * G items of a tile, so that a tile's
@@ -308,7 +321,14 @@ __global__ __launch_bounds__(256) void k_tconv2x_fewcin(ConvArgsT<T> a) {
     float4 r0[1], add[1], acc[1] = {make_float4(0.f, 0.f, 0.f, 0.f)};
     conv_epilogue_load4<T, 1>(a, offs, oks, r0, add);
     unsigned on = 0u;
-    for (int ci = 0; ci < c1; ci += 2) {
+    int c_end = c1;
+    if constexpr (MF) {
+      on = mie_mask_take(a.xm, b1, in);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) at[t] = ((on >> t) & 1u) != 0u ? at[t] : 0;
+      if (__ballot(on != 0u) == 0ull) c_end = 0;
+    }
+    for (int ci = 0; ci < c_end; ci += 2) {
       const int c2 = ci + 1 < c1 ? ci + 1 : ci;
       float x[4][2];
       float4 w[4][2];
@@ -319,7 +339,7 @@ __global__ __launch_bounds__(256) void k_tconv2x_fewcin(ConvArgsT<T> a) {
         w[t][0] = *reinterpret_cast<const float4*>(wp[t] + (long long)ci * 9 * cout);
         w[t][1] = *reinterpret_cast<const float4*>(wp[t] + (long long)c2 * 9 * cout);
       }
-      if (ci == 0) {
+      if (!MF && ci == 0) {
         mie_mask_asked();
         on = mie_mask_take(a.xm, b1, in);
       }
@@ -335,10 +355,29 @@ __global__ __launch_bounds__(256) void k_tconv2x_fewcin(ConvArgsT<T> a) {
   }
 }
 
+template <typename T, bool LARGE>
+__global__ __launch_bounds__(256) void k_tconv2x_fewcin(ConvArgsT<T> a) {
+  int n, y0, x0;
+  const int tk = mie_pick_tile(a.ts, blockIdx.x + conv_args_entry_zero(a), n, y0, x0);
+  if (tk == 0) return;
+  if (LARGE && mie_masks_first(a.ts, 64 * a.cout * 4)) tconv2x_fewcin_tile<T, true>(a, tk, n, y0, x0);
+  else tconv2x_fewcin_tile<T, false>(a, tk, n, y0, x0);
+}
+
+template <typename T, int CO, bool LARGE>
+void launch_conv1x1_as(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  if (a.c1 >= 128 || a.c2 >= 128) hipLaunchKernelGGL((k_conv1x1_smallco<T, 16, CO, LARGE>), dim3(cap, 4), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((k_conv1x1_smallco<T, 4, CO, LARGE>), dim3(cap), dim3(256), 0, st, a);
+}
 template <typename T, int CO>
 void launch_conv1x1(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
-  if (a.c1 >= 128 || a.c2 >= 128) hipLaunchKernelGGL((k_conv1x1_smallco<T, 16, CO>), dim3(cap, 4), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((k_conv1x1_smallco<T, 4, CO>), dim3(cap), dim3(256), 0, st, a);
+  // Both forms (mie_masks_first) from 40 MB of inputs on.  fp32, active pixels 1 % scattered / 20 % in blobs / all: 128->2 at
+  // 4x264x352 all at once 26.0 / 27.6 / 46.4 us, both forms 21.9 / 26.5 / 46.4; at 1x264x352 (45 MB) 8.7 / 9.2 / 14.3 and 8.1 /
+  // 8.9 / 14.6.  32->1 at 1x480x640 (38 MB) 6.8 / 7.4 / 11.2 and 6.6 / 7.3 / 12.0: nothing to gain any more.
+  const bool masks = a.xm != nullptr || (a.x2 != nullptr && a.x2m != nullptr);
+  if (masks && (long long)a.ts.n * a.h_in * a.w_in * (a.c1 + a.c2) * (int)sizeof(T) >= 40LL << 20)
+    launch_conv1x1_as<T, CO, true>(a, cap, st);
+  else launch_conv1x1_as<T, CO, false>(a, cap, st);
 }
 
 template <typename T, int K, int S>
@@ -570,9 +609,16 @@ int tconv_impl(const char* who, const T* x, const uint8_t* xmask, int cin, int h
   a.ts = mie_dev_tileset(out);
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
   if (k == 3 && stride == 2 && pad == 1 && out->h == 2 * h_in && out->w == 2 * w_in && cin <= 8 && cout % 4 == 0 &&
-      mie_aligned(filter, 16))
-    hipLaunchKernelGGL(k_tconv2x_fewcin<T>, dim3(cap, mie_div_up(16 * cout, 256)), dim3(256), 0, (hipStream_t)stream, a);
-  else
+      mie_aligned(filter, 16)) {
+    // Both forms (mie_masks_first) from 200 MB of outputs on: what masked pixels cost here are the filter's rows for them.  fp32,
+    // active pixels 1 % scattered / 20 % in blobs / all: 4->64 at 8x240x320 all at once 136 / 198 / 490 us, both forms 111 / 201 /
+    // 497; 2->32 at 8x120x160 (79 MB) 16.1 / 21.9 / 44.9 and 15.8 / 23.7 / 45.0.
+    const dim3 grid(cap, mie_div_up(16 * cout, 256));
+    if (xmask != nullptr && 4LL * out->n * out->h * out->w * cout >= 200LL << 20)
+      hipLaunchKernelGGL((k_tconv2x_fewcin<T, true>), grid, dim3(256), 0, (hipStream_t)stream, a);
+    else
+      hipLaunchKernelGGL((k_tconv2x_fewcin<T, false>), grid, dim3(256), 0, (hipStream_t)stream, a);
+  } else
     hipLaunchKernelGGL(k_tconv_valu<T>, dim3(cap, mie_div_up(cout, 64)), dim3(256), 0,
                        (hipStream_t)stream, a, k, stride);
   return mie_check_launch(who);

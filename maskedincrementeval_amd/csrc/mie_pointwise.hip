@@ -5,6 +5,8 @@
 // channels of the NHWC row (float4 when C % 4 == 0), so a wave reads whole
 // 8-pixel rows of the tile as contiguous segments.
 #include "mie_common.h"
+
+#include <type_traits>
 #include "mie_conv.h"
 
 namespace {
@@ -303,7 +305,8 @@ __device__ __forceinline__ void up2x_coef(int o, int in_size, int& i0, int& i1, 
 // pixels (rows y0/2-1 .. y0/2+4): the block is summed (a + b, masked) into LDS once, fp32, and every
 // output slot then reads its four taps from there -- 36 source pixels fetched per tile instead of
 // 4 per output pixel, which is what the kernel was bound by (load instructions, not bytes).
-template <typename T, int VEC>
+// TWO: b is there.  MF: masks first (mie_masks_first); otherwise masks and values go out together.
+template <typename T, int VEC, bool TWO, bool MF>
 __device__ __forceinline__ void up2x_tile(const TileSetDev& ts, const T* __restrict__ a,
                                           const uint8_t* __restrict__ ma, const T* __restrict__ b,
                                           const uint8_t* __restrict__ mb, int h_in, int w_in,
@@ -329,16 +332,31 @@ __device__ __forceinline__ void up2x_tile(const TileSetDev& ts, const T* __restr
       const int sp = idx / cvb, cq = idx - sp * cvb;
       const int sy = ry0 + sp / 6, sx = rx0 + sp % 6;
       const bool in = sy >= 0 && sy < h_in && sx >= 0 && sx < w_in;
-      // masks and values go out together
       const int at[1] = {in ? (n * h_in + sy) * w_in + sx : 0};
       const long long eo = (long long)at[0] * c + (long long)(cq0 + cq) * VEC;
-      const uint8_t* const m1 = b != nullptr ? mb : nullptr;
       unsigned b0[1], b1[1];
       mie_mask_ask(ma, a, at, b0);
-      mie_mask_ask(m1, a, at, b1);
-      Vec<VEC> t = Vec<VEC>::load(a + eo), u = Vec<VEC>::load((b != nullptr ? b : a) + eo);
-      mie_mask_asked();
-      const bool k0 = mie_mask_take(ma, b0, in ? 1u : 0u) != 0u, k1 = mie_mask_take(m1, b1, in && b != nullptr ? 1u : 0u) != 0u;
+      if constexpr (TWO) mie_mask_ask(mb, a, at, b1);
+      bool k0 = true, k1 = TWO;
+      auto take = [&]() {
+        k0 = mie_mask_take(ma, b0, in ? 1u : 0u) != 0u;
+        if constexpr (TWO) k1 = mie_mask_take(mb, b1, in ? 1u : 0u) != 0u;
+      };
+      Vec<VEC> t = Vec<VEC>::zero();
+      if constexpr (MF) {
+        take();
+        if (__ballot(k0 | k1) == 0ull) {
+          t.store(s_src + sp * cw + cq * VEC);
+          continue;
+        }
+      }
+      t = Vec<VEC>::load(a + (k0 ? eo : 0));
+      Vec<VEC> u = Vec<VEC>::zero();
+      if constexpr (TWO) u = Vec<VEC>::load(b + (k1 ? eo : 0));
+      if constexpr (!MF) {
+        mie_mask_asked();
+        take();
+      }
 #pragma unroll
       for (int e = 0; e < VEC; ++e) t[e] = (k0 ? t[e] : 0.f) + (k1 ? u[e] : 0.f);
       t.store(s_src + sp * cw + cq * VEC);
@@ -372,13 +390,15 @@ __device__ __forceinline__ void up2x_tile(const TileSetDev& ts, const T* __restr
   });
 }
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool TWO, bool LARGE>
 __global__ __launch_bounds__(256) void k_up2x_incr(TileSetDev ts, const T* __restrict__ a,
                                                    const uint8_t* __restrict__ ma,
                                                    const T* __restrict__ b,
                                                    const uint8_t* __restrict__ mb, int h_in,
                                                    int w_in, T* __restrict__ dout, int c) {
-  up2x_tile<T, VEC>(ts, a, ma, b, mb, h_in, w_in, dout, c);
+  if (LARGE && mie_no_tile(ts, blockIdx.x)) return;
+  if (LARGE && mie_masks_first(ts, 16 * c * (TWO ? 2 : 1) * (int)sizeof(T))) up2x_tile<T, VEC, TWO, true>(ts, a, ma, b, mb, h_in, w_in, dout, c);
+  else up2x_tile<T, VEC, TWO, false>(ts, a, ma, b, mb, h_in, w_in, dout, c);
 }
 
 // Two independent up-samplings of the same geometry (tensors, masks and tile sets of their own) in one
@@ -387,10 +407,12 @@ template <typename T>
 struct Up2xSet {
   TileSetDev ts; const T* a; const uint8_t* ma; T* out;
 };
-template <typename T, int VEC>
+template <typename T, int VEC, bool LARGE>
 __global__ __launch_bounds__(256) void k_up2x_pair(Up2xSet<T> s0, Up2xSet<T> s1, int h_in, int w_in, int c) {
-  if (blockIdx.z == 0) up2x_tile<T, VEC>(s0.ts, s0.a, s0.ma, (const T*)nullptr, (const uint8_t*)nullptr, h_in, w_in, s0.out, c);
-  else up2x_tile<T, VEC>(s1.ts, s1.a, s1.ma, (const T*)nullptr, (const uint8_t*)nullptr, h_in, w_in, s1.out, c);
+  const Up2xSet<T>& s = blockIdx.z == 0 ? s0 : s1;
+  if (LARGE && mie_no_tile(s.ts, blockIdx.x)) return;
+  if (LARGE && mie_masks_first(s.ts, 16 * c * (int)sizeof(T))) up2x_tile<T, VEC, false, true>(s.ts, s.a, s.ma, (const T*)nullptr, (const uint8_t*)nullptr, h_in, w_in, s.out, c);
+  else up2x_tile<T, VEC, false, false>(s.ts, s.a, s.ma, (const T*)nullptr, (const uint8_t*)nullptr, h_in, w_in, s.out, c);
 }
 
 // ---- max pooling increment and masked accumulate ---------------------------------
@@ -682,15 +704,27 @@ extern "C" int mie_upsample2x_incr(const void* a, const uint8_t* ma, const void*
   const unsigned ny_min = (unsigned)mie_div_up(c, 256);
   if (ny < ny_min) ny = ny_min;
   const size_t lds = (size_t)36 * mie_div_up(cv, (int)ny) * vec * sizeof(float);
-#define MIE_UP2X_LAUNCH(T_, V_)                                                                              \
-  hipLaunchKernelGGL((k_up2x_incr<T_, V_>), dim3(grid, ny), dim3(256), lds, (hipStream_t)stream, d, (const T_*)a, \
+  // Both forms (mie_masks_first) from 16 MB of inputs on.  a + b of 64 channels in fp32, active pixels 1 % scattered / 20 % in
+  // blobs / all: 8x120x160 all at once 28.1 / 39.5 / 52.3 us, both forms 20.7 / 28.6 / 52.4; 2x120x160 (20 MB) 10.4 / 13.6 / 16.8
+  // and 9.3 / 12.1 / 15.7; 1x128x128 (8 MB) 6.1 / 7.1 / 9.2 and 6.1 / 7.1 / 9.4.
+  const bool large = (ma != nullptr || mb != nullptr) && (long long)out->n * h_in * w_in * c * (bf ? 2 : 4) * (b ? 2 : 1) >= 16LL << 20;
+#define MIE_UP2X_FORM(T_, V_, TWO_, LARGE_)                                                                                        \
+  hipLaunchKernelGGL((k_up2x_incr<T_, V_, TWO_, LARGE_>), dim3(grid, ny), dim3(256), lds, (hipStream_t)stream, d, (const T_*)a, \
                      ma, (const T_*)b, mb, h_in, w_in, (T_*)out_delta, c)
+#define MIE_UP2X_LAUNCH(T_, V_)                                                      \
+  do {                                                                               \
+    if (b != nullptr && large) MIE_UP2X_FORM(T_, V_, true, true);                       \
+    else if (b != nullptr) MIE_UP2X_FORM(T_, V_, true, false);                       \
+    else if (large) MIE_UP2X_FORM(T_, V_, false, true);                                 \
+    else MIE_UP2X_FORM(T_, V_, false, false);                                        \
+  } while (0)
   if (bf) {
     if (vec == 8) MIE_UP2X_LAUNCH(mie_bf16, 8); else if (vec == 4) MIE_UP2X_LAUNCH(mie_bf16, 4); else MIE_UP2X_LAUNCH(mie_bf16, 1);
   } else {
     if (vec == 8) MIE_UP2X_LAUNCH(float, 8); else if (vec == 4) MIE_UP2X_LAUNCH(float, 4); else MIE_UP2X_LAUNCH(float, 1);
   }
 #undef MIE_UP2X_LAUNCH
+#undef MIE_UP2X_FORM
   return mie_check_launch(who);
 }
 
@@ -720,12 +754,13 @@ extern "C" int mie_upsample2x_pair_incr(const void* a0, const uint8_t* m0, const
   const unsigned ny_min = (unsigned)mie_div_up(c, 256);
   if (ny < ny_min) ny = ny_min;
   const size_t lds = (size_t)36 * mie_div_up(cv, (int)ny) * vec * sizeof(float);
+  const bool large = (m0 != nullptr || m1 != nullptr) && 2LL * out0->n * h_in * w_in * c * (bf ? 2 : 4) >= 16LL << 20;      // (as above)
 #define MIE_UP2X_PAIR(T_, V_)                                                                                  \
   do {                                                                                                         \
     Up2xSet<T_> s0{mie_dev_tileset(out0), (const T_*)a0, m0, (T_*)out_delta0};                                  \
     Up2xSet<T_> s1{mie_dev_tileset(out1), (const T_*)a1, m1, (T_*)out_delta1};                                  \
-    hipLaunchKernelGGL((k_up2x_pair<T_, V_>), dim3(grid, ny, 2), dim3(256), lds, (hipStream_t)stream, s0, s1,  \
-                       h_in, w_in, c);                                                                         \
+    if (large) hipLaunchKernelGGL((k_up2x_pair<T_, V_, true>), dim3(grid, ny, 2), dim3(256), lds, (hipStream_t)stream, s0, s1, h_in, w_in, c); \
+    else hipLaunchKernelGGL((k_up2x_pair<T_, V_, false>), dim3(grid, ny, 2), dim3(256), lds, (hipStream_t)stream, s0, s1, h_in, w_in, c);   \
   } while (0)
   if (bf) {
     if (vec == 8) MIE_UP2X_PAIR(mie_bf16, 8); else if (vec == 4) MIE_UP2X_PAIR(mie_bf16, 4); else MIE_UP2X_PAIR(mie_bf16, 1);

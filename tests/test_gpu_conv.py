@@ -973,3 +973,48 @@ def test_gates_conv_of_few_active_tiles(h, w, c2, hid):
             got = got.float().cpu().double()
             assert (got - want).abs().max().item() <= 4 * bound + want.abs().max().item() * 2.0 ** -8, (count, step)
             assert not got[(m == 0).expand_as(got) & (torch.nn.functional.max_pool2d(m.float(), 3, 1, 1) == 0).expand_as(got)].any()
+
+
+# Kernels of little else than loads take the masks of large planes first where a step is neither nearly empty nor nearly full:
+# two samples in one call (over the line) against the same samples one by one (below it), bit for bit, NaN in every inactive
+# input pixel; blobs, scattered pixels (waves with nothing to do between others), a few, all, none.
+@pytest.mark.parametrize("kind", ["conv1x1", "up2x", "up2x_one", "up2x_pair", "tconv"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_masks_first_on_large_planes(kind, dtype):
+    bf = dtype == torch.bfloat16
+    cin, cout, h, w = {"conv1x1": (256 if bf else 128, 2, 264, 170), "up2x_one": (256 if bf else 128, 0, 120, 157), "tconv": (4, 128, 230, 310)}.get(
+        kind, (128 if bf else 64, 0, 120, 157))
+    n, scale = 2, 1 if kind == "conv1x1" else 2
+    H, W = scale * h, scale * w
+    g = torch.Generator().manual_seed(8)
+    x, x2 = (torch.randn(n, cin, h, w, generator=g).to(DEV).to(dtype).contiguous(memory_format=torch.channels_last) for _ in range(2))
+    wt = torch.randn(*((cin, 3, 3, cout) if kind == "tconv" else (cin, 1, 1, max(cout, 1))), generator=g).to(DEV)
+    res0 = torch.randn(n, max(cout, 1), H, W, generator=g).to(DEV).contiguous(memory_format=torch.channels_last)
+    foot = {"conv1x1": (_lib.FOOT_CONV, 1, 1, 0), "tconv": (_lib.FOOT_TCONV, 3, 2, 1)}.get(kind, (_lib.FOOT_UP2X, 0, 0, 0))
+    sets = [[TileMask(k, H, W, DEV) for _ in range(2)] for k in (n, 1, 1)]
+    outs = [[ops.new_nhwc(k, cout or cin, H, W, DEV, dtype) for _ in range(2)] for k in (n, 1, 1)]
+    share = []
+    for dens, dots in ((0.2, False), (0.01, True), (0.0005, False), (1.0, False), (0.0, False), (0.1, True)):
+        m, m2 = ((torch.rand(n, 1, h, w, generator=g) < dens).to(torch.uint8) if dots else
+                 gaussian_delta(n, 1, h, w, dens, 1.0, seed=31 + 7 * k)[1] for k in range(2))
+        poison = lambda t, mm: torch.where(mm.to(DEV).bool(), t, torch.full_like(t, float("nan"))).contiguous(memory_format=torch.channels_last)
+        px, px2 = poison(x, m), poison(x2, m2)
+        for j, part in enumerate((slice(0, n), slice(0, 1), slice(1, 2))):
+            one = lambda t: ops.as_nhwc(t[part].contiguous(memory_format=torch.channels_last))
+            a, b, da, db = one(px), one(px2), m[part].contiguous().to(DEV), m2[part].contiguous().to(DEV)
+            (ts, ts2), (out, out2), k = sets[j], outs[j], a.shape[0]
+            ops.build_mask_tiles(da, db if kind == "up2x" else None, k, h, w, *foot, ts)
+            if kind == "conv1x1":
+                ops.conv_masked(a, da, None, None, wt, 1, 1, 0, ts, out, one(res0).clone(memory_format=torch.preserve_format), _lib.ACT_RELU)
+            elif kind == "tconv":
+                ops.tconv_masked(a, da, wt, 3, 2, 1, ts, out, one(res0).clone(memory_format=torch.preserve_format), _lib.ACT_LEAKY_RELU, 0.1)
+            elif kind == "up2x_pair":
+                ops.build_mask_tiles(db, None, k, h, w, *foot, ts2)
+                ops.upsample2x_pair_incr(a, da, ts, out, b, db, ts2, out2)
+            else:
+                ops.upsample2x_incr(a, da, b if kind == "up2x" else None, db if kind == "up2x" else None, ts, out)
+        share.append(int(sets[0][0].counts[0]) / sets[0][0].capacity)
+        for q in range(2 if kind == "up2x_pair" else 1):
+            assert torch.isfinite(outs[0][q]).all()
+            assert torch.equal(outs[0][q], torch.cat([outs[1][q], outs[2][q]], 0)), (kind, dens, dots)
+    assert any(0.3 < v < 0.8 for v in share) and share[3] == 1.0 and share[4] == 0.0
