@@ -1018,3 +1018,44 @@ def test_masks_first_on_large_planes(kind, dtype):
             assert torch.isfinite(outs[0][q]).all()
             assert torch.equal(outs[0][q], torch.cat([outs[1][q], outs[2][q]], 0)), (kind, dens, dots)
     assert any(0.3 < v < 0.8 for v in share) and share[3] == 1.0 and share[4] == 0.0
+
+
+@pytest.mark.parametrize("n,hid,h,w", [(10, 64, 56, 64), (10, 128, 33, 44), (8, 256, 17, 22)])
+def test_gates_pairs_error_against_fp64_beside_one_tile(n, hid, h, w):
+    """The bf16 gates conv with two tiles a workgroup (n samples at once) adds the K products of a sum in one fp32 accumulator, as the
+    one-tile form of 128 columns does that it stands for, only 16 channels x taps instead of taps x channels: against fp64 over the
+    same bf16 values 0.998 to 1.001 of that form's error.  Beside it here the samples one by one, which are small enough for the
+    32-column form: four accumulators of K / 4 products each, whose roundings, at random, add up to half as much (1.97 to 2.10
+    measured, 2.2 allowed).  Of the state deltas, rounded to bf16 at the end (1.66e-3 rms for evenly spread mantissas), it is no
+    part that shows."""
+    bf, c, cols = torch.bfloat16, hid, 4 * hid
+    wt = (he_normal_conv_weight(cols, 2 * c, 3, 31) * 0.5).to(bf)
+    filt = _filt(wt.float())
+    ns = cols // 128
+    tiles = ((h + 7) // 8) * ((w + 7) // 8)
+    assert (tiles // 2 + 1) * ns < 256 <= (n * tiles // 2 + 1) * ns and tiles * (cols // 32) > 128
+    g = torch.Generator().manual_seed(hid)
+    x, x2 = (torch.randn(n, c, h, w, generator=g).to(bf) for _ in range(2))
+    pad = F.pad(torch.cat([x, x2], 1).to(DEV).double(), (1, 1, 1, 1)).permute(0, 2, 3, 1).contiguous()
+    f64 = filt.plain.double()
+    d = sum(pad[:, y:y + h, z:z + w].reshape(-1, 2 * c) @ f64[:, y, z] for y in range(3) for z in range(3))
+    q = d.view(n, h, w, hid, 4)
+    dc = torch.sigmoid(q[..., 0]) * torch.tanh(q[..., 3])
+    want = {"sums": d.view(n, h, w, cols), "cell": dc, "hidden": torch.sigmoid(q[..., 2]) * torch.tanh(dc)}
+    err = []
+    for parts in ([slice(0, n)], [slice(i, i + 1) for i in range(n)]):
+        got = {k: [] for k in want}
+        for part in parts:
+            a, b = x[part], x2[part]
+            k = a.shape[0]
+            ts = TileMask(k, h, w, DEV)
+            ops.build_mask_tiles(None, None, k, h, w, _lib.FOOT_CONV, 3, 1, 1, ts)
+            res = [ops.new_nhwc(k, m, h, w, DEV).zero_() for m in (cols, hid, hid)]
+            dh, dcell = (ops.new_nhwc(k, hid, h, w, DEV, bf) for _ in range(2))
+            ops.conv_gates_incr(_dev(a.float()).to(bf), None, _dev(b.float()).to(bf), None, filt, ts, res[0], None, None, res[1], res[2], dh, dcell)
+            for name, t in (("sums", res[0]), ("cell", dcell), ("hidden", dh)):
+                got[name].append(t.permute(0, 2, 3, 1).double())
+        err.append({name: ((torch.cat(got[name]) - want[name]).norm() / want[name].norm()).item() for name in want})
+    print("hid %d at %dx%dx%d: two tiles %s, one %s" % (hid, n, h, w, *({k: "%.3e" % v for k, v in e.items()} for e in err)))
+    assert err[0]["sums"] <= 2.2 * err[1]["sums"], err
+    assert all(err[0][k] <= 1.002 * err[1][k] and err[0][k] < 1.8e-3 for k in ("cell", "hidden")), err

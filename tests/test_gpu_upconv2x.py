@@ -162,6 +162,51 @@ def test_fused_tail_at_input_resolution(n, h, w):
         res_ref, pres_ref = got_res, pres.cpu()
 
 
+@pytest.mark.parametrize("kind", ["white", "smooth"])
+@pytest.mark.parametrize("n,h,w", [(3, 100, 118), (1, 182, 183), (2, 129, 145)])
+def test_fused_tail_error_against_fp64_beside_the_one_tile_form(n, h, w, kind):
+    """The two forms of the fused tail (mie_upconv2x_pred_masked, mie_upconv_pred_masked) next to the decoder and the prediction in
+    fp64, over the fp32 weights of the decoder.  Each rounds the sum of its inputs (up-sampled or not) and its weights (combined
+    or not) to 8 bits before the sums, and the activation increment to 8 bits behind them; the accumulators are fp32 in both.  On
+    smooth inputs, as layers see them, this form is the closer one (the decoder's sums 0.64 - 0.67 of the one-tile form's error, the
+    prediction's 0.79 - 0.86, its delta 0.83 - 0.93); on white noise the blend of independent pixels spreads the one-tile form's
+    mantissas more evenly, as in test_error_against_fp64_beside_the_list_driven_form: 1.01 - 1.03, 1.04 allowed."""
+    bf = torch.bfloat16
+    c, cout, H, W = 64, 32, 2 * h, 2 * w
+    g = torch.Generator().manual_seed(h)
+    a, b = (torch.randn(n, c, h, w, generator=g) for _ in range(2))
+    if kind == "smooth":
+        a, b = (torch.nn.functional.avg_pool2d(t, 5, 1, 2) * 4.0 + 1.0 for t in (a, b))
+    skip = torch.randn(n, cout, H, W, generator=g)
+    wt = he_normal_conv_weight(cout, c, 5, 9)
+    filt = ops.ConvFilter(wt.permute(1, 2, 3, 0).contiguous().to(DEV))
+    pred_w = (torch.randn(2, cout, generator=g) * 0.3).to(DEV)
+    da, db, ds = _dev(a, bf), _dev(b, bf), _dev(skip, bf)
+    ts = TileMask(n, H, W, DEV)
+    ops.build_mask_tiles(None, None, n, H, W, _lib.FOOT_CONV, 1, 1, 0, ts)
+    r0, p0 = (torch.randn(n, k, H, W, generator=g) for k in (cout, 1))
+    up = torch.nn.functional.interpolate(da.double() + db.double(), scale_factor=2, mode="bilinear", align_corners=False)
+    up = torch.nn.functional.pad(up, (2, 2, 2, 2)).permute(0, 2, 3, 1).contiguous()
+    conv = sum(up[:, y:y + H, x:x + W].reshape(-1, c) @ filt.plain[:, y, x].double() for y in range(5) for x in range(5)).view(n, H, W, cout)
+    r = r0.to(DEV).double().permute(0, 2, 3, 1)
+    y = torch.relu(r + conv) - torch.relu(r)
+    z = (y * pred_w[0].double() + ds.double().permute(0, 2, 3, 1) * pred_w[1].double()).sum(3)
+    p = p0.to(DEV).double()[:, 0]
+    delta = torch.sigmoid(p + z) - torch.sigmoid(p)
+    err = []
+    for dense in (False, True):
+        res, pres, out = _dev(r0).clone(), _dev(p0).clone(), ops.new_nhwc(n, 1, H, W, DEV, bf)
+        assert ops.upconv_pred_takes(c, cout, 5, 1, 2, filt, bf, ts.capacity, _lib.ACT_RELU)
+        ops.upconv_pred_masked(da, None, db, None, filt, ts, res, _lib.ACT_RELU, 0.0, ds, None, pred_w, pres, _lib.ACT_SIGMOID, 0.0, out,
+                               dense_plane=dense)
+        rel = lambda got, want: ((got - want).norm() / want.norm()).item()
+        err.append((rel(res.double().permute(0, 2, 3, 1) - r, conv), rel(pres.double()[:, 0] - p, z), rel(out.double()[:, 0], delta)))
+    print("%s %dx%dx%d: decoder / prediction sums, delta: one tile %.3e %.3e %.3e, here %.3e %.3e %.3e" % (kind, n, h, w, *err[0], *err[1]))
+    assert err[1][0] < 3.0e-3, err      # (three roundings of 1.66e-3 rms; the prediction's sums cancel, more or less, by chance)
+    for one, here in zip(*err):
+        assert here <= (1.04 if kind == "white" else 1.0) * one, err
+
+
 @pytest.mark.parametrize("n,h,w", [(3, 100, 118), (1, 150, 170), (8, 35, 67), (2, 20, 801)])
 def test_decoder_conv_of_many_items(n, h, w):
     # 128 -> 64 channels in bf16 from three items of 8 x 16 positions a workgroup on: the persistent kernel makes all but the
