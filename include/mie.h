@@ -700,7 +700,8 @@ int mie_upconv_masked_ws(const void* a, const uint8_t* amask, const void* b,
  *   r1 = reservoir + conv;  y = act(r1) - act(reservoir)  (rounded to the delta type);  reservoir = r1
  *   z  = sum_c pred_filter[c] * y[c] + pred_filter[cout + c] * skip[c]
  *   p1 = pred_reservoir + z;  pred_delta = pred_act(p1) - pred_act(pred_reservoir);  pred_reservoir = p1
- * at every pixel of the active tiles of `out`, zeros in pred_delta ([n, 2*h_in, 2*w_in], element type `dtype`) on its
+ * at every pixel of the active tiles of `out` (also outside its pixmask: unlike in mie_conv_masked an infinity or a NaN
+ * in a reservoir there reaches the prediction), zeros in pred_delta ([n, 2*h_in, 2*w_in], element type `dtype`) on its
  * stale tiles.  `out` is the tile set of the PREDICTION: the union of the decoder's output set and the set of skip
  * (mie_build_mask_tiles with both as inputs, MIE_FOOT_CONV k = 1); the decoder's conv runs on all of its tiles.
  * pred_filter: fp32 [2][cout], the prediction conv's weights for y and for skip (the same row twice for
@@ -722,7 +723,9 @@ int mie_upconv_pred_masked(const void* a, const uint8_t* amask, const void* b,
  * mie_upconv_pred_masked with the tiles away from the plane's border computed at the resolution of a and b, as four 4x4
  * convs over a + b, one per output phase (mie_upconv2x_masked): filter_up is mie_pack_filter_up2x's combined filter of
  * `filter` in MIE_DTYPE_BF16, 16-byte aligned; a + b and the combined filter are rounded to bf16 (there: the blended
- * up-sampled values and the filter).  Two launches.  Planes of at least 3 x 3 tiles; all else as there.
+ * up-sampled values and the filter).  Two launches.  Planes of at least 3 x 3 tiles; all else as there.  The tile set's
+ * flags are read: it must be one of the library's builders'.  Items are 2 x 4 tiles: for planes whose active tiles lie
+ * together; tiles scattered over a plane run faster tile by tile (mie_upconv_pred_masked).
  */
 int mie_upconv2x_pred_masked(const void* a, const uint8_t* amask, const void* b,
                              const uint8_t* bmask, int c, int h_in, int w_in,
@@ -866,6 +869,8 @@ int mie_events_to_frame_bf16(const double* events, int n_events, int kind, int n
  *   dtype     : MIE_DTYPE_BF16, or MIE_DTYPE_F32_BF16X3 for fp32 deltas; c a multiple of 64 / 32, cout of 32;
  *               planes of at least 2x2 pixels
  *   the rest as in mie_upconv_masked.  The tile set's flags are read: it must be one of the library's builders'.
+ *   Whole blocks of 8 x 8 positions (128 -> 64 channels in bf16 on large planes: 8 x 16) run for any active tile in
+ *   them: for planes whose active tiles lie together (scattered ones: mie_upconv_masked).
  * bf16: what is rounded to bf16 is a + b and the combined weights, each once (mie_upconv_masked: the up-sampled sums and
  * the plain weights).
  */
