@@ -241,6 +241,13 @@ int mie_pack_filter(const float* filter, int cin, int k, int cout, void* packed,
 int mie_conv_f32x3_takes(int k, int stride, int c1, int c2, int cout);
 
 /*
+ * Whether mie_conv_masked, without a workspace, runs a conv of this shape (matrix-core path; `tiles` = mie_tile_capacity of
+ * its output, dtype with MIE_DTYPE_F32_BF16X3 where the call has it) in one launch faster than mie_conv_masked_ws runs it with one.
+ * Host logic only.
+ */
+int mie_conv_needs_no_workspace(int k, int stride, int c1, int c2, int cout, int tiles, int dtype);
+
+/*
  * Masked convolution of a delta: for every active tile of `out`
  *   acc = conv2d(x (++ x2), filter, bias = none, stride, pad)
  * and then, with reservoir == NULL:      out_delta  = acc

@@ -178,6 +178,11 @@ static __device__ __forceinline__ void conv_store_batch(const ConvArgsT<T>& a, c
 // beforehand.
 bool mie_launch_conv_mfma(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st);
 bool mie_launch_conv_mfma(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st);
+// The plain 3x3 stride-1 conv on planes of few tiles, without a workspace (mie_conv_deep.hip).  Returns false, launching nothing,
+// for other calls; mie_conv_deep_form says so beforehand (`dtype` as the caller gave it).
+bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype);
+bool mie_launch_conv_deep(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st);
+bool mie_launch_conv_deep(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st);
 // The 3x3 stride-1 conv of a ConvLSTM with the gate chain as its epilogue (a.hid > 0, a.cout = 4*hid,
 // filter columns in the gate-interleaved order of mie_conv_gates_masked).
 bool mie_launch_conv_gates_mfma(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);

@@ -2,7 +2,7 @@
 #include "mie_conv_mfma_impl.h"
 
 bool mie_launch_conv_mfma(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st) {
-  return launch_any<mie_bf16>(a, k, s, cap, st);
+  return mie_launch_conv_deep(a, k, s, cap, st) || launch_any<mie_bf16>(a, k, s, cap, st);
 }
 bool mie_launch_conv_gates_mfma(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) {
   return mie_launch_gates_pairs(a, cap, st) || launch_gates<mie_bf16>(a, cap, st);

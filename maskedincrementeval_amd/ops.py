@@ -808,8 +808,10 @@ def conv_masked(x, xmask, x2, x2mask, filt, k, stride, pad, out_ts: TileMask, ou
     if addend is not None and addend.shape != out_delta.shape:
         raise ValueError("addend shape %s != output %s" % (tuple(addend.shape), tuple(out_delta.shape)))
     _ready(out_ts)
-    # only launches the library would split get the shared buffer
-    ws_ptr, ws_bytes = _workspace_args(workspace, small and mc_ptr is not None, x.device)
+    # only launches the library would split, and has no better form for, get the shared buffer
+    small = small and mc_ptr is not None and workspace is None and split_enabled \
+        and not lib().mie_conv_needs_no_workspace(k, stride, c1, c2, cout, out_ts.capacity, code)
+    ws_ptr, ws_bytes = _workspace_args(workspace, small, x.device)
     check(lib().mie_conv_masked_ws(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1,
         nhwc_ptr(x2, "x2", dtype=dt), pix_ptr(x2mask, n, h, w, "x2mask"), c2, h, w,
