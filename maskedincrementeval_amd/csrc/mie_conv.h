@@ -35,15 +35,15 @@ typedef ConvArgsT<float> ConvArgs;
 
 // The argument block is five cache lines of device memory that no cache holds when a launch starts.  Left to itself the
 // compiler fetches a field where it is first used, and a workgroup then stalls on those lines one after the other on its
-// way to its first loads.  This reads one field of every line in one batch at the kernel's entry, so that the later
+// way to its first loads.  This wants one field of every line at the kernel's entry, so that they are read in one batch and the later
 // reads hit the scalar cache, and returns zero -- out of an instruction the compiler cannot see through, to be added to
-// the workgroup index, so that the reads can neither be dropped nor moved down.  (The asm is not volatile, which would
-// turn every later uniform load into a vector load.)  Measured on the 264x352 frame: 0.565 -> 0.562 ms.
+// the workgroup index, so that the reads can neither be dropped nor moved down.  The fields are operands of that one instruction:
+// with a sum of them before it the compiler took them two lines at a time.  (The asm is not volatile, which would
+// turn every later uniform load into a vector load.)
 template <typename T>
 static __device__ __forceinline__ int conv_args_entry_zero(const ConvArgsT<T>& a) {
-  const int touch = a.c1 ^ a.cout ^ a.hid ^ a.xcd_fs ^ a.ts.n;      // (the fifth line holds the list pointers, read next)
   int zero;
-  asm("s_and_b32 %0, %1, 0" : "=s"(zero) : "s"(touch) : "scc");
+  asm("s_and_b32 %0, %1, 0" : "=s"(zero) : "s"(a.c1), "s"(a.cout), "s"(a.hid), "s"(a.xcd_fs), "s"(a.ts.n) : "scc");
   return zero;
 }
 

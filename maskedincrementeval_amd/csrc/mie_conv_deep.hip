@@ -49,8 +49,7 @@ __global__ __launch_bounds__(64 * DEEP_WAVES) void k_conv_deep(ConvArgsT<T> a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kg = lane >> 4, l16 = lane & 15;
-  int bx = blockIdx.x + conv_args_entry_zero(a), by = blockIdx.y, bz = 0;
-  split_order(bx, by, bz);
+  const int by = blockIdx.x + conv_args_entry_zero(a), bx = blockIdx.y;
   const int co0 = by * DEEP_COLS, cout = a.cout;
 
   const int cg = wave % NCW, tc = wave / NCW;
@@ -220,7 +219,7 @@ __global__ __launch_bounds__(64 * DEEP_WAVES) void k_conv_deep(ConvArgsT<T> a) {
 
 template <typename T, int ROWS>
 void launch_rows(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
-  const dim3 grid(8 / ROWS * cap, a.cout / DEEP_COLS), block(64 * DEEP_WAVES);
+  const dim3 grid(a.cout / DEEP_COLS, 8 / ROWS * cap), block(64 * DEEP_WAVES);
   const int nch = (a.c1 + a.c2) / 32;
   if (nch >= 8) hipLaunchKernelGGL((k_conv_deep<T, 1, ROWS>), grid, block, 0, st, a);
   else if (nch >= 4) hipLaunchKernelGGL((k_conv_deep<T, 2, ROWS>), grid, block, 0, st, a);

@@ -334,14 +334,13 @@ __device__ void conv_quad_again(const ConvArgsT<T>& a, int n, int oy, int ox, in
 // Grids whose slices do not divide by 8 keep the launch order.  Whole passes, launch order -> this: optical flow 1x256x256
 // 366.7 -> 361.7 us (transposed convs), 467.9 -> 459.5 (up-sampling), e2depth 1x128x128 246.4 -> 243.8, 1x64x96 181.1 ->
 // 180.6 (two tiles: a slice was on two XCDs).
-__device__ __forceinline__ void split_order(int& bx, int& by, int& bz) {
-  const int gx = (int)gridDim.x, gy = (int)gridDim.y, slices = gy * (int)gridDim.z;
-  if ((slices & 7) != 0) return;
-  const int id = (bz * gy + by) * gx + bx, at = id >> 3, q = at / gx;
-  const int c = (id & 7) * (slices >> 3) + q;
-  bx = at - q * gx;
-  bz = c / gy;
-  by = c - bz * gy;
+// The grid is (slab, part) by tile for that: the hardware deals workgroups out to the XCDs in launch order, x fastest.
+template <typename T>
+__device__ __forceinline__ void split_order(const ConvArgsT<T>& a, int& bx, int& by, int& bz) {
+  const int slice = bx, lp = a.xcd_fs;        // (of a split launch: log2 of the parts)
+  bx = by;
+  by = slice >> lp;
+  bz = slice - (by << lp);
 }
 
 // UP: the conv input is up2x(x + x2), the bilinear x2 up-sampling of the sum of two deltas given at
@@ -350,7 +349,7 @@ __device__ __forceinline__ void split_order(int& bx, int& by, int& bz) {
 // from there.  5x5, stride 1, pad 2 only; a.h_in / a.w_in are the up-sampled size.
 //
 // SPLIT: launches with very few tiles (a 16x16 plane is 4 of them) leave most CUs idle.  The staged
-// chunks of every (tile, slab) are then split over gridDim.z workgroups; each writes its partial sums,
+// chunks of every (tile, slab) are then split over up to 8 workgroups; each writes its partial sums,
 // fp32 and unactivated, into its own plane of the workspace (a.ws, laid out like the output), and
 // k_conv_split_finish adds the planes in a fixed order and runs the epilogue.  Only the 32-channel
 // slab kernels (WN = 1) have this form.
@@ -425,8 +424,8 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   const int entry_zero = conv_args_entry_zero(a);      // every line of the argument block, fetched in one batch
   MIE_STAMP(0);
   int bx = blockIdx.x + entry_zero, by = blockIdx.y;
-  int bz = SPLIT ? (int)blockIdx.z : 0;
-  if constexpr (SPLIT) split_order(bx, by, bz);
+  int bz = 0;
+  if constexpr (SPLIT) split_order(a, bx, by, bz);
   int n, y0, x0, tk;
   if (!SPLIT && a.xcd_fs > 0) {
     const int cap = a.ts.n * a.ts.tiles_y * a.ts.tiles_x;
@@ -838,10 +837,9 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // All B loads below are unconditional: a conditional load would make the compiler's wait
   // counters conservative and collapse the prefetch distance.  After the last chunk the
   // "next chunk" pointer simply stays on the current one (a few redundant loads).
-  // SPLIT: part blockIdx.z of gridDim.z takes a contiguous range of the chunks (the host keeps
-  // gridDim.z <= nch, so no range is empty)
-  const int c_lo = SPLIT ? bz * nch / (int)gridDim.z : 0;
-  const int c_hi = SPLIT ? (bz + 1) * nch / (int)gridDim.z : nch;
+  // SPLIT: a part takes a contiguous range of the chunks (the host keeps the parts <= nch, so no range is empty)
+  const int c_lo = SPLIT ? bz * nch >> a.xcd_fs : 0;
+  const int c_hi = SPLIT ? (bz + 1) * nch >> a.xcd_fs : nch;
   const TL* ub_cur = chunk_b(c_lo);
   const TL* ub_next = ub_cur;
   MIE_STAMP(2);
@@ -1347,11 +1345,11 @@ int split_parts(ConvArgsT<T>& a, long long groups, int nch) {
     return e ? atoi(e) : 8;
   }();
   if (a.ws == nullptr || groups > max_groups || nch < 4) return 0;
-  a.xcd_fs = 0;
   a.ws_plane = (long long)a.ts.n * a.ts.h * a.ts.w * a.cout;
   int parts = 1;
   while (2 * parts <= most && 2 * parts <= nch && groups * (2 * parts) <= max_wgs && (long long)(2 * parts) * a.ws_plane <= a.ws_floats)
     parts *= 2;
+  a.xcd_fs = __builtin_ctz(parts);
   return parts < 2 ? 0 : parts;
 }
 
@@ -1375,7 +1373,7 @@ bool launch_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   ConvArgsT<T> a = a0;
   const int parts = split_parts(a, (long long)cap * (a0.cout / 32), (a0.c1 + a0.c2) / CC);
   if (parts == 0) return false;
-  const dim3 grid(cap, a.cout / 32, parts);
+  const dim3 grid(a.cout / 32 * parts, cap);
   const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
     if constexpr (HAS_X3) hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true, true>), grid, dim3(256), 0, st, a);
@@ -1406,9 +1404,9 @@ bool launch_up_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
     if constexpr (sizeof(T) == 4)
-      hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true, true>), dim3(cap, a.cout / 32, parts), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true, true>), dim3(a.cout / 32 * parts, cap), dim3(256), 0, st, a);
   } else {
-    hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true>), dim3(cap, a.cout / 32, parts), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true>), dim3(a.cout / 32 * parts, cap), dim3(256), 0, st, a);
   }
   launch_split_finish(a, cap, parts, st);
   return true;
@@ -1430,9 +1428,9 @@ bool launch_gates_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
     if constexpr (sizeof(T) == 4)
-      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true, true>), dim3(cap, a.cout / 32, parts), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true, true>), dim3(a.cout / 32 * parts, cap), dim3(256), 0, st, a);
   } else {
-    hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true>), dim3(cap, a.cout / 32, parts), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true>), dim3(a.cout / 32 * parts, cap), dim3(256), 0, st, a);
   }
   unsigned ny = (unsigned)((1024 + cap - 1) / cap);
   if (ny > (unsigned)(a.hid / 16)) ny = (unsigned)(a.hid / 16);

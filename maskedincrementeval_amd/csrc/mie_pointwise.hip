@@ -408,11 +408,16 @@ struct Up2xSet {
   TileSetDev ts; const T* a; const uint8_t* ma; T* out;
 };
 template <typename T, int VEC, bool LARGE>
-__global__ __launch_bounds__(256) void k_up2x_pair(Up2xSet<T> s0, Up2xSet<T> s1, int h_in, int w_in, int c) {
-  const Up2xSet<T>& s = blockIdx.z == 0 ? s0 : s1;
+__device__ __forceinline__ void up2x_one(const Up2xSet<T>& s, int h_in, int w_in, int c) {
   if (LARGE && mie_no_tile(s.ts, blockIdx.x)) return;
   if (LARGE && mie_masks_first(s.ts, 16 * c * (int)sizeof(T))) up2x_tile<T, VEC, false, true>(s.ts, s.a, s.ma, (const T*)nullptr, (const uint8_t*)nullptr, h_in, w_in, s.out, c);
   else up2x_tile<T, VEC, false, false>(s.ts, s.a, s.ma, (const T*)nullptr, (const uint8_t*)nullptr, h_in, w_in, s.out, c);
+}
+// (a branch and not a reference to the one or the other: through that, every field was a vector load of its own)
+template <typename T, int VEC, bool LARGE>
+__global__ __launch_bounds__(256) void k_up2x_pair(Up2xSet<T> s0, Up2xSet<T> s1, int h_in, int w_in, int c) {
+  if (blockIdx.z == 0) up2x_one<T, VEC, LARGE>(s0, h_in, w_in, c);
+  else up2x_one<T, VEC, LARGE>(s1, h_in, w_in, c);
 }
 
 // ---- max pooling increment and masked accumulate ---------------------------------

@@ -17,7 +17,7 @@
 // stride-2 OR): a block is live when any of its four output tiles is.  A live block writes all its 256
 // pixels (zeros where no input reaches, their reservoirs left alone), a stale block is zeroed, which covers every stale
 // output tile.
-// On planes of very few blocks the chunks are split over gridDim.z workgroups that write partial sums to the
+// On planes of very few blocks the chunks are split over up to 8 workgroups that write partial sums to the
 // workspace, and k_conv_split_finish (walking the OUTPUT tile set) adds them and runs the epilogue.
 #include "mie_conv_mfma_impl.h"
 #include <type_traits>
@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
   TL* const sbuf = reinterpret_cast<TL*>(smem);
 
   int n, y0, x0;                                             // block origin in INPUT coordinates
-  int bx = blockIdx.x + conv_args_entry_zero(a), by = blockIdx.y, bz = SPLIT ? (int)blockIdx.z : 0;
-  if constexpr (SPLIT) split_order(bx, by, bz);
+  int bx = blockIdx.x + conv_args_entry_zero(a), by = blockIdx.y, bz = 0;
+  if constexpr (SPLIT) split_order(a, bx, by, bz);
   const int tk = mie_pick_tile(pts, bx, n, y0, x0);
   if (tk == 0) return;
   const int tid = threadIdx.x;
@@ -192,8 +192,8 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
       bv[q] = *reinterpret_cast<const float4*>(ub + ((long long)(((qi * (K * K) + tap) * PL + q) * 2) * cout) * EPS + b_lane);
   };
 
-  const int c_lo = SPLIT ? bz * nch / (int)gridDim.z : 0;
-  const int c_hi = SPLIT ? (bz + 1) * nch / (int)gridDim.z : nch;
+  const int c_lo = SPLIT ? bz * nch >> a.xcd_fs : 0;
+  const int c_hi = SPLIT ? (bz + 1) * nch >> a.xcd_fs : nch;
   const TL* ub_cur = chunk_b(c_lo);
   const TL* ub_next = ub_cur;
   stage_load(c_lo);
@@ -348,8 +348,9 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
     while (2 * parts <= 8 && 2 * parts <= nch && groups * (2 * parts) <= 256 && (long long)(2 * parts) * a.ws_plane <= a.ws_floats)
       parts *= 2;
     if (parts >= 2) {
+      a.xcd_fs = __builtin_ctz(parts);
       const std::lock_guard<std::mutex> pair(mie_split_launches());
-      hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, true, X3>), dim3(cap_p, cout / 32, parts), dim3(256), 0, st, a, pts);
+      hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, true, X3>), dim3(cout / 32 * parts, cap_p), dim3(256), 0, st, a, pts);
       unsigned ny = (unsigned)((1024 + cap_out - 1) / cap_out);
       if (ny > (unsigned)(cout / 16)) ny = (unsigned)(cout / 16);
       if (ny < 1) ny = 1;
