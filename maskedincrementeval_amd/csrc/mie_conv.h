@@ -178,11 +178,17 @@ static __device__ __forceinline__ void conv_store_batch(const ConvArgsT<T>& a, c
 // beforehand.
 bool mie_launch_conv_mfma(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st);
 bool mie_launch_conv_mfma(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st);
-// The plain 3x3 stride-1 conv on planes of few tiles, without a workspace (mie_conv_deep.hip).  Returns false, launching nothing,
-// for other calls; mie_conv_deep_form says so beforehand (`dtype` as the caller gave it).
+// Convs on planes of few tiles, without a workspace (mie_conv_deep.hip): plain ones (3x3 stride 1, 5x5 stride 2), the gates conv of
+// a ConvLSTM and the 5x5 conv over up2x(a.x + a.x2).  They return false, launching nothing, for other calls; the _form functions say
+// so beforehand (`dtype` as the caller gave it; a gates conv: as the plain 3x3 one).
 bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype);
+bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype);
 bool mie_launch_conv_deep(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st);
 bool mie_launch_conv_deep(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st);
+bool mie_launch_gates_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);
+bool mie_launch_gates_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st);
+bool mie_launch_upconv_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);
+bool mie_launch_upconv_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st);
 // The 3x3 stride-1 conv of a ConvLSTM with the gate chain as its epilogue (a.hid > 0, a.cout = 4*hid,
 // filter columns in the gate-interleaved order of mie_conv_gates_masked).
 bool mie_launch_conv_gates_mfma(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);

@@ -650,6 +650,10 @@ extern "C" int mie_conv_needs_no_workspace(int k, int stride, int c1, int c2, in
   return mie_conv_deep_form(k, stride, c1, c2, cout, tiles, dtype) ? 1 : 0;
 }
 
+extern "C" int mie_upconv_needs_no_workspace(int c, int cout, int tiles, int dtype) {
+  return mie_upconv_deep_form(c, cout, tiles, dtype) ? 1 : 0;
+}
+
 extern "C" int mie_pack_filter(const float* filter, int cin, int k, int cout, void* packed,
                                int dtype, void* stream) {
   const char* who = "mie_pack_filter";

@@ -1,23 +1,37 @@
-// Masked 3x3 stride-1 conv on planes of few tiles: the whole contraction of an output inside one workgroup, one launch.
+// Masked convs on planes of few tiles -- 3x3 stride 1, also with the gate chain of a ConvLSTM as its epilogue, 5x5 stride 2, 5x5 over an
+// up-sampled sum -- with the whole contraction of an output inside one workgroup, in one launch.
 //
 // What bounds these layers (256 channels at 8x12 .. 32x32) is neither memory nor the matrix cores but the trips to memory one after
 // the other in a launch -- arguments, tile list, masks and pixels, sums -- and the launches themselves: the split form of
 // k_conv_mfma fills the chip with parts of the contraction and pays a second launch and a trip through memory for it.  Here
-// a workgroup is small in outputs instead: DEEP_COLS channels of ROWS rows of a tile, and its DEEP_WAVES waves share the contraction,
-// 32 channels (a chunk) a wave, with 64 or 128 channels some of the taps of a chunk.
-//   * Nothing is shared before the sums: a wave stages the window of its own chunk in its own part of the LDS, so there is no
-//     barrier until the partial sums meet there.  The window's pixels are asked for beside their mask bytes.
-//   * The filter of a wave's first chunk depends on the workgroup's number alone: it is asked for at the very start, into registers
-//     (9 taps x 3 terms x 16 bytes a lane), and arrives while the tile list, masks and pixels are on their way.  A later
-//     chunk's follow as the registers fall free.
-//   * The filter is the first operand of v_mfma_f32_16x16x32_bf16, so that a lane ends with four adjacent channels of a pixel.
+// a workgroup is small in outputs instead: DEEP_COLS channels of ROWS rows of a tile, and its DEEP_WAVES waves share the contraction:
+// NCW chunks of 32 input channels are in LDS at a time, and the taps of each are dealt out to DEEP_WAVES / NCW waves.
+//   * The filter of a wave's first chunk depends on the workgroup's number alone: it is asked for at the very start, into registers,
+//     behind the tile list's words, and arrives while list, masks and pixels are on their way.  A later chunk's follows as
+//     the registers fall free.  A workgroup's 16 columns come through a 64-byte path to its CU, 221 KB of them for 256 fp32 channels: 1.4 us.
+//   * The window's pixels are asked for beside their mask bytes.  With 8 chunks at a time a wave stages the one it multiplies
+//     itself (OWN), and nothing is shared before the sums; with fewer all waves stage, and meet.
+//   * Few chunks at a time mean few taps a wave: little filter in registers (48 of them for a 5x5 chunk dealt out to 8 waves), short code that
+//     every launch fetches anew, a second workgroup on the CU.  fp32 5x5 128->256 at 8x12 with 1, 2, 4 chunks at a time 9.7, 10.1, 15.9 us; 3x3
+//     256->256 8.0 with 2, 7.5 with 4, 6.9 with 8 of their own; at 64 channels 2 (4.5) beat 1 (4.8).
+//   * The filter is the first operand of v_mfma_f32_16x16x32_bf16, so that a lane ends with four adjacent channels of a pixel, or the
+//     four gates of a hidden channel: the gate chain runs on four times the threads it has in k_conv_mfma.
 //   * fp32 deltas as three bf16 terms (split3), the products by size in three accumulators, so that the large ones are added up
 //     among themselves: chains of 9 sums a chunk.  Error of the sums against fp64, relative 2-norm, split form -> this:
 //     256->256 1.20e-7 -> 1.07e-7, 512->512 1.90e-7 -> 1.44e-7, 64->64 1.4e-7 -> 0.8e-7.  bf16: three accumulators in turn.
-// Measured, back to back on one plane with all pixels active, split form (two launches) -> this: fp32 256->256 at 8x12 9.95 ->
-// 6.5 us, at 16x16 11.8 -> 7.5, at 16x24 11.8 -> 8.8, 512->512 at 16x16 15.9 -> 12.4, 128->128 9.2 -> 5.4, 64->64 at 16x24
-// 8.0 -> 4.7; bf16 8.0 -> 4.4, 8.8 -> 4.5, 9.2 -> 4.9, 11.4 -> 6.5, 6.4 -> 4.3, 5.7 -> 3.9.  The pass over several chunks is bound by the filter's
-// way from L2 (442 KB a workgroup for 512 fp32 channels).
+//   * Up-sampling: the sums of the source pixels in LDS, the window blended from them, as in k_conv_mfma.  fp32 layers of 256 channels are
+//     not taken: 25 taps of filter, 614 KB a workgroup, take as long as the split form (256->128 at 16x24 16.4 us, 14.6).
+// Measured back to back on one plane with all pixels active, the filter another each time, split form -> this, us:
+//                     fp32                                                    bf16
+//   3x3 256->256      8x12 15.8 -> 6.9, 16x16 15.9 -> 7.4, 24x24 14.3 -> 11.5   8.1 -> 4.5, 8.1 -> 4.6, 8.2 -> 6.2
+//   3x3 512->512      16x16 26.4 -> 14.9                                       11.3 -> 6.3
+//   3x3 64->64        32x32 8.2 -> 4.4, 64x64 8.7 -> 6.6                        5.9 -> 4.0, 6.1 -> 5.0
+//   gates 256         8x12 13.2 -> 9.7, two inputs at 16x16 28.1 -> 23.0        10.0 -> 5.0, 12.2 -> 10.0
+//   gates 128, 64     16x24 11.1 -> 8.5, 32x32 8.6 -> 6.7                       6.8 -> 5.3, 6.2 -> 5.1
+//   5x5 s2 32->64     32x48 10.3 -> 5.7, 64x64 10.9 -> 7.5                      8.1 -> 4.4, 8.2 -> 5.3
+//   5x5 s2 128->256   8x12 11.2 -> 8.6, 16x16 13.1 -> 9.8                       9.5 -> 5.2, 9.5 -> 5.5
+//   up 128->64, 64->32  32x48 13.5 -> 11.4, 64x64 15.9 -> 7.8                   11.9 -> 6.8, 8.5 -> 5.4
+// Whole passes: fp32 1x64x96 163.1 -> 147 us, 1x128x128 231 -> 215.
 #include "mie_conv_mfma_impl.h"
 
 namespace {
@@ -29,142 +43,275 @@ __device__ __forceinline__ void mma16(v4acc& acc, const float4& w, const float4&
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mie_bf16x8, w4), __builtin_bit_cast(mie_bf16x8, x4), acc, 0, 0, 0);
 }
 
-constexpr int DEEP_WAVES = 8, DEEP_COLS = 16;
+constexpr int DEEP_WAVES = 8, DEEP_COLS = 16, DEEP_THREADS = 64 * DEEP_WAVES, DEEP_WGS = 256;
+enum { DEEP_PLAIN = 0, DEEP_GATES = 1, DEEP_UP = 2 };
 
-// TPC: the waves a chunk's taps are dealt out to.  ROWS: rows of the workgroup's outputs.
-template <typename T, int TPC, int ROWS>
-__global__ __launch_bounds__(64 * DEEP_WAVES) void k_conv_deep(ConvArgsT<T> a) {
-  constexpr bool X3 = sizeof(T) == 4;
-  constexpr int K = 3, PL = X3 ? 3 : 1, GPS = X3 ? 2 : 1;
-  constexpr int CC = 32, EPS = 8, Q4 = CC / EPS, LS = CC + EPS;
-  constexpr int WX = 7 + K, WY = ROWS - 1 + K, NPIX = WX * WY;
-  constexpr int RP = row_pitch_dw(WX, LS / 2, 1) * 2, STAGE = WY * RP;      // elements: row, term plane
-  constexpr int NSLOT = NPIX * Q4, NLD = (NSLOT + 63) / 64;
-  constexpr int NCW = DEEP_WAVES / TPC, NT = (K * K + TPC - 1) / TPC;
-  constexpr int MB = ROWS * 8 / 16;
-  constexpr int OS = DEEP_COLS + 4;                                        // floats per pixel of a wave's parked sums
-  static_assert(OS * ROWS * 8 * 4 <= PL * STAGE * 2, "the sums fit where the pixels were");
-  __shared__ __attribute__((aligned(16))) mie_bf16 smem[DEEP_WAVES * PL * STAGE];
+// Sizes of a form; NCW: chunks of 32 channels in LDS at a time, ROWS: output rows of a tile.
+template <typename T, int K, int S, int NCW, int ROWS, int KIND>
+struct Deep {
+  static constexpr bool X3 = sizeof(T) == 4;
+  static constexpr int PL = X3 ? 3 : 1, GPS = X3 ? 2 : 1;      // term planes; 16-byte loads of 8 channels
+  static constexpr int CC = 32, EPS = 8, LS = CC + EPS;        // LDS elements per staged pixel of a chunk
+  static constexpr int TPC = DEEP_WAVES / NCW, NT = (K * K + TPC - 1) / TPC;
+  static constexpr int WX = 7 * S + K, WY = (ROWS - 1) * S + K, NPIX = WX * WY;
+  static constexpr int RP = row_pitch_dw(WX, LS / 2, S) * 2, STAGE = WY * RP;      // elements: row, term plane
+  static constexpr bool OWN = NCW == DEEP_WAVES && KIND != DEEP_UP;               // a wave stages its chunk itself, for itself
+  static constexpr int SPP = (OWN ? 1 : NCW) * (CC / EPS), STEP = (OWN ? 64 : DEEP_THREADS) / SPP;   // slots of 8 channels a pixel, pixels a round
+  static constexpr int NLD = (NPIX + STEP - 1) / STEP;
+  static constexpr int MB = ROWS * 8 / 16;
+  static constexpr int OS = DEEP_COLS + 4;                     // floats per pixel of a wave's parked sums
+  static constexpr int PARK = OWN ? PL * STAGE / 2 : ROWS * 8 * OS;                // floats from wave to wave (OWN: where its pixels were)
+  static_assert(PARK >= ROWS * 8 * OS, "the sums fit where the pixels were");
+  static constexpr bool UP = KIND == DEEP_UP;
+  static constexpr int SX = 8, SY = UP ? WY / 2 + 2 : 0, NLO = UP ? (SX * SY + STEP - 1) / STEP : 1;   // source pixels of a window
+  static constexpr int LOS = NCW * CC + 4;                     // floats per source pixel
+  static constexpr int WIN_B = NCW * PL * STAGE * 2, LO_B = SX * SY * LOS * 4, PARK_B = DEEP_WAVES * PARK * 4;
+  static constexpr int BYTES = WIN_B + LO_B > PARK_B ? WIN_B + LO_B : PARK_B;
+};
+
+template <typename T, int K, int S, int NCW, int ROWS, int KIND>
+__global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
+  typedef Deep<T, K, S, NCW, ROWS, KIND> D;
+  constexpr bool X3 = D::X3, UP = D::UP, GATES = KIND == DEEP_GATES, AGAIN = X3 && S == 2;
+  constexpr int PL = D::PL, GPS = D::GPS, CC = D::CC, EPS = D::EPS, LS = D::LS, TPC = D::TPC, NT = D::NT;
+  constexpr int WX = D::WX, NPIX = D::NPIX, RP = D::RP, STAGE = D::STAGE, SPP = D::SPP, STEP = D::STEP, NLD = D::NLD;
+  constexpr bool OWN = D::OWN;
+  constexpr int MB = D::MB, OS = D::OS, NLO = D::NLO, LOS = D::LOS;
+  static_assert(D::BYTES <= 160 * 1024, "LDS of a CU");
+  static_assert(!UP || (K == 5 && S == 1), "the up-sampling variant is the 5x5 stride-1 conv");
+  __shared__ __attribute__((aligned(16))) char smem[D::BYTES];
+  mie_bf16* const win = reinterpret_cast<mie_bf16*>(smem);
+  float* const s_lo = reinterpret_cast<float*>(smem + D::WIN_B);
+  float* const park = reinterpret_cast<float*>(smem);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kg = lane >> 4, l16 = lane & 15;
-  const int by = blockIdx.x + conv_args_entry_zero(a), bx = blockIdx.y;
+  // the slabs are dealt out to the XCDs in eighths: a filter slab is fetched by one of the L2s, and lines that neighbouring slabs
+  // share (a pixel's 16 channels are 32 or 64 bytes, of a gates conv 8 or 16) are written by one
+  const int slabs = a.cout / DEEP_COLS, bx = blockIdx.y;
+  int by = blockIdx.x + conv_args_entry_zero(a);
+  if ((slabs & 7) == 0) by = (by & 7) * (slabs >> 3) + (by >> 3);
   const int co0 = by * DEEP_COLS, cout = a.cout;
 
   const int cg = wave % NCW, tc = wave / NCW;
-  const int nch1 = a.c1 / CC, nch = nch1 + (a.x2 != nullptr ? a.c2 / CC : 0);
+  const int nch1 = a.c1 / CC, nch = nch1 + (!UP && a.x2 != nullptr ? a.c2 / CC : 0);
 
-  // filter of chunk c, this lane's part
-  const int w_lane = (((kg >> 1) * (K * K * PL * 2) + (kg & 1)) * cout + co0 + l16) * EPS;
-  auto chunk_w = [&](int c) -> const mie_bf16* {
-    return reinterpret_cast<const mie_bf16*>(a.filt_mc) + (long long)(c * (CC / 16)) * (K * K * PL * 2) * cout * EPS;
+  // Filter: where this wave's taps of chunk c start, and a lane's place in a term of a tap, in bytes.  Tap i of the wave to
+  // registers.
+  const unsigned w_step = 2u * cout * (2 * EPS);                // from term to term, and from the last of a tap to the next tap
+  const unsigned w_lane = (((kg >> 1) * (K * K * PL * 2) + (kg & 1)) * cout + co0 + l16) * (2 * EPS);
+  auto chunk_w = [&](int c) -> const char* {
+    return reinterpret_cast<const char*>(a.filt_mc) + ((long long)(c * (CC / 16)) * (K * K) + tc) * PL * w_step;
   };
   float4 w[NT][PL];
-  auto load_w = [&](const mie_bf16* p, int i) {
-    int tap = tc + TPC * i;
-    if (TPC > 1 && tap >= K * K) tap = K * K - 1;
+  // (The first chunk's taps from one base by a place that a lane works out for each; the later ones' bases by scalar sums, beside
+  // the matrix instructions.  The asm keeps the compiler from taking the one for the other.  fp32 256->256 at 8x12, one chunk a wave,
+  // 6.9 us, by scalar sums 7.3; 512->512 at 16x16, two, 14.8, by places of a lane 16.3.)
+  auto load_w = [&](const char* p, int i, auto first) {
+    const bool none = TPC > 1 && TPC * i + TPC > K * K && tc + TPC * i >= K * K;      // (no such tap: the last one again)
+    const unsigned at = (none ? K * K - 1 - tc : TPC * i) * PL * w_step;
 #pragma unroll
-    for (int q = 0; q < PL; ++q) w[i][q] = *reinterpret_cast<const float4*>(p + (long long)((tap * PL + q) * 2) * cout * EPS + w_lane);
+    for (int q = 0; q < PL; ++q) {
+      if constexpr (decltype(first)::value) {
+        w[i][q] = *reinterpret_cast<const float4*>(p + (w_lane + at + q * w_step));
+      } else {
+        const char* t = p + (at + q * w_step);
+        asm("" : "+s"(t));
+        w[i][q] = *reinterpret_cast<const float4*>(t + w_lane);
+      }
+    }
   };
-  if (cg < nch) {
-    const mie_bf16* p = chunk_w(cg);
+  const int pos = bx / (8 / ROWS);
+  TileAsk ask = mie_tile_ask(a.ts, pos);
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    const char* p = chunk_w(cg < nch ? cg : 0);
 #pragma unroll
-    for (int i = 0; i < NT; ++i) load_w(p, i);
+    for (int i = 0; i < NT; ++i) load_w(p, i, std::true_type());
   }
 
   int n, y0, x0;
-  const int tk = mie_pick_tile(a.ts, bx / (8 / ROWS), n, y0, x0);
+  const int tk = mie_tile_take(a.ts, pos, ask, n, y0, x0);
   y0 += ROWS * (bx % (8 / ROWS));
   const int hout = a.ts.h, wout = a.ts.w;
   if (tk == 0 || y0 >= hout) return;
 
-  // the outputs of this thread: pixel it >> 2, channels 4 * (it & 3) ... of the slab (threads of a higher number: the same again)
+  // the outputs of this thread: pixel it >> 2, channels 4 * (it & 3) ... of the slab, with GATES the four gates of one hidden
+  // channel (threads of a higher number: the same again)
   const int it = tid & (ROWS * 8 * 4 - 1);
   const int oy = y0 + (it >> 5), ox = x0 + ((it >> 2) & 7), co = co0 + 4 * (it & 3);
   const bool mine = tid < ROWS * 8 * 4 && oy < hout && ox < wout;
   const int opix = (oy < hout && ox < wout) ? (n * hout + oy) * wout + ox : 0;
   const long long off = (long long)opix * cout + co;
+  const long long ho = GATES ? (long long)opix * a.hid + co / 4 : 0;
   if (tk == 2) {
-    if (mine) mie_st4(a.out, off, make_float4(0.f, 0.f, 0.f, 0.f));
+    if (!mine) return;
+    if constexpr (GATES) {
+      mie_st(a.g_dh, ho, 0.f);
+      mie_st(a.g_dc, ho, 0.f);
+    } else {
+      mie_st4(a.out, off, make_float4(0.f, 0.f, 0.f, 0.f));
+    }
     return;
   }
 
-  // ---- the window's pixels, CC channels of them, for this wave alone
-  mie_bf16* const sw = smem + wave * (PL * STAGE);
-  int st_po[NLD], st_lds[NLD];
+  // ---- the window's pixels, NCW * CC channels of them at a time; UP: of the source block they are blended from
+  const int sq = (OWN ? lane : tid) % SPP, p0 = (OWN ? lane : tid) / SPP;
+  const int ck = OWN ? cg : sq / (CC / EPS), q8 = EPS * (sq % (CC / EPS));      // chunk of those in LDS and channel this thread stages
+  const int iy0 = y0 * S - a.pad, ix0 = x0 * S - a.pad;
+  const int h_lo = a.h_in >> 1, w_lo = a.w_in >> 1;
+  const int lo_y0 = (iy0 >> 1) - 1, lo_x0 = (ix0 >> 1) - 1;
+  constexpr int NL = UP ? NLO : NLD;
+  int st_po[NL];
   unsigned inb = 0u;
-  const int q8 = EPS * (lane & (Q4 - 1));
 #pragma unroll
-  for (int i = 0; i < NLD; ++i) {
-    const int pix = (lane + 64 * i) / Q4, ly = pix / WX, lx = pix - ly * WX;
-    const int iy = y0 - a.pad + ly, ix = x0 - a.pad + lx;
-    const bool k = pix < NPIX && iy >= 0 && iy < a.h_in && ix >= 0 && ix < a.w_in;
-    st_po[i] = k ? (n * a.h_in + iy) * a.w_in + ix : 0;
-    st_lds[i] = ly * RP + lx * LS + q8;
+  for (int i = 0; i < NL; ++i) {
+    const int pix = p0 + STEP * i;
+    const int ly = UP ? pix / D::SX : pix / WX, lx = UP ? pix % D::SX : pix - ly * WX;
+    const int iy = (UP ? lo_y0 : iy0) + ly, ix = (UP ? lo_x0 : ix0) + lx;
+    const int h = UP ? h_lo : a.h_in, wd = UP ? w_lo : a.w_in;
+    const bool k = pix < (UP ? D::SX * D::SY : NPIX) && iy >= 0 && iy < h && ix >= 0 && ix < wd;
+    st_po[i] = k ? (n * h + iy) * wd + ix : 0;
     inb |= (k ? 1u : 0u) << i;
   }
-  float4 xr[NLD][GPS];
-  auto load_x = [&](int c) {
-    const bool second = c >= nch1;
+  float4 xr[NL][GPS], xb[UP ? NL : 1][GPS];
+  auto load_x = [&](int pass) {
+    int c = pass * NCW + ck;
+    if (c >= nch) c = 0;
+    const bool second = !UP && c >= nch1;
     const T* p = second ? a.x2 : a.x;
     const int cs = second ? a.c2 : a.c1, ci0 = (second ? c - nch1 : c) * CC + q8;
 #pragma unroll
-    for (int i = 0; i < NLD; ++i)
+    for (int i = 0; i < NL; ++i)
 #pragma unroll
       for (int g = 0; g < GPS; ++g) xr[i][g] = *reinterpret_cast<const float4*>(p + (long long)st_po[i] * cs + ci0 + 4 * g);
+    if constexpr (UP) {
+      const T* pb = a.x2 != nullptr ? a.x2 : a.x;
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+#pragma unroll
+        for (int g = 0; g < GPS; ++g) xb[i][g] = *reinterpret_cast<const float4*>(pb + (long long)st_po[i] * cs + ci0 + 4 * g);
+    }
   };
-  auto store_x = [&](unsigned ok) {
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      if (64 * i + 63 >= NSLOT && lane + 64 * i >= NSLOT) continue;
-      const bool k = (ok >> i) & 1u;
+  auto kept = [](const float4& v, bool k) { return make_float4(k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f); };
+  auto put = [&](int at, const float (&f)[8]) {
+    if constexpr (X3) {
       float4 pl[3];
-      const float4 u = make_float4(k ? xr[i][0].x : 0.f, k ? xr[i][0].y : 0.f, k ? xr[i][0].z : 0.f, k ? xr[i][0].w : 0.f);
-      if constexpr (X3) {
-        const float4 v = make_float4(k ? xr[i][GPS - 1].x : 0.f, k ? xr[i][GPS - 1].y : 0.f, k ? xr[i][GPS - 1].z : 0.f, k ? xr[i][GPS - 1].w : 0.f);
-        const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-        split3(f, pl);
-      } else {
-        pl[0] = u;
-      }
+      split3(f, pl);
 #pragma unroll
-      for (int q = 0; q < PL; ++q) *reinterpret_cast<float4*>(sw + q * STAGE + st_lds[i]) = pl[q];
+      for (int q = 0; q < PL; ++q) *reinterpret_cast<float4*>(win + q * STAGE + at) = pl[q];
+    } else {
+      *reinterpret_cast<float4*>(win + at) = f32_to_slot(f, T());
     }
   };
   unsigned ok1 = 0u, ok2 = 0u;
+  const int st_c = ck * (PL * STAGE) + q8;      // this thread's place in a staged pixel
+  auto store_x = [&](int pass) {
+    const int c = pass * NCW + ck;
+    if constexpr (UP) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        const int pix = p0 + STEP * i;
+        if (pix >= D::SX * D::SY) continue;
+        const bool k1 = (ok1 >> i) & 1u, k2 = (ok2 >> i) & 1u;
+        float fa[8], fb[8];
+        const float4 a0 = kept(xr[i][0], k1), b0 = kept(xb[i][0], k2);
+        if constexpr (X3) {
+          const float4 a1 = kept(xr[i][GPS - 1], k1), b1 = kept(xb[i][GPS - 1], k2);
+          const float ta[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w}, tb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+          for (int e = 0; e < 8; ++e) fa[e] = ta[e], fb[e] = tb[e];
+        } else {
+          slot_to_f32(a0, fa, T());
+          slot_to_f32(b0, fb, T());
+        }
+        float* const d = s_lo + pix * LOS + 8 * sq;
+        *reinterpret_cast<float4*>(d) = make_float4(fa[0] + fb[0], fa[1] + fb[1], fa[2] + fb[2], fa[3] + fb[3]);
+        *reinterpret_cast<float4*>(d + 4) = make_float4(fa[4] + fb[4], fa[5] + fb[5], fa[6] + fb[6], fa[7] + fb[7]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) {
+        const int pix = p0 + STEP * i, ly = pix / WX, lx = pix - ly * WX;
+        if (pix >= NPIX) continue;
+        const int hy = iy0 + ly, hx = ix0 + lx;
+        float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (hy >= 0 && hy < a.h_in && hx >= 0 && hx < a.w_in) {
+          int r0, r1, q0, q1;
+          float lr0, lr1, lq0, lq1;
+          conv_up2x_coef(hy, h_lo, r0, r1, lr0, lr1);
+          conv_up2x_coef(hx, w_lo, q0, q1, lq0, lq1);
+          const float* v00 = s_lo + ((r0 - lo_y0) * D::SX + (q0 - lo_x0)) * LOS + 8 * sq;
+          const float* v01 = s_lo + ((r0 - lo_y0) * D::SX + (q1 - lo_x0)) * LOS + 8 * sq;
+          const float* v10 = s_lo + ((r1 - lo_y0) * D::SX + (q0 - lo_x0)) * LOS + 8 * sq;
+          const float* v11 = s_lo + ((r1 - lo_y0) * D::SX + (q1 - lo_x0)) * LOS + 8 * sq;
+#pragma unroll
+          for (int e = 0; e < 8; e += 4) {
+            const float4 t00 = *reinterpret_cast<const float4*>(v00 + e), t01 = *reinterpret_cast<const float4*>(v01 + e);
+            const float4 t10 = *reinterpret_cast<const float4*>(v10 + e), t11 = *reinterpret_cast<const float4*>(v11 + e);
+            o[e] = conv_up2x_v(lr0, lr1, conv_up2x_h(lq0, lq1, t00.x, t01.x), conv_up2x_h(lq0, lq1, t10.x, t11.x));
+            o[e + 1] = conv_up2x_v(lr0, lr1, conv_up2x_h(lq0, lq1, t00.y, t01.y), conv_up2x_h(lq0, lq1, t10.y, t11.y));
+            o[e + 2] = conv_up2x_v(lr0, lr1, conv_up2x_h(lq0, lq1, t00.z, t01.z), conv_up2x_h(lq0, lq1, t10.z, t11.z));
+            o[e + 3] = conv_up2x_v(lr0, lr1, conv_up2x_h(lq0, lq1, t00.w, t01.w), conv_up2x_h(lq0, lq1, t10.w, t11.w));
+          }
+        }
+        put(st_c + ly * RP + lx * LS, o);
+      }
+    } else {
+      const unsigned ok = c >= nch ? 0u : c >= nch1 ? ok2 : ok1;
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        const int pix = p0 + STEP * i, ly = pix / WX, lx = pix - ly * WX;
+        if (STEP * i + STEP > NPIX && pix >= NPIX) continue;
+        const bool k = (ok >> i) & 1u;
+        const float4 u = kept(xr[i][0], k);
+        if constexpr (X3) {
+          const float4 v = kept(xr[i][GPS - 1], k);
+          const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+          put(st_c + ly * RP + lx * LS, f);
+        } else {
+          *reinterpret_cast<float4*>(win + st_c + ly * RP + lx * LS) = u;
+        }
+      }
+    }
+  };
   const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
+  const uint8_t* const x2m = a.x2 != nullptr ? a.x2m : nullptr;
+  const uint8_t* const cp_m = GATES && a.g_cpd != nullptr ? a.g_cpm : nullptr;
   const long long offs[1] = {off};
   const int cos[1] = {co}, at[1] = {opix};
-  const bool oks[1] = {true};
   float4 r0[1], add[1];
-  unsigned live_b[1];
+  float g_cp = 0.f, g_cc = 0.f, g_dp = 0.f;
+  unsigned live_b[1], cp_b[1];
   {
-    unsigned b1[NLD], b2[NLD];
-    load_x(cg < nch ? cg : 0);
+    unsigned b1[NL], b2[NL];
+    load_x(0);
     mie_mask_ask(a.xm, a.filt_mc, st_po, b1);
-    mie_mask_ask(a.x2 != nullptr ? a.x2m : nullptr, a.filt_mc, st_po, b2);
+    mie_mask_ask(x2m, a.filt_mc, st_po, b2);
     mie_mask_ask(live_m, a.filt_mc, at, live_b);
-    conv_epilogue_load4<T, 1>(a, offs, oks, r0, add);
+    if constexpr (GATES) {
+      mie_mask_ask(cp_m, a.filt_mc, at, cp_b);
+      r0[0] = *reinterpret_cast<const float4*>(a.res + off);
+      g_cp = a.g_cpres[ho];
+      g_cc = a.g_cres[ho];
+      if (a.g_cpd != nullptr) g_dp = mie_ld(a.g_cpd, ho);
+    } else {
+      const bool oks[1] = {true};
+      conv_epilogue_load4<T, 1>(a, offs, oks, r0, add);
+    }
     mie_mask_asked();
     ok1 = mie_mask_take(a.xm, b1, inb);
-    ok2 = mie_mask_take(a.x2 != nullptr ? a.x2m : nullptr, b2, inb);
+    ok2 = mie_mask_take(x2m, b2, a.x2 != nullptr ? inb : 0u);
   }
 
   // ---- contraction
   v4acc acc[MB], sm[MB], sl[MB];      // fp32: products of 1, 2^-8 and 2^-16 of the largest
 #pragma unroll
   for (int b = 0; b < MB; ++b) acc[b] = v4acc{0.f, 0.f, 0.f, 0.f}, sm[b] = sl[b] = v4acc{0.f, 0.f, 0.f, 0.f};
-  const int x_lane = (l16 >> 3) * RP + (l16 & 7) * LS + EPS * kg;
-  auto chunk = [&](int c, auto more) {
+  const mie_bf16* const x_lane = win + cg * (PL * STAGE) + (l16 >> 3) * S * RP + (l16 & 7) * S * LS + EPS * kg;
+  auto chunk = [&](const char* next, auto more) {
     constexpr bool MORE = decltype(more)::value;
-    store_x(c >= nch1 ? ok2 : ok1);
-    __builtin_amdgcn_wave_barrier();
-    const mie_bf16* p = nullptr;
-    if constexpr (MORE) {
-      load_x(c + NCW);
-      p = chunk_w(c + NCW);
-    }
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int tap = tc + TPC * i;
@@ -174,7 +321,7 @@ __global__ __launch_bounds__(64 * DEEP_WAVES) void k_conv_deep(ConvArgsT<T> a) {
 #pragma unroll
         for (int b = 0; b < MB; ++b)
 #pragma unroll
-          for (int q = 0; q < PL; ++q) xv[b][q] = *reinterpret_cast<const float4*>(sw + q * STAGE + x_lane + (2 * b + ky) * RP + kx * LS);
+          for (int q = 0; q < PL; ++q) xv[b][q] = *reinterpret_cast<const float4*>(x_lane + q * STAGE + (2 * S * b + ky) * RP + kx * LS);
         if constexpr (X3) {
           auto term = [&](v4acc (&s)[MB], int tw, int tx) {
 #pragma unroll
@@ -187,67 +334,136 @@ __global__ __launch_bounds__(64 * DEEP_WAVES) void k_conv_deep(ConvArgsT<T> a) {
           for (int b = 0; b < MB; ++b) mma16(i % 3 == 0 ? acc[b] : i % 3 == 1 ? sm[b] : sl[b], w[i][0], xv[b][0]);
         }
       }
-      if constexpr (MORE) load_w(p, i);
+      if constexpr (MORE) load_w(next, i, std::false_type());
     }
-    __builtin_amdgcn_wave_barrier();
   };
-  int c = cg;
-  for (; c + NCW < nch; c += NCW) chunk(c, std::true_type());
-  if (c < nch) chunk(c, std::false_type());
+  for (int pass = 0, c = cg; pass * NCW < nch; ++pass, c += NCW) {
+    if (!OWN && pass > 0) __syncthreads();
+    store_x(pass);
+    if constexpr (OWN) __builtin_amdgcn_wave_barrier();
+    else __syncthreads();
+    if ((pass + 1) * NCW < nch) load_x(pass + 1);
+    if (c + NCW < nch) chunk(chunk_w(c + NCW), std::true_type());
+    else if (c < nch) chunk(nullptr, std::false_type());
+    if constexpr (OWN) __builtin_amdgcn_wave_barrier();
+  }
+  if constexpr (!OWN) __syncthreads();
 
-  // ---- the waves' sums meet in LDS, each in its wave's own part: pixel 16 * b + l16, channels 4 * kg ...
-  float* const park = reinterpret_cast<float*>(sw);
+  // ---- the waves' sums meet in LDS: pixel 16 * b + l16, channels 4 * kg ...
 #pragma unroll
   for (int b = 0; b < MB; ++b) {
     const v4acc s = acc[b] + (sm[b] + sl[b]);
-    *reinterpret_cast<float4*>(park + (16 * b + l16) * OS + 4 * kg) = make_float4(s[0], s[1], s[2], s[3]);
+    *reinterpret_cast<float4*>(park + wave * D::PARK + (16 * b + l16) * OS + 4 * kg) = make_float4(s[0], s[1], s[2], s[3]);
   }
   __syncthreads();
   if (!mine) return;
   float4 part[DEEP_WAVES];
 #pragma unroll
-  for (int k = 0; k < DEEP_WAVES; ++k)
-    part[k] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(smem + k * (PL * STAGE)) + (it >> 2) * OS + 4 * (it & 3));
+  for (int k = 0; k < DEEP_WAVES; ++k) part[k] = *reinterpret_cast<const float4*>(park + k * D::PARK + (it >> 2) * OS + 4 * (it & 3));
 #pragma unroll
   for (int k = 1; k < DEEP_WAVES; ++k) {
     part[0].x += part[k].x; part[0].y += part[k].y; part[0].z += part[k].z; part[0].w += part[k].w;
   }
-  const float4 sums[1] = {part[0]};
-  const bool live[1] = {mie_mask_take(live_m, live_b, 1u) != 0u};
-  conv_epilogue_store4<T, 1>(a, offs, cos, oks, sums, r0, add, live);
+  const bool on = mie_mask_take(live_m, live_b, 1u) != 0u;
+  if constexpr (GATES) {
+    const bool has_cp = a.g_cpd != nullptr && mie_mask_take(cp_m, cp_b, 1u) != 0u;
+    float dh = 0.f, dc = 0.f;
+    if (on) {
+      mie_lstm_gate_chain(r0[0].x, r0[0].y, r0[0].z, r0[0].w, part[0].x, part[0].y, part[0].z, part[0].w, g_cp, has_cp ? g_dp : 0.f, g_cc,
+                          dh, dc);
+      *reinterpret_cast<float4*>(a.res + off) = r0[0];
+      if (has_cp) a.g_cpres[ho] = g_cp;
+      a.g_cres[ho] = g_cc;
+    }
+    mie_st(a.g_dh, ho, dh);
+    mie_st(a.g_dc, ho, dc);
+  } else {
+    const float4 sums[1] = {part[0]};
+    const bool live[1] = {on};
+    const bool oks[1] = {!AGAIN || finite4(part[0])};
+    conv_epilogue_store4<T, 1>(a, offs, cos, oks, sums, r0, add, live);
+    if constexpr (AGAIN) {
+      if (__builtin_expect(__ballot(!oks[0]) != 0ull, 0))
+        if (!oks[0]) conv_quad_again<T, K, S>(conv_args_again<T>(), n, oy, ox, co);
+    }
+  }
 }
 
-template <typename T, int ROWS>
-void launch_rows(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
-  const dim3 grid(a.cout / DEEP_COLS, 8 / ROWS * cap), block(64 * DEEP_WAVES);
-  const int nch = (a.c1 + a.c2) / 32;
-  if (nch >= 8) hipLaunchKernelGGL((k_conv_deep<T, 1, ROWS>), grid, block, 0, st, a);
-  else if (nch >= 4) hipLaunchKernelGGL((k_conv_deep<T, 2, ROWS>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((k_conv_deep<T, 4, ROWS>), grid, block, 0, st, a);
+template <typename T, int K, int S, int NCW, int ROWS, int KIND>
+void launch_form(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  hipLaunchKernelGGL((k_conv_deep<T, K, S, NCW, ROWS, KIND>), dim3(a.cout / DEEP_COLS, 8 / ROWS * cap), dim3(DEEP_THREADS), 0, st, a);
 }
 
-// Two rows a workgroup while that makes one workgroup a CU at most (the filter is read twice as often: fp32 256->256 at 8x12 7.55
-// with four -> 6.50 us with two, at 16x16, 256 workgroups, 8.7 -> 7.5, at 16x24, 384, 8.8 -> 12.5).
+// Chunks in LDS at a time.
+template <typename T, int K, int S, int ROWS, int KIND>
+void launch_chunks(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  const int nch = (a.c1 + (KIND == DEEP_UP ? 0 : a.c2)) / 32;
+  if constexpr (KIND == DEEP_UP) {
+    if constexpr (sizeof(T) == 4) launch_form<T, K, S, 1, ROWS, KIND>(a, cap, st);
+    else if (ROWS < 8 && nch >= 4) launch_form<T, K, S, 4, ROWS < 8 ? ROWS : 4, KIND>(a, cap, st);
+    else launch_form<T, K, S, 2, ROWS, KIND>(a, cap, st);
+  } else if constexpr (S == 2) {
+    launch_form<T, K, S, 1, ROWS, KIND>(a, cap, st);
+  } else {
+    if (ROWS < 8 && nch >= 8) launch_form<T, K, S, 8, ROWS < 8 ? ROWS : 4, KIND>(a, cap, st);
+    else if (nch > 2) launch_form<T, K, S, 4, ROWS, KIND>(a, cap, st);
+    else launch_form<T, K, S, 2, ROWS, KIND>(a, cap, st);
+  }
+}
+
+// Workgroups of whole tiles.  The form is taken while they are one round of the chip, one a CU, and with as few rows as keep it that: two
+// beat four and these eight while there are CUs for them (fp32 256->256 at 8x12 7.4, 8.8, 11.7 us, bf16 5.2, 5.5, 6.6), and a second
+// round costs more than anything (at 16x24, 96 slabs: four rows 9.3, two 11.2; at 33x44, 480 slabs: 24.7 us, k_conv_mfma 20.7; a gates conv
+// of 64 channels at 32x48, 384: 12.1 and 8.9; 5x5 64->128 at 48x48, 288: 19.5 and 16.1).
+long long deep_slabs(long long tiles, int cout) { return tiles * (cout / DEEP_COLS); }
+
+template <typename T, int K, int S, int KIND>
+void launch_deep(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  const long long slabs = deep_slabs(cap, a.cout);
+  if (4 * slabs <= DEEP_WGS) launch_chunks<T, K, S, 2, KIND>(a, cap, st);
+  else if (2 * slabs <= DEEP_WGS) launch_chunks<T, K, S, 4, KIND>(a, cap, st);
+  else launch_chunks<T, K, S, 8, KIND>(a, cap, st);
+}
+
 template <typename T>
-bool launch_deep(const ConvArgsT<T>& a, int k, int s, unsigned cap, hipStream_t st) {
-  const int dtype = sizeof(T) == 2 ? MIE_DTYPE_BF16 : a.x3 ? MIE_DTYPE_F32_BF16X3 : MIE_DTYPE_F32;
-  if (a.ws != nullptr || !mie_conv_deep_form(k, s, a.c1, a.c2, a.cout, cap, dtype)) return false;
-  if (8 / 2 * (long long)cap * (a.cout / DEEP_COLS) <= 256) launch_rows<T, 2>(a, cap, st);
-  else launch_rows<T, 4>(a, cap, st);
+int deep_dtype(const ConvArgsT<T>& a) { return sizeof(T) == 2 ? MIE_DTYPE_BF16 : a.x3 ? MIE_DTYPE_F32_BF16X3 : MIE_DTYPE_F32; }
+
+template <typename T>
+bool deep_plain(const ConvArgsT<T>& a, int k, int s, unsigned cap, hipStream_t st) {
+  if (a.ws != nullptr || !mie_conv_deep_form(k, s, a.c1, a.c2, a.cout, cap, deep_dtype(a))) return false;
+  if (k == 5) launch_deep<T, 5, 2, DEEP_PLAIN>(a, cap, st);
+  else launch_deep<T, 3, 1, DEEP_PLAIN>(a, cap, st);
+  return true;
+}
+template <typename T>
+bool deep_gates(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  if (a.ws != nullptr || a.cout != 4 * a.hid || !mie_conv_deep_form(3, 1, a.c1, a.c2, a.cout, cap, deep_dtype(a))) return false;
+  launch_deep<T, 3, 1, DEEP_GATES>(a, cap, st);
+  return true;
+}
+template <typename T>
+bool deep_up(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  if (a.ws != nullptr || !mie_upconv_deep_form(a.c1, a.cout, cap, deep_dtype(a))) return false;
+  launch_deep<T, 5, 1, DEEP_UP>(a, cap, st);
   return true;
 }
 
 }  // namespace
 
-// From two chunks on, while the workgroups are one round of the chip: one a CU with the three terms' 129 KB of LDS and 208
-// registers, two in bf16.  (fp32 256->256 at 24x24, 288 workgroups: 14.0 us in the form of 64 columns, 15.1 in this; 128->512 at 16x24,
-// 384, 11.9 and 11.6; 256->512 at 32x32, 1024, 18.0 and 30.2.  bf16 128->256 at 32x32, 512 workgroups, 6.6 and 6.0; 256->256 at
-// 33x44, 960, 8.7 and 11.2.)
 bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype) {
-  if (k != 3 || s != 1 || (dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3)) return false;
-  if (c1 % 32 != 0 || c2 % 32 != 0 || c1 + c2 < 64 || cout % DEEP_COLS != 0) return false;
-  return 2 * tiles * (cout / DEEP_COLS) <= (dtype == MIE_DTYPE_BF16 ? 512 : 256);
+  if ((dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) || !((k == 3 && s == 1) || (k == 5 && s == 2))) return false;
+  if (c1 % 32 != 0 || c2 % 32 != 0 || c1 + c2 < (k == 3 ? 64 : 32) || cout % DEEP_COLS != 0) return false;
+  return deep_slabs(tiles, cout) <= DEEP_WGS;
+}
+// (fp32 of eight rows a workgroup: 128->64 at 64x64 17.8 us, k_upconv2x 16.1)
+bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype) {
+  if ((dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) || c % 32 != 0 || cout % DEEP_COLS != 0) return false;
+  return dtype == MIE_DTYPE_BF16 ? deep_slabs(tiles, cout) <= DEEP_WGS : 2 * deep_slabs(tiles, cout) <= DEEP_WGS && c <= 128;
 }
 
-bool mie_launch_conv_deep(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st) { return launch_deep(a, k, s, cap, st); }
-bool mie_launch_conv_deep(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st) { return launch_deep(a, k, s, cap, st); }
+bool mie_launch_conv_deep(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st) { return deep_plain(a, k, s, cap, st); }
+bool mie_launch_conv_deep(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st) { return deep_plain(a, k, s, cap, st); }
+bool mie_launch_gates_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) { return deep_gates(a, cap, st); }
+bool mie_launch_gates_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) { return deep_gates(a, cap, st); }
+bool mie_launch_upconv_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) { return deep_up(a, cap, st); }
+bool mie_launch_upconv_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) { return deep_up(a, cap, st); }

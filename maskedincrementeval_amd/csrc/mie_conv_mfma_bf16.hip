@@ -5,11 +5,11 @@ bool mie_launch_conv_mfma(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned c
   return mie_launch_conv_deep(a, k, s, cap, st) || launch_any<mie_bf16>(a, k, s, cap, st);
 }
 bool mie_launch_conv_gates_mfma(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) {
-  return mie_launch_gates_pairs(a, cap, st) || launch_gates<mie_bf16>(a, cap, st);
+  return mie_launch_gates_deep(a, cap, st) || mie_launch_gates_pairs(a, cap, st) || launch_gates<mie_bf16>(a, cap, st);
 }
 bool mie_launch_conv_up_mfma(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) {
   // 64 -> 32 channels on a large plane: the persistent kernel (mie_upconv_persist.hip)
-  return mie_launch_upconv_persist(a, cap, st) || launch_up<mie_bf16>(a, cap, st);
+  return mie_launch_upconv_deep(a, cap, st) || mie_launch_upconv_persist(a, cap, st) || launch_up<mie_bf16>(a, cap, st);
 }
 
 #ifdef MIE_WG_PROFILE

@@ -19,10 +19,10 @@ bool mie_launch_conv_mfma(const ConvArgsT<float>& a, int k, int s, unsigned cap,
   return mie_launch_conv_deep(a, k, s, cap, st) || launch_any<float>(a, k, s, cap, st);
 }
 bool mie_launch_conv_gates_mfma(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) {
-  return launch_gates<float>(a, cap, st);
+  return mie_launch_gates_deep(a, cap, st) || launch_gates<float>(a, cap, st);
 }
 bool mie_launch_conv_up_mfma(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) {
-  return launch_up<float>(a, cap, st);
+  return mie_launch_upconv_deep(a, cap, st) || launch_up<float>(a, cap, st);
 }
 
 #ifdef MIE_WG_PROFILE

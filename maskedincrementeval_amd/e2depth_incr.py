@@ -95,6 +95,8 @@ class ConvLSTMIncr(replay.Watched, nn.Module, _IncrBuffers):
     sigmoid1..3 / tanh1 / m1 / m2 / tanh2 / m3 module by module.
     """
 
+    one_launch = False       # ops.conv_gates_incr; on in a network's layers, a cell by itself leaves its parts in the workspace
+
     def __init__(self, input_size: int, hidden_size: int, kernel_size: int,
                  prev_c_res: IncrementReserve = None, fused: bool = True):
         super().__init__()
@@ -238,7 +240,7 @@ class ConvLSTMIncr(replay.Watched, nn.Module, _IncrBuffers):
             cp, cpm, _ = _unpack(prev_c_incr)
         filt, _ = self._gates_filter()
         ops.conv_gates_incr(x, pix, x2, pix2, filt, ts, self.gates_res.reservoir, cp, cpm,
-                            self.cprev_res.reservoir, self.cell_res.reservoir, dh, dc)
+                            self.cprev_res.reservoir, self.cell_res.reservoir, dh, dc, one_launch=self.one_launch)
         return [dh, ts], [dc, ts]
 
     def _forward_fused(self, input_incr, prev_h_incr, prev_c_incr):
@@ -370,6 +372,7 @@ class RecurrentConvLayerIncr(replay.Watched, nn.Module):
                                   activation, norm, fuse=fuse)
         self.recurrent_block = ConvLSTMIncr(input_size=out_channels, hidden_size=out_channels,
                                             kernel_size=3, fused=fuse)
+        self.recurrent_block.one_launch = True
 
     def forward(self, x_incr, prev_state_incr):
         x_incr = self.conv(x_incr)

@@ -411,7 +411,7 @@ class _ConvIncrMixin(_IncrBuffers):
         if not _is_gpu_delta(x):
             return None
         x = ops.as_nhwc(x)
-        if not ops.upconv2x_takes(x, self.out_channels, k, s, p, self.conv2d_weights):
+        if not ops.upconv2x_takes(x, self.out_channels, k, s, p, self.conv2d_weights, True):
             return None
         up._reset_incr(), self._reset_incr(), activation._reset_incr()
         n, _, h, w = x.shape

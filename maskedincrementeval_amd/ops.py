@@ -854,7 +854,9 @@ def upconv_masked(a, amask, b, bmask, filt, k, pad, out_ts: TileMask, out_delta,
     if reservoir is not None and reservoir.shape != out_delta.shape:
         raise ValueError("reservoir shape %s != output %s" % (tuple(reservoir.shape), tuple(out_delta.shape)))
     _ready(out_ts)
-    ws_ptr, ws_bytes = _workspace_args(workspace, c > 8 and mc_ptr is not None and out_ts.capacity * (cout // 32) <= 128, a.device)
+    small = c > 8 and mc_ptr is not None and out_ts.capacity * (cout // 32) <= 128 and workspace is None and split_enabled \
+        and not lib().mie_upconv_needs_no_workspace(c, cout, out_ts.capacity, code)
+    ws_ptr, ws_bytes = _workspace_args(workspace, small, a.device)
     check(lib().mie_upconv_masked_ws(
         nhwc_ptr(a, "a", dtype=dt), pix_ptr(amask, n, h, w, "amask"), nhwc_ptr(b, "b", dtype=dt),
         pix_ptr(bmask, n, h, w, "bmask"), c, h, w, plain.data_ptr(), mc_ptr, cin_total, k, pad, cout, out_ts.ref,
@@ -867,13 +869,14 @@ def upconv_masked(a, amask, b, bmask, filt, k, pad, out_ts: TileMask, out_delta,
 upconv2x_enabled = os.environ.get("MIE_UPCONV2X", "1") != "0"      # tuning knob, read once
 
 
-def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt) -> bool:
+def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt, refresh=False) -> bool:
     """Whether a decoder layer over `a` runs at the resolution of its inputs: upconv2x_masked has a kernel for it and is the
     faster form where all tiles are active (nnConvIncr._upconv_forward asks for that first).  It is not on planes so small that upconv_masked splits the contraction (256->128 at 16x16: 25 us against
     22, at 20x20 26 against 35), for bf16 layers of one staged chunk (64->32 at 8x240x320: 525 us against 417 in the
     persistent kernel), and where border strips and blocks filled in part undo the fewer taps: 16 for each of the four
     phases of an item against 25 for each tile, once that is more than a round of workgroups (256->128 at 8x19x23: 138
-    us against 123)."""
+    us against 123).  Nor, but for a refresh, where upconv_masked has its form for planes of few tiles (fp32 128->64 at 32x48 15.0 us
+    against 11.4, 64->32 at 64x64 10.3 against 7.8; bf16 9.8 against 6.8 and 7.4 against 5.4)."""
     n, c, h, w = a.shape
     chunk = mfma_chunk(a.dtype)
     if not (upconv2x_enabled and isinstance(filt, ConvFilter) and filt.plain.is_cuda and k == 5 and stride == 1 and pad == 2
@@ -882,6 +885,9 @@ def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt) -> bool:
             and n * c * h * w * a.element_size() < 0xffffff00):
         return False
     tiles, slabs = _lib.tile_capacity(n, 2 * h, 2 * w), cout // 32
+    code = _lib.DTYPE_BF16 if a.dtype == torch.bfloat16 else _lib.DTYPE_F32_BF16X3
+    if not refresh and lib().mie_upconv_needs_no_workspace(c, cout, tiles, code):
+        return False
     items = n * (-(-(h - 2) // 8) * -(-(w - 2) // 8) + 2 * -(-w // 32) + 2 * -(-(h - 2) // 32))
     if (c >= 4 * chunk and tiles * slabs <= 64) or (4 * items * slabs > 256 and 4 * 16 * items > 25 * tiles):
         return False
@@ -1378,9 +1384,11 @@ def gate_interleave_index(hid: int, device=None) -> torch.Tensor:
 
 
 def conv_gates_incr(x, xmask, x2, x2mask, filt: ConvFilter, out_ts: TileMask, gates_res, cprev_delta, cprev_mask,
-                    cprev_res, cell_res, h_delta, c_delta, workspace=None):
+                    cprev_res, cell_res, h_delta, c_delta, workspace=None, one_launch=False):
     """3x3 gates conv of a ConvLSTM with the gate chain as its epilogue; `filt` and `gates_res` are in the
-    gate-interleaved column order (gate_interleave_index).  workspace: as in conv_masked."""
+    gate-interleaved column order (gate_interleave_index).  workspace: as in conv_masked.  one_launch: planes that would be
+    split run in the form that needs no workspace where the library has one (256 channels at 8x12 fp32 13.2 -> 9.7 us, bf16
+    10.0 -> 5.0)."""
     n, c1, h, w = x.shape
     c2 = 0 if x2 is None else x2.shape[1]
     dt = x.dtype
@@ -1393,7 +1401,9 @@ def conv_gates_incr(x, xmask, x2, x2mask, filt: ConvFilter, out_ts: TileMask, ga
         if tuple(t.shape) != (n, hid, h, w):
             raise ValueError("%s shape %s, expected %s" % (name, tuple(t.shape), (n, hid, h, w)))
     _ready(out_ts)
-    ws_ptr, ws_bytes = _workspace_args(workspace, mc_ptr is not None and out_ts.capacity * (cout // 32) <= 128, x.device)
+    small = mc_ptr is not None and out_ts.capacity * (cout // 32) <= 128 and workspace is None and split_enabled \
+        and not (one_launch and lib().mie_conv_needs_no_workspace(3, 1, c1, c2, cout, out_ts.capacity, code))
+    ws_ptr, ws_bytes = _workspace_args(workspace, small, x.device)
     check(lib().mie_conv_gates_masked_ws(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1,
         nhwc_ptr(x2, "x2", dtype=dt), pix_ptr(x2mask, n, h, w, "x2mask"), c2, h, w,
