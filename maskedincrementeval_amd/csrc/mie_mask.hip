@@ -760,13 +760,16 @@ extern "C" int mie_build_mask_tiles_thresholded(const void* delta, int c, int dt
 // tiles.  Slots of LDS are handed out on the host by lifetime in levels.
 // Measured, both kernels together (before: one step a level, 28 words of parameters read by all 16 waves in every step, the
 // masks written between the steps, two launches): E2Depth-incr 64x96 25.8 -> 17.0 us, 264x352 37.2 -> 24.5, EVFlowNet-incr
-// 256x256 45.1 -> 23.7, 8x480x640 75.8 -> 58.6.
+// 256x256 45.1 -> 23.7, 8x480x640 75.8 -> 58.6.  (Windows over up-samplings in one level: whole passes 1x64x96 146.6 -> 144.6 us, 1x128x128
+// 220.3 -> 218.9, 1x264x352 470.5 -> 468.6.  Tried: the code of the later levels fetched during level 0 by waves that it leaves over: the first
+// level 1.2 us shorter, level 0 2.5 longer.)
 namespace {
 
 constexpr int PLAN_THREADS = 1024;
 constexpr int PLAN_WAVES = PLAN_THREADS / 64;
 constexpr int PLAN_COMPUTE_WAVES = 12;                 // of a level's bitmaps where the others write the level before it
 constexpr int PLAN_WRITE_WAVES = PLAN_WAVES - PLAN_COMPUTE_WAVES;
+constexpr int PLAN_UP_WORDS = PLAN_THREADS;            // of a plane whose window over an up-sampling is read from below that
 constexpr int PLAN_LEVEL_STEPS = 8;                    // steps of a level (not resident: at least one writing wave each)
 constexpr int PLAN_MAX_SHARES = 64;                    // workgroups per sample
 constexpr int PLAN_PIXELS_PER_SHARE = 8192;            // of the plan's largest plane
@@ -875,7 +878,7 @@ __device__ __forceinline__ uint32_t plan_valid(int w, int j) {
 
 // specialised forms of the footprint (kernel size, stride and "same" padding K / 2 at compile time)
 enum { PLAN_KEY_GENERIC = 0, PLAN_KEY_C11, PLAN_KEY_C31, PLAN_KEY_C51, PLAN_KEY_C71, PLAN_KEY_C91, PLAN_KEY_C111, PLAN_KEY_C32, PLAN_KEY_C52,
-       PLAN_KEY_C72, PLAN_KEY_C92, PLAN_KEY_UP, PLAN_KEY_T32, PLAN_KEY_T52, PLAN_KEY_ALL };
+       PLAN_KEY_C72, PLAN_KEY_C92, PLAN_KEY_UP, PLAN_KEY_UP3, PLAN_KEY_UP5, PLAN_KEY_T32, PLAN_KEY_T52, PLAN_KEY_ALL };
 constexpr int PLAN_MAX_K1 = 11, PLAN_MAX_K2 = 9;       // widest windows of stride 1 and 2 among them
 constexpr int plan_key_size(int key) {
   return key == PLAN_KEY_C31 || key == PLAN_KEY_C32 || key == PLAN_KEY_T32 ? 3 : key == PLAN_KEY_C51 || key == PLAN_KEY_C52 || key == PLAN_KEY_T52 ? 5
@@ -967,6 +970,12 @@ __device__ __forceinline__ void plan_foot_words(const PlanIn& in, int y, int j, 
       // out[2m] = in[m-1] | in[m], out[2m+1] = in[m] | in[m+1], rows and columns alike (clamping at the border adds
       // nothing: the clamped neighbour is the pixel itself)
       plan_rows<2, 3, 1, R, TWO>(in, m - 1 + e, js - 1, v);
+    } else if constexpr (KEY == PLAN_KEY_UP3) {
+      // ... and a 3x3 window over that: in[m-1 .. m+1], for both
+      plan_rows<3, 3, 0, R, TWO>(in, m - 1, js - 1, v);
+    } else if constexpr (KEY == PLAN_KEY_UP5) {
+      // ... and a 5x5 window: in[m-2 .. m+1], in[m-1 .. m+2]
+      plan_rows<4, 3, 1, R, TWO>(in, m - 2 + e, js - 1, v);
     } else {
       // transposed conv, stride 2: output 2m + e sees input m + (e + P - kk) / 2 for the taps kk with e + P - kk even:
       // K = 3: {m} for e = 0, {m, m+1} for e = 1;  K = 5: {m-1, m, m+1}, {m, m+1}
@@ -988,6 +997,9 @@ __device__ __forceinline__ void plan_foot_words(const PlanIn& in, int y, int j, 
       if constexpr (KEY == PLAN_KEY_UP) {
         ev = v[i][1] | plan_shift(vp, v[i][1], vn, -1);
         od = v[i][1] | plan_shift(vp, v[i][1], vn, 1);
+      } else if constexpr (KEY == PLAN_KEY_UP3 || KEY == PLAN_KEY_UP5) {
+        ev = od = v[i][1] | plan_shift(vp, v[i][1], vn, -1) | plan_shift(vp, v[i][1], vn, 1);
+        if (KEY == PLAN_KEY_UP5) ev |= plan_shift(vp, v[i][1], vn, -2), od |= plan_shift(vp, v[i][1], vn, 2);
       } else {
 #pragma unroll
         for (int kx = 0; kx < K; ++kx) {
@@ -1108,6 +1120,8 @@ __device__ void plan_compute(uint32_t pw, uint32_t* lds, int zero, int r, int nt
       else if (two) plan_foot_all<PLAN_KEY_UP, true, 1>(in, out, ho, wo, mw, geom, r, nthr);
       else plan_foot_all<PLAN_KEY_UP, false, 1>(in, out, ho, wo, mw, geom, r, nthr);
       break;
+    PLAN_CASE(PLAN_KEY_UP3);
+    PLAN_CASE(PLAN_KEY_UP5);
     PLAN_CASE(PLAN_KEY_T32);
     PLAN_CASE(PLAN_KEY_T52);
 #undef PLAN_CASE_R
@@ -1498,6 +1512,7 @@ struct PlanHost {
     long long words;
     int level, last;            // when its bitmap is made, and the last level that reads it (writing waves included)
     int rec;                    // the allocation its bitmap lies in
+    bool up;                    // a window over an up-sampling, read from that one's inputs
   };
   struct Alloc { long long words, off; int born, rel; };
   Step st[MAX];
@@ -1507,7 +1522,9 @@ struct PlanHost {
   long long top = 0;            // words of LDS of all bitmaps
 
   // A conv window with "same" padding over the result of a stride-1 window with "same" padding is one wider window over
-  // that one's input: read that, where the wide window has a form of its own.
+  // that one's input: read that, where the wide window has a form of its own.  So is a 3x3 or 5x5 window over a bilinear
+  // up-sampling one over what that read: a decoder layer is one level and not two, while it and the up-sampling's own set have a
+  // thread for every word (264x352: 1.1 us for 1.3 + 0.85 at a quarter of the resolution, 1.8 for 1.3 + 1.3 at half, 4.1 for 1.9 + 1.8 at the full one).
   void widen(const mie_plan_op* ops) {
     auto same = [&](const Step& s, int stride) {
       if (s.op < 0 || s.src[0] < 0) return false;
@@ -1519,8 +1536,14 @@ struct PlanHost {
       const bool one = same(s, 1);
       if (!(one || same(s, 2)) || s.src[1] >= 0) continue;
       const Step& m = st[s.src[0]];
+      if (one && (s.k == 3 || s.k == 5) && m.op >= 0 && ops[m.op].foot == MIE_FOOT_UP2X && m.src[0] >= 0 && s.words <= PLAN_UP_WORDS) {
+        s.in[0] = m.src[0];
+        s.in[1] = m.src[1];
+        s.up = true;
+        continue;
+      }
       const int k = s.k + m.k - 1;
-      if (!same(m, 1) || k > (one ? PLAN_MAX_K1 : PLAN_MAX_K2)) continue;
+      if (m.up || !same(m, 1) || k > (one ? PLAN_MAX_K1 : PLAN_MAX_K2)) continue;
       s.in[0] = m.in[0];
       s.in[1] = m.in[1];
       s.k = k;
@@ -1531,6 +1554,7 @@ struct PlanHost {
       st[i].in[0] = st[i].src[0];
       st[i].in[1] = st[i].src[1];
       st[i].k = st[i].op >= 0 ? ops[st[i].op].k : 0;
+      st[i].up = false;
     }
   }
 
@@ -1538,7 +1562,7 @@ struct PlanHost {
   long long cost(int i, const mie_plan_op* ops) const {
     if (st[i].op < 0) return 20;
     const mie_plan_op& op = ops[st[i].op];
-    const int rows = op.foot == MIE_FOOT_CONV ? st[i].k : 2, words = op.foot == MIE_FOOT_CONV && op.stride == 2 ? 4 : 3;
+    const int rows = st[i].up ? (st[i].k == 5 ? 4 : 3) : op.foot == MIE_FOOT_CONV ? st[i].k : 2, words = op.foot == MIE_FOOT_CONV && op.stride == 2 ? 4 : 3;
     return rows * words * (st[i].in[1] >= 0 ? 2 : 1) + 20;
   }
 
@@ -1871,11 +1895,12 @@ int build_mask_plan(const char* who, const mie_plan_op* ops, int n_ops, int wg_c
         p[PS_IN] = (s.in[0] < 0 ? PLAN_IN_NONE : offset(s.in[0])) | (s.in[1] < 0 ? PLAN_IN_NONE : offset(s.in[1])) << 16;
         if (s.op >= 0) {
           const mie_plan_op& op = ops[s.op];
-          h_in = op.h_in;
-          w_in = op.w_in;
+          h_in = s.up ? s.h / 2 : op.h_in;
+          w_in = s.up ? s.w / 2 : op.w_in;
           // the specialised forms have kernel size, stride and the padding k / 2 built in
           if (op.in_mask == nullptr) key = PLAN_KEY_ALL;
           else if (op.foot == MIE_FOOT_UP2X) key = PLAN_KEY_UP;
+          else if (s.up) key = s.k == 3 ? PLAN_KEY_UP3 : PLAN_KEY_UP5;
           else if (op.pad == op.k / 2) {
             const int k = s.k;
             if (op.foot == MIE_FOOT_CONV && op.stride == 1 && (k & 1) && k <= PLAN_MAX_K1) key = PLAN_KEY_C11 + k / 2;

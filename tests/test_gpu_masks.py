@@ -498,3 +498,31 @@ def test_mask_plan_holds_a_whole_unet_chain_at_full_resolution():
             assert np.array_equal(sets[name].stale_tiles().cpu().numpy(),
                                   mo.stale_list(prev_lists.get(name, np.zeros(0, dtype=np.int32)), tiles)), name
             prev_lists[name] = tiles
+
+
+# planes of one word and of one word a row more than a row, whole words, an odd number of source rows; the last plane whose
+# windows are read from below the up-sampling (1024 words), and the first that is not
+@pytest.mark.parametrize("n,h,w", [(1, 1, 1), (1, 2, 17), (2, 5, 16), (1, 33, 31), (1, 9, 70), (1, 64, 128), (1, 64, 129), (1, 128, 64)])
+def test_mask_plan_with_windows_over_an_up_sampling(n, h, w):
+    C, U = _lib.FOOT_CONV, _lib.FOOT_UP2X
+    big = (2 * h, 2 * w)
+    chain = [
+        ("u2", ("x", "y"), U, 0, 0, 0, big), ("c5", ("u2",), C, 5, 1, 2, big), ("c3", ("u2",), C, 3, 1, 1, big),
+        ("u1", ("x",), U, 0, 0, 0, big), ("d5", ("u1",), C, 5, 1, 2, big), ("d3", ("u1",), C, 3, 1, 1, big),
+        ("e", ("d3",), C, 3, 1, 1, big), ("v", ("c5", "e"), C, 1, 1, 0, big), ("p", ("u1",), C, 5, 1, 1, (2 * h - 2, 2 * w - 2)),
+    ]
+    if min(h, w) < 2:
+        chain = chain[:-1]
+    mk = lambda: {name: TileMask(n, plane[0], plane[1], DEV) for name, _, _, _, _, _, plane in chain}
+    seq, plan = mk(), mk()
+    for step, dens in enumerate((0.02, 0.0, 0.2)):
+        g = np.random.default_rng(70 + step)
+        dev = {k: _to_dev_mask((g.random((n, h, w)) < dens).astype(np.uint8)) for k in "xy"}
+        _run_chain(chain, seq, dev, n, planned=False)
+        _run_chain(chain, plan, dev, n, planned=True)
+        torch.cuda.synchronize()
+        for name, *_ in chain:
+            a, b = seq[name], plan[name]
+            na, ns = int(a.counts[0].item()), int(a.counts[1].item())
+            assert torch.equal(a.pixmask, b.pixmask) and torch.equal(a.counts, b.counts) and torch.equal(a.flags, b.flags), (step, name)
+            assert torch.equal(a.tiles[:na], b.tiles[:na]) and torch.equal(a.stale[:ns], b.stale[:ns]), (step, name)
