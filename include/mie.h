@@ -83,9 +83,9 @@ extern "C" {
  * mie_conv_f32x3_takes) and mie_tconv2x_masked / mie_tconv2x_refresh (c1, c2 multiples of 64), with filter_mc
  * packed for it; every buffer is what it is for MIE_DTYPE_F32.  Values must be finite and below the bf16
  * maximum (3.39e38): an infinity, or a value that rounds to one in bf16, splits into inf - inf and gives
- * NaN where the fp32 instruction would give an infinity -- except in convs at stride 2 on few tiles with a
- * workspace (mie_conv_masked_ws: tiles x cout/32 <= 128), which compute the outputs concerned again in fp32
- * and give what the fp32 instruction gives. */
+ * NaN where the fp32 instruction would give an infinity -- except in convs at stride 2 on few tiles, with a
+ * workspace (mie_conv_masked_ws: tiles x cout/32 <= 128) or in the form that needs none (mie_conv_needs_no_workspace), which
+ * compute the outputs concerned again in fp32 and give what the fp32 instruction gives. */
 #define MIE_DTYPE_F32_BF16X3 2
 
 /* frame kinds of mie_events_to_frame */
@@ -244,6 +244,8 @@ int mie_conv_f32x3_takes(int k, int stride, int c1, int c2, int cout);
  * Whether mie_conv_masked, without a workspace, runs a conv of this shape (matrix-core path; `tiles` = mie_tile_capacity of
  * its output, dtype with MIE_DTYPE_F32_BF16X3 where the call has it) in one launch faster than mie_conv_masked_ws runs it with one.
  * The same for mie_conv_gates_masked (k = 3, stride = 1, cout = 4 * hid) and mie_conv_gates_masked_ws.  Host logic only.
+ * With MIE_DTYPE_F32_BF16X3 it also says where that call takes a 3x3 conv of stride 2 (which mie_conv_f32x3_takes does not name:
+ * on planes of more tiles it runs on the fp32 instruction).
  */
 int mie_conv_needs_no_workspace(int k, int stride, int c1, int c2, int cout, int tiles, int dtype);
 

@@ -178,7 +178,7 @@ static __device__ __forceinline__ void conv_store_batch(const ConvArgsT<T>& a, c
 // beforehand.
 bool mie_launch_conv_mfma(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st);
 bool mie_launch_conv_mfma(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st);
-// Convs on planes of few tiles, without a workspace (mie_conv_deep.hip): plain ones (3x3 stride 1, 5x5 stride 2), the gates conv of
+// Convs on planes of few tiles, without a workspace (mie_conv_deep.hip): plain ones (3x3, 5x5 stride 2), the gates conv of
 // a ConvLSTM and the 5x5 conv over up2x(a.x + a.x2).  They return false, launching nothing, for other calls; the _form functions say
 // so beforehand (`dtype` as the caller gave it; a gates conv: as the plain 3x3 one).
 bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype);

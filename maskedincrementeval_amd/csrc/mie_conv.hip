@@ -486,7 +486,10 @@ int conv_impl(const char* who, const T* x, const uint8_t* xmask, int c1, const T
               MIE_ERR_INVALID_ARG, "%s: workspace must not alias an operand", who);
   MIE_REQUIRE(!x3 || (sizeof(T) == 4 && path != MIE_PATH_VALU), MIE_ERR_INVALID_ARG,
               "%s: MIE_DTYPE_F32_BF16X3 is a mode of the matrix-core path for fp32 deltas", who);
-  const bool mfma_ok = x3 ? (filter_mc != nullptr && cin_total % 16 == 0 && mie_conv_x3_takes(k, stride, c1, c2, cout))
+  // (3x3 stride 2: on planes of few tiles only)
+  const bool x3_deep = x3 && k == 3 && stride == 2 && workspace == nullptr &&
+                       mie_conv_deep_form(k, stride, c1, c2, cout, mie_tile_capacity(out->n, out->h, out->w), MIE_DTYPE_F32_BF16X3);
+  const bool mfma_ok = x3 ? (filter_mc != nullptr && cin_total % 16 == 0 && (x3_deep || mie_conv_x3_takes(k, stride, c1, c2, cout)))
                           : ((filter_mc != nullptr) && (cin_total % pmul == 0) &&
                              mie_conv_mfma_takes(k, stride, dtype_of<T>(), c1, c2, cout));
   MIE_REQUIRE(!x3 || mfma_ok, MIE_ERR_UNSUPPORTED,

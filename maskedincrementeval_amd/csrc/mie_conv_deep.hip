@@ -1,5 +1,5 @@
-// Masked convs on planes of few tiles -- 3x3 stride 1, also with the gate chain of a ConvLSTM as its epilogue, 5x5 stride 2, 5x5 over an
-// up-sampled sum -- with the whole contraction of an output inside one workgroup, in one launch.
+// Masked convs on planes of few tiles -- 3x3 stride 1, also with the gate chain of a ConvLSTM as its epilogue, 3x3 and 5x5 stride 2, 5x5 over
+// an up-sampled sum -- with the whole contraction of an output inside one workgroup, in one launch.
 //
 // What bounds these layers (256 channels at 8x12 .. 32x32) is neither memory nor the matrix cores but the trips to memory one after
 // the other in a launch -- arguments, tile list, masks and pixels, sums -- and the launches themselves: the split form of
@@ -30,6 +30,8 @@
 //   gates 128, 64     16x24 11.1 -> 8.5, 32x32 8.6 -> 6.7                       6.8 -> 5.3, 6.2 -> 5.1
 //   5x5 s2 32->64     32x48 10.3 -> 5.7, 64x64 10.9 -> 7.5                      8.1 -> 4.4, 8.2 -> 5.3
 //   5x5 s2 128->256   8x12 11.2 -> 8.6, 16x16 13.1 -> 9.8                       9.5 -> 5.2, 9.5 -> 5.5
+//   3x3 s2 64->128    32x32 11.6 -> 5.9 (from the fp32 instruction)              7.0 -> 4.6
+//   3x3 s2 256->512   16x16 16.1 -> 12.0                                       10.7 -> 6.1
 //   up 128->64, 64->32  32x48 13.5 -> 11.4, 64x64 15.9 -> 7.8                   11.9 -> 6.8, 8.5 -> 5.4
 // Whole passes: fp32 1x64x96 163.1 -> 147 us, 1x128x128 231 -> 215.
 #include "mie_conv_mfma_impl.h"
@@ -402,6 +404,10 @@ void launch_chunks(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
     if constexpr (sizeof(T) == 4) launch_form<T, K, S, 1, ROWS, KIND>(a, cap, st);
     else if (ROWS < 8 && nch >= 4) launch_form<T, K, S, 4, ROWS < 8 ? ROWS : 4, KIND>(a, cap, st);
     else launch_form<T, K, S, 2, ROWS, KIND>(a, cap, st);
+  } else if constexpr (S == 2 && K == 3) {
+    // (fp32 128->256 at 16x16 with 1, 2, 4: 6.7, 6.1, 6.4 us, 256->512 13.8, 12.0, 12.0; bf16 4.9, 4.7, 4.3 and 7.3, 6.5, 6.1)
+    if (sizeof(T) == 4 || nch < 4) launch_form<T, K, S, 2, ROWS, KIND>(a, cap, st);
+    else launch_form<T, K, S, sizeof(T) == 4 ? 2 : 4, ROWS, KIND>(a, cap, st);
   } else if constexpr (S == 2) {
     launch_form<T, K, S, 1, ROWS, KIND>(a, cap, st);
   } else {
@@ -432,6 +438,7 @@ template <typename T>
 bool deep_plain(const ConvArgsT<T>& a, int k, int s, unsigned cap, hipStream_t st) {
   if (a.ws != nullptr || !mie_conv_deep_form(k, s, a.c1, a.c2, a.cout, cap, deep_dtype(a))) return false;
   if (k == 5) launch_deep<T, 5, 2, DEEP_PLAIN>(a, cap, st);
+  else if (s == 2) launch_deep<T, 3, 2, DEEP_PLAIN>(a, cap, st);
   else launch_deep<T, 3, 1, DEEP_PLAIN>(a, cap, st);
   return true;
 }
@@ -451,7 +458,8 @@ bool deep_up(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
 }  // namespace
 
 bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype) {
-  if ((dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) || !((k == 3 && s == 1) || (k == 5 && s == 2))) return false;
+  if (dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) return false;
+  if (!((k == 3 && (s == 1 || s == 2)) || (k == 5 && s == 2))) return false;
   if (c1 % 32 != 0 || c2 % 32 != 0 || c1 + c2 < (k == 3 ? 64 : 32) || cout % DEEP_COLS != 0) return false;
   return deep_slabs(tiles, cout) <= DEEP_WGS;
 }

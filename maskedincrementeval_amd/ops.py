@@ -710,15 +710,15 @@ class ConvFilter:
         return sub
 
 
-def _filter_args(filt, k, dtype=torch.float32, x3_shape=None, with_code=False):
+def _filter_args(filt, k, dtype=torch.float32, x3_shape=None, with_code=False, three_term=False):
     """(plain tensor, pointer of the matrix-core copy or None) of a Tensor or ConvFilter; with_code: a third value,
     the MIE_DTYPE_* code of the call.  x3_shape = (stride, c1, c2, cout): fp32 deltas take the three-term bf16 form
-    (its filter copy, its code) where the setting (f32_matmul) and the library allow it."""
+    (its filter copy, its code) where the setting (f32_matmul) and the library allow it; three_term: so the caller has found."""
     mc = None
     code = _DTYPES.get(dtype)
     if isinstance(filt, ConvFilter):
         x3 = (x3_shape is not None and dtype == torch.float32 and filt.plain.shape[0] % 16 == 0
-              and f32x3_takes(k, *x3_shape))
+              and (three_term or f32x3_takes(k, *x3_shape)))
         filt, mc = filt.for_dtype(dtype, x3)
         if x3:
             code = _lib.DTYPE_F32_BF16X3
@@ -799,7 +799,10 @@ def conv_masked(x, xmask, x2, x2mask, filt, k, stride, pad, out_ts: TileMask, ou
     # launches the library would split over the contraction (k = 3 or 5, few tiles: see launch_split)
     small = k in (3, 5) and out_ts.capacity * (filt.shape[3] // 32) <= 128
     x3_shape = (stride, c1, c2, filt.shape[3]) if path != _lib.PATH_VALU else None
-    filt, mc_ptr, code = _filter_args(filt, k, dt, x3_shape, with_code=True)
+    # (3x3 stride 2 runs on the fp32 instruction but for planes of few tiles)
+    three_term = (k, stride) == (3, 2) and x3_shape is not None and workspace is None and f32_matmul == "bf16x3" and dt == torch.float32 \
+        and bool(lib().mie_conv_needs_no_workspace(k, stride, c1, c2, filt.shape[3], out_ts.capacity, _lib.DTYPE_F32_BF16X3))
+    filt, mc_ptr, code = _filter_args(filt, k, dt, x3_shape, with_code=True, three_term=three_term)
     cin_total, cout = filt.shape[0], filt.shape[3]
     if tuple(out_delta.shape) != (n, cout, out_ts.h, out_ts.w) or out_ts.n != n:
         raise ValueError("out_delta shape %s, expected %s" % (tuple(out_delta.shape), (n, cout, out_ts.h, out_ts.w)))

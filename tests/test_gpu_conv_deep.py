@@ -25,7 +25,9 @@ def _dev(t):
     (1, 64, 64, 512, 16, 16, 1), (1, 64, 0, 512, 16, 24, 1), (2, 64, 0, 512, 16, 16, 1), (1, 128, 0, 512, 24, 24, 1),
     (1, 64, 0, 256, 32, 32, 1), (1, 96, 64, 256, 31, 29, 1), (1, 64, 0, 256, 32, 33, 1)]] + [(5, 2) + shape for shape in [
         (1, 32, 0, 32, 1, 1, 2), (2, 64, 32, 64, 6, 5, 2), (1, 96, 0, 32, 17, 33, 1), (1, 128, 0, 256, 16, 24, 2), (1, 32, 0, 64, 127, 128, 2),
-        (1, 64, 0, 128, 64, 64, 2), (1, 32, 0, 64, 136, 128, 2)]])
+        (1, 64, 0, 128, 64, 64, 2), (1, 32, 0, 64, 136, 128, 2)]] + [(3, 2) + shape for shape in [
+        (1, 64, 0, 32, 1, 1, 1), (2, 64, 32, 64, 5, 18, 1), (1, 128, 0, 512, 15, 16, 1), (1, 256, 64, 128, 31, 29, 1), (1, 64, 0, 256, 64, 64, 1),
+        (1, 64, 32, 64, 128, 127, 0), (1, 64, 0, 256, 64, 66, 1)]])
 def test_whole_contraction_in_a_workgroup(k, s, n, c1, c2, cout, h, w, pad, dtype):
     cin, bf = c1 + c2, dtype == torch.bfloat16
     q = (lambda t: t.to(dtype).float()) if bf else (lambda t: t)
@@ -83,10 +85,11 @@ def _split_workspace():
     return torch.full((ops.SPLIT_WORKSPACE_BYTES // 4,), float("nan"), device=DEV)
 
 
-def test_infinite_deltas_pass_the_strided_form():
+@pytest.mark.parametrize("k", [3, 5])
+def test_infinite_deltas_pass_the_strided_form(k):
     # as through the split form, whose sums are taken again in fp32 where they are not finite
     c, cout, h, w = 64, 32, 9, 12
-    wt = he_normal_conv_weight(cout, c, 5, 4)
+    wt = he_normal_conv_weight(cout, c, k, 4)
     filt = ops.ConvFilter(wt.permute(1, 2, 3, 0).contiguous().to(DEV))
     x = torch.randn(1, c, h, w, generator=torch.Generator().manual_seed(1))
     x[0, 3, 4, 5], x[0, 7, 0, 0] = float("inf"), 3.4e38
@@ -95,12 +98,12 @@ def test_infinite_deltas_pass_the_strided_form():
     got = []
     for ws in (None, _split_workspace()):
         out = ops.new_nhwc(1, cout, 5, 6, DEV)
-        ops.conv_masked(_dev(x), None, None, None, filt, 5, 2, 2, ts, out, workspace=ws)
+        ops.conv_masked(_dev(x), None, None, None, filt, k, 2, k // 2, ts, out, workspace=ws)
         got.append(out.cpu())
     fin = torch.isfinite(got[1])
     assert (torch.isfinite(got[0]) == fin).all() and not fin.all() and torch.equal(got[0].isnan(), got[1].isnan())
-    ref = F.conv2d(x.double(), wt.double(), padding=2, stride=2)
-    bound = F.conv2d(x.double().abs(), wt.double().abs(), padding=2, stride=2)
+    ref = F.conv2d(x.double(), wt.double(), padding=k // 2, stride=2)
+    bound = F.conv2d(x.double().abs(), wt.double().abs(), padding=k // 2, stride=2)
     assert ((got[0].double() - ref).abs()[fin] <= (4e-7 * bound)[fin]).all()
 
 
