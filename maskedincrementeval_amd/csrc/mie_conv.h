@@ -25,7 +25,7 @@ struct ConvArgsT {
   // one plane of n*h*w*cout floats per part.  NULL: such launches are not split.
   float* ws; long long ws_floats; long long ws_plane;
   // Matrix-core path: launch order permuted per XCD (number of slab groups, 0 = plain order); set by the launchers.
-  int xcd_fs;
+  int xcd_fs; unsigned xcd_m;      // (xcd_m: mie_tile_div by the slabs of a group)
   // Matrix-core path, fp32 deltas: filt_mc is the three-term bf16 copy and the contraction runs as six bf16 products
   // per term pair (MIE_DTYPE_F32_BF16X3).
   int x3;

@@ -512,7 +512,7 @@ int conv_impl(const char* who, const T* x, const uint8_t* xmask, int c1, const T
   a.slope = slope; a.addend = addend; a.refresh = refresh ? 1 : 0; a.bias = bias;
   a.hid = 0; a.g_cpd = nullptr; a.g_cpm = nullptr; a.g_cpres = nullptr; a.g_cres = nullptr;
   a.g_dh = nullptr; a.g_dc = nullptr;
-  a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.x3 = x3 ? 1 : 0;
+  a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = x3 ? 1 : 0;
   a.ts = mie_dev_tileset(out);
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
   hipStream_t st = (hipStream_t)stream;
@@ -608,7 +608,7 @@ int tconv_impl(const char* who, const T* x, const uint8_t* xmask, int cin, int h
   a.slope = slope; a.addend = nullptr; a.refresh = refresh ? 1 : 0; a.bias = bias;
   a.hid = 0; a.g_cpd = nullptr; a.g_cpm = nullptr; a.g_cpres = nullptr; a.g_cres = nullptr;
   a.g_dh = nullptr; a.g_dc = nullptr;
-  a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.x3 = 0;
+  a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = 0;
   a.ts = mie_dev_tileset(out);
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
   if (k == 3 && stride == 2 && pad == 1 && out->h == 2 * h_in && out->w == 2 * w_in && cin <= 8 && cout % 4 == 0 &&
@@ -932,7 +932,7 @@ int upconv_entry(const char* who, const void* a_lo, const uint8_t* amask, const 
   a.slope = slope; a.addend = (const T*)addend; a.refresh = 0; a.bias = nullptr;
   a.hid = 0; a.g_cpd = nullptr; a.g_cpm = nullptr; a.g_cpres = nullptr; a.g_cres = nullptr;
   a.g_dh = nullptr; a.g_dc = nullptr;
-  a.ws = few ? nullptr : (float*)workspace; a.ws_floats = few ? 0 : workspace_bytes / 4; a.ws_plane = 0; a.xcd_fs = 0;
+  a.ws = few ? nullptr : (float*)workspace; a.ws_floats = few ? 0 : workspace_bytes / 4; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0;
   a.x3 = (x3 && !few) ? 1 : 0;
   a.ts = mie_dev_tileset(out);
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
@@ -1006,7 +1006,7 @@ static int upconv_pred_entry(const char* who, const void* filter_up, const void*
   a.slope = slope; a.addend = nullptr; a.refresh = 0; a.bias = nullptr;
   a.hid = 0; a.g_cpd = nullptr; a.g_cpm = nullptr; a.g_cpres = nullptr; a.g_cres = nullptr;
   a.g_dh = nullptr; a.g_dc = nullptr;
-  a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.x3 = 0;
+  a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = 0;
   a.ts = mie_dev_tileset(out);
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
   if (filter_up != nullptr) {

@@ -412,15 +412,15 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // (tile-list position, slab, part) of this workgroup.  Each of the 8 XCDs has an L2 of its own and the
   // hardware hands workgroups to the XCDs round robin in launch order (x fastest); with a.xcd_fs > 0 the
   // grid's x extent is a multiple of 8, so the XCD of a workgroup is blockIdx.x % 8, and the launch order
-  // is permuted.  The live (tile, slab) pairs are put in the order (slab group, tile, slab within the
-  // group) -- a.xcd_fs groups of slabs, tiles in list order, i.e. along the rows of the image -- and each
-  // XCD takes a contiguous eighth of it, in that order.  A slab of the filter then reaches 8 / xcd_fs
+  // is permuted.  The slabs are cut into a.xcd_fs groups; a group's 8 / xcd_fs XCDs take its (tile, slab) pairs in the order
+  // (tile, slab within the group), tiles in list order, i.e. along the rows of the image, each a contiguous
+  // share.  A slab of the filter then reaches 8 / xcd_fs
   // L2s instead of all 8, an input tile about xcd_fs of them, once, for all slabs of the group at a
   // time, and neighbouring tiles, which share their halo, meet in one L2 (measured on the 5x5 256->128
   // conv at 66x88: 65 -> 31 MB fetched per launch).  Active and stale tiles are dealt out separately
-  // (a stale tile costs next to nothing); the shares depend on their numbers, read from the tile set
-  // (one more dependent load at the start of a workgroup: measured, it costs nothing even on launches
-  // of a few dozen workgroups), and idle positions of the capacity-sized grid fall off the end.
+  // (a stale tile costs next to nothing); the shares depend on their numbers, read from the tile set; the list's entry is asked for
+  // together with these, as if every tile were active, and again where they are not.  Idle positions of the capacity-sized grid
+  // fall off the end.
   const int entry_zero = conv_args_entry_zero(a);      // every line of the argument block, fetched in one batch
   MIE_STAMP(0);
   int bx = blockIdx.x + entry_zero, by = blockIdx.y;
@@ -429,32 +429,24 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   int n, y0, x0, tk;
   if (!SPLIT && a.xcd_fs > 0) {
     const int cap = a.ts.n * a.ts.tiles_y * a.ts.tiles_x;
-    const int n_act = a.ts.counts[MIE_CNT_ACTIVE], n_st = a.ts.counts[MIE_CNT_STALE];
+    const int lg = __builtin_ctz(a.xcd_fs), sh = 3 - lg, up = (1 << sh) - 1;      // groups, XCDs of a group
+    const int spg = (a.cout / CO_BLK) >> lg;                 // slabs per group
+    const int xcd = bx & 7, k = xcd & up;
+    const int slot = by * ((((cap + 7) & ~7) + 16) >> 3) + (bx >> 3);             // launch order within the XCD
+    const int guess = mie_tile_div(k * ((cap * spg + up) >> sh) + slot, spg, a.xcd_m);
+    TileAsk ask = mie_tile_ask(a.ts, guess);
+    asm("" : "+s"(ask.spec), "+s"(ask.n_active), "+s"(ask.n_stale));
+    const int n_act = ask.n_active, n_st = ask.n_stale;
     if (n_act < 0 || n_st < 0 || n_act > cap || n_st > cap) return;
-    const int ns = (int)gridDim.y;
-    const int w_act = n_act * ns, w_st = n_st * ns;          // live workgroups
-    const int c_act = (w_act + 7) >> 3, c_st = (w_st + 7) >> 3;   // per XCD
-    const int xcd = bx & 7;
-    const int slot = by * ((int)gridDim.x >> 3) + (bx >> 3);      // launch order within the XCD
-    const int spg = ns / a.xcd_fs;                           // slabs per group
-    int v, tiles_of_kind;
+    const int c_act = (n_act * spg + up) >> sh, c_st = (n_st * spg + up) >> sh;   // a share
     const bool active = slot < c_act;
-    if (active) {
-      v = xcd * c_act + slot;
-      if (v >= w_act) return;
-      tiles_of_kind = n_act;
-    } else {
-      if (slot - c_act >= c_st) return;
-      v = xcd * c_st + (slot - c_act);
-      if (v >= w_st) return;
-      tiles_of_kind = n_st;
-    }
-    const int per_group = tiles_of_kind * spg;
-    const int sg = v / per_group, r = v - sg * per_group;
-    const int t = r / spg;
-    by = sg * spg + (r - t * spg);
+    const int u = active ? k * c_act + slot : k * c_st + (slot - c_act);
+    if (u >= (active ? n_act : n_st) * spg || (!active && slot - c_act >= c_st)) return;
+    const int t = mie_tile_div(u, spg, a.xcd_m);
+    by = (xcd >> sh) * spg + (u - t * spg);
     bx = active ? t : n_act + t;
-    tk = mie_pick_tile_loaded(a.ts, bx, active ? a.ts.tiles[t] : 0, n_act, n_st, n, y0, x0);
+    if (active && t != guess) ask.spec = a.ts.tiles[t];
+    tk = mie_pick_tile_loaded(a.ts, bx, ask.spec, n_act, n_st, n, y0, x0);
   } else {
     tk = mie_pick_tile(a.ts, bx, n, y0, x0);
   }
@@ -1496,6 +1488,7 @@ unsigned xcd_plan(ConvArgsT<T>& a, unsigned cap, int nslabs, int k, bool up = fa
   }
   if (forced > 0 && 8 % forced == 0 && nslabs % forced == 0) best = forced;
   a.xcd_fs = best;
+  a.xcd_m = mie_tile_magic((long long)cap * (nslabs / best), nslabs / best);
   return ((cap + 7u) & ~7u) + 16u;
 }
 

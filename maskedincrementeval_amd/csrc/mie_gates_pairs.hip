@@ -226,15 +226,15 @@ __global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
   const bool one = n_act * ns <= ONE_MOST;
   const int p_act = one ? n_act : (n_act + 1) >> 1, p_st = (n_st + 1) >> 1;
   const int w_act = p_act * ns, w_st = p_st * ns;
-  const int c_act = (w_act + 7) >> 3, c_st = (w_st + 7) >> 3;
-  const int xcd = bx & 7, slot = (int)blockIdx.y * ((int)gridDim.x >> 3) + (bx >> 3);
-  const int spg = ns / a.xcd_fs;
+  const int lg = __builtin_ctz(a.xcd_fs), sh = 3 - lg, up = (1 << sh) - 1, spg = ns >> lg;
+  const int g_act = w_act >> lg, g_st = w_st >> lg;            // of a group of slabs
+  const int c_act = (g_act + up) >> sh, c_st = (g_st + up) >> sh;
+  const int xcd = bx & 7, k = xcd & up, slot = (int)blockIdx.y * ((int)gridDim.x >> 3) + (bx >> 3);
   const bool active = slot < c_act;
-  const int v = active ? xcd * c_act + slot : xcd * c_st + (slot - c_act);
-  if (v >= (active ? w_act : w_st) || (!active && slot - c_act >= c_st)) return;
-  const int per_group = (active ? p_act : p_st) * spg;
-  const int sg = v / per_group, r0 = v - sg * per_group, pair = r0 / spg;
-  const int co0 = (sg * spg + (r0 - pair * spg)) * COLS;
+  const int v = active ? k * c_act + slot : k * c_st + (slot - c_act);
+  if (v >= (active ? g_act : g_st) || (!active && slot - c_act >= c_st)) return;
+  const int pair = mie_tile_div(v, spg, a.xcd_m);
+  const int co0 = ((xcd >> sh) * spg + (v - pair * spg)) * COLS;
   const int count = active ? n_act : n_st, at = one && active ? pair : 2 * pair;
   const int32_t* const list = active ? a.ts.tiles : a.ts.stale;
   const int tiles[2] = {list[at], list[at + 1 < count ? at + 1 : at]};
@@ -243,9 +243,9 @@ __global__ __launch_bounds__(256, 2) void k_gates_pairs(ConvArgsT<T> a) {
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     if (tiles[t] < 0 || tiles[t] >= cap) return;      // corrupt list entry: skip rather than touch memory
-    const int ty = tiles[t] / a.ts.tiles_x;
+    const int ty = mie_tile_div(tiles[t], a.ts.tiles_x, a.ts.mx);
     x0[t] = (tiles[t] - ty * a.ts.tiles_x) * MIE_TILE;
-    n[t] = ty / a.ts.tiles_y;
+    n[t] = mie_tile_div(ty, a.ts.tiles_y, a.ts.my);
     y0[t] = (ty - n[t] * a.ts.tiles_y) * MIE_TILE;
   }
   if (!active) {

@@ -336,7 +336,7 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
   constexpr int CC = X3 ? 64 : stage_channels(K, 1) * (4 / (int)sizeof(T));
   if (a0.filt_mc == nullptr || a0.c1 % CC != 0 || a0.c2 % CC != 0 || a0.cout % 32 != 0) return false;
   ConvArgsT<T> a = a0;
-  a.xcd_fs = 0;
+  a.xcd_fs = 0; a.xcd_m = 0;
   const unsigned cap_p = (unsigned)(pts.n * pts.tiles_y * pts.tiles_x);
   const unsigned cap_out = (unsigned)(a.ts.n * a.ts.tiles_y * a.ts.tiles_x);
   const int cout = a.cout;
@@ -418,7 +418,7 @@ int tconv2x_impl(const char* who, const void* x, const uint8_t* xmask, int c1, c
   a.pad = k / 2; a.cout = cout; a.out = (T*)out_delta; a.res = reservoir; a.act = act_kind; a.slope = slope;
   a.addend = (const T*)addend; a.refresh = refresh ? 1 : 0; a.bias = bias;
   a.hid = 0; a.g_cpd = nullptr; a.g_cpm = nullptr; a.g_cpres = nullptr; a.g_cres = nullptr; a.g_dh = nullptr; a.g_dc = nullptr;
-  a.ws = (float*)workspace; a.ws_floats = workspace_bytes / 4; a.ws_plane = 0; a.xcd_fs = 0; a.x3 = x3 ? 1 : 0;
+  a.ws = (float*)workspace; a.ws_floats = workspace_bytes / 4; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = x3 ? 1 : 0;
   a.ts = mie_dev_tileset(out);
   const TileSetDev pts = mie_dev_tileset(blocks);
   bool ok;

@@ -40,6 +40,8 @@ struct Up2xOrder {
   int items;                              // of a sample: the blocks, then the strips
   int combos, groups;                     // (phase, slab) pairs, and how many parts of the launch order they are cut into
   int total;                              // samples * items * combos
+  int cpg, per_group;                     // combos, and places of the order, of a group
+  unsigned m_group, m_cpg, m_items, m_bx;                  // mie_tile_div by per_group, cpg, items, blocks_x
   int nci;                                // blocks of 16 input channels in the filter
 };
 
@@ -175,11 +177,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   const int share = (od.total + 7) >> 3;
   const int v = (bid & 7) * share + (bid >> 3);
   if ((bid >> 3) >= share || v >= od.total) return;
-  const int cpg = od.combos / od.groups, per_group = a.ts.n * od.items * cpg;
-  const int cg = v / per_group, rem = v - cg * per_group;
-  const int it = rem / cpg, combo = cg * cpg + (rem - it * cpg);
+  const int cg = mie_tile_div(v, od.per_group, od.m_group), rem = v - cg * od.per_group;
+  const int it = mie_tile_div(rem, od.cpg, od.m_cpg), combo = cg * od.cpg + (rem - it * od.cpg);
   const int phase = combo & 3, slab = combo >> 2;
-  const int n = it / od.items;
+  const int n = mie_tile_div(it, od.items, od.m_items);
   const int py = phase >> 1, px = phase & 1;
   const int H = a.h_in, W = a.w_in, hout = a.ts.h, wout = a.ts.w;
   // side: 0 a block at (y0, x0), rows x cols positions; 1 .. 4 a strip at the top, bottom, left, right
@@ -188,7 +189,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
     int k = it - n * od.items;
     const int nb = od.blocks_y * od.blocks_x;
     if (k < nb) {
-      y0 = 1 + 8 * (k / od.blocks_x); x0 = 1 + 8 * (k % od.blocks_x);
+      const int by = mie_tile_div(k, od.blocks_x, od.m_bx);
+      y0 = 1 + 8 * by; x0 = 1 + 8 * (k - by * od.blocks_x);
       rows = H - 1 - y0 < 8 ? H - 1 - y0 : 8; cols = W - 1 - x0 < 8 ? W - 1 - x0 : 8;
     } else if ((k -= nb) < 2 * od.strips_x) {
       side = 1 + (k >= od.strips_x ? 1 : 0);
@@ -551,6 +553,12 @@ void launch_one(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
   od.groups = 1;
   for (int g = 2; g <= 8 && od.combos % g == 0; g *= 2)
     if (8 / g * filt + g * in < best) { best = 8 / g * filt + g * in; od.groups = g; }
+  od.cpg = od.combos / od.groups;
+  od.per_group = a.ts.n * od.items * od.cpg;
+  od.m_group = mie_tile_magic(od.total, od.per_group);
+  od.m_cpg = mie_tile_magic(od.per_group, od.cpg);
+  od.m_items = mie_tile_magic((long long)a.ts.n * od.items, od.items);
+  od.m_bx = od.blocks_x > 0 ? mie_tile_magic(od.items, od.blocks_x) : 0u;
   hipLaunchKernelGGL((k_upconv2x<T, WN>), dim3(8 * ((od.total + 7) / 8)), dim3(256), 0, st, a, od);
 }
 
