@@ -546,6 +546,19 @@ int mie_convgru_gates_incr(const void* gates_delta, float* update_res,
                            const mie_tileset* ts, int dtype, void* stream);
 
 /*
+ * The stacked gates conv of a ConvGRU whose state is reset each step (3x3, stride 1, pad 1, cin -> 2*hid channels) with
+ * mie_convgru_gates_incr as its epilogue, so that the 2*hid-channel delta is never written to memory.  Matrix-core path only,
+ * bf16 deltas or fp32 in the three-term form (MIE_DTYPE_F32_BF16X3): needs filter_mc, cin in whole staging chunks and hid % 16 == 0;
+ * otherwise MIE_ERR_UNSUPPORTED (use the two calls then).  The filter's columns are interleaved in groups of four: column 8*j + e
+ * is the update gate of hidden channel 4*j + e for e < 4, the candidate of hidden channel 4*j + e - 4 for e >= 4.  update_res,
+ * cand_res, h_delta as in mie_convgru_gates_incr, plain channel order.
+ * Replaces what mie_convgru_gates_incr does, and the two convs in front of it.
+ */
+int mie_conv_gru_masked(const void* x, const uint8_t* xmask, int cin, int h_in, int w_in, const float* filter, const void* filter_mc,
+                        int cin_total, int hid, const mie_tileset* out, float* update_res, float* cand_res, void* h_delta,
+                        int dtype, void* stream);
+
+/*
  * The gates conv of a ConvLSTM and its gate chain in ONE kernel: the 3x3,
  * stride 1, pad 1 conv of mie_conv_masked (x ++ x2 -> 4*hid channels) whose
  * epilogue is mie_convlstm_gates_incr, so that the 4*hid-channel gate delta is

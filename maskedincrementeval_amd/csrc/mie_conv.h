@@ -193,6 +193,12 @@ bool mie_launch_upconv_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStrea
 // filter columns in the gate-interleaved order of mie_conv_gates_masked).
 bool mie_launch_conv_gates_mfma(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);
 bool mie_launch_conv_gates_mfma(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st);
+// The stacked gates conv of a ConvGRU with its gate math as the epilogue (a.cout = 2 * hid, filter columns as in
+// mie_conv_gru_masked; a.res / a.g_cres: the update and candidate pre-activations, a.g_dh: the state delta).
+bool mie_launch_conv_gru(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);
+bool mie_launch_conv_gru(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st);
+bool mie_launch_gru_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);
+bool mie_launch_gru_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st);
 // The same for bf16 deltas on planes of many tiles, two of them a workgroup (mie_gates_pairs.hip).  Returns false, launching
 // nothing, for other calls.
 bool mie_launch_gates_pairs(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st);
@@ -280,6 +286,25 @@ static __device__ __forceinline__ void mie_lstm_gate_chain(float& ri, float& rf,
   ri = ri1; rf = rf1; ro = ro1; rg = rg1;
   cp += dP;
   cc = c1;
+}
+// ConvGRU with a state of zero each step, four hidden channels: update (u) and candidate (c) pre-activations and their deltas ->
+// the delta of sigmoid(u) * tanh(c) by the product rule; the pre-activations are updated.  One loop over the four, which move up a
+// place each time round: inlined once each, expf and tanhf are 5 KB (as in mie_act_n).
+static __device__ __forceinline__ float4 mie_gru_gates4(float4& u, float4& c, const float4& du, const float4& dc) {
+  float ru[4] = {u.x, u.y, u.z, u.w}, rc[4] = {c.x, c.y, c.z, c.w}, o[4] = {0.f, 0.f, 0.f, 0.f};
+  u = make_float4(u.x + du.x, u.y + du.y, u.z + du.z, u.w + du.w);
+  c = make_float4(c.x + dc.x, c.y + dc.y, c.z + dc.z, c.w + dc.w);
+  float u1[4] = {u.x, u.y, u.z, u.w}, c1[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll 1
+  for (int k = 0; k < 4; ++k) {
+    const float s0 = mie_sigm(ru[0]), ds = mie_sigm(u1[0]) - s0;
+    const float t0 = tanhf(rc[0]), dt = tanhf(c1[0]) - t0;
+    const float h = (ds + s0) * dt + t0 * ds;             // IncrPointwiseMultiply(candidate, update)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) ru[i] = ru[i + 1], rc[i] = rc[i + 1], u1[i] = u1[i + 1], c1[i] = c1[i + 1], o[i] = o[i + 1];
+    o[3] = h;
+  }
+  return make_float4(o[0], o[1], o[2], o[3]);
 }
 bool mie_conv_mfma_takes(int k, int s, int dtype, int c1, int c2, int cout);
 // The same for the three-term form of fp32 deltas (MIE_DTYPE_F32_BF16X3).

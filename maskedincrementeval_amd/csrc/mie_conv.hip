@@ -418,6 +418,7 @@ struct GatesOperands {
   int hid;
   const T* cprev_delta; const uint8_t* cprev_mask; float* cprev_res; float* cell_res;
   T* h_delta; T* c_delta;
+  bool gru;                // update_res is conv_impl's reservoir, cell_res the candidate's
 };
 
 template <typename T>
@@ -517,6 +518,13 @@ int conv_impl(const char* who, const T* x, const uint8_t* xmask, int c1, const T
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
   hipStream_t st = (hipStream_t)stream;
   if (gates != nullptr) {
+    if (gates->gru) {
+      MIE_REQUIRE(mfma_ok && cout == 2 * gates->hid && cout % 32 == 0, MIE_ERR_UNSUPPORTED,
+                  "%s: needs filter_mc, whole 32-channel (bf16: 64) input chunks and hid %% 16 == 0 (cin=%d hid=%d)", who, c1, gates->hid);
+      a.hid = gates->hid; a.g_cres = gates->cell_res; a.g_dh = gates->h_delta;
+      MIE_REQUIRE(mie_launch_conv_gru(a, cap, st), MIE_ERR_UNSUPPORTED, "%s: no kernel variant for cin=%d hid=%d", who, c1, gates->hid);
+      return mie_check_launch(who);
+    }
     MIE_REQUIRE(mfma_ok && gates->hid % 8 == 0 && cout == 4 * gates->hid, MIE_ERR_UNSUPPORTED,
                 "%s: needs filter_mc, whole 32-channel (bf16: 64) input chunks and hid %% 8 == 0 "
                 "(c1=%d c2=%d hid=%d)", who, c1, c2, gates->hid);
@@ -835,7 +843,7 @@ int conv_gates_entry(const char* who, const void* x, const uint8_t* xmask, int c
               MIE_ERR_INVALID_ARG, "%s: buffers must be 16-byte aligned", who);
   GatesOperands<T> g;
   g.hid = hid; g.cprev_delta = (const T*)cprev_delta; g.cprev_mask = cprev_mask; g.cprev_res = cprev_res;
-  g.cell_res = cell_res; g.h_delta = (T*)h_delta; g.c_delta = (T*)c_delta;
+  g.cell_res = cell_res; g.h_delta = (T*)h_delta; g.c_delta = (T*)c_delta; g.gru = false;
   return conv_impl<T>(who, (const T*)x, xmask, c1, (const T*)x2, x2mask, c2, h_in, w_in, filter,
                       (const T*)filter_mc, cin_total, 3, 1, 1, 4 * hid, out, (T*)nullptr, (const T*)nullptr,
                       gates_res, MIE_ACT_NONE, 0.f, MIE_PATH_MFMA, false, nullptr, stream, &g, workspace, workspace_bytes, x3);
@@ -1080,4 +1088,33 @@ extern "C" int mie_conv_gates_masked(const void* x, const uint8_t* xmask, int c1
   return mie_conv_gates_masked_ws(x, xmask, c1, x2, x2mask, c2, h_in, w_in, filter, filter_mc, cin_total, hid, out,
                                   gates_res, cprev_delta, cprev_mask, cprev_res, cell_res, h_delta, c_delta, dtype,
                                   nullptr, 0, stream);
+}
+
+namespace {
+template <typename T>
+int conv_gru_entry(const char* who, const void* x, const uint8_t* xmask, int cin, int h, int w, const float* filter, const void* filter_mc,
+                   int cin_total, int hid, const mie_tileset* out, float* update_res, float* cand_res, void* h_delta, void* stream, bool x3) {
+  MIE_REQUIRE(hid > 0 && hid <= (1 << 20), MIE_ERR_INVALID_ARG, "%s: hid = %d out of range", who, hid);
+  MIE_REQUIRE(update_res && cand_res && h_delta, MIE_ERR_INVALID_ARG, "%s: NULL pointer", who);
+  MIE_REQUIRE(update_res != cand_res, MIE_ERR_INVALID_ARG, "%s: the two reservoirs must be distinct", who);
+  MIE_REQUIRE(mie_aligned(update_res, 16) && mie_aligned(cand_res, 16) && mie_aligned(h_delta, 16), MIE_ERR_INVALID_ARG,
+              "%s: buffers must be 16-byte aligned", who);
+  GatesOperands<T> g = {};
+  g.hid = hid; g.cell_res = cand_res; g.h_delta = (T*)h_delta; g.gru = true;
+  return conv_impl<T>(who, (const T*)x, xmask, cin, (const T*)nullptr, nullptr, 0, h, w, filter, (const T*)filter_mc, cin_total, 3, 1, 1,
+                      2 * hid, out, (T*)nullptr, (const T*)nullptr, update_res, MIE_ACT_NONE, 0.f, MIE_PATH_MFMA, false, nullptr, stream, &g,
+                      nullptr, 0, x3);
+}
+}  // namespace
+
+extern "C" int mie_conv_gru_masked(const void* x, const uint8_t* xmask, int cin, int h_in, int w_in, const float* filter, const void* filter_mc,
+                                   int cin_total, int hid, const mie_tileset* out, float* update_res, float* cand_res, void* h_delta,
+                                   int dtype, void* stream) {
+  const char* who = "mie_conv_gru_masked";
+  bool x3 = false;
+  MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
+  if (dtype == MIE_DTYPE_BF16)
+    return conv_gru_entry<mie_bf16>(who, x, xmask, cin, h_in, w_in, filter, filter_mc, cin_total, hid, out, update_res, cand_res, h_delta, stream, false);
+  MIE_REQUIRE(x3, MIE_ERR_UNSUPPORTED, "%s: fp32 deltas in the three-term form only (MIE_DTYPE_F32_BF16X3)", who);
+  return conv_gru_entry<float>(who, x, xmask, cin, h_in, w_in, filter, filter_mc, cin_total, hid, out, update_res, cand_res, h_delta, stream, true);
 }

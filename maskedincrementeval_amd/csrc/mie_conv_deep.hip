@@ -46,7 +46,7 @@ __device__ __forceinline__ void mma16(v4acc& acc, const float4& w, const float4&
 }
 
 constexpr int DEEP_WAVES = 8, DEEP_COLS = 16, DEEP_THREADS = 64 * DEEP_WAVES, DEEP_WGS = 256;
-enum { DEEP_PLAIN = 0, DEEP_GATES = 1, DEEP_UP = 2 };
+enum { DEEP_PLAIN = 0, DEEP_GATES = 1, DEEP_UP = 2, DEEP_GRU = 3 };
 
 // Sizes of a form; NCW: chunks of 32 channels in LDS at a time, ROWS: output rows of a tile.
 template <typename T, int K, int S, int NCW, int ROWS, int KIND>
@@ -74,7 +74,7 @@ struct Deep {
 template <typename T, int K, int S, int NCW, int ROWS, int KIND>
 __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   typedef Deep<T, K, S, NCW, ROWS, KIND> D;
-  constexpr bool X3 = D::X3, UP = D::UP, GATES = KIND == DEEP_GATES, AGAIN = X3 && S == 2;
+  constexpr bool X3 = D::X3, UP = D::UP, GATES = KIND == DEEP_GATES, GRU = KIND == DEEP_GRU, AGAIN = X3 && S == 2;
   constexpr int PL = D::PL, GPS = D::GPS, CC = D::CC, EPS = D::EPS, LS = D::LS, TPC = D::TPC, NT = D::NT;
   constexpr int WX = D::WX, NPIX = D::NPIX, RP = D::RP, STAGE = D::STAGE, SPP = D::SPP, STEP = D::STEP, NLD = D::NLD;
   constexpr bool OWN = D::OWN;
@@ -146,10 +146,14 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   const bool mine = tid < ROWS * 8 * 4 && oy < hout && ox < wout;
   const int opix = (oy < hout && ox < wout) ? (n * hout + oy) * wout + ox : 0;
   const long long off = (long long)opix * cout + co;
-  const long long ho = GATES ? (long long)opix * a.hid + co / 4 : 0;
+  // (GRU: the first groups of four of every eight columns, update gates, work for the second, candidates, too)
+  const bool idle = GRU && (it & 1) != 0;
+  const long long ho = GATES ? (long long)opix * a.hid + co / 4 : GRU ? (long long)opix * a.hid + (co & ~7) / 2 : 0;
   if (tk == 2) {
-    if (!mine) return;
-    if constexpr (GATES) {
+    if (!mine || idle) return;
+    if constexpr (GRU) {
+      mie_st4(a.g_dh, ho, make_float4(0.f, 0.f, 0.f, 0.f));
+    } else if constexpr (GATES) {
       mie_st(a.g_dh, ho, 0.f);
       mie_st(a.g_dc, ho, 0.f);
     } else {
@@ -298,6 +302,9 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
       g_cp = a.g_cpres[ho];
       g_cc = a.g_cres[ho];
       if (a.g_cpd != nullptr) g_dp = mie_ld(a.g_cpd, ho);
+    } else if constexpr (GRU) {
+      r0[0] = *reinterpret_cast<const float4*>(a.res + ho);
+      add[0] = *reinterpret_cast<const float4*>(a.g_cres + ho);
     } else {
       const bool oks[1] = {true};
       conv_epilogue_load4<T, 1>(a, offs, oks, r0, add);
@@ -358,7 +365,7 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
     *reinterpret_cast<float4*>(park + wave * D::PARK + (16 * b + l16) * OS + 4 * kg) = make_float4(s[0], s[1], s[2], s[3]);
   }
   __syncthreads();
-  if (!mine) return;
+  if (!mine || idle) return;
   float4 part[DEEP_WAVES];
 #pragma unroll
   for (int k = 0; k < DEEP_WAVES; ++k) part[k] = *reinterpret_cast<const float4*>(park + k * D::PARK + (it >> 2) * OS + 4 * (it & 3));
@@ -367,7 +374,21 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
     part[0].x += part[k].x; part[0].y += part[k].y; part[0].z += part[k].z; part[0].w += part[k].w;
   }
   const bool on = mie_mask_take(live_m, live_b, 1u) != 0u;
-  if constexpr (GATES) {
+  if constexpr (GRU) {
+    float4 dc = *reinterpret_cast<const float4*>(park + (it >> 2) * OS + 4 * (it & 3) + 4);
+#pragma unroll
+    for (int k = 1; k < DEEP_WAVES; ++k) {
+      const float4 v = *reinterpret_cast<const float4*>(park + k * D::PARK + (it >> 2) * OS + 4 * (it & 3) + 4);
+      dc.x += v.x; dc.y += v.y; dc.z += v.z; dc.w += v.w;
+    }
+    float4 h = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (on) {
+      h = mie_gru_gates4(r0[0], add[0], part[0], dc);
+      *reinterpret_cast<float4*>(a.res + ho) = r0[0];
+      *reinterpret_cast<float4*>(a.g_cres + ho) = add[0];
+    }
+    mie_st4(a.g_dh, ho, h);
+  } else if constexpr (GATES) {
     const bool has_cp = a.g_cpd != nullptr && mie_mask_take(cp_m, cp_b, 1u) != 0u;
     float dh = 0.f, dc = 0.f;
     if (on) {
@@ -449,6 +470,12 @@ bool deep_gates(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
   return true;
 }
 template <typename T>
+bool deep_gru(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  if (a.cout != 2 * a.hid || !mie_conv_deep_form(3, 1, a.c1, a.c2, a.cout, cap, deep_dtype(a))) return false;
+  launch_deep<T, 3, 1, DEEP_GRU>(a, cap, st);
+  return true;
+}
+template <typename T>
 bool deep_up(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
   if (a.ws != nullptr || !mie_upconv_deep_form(a.c1, a.cout, cap, deep_dtype(a))) return false;
   launch_deep<T, 5, 1, DEEP_UP>(a, cap, st);
@@ -473,5 +500,7 @@ bool mie_launch_conv_deep(const ConvArgsT<float>& a, int k, int s, unsigned cap,
 bool mie_launch_conv_deep(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st) { return deep_plain(a, k, s, cap, st); }
 bool mie_launch_gates_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) { return deep_gates(a, cap, st); }
 bool mie_launch_gates_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) { return deep_gates(a, cap, st); }
+bool mie_launch_gru_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) { return deep_gru(a, cap, st); }
+bool mie_launch_gru_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) { return deep_gru(a, cap, st); }
 bool mie_launch_upconv_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) { return deep_up(a, cap, st); }
 bool mie_launch_upconv_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) { return deep_up(a, cap, st); }

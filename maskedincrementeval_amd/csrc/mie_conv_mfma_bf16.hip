@@ -7,6 +7,9 @@ bool mie_launch_conv_mfma(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned c
 bool mie_launch_conv_gates_mfma(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) {
   return mie_launch_gates_deep(a, cap, st) || mie_launch_gates_pairs(a, cap, st) || launch_gates<mie_bf16>(a, cap, st);
 }
+bool mie_launch_conv_gru(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) {
+  return mie_launch_gru_deep(a, cap, st) || launch_gru<mie_bf16>(a, cap, st);
+}
 bool mie_launch_conv_up_mfma(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) {
   // 64 -> 32 channels on a large plane: the persistent kernel (mie_upconv_persist.hip)
   return mie_launch_upconv_deep(a, cap, st) || mie_launch_upconv_persist(a, cap, st) || launch_up<mie_bf16>(a, cap, st);

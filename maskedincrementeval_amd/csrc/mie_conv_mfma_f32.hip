@@ -21,6 +21,9 @@ bool mie_launch_conv_mfma(const ConvArgsT<float>& a, int k, int s, unsigned cap,
 bool mie_launch_conv_gates_mfma(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) {
   return mie_launch_gates_deep(a, cap, st) || launch_gates<float>(a, cap, st);
 }
+bool mie_launch_conv_gru(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) {
+  return mie_launch_gru_deep(a, cap, st) || launch_gru<float>(a, cap, st);
+}
 bool mie_launch_conv_up_mfma(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) {
   return mie_launch_upconv_deep(a, cap, st) || launch_up<float>(a, cap, st);
 }

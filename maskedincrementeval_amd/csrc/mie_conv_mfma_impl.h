@@ -363,8 +363,10 @@ __device__ __forceinline__ void split_order(const ConvArgsT<T>& a, int& bx, int&
 // has units it is over (sub-chunk, tap class).  Global loads, masks, epilogue: fp32.
 //
 // AGAIN (X3 only): outputs whose sum is not finite are computed again in fp32 (conv_quad_again).
+// GRU (with GATES): the gate math of a ConvGRU in place of the ConvLSTM's chain; eight columns, update and candidate, to four
+// hidden channels.
 template <typename T, int K, int S, int WN, int NB, bool HALF, bool GATES = false, bool UP = false, bool SPLIT = false,
-          bool X3 = false, bool AGAIN = false>
+          bool X3 = false, bool AGAIN = false, bool GRU = false>
 // (Build with -mllvm -pragma-unroll-threshold=65536: the unit loop of the 128-column 5x5 / 7x7 kernels is 100 / 196
 // positions long, and where the compiler refuses to unroll it the operand ring is indexed at run time and lands in
 // scratch memory -- a factor of three in time.)
@@ -464,14 +466,14 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   static_assert(!SPLIT || (WN == 1 && !GATES), "the split form is a 32-channel slab kernel (the gates conv splits as a plain conv)");
   if (SPLIT && tk == 2) return;      // stale tiles are zeroed by k_conv_split_finish
   if (GATES && tk == 2) {  // stale tile: zero the hidden / cell deltas of this workgroup's hidden channels
-    constexpr int HG = CO_BLK / 16;          // groups of four hidden channels
+    constexpr int HG = CO_BLK / (GRU ? 8 : 16);          // groups of four hidden channels
     for (int idx = tid; idx < 64 * HG; idx += 256) {
       const int p = idx / HG, g4 = idx - p * HG;
       const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
       if (oy < hout && ox < wout) {
-        const long long o = (((long long)n * hout + oy) * wout + ox) * a.hid + co0 / 4 + 4 * g4;
+        const long long o = (((long long)n * hout + oy) * wout + ox) * a.hid + co0 / (GRU ? 2 : 4) + 4 * g4;
         mie_st4(a.g_dh, o, make_float4(0.f, 0.f, 0.f, 0.f));
-        mie_st4(a.g_dc, o, make_float4(0.f, 0.f, 0.f, 0.f));
+        if (!GRU) mie_st4(a.g_dc, o, make_float4(0.f, 0.f, 0.f, 0.f));
       }
     }
     return;
@@ -871,11 +873,11 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   for (int i = 0; i < (PD > 0 ? PD : 1); ++i) load_b(ub_cur, i, bring[i % RING]);
   // the output pixel mask of this thread's groups (or items of the gate chain, with their previous-cell masks): asked for
   // behind the first loads, taken behind their barrier
-  constexpr int HG = CO_BLK / 16;                            // groups of four hidden channels
+  constexpr int HG = CO_BLK / (GRU ? 8 : 16);                // groups of four hidden channels
   constexpr int PERG = (64 * HG + 255) / 256;                // items per thread (the 32-column slab has 128: half the threads idle)
   constexpr int NLIVE = GATES ? PERG : PER;
   const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
-  const uint8_t* const cp_m = GATES && a.g_cpd != nullptr ? a.g_cpm : nullptr;
+  const uint8_t* const cp_m = GATES && !GRU && a.g_cpd != nullptr ? a.g_cpm : nullptr;
   unsigned live_in = 0u, live_b[NLIVE], cp_b[NLIVE];
   if (!SPLIT) {
     int at[NLIVE];
@@ -888,7 +890,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       live_in |= (k ? 1u : 0u) << g;
     }
     mie_mask_ask(live_m, a.filt_mc, at, live_b);
-    if (GATES) mie_mask_ask(cp_m, a.filt_mc, at, cp_b);
+    if (GATES && !GRU) mie_mask_ask(cp_m, a.filt_mc, at, cp_b);
     mie_mask_asked();
   }
   // (masked pixels that the first chunk's loads fetched are zeroed here)
@@ -897,7 +899,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   __syncthreads();
   unsigned cp_bits = 0u;
   if (!SPLIT) live_bits = mie_mask_take(live_m, live_b, live_in);
-  if (GATES) cp_bits = mie_mask_take(cp_m, cp_b, a.g_cpd != nullptr ? live_bits : 0u);
+  if (GATES && !GRU) cp_bits = mie_mask_take(cp_m, cp_b, a.g_cpd != nullptr ? live_bits : 0u);
   if (!GATES && !SPLIT && EARLY) epilogue_fetch(0);
   MIE_STAMP(3);
 
@@ -1073,7 +1075,56 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[mb][nb][r] += accs[mb][nb][r];
   }
-  if constexpr (GATES) {
+  if constexpr (GRU) {
+    // Gate math of a ConvGRU: column 8 * j + e is the update gate of hidden channel 4 * j + e (e < 4) or the candidate of 4 * j + e - 4.
+    // An item is a pixel x four adjacent hidden channels: two 16-byte groups in LDS, 16 bytes of either reservoir, 16 (bf16: 8) of
+    // the state delta.  Against a conv that stores the gates' deltas and a launch that reads them again, passes of optical flow at
+    // 256x256, fp32 (four such layers; what goes is a launch and its trips to memory): 343.9 -> 326.4 and 434.8 -> 419.1 us.
+    float4 ru[PERG], rc[PERG];
+    long long ho[PERG];
+#pragma unroll
+    for (int i = 0; i < PERG; ++i) {
+      const int idx = tid + 256 * i, p = idx / HG, g4 = idx - p * HG;
+      ho[i] = (((long long)n * hout + y0 + (p >> 3)) * wout + x0 + (p & 7)) * a.hid + co0 / 2 + 4 * g4;
+      const long long at = ((live_bits >> i) & 1u) ? ho[i] : 0;
+      ru[i] = *reinterpret_cast<const float4*>(a.res + at);
+      rc[i] = *reinterpret_cast<const float4*>(a.g_cres + at);
+    }
+    float* red = smem + wk * (64 * CO_BLK);
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int p = mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          red[p * CO_BLK + wn * (32 * NB) + nb * 32 + l32] = acc[mb][nb][r];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PERG; ++i) {
+      if (!((live_in >> i) & 1u)) continue;
+      if (!((live_bits >> i) & 1u)) {
+        mie_st4(a.g_dh, ho[i], make_float4(0.f, 0.f, 0.f, 0.f));
+        continue;
+      }
+      const int idx = tid + 256 * i, p = idx / HG, g4 = idx - p * HG;
+      float4 dg[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        dg[j] = *reinterpret_cast<const float4*>(&smem[p * CO_BLK + 8 * g4 + 4 * j]);
+#pragma unroll
+        for (int k2 = 1; k2 < WK; ++k2) {
+          const float4 part = *reinterpret_cast<const float4*>(&smem[k2 * (64 * CO_BLK) + p * CO_BLK + 8 * g4 + 4 * j]);
+          dg[j].x += part.x; dg[j].y += part.y; dg[j].z += part.z; dg[j].w += part.w;
+        }
+      }
+      const float4 h = mie_gru_gates4(ru[i], rc[i], dg[0], dg[1]);
+      *reinterpret_cast<float4*>(a.res + ho[i]) = ru[i];
+      *reinterpret_cast<float4*>(a.g_cres + ho[i]) = rc[i];
+      mie_st4(a.g_dh, ho[i], h);
+    }
+  } else if constexpr (GATES) {
     // ConvLSTM gate chain as the epilogue.  The filter columns are interleaved by gate: column 4*hc + g is
     // gate g (in, remember, out, cell) of hidden channel hc, so a workgroup owns all four gates of its
     // CO_BLK/4 hidden channels.  Every wave parks its accumulators in LDS; a thread then sums the k-split
@@ -1622,6 +1673,29 @@ bool launch_gates(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
       return true;
     case 32:
       hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, true>), dim3(xcd_plan(a, cap, cout / 32, 3), cout / 32), dim3(256), 0, st, a);
+      return true;
+    default:
+      return false;
+  }
+}
+
+// The stacked gates conv of a ConvGRU, gate math in the epilogue.
+template <typename T>
+bool launch_gru(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
+  constexpr bool X3 = sizeof(T) == 4;
+  constexpr int CC = X3 ? 32 : 64;
+  ConvArgsT<T> a = a0;
+  const int cout = a.cout;
+  if ((X3 && !a.x3) || a.c1 % CC != 0 || a.c2 % CC != 0 || cout != 2 * a.hid || cout % 32 != 0) return false;
+  switch (X3 ? pick_slab_x3(cout, cap, 1) : pick_slab<3, 1, false>(cout, cap)) {
+    case 128:
+      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 4, 1, false, true, false, false, X3, false, true>), dim3(xcd_plan(a, cap, cout / 128, 3), cout / 128), dim3(256), 0, st, a);
+      return true;
+    case 64:
+      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 2, 1, false, true, false, false, X3, false, true>), dim3(xcd_plan(a, cap, cout / 64, 3), cout / 64), dim3(256), 0, st, a);
+      return true;
+    case 32:
+      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, true, false, false, X3, false, true>), dim3(xcd_plan(a, cap, cout / 32, 3), cout / 32), dim3(256), 0, st, a);
       return true;
     default:
       return false;

@@ -75,6 +75,8 @@ class nnCatIncr(replay.Watched, nn.Module, _IncrBuffers):
 class ConvGRUIncr(replay.Watched, nn.Module, _IncrBuffers):
     """Incremental ConvGRU (reference :18-96)."""
 
+    one_launch = False       # the stacked form in one kernel; on in a network's layers, a cell by itself keeps the gates' delta
+
     def __init__(self, input_size, hidden_size, kernel_size, activation=None, fuse=True, stacked=True):
         super().__init__()
         self.stacked = stacked          # with fuse: both gate convs as one conv + the gate-math kernel
@@ -106,13 +108,18 @@ class ConvGRUIncr(replay.Watched, nn.Module, _IncrBuffers):
         return act(conv(x_incr, h_incr))
 
     # -- one conv for both gates + one gate-math kernel (state reset each step) -------------------
-    def _stacked_filter(self):
-        """ConvFilter of the update-gate and out-gate filters side by side: columns [0, hid) | [hid, 2*hid)."""
+    def _stacked_filter(self, interleaved=False):
+        """ConvFilter of the update-gate and out-gate filters side by side: columns [0, hid) | [hid, 2*hid), or (interleaved) in the
+        order of ops.gru_interleave_index."""
         wu, wo = self.update_gate.weight, self.out_gate.weight
-        tag = (wu.data_ptr(), wu._version, wo.data_ptr(), wo._version, str(wu.device))
+        tag = (wu.data_ptr(), wu._version, wo.data_ptr(), wo._version, str(wu.device), interleaved)
         cached = self.__dict__.get("_stacked_filt_cache")
         if cached is None or cached[0] != tag:
-            both = torch.cat((wu.detach(), wo.detach()), 0)                    # [2*hid, cin, k, k]
+            wu, wo = wu.detach(), wo.detach()
+            if interleaved:
+                both = torch.stack([t.reshape(-1, 4, *t.shape[1:]) for t in (wu, wo)], 1).flatten(0, 2)
+            else:
+                both = torch.cat((wu, wo), 0)                                  # [2*hid, cin, k, k]
             cached = (tag, ops.ConvFilter(both.permute(1, 2, 3, 0).contiguous().float()))
             self.__dict__["_stacked_filt_cache"] = cached
         return cached[1]
@@ -127,6 +134,11 @@ class ConvGRUIncr(replay.Watched, nn.Module, _IncrBuffers):
         x, pix, _ = _unpack(input_incr)
         n, _, h, w = x.shape
         ts = conv._conv_tile_set("out_act", x, pix, None, None, k, s, p)
+        if self.one_launch and (k, s, p) == (3, 1, 1) and x.is_cuda and ops.conv_gru_takes(x.shape[1], conv.weight.shape[1],
+                                                                                           self.hidden_size, x.dtype):
+            new_state = self._delta_buf("gru_state", (n, self.hidden_size, h, w), x.device, x.dtype)
+            ops.conv_gru_incr(x, pix, self._stacked_filter(True), ts, self.sigmoid1.in_res.reservoir, self.tanh.in_res.reservoir, new_state)
+            return [new_state, ts]
         gates = self._delta_buf("gru_gates", (n, 2 * self.hidden_size, h, w), x.device, x.dtype)
         ops.conv_masked(x, pix, None, None, self._stacked_filter(), k, s, p, ts, gates)
         new_state = self._delta_buf("gru_state", (n, self.hidden_size, h, w), x.device, x.dtype)
@@ -235,6 +247,7 @@ class RecurrentConvLayerIncr(replay.Watched, nn.Module):
                                   BN_momentum=BN_momentum, fuse=fuse)
         self.recurrent_block = ConvGRUIncr(input_size=out_channels, hidden_size=out_channels,
                                            kernel_size=3, activation=activation_rec, fuse=fuse)
+        self.recurrent_block.one_launch = True
 
     def forward(self, x, prev_state):
         x = self.conv(x)

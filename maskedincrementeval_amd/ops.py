@@ -1418,6 +1418,36 @@ def conv_gates_incr(x, xmask, x2, x2mask, filt: ConvFilter, out_ts: TileMask, ga
     return h_delta, c_delta
 
 
+def gru_interleave_index(hid: int, device=None) -> torch.Tensor:
+    """Column order of conv_gru_incr's filter: entry c' = 8*j + e holds column 4*j + e of [update | candidate] x hid (e < 4: update, else
+    candidate, four further on)."""
+    cp = torch.arange(2 * hid, device=device)
+    return (cp // 4 % 2) * hid + cp // 8 * 4 + cp % 4
+
+
+def conv_gru_takes(cin: int, cin_total: int, hid: int, dtype) -> bool:
+    """Whether conv_gru_incr has a kernel for the layer (else: conv_masked + convgru_gates_incr): `cin` channels of input, a filter
+    of `cin_total`."""
+    return (hid % 16 == 0 and cin_total % 16 == 0
+            and (cin % 64 == 0 if dtype == torch.bfloat16 else dtype == torch.float32 and f32x3_takes(3, 1, cin, 0, 2 * hid)))
+
+
+def conv_gru_incr(x, xmask, filt: ConvFilter, out_ts: TileMask, update_res, cand_res, h_delta):
+    """3x3 stacked gates conv of a ConvGRU with the gate math as its epilogue; `filt` in the column order of gru_interleave_index."""
+    n, c, h, w = x.shape
+    dt = x.dtype
+    plain, mc_ptr, code = _filter_args(filt, 3, dt, (1, c, 0, filt.shape[3]), with_code=True)
+    hid = plain.shape[3] // 2
+    for name, t in (("update_res", update_res), ("cand_res", cand_res), ("h_delta", h_delta)):
+        if tuple(t.shape) != (n, hid, h, w):
+            raise ValueError("%s shape %s, expected %s" % (name, tuple(t.shape), (n, hid, h, w)))
+    _ready(out_ts)
+    check(lib().mie_conv_gru_masked(
+        nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c, h, w, plain.data_ptr(), mc_ptr, plain.shape[0], hid, out_ts.ref,
+        nhwc_ptr(update_res, "update_res"), nhwc_ptr(cand_res, "cand_res"), nhwc_ptr(h_delta, "h_delta", dtype=dt), code, _stream(x)))
+    return h_delta
+
+
 def mfma_chunk(dtype) -> int:
     """Input channels per staging chunk of the 3x3 / 5x5 stride-1 matrix-core kernels."""
     return 32 if dtype == torch.float32 else 64
@@ -1435,6 +1465,6 @@ replay.bind_ops(globals(), _pass, (
     "upconv_pred_masked", "upconv2x_masked", "upconv2x_refresh", "conv_refresh", "tconv_masked", "tconv_refresh", "tconv2x_masked", "tconv2x_refresh", "act_incr",
     "kfence_incr", "mul_incr", "add_incr", "maxpool_incr", "accumulate", "scale_incr", "avgpool_incr", "upsample2x_incr",
     "upsample2x_pair_incr", "convlstm_gates_incr", "convgru_gates_incr", "convlstm_gates_refresh",
-    "convgru_gates_refresh", "mul_dense", "conv_gates_incr", "nhwc_ptr", "pix_ptr", "as_nhwc", "pixel_mask_of"), (
+    "convgru_gates_refresh", "mul_dense", "conv_gates_incr", "conv_gru_incr", "nhwc_ptr", "pix_ptr", "as_nhwc", "pixel_mask_of"), (
     "f32_matmul", "split_enabled", "fused_plan", "fused_threshold_build", "upconv2x_enabled", "upconv_max_tiles", "upconv_max_chunks",
     "upconv_pred_enabled", "UPCONV_PRED_MIN_TILES", "UPCONV_PRED_MAX_TILES", "SPLIT_WORKSPACE_BYTES"))
