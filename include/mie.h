@@ -797,8 +797,9 @@ int mie_tconv_masked(const void* x, const uint8_t* xmask, int cin, int h_in,
  *   addend, reservoir, act_kind, slope : epilogue of mie_conv_masked (addend:
  *        e.g. the contribution of a few more input channels computed by
  *        mie_tconv_masked, covered by `out`)
- *   workspace / workspace_bytes : as in mie_conv_masked_ws (planes of very few
- *        blocks split their contraction over up to 8 workgroups); may be NULL
+ *   workspace / workspace_bytes : as in mie_conv_masked_ws (on planes of very few
+ *        blocks k = 5 and MIE_DTYPE_F32 split their contraction over up to 8
+ *        workgroups; k = 3 in the other types has no use for it); may be NULL
  * Replaces: transposed_conv2d_from_module
  * (incr_modules/mask_incr_functional.py:64-66) inside TransposedConvLayerIncr
  * (incr_modules/e2depth_incr.py:243-282).

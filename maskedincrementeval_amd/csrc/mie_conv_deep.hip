@@ -45,6 +45,14 @@ __device__ __forceinline__ void mma16(v4acc& acc, const float4& w, const float4&
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mie_bf16x8, w4), __builtin_bit_cast(mie_bf16x8, x4), acc, 0, 0, 0);
 }
 
+// A place in global memory by its type: behind an asm the compiler no longer sees where a plain pointer came from and makes flat loads
+// of it, which a wait for LDS waits for too.
+typedef const __attribute__((address_space(1))) char* GlobalBytes;
+__device__ __forceinline__ float4 global_ld4(GlobalBytes p) {
+  const v4f v = *(const __attribute__((address_space(1))) v4f*)p;
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+
 constexpr int DEEP_WAVES = 8, DEEP_COLS = 16, DEEP_THREADS = 64 * DEEP_WAVES, DEEP_WGS = 256;
 enum { DEEP_PLAIN = 0, DEEP_GATES = 1, DEEP_UP = 2, DEEP_GRU = 3 };
 
@@ -118,9 +126,9 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
       if constexpr (decltype(first)::value) {
         w[i][q] = *reinterpret_cast<const float4*>(p + (w_lane + at + q * w_step));
       } else {
-        const char* t = p + (at + q * w_step);
+        GlobalBytes t = (GlobalBytes)p + (at + q * w_step);
         asm("" : "+s"(t));
-        w[i][q] = *reinterpret_cast<const float4*>(t + w_lane);
+        w[i][q] = global_ld4(t + w_lane);
       }
     }
   };
@@ -438,6 +446,232 @@ void launch_chunks(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
   }
 }
 
+// ---- the stride-2 transposed conv (3x3, pad 1, the output twice the input; phases and block tile set as in mie_tconv_mfma.hip) ----
+// A workgroup takes ROWS x 8 input positions of a block, i.e. 2 * ROWS x 16 output pixels, times 16 columns; each of the waves a
+// chunk of 32 channels in eight, which it stages itself, all nine taps: a tap's phase is then known at compile time, and a staged
+// pixel is read once for each of the four shifts instead of for nine taps.  Bound by the serial trips and by the filter, which
+// every workgroup of a slab fetches for itself.  In place of a split launch and its finish, us per layer (graph of 24, filters cold):
+//                                   fp32             bf16
+//   256+256->256 from 16x16      16.4 -> 10.4     13.5 -> 5.2
+//   128+128->128 from 32x32      16.1 -> 9.0      13.4 -> 6.2
+//   128+128->64 from 64x64       20.7 -> 17.0     14.9 -> 10.4   (two rounds of the chip)
+// Whole pass of optical flow, 1x256x256 fp32, transposed decoder: 334.0 -> 314.3 us, with the two-round shapes 312.1.
+template <typename T, int ROWS>
+__global__ __launch_bounds__(DEEP_THREADS) void k_tconv_deep(ConvArgsT<T> a, TileSetDev pts) {
+  constexpr bool X3 = sizeof(T) == 4;
+  constexpr int PL = X3 ? 3 : 1, GPS = X3 ? 2 : 1, CC = 32, EPS = 8, LS = CC + EPS;
+  constexpr int WX = 9, WY = ROWS + 1, NPIX = WX * WY, RP = row_pitch_dw(WX, LS / 2, 1) * 2, STAGE = WY * RP;
+  constexpr int SPP = CC / EPS, STEP = 64 / SPP, NLD = (NPIX + STEP - 1) / STEP, MB = ROWS / 2, OS = DEEP_COLS + 4;
+  constexpr int SUMS = 4 * ROWS * 8 * OS, OWN = PL * STAGE / 2 > SUMS ? PL * STAGE / 2 : SUMS;      // floats of a wave: its pixels, then its sums
+  constexpr int ITEMS = 4 * ROWS * 8 * (DEEP_COLS / 4);
+  static_assert(OWN * 4 * DEEP_WAVES <= 160 * 1024 && ITEMS <= DEEP_THREADS && OWN % 4 == 0, "LDS of a CU, an item a thread");
+  __shared__ __attribute__((aligned(16))) float smem[OWN * DEEP_WAVES];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = lane >> 4, l16 = lane & 15;
+  mie_bf16* const win = reinterpret_cast<mie_bf16*>(smem + wave * OWN);
+  const int slabs = a.cout / DEEP_COLS, bx = blockIdx.y;
+  int by = blockIdx.x + conv_args_entry_zero(a);
+  if ((slabs & 7) == 0) by = (by & 7) * (slabs >> 3) + (by >> 3);      // (as in k_conv_deep)
+  const int co0 = by * DEEP_COLS, cout = a.cout;
+  const int nch1 = a.c1 / CC, nch = nch1 + (a.x2 != nullptr ? a.c2 / CC : 0);
+
+  const unsigned w_step = 2u * cout * (2 * EPS);
+  const unsigned w_lane = (((kg >> 1) * (9 * PL * 2) + (kg & 1)) * cout + co0 + l16) * (2 * EPS);
+  auto chunk_w = [&](int c) -> const char* { return reinterpret_cast<const char*>(a.filt_mc) + (long long)(c * (CC / 16)) * 9 * PL * w_step; };
+  // Taps in the order of their shifts (a direction's tap 0: phase 1 from the next pixel, 1: phase 0, 2: phase 1).  fp32 of four rows
+  // has registers for RING of them beside its sums (with all nine it kept 130 in scratch memory).
+  constexpr int RING = X3 && ROWS == 4 ? 3 : 9;
+  constexpr int TAPS[9] = {0, 1, 2, 3, 6, 4, 5, 7, 8};
+  float4 w[RING][PL];
+  auto load_w = [&](const char* p, int j, auto first) {      // (first chunk, later ones: as in k_conv_deep)
+#pragma unroll
+    for (int q = 0; q < PL; ++q) {
+      if constexpr (decltype(first)::value) {
+        w[j % RING][q] = *reinterpret_cast<const float4*>(p + (w_lane + (TAPS[j] * PL + q) * w_step));
+      } else {
+        GlobalBytes t = (GlobalBytes)p + (TAPS[j] * PL + q) * w_step;
+        asm("" : "+s"(t));
+        w[j % RING][q] = global_ld4(t + w_lane);
+      }
+    }
+  };
+  const int pos = bx / (8 / ROWS);
+  TileAsk ask = mie_tile_ask(pts, pos);
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    const char* p = chunk_w(wave < nch ? wave : 0);
+#pragma unroll
+    for (int i = 0; i < RING; ++i) load_w(p, i, std::true_type());
+  }
+  int n, y0, x0;      // in input pixels
+  const int tk = mie_tile_take(pts, pos, ask, n, y0, x0);
+  y0 += ROWS * (bx % (8 / ROWS));
+  const int hout = a.ts.h, wout = a.ts.w;
+  if (tk == 0 || y0 >= a.h_in) return;
+
+  // the output of this thread: pixel it >> 2 of the 2 * ROWS x 16, channels 4 * (it & 3) ... of the slab
+  const int it = tid & (ITEMS - 1), ly = it >> 6, lx = (it >> 2) & 15;
+  const int oy = 2 * y0 + ly, ox = 2 * x0 + lx, co = co0 + 4 * (it & 3);
+  const bool in = oy < hout && ox < wout, mine = tid < ITEMS && in;
+  const int opix = in ? (n * hout + oy) * wout + ox : 0;
+  const long long off = (long long)opix * cout + co;
+  if (tk == 2) {
+    if (mine) mie_st4(a.out, off, make_float4(0.f, 0.f, 0.f, 0.f));
+    return;
+  }
+
+  const int q8 = EPS * (lane % SPP), p0 = lane / SPP;
+  int st_po[NLD];
+  unsigned inb = 0u;
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) {
+    const int pix = p0 + STEP * i, py = pix / WX, iy = y0 + py, ix = x0 + pix - py * WX;
+    const bool k = pix < NPIX && iy < a.h_in && ix < a.w_in;
+    st_po[i] = k ? (n * a.h_in + iy) * a.w_in + ix : 0;
+    inb |= (k ? 1u : 0u) << i;
+  }
+  float4 xr[NLD][GPS];
+  auto load_x = [&](int c) {
+    if (c >= nch) c = 0;
+    const bool second = c >= nch1;
+    const T* p = second ? a.x2 : a.x;
+    const int cs = second ? a.c2 : a.c1, ci0 = (second ? c - nch1 : c) * CC + q8;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i)
+#pragma unroll
+      for (int g = 0; g < GPS; ++g) xr[i][g] = *reinterpret_cast<const float4*>(p + (long long)st_po[i] * cs + ci0 + 4 * g);
+  };
+  auto kept = [](const float4& v, bool k) { return make_float4(k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f); };
+  const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
+  const uint8_t* const x2m = a.x2 != nullptr ? a.x2m : nullptr;
+  const long long offs[1] = {off};
+  const int cos[1] = {co}, at[1] = {opix};
+  const bool oks[1] = {true};
+  float4 r0[1], add[1];
+  unsigned live_b[1], ok1, ok2;
+  {
+    unsigned b1[NLD], b2[NLD];
+    load_x(wave);
+    mie_mask_ask(a.xm, a.filt_mc, st_po, b1);
+    mie_mask_ask(x2m, a.filt_mc, st_po, b2);
+    mie_mask_ask(live_m, a.filt_mc, at, live_b);
+    conv_epilogue_load4<T, 1>(a, offs, oks, r0, add);
+    mie_mask_asked();
+    ok1 = mie_mask_take(a.xm, b1, inb);
+    ok2 = mie_mask_take(x2m, b2, a.x2 != nullptr ? inb : 0u);
+  }
+  auto store_x = [&](int c) {
+    const unsigned ok = c >= nch1 ? ok2 : ok1;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const int pix = p0 + STEP * i, py = pix / WX;
+      if (STEP * i + STEP > NPIX && pix >= NPIX) continue;
+      const bool k = (ok >> i) & 1u;
+      mie_bf16* const d = win + py * RP + (pix - py * WX) * LS + q8;
+      const float4 u = kept(xr[i][0], k);
+      if constexpr (X3) {
+        const float4 v = kept(xr[i][GPS - 1], k);
+        const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+        float4 pl[3];
+        split3(f, pl);
+#pragma unroll
+        for (int q = 0; q < PL; ++q) *reinterpret_cast<float4*>(d + q * STAGE) = pl[q];
+      } else {
+        *reinterpret_cast<float4*>(d) = u;
+      }
+    }
+  };
+
+  v4acc acc[4][MB], sm[X3 ? 4 : 1][MB];      // by phase; fp32: products of the first terms, and the smaller ones
+#pragma unroll
+  for (int b = 0; b < MB; ++b) {
+#pragma unroll
+    for (int ph = 0; ph < 4; ++ph) acc[ph][b] = v4acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ph = 0; ph < (X3 ? 4 : 1); ++ph) sm[ph][b] = v4acc{0.f, 0.f, 0.f, 0.f};
+  }
+  const mie_bf16* const x_lane = win + (l16 >> 3) * RP + (l16 & 7) * LS + EPS * kg;
+  auto chunk = [&](const char* cur, const char* next, auto more) {
+    float4 xv[MB][PL];
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+      const int ky = TAPS[j] / 3, kx = TAPS[j] % 3, ph = (ky == 1 ? 0 : 2) + (kx == 1 ? 0 : 1);
+      if (j == 0 || j == 1 || j == 3 || j == 5) {      // another shift
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+          for (int q = 0; q < PL; ++q)
+            xv[b][q] = *reinterpret_cast<const float4*>(x_lane + q * STAGE + (2 * b + (ky == 0)) * RP + (kx == 0) * LS);
+      }
+      if constexpr (X3) {
+        auto term = [&](v4acc (&t)[MB], int tw, int tx) {
+#pragma unroll
+          for (int b = 0; b < MB; ++b) mma16(t[b], w[j % RING][tw], xv[b][tx]);
+        };
+        term(sm[ph], 0, 2); term(acc[ph], 0, 0); term(sm[ph], 1, 1);
+        term(sm[ph], 2, 0); term(sm[ph], 0, 1); term(sm[ph], 1, 0);
+      } else {
+#pragma unroll
+        for (int b = 0; b < MB; ++b) mma16(acc[ph][b], w[j % RING][0], xv[b][0]);
+      }
+      if (RING < 9 && j + RING < 9) load_w(cur, j + RING, std::false_type());
+      else if (decltype(more)::value) load_w(next, (j + RING) % 9, std::false_type());
+      if constexpr (RING < 9) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  for (int c = wave; c < nch; c += DEEP_WAVES) {
+    store_x(c);
+    __builtin_amdgcn_wave_barrier();
+    if (RING < 9 || c + DEEP_WAVES < nch) {      // (RING < 9: the chunk after the last is the first again, one form of the loop)
+      load_x(c + DEEP_WAVES);
+      chunk(chunk_w(c), chunk_w(c + DEEP_WAVES < nch ? c + DEEP_WAVES : 0), std::true_type());
+    } else {
+      chunk(chunk_w(c), nullptr, std::false_type());
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+
+  // ---- the waves' sums meet in LDS: phase, position 16 * b + l16, channels 4 * kg ... (each where its own pixels were)
+#pragma unroll
+  for (int ph = 0; ph < 4; ++ph)
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+      v4acc s = acc[ph][b];
+      if constexpr (X3) s += sm[ph][b];
+      *reinterpret_cast<float4*>(smem + wave * OWN + ((ph * MB + b) * 16 + l16) * OS + 4 * kg) = make_float4(s[0], s[1], s[2], s[3]);
+    }
+  __syncthreads();
+  if (!mine) return;
+  const int from = ((2 * (ly & 1) + (lx & 1)) * (ROWS * 8) + (ly >> 1) * 8 + (lx >> 1)) * OS + 4 * (it & 3);
+  float4 part[DEEP_WAVES];
+#pragma unroll
+  for (int k = 0; k < DEEP_WAVES; ++k) part[k] = *reinterpret_cast<const float4*>(smem + k * OWN + from);
+#pragma unroll
+  for (int k = 1; k < DEEP_WAVES; ++k) {
+    part[0].x += part[k].x; part[0].y += part[k].y; part[0].z += part[k].z; part[0].w += part[k].w;
+  }
+  const float4 sums[1] = {part[0]};
+  const bool live[1] = {mie_mask_take(live_m, live_b, 1u) != 0u};
+  conv_epilogue_store4<T, 1>(a, offs, cos, oks, sums, r0, add, live);
+}
+
+// Two rows of input positions a workgroup while that is one round of the chip, else four: in one round or in two (fp32 and bf16, two
+// rounds against the split form: 512->256 from 24x32 24.3 -> 21.4 and 14.9 -> 10.4 us, 64+64->64 from 64x64 16.8 -> 12.6 and 12.1 -> 9.2).
+template <typename T>
+bool deep_tconv(const ConvArgsT<T>& a, const TileSetDev& pts, hipStream_t st) {
+  if ((sizeof(T) == 4 && !a.x3) || a.c1 % 32 != 0 || a.c2 % 32 != 0 || a.c1 + a.c2 < 128 || a.cout % DEEP_COLS != 0) return false;
+  const long long cap = (long long)pts.n * pts.tiles_y * pts.tiles_x, slabs = cap * (a.cout / DEEP_COLS);
+  if (4 * slabs <= DEEP_WGS)
+    hipLaunchKernelGGL((k_tconv_deep<T, 2>), dim3(a.cout / DEEP_COLS, 4 * (unsigned)cap), dim3(DEEP_THREADS), 0, st, a, pts);
+  else if (slabs <= DEEP_WGS)
+    hipLaunchKernelGGL((k_tconv_deep<T, 4>), dim3(a.cout / DEEP_COLS, 2 * (unsigned)cap), dim3(DEEP_THREADS), 0, st, a, pts);
+  else
+    return false;
+  return true;
+}
+
 // Workgroups of whole tiles.  The form is taken while they are one round of the chip, one a CU, and with as few rows as keep it that: two
 // beat four and these eight while there are CUs for them (fp32 256->256 at 8x12 7.4, 8.8, 11.7 us, bf16 5.2, 5.5, 6.6), and a second
 // round costs more than anything (at 16x24, 96 slabs: four rows 9.3, two 11.2; at 33x44, 480 slabs: 24.7 us, k_conv_mfma 20.7; a gates conv
@@ -504,3 +738,5 @@ bool mie_launch_gru_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st
 bool mie_launch_gru_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) { return deep_gru(a, cap, st); }
 bool mie_launch_upconv_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) { return deep_up(a, cap, st); }
 bool mie_launch_upconv_deep(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st) { return deep_up(a, cap, st); }
+bool mie_launch_tconv_deep(const ConvArgsT<float>& a, const TileSetDev& blocks, hipStream_t st) { return deep_tconv(a, blocks, st); }
+bool mie_launch_tconv_deep(const ConvArgsT<mie_bf16>& a, const TileSetDev& blocks, hipStream_t st) { return deep_tconv(a, blocks, st); }

@@ -17,8 +17,9 @@
 // stride-2 OR): a block is live when any of its four output tiles is.  A live block writes all its 256
 // pixels (zeros where no input reaches, their reservoirs left alone), a stale block is zeroed, which covers every stale
 // output tile.
-// On planes of very few blocks the chunks are split over up to 8 workgroups that write partial sums to the
-// workspace, and k_conv_split_finish (walking the OUTPUT tile set) adds them and runs the epilogue.
+// On planes of very few blocks the 3x3 form is another kernel, one launch (k_tconv_deep), for bf16 deltas and fp32 in three terms.
+// Of the others the chunks are split there over up to 8 workgroups that write partial sums to the workspace, and
+// k_conv_split_finish (walking the OUTPUT tile set) adds them and runs the epilogue.
 #include "mie_conv_mfma_impl.h"
 #include <type_traits>
 
@@ -335,27 +336,31 @@ template <typename T, int K, bool X3 = false>
 bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st) {
   constexpr int CC = X3 ? 64 : stage_channels(K, 1) * (4 / (int)sizeof(T));
   if (a0.filt_mc == nullptr || a0.c1 % CC != 0 || a0.c2 % CC != 0 || a0.cout % 32 != 0) return false;
+  constexpr bool DEEP = K == 3 && (X3 || sizeof(T) == 2);      // (takes every launch of these that could be split)
+  if (DEEP && mie_launch_tconv_deep(a0, pts, st)) return true;
   ConvArgsT<T> a = a0;
   a.xcd_fs = 0; a.xcd_m = 0;
   const unsigned cap_p = (unsigned)(pts.n * pts.tiles_y * pts.tiles_x);
-  const unsigned cap_out = (unsigned)(a.ts.n * a.ts.tiles_y * a.ts.tiles_x);
   const int cout = a.cout;
-  const long long groups = (long long)cap_p * (cout / 32);
-  const int nch = (a.c1 + a.c2) / CC;
-  if (a.ws != nullptr && !a.refresh && groups <= 128 && nch >= 4) {
-    a.ws_plane = (long long)a.ts.n * a.ts.h * a.ts.w * cout;
-    int parts = 1;
-    while (2 * parts <= 8 && 2 * parts <= nch && groups * (2 * parts) <= 256 && (long long)(2 * parts) * a.ws_plane <= a.ws_floats)
-      parts *= 2;
-    if (parts >= 2) {
-      a.xcd_fs = __builtin_ctz(parts);
-      const std::lock_guard<std::mutex> pair(mie_split_launches());
-      hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, true, X3>), dim3(cout / 32 * parts, cap_p), dim3(256), 0, st, a, pts);
-      unsigned ny = (unsigned)((1024 + cap_out - 1) / cap_out);
-      if (ny > (unsigned)(cout / 16)) ny = (unsigned)(cout / 16);
-      if (ny < 1) ny = 1;
-      hipLaunchKernelGGL(k_conv_split_finish<T>, dim3(cap_out, ny), dim3(256), 0, st, a, parts);
-      return true;
+  if constexpr (!DEEP) {
+    const unsigned cap_out = (unsigned)(a.ts.n * a.ts.tiles_y * a.ts.tiles_x);
+    const long long groups = (long long)cap_p * (cout / 32);
+    const int nch = (a.c1 + a.c2) / CC;
+    if (a.ws != nullptr && !a.refresh && groups <= 128 && nch >= 4) {
+      a.ws_plane = (long long)a.ts.n * a.ts.h * a.ts.w * cout;
+      int parts = 1;
+      while (2 * parts <= 8 && 2 * parts <= nch && groups * (2 * parts) <= 256 && (long long)(2 * parts) * a.ws_plane <= a.ws_floats)
+        parts *= 2;
+      if (parts >= 2) {
+        a.xcd_fs = __builtin_ctz(parts);
+        const std::lock_guard<std::mutex> pair(mie_split_launches());
+        hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, true, X3>), dim3(cout / 32 * parts, cap_p), dim3(256), 0, st, a, pts);
+        unsigned ny = (unsigned)((1024 + cap_out - 1) / cap_out);
+        if (ny > (unsigned)(cout / 16)) ny = (unsigned)(cout / 16);
+        if (ny < 1) ny = 1;
+        hipLaunchKernelGGL(k_conv_split_finish<T>, dim3(cap_out, ny), dim3(256), 0, st, a, parts);
+        return true;
+      }
     }
   }
   a.ws = nullptr;

@@ -1100,7 +1100,8 @@ def tconv2x_masked(x, xmask, x2, x2mask, filt, k, out_ts: TileMask, block_ts: Ti
     dt = x.dtype
     _ready(out_ts)
     _ready(block_ts)
-    ws_ptr, ws_bytes = _workspace_args(workspace, block_ts.capacity * (cout // 32) <= 128, x.device)
+    # (3x3 on bf16 deltas and in the three-term form: one launch on planes of few blocks)
+    ws_ptr, ws_bytes = _workspace_args(workspace, block_ts.capacity * (cout // 32) <= 128 and (k != 3 or code == _lib.DTYPE_F32), x.device)
     check(lib().mie_tconv2x_masked(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1, nhwc_ptr(x2, "x2", dtype=dt),
         pix_ptr(x2mask, n, h, w, "x2mask"), c2, h, w, plain.data_ptr(), mc_ptr, cin_total, k, cout, out_ts.ref,
