@@ -722,6 +722,10 @@ bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles,
   if (dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) return false;
   if (!((k == 3 && (s == 1 || s == 2)) || (k == 5 && s == 2))) return false;
   if (c1 % 32 != 0 || c2 % 32 != 0 || c1 + c2 < (k == 3 ? 64 : 32) || cout % DEEP_COLS != 0) return false;
+  // (fp32 of eight rows a workgroup splits its pixels into terms for 16 columns only, one pass of chunks behind the other: with more than
+  // two passes' worth of 256 channels the split form is faster.  512+512->512 at 16x32 39.1 us, 34.5 there, ->256 at 32x32 38.3, 34.6;
+  // the other way 512->512 at 16x32 22.3 and 23.4, 256+256->256 at 32x32 21.4 and 22.4.  Optical flow, up-sampling decoder, 433.1 -> 428.2)
+  if (dtype == MIE_DTYPE_F32_BF16X3 && k == 3 && s == 1 && 2 * deep_slabs(tiles, cout) > DEEP_WGS && c1 + c2 > 512) return false;
   return deep_slabs(tiles, cout) <= DEEP_WGS;
 }
 // (fp32 of eight rows a workgroup: 128->64 at 64x64 17.8 us, k_upconv2x 16.1)
