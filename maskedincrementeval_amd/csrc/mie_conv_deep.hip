@@ -1,5 +1,5 @@
-// Masked convs on planes of few tiles -- 3x3 stride 1, also with the gate chain of a ConvLSTM as its epilogue, 3x3 and 5x5 stride 2, 5x5 over
-// an up-sampled sum -- with the whole contraction of an output inside one workgroup, in one launch.
+// Masked convs on planes of few tiles -- 3x3 stride 1, also with the gate chain of a ConvLSTM or ConvGRU as its epilogue, 3x3 and 5x5
+// stride 2, 5x5 over an up-sampled sum, the 3x3 transposed conv -- with the whole contraction of an output inside one workgroup, in one launch.
 //
 // What bounds these layers (256 channels at 8x12 .. 32x32) is neither memory nor the matrix cores but the trips to memory one after
 // the other in a launch -- arguments, tile list, masks and pixels, sums -- and the launches themselves: the split form of
@@ -723,7 +723,7 @@ bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles,
   if (!((k == 3 && (s == 1 || s == 2)) || (k == 5 && s == 2))) return false;
   if (c1 % 32 != 0 || c2 % 32 != 0 || c1 + c2 < (k == 3 ? 64 : 32) || cout % DEEP_COLS != 0) return false;
   // (fp32 of eight rows a workgroup splits its pixels into terms for 16 columns only, one pass of chunks behind the other: with more than
-  // two passes' worth of 256 channels the split form is faster.  512+512->512 at 16x32 39.1 us, 34.5 there, ->256 at 32x32 38.3, 34.6;
+  // 512 channels the split form is faster.  512+512->512 at 16x32 39.1 us, 34.5 there, ->256 at 32x32 38.3, 34.6;
   // the other way 512->512 at 16x32 22.3 and 23.4, 256+256->256 at 32x32 21.4 and 22.4.  Optical flow, up-sampling decoder, 433.1 -> 428.2)
   if (dtype == MIE_DTYPE_F32_BF16X3 && k == 3 && s == 1 && 2 * deep_slabs(tiles, cout) > DEEP_WGS && c1 + c2 > 512) return false;
   return deep_slabs(tiles, cout) <= DEEP_WGS;
