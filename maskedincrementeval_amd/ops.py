@@ -1439,9 +1439,13 @@ def conv_gru_incr(x, xmask, filt: ConvFilter, out_ts: TileMask, update_res, cand
     dt = x.dtype
     plain, mc_ptr, code = _filter_args(filt, 3, dt, (1, c, 0, filt.shape[3]), with_code=True)
     hid = plain.shape[3] // 2
+    if plain.shape[3] != 2 * hid:
+        raise ValueError("gates filter needs 2*hid columns, got %d" % plain.shape[3])
     for name, t in (("update_res", update_res), ("cand_res", cand_res), ("h_delta", h_delta)):
         if tuple(t.shape) != (n, hid, h, w):
             raise ValueError("%s shape %s, expected %s" % (name, tuple(t.shape), (n, hid, h, w)))
+    if (out_ts.n, out_ts.h, out_ts.w) != (n, h, w):
+        raise ValueError("tile set %s does not match the input %s" % ((out_ts.n, out_ts.h, out_ts.w), (n, h, w)))
     _ready(out_ts)
     check(lib().mie_conv_gru_masked(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c, h, w, plain.data_ptr(), mc_ptr, plain.shape[0], hid, out_ts.ref,

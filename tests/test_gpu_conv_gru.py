@@ -86,6 +86,11 @@ def test_what_it_refuses():
         ops.conv_gru_incr(x, m, filt, ts, u, u, dh)
     with pytest.raises(ValueError):
         ops.conv_gru_incr(x, m, filt, ts, u, c, dh[:, :16])
+    for wrong in (TileMask(2, 8, 8, DEV), TileMask(1, 8, 16, DEV)):
+        with pytest.raises(ValueError, match="tile set"):
+            ops.conv_gru_incr(x, m, filt, wrong, u, c, dh)
+    with pytest.raises(ValueError, match="columns"):
+        ops.conv_gru_incr(x, m, ops.ConvFilter(torch.randn(64, 3, 3, 65, device=DEV)), ts, u, c, dh)
     plain, mc = filt.for_dtype(torch.float32, False)
     assert _lib.lib().mie_conv_gru_masked(x.data_ptr(), m.data_ptr(), 64, 8, 8, plain.data_ptr(), mc.data_ptr(), 64, 32, ts.ref,
                                           u.data_ptr(), c.data_ptr(), dh.data_ptr(), _lib.DTYPE_F32, None) == -2
