@@ -142,6 +142,10 @@ class LayerProbe:
             return dict(kind="conv", k=3, s=1, cin=c1 + c2, cout=filt.shape[3], h=h, w=w, n=n,
                         xmask=xmask, x2mask=x2mask, ts=out_ts, fused=True, gates=True)
 
+        def conv_gru_desc(x, xmask, filt, out_ts, *a, **kw):
+            n, c1, h, w = x.shape
+            return dict(kind="conv", k=3, s=1, cin=c1, cout=filt.shape[3], h=h, w=w, n=n, xmask=xmask, x2mask=None, ts=out_ts, fused=True, gru=True)
+
         def upconv_desc(a_, amask, b_, bmask, filt, k, pad, out_ts, out_delta, reservoir=None, *a, **kw):
             n, c, h, w = a_.shape
             return dict(kind="conv", k=k, s=1, cin=c, cout=filt.shape[3], h=h, w=w, n=n, xmask=amask,
@@ -174,6 +178,7 @@ class LayerProbe:
         self._wrap("upconv2x_masked", upconv2x_desc)
         self._wrap("upconv_pred_masked", upconv_pred_desc)
         self._wrap("conv_gates_incr", conv_gates_desc)
+        self._wrap("conv_gru_incr", conv_gru_desc)
         self._wrap("act_incr", pw_desc("act", 1, 1))
         self._wrap("add_incr", pw_desc("add", 2, 0))
         self._wrap("mul_incr", pw_desc("mul", 2, 2))
@@ -211,6 +216,9 @@ class LayerProbe:
                     # hidden and cell deltas written; the 4*hid-channel gate delta never reaches memory
                     hid = cout // 4
                     byts += a_out * (2 * cout * 4 + 2 * hid * 4 + hid * 4 + 2 * hid * es)
+                elif d.get("gru"):
+                    # update and candidate reservoirs read + written, the state's delta written
+                    byts += a_out * (2 * cout * 4 + cout // 2 * es)
                 elif d.get("pred"):
                     # fused tail: the layer's reservoir read + written, its delta never stored; the second delta of the
                     # prediction conv read where its mask is set; prediction reservoir read + written, prediction delta
@@ -226,7 +234,7 @@ class LayerProbe:
                     flops = 2 * a_out * cin * cout * k * k // (d["s"] * d["s"])
                 row.update(shape="%s%dx%d s%d %d->%d%s @%dx%d" % ("up2x+" if d.get("up") else ("tconv " if d.get("tconv") else ""),
                                                                    k, k, d["s"], cin, cout,
-                                                                   "+lstm" if d.get("gates") else ("+pred" if d.get("pred") else ""),
+                                                                   "+lstm" if d.get("gates") else "+gru" if d.get("gru") else ("+pred" if d.get("pred") else ""),
                                                                    ts.h, ts.w),
                            active_tiles=int(ts.counts[0].item()), tiles=ts.capacity, a_out=a_out,
                            bytes=byts, flops=flops)
@@ -518,7 +526,7 @@ class NetBench:
         tile set, same buffers) launched `reps` times on the launch stream, each launch between two HIP events
         of its own; `us` is the mean of the pairs less what an empty pair reads."""
         torch = self.torch
-        convs = [l for l in layers if l["op"] in ("conv_masked", "conv_gates_incr", "upconv_masked", "upconv2x_masked", "upconv_pred_masked",
+        convs = [l for l in layers if l["op"] in ("conv_masked", "conv_gates_incr", "conv_gru_incr", "upconv_masked", "upconv2x_masked", "upconv_pred_masked",
                                             "tconv2x_masked")]
         dom = max(convs, key=lambda l: l["us"])
         orig, cargs, ckw = agg[layers.index(dom)]["call"]
@@ -569,7 +577,7 @@ class NetBench:
         else:
             roofline = dict(bound="hbm", achieved=dom["gbs"], peak=PEAK_HBM_GBS, unit="GB/s",
                             frac=round(dom["gbs"] / PEAK_HBM_GBS, 4), traffic=None)
-        roofline.update(kernel="mie_%s %s" % (dom["op"].replace("_incr", "").replace("conv_gates", "conv_gates_masked"),
+        roofline.update(kernel="mie_%s %s" % (dom["op"].replace("_incr", "").replace("conv_gates", "conv_gates_masked").replace("conv_gru", "conv_gru_masked"),
                                               dom["shape"]), us=dom["us"],
                         algorithmic_bytes=dom["bytes"], algorithmic_flops=dom["flops"],
                         us_event_pair=round(pair_us, 2), us_graph_of_identical_launches=round(graph_us, 2),
