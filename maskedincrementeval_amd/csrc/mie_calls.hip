@@ -88,7 +88,7 @@ const Row kRows[] = {
     ROW(mie_avgpool_incr), ROW(mie_linear_incr), ROW(mie_upconv_masked), ROW(mie_upconv_masked_ws),
     ROW(mie_upconv_pred_masked), ROW(mie_upconv2x_pred_masked), ROW(mie_tconv_masked), ROW(mie_tconv_refresh), ROW(mie_tconv2x_masked),
     ROW(mie_tconv2x_refresh), ROW(mie_upconv2x_masked), ROW(mie_upconv2x_refresh), ROW(mie_events_to_frame), ROW(mie_events_to_frame_bf16),
-    ROW(mie_conv_gru_masked),
+    ROW(mie_conv_gru_masked), ROW(mie_tconv2x_lead_masked),
 };
 #undef ROW
 constexpr int kRowCount = (int)(sizeof(kRows) / sizeof(kRows[0]));

@@ -633,6 +633,34 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_tconv_deep(ConvArgsT<T> a, Til
     __builtin_amdgcn_wave_barrier();
   }
 
+  // ---- two more input channels (a.g_cpd with its mask a.g_cpm, plain filter rows a.g_cpres), in fp32: an output pixel sees the one, two or
+  // four taps of its phase.  Asked for here, where the filter's registers are free, and added behind the sums.  (As a launch of their
+  // own and an addend, optical flow with transposed decoders, two such layers: 312.4 -> 304.9 us a pass.)
+  float2 lx2[4];
+  float4 lf[4][2];
+  unsigned lead_b[4], lead_in = 0u;
+  const bool lead = a.g_cpd != nullptr;
+  if (lead) {
+    int lat[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = q >> 1, c = q & 1, iy = y0 + (ly >> 1) + r, ix = x0 + (lx >> 1) + c;
+      const bool k = in && (r == 0 || (ly & 1)) && (c == 0 || (lx & 1)) && iy < a.h_in && ix < a.w_in;
+      const int ky = r != 0 ? 0 : (ly & 1) ? 2 : 1, kx = c != 0 ? 0 : (lx & 1) ? 2 : 1;
+      lat[q] = k ? (n * a.h_in + iy) * a.w_in + ix : 0;
+      lead_in |= (k ? 1u : 0u) << q;
+      if constexpr (X3) {
+        lx2[q] = *reinterpret_cast<const float2*>(a.g_cpd + 2LL * lat[q]);
+      } else {
+        const uint32_t v = *reinterpret_cast<const uint32_t*>(a.g_cpd + 2LL * lat[q]);
+        lx2[q] = make_float2(__uint_as_float(v << 16), __uint_as_float(v & 0xffff0000u));
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) lf[q][i] = *reinterpret_cast<const float4*>(a.g_cpres + (long long)(9 * i + 3 * ky + kx) * cout + co);
+    }
+    mie_mask_ask(a.g_cpm, a.filt_mc, lat, lead_b);
+  }
+
   // ---- the waves' sums meet in LDS: phase, position 16 * b + l16, channels 4 * kg ... (each where its own pixels were)
 #pragma unroll
   for (int ph = 0; ph < 4; ++ph)
@@ -652,23 +680,36 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_tconv_deep(ConvArgsT<T> a, Til
   for (int k = 1; k < DEEP_WAVES; ++k) {
     part[0].x += part[k].x; part[0].y += part[k].y; part[0].z += part[k].z; part[0].w += part[k].w;
   }
+  if (lead) {
+    const unsigned k = mie_mask_take(a.g_cpm, lead_b, lead_in);
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float u = (k >> q) & 1u ? lx2[q].x : 0.f, v = (k >> q) & 1u ? lx2[q].y : 0.f;
+      s.x += u * lf[q][0].x + v * lf[q][1].x; s.y += u * lf[q][0].y + v * lf[q][1].y;
+      s.z += u * lf[q][0].z + v * lf[q][1].z; s.w += u * lf[q][0].w + v * lf[q][1].w;
+    }
+    part[0].x += s.x; part[0].y += s.y; part[0].z += s.z; part[0].w += s.w;
+  }
   const float4 sums[1] = {part[0]};
   const bool live[1] = {mie_mask_take(live_m, live_b, 1u) != 0u};
   conv_epilogue_store4<T, 1>(a, offs, cos, oks, sums, r0, add, live);
 }
 
+long long deep_slabs(long long tiles, int cout) { return tiles * (cout / DEEP_COLS); }
+template <typename T>
+int deep_dtype(const ConvArgsT<T>& a) { return sizeof(T) == 2 ? MIE_DTYPE_BF16 : a.x3 ? MIE_DTYPE_F32_BF16X3 : MIE_DTYPE_F32; }
+
 // Two rows of input positions a workgroup while that is one round of the chip, else four: in one round or in two (fp32 and bf16, two
 // rounds against the split form: 512->256 from 24x32 24.3 -> 21.4 and 14.9 -> 10.4 us, 64+64->64 from 64x64 16.8 -> 12.6 and 12.1 -> 9.2).
 template <typename T>
 bool deep_tconv(const ConvArgsT<T>& a, const TileSetDev& pts, hipStream_t st) {
-  if ((sizeof(T) == 4 && !a.x3) || a.c1 % 32 != 0 || a.c2 % 32 != 0 || a.c1 + a.c2 < 128 || a.cout % DEEP_COLS != 0) return false;
-  const long long cap = (long long)pts.n * pts.tiles_y * pts.tiles_x, slabs = cap * (a.cout / DEEP_COLS);
+  const long long cap = (long long)pts.n * pts.tiles_y * pts.tiles_x, slabs = deep_slabs(cap, a.cout);
+  if (!mie_tconv_deep_form(a.c1, a.c2, a.cout, cap, deep_dtype(a))) return false;
   if (4 * slabs <= DEEP_WGS)
     hipLaunchKernelGGL((k_tconv_deep<T, 2>), dim3(a.cout / DEEP_COLS, 4 * (unsigned)cap), dim3(DEEP_THREADS), 0, st, a, pts);
-  else if (slabs <= DEEP_WGS)
-    hipLaunchKernelGGL((k_tconv_deep<T, 4>), dim3(a.cout / DEEP_COLS, 2 * (unsigned)cap), dim3(DEEP_THREADS), 0, st, a, pts);
   else
-    return false;
+    hipLaunchKernelGGL((k_tconv_deep<T, 4>), dim3(a.cout / DEEP_COLS, 2 * (unsigned)cap), dim3(DEEP_THREADS), 0, st, a, pts);
   return true;
 }
 
@@ -676,8 +717,6 @@ bool deep_tconv(const ConvArgsT<T>& a, const TileSetDev& pts, hipStream_t st) {
 // beat four and these eight while there are CUs for them (fp32 256->256 at 8x12 7.4, 8.8, 11.7 us, bf16 5.2, 5.5, 6.6), and a second
 // round costs more than anything (at 16x24, 96 slabs: four rows 9.3, two 11.2; at 33x44, 480 slabs: 24.7 us, k_conv_mfma 20.7; a gates conv
 // of 64 channels at 32x48, 384: 12.1 and 8.9; 5x5 64->128 at 48x48, 288: 19.5 and 16.1).
-long long deep_slabs(long long tiles, int cout) { return tiles * (cout / DEEP_COLS); }
-
 template <typename T, int K, int S, int KIND>
 void launch_deep(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
   const long long slabs = deep_slabs(cap, a.cout);
@@ -685,9 +724,6 @@ void launch_deep(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
   else if (2 * slabs <= DEEP_WGS) launch_chunks<T, K, S, 4, KIND>(a, cap, st);
   else launch_chunks<T, K, S, 8, KIND>(a, cap, st);
 }
-
-template <typename T>
-int deep_dtype(const ConvArgsT<T>& a) { return sizeof(T) == 2 ? MIE_DTYPE_BF16 : a.x3 ? MIE_DTYPE_F32_BF16X3 : MIE_DTYPE_F32; }
 
 template <typename T>
 bool deep_plain(const ConvArgsT<T>& a, int k, int s, unsigned cap, hipStream_t st) {
@@ -727,6 +763,10 @@ bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles,
   // the other way 512->512 at 16x32 22.3 and 23.4, 256+256->256 at 32x32 21.4 and 22.4.  Optical flow, up-sampling decoder, 433.1 -> 428.2)
   if (dtype == MIE_DTYPE_F32_BF16X3 && k == 3 && s == 1 && 2 * deep_slabs(tiles, cout) > DEEP_WGS && c1 + c2 > 512) return false;
   return deep_slabs(tiles, cout) <= DEEP_WGS;
+}
+bool mie_tconv_deep_form(int c1, int c2, int cout, long long blocks, int dtype) {
+  return (dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3) && c1 % 32 == 0 && c2 % 32 == 0 && c1 + c2 >= 128 && cout % DEEP_COLS == 0 &&
+         deep_slabs(blocks, cout) <= DEEP_WGS;
 }
 // (fp32 of eight rows a workgroup: 128->64 at 64x64 17.8 us, k_upconv2x 16.1)
 bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype) {

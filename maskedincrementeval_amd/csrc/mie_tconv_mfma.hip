@@ -380,7 +380,8 @@ int tconv2x_impl(const char* who, const void* x, const uint8_t* xmask, int c1, c
                  const uint8_t* x2mask, int c2, int h_in, int w_in, const float* filter, const void* filter_mc,
                  int cin_total, int k, int cout, const mie_tileset* out, const mie_tileset* blocks,
                  void* out_delta, const void* addend, float* reservoir, int act_kind, float slope, bool refresh,
-                 const float* bias, void* workspace, long long workspace_bytes, void* stream, bool x3 = false) {
+                 const float* bias, void* workspace, long long workspace_bytes, void* stream, bool x3 = false,
+                 const void* lead = nullptr, const uint8_t* lead_mask = nullptr, const float* lead_filter = nullptr) {
   int rc = mie_check_tileset(out, who);
   if (rc != MIE_OK) return rc;
   rc = mie_check_tileset(blocks, who);
@@ -426,6 +427,16 @@ int tconv2x_impl(const char* who, const void* x, const uint8_t* xmask, int c1, c
   a.ws = (float*)workspace; a.ws_floats = workspace_bytes / 4; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = x3 ? 1 : 0;
   a.ts = mie_dev_tileset(out);
   const TileSetDev pts = mie_dev_tileset(blocks);
+  if (lead != nullptr) {
+    const int dtype = sizeof(T) == 2 ? MIE_DTYPE_BF16 : x3 ? MIE_DTYPE_F32_BF16X3 : MIE_DTYPE_F32;
+    MIE_REQUIRE(lead_filter != nullptr && mie_aligned(lead, 2 * sizeof(T)) && mie_aligned(lead_filter, 16) && lead != out_delta, MIE_ERR_INVALID_ARG,
+                "%s: lead and its filter rows must be given together, aligned, and not alias the output", who);
+    MIE_REQUIRE(k == 3 && mie_tconv_deep_form(c1, c2, cout, (long long)pts.n * pts.tiles_y * pts.tiles_x, dtype), MIE_ERR_UNSUPPORTED,
+                "%s: only where mie_tconv2x_takes_lead (k=%d c1=%d c2=%d cout=%d)", who, k, c1, c2, cout);
+    a.g_cpd = (const T*)lead; a.g_cpm = lead_mask; a.g_cpres = const_cast<float*>(lead_filter);
+    mie_launch_tconv_deep(a, pts, (hipStream_t)stream);
+    return mie_check_launch(who);
+  }
   bool ok;
   if constexpr (sizeof(T) == 4) {
     if (x3) ok = (k == 3) ? launch_tconv<T, 3, true>(a, pts, (hipStream_t)stream) : launch_tconv<T, 5, true>(a, pts, (hipStream_t)stream);
@@ -472,4 +483,23 @@ extern "C" int mie_tconv2x_refresh(const void* x, int c1, const void* x2, int c2
                                   blocks, out_dense, addend, reservoir, act_kind, slope, true, bias, nullptr, 0, stream);
   return tconv2x_impl<float>(who, x, nullptr, c1, x2, nullptr, c2, h_in, w_in, filter, filter_mc, cin_total, k, cout, out, blocks,
                              out_dense, addend, reservoir, act_kind, slope, true, bias, nullptr, 0, stream, x3);
+}
+
+extern "C" int mie_tconv2x_takes_lead(int c1, int c2, int cout, int blocks, int dtype) {
+  return mie_tconv_deep_form(c1, c2, cout, blocks, dtype) ? 1 : 0;
+}
+
+extern "C" int mie_tconv2x_lead_masked(const void* lead, const uint8_t* lead_mask, const float* lead_filter, const void* x, const uint8_t* xmask,
+                                       int c1, const void* x2, const uint8_t* x2mask, int c2, int h_in, int w_in, const float* filter,
+                                       const void* filter_mc, int cin_total, int cout, const mie_tileset* out, const mie_tileset* blocks,
+                                       void* out_delta, float* reservoir, int act_kind, float slope, int dtype, void* stream) {
+  const char* who = "mie_tconv2x_lead_masked";
+  mie_clear_error();
+  MIE_REQUIRE(lead != nullptr, MIE_ERR_INVALID_ARG, "%s: NULL pointer", who);
+  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3, MIE_ERR_UNSUPPORTED, "%s: bf16 or three-term fp32 deltas, not dtype %d", who, dtype);
+  if (dtype == MIE_DTYPE_BF16)
+    return tconv2x_impl<mie_bf16>(who, x, xmask, c1, x2, x2mask, c2, h_in, w_in, filter, filter_mc, cin_total, 3, cout, out, blocks, out_delta,
+                                  nullptr, reservoir, act_kind, slope, false, nullptr, nullptr, 0, stream, false, lead, lead_mask, lead_filter);
+  return tconv2x_impl<float>(who, x, xmask, c1, x2, x2mask, c2, h_in, w_in, filter, filter_mc, cin_total, 3, cout, out, blocks, out_delta, nullptr,
+                             reservoir, act_kind, slope, false, nullptr, nullptr, 0, stream, true, lead, lead_mask, lead_filter);
 }

@@ -643,8 +643,9 @@ class nnConvTranspose2dIncr(replay.Watched, nn.ConvTranspose2d, _IncrBuffers):
         return k, s, p, op
 
     def forward(self, x_incr: Masked, reservoir=None, act=_lib.ACT_NONE, slope=0.0, x2_incr: Masked = None,
-                addend_incr: Masked = None, filt=None, out_name="out") -> Masked:
+                addend_incr: Masked = None, filt=None, out_name="out", lead_incr: Masked = None, lead_filt=None) -> Masked:
         """x2_incr: second input (the conv runs over the channel concat of the two without forming it);
+        lead_incr, lead_filt: a part of two channels in front of them and its rows, where ops.tconv2x_takes_lead;
         addend_incr: delta added before the epilogue, covered by the output mask; filt: a row slice of
         self._filter() when only part of the input channels is fed.  Two inputs and the addend need the
         matrix-core form."""
@@ -668,9 +669,10 @@ class nnConvTranspose2dIncr(replay.Watched, nn.ConvTranspose2d, _IncrBuffers):
             blocks = self._tile_set(out_name + "_blocks", n, h, w, x.device)
             ops.build_mask_tiles(ts, None, n, ho, wo, _lib.FOOT_CONV, 2, 2, 0, blocks)
             addend = None if addend_incr is None else ops.as_nhwc(addend_incr[0])
-            ops.tconv2x_masked(x, pix, x2, pix2, filt, k, ts, blocks, out, reservoir, act, slope, addend)
+            lead = None if lead_incr is None else _unpack(lead_incr)[:2] + (lead_filt,)
+            ops.tconv2x_masked(x, pix, x2, pix2, filt, k, ts, blocks, out, reservoir, act, slope, addend, lead=lead)
             return [out, ts]
-        if x2 is not None or addend_incr is not None:
+        if x2 is not None or addend_incr is not None or lead_incr is not None:
             raise NotImplementedError("transposed conv over two inputs / with an addend needs the matrix-core form "
                                       "(stride 2, k in {3, 5}, padding k // 2, output_padding 1, channels in whole chunks)")
         ops.tconv_masked(x, pix, filt, k, s, p, ts, out, reservoir, act, slope)

@@ -1061,6 +1061,14 @@ def tconv2x_takes(c1: int, c2: int, cout: int, k: int, stride: int, pad: int, ou
             and c1 % chunk == 0 and c2 % chunk == 0 and cout % 32 == 0 and filt.for_dtype(dtype)[1] is not None)
 
 
+def tconv2x_takes_lead(lead_c: int, c1: int, c2: int, cout: int, k: int, blocks: int, dtype) -> bool:
+    """Whether tconv2x_masked, where it takes a layer of this shape, takes a leading part of `lead_c` channels too (blocks: capacity of
+    its block set)."""
+    code = _lib.DTYPE_BF16 if dtype == torch.bfloat16 else _lib.DTYPE_F32_BF16X3
+    return (lead_c == 2 and k == 3 and c1 % 64 == 0 and c2 % 64 == 0 and (dtype == torch.bfloat16 or f32_matmul == "bf16x3")
+            and bool(lib().mie_tconv2x_takes_lead(c1, c2, cout, blocks, code)))
+
+
 def _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out, addend, reservoir):
     n, c1, h, w = x.shape
     c2 = 0 if x2 is None else x2.shape[1]
@@ -1090,9 +1098,9 @@ def _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out, addend, reservoir):
 
 
 def tconv2x_masked(x, xmask, x2, x2mask, filt, k, out_ts: TileMask, block_ts: TileMask, out_delta, reservoir=None,
-                   act=_lib.ACT_NONE, slope=0.0, addend=None, workspace=None):
+                   act=_lib.ACT_NONE, slope=0.0, addend=None, workspace=None, lead=None):
     """Stride-2 transposed conv (k in {3, 5}, pad k // 2, output twice the input) of x ++ x2 on the matrix
-    cores.  out_ts: MIE_FOOT_TCONV tile set of the output; block_ts: tile set of the 16x16 output blocks at
+    cores.  lead: (delta, pixel mask, ConvFilter of its rows) of two more input channels, where tconv2x_takes_lead, without an addend.  out_ts: MIE_FOOT_TCONV tile set of the output; block_ts: tile set of the 16x16 output blocks at
     input resolution (build_mask_tiles(out_ts, None, ..., FOOT_CONV, 2, 2, 0, block_ts)).
     workspace: as in conv_masked (None: the stream's shared one when the plane is small, False: none)."""
     n, c1, c2, h, w, plain, mc_ptr, cin_total, cout, code = _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out_delta,
@@ -1100,6 +1108,17 @@ def tconv2x_masked(x, xmask, x2, x2mask, filt, k, out_ts: TileMask, block_ts: Ti
     dt = x.dtype
     _ready(out_ts)
     _ready(block_ts)
+    if lead is not None:
+        x0, mask0, filt0 = lead
+        if k != 3 or addend is not None or tuple(x0.shape) != (n, 2, h, w) or tuple(filt0.shape) != (2, 3, 3, cout):
+            raise ValueError("lead %s with filter %s does not fit the input %s" % (tuple(x0.shape), tuple(filt0.shape), tuple(x.shape)))
+        plain0, _ = _filter_args(filt0, 3, dt)
+        check(lib().mie_tconv2x_lead_masked(
+            nhwc_ptr(x0, "lead", dtype=dt), pix_ptr(mask0, n, h, w, "lead mask"), plain0.data_ptr(),
+            nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1, nhwc_ptr(x2, "x2", dtype=dt),
+            pix_ptr(x2mask, n, h, w, "x2mask"), c2, h, w, plain.data_ptr(), mc_ptr, cin_total, cout, out_ts.ref,
+            block_ts.ref, nhwc_ptr(out_delta, "out_delta", dtype=dt), nhwc_ptr(reservoir, "reservoir"), act, float(slope), code, _stream(x)))
+        return out_delta
     # (3x3 on bf16 deltas and in the three-term form: one launch on planes of few blocks)
     ws_ptr, ws_bytes = _workspace_args(workspace, block_ts.capacity * (cout // 32) <= 128 and (k != 3 or code == _lib.DTYPE_F32), x.device)
     check(lib().mie_tconv2x_masked(

@@ -61,3 +61,52 @@ def test_transposed_conv_in_one_launch(n, c1, c2, cout, h, w, dtype):
     ops.tconv2x_refresh(_dev(d[:, :c1]).to(dtype), _dev(d[:, c1:]).to(dtype) if c2 else None, filt, bias.to(DEV), 3, ts, blocks, out, res)
     want = up(d, wt) + bias.double().view(1, -1, 1, 1)
     assert ((res.cpu().double() - want).abs() <= 4e-7 * bound + 2.0 ** -23 * want.abs()).all()
+
+
+# two more input channels in front (a part whose mask the wide parts' covers): every phase, planes cut off at both edges, two and four rows
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,c1,c2,cout,h,w", [(1, 128, 0, 32, 1, 1), (2, 64, 64, 32, 5, 9), (1, 128, 128, 128, 31, 32), (1, 64, 64, 64, 63, 64)])
+def test_transposed_conv_with_a_leading_part(n, c1, c2, cout, h, w, dtype):
+    bf, cin = dtype == torch.bfloat16, c1 + c2
+    q = (lambda t: t.to(dtype).float()) if bf else (lambda t: t)
+    wt = q(torch.randn(2 + cin, cout, 3, 3, generator=torch.Generator().manual_seed(cin)) * (2.0 / (9 * cin)) ** 0.5)
+    filt = ops.ConvFilter(wt.permute(0, 2, 3, 1).contiguous().to(DEV))
+    ho, wo = 2 * h, 2 * w
+    ts, blocks, out = TileMask(n, ho, wo, DEV), TileMask(n, h, w, DEV), ops.new_nhwc(n, cout, ho, wo, DEV, dtype)
+    assert ops.tconv2x_takes_lead(2, c1, c2, cout, 3, blocks.capacity, dtype)
+    up = lambda x, f: F.conv_transpose2d(x.double(), f.double(), stride=2, padding=1, output_padding=1)
+    ref = torch.zeros(n, cout, ho, wo, dtype=torch.float64)
+    res, tol = _dev(ref.float()), torch.zeros_like(ref)
+    for step, dens in enumerate((0.2, 1.0)):
+        d, m = gaussian_delta(n, cin, h, w, dens, 0.5, seed=900 + step)
+        m0 = m if step else m * (torch.rand(m.shape, generator=torch.Generator().manual_seed(3)) < 0.5).to(m.dtype)
+        d0 = q(torch.randn(n, 2, h, w, generator=torch.Generator().manual_seed(4 + step))) * m0
+        d = torch.cat([d0, q(d)], 1)
+        x = torch.where(torch.cat([m0.expand(-1, 2, -1, -1), m.expand(-1, cin, -1, -1)], 1).bool(), d, torch.full((), float("nan"))).to(dtype)
+        dm, dm0 = m.to(DEV), m0.to(DEV)
+        ops.build_mask_tiles(dm, None, n, h, w, _lib.FOOT_TCONV, 3, 2, 1, ts)
+        ops.build_mask_tiles(ts, None, n, ho, wo, _lib.FOOT_CONV, 2, 2, 0, blocks)
+        ops.tconv2x_masked(_dev(x[:, 2:2 + c1]), dm, _dev(x[:, 2 + c1:]) if c2 else None, dm if c2 else None, filt.rows(2, 2 + cin), 3, ts, blocks,
+                           out, res, lead=(_dev(x[:, :2]), dm0 if step == 0 else None, filt.rows(0, 2)))
+        torch.cuda.synchronize()
+        sums, bound = up(d, wt), up(d.abs(), wt.abs())
+        tol = tol + 4e-7 * bound + 2.0 ** -23 * (ref.abs() + sums.abs())
+        ref = ref + sums
+        assert ((res.cpu().double() - ref).abs() <= tol).all(), step
+        got = out.cpu().double()
+        assert ((got - sums).abs() <= 2 * tol + (2.0 ** -8 if bf else 0.0) * sums.abs()).all(), step
+    with pytest.raises(ValueError):
+        ops.tconv2x_masked(_dev(x[:, 2:2 + c1]), dm, _dev(x[:, 2 + c1:]) if c2 else None, dm if c2 else None, filt.rows(2, 2 + cin), 3, ts, blocks,
+                           out, res, lead=(_dev(x[:, :1]), dm0, filt.rows(0, 1)))
+
+
+def test_leading_part_only_where_the_one_launch_form_is():
+    assert not ops.tconv2x_takes_lead(2, 64, 0, 64, 3, 4, torch.float32) and not ops.tconv2x_takes_lead(2, 128, 0, 64, 5, 4, torch.float32)
+    assert not ops.tconv2x_takes_lead(3, 128, 0, 64, 3, 4, torch.bfloat16) and not ops.tconv2x_takes_lead(2, 128, 0, 64, 3, 65, torch.bfloat16)
+    filt = ops.ConvFilter(torch.randn(66, 3, 3, 64, device=DEV))
+    ts, blocks = TileMask(1, 16, 16, DEV), TileMask(1, 8, 8, DEV)
+    for t, s in ((ts, 16), (blocks, 8)):
+        ops.build_mask_tiles(None, None, 1, s, s, _lib.FOOT_CONV, 1, 1, 0, t)
+    x, out = ops.new_nhwc(1, 64, 8, 8, DEV).zero_(), ops.new_nhwc(1, 64, 16, 16, DEV)
+    with pytest.raises(Exception, match="takes_lead"):
+        ops.tconv2x_masked(x, None, None, None, filt.rows(2, 66), 3, ts, blocks, out, lead=(ops.new_nhwc(1, 2, 8, 8, DEV).zero_(), None, filt.rows(0, 2)))
