@@ -817,10 +817,8 @@ int mie_tconv2x_masked(const void* x, const uint8_t* xmask, int c1,
  * The same for k = 3 with two more input channels in front, a narrow part of the concat (a flow estimate of the scale before):
  *   lead, lead_mask : [n,h_in,w_in,2] delta and its pixel mask (NULL: all), covered by `out`
  *   lead_filter     : [2][3][3][cout] fp32, its rows of the filter (bf16 deltas: the weights rounded to bf16)
- * in place of mie_tconv_masked of the lead and an addend.  On planes of few blocks only, where mie_tconv2x_takes_lead (host logic; `blocks` =
- * mie_tile_capacity of the block set, dtype MIE_DTYPE_BF16 or MIE_DTYPE_F32_BF16X3); MIE_ERR_UNSUPPORTED elsewhere.
+ * in place of mie_tconv_masked of the lead and an addend.  MIE_DTYPE_BF16 or MIE_DTYPE_F32_BF16X3 (MIE_ERR_UNSUPPORTED otherwise).
  */
-int mie_tconv2x_takes_lead(int c1, int c2, int cout, int blocks, int dtype);
 int mie_tconv2x_lead_masked(const void* lead, const uint8_t* lead_mask, const float* lead_filter, const void* x, const uint8_t* xmask, int c1,
                             const void* x2, const uint8_t* x2mask, int c2, int h_in, int w_in, const float* filter, const void* filter_mc,
                             int cin_total, int cout, const mie_tileset* out, const mie_tileset* blocks, void* out_delta, float* reservoir,

@@ -38,7 +38,7 @@ EXPORTS = (
     "mie_conv_masked_ws", "mie_convgru_gates_incr", "mie_upsample2x_pair_incr", "mie_conv_masked_noalloc",
     "mie_convlstm_gates_refresh", "mie_convgru_gates_refresh", "mie_mul_dense", "mie_tconv2x_masked",
     "mie_tconv2x_refresh", "mie_conv_f32x3_takes", "mie_conv_needs_no_workspace", "mie_upconv_needs_no_workspace", "mie_conv_gru_masked", "mie_tconv2x_lead_masked",
-    "mie_tconv2x_takes_lead", "mie_build_mask_plan", "mie_build_mask_plan_wgs",
+    "mie_build_mask_plan", "mie_build_mask_plan_wgs",
     "mie_upconv2x_masked", "mie_upconv2x_refresh", "mie_pack_filter_up2x", "mie_call_index", "mie_call_signature", "mie_run_calls",
 )
 PLAN_MAX_STEPS = 40
@@ -119,8 +119,6 @@ def _declare(l):
     l.mie_tconv2x_masked.restype = ci
     l.mie_tconv2x_masked.argtypes = [vp, vp, ci, vp, vp, ci, ci, ci, vp, vp, ci, ci, ci, tsp, tsp, vp, vp, vp, ci, cf, ci,
                                      vp, ctypes.c_longlong, vp]
-    l.mie_tconv2x_takes_lead.restype = ci
-    l.mie_tconv2x_takes_lead.argtypes = [ci, ci, ci, ci, ci]
     l.mie_tconv2x_lead_masked.restype = ci
     l.mie_tconv2x_lead_masked.argtypes = [vp, vp, vp, vp, vp, ci, vp, vp, ci, ci, ci, vp, vp, ci, ci, tsp, tsp, vp, vp, ci, cf, ci, vp]
     l.mie_tconv2x_refresh.restype = ci

@@ -199,7 +199,6 @@ bool mie_launch_conv_gru(const ConvArgsT<float>& a, unsigned cap, hipStream_t st
 bool mie_launch_conv_gru(const ConvArgsT<mie_bf16>& a, unsigned cap, hipStream_t st);
 // The 3x3 stride-2 transposed conv on planes of few blocks, in one launch; a.g_cpd, a.g_cpm, a.g_cpres: two more input channels, their
 // mask and their filter rows.
-bool mie_tconv_deep_form(int c1, int c2, int cout, long long blocks, int dtype);
 bool mie_launch_tconv_deep(const ConvArgsT<float>& a, const TileSetDev& blocks, hipStream_t st);
 bool mie_launch_tconv_deep(const ConvArgsT<mie_bf16>& a, const TileSetDev& blocks, hipStream_t st);
 bool mie_launch_gru_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);

@@ -635,7 +635,7 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_tconv_deep(ConvArgsT<T> a, Til
 
   // ---- two more input channels (a.g_cpd with its mask a.g_cpm, plain filter rows a.g_cpres), in fp32: an output pixel sees the one, two or
   // four taps of its phase.  Asked for here, where the filter's registers are free, and added behind the sums.  (As a launch of their
-  // own and an addend, optical flow with transposed decoders, two such layers: 312.4 -> 304.9 us a pass.)
+  // own and an addend, optical flow with transposed decoders, two such layers: 312.4 -> 304.9 us a pass, a third in k_tconv_mfma -> 300.3.)
   float2 lx2[4];
   float4 lf[4][2];
   unsigned lead_b[4], lead_in = 0u;
@@ -705,7 +705,7 @@ int deep_dtype(const ConvArgsT<T>& a) { return sizeof(T) == 2 ? MIE_DTYPE_BF16 :
 template <typename T>
 bool deep_tconv(const ConvArgsT<T>& a, const TileSetDev& pts, hipStream_t st) {
   const long long cap = (long long)pts.n * pts.tiles_y * pts.tiles_x, slabs = deep_slabs(cap, a.cout);
-  if (!mie_tconv_deep_form(a.c1, a.c2, a.cout, cap, deep_dtype(a))) return false;
+  if ((sizeof(T) == 4 && !a.x3) || a.c1 % 32 != 0 || a.c2 % 32 != 0 || a.c1 + a.c2 < 128 || a.cout % DEEP_COLS != 0 || slabs > DEEP_WGS) return false;
   if (4 * slabs <= DEEP_WGS)
     hipLaunchKernelGGL((k_tconv_deep<T, 2>), dim3(a.cout / DEEP_COLS, 4 * (unsigned)cap), dim3(DEEP_THREADS), 0, st, a, pts);
   else
@@ -763,10 +763,6 @@ bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles,
   // the other way 512->512 at 16x32 22.3 and 23.4, 256+256->256 at 32x32 21.4 and 22.4.  Optical flow, up-sampling decoder, 433.1 -> 428.2)
   if (dtype == MIE_DTYPE_F32_BF16X3 && k == 3 && s == 1 && 2 * deep_slabs(tiles, cout) > DEEP_WGS && c1 + c2 > 512) return false;
   return deep_slabs(tiles, cout) <= DEEP_WGS;
-}
-bool mie_tconv_deep_form(int c1, int c2, int cout, long long blocks, int dtype) {
-  return (dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3) && c1 % 32 == 0 && c2 % 32 == 0 && c1 + c2 >= 128 && cout % DEEP_COLS == 0 &&
-         deep_slabs(blocks, cout) <= DEEP_WGS;
 }
 // (fp32 of eight rows a workgroup: 128->64 at 64x64 17.8 us, k_upconv2x 16.1)
 bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype) {

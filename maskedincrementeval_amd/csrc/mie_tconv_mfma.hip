@@ -318,6 +318,49 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
     } else {
       float4 r0[PER], add[PER];
       conv_epilogue_load4<T, PER>(a, off, ok, r0, add);
+      if constexpr (K == 3) {
+        // two more input channels, as in k_tconv_deep, in the epilogue's trip (a thread's groups have one column).  Against a launch
+        // of their own and an addend, all active, fp32 / bf16: 64+64->32 from 128x128 29.0 -> 20.0 / 21.5 -> 14.7 us, from 2x240x320
+        // 238 -> 187 / 111 -> 74, 128->128 from 132x176 115 -> 95 / 70 -> 47.
+        if (a.g_cpd != nullptr) {
+          constexpr int NT = (1 + py) * (1 + px);
+          int lat[NT * PER];
+          float2 lx[NT * PER];
+          float4 lf[NT][2];
+          unsigned in = 0u, lb[NT * PER];
+#pragma unroll
+          for (int q = 0; q < NT; ++q) {
+            const int r = px ? q >> 1 : q, c = px ? q & 1 : 0;
+            const int ky = r != 0 ? 0 : py ? 2 : 1, kx = c != 0 ? 0 : px ? 2 : 1;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) lf[q][e] = *reinterpret_cast<const float4*>(a.g_cpres + (long long)(9 * e + 3 * ky + kx) * cout + co[0]);
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+              const int p = (tid + 256 * i) / QPP, iy = y0 + (p >> 3) + r, ix = x0 + (p & 7) + c, at = q * PER + i;
+              const bool k = ok[i] && iy < a.h_in && ix < a.w_in;
+              lat[at] = k ? (n * a.h_in + iy) * a.w_in + ix : 0;
+              in |= (k ? 1u : 0u) << at;
+              if constexpr (sizeof(T) == 4) {
+                lx[at] = *reinterpret_cast<const float2*>(a.g_cpd + 2LL * lat[at]);
+              } else {
+                const uint32_t b = *reinterpret_cast<const uint32_t*>(a.g_cpd + 2LL * lat[at]);
+                lx[at] = make_float2(__uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u));
+              }
+            }
+          }
+          mie_mask_ask(a.g_cpm, a.filt_mc, lat, lb);
+          const unsigned kk = mie_mask_take(a.g_cpm, lb, in);
+#pragma unroll
+          for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+              const int at = q * PER + i;
+              const float u = (kk >> at) & 1u ? lx[at].x : 0.f, w = (kk >> at) & 1u ? lx[at].y : 0.f;
+              v[i].x += u * lf[q][0].x + w * lf[q][1].x; v[i].y += u * lf[q][0].y + w * lf[q][1].y;
+              v[i].z += u * lf[q][0].z + w * lf[q][1].z; v[i].w += u * lf[q][0].w + w * lf[q][1].w;
+            }
+        }
+      }
       const unsigned live_bits = mie_mask_take(live_m, live_b, ~0u);
       bool live[PER];
 #pragma unroll
@@ -428,14 +471,9 @@ int tconv2x_impl(const char* who, const void* x, const uint8_t* xmask, int c1, c
   a.ts = mie_dev_tileset(out);
   const TileSetDev pts = mie_dev_tileset(blocks);
   if (lead != nullptr) {
-    const int dtype = sizeof(T) == 2 ? MIE_DTYPE_BF16 : x3 ? MIE_DTYPE_F32_BF16X3 : MIE_DTYPE_F32;
     MIE_REQUIRE(lead_filter != nullptr && mie_aligned(lead, 2 * sizeof(T)) && mie_aligned(lead_filter, 16) && lead != out_delta, MIE_ERR_INVALID_ARG,
                 "%s: lead and its filter rows must be given together, aligned, and not alias the output", who);
-    MIE_REQUIRE(k == 3 && mie_tconv_deep_form(c1, c2, cout, (long long)pts.n * pts.tiles_y * pts.tiles_x, dtype), MIE_ERR_UNSUPPORTED,
-                "%s: only where mie_tconv2x_takes_lead (k=%d c1=%d c2=%d cout=%d)", who, k, c1, c2, cout);
     a.g_cpd = (const T*)lead; a.g_cpm = lead_mask; a.g_cpres = const_cast<float*>(lead_filter);
-    mie_launch_tconv_deep(a, pts, (hipStream_t)stream);
-    return mie_check_launch(who);
   }
   bool ok;
   if constexpr (sizeof(T) == 4) {
@@ -483,10 +521,6 @@ extern "C" int mie_tconv2x_refresh(const void* x, int c1, const void* x2, int c2
                                   blocks, out_dense, addend, reservoir, act_kind, slope, true, bias, nullptr, 0, stream);
   return tconv2x_impl<float>(who, x, nullptr, c1, x2, nullptr, c2, h_in, w_in, filter, filter_mc, cin_total, k, cout, out, blocks,
                              out_dense, addend, reservoir, act_kind, slope, true, bias, nullptr, 0, stream, x3);
-}
-
-extern "C" int mie_tconv2x_takes_lead(int c1, int c2, int cout, int blocks, int dtype) {
-  return mie_tconv_deep_form(c1, c2, cout, blocks, dtype) ? 1 : 0;
 }
 
 extern "C" int mie_tconv2x_lead_masked(const void* lead, const uint8_t* lead_mask, const float* lead_filter, const void* x, const uint8_t* xmask,

@@ -499,9 +499,7 @@ class TransposedConvLayerIncr(replay.Watched, nn.Module):
                 # the flow estimate of the previous scale shares the mask of x (a 1x1 conv + tanh of it), so the
                 # wide conv's output mask covers this partial result
                 lead_c = chans[0]
-                n, _, h, w = parts[0][0].shape
-                if ops.tconv2x_takes_lead(lead_c, chans[1], chans[2], tc.out_channels, tc._geometry()[0], n * ((h + 7) // 8) * ((w + 7) // 8),
-                                          ops.delta_torch_dtype(parts[0][0])):
+                if ops.tconv2x_takes_lead(lead_c, chans[1], chans[2], tc.out_channels, tc._geometry()[0], ops.delta_torch_dtype(parts[0][0])):
                     kind, slope = activation_kind(self.activation.op)
                     return tc.forward(parts[1], self.activation.in_res.reservoir, kind, slope, x2_incr=parts[2],
                                       filt=filt.rows(lead_c, filt.shape[0]), lead_incr=parts[0], lead_filt=filt.rows(0, lead_c))

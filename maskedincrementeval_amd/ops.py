@@ -1061,12 +1061,10 @@ def tconv2x_takes(c1: int, c2: int, cout: int, k: int, stride: int, pad: int, ou
             and c1 % chunk == 0 and c2 % chunk == 0 and cout % 32 == 0 and filt.for_dtype(dtype)[1] is not None)
 
 
-def tconv2x_takes_lead(lead_c: int, c1: int, c2: int, cout: int, k: int, blocks: int, dtype) -> bool:
-    """Whether tconv2x_masked, where it takes a layer of this shape, takes a leading part of `lead_c` channels too (blocks: capacity of
-    its block set)."""
-    code = _lib.DTYPE_BF16 if dtype == torch.bfloat16 else _lib.DTYPE_F32_BF16X3
-    return (lead_c == 2 and k == 3 and c1 % 64 == 0 and c2 % 64 == 0 and (dtype == torch.bfloat16 or f32_matmul == "bf16x3")
-            and bool(lib().mie_tconv2x_takes_lead(c1, c2, cout, blocks, code)))
+def tconv2x_takes_lead(lead_c: int, c1: int, c2: int, cout: int, k: int, dtype) -> bool:
+    """Whether tconv2x_masked takes a leading part of `lead_c` channels along with a layer of this shape."""
+    return (lead_c == 2 and k == 3 and c1 % 64 == 0 and c2 % 64 == 0 and cout % 32 == 0
+            and (dtype == torch.bfloat16 or (dtype == torch.float32 and f32_matmul == "bf16x3")))
 
 
 def _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out, addend, reservoir):

@@ -65,7 +65,8 @@ def test_transposed_conv_in_one_launch(n, c1, c2, cout, h, w, dtype):
 
 # two more input channels in front (a part whose mask the wide parts' covers): every phase, planes cut off at both edges, two and four rows
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("n,c1,c2,cout,h,w", [(1, 128, 0, 32, 1, 1), (2, 64, 64, 32, 5, 9), (1, 128, 128, 128, 31, 32), (1, 64, 64, 64, 63, 64)])
+@pytest.mark.parametrize("n,c1,c2,cout,h,w", [(1, 128, 0, 32, 1, 1), (2, 64, 64, 32, 5, 9), (1, 128, 128, 128, 31, 32), (1, 64, 64, 64, 63, 64),
+                                              (1, 64, 0, 32, 13, 11), (2, 64, 64, 32, 100, 125), (1, 64, 0, 128, 150, 170)])
 def test_transposed_conv_with_a_leading_part(n, c1, c2, cout, h, w, dtype):
     bf, cin = dtype == torch.bfloat16, c1 + c2
     q = (lambda t: t.to(dtype).float()) if bf else (lambda t: t)
@@ -73,7 +74,7 @@ def test_transposed_conv_with_a_leading_part(n, c1, c2, cout, h, w, dtype):
     filt = ops.ConvFilter(wt.permute(0, 2, 3, 1).contiguous().to(DEV))
     ho, wo = 2 * h, 2 * w
     ts, blocks, out = TileMask(n, ho, wo, DEV), TileMask(n, h, w, DEV), ops.new_nhwc(n, cout, ho, wo, DEV, dtype)
-    assert ops.tconv2x_takes_lead(2, c1, c2, cout, 3, blocks.capacity, dtype)
+    assert ops.tconv2x_takes_lead(2, c1, c2, cout, 3, dtype)
     up = lambda x, f: F.conv_transpose2d(x.double(), f.double(), stride=2, padding=1, output_padding=1)
     ref = torch.zeros(n, cout, ho, wo, dtype=torch.float64)
     res, tol = _dev(ref.float()), torch.zeros_like(ref)
@@ -100,13 +101,6 @@ def test_transposed_conv_with_a_leading_part(n, c1, c2, cout, h, w, dtype):
                            out, res, lead=(_dev(x[:, :1]), dm0, filt.rows(0, 1)))
 
 
-def test_leading_part_only_where_the_one_launch_form_is():
-    assert not ops.tconv2x_takes_lead(2, 64, 0, 64, 3, 4, torch.float32) and not ops.tconv2x_takes_lead(2, 128, 0, 64, 5, 4, torch.float32)
-    assert not ops.tconv2x_takes_lead(3, 128, 0, 64, 3, 4, torch.bfloat16) and not ops.tconv2x_takes_lead(2, 128, 0, 64, 3, 65, torch.bfloat16)
-    filt = ops.ConvFilter(torch.randn(66, 3, 3, 64, device=DEV))
-    ts, blocks = TileMask(1, 16, 16, DEV), TileMask(1, 8, 8, DEV)
-    for t, s in ((ts, 16), (blocks, 8)):
-        ops.build_mask_tiles(None, None, 1, s, s, _lib.FOOT_CONV, 1, 1, 0, t)
-    x, out = ops.new_nhwc(1, 64, 8, 8, DEV).zero_(), ops.new_nhwc(1, 64, 16, 16, DEV)
-    with pytest.raises(Exception, match="takes_lead"):
-        ops.tconv2x_masked(x, None, None, None, filt.rows(2, 66), 3, ts, blocks, out, lead=(ops.new_nhwc(1, 2, 8, 8, DEV).zero_(), None, filt.rows(0, 2)))
+def test_where_a_leading_part_goes_along():
+    assert not ops.tconv2x_takes_lead(2, 96, 0, 64, 3, torch.float32) and not ops.tconv2x_takes_lead(2, 128, 0, 64, 5, torch.float32)
+    assert not ops.tconv2x_takes_lead(3, 128, 0, 64, 3, torch.bfloat16) and not ops.tconv2x_takes_lead(2, 128, 0, 48, 3, torch.bfloat16)
