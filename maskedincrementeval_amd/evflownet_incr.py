@@ -461,8 +461,8 @@ class TransposedConvLayerIncr(replay.Watched, nn.Module):
     """Transposed conv (stride 2, output_padding 1) -> activation over the concat of the parts:
     the decoder kind the benchmark configuration of this network names.  As in the up-sampling
     decoder the concat [previous flow (2 ch, optional), x, skip] is never formed: the two wide parts
-    are the two input pointers of the matrix-core transposed conv, the narrow leading part goes
-    through the gather kernel and rides in as the addend."""
+    are the two input pointers of the matrix-core transposed conv; the narrow leading part goes along in
+    its epilogue (ops.tconv2x_takes_lead), else through a kernel of its own and in as the addend."""
 
     def __init__(self, in_channels, out_channels, kernel_size, activation="relu", padding=None, norm=None,
                  fuse=True):
