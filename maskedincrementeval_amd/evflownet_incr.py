@@ -110,18 +110,19 @@ class ConvGRUIncr(replay.Watched, nn.Module, _IncrBuffers):
     # -- one conv for both gates + one gate-math kernel (state reset each step) -------------------
     def _stacked_filter(self, interleaved=False):
         """ConvFilter of the update-gate and out-gate filters side by side: columns [0, hid) | [hid, 2*hid), or (interleaved) in the
-        order of ops.gru_interleave_index."""
+        order of ops.gru_interleave_index.  Which of the two a step takes follows ops.f32_matmul and the deltas' type, call by call; a
+        captured step holds addresses, so each order keeps its own while the weights are the same."""
         wu, wo = self.update_gate.weight, self.out_gate.weight
-        tag = (wu.data_ptr(), wu._version, wo.data_ptr(), wo._version, str(wu.device), interleaved)
-        cached = self.__dict__.get("_stacked_filt_cache")
+        tag = (wu.data_ptr(), wu._version, wo.data_ptr(), wo._version, str(wu.device))
+        cache = self.__dict__.setdefault("_stacked_filters", {})
+        cached = cache.get(interleaved)
         if cached is None or cached[0] != tag:
             wu, wo = wu.detach(), wo.detach()
             if interleaved:
                 both = torch.stack([t.reshape(-1, 4, *t.shape[1:]) for t in (wu, wo)], 1).flatten(0, 2)
             else:
                 both = torch.cat((wu, wo), 0)                                  # [2*hid, cin, k, k]
-            cached = (tag, ops.ConvFilter(both.permute(1, 2, 3, 0).contiguous().float()))
-            self.__dict__["_stacked_filt_cache"] = cached
+            cached = cache[interleaved] = (tag, ops.ConvFilter(both.permute(1, 2, 3, 0).contiguous().float()))
         return cached[1]
 
     def _forward_stacked(self, input_incr):
