@@ -755,8 +755,12 @@ bool deep_up(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
 }  // namespace
 
 bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype) {
-  if (dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) return false;
+  if (c1 <= 0 || c2 < 0 || cout <= 0 || tiles <= 0) return false;
   if (!((k == 3 && (s == 1 || s == 2)) || (k == 5 && s == 2))) return false;
+  // what comes to the matrix cores at all (the query must not name other layers: they run on the VALU); 3x3 stride 2 in three terms
+  // does in this form only
+  if (dtype == MIE_DTYPE_BF16 ? !mie_conv_mfma_takes(k, s, dtype, c1, c2, cout)
+                              : dtype != MIE_DTYPE_F32_BF16X3 || !((k == 3 && s == 2) || mie_conv_x3_takes(k, s, c1, c2, cout))) return false;
   if (c1 % 32 != 0 || c2 % 32 != 0 || c1 + c2 < (k == 3 ? 64 : 32) || cout % DEEP_COLS != 0) return false;
   // (fp32 of eight rows a workgroup splits its pixels into terms for 16 columns only, one pass of chunks behind the other: with more than
   // 512 channels the split form is faster.  512+512->512 at 16x32 39.1 us, 34.5 there, ->256 at 32x32 38.3, 34.6;
@@ -766,7 +770,8 @@ bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles,
 }
 // (fp32 of eight rows a workgroup: 128->64 at 64x64 17.8 us, k_upconv2x 16.1)
 bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype) {
-  if ((dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) || c % 32 != 0 || cout % DEEP_COLS != 0) return false;
+  if ((dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) || c <= 0 || cout <= 0 || tiles <= 0) return false;
+  if (c % (dtype == MIE_DTYPE_BF16 ? 64 : 32) != 0 || cout % 32 != 0) return false;      // (other layers are refused)
   return dtype == MIE_DTYPE_BF16 ? deep_slabs(tiles, cout) <= DEEP_WGS : 2 * deep_slabs(tiles, cout) <= DEEP_WGS && c <= 128;
 }
 

@@ -370,6 +370,22 @@ def test_three_term_shape_query_needs_no_gpu(mie_lib):
     assert takes(3, 1, 48, 0, 64) == 0 and takes(3, 1, 64, 0, 48) == 0 and takes(5, 2, 24, 0, 64) == 0
 
 
+def test_workspace_queries_name_layers_of_the_matrix_cores_only(mie_lib):
+    """mie_conv_needs_no_workspace / mie_upconv_needs_no_workspace: host logic; layers that run on the VALU, or are refused, are not named."""
+    bf, x3 = _lib.DTYPE_BF16, _lib.DTYPE_F32_BF16X3
+    q = mie_lib.mie_conv_needs_no_workspace
+    assert q(3, 1, 128, 64, 256, 16, bf) == 1 and q(3, 1, 96, 64, 256, 16, bf) == 0 and q(3, 1, 64, 0, 48, 2, bf) == 0
+    assert q(5, 2, 32, 0, 64, 6, bf) == 1 and q(5, 2, 32, 0, 32, 6, bf) == 0 and q(5, 2, 64, 0, 32, 6, bf) == 1
+    assert q(3, 2, 64, 32, 64, 2, bf) == 1 and q(3, 2, 64, 32, 32, 2, bf) == 0 and q(3, 2, 64, 0, 48, 2, bf) == 0
+    assert q(3, 1, 96, 64, 256, 16, x3) == 1 and q(3, 1, 64, 0, 48, 2, x3) == 0 and q(5, 2, 32, 0, 48, 2, x3) == 0
+    assert q(3, 2, 64, 0, 48, 2, x3) == 1 and q(3, 2, 48, 48, 32, 2, x3) == 0 and q(3, 2, 64, 0, 64, 2, _lib.DTYPE_F32) == 0
+    for wrong in ((0, 64, 64, 2), (128, -32, 64, 2), (64, 0, 0, 2), (64, 0, 64, 0), (64, 0, 64, -1)):
+        assert q(3, 1, *wrong, bf) == 0 and q(3, 1, *wrong, x3) == 0, wrong
+    u = mie_lib.mie_upconv_needs_no_workspace
+    assert u(64, 32, 4, bf) == 1 and u(32, 32, 4, bf) == 0 and u(64, 48, 4, bf) == 0
+    assert u(32, 32, 4, x3) == 1 and u(48, 32, 4, x3) == 0 and u(32, 48, 4, x3) == 0 and u(64, 32, 0, x3) == 0 and u(0, 32, 4, bf) == 0
+
+
 def test_call_sequences_check_what_they_are_given(mie_lib):
     # every sequence below is rejected before a launch, or ends at a call whose own validation rejects it
     idx = mie_lib.mie_call_index(b"mie_mask_from_delta")

@@ -23,10 +23,10 @@ def _dev(t):
     (1, 64, 0, 32, 1, 1, 1), (2, 64, 64, 64, 3, 2, 1), (1, 192, 0, 32, 5, 9, 1), (1, 256, 128, 96, 13, 11, 0), (1, 320, 0, 32, 9, 7, 2),
     (1, 512, 0, 64, 16, 17, 1), (3, 256, 64, 32, 12, 8, 3), (1, 128, 0, 256, 16, 16, 1), (1, 64, 0, 256, 16, 24, 1),
     (1, 64, 64, 512, 16, 16, 1), (1, 64, 0, 512, 16, 24, 1), (2, 64, 0, 512, 16, 16, 1), (1, 128, 0, 512, 24, 24, 1),
-    (1, 64, 0, 256, 32, 32, 1), (1, 96, 64, 256, 31, 29, 1), (1, 64, 0, 256, 32, 33, 1), (1, 512, 32, 512, 16, 25, 1)]] + [(5, 2) + shape for shape in [
-        (1, 32, 0, 32, 1, 1, 2), (2, 64, 32, 64, 6, 5, 2), (1, 96, 0, 32, 17, 33, 1), (1, 128, 0, 256, 16, 24, 2), (1, 32, 0, 64, 127, 128, 2),
+    (1, 64, 0, 256, 32, 32, 1), (1, 96, 64, 256, 31, 29, 1), (1, 128, 64, 256, 31, 29, 1), (1, 64, 0, 256, 32, 33, 1), (1, 512, 32, 512, 16, 25, 1)]] + [(5, 2) + shape for shape in [
+        (1, 32, 0, 32, 1, 1, 2), (1, 32, 0, 64, 1, 1, 2), (2, 64, 32, 64, 6, 5, 2), (1, 96, 0, 32, 17, 33, 1), (1, 96, 0, 64, 17, 33, 1), (1, 128, 0, 256, 16, 24, 2), (1, 32, 0, 64, 127, 128, 2),
         (1, 64, 0, 128, 64, 64, 2), (1, 32, 0, 64, 136, 128, 2)]] + [(3, 2) + shape for shape in [
-        (1, 64, 0, 32, 1, 1, 1), (2, 64, 32, 64, 5, 18, 1), (1, 128, 0, 512, 15, 16, 1), (1, 256, 64, 128, 31, 29, 1), (1, 64, 0, 256, 64, 64, 1),
+        (1, 64, 0, 32, 1, 1, 1), (2, 64, 32, 64, 5, 18, 1), (1, 64, 32, 48, 19, 21, 1), (1, 128, 0, 512, 15, 16, 1), (1, 256, 64, 128, 31, 29, 1), (1, 64, 0, 256, 64, 64, 1),
         (1, 64, 32, 64, 128, 127, 0), (1, 64, 0, 256, 64, 66, 1)]])
 def test_whole_contraction_in_a_workgroup(k, s, n, c1, c2, cout, h, w, pad, dtype):
     cin, bf = c1 + c2, dtype == torch.bfloat16
@@ -37,7 +37,10 @@ def test_whole_contraction_in_a_workgroup(k, s, n, c1, c2, cout, h, w, pad, dtyp
     ts = TileMask(n, ho, wo, DEV)
     tiles = ts.capacity
     takes = _lib.lib().mie_conv_needs_no_workspace(k, s, c1, c2, cout, tiles, _lib.DTYPE_BF16 if bf else _lib.DTYPE_F32_BF16X3)
-    assert takes == (tiles * (cout // 16) <= 256 and not (not bf and (k, s) == (3, 1) and tiles * (cout // 16) > 128 and cin > 512))
+    # (bf16 of other chunks of channels, and slabs of columns, than the matrix cores take: the VALU, not named)
+    whole = lambda c, m: c1 % c == 0 and c2 % c == 0 and cout % m == 0
+    matrix = whole(64, 32) or (s == 2 and whole(32, 64)) if bf else whole(32, 16 if (k, s) == (3, 2) else 32)
+    assert takes == (matrix and tiles * (cout // 16) <= 256 and not (not bf and (k, s) == (3, 1) and tiles * (cout // 16) > 128 and cin > 512))
     outs = [ops.new_nhwc(n, cout, ho, wo, DEV, dtype) for _ in range(2)]
     r0 = torch.randn(n, cout, ho, wo, generator=torch.Generator().manual_seed(5))
     ress = [_dev(r0) for _ in range(2)]
@@ -60,7 +63,7 @@ def test_whole_contraction_in_a_workgroup(k, s, n, c1, c2, cout, h, w, pad, dtyp
         before, tol = tol, tol + 4e-7 * bound + 2.0 ** -23 * (ref.abs() + sums.abs())
         for i, ws in enumerate((None, split)):
             ops.conv_masked(x1, dm, x2, None if x2 is None else dm, filt, k, s, pad, ts, outs[i], ress[i], _lib.ACT_RELU, 0.0,
-                            _lib.PATH_AUTO, None if add is None else _dev(add).to(dtype), workspace=ws)
+                            _lib.PATH_MFMA if takes and ws is None else _lib.PATH_AUTO, None if add is None else _dev(add).to(dtype), workspace=ws)
             torch.cuda.synchronize()
             off = (ress[i].cpu().double() - (ref + sums)).abs()
             assert (off <= tol).all(), (step, i)
