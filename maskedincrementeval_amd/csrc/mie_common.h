@@ -65,6 +65,13 @@ __device__ __forceinline__ unsigned mie_mask_take(const uint8_t* m, const unsign
   return (m == nullptr ? ~0u : bits) & want;
 }
 
+// Between what lanes of one wave write to LDS and what others of it read: LDS requests of a wave are served in order, so
+// only the compiler has to keep it, which the barrier alone (it touches no memory) does not ask of it.
+__device__ __forceinline__ void mie_wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // ---- host side: launches that share a workspace ----------------------------
 // The two launches of a split form belong together: between them the workspace holds the partial sums.  Threads that
 // enqueue on one stream with one workspace take turns pair by pair (the lock is held while two launches are enqueued).

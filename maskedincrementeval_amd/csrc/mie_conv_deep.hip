@@ -357,12 +357,12 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   for (int pass = 0, c = cg; pass * NCW < nch; ++pass, c += NCW) {
     if (!OWN && pass > 0) __syncthreads();
     store_x(pass);
-    if constexpr (OWN) __builtin_amdgcn_wave_barrier();
+    if constexpr (OWN) mie_wave_order();
     else __syncthreads();
     if ((pass + 1) * NCW < nch) load_x(pass + 1);
     if (c + NCW < nch) chunk(chunk_w(c + NCW), std::true_type());
     else if (c < nch) chunk(nullptr, std::false_type());
-    if constexpr (OWN) __builtin_amdgcn_wave_barrier();
+    if constexpr (OWN) mie_wave_order();
   }
   if constexpr (!OWN) __syncthreads();
 
@@ -623,14 +623,14 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_tconv_deep(ConvArgsT<T> a, Til
   };
   for (int c = wave; c < nch; c += DEEP_WAVES) {
     store_x(c);
-    __builtin_amdgcn_wave_barrier();
+    mie_wave_order();
     if (RING < 9 || c + DEEP_WAVES < nch) {      // (RING < 9: the chunk after the last is the first again, one form of the loop)
       load_x(c + DEEP_WAVES);
       chunk(chunk_w(c), chunk_w(c + DEEP_WAVES < nch ? c + DEEP_WAVES : 0), std::true_type());
     } else {
       chunk(chunk_w(c), nullptr, std::false_type());
     }
-    __builtin_amdgcn_wave_barrier();
+    mie_wave_order();
   }
 
   // ---- two more input channels (a.g_cpd with its mask a.g_cpm, plain filter rows a.g_cpres), in fp32: an output pixel sees the one, two or

@@ -224,13 +224,6 @@ typedef __bf16 fc_bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int FH_WAVES = 8;
 constexpr unsigned FH_GRID = 512;                 // two workgroups per CU
 
-// Between what lanes of one wave write to LDS and what others of it read: LDS requests of a wave are served in order, so
-// only the compiler has to keep it.
-__device__ __forceinline__ void fh_order() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 __device__ __forceinline__ unsigned fh_finite(unsigned v) {            // two bf16 values, zero where not finite
   const unsigned lo = (v & 0x7f80u) == 0x7f80u ? 0u : v & 0xffffu, hi = (v & 0x7f800000u) == 0x7f800000u ? 0u : v & 0xffff0000u;
   return lo | hi;
@@ -361,7 +354,7 @@ __global__ __launch_bounds__(64 * FH_WAVES, 4) void k_conv_fewcin_bf16(ConvArgsT
       r0[g] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (fast && ((live >> g) & 1u)) r0[g] = mie_ld4(a.res, (obase + (long long)g * wout) * cout + co0 + col);
     }
-    fh_order();
+    mie_wave_order();
 
     // ---- contraction: 8 rows of 8 pixels as two blocks of 32
     v16f acc[2];
@@ -376,7 +369,7 @@ __global__ __launch_bounds__(64 * FH_WAVES, 4) void k_conv_fewcin_bf16(ConvArgsT
         const uint4 u = s_in[pix];
         s_in[pix] = make_uint4(fh_finite(u.x), fh_finite(u.y), fh_finite(u.z), fh_finite(u.w));
       }
-      fh_order();
+      mie_wave_order();
     }
     const auto mul = [](v16f& c, const uint4& d, const uint4& w) {
       c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fc_bf16x8, d), __builtin_bit_cast(fc_bf16x8, w), c, 0, 0, 0);
@@ -396,7 +389,7 @@ __global__ __launch_bounds__(64 * FH_WAVES, 4) void k_conv_fewcin_bf16(ConvArgsT
       __builtin_amdgcn_sched_barrier(0);         // (operands of several units ahead would not fit the registers)
     }
     if (any_odd) {                               // ... and the others follow with the large terms
-      fh_order();
+      mie_wave_order();
 #pragma unroll 1
       for (int pix = lane; pix < NPIX; pix += 64) {
         const int iy = iy0 + pix / IT, ix = ix0 + pix % IT;
@@ -410,7 +403,7 @@ __global__ __launch_bounds__(64 * FH_WAVES, 4) void k_conv_fewcin_bf16(ConvArgsT
           dst[ch] = (f & 0x7f80) == 0x7f80 ? f : (unsigned short)0;
         }
       }
-      fh_order();
+      mie_wave_order();
 #pragma unroll 1
       for (int u = 0; u < UN; ++u) {
         const int t = 2 * u + half;
@@ -423,10 +416,10 @@ __global__ __launch_bounds__(64 * FH_WAVES, 4) void k_conv_fewcin_bf16(ConvArgsT
     // ---- epilogue: through LDS (over the staged tile, which is done with) to 16-byte groups of channels
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb) {
-      fh_order();
+      mie_wave_order();
 #pragma unroll
       for (int r = 0; r < 16; ++r) s_out[(8 * (r >> 2) + 4 * half + (r & 3)) * 32 + l32] = acc[mb][r];
-      fh_order();
+      mie_wave_order();
       if (fast) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -454,7 +447,7 @@ __global__ __launch_bounds__(64 * FH_WAVES, 4) void k_conv_fewcin_bf16(ConvArgsT
         }
       }
     }
-    fh_order();
+    mie_wave_order();
   }
 }
 

@@ -386,6 +386,20 @@ def test_workspace_queries_name_layers_of_the_matrix_cores_only(mie_lib):
     assert u(32, 32, 4, x3) == 1 and u(48, 32, 4, x3) == 0 and u(32, 48, 4, x3) == 0 and u(64, 32, 0, x3) == 0 and u(0, 32, 4, bf) == 0
 
 
+def test_wave_barriers_order_memory():
+    """__builtin_amdgcn_wave_barrier by itself does not order a wave's LDS accesses for the compiler: mie_wave_order, its fence with it, does."""
+    csrc = os.path.join(ROOT, "maskedincrementeval_amd", "csrc")
+    uses = {}
+    for name in sorted(os.listdir(csrc)):
+        if name.endswith((".hip", ".h")):
+            with open(os.path.join(csrc, name)) as f:
+                text = f.read()
+            if "amdgcn_wave_barrier" in text:
+                uses[name] = text
+    assert list(uses) == ["mie_common.h"], list(uses)
+    assert re.search(r'amdgcn_fence\(__ATOMIC_ACQ_REL, "wavefront"\);\s*__builtin_amdgcn_wave_barrier\(\);', uses["mie_common.h"])
+
+
 def test_call_sequences_check_what_they_are_given(mie_lib):
     # every sequence below is rejected before a launch, or ends at a call whose own validation rejects it
     idx = mie_lib.mie_call_index(b"mie_mask_from_delta")
