@@ -722,7 +722,7 @@ void launch_deep(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
   const long long slabs = deep_slabs(cap, a.cout);
   if (4 * slabs <= DEEP_WGS) launch_chunks<T, K, S, 2, KIND>(a, cap, st);
   else if (2 * slabs <= DEEP_WGS) launch_chunks<T, K, S, 4, KIND>(a, cap, st);
-  else launch_chunks<T, K, S, 8, KIND>(a, cap, st);
+  else if constexpr (!(sizeof(T) == 4 && KIND == DEEP_UP)) launch_chunks<T, K, S, 8, KIND>(a, cap, st);      // (mie_upconv_deep_form: not fp32)
 }
 
 template <typename T>

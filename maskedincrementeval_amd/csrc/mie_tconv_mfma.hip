@@ -318,7 +318,7 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
     } else {
       float4 r0[PER], add[PER];
       conv_epilogue_load4<T, PER>(a, off, ok, r0, add);
-      if constexpr (K == 3) {
+      if constexpr (K == 3 && (X3 || sizeof(T) == 2)) {      // (the types that mie_tconv2x_lead_masked takes)
         // two more input channels, as in k_tconv_deep, in the epilogue's trip (a thread's groups have one column).  Against a launch
         // of their own and an addend, all active, fp32 / bf16: 64+64->32 from 128x128 29.0 -> 20.0 / 21.5 -> 14.7 us, from 2x240x320
         // 238 -> 187 / 111 -> 74, 128->128 from 132x176 115 -> 95 / 70 -> 47.
