@@ -97,6 +97,10 @@ static __device__ long long* mie_prof_buf;       // set by mie_set_profile_buffe
 __host__ __device__ constexpr int stage_channels(int K, int S, bool HALF = false) {
   return ((K <= 5) ? 32 : 16) / (HALF ? 2 : 1);
 }
+// x extent of a grid in the XCD-aware launch order: the tile capacity rounded up to a multiple of 8, plus 16 (the shares of active
+// and of stale work are rounded up separately).  The kernel works its place out of it by the same formula: gridDim.x would be
+// one more trip to the launch's packet.
+__host__ __device__ constexpr int xcd_grid_x(int cap) { return ((cap + 7) & ~7) + 16; }
 // bf16 tiles are single-buffered at stride 1 as well: a bf16 workgroup spends a few microseconds on
 // the matrix cores, so what hides its latencies is the number of workgroups resident on the CU (LDS
 // per workgroup halves), not the overlap inside one (measured: +10 % on the 8x480x640 decoder conv).
@@ -328,13 +332,13 @@ __device__ void conv_quad_again(const ConvArgsT<T>& a, int n, int oy, int ox, in
   conv_store(a, off, co, s.x); conv_store(a, off + 1, co + 1, s.y); conv_store(a, off + 2, co + 2, s.z); conv_store(a, off + 3, co + 3, s.w);
 }
 
-// (tile, slab, part) of a workgroup of a split launch (x, y, z of the grid).  A few per cent of such a launch are its filter's way
-// into the L2s: in launch order the tiles of a (slab, part) -- a filter slice -- lie on different XCDs (4 tiles, two slabs:
-// all 8), and each of them fetches the slice.  Here every tile of a slice is on one XCD, an eighth of the slices on each.
-// Grids whose slices do not divide by 8 keep the launch order.  Whole passes, launch order -> this: optical flow 1x256x256
-// 366.7 -> 361.7 us (transposed convs), 467.9 -> 459.5 (up-sampling), e2depth 1x128x128 246.4 -> 243.8, 1x64x96 181.1 ->
-// 180.6 (two tiles: a slice was on two XCDs).
-// The grid is (slab, part) by tile for that: the hardware deals workgroups out to the XCDs in launch order, x fastest.
+// (tile, slab, part) of a workgroup of a split launch, whose grid is (slab x part, tile).  A few per cent of such a launch are its
+// filter's way into the L2s: a filter slice, of one slab and part, is fetched by every XCD that has one of its tiles.  The hardware
+// deals workgroups out to the XCDs in launch order, x fastest, so that where the slices are a multiple of 8 all tiles of a slice are on
+// one XCD, an eighth of the slices on each; of other numbers the tiles of a slice spread over 8 / gcd(8, slices) of them (4 slices,
+// one slab in four parts: two).  Whole passes, (tile, slab, part) grid -> this: optical flow
+// 1x256x256 366.7 -> 361.7 us (transposed convs), 467.9 -> 459.5 (up-sampling), e2depth 1x128x128 246.4 -> 243.8, 1x64x96 181.1 -> 180.6
+// (two tiles: a slice was on two XCDs).
 template <typename T>
 __device__ __forceinline__ void split_order(const ConvArgsT<T>& a, int& bx, int& by, int& bz) {
   const int slice = bx, lp = a.xcd_fs;        // (of a split launch: log2 of the parts)
@@ -434,7 +438,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     const int lg = __builtin_ctz(a.xcd_fs), sh = 3 - lg, up = (1 << sh) - 1;      // groups, XCDs of a group
     const int spg = (a.cout / CO_BLK) >> lg;                 // slabs per group
     const int xcd = bx & 7, k = xcd & up;
-    const int slot = by * ((((cap + 7) & ~7) + 16) >> 3) + (bx >> 3);             // launch order within the XCD
+    const int slot = by * (xcd_grid_x(cap) >> 3) + (bx >> 3);                     // launch order within the XCD
     const int guess = mie_tile_div(k * ((cap * spg + up) >> sh) + slot, spg, a.xcd_m);
     TileAsk ask = mie_tile_ask(a.ts, guess);
     asm("" : "+s"(ask.spec), "+s"(ask.n_active), "+s"(ask.n_stale));
@@ -1515,8 +1519,7 @@ int pick_slab(int cout, unsigned cap) {
 
 // XCD-aware launch order (see the kernel): chooses the number of slab groups a.xcd_fs in {1, 2, 4, 8}
 // (a divisor of the slab count) that minimises what the 8 L2s fetch in total -- the filter 8 / xcd_fs
-// times plus the input xcd_fs times -- and returns the grid's x extent: the tile capacity rounded up to a
-// multiple of 8, plus 16 (the shares of active and of stale work are rounded up separately).  The
+// times plus the input xcd_fs times -- and returns the grid's x extent (xcd_grid_x).  The
 // environment variable MIE_CONV_XCD forces the number of groups (0: plain launch order, a.xcd_fs = 0) --
 // a tuning knob for measurements, read once.
 template <typename T>
@@ -1540,7 +1543,7 @@ unsigned xcd_plan(ConvArgsT<T>& a, unsigned cap, int nslabs, int k, bool up = fa
   if (forced > 0 && 8 % forced == 0 && nslabs % forced == 0) best = forced;
   a.xcd_fs = best;
   a.xcd_m = mie_tile_magic((long long)cap * (nslabs / best), nslabs / best);
-  return ((cap + 7u) & ~7u) + 16u;
+  return (unsigned)xcd_grid_x((int)cap);
 }
 
 // X3 kernels (fp32 deltas, a.x3 set, the filter copy in the three-term layout): 3x3 / 5x5, stride 1, input channels in
