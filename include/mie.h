@@ -243,12 +243,16 @@ int mie_conv_f32x3_takes(int k, int stride, int c1, int c2, int cout);
 /*
  * Whether mie_conv_masked, without a workspace, runs a conv of this shape (matrix-core path; `tiles` = mie_tile_capacity of
  * its output, dtype with MIE_DTYPE_F32_BF16X3 where the call has it) in one launch faster than mie_conv_masked_ws runs it with one.
- * 0 for layers that the matrix-core path does not take, whatever their filter copy.
- * The same for mie_conv_gates_masked (k = 3, stride = 1, cout = 4 * hid) and mie_conv_gates_masked_ws.  Host logic only.
- * With MIE_DTYPE_F32_BF16X3 it also says where that call takes a 3x3 conv of stride 2 (which mie_conv_f32x3_takes does not name:
+ * 0 for layers that the matrix-core path does not take, whatever their filter copy.  Host logic only.
+ * Where it is 1 with MIE_DTYPE_F32_BF16X3, that call takes a 3x3 conv of stride 2 too (which mie_conv_f32x3_takes does not name:
  * on planes of more tiles it runs on the fp32 instruction).
  */
 int mie_conv_needs_no_workspace(int k, int stride, int c1, int c2, int cout, int tiles, int dtype);
+
+/*
+ * The same for mie_conv_gates_masked and mie_conv_gates_masked_ws.
+ */
+int mie_conv_gates_needs_no_workspace(int c1, int c2, int hid, int tiles, int dtype);
 
 /*
  * The same for mie_upconv_masked and mie_upconv_masked_ws, of more than 8 channels (c = channels of a and of b); 0 for layers that they refuse.

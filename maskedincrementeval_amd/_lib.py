@@ -37,7 +37,7 @@ EXPORTS = (
     "mie_maxpool_incr", "mie_accumulate", "mie_scale_incr", "mie_avgpool_incr", "mie_linear_incr", "mie_upconv_masked", "mie_upconv_masked_ws", "mie_upconv_pred_masked", "mie_upconv2x_pred_masked",
     "mie_conv_masked_ws", "mie_convgru_gates_incr", "mie_upsample2x_pair_incr", "mie_conv_masked_noalloc",
     "mie_convlstm_gates_refresh", "mie_convgru_gates_refresh", "mie_mul_dense", "mie_tconv2x_masked",
-    "mie_tconv2x_refresh", "mie_conv_f32x3_takes", "mie_conv_needs_no_workspace", "mie_upconv_needs_no_workspace", "mie_conv_gru_masked", "mie_tconv2x_lead_masked",
+    "mie_tconv2x_refresh", "mie_conv_f32x3_takes", "mie_conv_needs_no_workspace", "mie_conv_gates_needs_no_workspace", "mie_upconv_needs_no_workspace", "mie_conv_gru_masked", "mie_tconv2x_lead_masked",
     "mie_build_mask_plan", "mie_build_mask_plan_wgs",
     "mie_upconv2x_masked", "mie_upconv2x_refresh", "mie_pack_filter_up2x", "mie_call_index", "mie_call_signature", "mie_run_calls",
 )
@@ -143,6 +143,8 @@ def _declare(l):
     l.mie_conv_f32x3_takes.argtypes = [ci, ci, ci, ci, ci]
     l.mie_conv_needs_no_workspace.restype = ci
     l.mie_conv_needs_no_workspace.argtypes = [ci, ci, ci, ci, ci, ci, ci]
+    l.mie_conv_gates_needs_no_workspace.restype = ci
+    l.mie_conv_gates_needs_no_workspace.argtypes = [ci, ci, ci, ci, ci]
     l.mie_upconv_needs_no_workspace.restype = ci
     l.mie_upconv_needs_no_workspace.argtypes = [ci, ci, ci, ci]
     l.mie_pack_filter.restype = ci

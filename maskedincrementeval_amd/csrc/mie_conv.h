@@ -183,6 +183,9 @@ bool mie_launch_conv_mfma(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned c
 // so beforehand (`dtype` as the caller gave it; a gates conv: as the plain 3x3 one).
 bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype);
 bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype);
+// Whether they are also the faster form for a caller with a workspace.
+bool mie_conv_deep_faster(int k, int s, int c1, int c2, int cout, long long tiles, int dtype, bool gates);
+bool mie_upconv_deep_faster(int c, int cout, long long tiles, int dtype);
 bool mie_launch_conv_deep(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st);
 bool mie_launch_conv_deep(const ConvArgsT<mie_bf16>& a, int k, int s, unsigned cap, hipStream_t st);
 bool mie_launch_gates_deep(const ConvArgsT<float>& a, unsigned cap, hipStream_t st);

@@ -658,11 +658,15 @@ extern "C" int mie_conv_f32x3_takes(int k, int stride, int c1, int c2, int cout)
 }
 
 extern "C" int mie_conv_needs_no_workspace(int k, int stride, int c1, int c2, int cout, int tiles, int dtype) {
-  return mie_conv_deep_form(k, stride, c1, c2, cout, tiles, dtype) ? 1 : 0;
+  return mie_conv_deep_faster(k, stride, c1, c2, cout, tiles, dtype, false) ? 1 : 0;
+}
+
+extern "C" int mie_conv_gates_needs_no_workspace(int c1, int c2, int hid, int tiles, int dtype) {
+  return hid > 0 && hid <= (1 << 20) && mie_conv_deep_faster(3, 1, c1, c2, 4 * hid, tiles, dtype, true) ? 1 : 0;
 }
 
 extern "C" int mie_upconv_needs_no_workspace(int c, int cout, int tiles, int dtype) {
-  return mie_upconv_deep_form(c, cout, tiles, dtype) ? 1 : 0;
+  return mie_upconv_deep_faster(c, cout, tiles, dtype) ? 1 : 0;
 }
 
 extern "C" int mie_pack_filter(const float* filter, int cin, int k, int cout, void* packed,

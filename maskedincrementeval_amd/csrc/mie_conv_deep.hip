@@ -697,6 +697,7 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_tconv_deep(ConvArgsT<T> a, Til
 }
 
 long long deep_slabs(long long tiles, int cout) { return tiles * (cout / DEEP_COLS); }
+int deep_rows(long long slabs) { return 4 * slabs <= DEEP_WGS ? 2 : 2 * slabs <= DEEP_WGS ? 4 : 8; }      // (launch_deep)
 template <typename T>
 int deep_dtype(const ConvArgsT<T>& a) { return sizeof(T) == 2 ? MIE_DTYPE_BF16 : a.x3 ? MIE_DTYPE_F32_BF16X3 : MIE_DTYPE_F32; }
 
@@ -719,9 +720,9 @@ bool deep_tconv(const ConvArgsT<T>& a, const TileSetDev& pts, hipStream_t st) {
 // of 64 channels at 32x48, 384: 12.1 and 8.9; 5x5 64->128 at 48x48, 288: 19.5 and 16.1).
 template <typename T, int K, int S, int KIND>
 void launch_deep(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
-  const long long slabs = deep_slabs(cap, a.cout);
-  if (4 * slabs <= DEEP_WGS) launch_chunks<T, K, S, 2, KIND>(a, cap, st);
-  else if (2 * slabs <= DEEP_WGS) launch_chunks<T, K, S, 4, KIND>(a, cap, st);
+  const int rows = deep_rows(deep_slabs(cap, a.cout));
+  if (rows == 2) launch_chunks<T, K, S, 2, KIND>(a, cap, st);
+  else if (rows == 4) launch_chunks<T, K, S, 4, KIND>(a, cap, st);
   else if constexpr (!(sizeof(T) == 4 && KIND == DEEP_UP)) launch_chunks<T, K, S, 8, KIND>(a, cap, st);      // (mie_upconv_deep_form: not fp32)
 }
 
@@ -757,7 +758,7 @@ bool deep_up(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
 bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype) {
   if (c1 <= 0 || c2 < 0 || cout <= 0 || tiles <= 0) return false;
   if (!((k == 3 && (s == 1 || s == 2)) || (k == 5 && s == 2))) return false;
-  // what comes to the matrix cores at all (the query must not name other layers: they run on the VALU); 3x3 stride 2 in three terms
+  // what comes to the matrix cores at all (the queries must not name other layers: they run on the VALU); 3x3 stride 2 in three terms
   // does in this form only
   if (dtype == MIE_DTYPE_BF16 ? !mie_conv_mfma_takes(k, s, dtype, c1, c2, cout)
                               : dtype != MIE_DTYPE_F32_BF16X3 || !((k == 3 && s == 2) || mie_conv_x3_takes(k, s, c1, c2, cout))) return false;
@@ -773,6 +774,32 @@ bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype) {
   if ((dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) || c <= 0 || cout <= 0 || tiles <= 0) return false;
   if (c % (dtype == MIE_DTYPE_BF16 ? 64 : 32) != 0 || cout % 32 != 0) return false;      // (other layers are refused)
   return dtype == MIE_DTYPE_BF16 ? deep_slabs(tiles, cout) <= DEEP_WGS : 2 * deep_slabs(tiles, cout) <= DEEP_WGS && c <= 128;
+}
+
+// Whether the one-launch form is the faster one where the caller has a workspace for the split form.  A workgroup here has the
+// whole contraction, a few chunks at a time, and takes as long as there are channels; the split form has an eighth of it behind a
+// fixed cost of a second launch.  So the line is a number of input channels, and hardly depends on anything but the kind of
+// layer, the type and the rows a workgroup (2, 4, 8: how many columns and tiles there are).  One launch over split, median of 5 to 20
+// layers of other sizes and densities each, at the line and at the next count that was measured above it:
+//                  fp32, two rows     four               eight              bf16, two           four                eight
+//   3x3           512 .98, 640 1.05  576 .99, 640 1.03  256 .89, 320 1.05  1536 .97, 2048 1.2  1536 .91            1024 .96, 1280 1.04
+//   3x3 s2        448 .98, 512 1.05  640 .98, 768 1.02  1024 .97, 1280 1.02  896 .99, 1024 1.08  896 .96, 1536 1.2  576 1.0, 704 1.06
+//   5x5 s2        160 .96, 192 1.04  160 .91, 256 1.10  256 .98, 320 1.01  448 .99, 512 1.4    384 .98, 448 1.09   320 .92, 384 1.07
+//   gates         640 .91, 768 1.02  1024 .93, 1536 1.07  512 .76          2048 .94, 2560 1.04  3072 .83           3072 .73
+//   up            128 .84            128 .89            (none)             448 .97, 512 1.28   384 .87, 448 1.01   512 .99, 768 1.07
+// (3x3 fp32 of eight rows: 384 and 512, which fill its passes of four chunks, .98 and 1.01; 448 1.05.)  Far above it, 5x5 stride 2
+// of 512 / 1024 channels: fp32 1.6 / 2.1, up to 2.9 times as long, bf16 1.4 / 2.0.
+bool mie_conv_deep_faster(int k, int s, int c1, int c2, int cout, long long tiles, int dtype, bool gates) {
+  if (!mie_conv_deep_form(k, s, c1, c2, cout, tiles, dtype)) return false;
+  static const int most[4][2][3] = {{{512, 576, 256}, {1536, 1536, 1024}}, {{448, 640, 1024}, {896, 896, 576}}, {{160, 160, 256}, {448, 384, 320}},
+                                    {{640, 1024, 512}, {2048, 3072, 3072}}};
+  const int kind = gates ? 3 : k == 5 ? 2 : s - 1, bf = dtype == MIE_DTYPE_BF16 ? 1 : 0, rows = deep_rows(deep_slabs(tiles, cout)), c = c1 + c2;
+  return c <= most[kind][bf][rows / 4] || (kind == 0 && bf == 0 && rows == 8 && c % 128 == 0);
+}
+bool mie_upconv_deep_faster(int c, int cout, long long tiles, int dtype) {
+  if (!mie_upconv_deep_form(c, cout, tiles, dtype)) return false;
+  static const int most[3] = {448, 384, 512};
+  return dtype != MIE_DTYPE_BF16 || c <= most[deep_rows(deep_slabs(tiles, cout)) / 4];
 }
 
 bool mie_launch_conv_deep(const ConvArgsT<float>& a, int k, int s, unsigned cap, hipStream_t st) { return deep_plain(a, k, s, cap, st); }

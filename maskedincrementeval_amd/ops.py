@@ -1423,7 +1423,7 @@ def conv_gates_incr(x, xmask, x2, x2mask, filt: ConvFilter, out_ts: TileMask, ga
             raise ValueError("%s shape %s, expected %s" % (name, tuple(t.shape), (n, hid, h, w)))
     _ready(out_ts)
     small = mc_ptr is not None and out_ts.capacity * (cout // 32) <= 128 and workspace is None and split_enabled \
-        and not (one_launch and lib().mie_conv_needs_no_workspace(3, 1, c1, c2, cout, out_ts.capacity, code))
+        and not (one_launch and lib().mie_conv_gates_needs_no_workspace(c1, c2, hid, out_ts.capacity, code))
     ws_ptr, ws_bytes = _workspace_args(workspace, small, x.device)
     check(lib().mie_conv_gates_masked_ws(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1,

@@ -386,6 +386,24 @@ def test_workspace_queries_name_layers_of_the_matrix_cores_only(mie_lib):
     assert u(32, 32, 4, x3) == 1 and u(48, 32, 4, x3) == 0 and u(32, 48, 4, x3) == 0 and u(64, 32, 0, x3) == 0 and u(0, 32, 4, bf) == 0
 
 
+def test_workspace_queries_draw_the_line_where_the_split_form_is_faster(mie_lib):
+    """One launch up to so many input channels, by kind of layer, type and rows a workgroup (2, 4, 8: slabs of 16 columns x tiles)."""
+    bf, x3 = _lib.DTYPE_BF16, _lib.DTYPE_F32_BF16X3
+    conv = lambda k, s: lambda c, slabs, dt: mie_lib.mie_conv_needs_no_workspace(k, s, c, 0, 64, slabs // 4, dt)
+    gates = lambda c, slabs, dt: mie_lib.mie_conv_gates_needs_no_workspace(c - 64, 64, 16, slabs // 4, dt)
+    up = lambda c, slabs, dt: mie_lib.mie_upconv_needs_no_workspace(c, 64, slabs // 4, dt)
+    lines = [(conv(3, 1), x3, (512, 576, 256)), (conv(3, 1), bf, (1536, 1536, 1024)), (conv(3, 2), x3, (448, 640, 1024)), (conv(3, 2), bf, (896, 896, 576)),
+             (conv(5, 2), x3, (160, 160, 256)), (conv(5, 2), bf, (448, 384, 320)), (gates, x3, (640, 1024, 512)), (gates, bf, (2048, 3072, 3072)),
+             (up, x3, (128, 128)), (up, bf, (448, 384, 512))]
+    for query, dt, most in lines:
+        for line, (lo, hi) in zip(most, ((4, 64), (68, 128), (132, 256))):
+            assert [query(c, slabs, dt) for slabs in (lo, hi) for c in (line, line + 64)] == [1, 0, 1, 0], (dt, most, line)
+    assert [conv(3, 1)(c, 256, x3) for c in (384, 448, 512)] == [1, 0, 1]        # (whole passes of four chunks)
+    assert conv(3, 1)(64, 260, bf) == 0 and gates(128, 260, x3) == 0 and up(64, 132, x3) == 0 and up(64, 260, bf) == 0
+    for hid in (0, -4, (1 << 20) + 1):
+        assert mie_lib.mie_conv_gates_needs_no_workspace(64, 0, hid, 1, bf) == 0
+
+
 def test_wave_barriers_order_memory():
     """__builtin_amdgcn_wave_barrier by itself does not order a wave's LDS accesses for the compiler: mie_wave_order, its fence with it, does."""
     csrc = os.path.join(ROOT, "maskedincrementeval_amd", "csrc")
