@@ -136,7 +136,7 @@ class ConvGRUIncr(replay.Watched, nn.Module, _IncrBuffers):
         n, _, h, w = x.shape
         ts = conv._conv_tile_set("out_act", x, pix, None, None, k, s, p)
         if self.one_launch and (k, s, p) == (3, 1, 1) and x.is_cuda and ops.conv_gru_takes(x.shape[1], conv.weight.shape[1],
-                                                                                           self.hidden_size, x.dtype):
+                                                                                           self.hidden_size, x.dtype, ts.capacity):
             new_state = self._delta_buf("gru_state", (n, self.hidden_size, h, w), x.device, x.dtype)
             ops.conv_gru_incr(x, pix, self._stacked_filter(True), ts, self.sigmoid1.in_res.reservoir, self.tanh.in_res.reservoir, new_state)
             return [new_state, ts]
