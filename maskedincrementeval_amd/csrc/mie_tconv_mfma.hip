@@ -33,9 +33,14 @@ __host__ __device__ constexpr int tc_shift(int k, int pad) { return (tc_phase(k,
 // k-split stays over whole sub-chunks and every tap's phase is known at compile time), three bf16 planes in LDS,
 // single-buffered.  With the accumulators of four phases it needs 140-176 registers beside them: one workgroup per CU
 // (forcing two makes it spill and costs 1 % of the EVFlowNet frame; as it is the form gains 1-2 % there).
-template <typename T, int K, int WN, bool SPLIT, bool X3 = false>
+// LEAD: with two more input channels (a.g_cpd with its mask a.g_cpm, filter rows a.g_cpres).  Kernels of up to 64 columns take them
+// along by a branch; of 128 that costs registers where there are none (364 -> 408; bf16 128->128 from 2x120x160 96.9 us, with the
+// branch 98.3, from 150x170 66.8, 68.1), and they are two forms (with the two channels 79.4, by the branch 81.0; of 64 columns a form of its
+// own was slower, 27.3 -> 30.2).
+template <typename T, int K, int WN, bool SPLIT, bool X3 = false, bool LEAD = false>
 __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(ConvArgsT<T> a, TileSetDev pts) {
   static_assert(!X3 || sizeof(T) == 4, "X3: fp32 deltas");
+  constexpr bool ANY_LEAD = K == 3 && !SPLIT && (X3 || sizeof(T) == 2) && WN < 4;      // (the types that mie_tconv2x_lead_masked takes)
   using TL = std::conditional_t<X3, mie_bf16, T>;            // element type in LDS and on the matrix cores
   constexpr int PL = X3 ? 3 : 1;                             // operand planes (terms per value)
   constexpr int GPS = X3 ? 2 : 1;                            // 16-byte global loads per staging slot
@@ -318,11 +323,11 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
     } else {
       float4 r0[PER], add[PER];
       conv_epilogue_load4<T, PER>(a, off, ok, r0, add);
-      if constexpr (K == 3 && (X3 || sizeof(T) == 2)) {      // (the types that mie_tconv2x_lead_masked takes)
+      if constexpr (LEAD || ANY_LEAD) {
         // two more input channels, as in k_tconv_deep, in the epilogue's trip (a thread's groups have one column).  Against a launch
         // of their own and an addend, all active, fp32 / bf16: 64+64->32 from 128x128 29.0 -> 20.0 / 21.5 -> 14.7 us, from 2x240x320
         // 238 -> 187 / 111 -> 74, 128->128 from 132x176 115 -> 95 / 70 -> 47.
-        if (a.g_cpd != nullptr) {
+        if (LEAD || a.g_cpd != nullptr) {
           constexpr int NT = (1 + py) * (1 + px);
           int lat[NT * PER];
           float2 lx[NT * PER];
@@ -409,12 +414,16 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
   a.ws = nullptr;
   // (the 128-column kernel holds 4 phases x 2 blocks of accumulators and a four-column operand ring: in the three-term
   // form it would spill, so that form stops at 64 columns)
-  if (!X3 && cout % 128 == 0 && (long long)cap_p * (cout / 128) >= 400)
-    hipLaunchKernelGGL((k_tconv_mfma<T, K, 4, false, false>), dim3(cap_p, cout / 128), dim3(256), 0, st, a, pts);
-  else if (cout % 64 == 0 && (long long)cap_p * (cout / 64) >= 400)
+  if (!X3 && cout % 128 == 0 && (long long)cap_p * (cout / 128) >= 400) {
+    if (DEEP && a.g_cpd != nullptr)
+      hipLaunchKernelGGL((k_tconv_mfma<T, K, 4, false, false, DEEP && !X3>), dim3(cap_p, cout / 128), dim3(256), 0, st, a, pts);
+    else
+      hipLaunchKernelGGL((k_tconv_mfma<T, K, 4, false, false>), dim3(cap_p, cout / 128), dim3(256), 0, st, a, pts);
+  } else if (cout % 64 == 0 && (long long)cap_p * (cout / 64) >= 400) {
     hipLaunchKernelGGL((k_tconv_mfma<T, K, 2, false, X3>), dim3(cap_p, cout / 64), dim3(256), 0, st, a, pts);
-  else
+  } else {
     hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, false, X3>), dim3(cap_p, cout / 32), dim3(256), 0, st, a, pts);
+  }
   return true;
 }
 

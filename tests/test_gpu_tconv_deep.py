@@ -66,7 +66,7 @@ def test_transposed_conv_in_one_launch(n, c1, c2, cout, h, w, dtype):
 # two more input channels in front (a part whose mask the wide parts' covers): every phase, planes cut off at both edges, two and four rows
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,c1,c2,cout,h,w", [(1, 128, 0, 32, 1, 1), (2, 64, 64, 32, 5, 9), (1, 128, 128, 128, 31, 32), (1, 64, 64, 64, 63, 64),
-                                              (1, 64, 0, 32, 13, 11), (2, 64, 64, 32, 100, 125), (1, 64, 0, 128, 150, 170)])
+                                              (1, 64, 0, 32, 13, 11), (2, 64, 64, 32, 100, 125), (1, 64, 0, 64, 150, 170), (1, 64, 0, 128, 150, 170)])
 def test_transposed_conv_with_a_leading_part(n, c1, c2, cout, h, w, dtype):
     bf, cin = dtype == torch.bfloat16, c1 + c2
     q = (lambda t: t.to(dtype).float()) if bf else (lambda t: t)
