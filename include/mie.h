@@ -803,8 +803,9 @@ int mie_tconv_masked(const void* x, const uint8_t* xmask, int cin, int h_in,
  *        e.g. the contribution of a few more input channels computed by
  *        mie_tconv_masked, covered by `out`)
  *   workspace / workspace_bytes : as in mie_conv_masked_ws (on planes of very few
- *        blocks k = 5 and MIE_DTYPE_F32 split their contraction over up to 8
- *        workgroups; k = 3 in the other types has no use for it); may be NULL
+ *        blocks k = 5, MIE_DTYPE_F32 and MIE_DTYPE_F32_BF16X3 of more than 1408
+ *        channels split their contraction over up to 8 workgroups; k = 3 has no
+ *        other use for it); may be NULL
  * Replaces: transposed_conv2d_from_module
  * (incr_modules/mask_incr_functional.py:64-66) inside TransposedConvLayerIncr
  * (incr_modules/e2depth_incr.py:243-282).

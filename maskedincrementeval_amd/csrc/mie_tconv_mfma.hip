@@ -18,7 +18,7 @@
 // pixels (zeros where no input reaches, their reservoirs left alone), a stale block is zeroed, which covers every stale
 // output tile.
 // On planes of very few blocks the 3x3 form is another kernel, one launch (k_tconv_deep), for bf16 deltas and fp32 in three terms.
-// Of the others the chunks are split there over up to 8 workgroups that write partial sums to the workspace, and
+// Of the others, and of fp32 of very many channels, the chunks are split there over up to 8 workgroups that write partial sums to the workspace, and
 // k_conv_split_finish (walking the OUTPUT tile set) adds them and runs the epilogue.
 #include "mie_conv_mfma_impl.h"
 #include <type_traits>
@@ -384,17 +384,20 @@ template <typename T, int K, bool X3 = false>
 bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st) {
   constexpr int CC = X3 ? 64 : stage_channels(K, 1) * (4 / (int)sizeof(T));
   if (a0.filt_mc == nullptr || a0.c1 % CC != 0 || a0.c2 % CC != 0 || a0.cout % 32 != 0) return false;
-  constexpr bool DEEP = K == 3 && (X3 || sizeof(T) == 2);      // (takes every launch of these that could be split)
-  if (DEEP && mie_launch_tconv_deep(a0, pts, st)) return true;
+  constexpr bool DEEP = K == 3 && (X3 || sizeof(T) == 2);
+  const unsigned cap_p = (unsigned)(pts.n * pts.tiles_y * pts.tiles_x);
+  const int cout = a0.cout;
+  // The one-launch form takes every launch of its types that could be split, but for fp32 of so many channels that the split contraction
+  // makes up for its second launch.  One launch over split, 2 to 64 slabs: 1280 channels .89 to 1.05, 1408 .88 to 1.11, 1536 .92 to 1.17,
+  // 2048 1.04 to 1.31; 128 slabs of four tiles or fewer, 1536 .97 to 1.18, 2048 1.05 to 1.26, of more .75 to .97 (bf16 of 2048: .5 to 1.0).
+  const bool split = !DEEP || (X3 && a0.g_cpd == nullptr && a0.c1 + a0.c2 > 1408 && (long long)cap_p * (cout / 16) <= (cap_p <= 4 ? 128 : 64));
   ConvArgsT<T> a = a0;
   a.xcd_fs = 0; a.xcd_m = 0;
-  const unsigned cap_p = (unsigned)(pts.n * pts.tiles_y * pts.tiles_x);
-  const int cout = a.cout;
-  if constexpr (!DEEP) {
+  if constexpr (!DEEP || X3) {
     const unsigned cap_out = (unsigned)(a.ts.n * a.ts.tiles_y * a.ts.tiles_x);
     const long long groups = (long long)cap_p * (cout / 32);
     const int nch = (a.c1 + a.c2) / CC;
-    if (a.ws != nullptr && !a.refresh && groups <= 128 && nch >= 4) {
+    if (split && a.ws != nullptr && !a.refresh && groups <= 128 && nch >= 4) {
       a.ws_plane = (long long)a.ts.n * a.ts.h * a.ts.w * cout;
       int parts = 1;
       while (2 * parts <= 8 && 2 * parts <= nch && groups * (2 * parts) <= 256 && (long long)(2 * parts) * a.ws_plane <= a.ws_floats)
@@ -411,6 +414,7 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
       }
     }
   }
+  if (DEEP && mie_launch_tconv_deep(a0, pts, st)) return true;
   a.ws = nullptr;
   // (the 128-column kernel holds 4 phases x 2 blocks of accumulators and a four-column operand ring: in the three-term
   // form it would spill, so that form stops at 64 columns)

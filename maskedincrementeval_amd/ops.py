@@ -1117,8 +1117,9 @@ def tconv2x_masked(x, xmask, x2, x2mask, filt, k, out_ts: TileMask, block_ts: Ti
             pix_ptr(x2mask, n, h, w, "x2mask"), c2, h, w, plain.data_ptr(), mc_ptr, cin_total, cout, out_ts.ref,
             block_ts.ref, nhwc_ptr(out_delta, "out_delta", dtype=dt), nhwc_ptr(reservoir, "reservoir"), act, float(slope), code, _stream(x)))
         return out_delta
-    # (3x3 on bf16 deltas and in the three-term form: one launch on planes of few blocks)
-    ws_ptr, ws_bytes = _workspace_args(workspace, block_ts.capacity * (cout // 32) <= 128 and (k != 3 or code == _lib.DTYPE_F32), x.device)
+    # (3x3 on bf16 deltas and in the three-term form, but for very many channels there: one launch on planes of few blocks)
+    split = k != 3 or code == _lib.DTYPE_F32 or (code == _lib.DTYPE_F32_BF16X3 and c1 + c2 > 1408)
+    ws_ptr, ws_bytes = _workspace_args(workspace, block_ts.capacity * (cout // 32) <= 128 and split, x.device)
     check(lib().mie_tconv2x_masked(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1, nhwc_ptr(x2, "x2", dtype=dt),
         pix_ptr(x2mask, n, h, w, "x2mask"), c2, h, w, plain.data_ptr(), mc_ptr, cin_total, k, cout, out_ts.ref,

@@ -63,6 +63,29 @@ def test_transposed_conv_in_one_launch(n, c1, c2, cout, h, w, dtype):
     assert ((res.cpu().double() - want).abs() <= 4e-7 * bound + 2.0 ** -23 * want.abs()).all()
 
 
+# fp32 of very many channels: split where there is a workspace that holds two parts, else one launch
+def test_transposed_conv_of_very_many_channels():
+    n, c1, c2, cout, h, w = 1, 768, 704, 32, 5, 9
+    wt = torch.randn(c1 + c2, cout, 3, 3, generator=torch.Generator().manual_seed(2)) * (2.0 / (9 * (c1 + c2))) ** 0.5
+    filt = ops.ConvFilter(wt.permute(0, 2, 3, 1).contiguous().to(DEV))
+    ts, blocks = TileMask(n, 2 * h, 2 * w, DEV), TileMask(n, h, w, DEV)
+    d, m = gaussian_delta(n, c1 + c2, h, w, 0.4, 0.5, seed=3)
+    dm = m.to(DEV)
+    up = lambda x, f: F.conv_transpose2d(x.double(), f.double(), stride=2, padding=1, output_padding=1)
+    want, bound = up(d, wt), up(d.abs(), wt.abs())
+    got = {}
+    for name, ws in (("shared", None), ("own", torch.full((ops.SPLIT_WORKSPACE_BYTES // 4,), float("nan"), device=DEV)),
+                     ("too small", torch.full((4 * h * w * cout,), float("nan"), device=DEV)), ("none", False)):
+        ops.build_mask_tiles(dm, None, n, h, w, _lib.FOOT_TCONV, 3, 2, 1, ts)
+        ops.build_mask_tiles(ts, None, n, 2 * h, 2 * w, _lib.FOOT_CONV, 2, 2, 0, blocks)
+        out, res = ops.new_nhwc(n, cout, 2 * h, 2 * w, DEV), ops.new_nhwc(n, cout, 2 * h, 2 * w, DEV)
+        ops.tconv2x_masked(_dev(d[:, :c1]), dm, _dev(d[:, c1:]), dm, filt, 3, ts, blocks, out, res, workspace=ws)
+        assert ((res.cpu().double() - want).abs() <= 4e-7 * bound).all(), name
+        assert ws is None or ws is False or torch.isfinite(ws).any() == (name == "own")
+        got[name] = res
+    assert torch.equal(got["shared"], got["own"]) and torch.equal(got["too small"], got["none"])
+
+
 # two more input channels in front (a part whose mask the wide parts' covers): every phase, planes cut off at both edges, two and four rows
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,c1,c2,cout,h,w", [(1, 128, 0, 32, 1, 1), (2, 64, 64, 32, 5, 9), (1, 128, 128, 128, 31, 32), (1, 64, 64, 64, 63, 64),
