@@ -26,11 +26,13 @@ def _close(got, ref, what="", rtol=1e-4, atol=1e-5):
     assert torch.allclose(got, ref, rtol=rtol, atol=atol), "%s max|diff| = %.3e" % (what, err)
 
 
-@pytest.mark.parametrize("fuse,stacked", [(True, True), (True, False), (False, False)])
-@pytest.mark.parametrize("c", [32, 12])
-def test_convgru_module_matches_oracle(fuse, stacked, c):
-    # stacked: both gate convs as one conv of 2*hid channels + mie_convgru_gates_incr; c = 12 keeps the conv
-    # off the matrix-core path and the gate kernel on 4-channel vectors
+@pytest.mark.parametrize("fuse,stacked,one_launch", [(True, True, "never"), (True, True, "always"), (True, True, "in turn"), (True, False, "never"),
+                                                     (False, False, "never")])
+@pytest.mark.parametrize("c", [64, 32, 12])
+def test_convgru_module_matches_oracle(fuse, stacked, one_launch, c):
+    # stacked: both gate convs as one conv of 2*hid channels + mie_convgru_gates_incr, or (one_launch) mie_conv_gru_masked, on the
+    # kernel for planes of few tiles (c = 64) and the general one (32); c = 12 keeps the conv off the matrix-core path and the gate kernel
+    # on 4-channel vectors
     n, h, w = 1, 20, 28
     cell = seed_module_(ConvGRUIncr(c, c, 3, fuse=fuse, stacked=stacked), 41).to(DEV).eval()
     params = {"g." + k: v for k, v in cell.state_dict().items()}
@@ -41,6 +43,7 @@ def test_convgru_module_matches_oracle(fuse, stacked, c):
     _close(hd, ref.refresh(x, None), "refresh")
     for step in range(4):
         d, m = gaussian_delta(n, c, h, w, 0.08, 0.3, seed=4300 + step)
+        cell.one_launch = one_launch == "always" or (one_launch == "in turn" and step % 2 == 0)
         with torch.no_grad():
             dh, _ = cell([_cl(d), m.to(DEV)], None)
         torch.cuda.synchronize()
@@ -48,7 +51,7 @@ def test_convgru_module_matches_oracle(fuse, stacked, c):
         # clean-delta invariant: nothing outside the 3x3 footprint of the input mask
         foot = torch.from_numpy(mo.footprint_conv(m[:, 0].numpy(), 3, 1, 1)).bool().unsqueeze(1)
         assert torch.count_nonzero(dh[0].cpu() * (~foot)) == 0
-    assert ("gru_gates" in str(list(cell._ib().keys()))) == (fuse and stacked)
+    assert ("gru_gates" in str(list(cell._ib().keys()))) == (fuse and stacked and (c == 12 or one_launch != "always"))
 
 
 def _run(decoder, h, w, steps, edges, fuse=True):
