@@ -79,9 +79,9 @@ extern "C" {
  * that matter are accumulated in fp32 -- what is dropped is at most 2^-23 of |x*w| per product and 2^-26
  * typically (an fp32 multiply-add rounds at 2^-24); measured against fp64, whole convs come out at 0.6 to 1.1
  * times the error of the fp32 matrix-core instruction.  Taken by mie_pack_filter and by the `dtype` of
- * mie_conv_masked / _ws / _noalloc, mie_conv_refresh, mie_upconv_masked, mie_conv_gates_masked (shapes:
- * mie_conv_f32x3_takes) and mie_tconv2x_masked / mie_tconv2x_refresh (c1, c2 multiples of 64), with filter_mc
- * packed for it; every buffer is what it is for MIE_DTYPE_F32.  Values must be finite and below the bf16
+ * mie_conv_masked / _ws / _noalloc, mie_conv_refresh, mie_upconv_masked, mie_conv_gates_masked, mie_conv_gru_masked (shapes:
+ * mie_conv_f32x3_takes), mie_upconv2x_masked / mie_upconv2x_refresh and mie_tconv2x_masked / mie_tconv2x_lead_masked /
+ * mie_tconv2x_refresh (c1, c2 multiples of 64), with filter_mc packed for it; every buffer is what it is for MIE_DTYPE_F32.  Values must be finite and below the bf16
  * maximum (3.39e38): an infinity, or a value that rounds to one in bf16, splits into inf - inf and gives
  * NaN where the fp32 instruction would give an infinity -- except in convs at stride 2 on few tiles, with a
  * workspace (mie_conv_masked_ws: tiles x cout/32 <= 128) or in the form that needs none (mie_conv_needs_no_workspace), which

@@ -34,6 +34,9 @@
 //   3x3 s2 256->512   16x16 16.1 -> 12.0                                       10.7 -> 6.1
 //   up 128->64, 64->32  32x48 13.5 -> 11.4, 64x64 15.9 -> 7.8                   11.9 -> 6.8, 8.5 -> 5.4
 // Whole passes: fp32 1x64x96 163.1 -> 147 us, 1x128x128 231 -> 215.
+// With more input channels than these the split form is the faster one (mie_conv_deep_faster).  Counters (256->256 at 8x12, fp32): matrix
+// cores busy 12 % of a CU's time, 250 KB a workgroup through its path to the L2s (1.6 of 7.7 us), 47 % of the LDS cycles bank conflicts.
+// The fp32 gates forms of eight rows are at 256 registers and keep 20 (ConvLSTM) and 12 (ConvGRU) bytes a lane in scratch memory.
 #include "mie_conv_mfma_impl.h"
 
 namespace {

@@ -95,7 +95,10 @@ class ConvLSTMIncr(replay.Watched, nn.Module, _IncrBuffers):
     sigmoid1..3 / tanh1 / m1 / m2 / tanh2 / m3 module by module.
     """
 
-    one_launch = False       # ops.conv_gates_incr; on in a network's layers, a cell by itself leaves its parts in the workspace
+    # ops.conv_gates_incr in one launch on planes of few tiles, the faster form (256 channels at 8x12: 13.2 -> 9.7 us).  A network's layers
+    # have it on.  Off in a cell by itself only because its split form, sums left in the workspace, is what such cells were given
+    # out with; set it to have the faster one.
+    one_launch = False
 
     def __init__(self, input_size: int, hidden_size: int, kernel_size: int,
                  prev_c_res: IncrementReserve = None, fused: bool = True):

@@ -75,7 +75,10 @@ class nnCatIncr(replay.Watched, nn.Module, _IncrBuffers):
 class ConvGRUIncr(replay.Watched, nn.Module, _IncrBuffers):
     """Incremental ConvGRU (reference :18-96)."""
 
-    one_launch = False       # the stacked form in one kernel; on in a network's layers, a cell by itself keeps the gates' delta
+    # The stacked form in one kernel, the faster one (four such cells of optical flow at 256x256: 344 -> 326 us a pass).  A network's layers
+    # have it on.  Off in a cell by itself only because such cells were given out with the gates' delta in a buffer of its own; set it
+    # to have the faster one.
+    one_launch = False
 
     def __init__(self, input_size, hidden_size, kernel_size, activation=None, fuse=True, stacked=True):
         super().__init__()

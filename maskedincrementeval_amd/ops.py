@@ -636,8 +636,9 @@ def pack_filter(filt: torch.Tensor, dtype=torch.float32, x3: bool = False) -> to
 # per multiply on the bf16 matrix-core instruction (fp32 accuracy: the three dropped products are at most 2^-23 of
 # |x * w|, typically 2^-26, and the measured error against fp64 is 0.6-1.1 times the fp32 instruction's; about twice
 # its rate), where the library has that form (mie_conv_f32x3_takes: 3x3 / 5x5 at stride 1 with channel counts in
-# multiples of 32, 5x5 at stride 2 in multiples of 16; the stride-2 transposed conv in multiples of 64);
-# "native" = v_mfma_f32_32x32x2_f32 everywhere.  Environment variable MIE_F32_MATMUL.
+# multiples of 32, 5x5 at stride 2 in multiples of 16; the stride-2 transposed conv in multiples of 64), and on planes of few tiles
+# 3x3 at stride 2 (mie_conv_needs_no_workspace: 64..512 channels there, error against fp64 0.35-0.73 times the fp32
+# instruction's); "native" = v_mfma_f32_32x32x2_f32 everywhere.  Environment variable MIE_F32_MATMUL.
 f32_matmul = os.environ.get("MIE_F32_MATMUL", "bf16x3")
 
 
@@ -1409,8 +1410,8 @@ def conv_gates_incr(x, xmask, x2, x2mask, filt: ConvFilter, out_ts: TileMask, ga
                     cprev_res, cell_res, h_delta, c_delta, workspace=None, one_launch=False):
     """3x3 gates conv of a ConvLSTM with the gate chain as its epilogue; `filt` and `gates_res` are in the
     gate-interleaved column order (gate_interleave_index).  workspace: as in conv_masked.  one_launch: planes that would be
-    split run in the form that needs no workspace where the library has one (256 channels at 8x12 fp32 13.2 -> 9.7 us, bf16
-    10.0 -> 5.0)."""
+    split run in the form that needs no workspace where that is the faster one (mie_conv_gates_needs_no_workspace; 256 channels
+    at 8x12 fp32 13.2 -> 9.7 us, bf16 10.0 -> 5.0)."""
     n, c1, h, w = x.shape
     c2 = 0 if x2 is None else x2.shape[1]
     dt = x.dtype
