@@ -491,6 +491,15 @@ class TransposedConvLayerIncr(replay.Watched, nn.Module):
                 and ops.tconv2x_takes(shapes[-2], shapes[-1], tc.out_channels, k, s, p, op,
                                       filt.rows(lead_c, filt.shape[0]), dtype))
 
+    def _lead_planned(self, along):
+        """Whether the leading part has a tile set of its own in the plan of this pass (as a launch of its own it needs one, in the wide
+        conv's epilogue not).  ops.f32_matmul may change between a plan and its step, and the form with it: a set that was planned is
+        used, so that it does not forget which tiles hold data, and one that was not is built by the step."""
+        sets, parity = self.__dict__.setdefault("_lead_sets", {}), ops._pass.buffer_parity
+        if ops._pass.phase == "plan":
+            sets[parity] = not along
+        return sets.get(parity, not along) if ops._pass.phase == "compute" else not along
+
     def forward(self, parts):
         tc = self.transposed_conv2d
         chans = [p_[0].shape[1] for p_ in parts]
@@ -503,11 +512,13 @@ class TransposedConvLayerIncr(replay.Watched, nn.Module):
                 # the flow estimate of the previous scale shares the mask of x (a 1x1 conv + tanh of it), so the
                 # wide conv's output mask covers this partial result
                 lead_c = chans[0]
-                if ops.tconv2x_takes_lead(lead_c, chans[1], chans[2], tc.out_channels, tc._geometry()[0], ops.delta_torch_dtype(parts[0][0])):
+                along = ops.tconv2x_takes_lead(lead_c, chans[1], chans[2], tc.out_channels, tc._geometry()[0], ops.delta_torch_dtype(parts[0][0]))
+                planned = self._lead_planned(along)
+                if along and not planned:
                     kind, slope = activation_kind(self.activation.op)
                     return tc.forward(parts[1], self.activation.in_res.reservoir, kind, slope, x2_incr=parts[2],
                                       filt=filt.rows(lead_c, filt.shape[0]), lead_incr=parts[0], lead_filt=filt.rows(0, lead_c))
-                addend = tc.forward(parts[0], filt=filt.rows(0, lead_c), out_name="lead")
+                addend = tc.forward(parts[0], filt=filt.rows(0, lead_c), out_name="lead", planned=planned)
             kind, slope = activation_kind(self.activation.op)
             return tc.forward(parts[-2], self.activation.in_res.reservoir, kind, slope, x2_incr=parts[-1],
                               addend_incr=addend, filt=filt.rows(lead_c, filt.shape[0]))

@@ -643,9 +643,11 @@ class nnConvTranspose2dIncr(replay.Watched, nn.ConvTranspose2d, _IncrBuffers):
         return k, s, p, op
 
     def forward(self, x_incr: Masked, reservoir=None, act=_lib.ACT_NONE, slope=0.0, x2_incr: Masked = None,
-                addend_incr: Masked = None, filt=None, out_name="out", lead_incr: Masked = None, lead_filt=None) -> Masked:
+                addend_incr: Masked = None, filt=None, out_name="out", lead_incr: Masked = None, lead_filt=None,
+                planned=True) -> Masked:
         """x2_incr: second input (the conv runs over the channel concat of the two without forming it);
         lead_incr, lead_filt: a part of two channels in front of them and its rows, where ops.tconv2x_takes_lead;
+        planned: whether the plan of the pass, if it has one, has the tile set;
         addend_incr: delta added before the epilogue, covered by the output mask; filt: a row slice of
         self._filter() when only part of the input channels is fed.  Two inputs and the addend need the
         matrix-core form."""
@@ -663,7 +665,8 @@ class nnConvTranspose2dIncr(replay.Watched, nn.ConvTranspose2d, _IncrBuffers):
             m1 = m2 = None
         else:
             m1, m2 = pix, pix2
-        ops.build_mask_tiles(m1, m2, n, h, w, _lib.FOOT_TCONV, k, s, p, ts)
+        build = ops.build_mask_tiles if planned or ops._pass.phase != "compute" else ops.build_unplanned_tiles
+        build(m1, m2, n, h, w, _lib.FOOT_TCONV, k, s, p, ts)
         filt = self._filter() if filt is None else filt
         if ops.tconv2x_takes(c1, c2, self.out_channels, k, s, p, op, filt, ops.delta_torch_dtype(x)):
             blocks = self._tile_set(out_name + "_blocks", n, h, w, x.device)

@@ -612,6 +612,15 @@ def build_mask_tiles(in_mask, in_mask2, n, h_in, w_in, foot, k, stride, pad, out
     return out
 
 
+def build_unplanned_tiles(*args):
+    """build_mask_tiles of a set that the plan of this pass did not have, where its compute pass needs it."""
+    phase, _pass.phase = _pass.phase, None
+    try:
+        return build_mask_tiles(*args)
+    finally:
+        _pass.phase = phase
+
+
 def pack_filter(filt: torch.Tensor, dtype=torch.float32, x3: bool = False) -> torch.Tensor:
     """Matrix-core copy of a contiguous fp32 [Cin,K,K,Cout] filter in `dtype`, shape
     [Cin/B, K*K, 2, Cout, B/2] with B = 8 (fp32) or 16 (bf16) input channels per block:

@@ -216,3 +216,26 @@ def test_concat_layers_refuse_the_planning_stream():
         with pytest.raises(NotImplementedError, match="asynchronous mask planning"):
             m([_cl(gaussian_delta(1, 4, h, w, 0.05, 0.3, seed=2)[0]), None])
     assert ops._planner is None and ops._phase is None
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("decoder", ["transposed", "upsample"])
+def test_a_step_planned_under_one_setting_runs_under_another(decoder, dtype, monkeypatch):
+    # ops.f32_matmul is chosen per call, also between a plan and its step: which tile sets the step needs follows it.  (Deltas are
+    # differences of values of order one: sums in another order, all that a plan of the other setting changes, show as some 1e-7)
+    h, w = 64, 96
+    a, b = (seed_module_(MultiResUNetRecurrentIncr(num_bins=4, decoder=decoder), seed=3).to(DEV).eval() for _ in range(2))
+    gen = MovingEdges(h, w, seed=5)
+    x3, native = "bf16x3", "native"
+    with torch.no_grad():
+        x0 = _cl(torch.randn(1, 4, h, w, generator=torch.Generator().manual_seed(1))).to(dtype)
+        a.forward_refresh_reservoirs(x0), b.forward_refresh_reservoirs(x0)
+        for i, (planned, run) in enumerate([(x3, x3), (x3, native), (native, native), (native, x3), (native, native), (native, x3), (x3, native), (x3, x3)]):
+            d = _cl(gen.step()[0]).to(dtype)
+            monkeypatch.setattr(ops, "f32_matmul", planned)
+            a.plan_ahead([d, None], i % 2)
+            monkeypatch.setattr(ops, "f32_matmul", run)
+            got, want = a.forward_planned([d, None], i % 2), b([d, None])
+            torch.cuda.synchronize()
+            for (g, _), (v, _) in zip(got, want):
+                assert (g - v).abs().max() <= (2e-6 if dtype == torch.float32 else 0), i
