@@ -889,7 +889,8 @@ def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt, refresh=Fa
     persistent kernel), and where border strips and blocks filled in part undo the fewer taps: 16 for each of the four
     phases of an item against 25 for each tile, once that is more than a round of workgroups (256->128 at 8x19x23: 138
     us against 123).  Nor, but for a refresh, where upconv_masked has its form for planes of few tiles (fp32 128->64 at 32x48 15.0 us
-    against 11.4, 64->32 at 64x64 10.3 against 7.8; bf16 9.8 against 6.8 and 7.4 against 5.4)."""
+    against 11.4, 64->32 at 64x64 10.3 against 7.8; bf16 9.8 against 6.8 and 7.4 against 5.4), in bf16 on all such planes, also where the
+    split form is the faster there (40 layers of 448 to 1536 channels: .97 to 1.7 times as long, 768->128 at 11x30 49.5 us against 29.5)."""
     n, c, h, w = a.shape
     chunk = mfma_chunk(a.dtype)
     if not (upconv2x_enabled and isinstance(filt, ConvFilter) and filt.plain.is_cuda and k == 5 and stride == 1 and pad == 2
@@ -898,8 +899,8 @@ def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt, refresh=Fa
             and n * c * h * w * a.element_size() < 0xffffff00):
         return False
     tiles, slabs = _lib.tile_capacity(n, 2 * h, 2 * w), cout // 32
-    code = _lib.DTYPE_BF16 if a.dtype == torch.bfloat16 else _lib.DTYPE_F32_BF16X3
-    if not refresh and lib().mie_upconv_needs_no_workspace(c, cout, tiles, code):
+    if not refresh and (tiles * (cout // 16) <= 256 if a.dtype == torch.bfloat16 else
+                        lib().mie_upconv_needs_no_workspace(c, cout, tiles, _lib.DTYPE_F32_BF16X3)):
         return False
     items = n * (-(-(h - 2) // 8) * -(-(w - 2) // 8) + 2 * -(-w // 32) + 2 * -(-(h - 2) // 32))
     if (c >= 4 * chunk and tiles * slabs <= 64) or (4 * items * slabs > 256 and 4 * 16 * items > 25 * tiles):

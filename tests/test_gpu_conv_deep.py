@@ -230,6 +230,7 @@ def test_layers_of_many_channels_are_split(kind, dtype, c1, c2):
             ops.build_mask_tiles(up, None, n, ho, wo, _lib.FOOT_CONV, 5, 1, 2, ts)
             ops.upconv_masked(x, dm, None, None, filt, 5, 2, ts, out, res, _lib.ACT_RELU, 0.0, workspace=ws)
             got.append((out, res))
+            assert not ops.upconv2x_takes(x, cout, 5, 1, 2, filt)
         elif kind == "gates":
             ops.build_mask_tiles(dm, None, n, h, w, _lib.FOOT_CONV, k, s, k // 2, ts)
             cells = [ops.new_nhwc(n, cout // 4, h, w, DEV) for _ in range(2)] + [ops.new_nhwc(n, cout // 4, h, w, DEV, dtype) for _ in range(2)]
