@@ -87,9 +87,9 @@ def parse_args():
                     help="skip the other benchmark configurations (single conv, activation chain, EVFlowNet-incr, batched bf16)")
     ap.add_argument("--no-lossy", dest="lossy", action="store_false", help="skip the lossy frontier")
     ap.add_argument("--no-refresh", dest="refresh", action="store_false", help="skip the dense-refresh timing")
-    ap.add_argument("--f32-matmul", choices=["bf16x3", "native"], default=None,
-                    help="how the matrix-core kernels multiply fp32 deltas (default: the library setting, bf16x3 = "
-                         "three bf16 terms per value on the bf16 instruction, fp32 accuracy)")
+    ap.add_argument("--f32-matmul", choices=["f16x2", "bf16x3", "native"], default=None,
+                    help="how the matrix-core kernels multiply fp32 deltas (default: the library setting, f16x2 = "
+                         "two fp16 terms per value on the fp16 instruction; bf16x3 = three bf16 terms; both fp32 accuracy)")
     ap.add_argument("--no-native", dest="native", action="store_false",
                     help="skip the comparison run with the fp32 matrix-core instruction")
     ap.add_argument("--detail-file", default=os.path.join(ROOT, "gpurun_out", "bench_detail.json"),
@@ -563,13 +563,15 @@ class NetBench:
         mfma_bound = dom["flops"] / max(dom["bytes"], 1) > self.peak_mfma * 1e12 / (PEAK_HBM_GBS * 1e9)
         x3 = self.wl.dtype == "f32" and self._takes_x3(dom)
         if mfma_bound and x3:
-            # fp32 deltas multiplied as three bf16 terms: six bf16 matrix-core products per algorithmic multiply, so
-            # the bound is the bf16 peak over six; the fraction of the fp32 instruction's peak is given beside it
-            peak = round(PEAK_BF16_MFMA_TFLOPS / 6.0, 1)
+            # fp32 deltas multiplied in terms: three fp16 (two terms a value) or six bf16 (three) matrix-core products per
+            # algorithmic multiply, so the bound is the peak of these instructions over three or six; the fraction of the fp32
+            # instruction's peak is given beside it
+            products = self._products(dom)
+            peak = round(PEAK_BF16_MFMA_TFLOPS / products, 1)
             roofline = dict(bound="mfma", achieved=dom["tflops"], peak=peak, unit="TFLOP/s",
                             frac=round(dom["tflops"] / peak, 4), traffic=None,
-                            peak_basis="bf16 matrix-core peak %.0f TFLOP/s / 6 term products per fp32 multiply" % PEAK_BF16_MFMA_TFLOPS,
-                            executed_bf16_tflops=round(6 * dom["tflops"], 1),
+                            peak_basis="16-bit matrix-core peak %.0f TFLOP/s / %d term products per fp32 multiply" % (PEAK_BF16_MFMA_TFLOPS, products),
+                            executed_bf16_tflops=round(products * dom["tflops"], 1),
                             frac_of_fp32_mfma_peak=round(dom["tflops"] / PEAK_FP32_MFMA_TFLOPS, 4))
         elif mfma_bound:
             roofline = dict(bound="mfma", achieved=dom["tflops"], peak=self.peak_mfma, unit="TFLOP/s",
@@ -587,13 +589,17 @@ class NetBench:
         # shape (FETCH_SIZE + WRITE_SIZE, scaled by the copy-kernel calibration)
         try:
             with open(os.path.join(ROOT, "profiles", "pmc_traffic.json")) as f:
-                roofline["traffic"] = json.load(f).get(dom["shape"] + (" bf16x3" if x3 else ""), {}).get("hbm_bytes_per_launch")
+                roofline["traffic"] = json.load(f).get(dom["shape"] + (" " + self.ops.f32_matmul if x3 else ""), {}).get("hbm_bytes_per_launch")
         except OSError:
             pass
         return roofline
 
+    def _products(self, layer):
+        """Term products per multiply of a launch that ran in terms (decoders at the resolution of their inputs: six)."""
+        return 6 if self.ops.f32_matmul == "bf16x3" or layer["op"].startswith("upconv2x") else 3
+
     def _takes_x3(self, layer):
-        """Whether the launch of a per-launch table row ran in the three-term bf16 form (its shape string is
+        """Whether the launch of a per-launch table row ran in terms (its shape string is
         "KxK sS CIN->COUT..." with the input channels of the first operand)."""
         import re
         m = re.search(r"(\d)x\d s(\d) (\d+)->(\d+)", layer["shape"])
@@ -811,14 +817,14 @@ def main():
 
     # ---- the same network with the fp32 matrix-core instruction (v_mfma_f32_32x32x2_f32) ------------------
     native = None
-    if args.native and args.dtype == "f32" and ops.f32_matmul == "bf16x3":
-        ops.f32_matmul = "native"
+    if args.native and args.dtype == "f32" and ops.f32_matmul != "native":
+        in_terms, ops.f32_matmul = ops.f32_matmul, "native"
         try:
             nat_model = nb.new_model(async_masks=not args.sync_masks, plan_first=args.plan_first)
             nat_sec, _, _ = nb.timed_run(nat_model, "incremental, fp32 matrix-core instruction", repeats=max(3, args.repeats // 2))
             del nat_model
         finally:
-            ops.f32_matmul = "bf16x3"
+            ops.f32_matmul = in_terms
         native = dict(ms_per_step=round(1e3 * nat_sec, 4), frames_per_s=round(NB / nat_sec, 1))
 
     # ---- dense comparator: same kernels, every tile active ---------------------------------------
@@ -916,10 +922,10 @@ def main():
                           "delta, as the reference executes it), torch-CPU fp32" % (args.cpu_steps, NET_NAME, H, W))
         log("cpu baseline: %.1f ms/frame on %d threads" % (1e3 * cdt, cpu["cores"]))
 
-    x3 = args.dtype == "f32" and ops.f32_matmul == "bf16x3"
+    products = {"f16x2": 3.0, "bf16x3": 6.0}.get(ops.f32_matmul) if args.dtype == "f32" else None
     # one basis for every matrix-core fraction of the line: the peak of the instruction that runs (for fp32 deltas
-    # in the three-term form the bf16 peak over the six term products of a multiply)
-    mfma_peak = PEAK_BF16_MFMA_TFLOPS / 6.0 if x3 else nb.peak_mfma
+    # in terms the 16-bit peak over the three or six term products of a multiply)
+    mfma_peak = PEAK_BF16_MFMA_TFLOPS / products if products else nb.peak_mfma
     detail = {
         "metric": "incremental frames/s + HBM GB/s, %s %dx%d @%g%% delta density" % (NET_NAME, H, W, 100 * dens),
         "value": round(NB / sec_per_step, 2),
@@ -981,6 +987,8 @@ def main():
 
 
 ARITHMETIC = {
+    "f16x2": "fp32 deltas, reservoirs, accumulators; matrix-core products as two fp16 terms per value "
+             "(three term products per multiply; fp32-class error: tests/test_gpu_f16x2.py; some layers three bf16 terms)",
     "bf16x3": "fp32 deltas, reservoirs, accumulators; matrix-core products as three bf16 terms per value "
               "(six term products per multiply, fp32-class error: tests/test_gpu_f32x3.py)",
     "native": "fp32 deltas, reservoirs, accumulators and matrix-core instruction",

@@ -87,6 +87,17 @@ extern "C" {
  * workspace (mie_conv_masked_ws: tiles x cout/32 <= 128) or in the form that needs none (mie_conv_needs_no_workspace), which
  * compute the outputs concerned again in fp32 and give what the fp32 instruction gives. */
 #define MIE_DTYPE_F32_BF16X3 2
+/* The same with two fp16 terms and three term products: value * scale = hi + lo, the scale a power of two that a
+ * workgroup takes from its own input (and mie_pack_filter from the weights), 23 bits of every value.  Half the matrix
+ * instructions of MIE_DTYPE_F32_BF16X3, and less error against fp64 (fewer roundings at the size of the sum).  Where a
+ * workgroup's input does not lie within fp16's range of its scale -- groups of eight channels of a pixel 2^23 below the largest value
+ * or 2^6 above it, infinities, NaN -- it contracts in fp32 instead, as for MIE_DTYPE_F32, from a copy of the filter
+ * that the packed one holds too: correct, and slower.  Forms that add up the products of three terms more finely than that -- those
+ * without a workspace on planes of few tiles, the transposed convs -- keep the three (the packed copy holds them as well).
+ * Taken, for the same shapes, wherever MIE_DTYPE_F32_BF16X3 is. */
+#define MIE_DTYPE_F32_F16X2 3
+/* bytes behind the weights of a filter copy packed for it (scale, whether all weights fit it, workspace of the packing) */
+#define MIE_F16X2_END_BYTES 8240
 
 /* frame kinds of mie_events_to_frame */
 #define MIE_EVENTS_VOXEL 0      /* num_bins channels, linear weights in time   */
@@ -223,8 +234,11 @@ int mie_build_mask_plan_wgs(const mie_plan_op* ops, int n_ops, int max_workgroup
  *   MIE_DTYPE_BF16 (cin % 16 == 0): P[ci/16][tap][(ci%16)/8][co][ci%8], bf16
  *   MIE_DTYPE_F32_BF16X3 (cin % 16 == 0): P[ci/16][tap][term][(ci%16)/8][co][ci%8], bf16,
  *        term 0 / 1 / 2 = the weight rounded to bf16, the rest of it rounded to bf16, what is left
+ *   MIE_DTYPE_F32_F16X2 (cin % 16 == 0): the copy for MIE_DTYPE_F32_BF16X3, then P[ci/16][tap][term][(ci%16)/8][co][ci%8], fp16,
+ *        term 0 / 1 = weight * scale rounded to fp16, 2048 times the rest, then Q[ci/16][tap][(ci%8)/4][(ci%16)/8][co][ci%4], fp32, and
+ *        MIE_F16X2_END_BYTES: two floats, 1 / scale and whether the weights fit it (0: they do not), then the call's own
  * `packed` holds cin*k*k*cout elements of that type (three times that many bf16 for
- * MIE_DTYPE_F32_BF16X3); do this once per weight update.
+ * MIE_DTYPE_F32_BF16X3; 14 bytes a weight and the end for MIE_DTYPE_F32_F16X2); do this once per weight update.
  * Replaces: convert_filter_out_channels_last
  * (ext/pointops/pointops_functional.py:13-14), which plays the same role for
  * the reference kernel.

@@ -23,7 +23,8 @@ NOALLOC_WS_BYTES = 8 * 1024 * 1024
 ACT_NONE, ACT_RELU, ACT_LEAKY_RELU, ACT_SIGMOID, ACT_TANH = 0, 1, 2, 3, 4
 FOOT_CONV, FOOT_UP2X, FOOT_TCONV = 0, 1, 2
 EVENTS_VOXEL, EVENTS_HISTOGRAM = 0, 1
-DTYPE_F32, DTYPE_BF16, DTYPE_F32_BF16X3 = 0, 1, 2
+DTYPE_F32, DTYPE_BF16, DTYPE_F32_BF16X3, DTYPE_F32_F16X2 = 0, 1, 2, 3
+F16X2_END_BYTES = 8240
 PATH_AUTO, PATH_VALU, PATH_MFMA = 0, 1, 2
 FLAG_KEEP_RESERVOIR = 1
 CNT_ACTIVE, CNT_STALE, CNT_TICKET, CNT_WORDS = 0, 1, 2, 4

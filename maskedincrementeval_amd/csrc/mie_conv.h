@@ -26,8 +26,8 @@ struct ConvArgsT {
   float* ws; long long ws_floats; long long ws_plane;
   // Matrix-core path: launch order permuted per XCD (number of slab groups, 0 = plain order); set by the launchers.
   int xcd_fs; unsigned xcd_m;      // (xcd_m: mie_tile_div by the slabs of a group)
-  // Matrix-core path, fp32 deltas: filt_mc is the three-term bf16 copy and the contraction runs as six bf16 products
-  // per term pair (MIE_DTYPE_F32_BF16X3).
+  // Matrix-core path, fp32 deltas: 1: filt_mc is the three-term bf16 copy and the contraction runs as six bf16 products
+  // per term pair (MIE_DTYPE_F32_BF16X3); 2: the two-term fp16 copy, three products (MIE_DTYPE_F32_F16X2).
   int x3;
   TileSetDev ts;
 };

@@ -14,6 +14,7 @@
 // increment, or (dense refresh) bias + activation + reservoir fill.
 #include "mie_common.h"
 #include "mie_conv.h"
+#include "mie_pack_terms.h"
 #include <mutex>
 
 namespace {
@@ -429,7 +430,7 @@ int conv_impl(const char* who, const T* x, const uint8_t* xmask, int c1, const T
               T* out_delta, const T* addend, float* reservoir, int act_kind, float slope,
               int path, bool refresh, const float* bias, void* stream,
               const GatesOperands<T>* gates = nullptr, void* workspace = nullptr,
-              long long workspace_bytes = 0, bool x3 = false) {
+              long long workspace_bytes = 0, int x3 = 0) {
   mie_clear_error();
   int rc = mie_check_tileset(out, who);
   if (rc != MIE_OK) return rc;
@@ -486,7 +487,7 @@ int conv_impl(const char* who, const T* x, const uint8_t* xmask, int c1, const T
                                        workspace != (const void*)x && workspace != (const void*)x2),
               MIE_ERR_INVALID_ARG, "%s: workspace must not alias an operand", who);
   MIE_REQUIRE(!x3 || (sizeof(T) == 4 && path != MIE_PATH_VALU), MIE_ERR_INVALID_ARG,
-              "%s: MIE_DTYPE_F32_BF16X3 is a mode of the matrix-core path for fp32 deltas", who);
+              "%s: MIE_DTYPE_F32_BF16X3 and MIE_DTYPE_F32_F16X2 are modes of the matrix-core path for fp32 deltas", who);
   // (3x3 stride 2: on planes of few tiles only)
   const bool x3_deep = x3 && k == 3 && stride == 2 && workspace == nullptr &&
                        mie_conv_deep_form(k, stride, c1, c2, cout, mie_tile_capacity(out->n, out->h, out->w), MIE_DTYPE_F32_BF16X3);
@@ -494,7 +495,7 @@ int conv_impl(const char* who, const T* x, const uint8_t* xmask, int c1, const T
                           : ((filter_mc != nullptr) && (cin_total % pmul == 0) &&
                              mie_conv_mfma_takes(k, stride, dtype_of<T>(), c1, c2, cout));
   MIE_REQUIRE(!x3 || mfma_ok, MIE_ERR_UNSUPPORTED,
-              "%s: MIE_DTYPE_F32_BF16X3 needs filter_mc packed in that layout, k = 3 or 5 and channel counts "
+              "%s: MIE_DTYPE_F32_BF16X3 (or MIE_DTYPE_F32_F16X2) needs filter_mc packed in that layout, k = 3 or 5 and channel counts "
               "in whole chunks (32, stride 2: 16; k=%d stride=%d c1=%d c2=%d cout=%d); see mie_conv_f32x3_takes", who, k, stride,
               c1, c2, cout);
   MIE_REQUIRE(path == MIE_PATH_AUTO || path == MIE_PATH_VALU || path == MIE_PATH_MFMA,
@@ -513,7 +514,7 @@ int conv_impl(const char* who, const T* x, const uint8_t* xmask, int c1, const T
   a.slope = slope; a.addend = addend; a.refresh = refresh ? 1 : 0; a.bias = bias;
   a.hid = 0; a.g_cpd = nullptr; a.g_cpm = nullptr; a.g_cpres = nullptr; a.g_cres = nullptr;
   a.g_dh = nullptr; a.g_dc = nullptr;
-  a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = x3 ? 1 : 0;
+  a.ws = nullptr; a.ws_floats = 0; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = x3;
   a.ts = mie_dev_tileset(out);
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
   hipStream_t st = (hipStream_t)stream;
@@ -643,11 +644,12 @@ int tconv_impl(const char* who, const T* x, const uint8_t* xmask, int cin, int h
     MIE_REQUIRE((dtype) == MIE_DTYPE_F32 || (dtype) == MIE_DTYPE_BF16, MIE_ERR_UNSUPPORTED, \
                 "%s: unknown delta dtype %d", who, (int)(dtype));                         \
   } while (0)
-// The entry points of the matrix-core conv also take MIE_DTYPE_F32_BF16X3: fp32 deltas, three-term filter copy.
+// The entry points of the matrix-core conv also take MIE_DTYPE_F32_BF16X3 and MIE_DTYPE_F32_F16X2: fp32 deltas, the filter copy in three
+// or two terms (x3 = 1, 2; 0 otherwise).
 #define MIE_CONV_DTYPE_X3_OK(dtype, who, x3)                                              \
   do {                                                                                    \
-    if ((dtype) == MIE_DTYPE_F32_BF16X3) {                                                \
-      x3 = true;                                                                          \
+    if ((dtype) == MIE_DTYPE_F32_BF16X3 || (dtype) == MIE_DTYPE_F32_F16X2) {              \
+      x3 = (dtype) == MIE_DTYPE_F32_BF16X3 ? 1 : 2;                                       \
       dtype = MIE_DTYPE_F32;                                                              \
     }                                                                                     \
     MIE_CONV_DTYPE_OK(dtype, who);                                                        \
@@ -672,7 +674,7 @@ extern "C" int mie_upconv_needs_no_workspace(int c, int cout, int tiles, int dty
 extern "C" int mie_pack_filter(const float* filter, int cin, int k, int cout, void* packed,
                                int dtype, void* stream) {
   const char* who = "mie_pack_filter";
-  bool x3 = false;
+  int x3 = 0;
   MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
   MIE_REQUIRE(filter && packed, MIE_ERR_INVALID_ARG, "%s: NULL pointer", who);
   MIE_REQUIRE(cin > 0 && k > 0 && cout > 0, MIE_ERR_INVALID_ARG, "%s: sizes must be positive", who);
@@ -683,7 +685,9 @@ extern "C" int mie_pack_filter(const float* filter, int cin, int k, int cout, vo
   const long long total = (long long)cin * k * k * cout;
   MIE_REQUIRE(total < (1LL << 40), MIE_ERR_CAPACITY, "%s: filter too large", who);
   const dim3 grid((unsigned)((total + 255) / 256));
-  if (x3)
+  if (x3 == 2)
+    mie_pack_f16x2(filter, cin, k * k, cout, packed, (hipStream_t)stream);
+  else if (x3)
     hipLaunchKernelGGL(k_pack_filter_x3, grid, dim3(256), 0, (hipStream_t)stream, filter, (mie_bf16*)packed, cin,
                        k * k, cout);
   else if (dtype == MIE_DTYPE_BF16)
@@ -702,7 +706,7 @@ extern "C" int mie_conv_masked(const void* x, const uint8_t* xmask, int c1, cons
                                void* out_delta, const void* addend, float* reservoir,
                                int act_kind, float slope, int path, int dtype, void* stream) {
   const char* who = "mie_conv_masked";
-  bool x3 = false;
+  int x3 = 0;
   MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
   if (dtype == MIE_DTYPE_BF16) {
     typedef mie_bf16 T;
@@ -724,7 +728,7 @@ extern "C" int mie_conv_masked_ws(const void* x, const uint8_t* xmask, int c1, c
                                   int act_kind, float slope, int path, int dtype, void* workspace,
                                   long long workspace_bytes, void* stream) {
   const char* who = "mie_conv_masked_ws";
-  bool x3 = false;
+  int x3 = 0;
   MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
   if (dtype == MIE_DTYPE_BF16) {
     typedef mie_bf16 T;
@@ -779,7 +783,7 @@ extern "C" int mie_conv_masked_noalloc(const void* x, const uint8_t* xmask, int 
                                        void* out_delta, const void* addend, float* reservoir,
                                        int act_kind, float slope, int path, int dtype, void* stream) {
   const char* who = "mie_conv_masked_noalloc";
-  bool x3 = false;
+  int x3 = 0;
   MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
   int rc = mie_check_tileset(out, who);
   if (rc != MIE_OK) return rc;
@@ -815,7 +819,7 @@ extern "C" int mie_conv_refresh(const void* x, int c1, const void* x2, int c2, i
                                 void* out_dense, const void* addend, float* reservoir,
                                 int act_kind, float slope, int path, int dtype, void* stream) {
   const char* who = "mie_conv_refresh";
-  bool x3 = false;
+  int x3 = 0;
   MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
   if (dtype == MIE_DTYPE_BF16) {
     typedef mie_bf16 T;
@@ -836,7 +840,7 @@ int conv_gates_entry(const char* who, const void* x, const uint8_t* xmask, int c
                      const void* filter_mc, int cin_total, int hid, const mie_tileset* out,
                      float* gates_res, const void* cprev_delta, const uint8_t* cprev_mask,
                      float* cprev_res, float* cell_res, void* h_delta, void* c_delta, void* workspace,
-                     long long workspace_bytes, void* stream, bool x3 = false) {
+                     long long workspace_bytes, void* stream, int x3 = 0) {
   MIE_REQUIRE(hid > 0 && hid <= (1 << 20), MIE_ERR_INVALID_ARG, "%s: hid = %d out of range", who, hid);
   MIE_REQUIRE(gates_res && cprev_res && cell_res && h_delta && c_delta, MIE_ERR_INVALID_ARG,
               "%s: NULL pointer", who);
@@ -905,7 +909,7 @@ template <typename T>
 int upconv_entry(const char* who, const void* a_lo, const uint8_t* amask, const void* b_lo, const uint8_t* bmask,
                  int c, int h_lo, int w_lo, const float* filter, const void* filter_mc, int cin_total, int k,
                  int pad, int cout, const mie_tileset* out, void* out_delta, const void* addend, float* reservoir,
-                 int act_kind, float slope, void* workspace, long long workspace_bytes, void* stream, bool x3 = false) {
+                 int act_kind, float slope, void* workspace, long long workspace_bytes, void* stream, int x3 = 0) {
   int rc = mie_check_tileset(out, who);
   if (rc != MIE_OK) return rc;
   MIE_REQUIRE(a_lo && filter, MIE_ERR_INVALID_ARG, "%s: NULL pointer (a and filter are required)", who);
@@ -945,7 +949,7 @@ int upconv_entry(const char* who, const void* a_lo, const uint8_t* amask, const 
   a.hid = 0; a.g_cpd = nullptr; a.g_cpm = nullptr; a.g_cpres = nullptr; a.g_cres = nullptr;
   a.g_dh = nullptr; a.g_dc = nullptr;
   a.ws = few ? nullptr : (float*)workspace; a.ws_floats = few ? 0 : workspace_bytes / 4; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0;
-  a.x3 = (x3 && !few) ? 1 : 0;
+  a.x3 = few ? 0 : x3;
   a.ts = mie_dev_tileset(out);
   const unsigned cap = (unsigned)mie_tile_capacity(out->n, out->h, out->w);
   if (few) {
@@ -965,7 +969,7 @@ extern "C" int mie_upconv_masked_ws(const void* a, const uint8_t* amask, const v
                                     const void* addend, float* reservoir, int act_kind, float slope, int dtype,
                                     void* workspace, long long workspace_bytes, void* stream) {
   const char* who = "mie_upconv_masked";
-  bool x3 = false;
+  int x3 = 0;
   MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
   if (dtype == MIE_DTYPE_BF16)
     return upconv_entry<mie_bf16>(who, a, amask, b, bmask, c, h_in, w_in, filter, filter_mc, cin_total, k, pad, cout,
@@ -1068,7 +1072,7 @@ extern "C" int mie_conv_gates_masked_ws(const void* x, const uint8_t* xmask, int
                                         void* c_delta, int dtype, void* workspace, long long workspace_bytes,
                                         void* stream) {
   const char* who = "mie_conv_gates_masked";
-  bool x3 = false;
+  int x3 = 0;
   MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
   MIE_REQUIRE(workspace == nullptr || (workspace != (void*)gates_res && workspace != (void*)cprev_res && workspace != (void*)cell_res &&
                                        workspace != h_delta && workspace != c_delta && workspace != cprev_delta),
@@ -1097,7 +1101,7 @@ extern "C" int mie_conv_gates_masked(const void* x, const uint8_t* xmask, int c1
 namespace {
 template <typename T>
 int conv_gru_entry(const char* who, const void* x, const uint8_t* xmask, int cin, int h, int w, const float* filter, const void* filter_mc,
-                   int cin_total, int hid, const mie_tileset* out, float* update_res, float* cand_res, void* h_delta, void* stream, bool x3) {
+                   int cin_total, int hid, const mie_tileset* out, float* update_res, float* cand_res, void* h_delta, void* stream, int x3) {
   MIE_REQUIRE(hid > 0 && hid <= (1 << 20), MIE_ERR_INVALID_ARG, "%s: hid = %d out of range", who, hid);
   MIE_REQUIRE(update_res && cand_res && h_delta, MIE_ERR_INVALID_ARG, "%s: NULL pointer", who);
   MIE_REQUIRE(update_res != cand_res, MIE_ERR_INVALID_ARG, "%s: the two reservoirs must be distinct", who);
@@ -1115,10 +1119,10 @@ extern "C" int mie_conv_gru_masked(const void* x, const uint8_t* xmask, int cin,
                                    int cin_total, int hid, const mie_tileset* out, float* update_res, float* cand_res, void* h_delta,
                                    int dtype, void* stream) {
   const char* who = "mie_conv_gru_masked";
-  bool x3 = false;
+  int x3 = 0;
   MIE_CONV_DTYPE_X3_OK(dtype, who, x3);
   if (dtype == MIE_DTYPE_BF16)
-    return conv_gru_entry<mie_bf16>(who, x, xmask, cin, h_in, w_in, filter, filter_mc, cin_total, hid, out, update_res, cand_res, h_delta, stream, false);
-  MIE_REQUIRE(x3, MIE_ERR_UNSUPPORTED, "%s: fp32 deltas in the three-term form only (MIE_DTYPE_F32_BF16X3)", who);
-  return conv_gru_entry<float>(who, x, xmask, cin, h_in, w_in, filter, filter_mc, cin_total, hid, out, update_res, cand_res, h_delta, stream, true);
+    return conv_gru_entry<mie_bf16>(who, x, xmask, cin, h_in, w_in, filter, filter_mc, cin_total, hid, out, update_res, cand_res, h_delta, stream, 0);
+  MIE_REQUIRE(x3, MIE_ERR_UNSUPPORTED, "%s: fp32 deltas in terms only (MIE_DTYPE_F32_BF16X3, MIE_DTYPE_F32_F16X2)", who);
+  return conv_gru_entry<float>(who, x, xmask, cin, h_in, w_in, filter, filter_mc, cin_total, hid, out, update_res, cand_res, h_delta, stream, x3);
 }

@@ -19,6 +19,8 @@
 //   * fp32 deltas as three bf16 terms (split3), the products by size in three accumulators, so that the large ones are added up
 //     among themselves: chains of 9 sums a chunk.  Error of the sums against fp64, relative 2-norm, split form -> this:
 //     256->256 1.20e-7 -> 1.07e-7, 512->512 1.90e-7 -> 1.44e-7, 64->64 1.4e-7 -> 0.8e-7.  bf16: three accumulators in turn.
+//     (For MIE_DTYPE_F32_F16X2 too: with two fp16 terms these would be 1.42e-7, 1.77e-7 and 1.15e-7, whose 23 bits a value show where so
+//     little else is rounded.)
 //   * Up-sampling: the sums of the source pixels in LDS, the window blended from them, as in k_conv_mfma.  fp32 layers of 256 channels are
 //     not taken: 25 taps of filter, 614 KB a workgroup, take as long as the split form (256->128 at 16x24 16.4 us, 14.6).
 // Measured back to back on one plane with all pixels active, the filter another each time, split form -> this, us:
@@ -759,6 +761,7 @@ bool deep_up(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
 }  // namespace
 
 bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles, int dtype) {
+  if (dtype == MIE_DTYPE_F32_F16X2) dtype = MIE_DTYPE_F32_BF16X3;      // (what this form multiplies for it)
   if (c1 <= 0 || c2 < 0 || cout <= 0 || tiles <= 0) return false;
   if (!((k == 3 && (s == 1 || s == 2)) || (k == 5 && s == 2))) return false;
   // what comes to the matrix cores at all (the queries must not name other layers: they run on the VALU); 3x3 stride 2 in three terms
@@ -774,6 +777,7 @@ bool mie_conv_deep_form(int k, int s, int c1, int c2, int cout, long long tiles,
 }
 // (fp32 of eight rows a workgroup: 128->64 at 64x64 17.8 us, k_upconv2x 16.1)
 bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype) {
+  if (dtype == MIE_DTYPE_F32_F16X2) dtype = MIE_DTYPE_F32_BF16X3;
   if ((dtype != MIE_DTYPE_BF16 && dtype != MIE_DTYPE_F32_BF16X3) || c <= 0 || cout <= 0 || tiles <= 0) return false;
   if (c % (dtype == MIE_DTYPE_BF16 ? 64 : 32) != 0 || cout % 32 != 0) return false;      // (other layers are refused)
   return dtype == MIE_DTYPE_BF16 ? deep_slabs(tiles, cout) <= DEEP_WGS : 2 * deep_slabs(tiles, cout) <= DEEP_WGS && c <= 128;

@@ -208,6 +208,93 @@ __device__ __forceinline__ void split3(const float (&f)[8], float4 (&pl)[3]) {
   split3_pair(f[4], f[5], pl[0].z, pl[1].z, pl[2].z);
   split3_pair(f[6], f[7], pl[0].w, pl[1].w, pl[2].w);
 }
+// F2 (fp32 deltas multiplied as two fp16 terms each): v * s = hi + lo with s a power of two, hi = v * s rounded to fp16, lo the
+// rest of it, kept as lo * 2^11 so that it has the exponents of hi.  The two carry 23 bits of v, sign included, and the three products
+// hi*hi, lo*hi, hi*lo (what is left out, lo*lo, is at most 2^-24 of |a*b|) are exact in the fp32 accumulator's input: half the
+// matrix instructions of the three bf16 terms, two thirds of their LDS and filter bytes.  Only one rounding a unit at the size of
+// the sum instead of three (the cross products are added up among themselves) more than pays for the bit: error of whole contractions
+// against fp64, relative 2-norm, of 288 / 1152 / 4608 terms in four chains 1.05 / 1.40 / 2.33e-7, three bf16 terms 1.09 / 1.89 /
+// 3.70e-7.
+// The price is fp16's range.  A workgroup takes s from the largest value of its first chunk (of both inputs'), which goes to [2^12, 2^13),
+// so that a value is held to 2^-23 of itself or 2^-48 of that largest one, whichever is more: within 2^26 of it nothing is lost.  The largest
+// of every eight staged channels of a pixel has to lie below 65000 and not below 2^-24, where 11 bits are left of it, or be zero.
+// Where one does not, infinities and NaN included, the workgroup does its contraction over on v_mfma_f32_32x32x2_f32, from the
+// same places of LDS and of a second, fp32, copy of the filter.  Over the networks' steps the largest value of a window was up to 3.5 times
+// its first chunk's, and such groups lay within 2^24 of it but for a few tiles of a recurrent state fed back (within 2^30, 2 tiles of 4767
+// 2^36).  The filter's scale takes its largest weight to [2^14, 2^15); a filter one of whose groups of eight input channels lies below 2^-29
+// of it is marked and contracted in fp32 always.
+typedef _Float16 mie_f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 mie_f16x8 __attribute__((ext_vector_type(8)));
+constexpr float F2_STEP = 2048.f;
+// (as multiply-adds whose results are fp16: seven instructions a pair)
+__device__ __forceinline__ void split2_pair(float f0, float f1, float s, float s_lo, float& p0, float& p1) {
+  const mie_f16x2 hi = {(_Float16)__builtin_fmaf(f0, s, 0.f), (_Float16)__builtin_fmaf(f1, s, 0.f)};
+  const mie_f16x2 lo = {(_Float16)__builtin_fmaf((float)hi[0], -F2_STEP, f0 * s_lo), (_Float16)__builtin_fmaf((float)hi[1], -F2_STEP, f1 * s_lo)};
+  p0 = __builtin_bit_cast(float, hi);
+  p1 = __builtin_bit_cast(float, lo);
+}
+__device__ __forceinline__ void split2(const float (&f)[8], float s, float4 (&pl)[2]) {
+  const float s_lo = s * F2_STEP;
+  split2_pair(f[0], f[1], s, s_lo, pl[0].x, pl[1].x);
+  split2_pair(f[2], f[3], s, s_lo, pl[0].y, pl[1].y);
+  split2_pair(f[4], f[5], s, s_lo, pl[0].z, pl[1].z);
+  split2_pair(f[6], f[7], s, s_lo, pl[0].w, pl[1].w);
+}
+// (NaN if one of them is)
+__device__ __forceinline__ float f2_max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
+__device__ __forceinline__ float f2_amax8(const float (&f)[8]) {
+  const float m = f2_max3(fabsf(f[0]), fabsf(f[1]), fabsf(f[2]));
+  return __builtin_elementwise_maximum(f2_max3(f2_max3(m, fabsf(f[3]), fabsf(f[4])), fabsf(f[5]), fabsf(f[6])), fabsf(f[7]));
+}
+// Largest magnitude of a wave's lanes (m >= 0), the same for all of them.
+__device__ __forceinline__ float f2_wave_max(float m) {
+  const auto step = [&](auto ctrl) {
+    m = __builtin_elementwise_maximum(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), decltype(ctrl)::value, 0xf, 0xf, false)));
+  };
+  step(std::integral_constant<int, 0x111>()); step(std::integral_constant<int, 0x112>());      // row_shr 1, 2, 4, 8
+  step(std::integral_constant<int, 0x114>()); step(std::integral_constant<int, 0x118>());
+  step(std::integral_constant<int, 0x142>()); step(std::integral_constant<int, 0x143>());      // row_bcast 15, 31
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), 63));
+}
+// The scale for values whose largest is m (anything: what does not fit is found later).
+__device__ __forceinline__ float f2_scale(float m) {
+  int e = (__float_as_int(m) >> 23) - 127;
+  e = m == 0.f ? 12 : e < -28 ? -28 : e > 52 ? 52 : e;
+  return __int_as_float((127 + 12 - e) << 23);
+}
+__device__ __forceinline__ float f2_unscale(float s) { return __int_as_float((254 << 23) - __float_as_int(s)); }      // 1 / s
+// The groups a thread stages: in terms at their scale, and noted.
+struct F2Groups {
+  float scale;
+  unsigned most, least;                   // bits of the largest, bits less one of the least, zeros left out
+  __device__ __forceinline__ void start(float s) { scale = s; most = 0u; least = ~0u; }
+  __device__ __forceinline__ void terms(const float (&f)[8], float4 (&pl)[2]) {
+    const unsigned u = __float_as_uint(f2_amax8(f));
+    most = max(most, u);
+    least = min(least, u - 1u);
+    split2(f, scale, pl);
+  }
+  __device__ __forceinline__ bool misfit() const {      // (the scale's exponent taken off the bounds)
+    const unsigned k = __float_as_uint(scale) - (127u << 23), lo = (127u - 24u) << 23, hi = 0x477de800u;      // 2^-24, 65000
+    return most > hi - k || least < lo - k - 1u;
+  }
+};
+// What a filter copy of this form ends with: 1 / (its scale), and whether all of it fits.
+template <typename T>
+__device__ __forceinline__ const float* f2_filter_end(const T* filt_mc, long long weights) {
+  return reinterpret_cast<const float*>(reinterpret_cast<const char*>(filt_mc) + 8 * weights);
+}
+__device__ __forceinline__ void mma_f16(v16f& acc, const float4& a, const float4& b) {
+  const v4f a4 = {a.x, a.y, a.z, a.w}, b4 = {b.x, b.y, b.z, b.w};
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mie_f16x8, a4), __builtin_bit_cast(mie_f16x8, b4), acc, 0, 0, 0);
+}
+__device__ __forceinline__ void mma_unit2_f2(v16f& acc0, v16f& acc1, v16f& sm0, v16f& sm1, const float4 (&a0)[2], const float4 (&a1)[2],
+                                             const float4 (&b)[2]) {
+  mma_f16(acc0, a0[0], b[0]); mma_f16(acc1, a1[0], b[0]);
+  mma_f16(sm0, a0[1], b[0]);  mma_f16(sm1, a1[1], b[0]);
+  mma_f16(sm0, a0[0], b[1]);  mma_f16(sm1, a1[0], b[1]);
+}
+
 // One unit (16 input channels of a tap) of the X3 contraction for the two pixel blocks of a tile: six bf16 MFMAs
 // per block.  The three large products (hi*hi, mid*hi, hi*mid) and the three small ones (lo*hi, mid*mid, hi*lo, 2^-16 of
 // the first) go to accumulators of their own, added in the epilogue: four independent chains, so that no MFMA
@@ -366,18 +453,20 @@ __device__ __forceinline__ void split_order(const ConvArgsT<T>& a, int& bx, int&
 // staged tile is four times the size: 16 channels, one unit per tap); where the k-split has more waves than a tap
 // has units it is over (sub-chunk, tap class).  Global loads, masks, epilogue: fp32.
 //
+// ARITH: 1 is X3, 2 the form F2 above, 0 neither.
 // AGAIN (X3 only): outputs whose sum is not finite are computed again in fp32 (conv_quad_again).
 // GRU (with GATES): the gate math of a ConvGRU in place of the ConvLSTM's chain; eight columns, update and candidate, to four
 // hidden channels.
 template <typename T, int K, int S, int WN, int NB, bool HALF, bool GATES = false, bool UP = false, bool SPLIT = false,
-          bool X3 = false, bool AGAIN = false, bool GRU = false>
+          int ARITH = 0, bool AGAIN = false, bool GRU = false>
 // (Build with -mllvm -pragma-unroll-threshold=65536: the unit loop of the 128-column 5x5 / 7x7 kernels is 100 / 196
 // positions long, and where the compiler refuses to unroll it the operand ring is indexed at run time and lands in
 // scratch memory -- a factor of three in time.)
-__global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GATES, UP, SPLIT, X3)) void k_conv_mfma(ConvArgsT<T> a) {
+__global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GATES, UP, SPLIT, ARITH != 0)) void k_conv_mfma(ConvArgsT<T> a) {
+  constexpr bool X3 = ARITH != 0, F2 = ARITH == 2;           // values in terms; in two of them
   static_assert(!X3 || (sizeof(T) == 4 && !HALF && (K == 3 || K == 5)), "X3: fp32 deltas, 3x3 / 5x5");
   using TL = std::conditional_t<X3, mie_bf16, T>;            // element type in LDS and on the matrix cores
-  constexpr int PL = X3 ? 3 : 1;                             // operand planes (terms per value)
+  constexpr int PL = F2 ? 2 : X3 ? 3 : 1;                    // operand planes (terms per value)
   constexpr int GPS = X3 ? 2 : 1;                            // 16-byte global loads per staging slot
   constexpr int NBUF = X3 ? ((K == 3 && S == 1) ? 2 : 1) : stage_buffers(S, (int)sizeof(T));
   constexpr int EPS = 16 / (int)sizeof(TL);                  // elements per 16-byte slot (4 / 8)
@@ -412,6 +501,8 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   constexpr int SMEM = (STAGE_F + LO_F > RED) ? STAGE_F + LO_F : RED;
   static_assert(SMEM * 4 <= 65536, "LDS budget");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
+  __shared__ float s_f2[F2 ? 5 : 1];                         // largest values of the waves' first slots; whether a group does not fit
+  static_assert(!F2 || !AGAIN, "two terms: what does not fit is contracted in fp32");
   TL* const sbuf = reinterpret_cast<TL*>(smem);
   float* const s_lo = smem + STAGE_F;
 
@@ -593,7 +684,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // masked pixels are zeroed when they are stored; from the second chunk on -- and in layers of fewer
   // chunks, where that would be a large share of the reads -- a masked pixel is not fetched at all.
   float4 st_reg[NLD][GPS];
-  auto load_slots = [&](float4 (&regs)[NLD][GPS], int c, bool first) {
+  auto load_slots = [&](float4 (&regs)[NLD][GPS], int c, bool first) __attribute__((always_inline)) {
     const bool second = c >= nch1;
     const T* xin = second ? a.x2 : a.x;
     const int cs = second ? a.c2 : a.c1;
@@ -616,7 +707,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       }
     }
   };
-  auto stage_load = [&](int c, bool first = false) {
+  auto stage_load = [&](int c, bool first = false) __attribute__((always_inline)) {
     if constexpr (UP) {
       const T* dummy = a.filt_mc;
 #pragma unroll
@@ -636,8 +727,16 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     load_slots(st_reg, c, first);
   };
   // one staged slot to LDS: as it is, or (X3) its eight fp32 values as three bf16 planes
-  auto store_slot = [&](TL* dst, const float4 (&raw)[GPS]) {
-    if constexpr (X3) {
+  F2Groups groups;
+  bool filt_fits = true;                    // F2
+  auto store_slot = [&](TL* dst, const float4 (&raw)[GPS]) __attribute__((always_inline)) {
+    if constexpr (F2) {
+      const float f[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[GPS - 1].x, raw[GPS - 1].y, raw[GPS - 1].z, raw[GPS - 1].w};
+      float4 pl[2];
+      groups.terms(f, pl);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) *reinterpret_cast<float4*>(dst + q * STAGE) = pl[q];
+    } else if constexpr (X3) {
       const float f[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
       float4 pl[3];
       split3(f, pl);
@@ -647,8 +746,13 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       *reinterpret_cast<float4*>(dst) = raw[0];
     }
   };
-  auto kept = [](const float4& v, bool k) { return make_float4(k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f); };
-  auto store_slots = [&](const float4 (&regs)[NLD][GPS], int buf, unsigned ok) {
+  // F2's fp32 form: the first four channels of a slot where the leading terms would be, the others where the rests would
+  auto store_raw = [&](TL* dst, const float4 (&raw)[GPS]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < GPS; ++g) *reinterpret_cast<float4*>(dst + g * STAGE) = raw[g];
+  };
+  auto kept = [](const float4& v, bool k) __attribute__((always_inline)) { return make_float4(k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f); };
+  auto store_slots = [&](const float4 (&regs)[NLD][GPS], int buf, unsigned ok) __attribute__((always_inline)) {
     TL* dst = sbuf + buf * (PL * STAGE);
 #pragma unroll
     for (int i = 0; i < NLD; ++i)
@@ -659,11 +763,33 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         store_slot(dst + st_lds[i], r);
       }
   };
-  // (c: the chunk in the registers)
-  auto stage_store = [&](int buf, int c) {
+  // F2: the scale, from the first chunk's values (the sums of two, where they are added)
+  auto scale_of = [&](float m) __attribute__((always_inline)) {
+    m = f2_wave_max(m);
+    if (lane == 0) s_f2[wave] = m;
+    if (tid == 0) s_f2[F2 ? 4 : 0] = 0.f;
+    __syncthreads();
+    groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(
+        __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[F2 ? 1 : 0], s_f2[F2 ? 2 : 0]), s_f2[F2 ? 3 : 0]))))));
+  };
+  auto slots_max = [&](const float4 (&regs)[NLD][GPS], unsigned ok) __attribute__((always_inline)) {
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const float4 u = regs[i][0], v = regs[i][GPS - 1];
+      const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+      const float g = f2_amax8(f);
+      m = __builtin_elementwise_maximum(m, (ok >> i) & 1u ? g : 0.f);
+    }
+    return m;
+  };
+  // (c: the chunk in the registers; terms: in terms, or F2's fp32 form; first: the first chunk, F2's scale from its sums)
+  auto stage_store = [&](int buf, int c, auto terms, bool first = false) __attribute__((always_inline)) {
+    constexpr bool TERMS = decltype(terms)::value;
     TL* dst = sbuf + buf * (PL * STAGE);
     if constexpr (UP) {
       // x + x2 of the source block to LDS in fp32 (bit pattern zero = 0 in both element types) ...
+      float lo_max = 0.f;
 #pragma unroll
       for (int i = 0; i < NLO; ++i) {
         const int slot = tid + 256 * i;
@@ -686,9 +812,22 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
           for (int e = 0; e < EPS; e += 4)
             *reinterpret_cast<float4*>(&s_lo[lpix * LOS + q4 * EPS + e]) =
                 make_float4(fa[e] + fb[e], fa[e + 1] + fb[e + 1], fa[e + 2] + fb[e + 2], fa[e + 3] + fb[e + 3]);
+          if constexpr (F2 && TERMS) {
+            if (first) {
+              float f[8];
+#pragma unroll
+              for (int e = 0; e < 8; ++e) f[e] = fa[e] + fb[e];
+              lo_max = __builtin_elementwise_maximum(lo_max, f2_amax8(f));
+            }
+          }
         }
       }
-      __syncthreads();
+      if constexpr (F2 && TERMS) {
+        if (first) scale_of(lo_max);      // (with the barrier)
+        else __syncthreads();
+      } else {
+        __syncthreads();
+      }
       // ... and the staged tile blended from it; pixels outside the up-sampled image are the conv's zero padding.
       // The taps' LDS offsets and weights depend on the tile only, and the compiler computes them once
       // and keeps 40 registers alive through the contraction.  fp32 kernels have the registers to spare
@@ -728,7 +867,11 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         }
         const int lrow = pix / IT;
         TL* d = dst + lrow * RP + (pix - lrow * IT) * LS + EPS * q4;
-        if constexpr (X3) {
+        if constexpr (F2) {
+          const float4 raw[GPS] = {make_float4(o[0], o[1], o[2], o[3]), make_float4(o[4], o[5], o[6], o[7])};
+          if constexpr (TERMS) store_slot(d, raw);
+          else store_raw(d, raw);
+        } else if constexpr (X3) {
           float4 pl[3];
           split3(o, pl);
 #pragma unroll
@@ -739,7 +882,19 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       }
       return;
     }
-    store_slots(st_reg, buf, c >= nch1 ? ok2 : ok1);
+    const unsigned ok = c >= nch1 ? ok2 : ok1;
+    if constexpr (TERMS) {
+      store_slots(st_reg, buf, ok);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NLD; ++i)
+        if (tid + 256 * i < NSLOT) {
+          float4 r[GPS];
+#pragma unroll
+          for (int g = 0; g < GPS; ++g) r[g] = kept(st_reg[i][g], (ok >> i) & 1u);
+          store_raw(dst + st_lds[i], r);
+        }
+    }
   };
 
   // ---- operand addressing ------------------------------------------------------------------------
@@ -755,18 +910,20 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   auto unit_sub = [&](int unit) { return TPAR ? 0 : unit % NQW; };
   const int cob0 = co0 + wn * (32 * NB);                       // first column of this wave
   const int b_lane = (half * cout + l32) * EPS;                // lane part of the packed filter index
-  int a_lane[2][2];                                            // lane part of the LDS index
+  int a_lane[2], a_swap[2];                                    // lane part of the LDS index, what the other half adds to it
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb) {
     const int p = mb * 32 + l32;
     const int rowcol = ((p >> 3) * S) * RP + ((p & 7) * S) * LS + SUB * q0w;
     // stride 2: tile row r reads input row 2r + ky, whose halves are swapped iff (r + ky/2) is odd
     const int h0 = (S == 2) ? (half ^ ((p >> 3) & 1)) : half;
-    a_lane[mb][0] = rowcol + EPS * h0;
-    a_lane[mb][1] = rowcol + EPS * (h0 ^ 1);
+    a_lane[mb] = rowcol + EPS * h0;
+    a_swap[mb] = EPS * (1 - 2 * h0);
   }
+  // (where the tap depends on the wave, an index into the two would send them to LDS)
+  auto swapped = [&](int mb, int ky) __attribute__((always_inline)) { return (S == 2 && ((ky >> 1) & 1) != 0) ? a_lane[mb] + a_swap[mb] : a_lane[mb]; };
   // filter row block of chunk c for this wave (c1 and c2 are multiples of CC: no partial chunks)
-  auto chunk_b = [&](int c) -> const TL* {
+  auto chunk_b = [&](int c) __attribute__((always_inline)) -> const TL* {
     const bool second = c >= nch1;
     const int ci0 = (second ? c - nch1 : c) * CC;
     const int fb = second ? a.c1 : 0;
@@ -777,7 +934,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // the three term planes of a (block, tap) next to each other, P[ci/16][tap][term][(ci%16)/8][co][ci%8]).  The
   // k-steps of a unit are one 16-byte load per lane (and term), 512 contiguous bytes per half wave.
   float4 bring[RING][NB][PL];
-  auto load_b = [&](const TL* ub, int unit, float4 (&bv)[NB][PL]) {
+  auto load_b = [&](const TL* ub, int unit, float4 (&bv)[NB][PL]) __attribute__((always_inline)) {
     if (TPAR && unit * TP >= K * K) return;          // padding position: no unit for any wave
     int tap = unit_tap(unit);                        // compile-time after unrolling, but for the k-split over taps
     const int qi = unit_sub(unit);
@@ -800,6 +957,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // behind them.  (3x3 256->256: a chunk 1.55 -> 1.2 us in a launch of 16 workgroups, 18.3 -> 16.2 us together; at 33x44,
   // 240 workgroups, 20.0 -> 18.6; 512->512 at 8x12, unsplit, 30.7 -> 25.8.  On the full chip the matrix cores are held to
   // 1.6 .. 2.0 GHz by their power, and a launch that wastes less time runs at a lower clock.)
+  const auto in_terms = std::true_type();
   constexpr bool WOVEN = X3 && NBUF == 2 && !UP && UPC >= NLD + 3;
   constexpr int TRASH = IT * LS;                             // behind the pixels of row 0: where slots that do not exist go
   static_assert(!WOVEN || RP - IT * LS >= EPS, "room for a slot in the row padding");
@@ -807,7 +965,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
 #pragma unroll
   for (int i = 0; i < NLD; ++i) st_at[i] = tid + 256 * i < NSLOT ? st_lds[i] : TRASH;
   unsigned ok_n = 0u;                                        // which slots of the chunk in st_reg count
-  auto load_raw = [&](int c, bool first = false) {
+  auto load_raw = [&](int c, bool first = false) __attribute__((always_inline)) {
     const bool second = c >= nch1;
     const T* xin = second ? a.x2 : a.x;
     const int cs = second ? a.c2 : a.c1;
@@ -822,14 +980,18 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       for (int g = 0; g < GPS; ++g) st_reg[i][g] = *reinterpret_cast<const float4*>(p + 4 * g);
     }
   };
-  auto store_one = [&](int i, TL* dst) {
+  auto store_one = [&](int i, TL* dst) __attribute__((always_inline)) {
     const bool k = (ok_n >> i) & 1u;
     const float4 u = st_reg[i][0], v = st_reg[i][GPS - 1];
     const float f[8] = {k ? u.x : 0.f, k ? u.y : 0.f, k ? u.z : 0.f, k ? u.w : 0.f, k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f};
-    float4 pl[3];
-    split3(f, pl);
+    float4 pl[PL];
+    if constexpr (F2) {
+      groups.terms(f, pl);
+    } else if constexpr (X3) {
+      split3(f, pl);
+    }
 #pragma unroll
-    for (int q = 0; q < 3; ++q) *reinterpret_cast<float4*>(dst + st_at[i] + q * STAGE) = pl[q];
+    for (int q = 0; q < PL; ++q) *reinterpret_cast<float4*>(dst + st_at[i] + q * STAGE) = pl[q];
   };
   float4 st_first[WOVEN ? NLD : 1][GPS];
   // All B loads below are unconditional: a conditional load would make the compiler's wait
@@ -840,11 +1002,25 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   const int c_hi = SPLIT ? (bz + 1) * nch >> a.xcd_fs : nch;
   const TL* ub_cur = chunk_b(c_lo);
   const TL* ub_next = ub_cur;
+  // F2: the filter's scale and whether it fits, on their way from here on
+  float filt_unscale = 1.f;
+  if constexpr (F2) {
+    const float* const end = f2_filter_end(a.filt_mc, (long long)a.cin_total * (K * K) * cout);
+    filt_unscale = end[0];
+    filt_fits = end[1] != 0.f;
+  }
   MIE_STAMP(2);
   const bool early = c_hi - c_lo >= 4;      // uniform over the workgroup
   if constexpr (WOVEN) {
     if (early) load_slots(st_first, c_lo, true);
   } else if (early) stage_load(c_lo, true);
+  // F2, two inputs: the scale is for both, so it looks at the first chunk of the second one, too (a ConvLSTM's state deltas lie where the
+  // events of earlier steps were: where the input is zero, nothing is known of them)
+  const bool both = F2 && !UP && c_lo < nch1 && nch1 < c_hi;
+  float4 st_two[F2 && !UP ? NLD : 1][GPS];
+  if constexpr (F2 && !UP) {
+    if (both) load_slots(st_two, nch1, true);
+  }
   // the pixel-mask bytes, behind the first chunk's loads (pixel 0 stands in for slots outside the image, so that
   // these loads are unconditional too)
   {
@@ -898,8 +1074,15 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     mie_mask_asked();
   }
   // (masked pixels that the first chunk's loads fetched are zeroed here)
+  if constexpr (F2 && !UP) {
+    float m;
+    if constexpr (WOVEN) m = slots_max(st_first, c_lo >= nch1 ? ok2 : ok1);
+    else m = slots_max(st_reg, c_lo >= nch1 ? ok2 : ok1);
+    if (both) m = __builtin_elementwise_maximum(m, slots_max(st_two, ok2));
+    scale_of(m);
+  }
   if constexpr (WOVEN) store_slots(st_first, 0, c_lo >= nch1 ? ok2 : ok1);
-  else stage_store(0, c_lo);
+  else stage_store(0, c_lo, in_terms, true);
   __syncthreads();
   unsigned cp_bits = 0u;
   if (!SPLIT) live_bits = mie_mask_take(live_m, live_b, live_in);
@@ -908,7 +1091,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   MIE_STAMP(3);
 
   // A operand of unit `unit` from the staged chunk at `sin` (one 16-byte LDS read per pixel block).
-  auto load_a = [&](const TL* sin, int unit, float4 (&dst)[2][PL]) {
+  auto load_a = [&](const TL* sin, int unit, float4 (&dst)[2][PL]) __attribute__((always_inline)) {
     if (TPAR && unit * TP >= K * K) return;
     int tap = unit_tap(unit);
     const int qi = unit_sub(unit);
@@ -919,15 +1102,16 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
 #pragma unroll
       for (int q = 0; q < PL; ++q)
         dst[mb][q] = *reinterpret_cast<const float4*>(
-            &sin[q * STAGE + a_lane[mb][(S == 2) ? ((ky >> 1) & 1) : 0] + ky * RP + kx * LS + SUB * qi]);
+            &sin[q * STAGE + swapped(mb, ky) + ky * RP + kx * LS + SUB * qi]);
   };
   // the MFMAs of one unit position
-  auto mma = [&](int unit, const float4 (&av)[2][PL], const float4 (&bv)[NB][PL]) {
+  auto mma = [&](int unit, const float4 (&av)[2][PL], const float4 (&bv)[NB][PL]) __attribute__((always_inline)) {
     if (TPAR && unit * TP >= K * K) return;
     if (TPAR && unit * TP + TP > K * K && unit_tap(unit) >= K * K) return;     // uniform over the wave
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      if constexpr (X3) mma_unit2_x3(acc[0][nb], acc[1][nb], accs[0][nb], accs[1][nb], av[0], av[1], bv[nb]);
+      if constexpr (F2) mma_unit2_f2(acc[0][nb], acc[1][nb], accs[0][nb], accs[1][nb], av[0], av[1], bv[nb]);
+      else if constexpr (X3) mma_unit2_x3(acc[0][nb], acc[1][nb], accs[0][nb], accs[1][nb], av[0], av[1], bv[nb]);
       else mma_unit2(acc[0][nb], acc[1][nb], av[0][0], av[1][0], bv[nb][0], T());
     }
   };
@@ -973,9 +1157,9 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         }
         if (i <= NLD) {
 #pragma unroll
-          for (int j = 0; j < 12 * NB; ++j) {
+          for (int j = 0; j < (F2 ? 6 : 12) * NB; ++j) {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, F2 ? 8 : 5, 0);
             __builtin_amdgcn_sched_group_barrier(0x4, 3, 0);
           }
         }
@@ -1019,7 +1203,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
           __builtin_amdgcn_sched_barrier(0);
         }
         if (i == UPC - 3) {
-          if (more) stage_store((c - c_lo + 1) & 1, c + 1);    // the other buffer: nobody reads it during this chunk
+          if (more) stage_store((c - c_lo + 1) & 1, c + 1, in_terms);    // the other buffer: nobody reads it during this chunk
           __builtin_amdgcn_sched_barrier(0);
         }
         if (i == UPC - 2) {
@@ -1061,7 +1245,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         if (PD == 0) load_b(ub_next, 0, bring[0]);   // ring of one: reload right after use
       }
       if (NBUF == 1 && !UP) __syncthreads();   // every wave is done reading the only buffer (UP: stage_store syncs)
-      if (more) stage_store((c - c_lo + 1) % NBUF, c + 1);
+      if (more) stage_store((c - c_lo + 1) % NBUF, c + 1, in_terms);
       __syncthreads();
       ub_cur = ub_next;
       MIE_STAMP(4 + (c - c_lo));
@@ -1071,7 +1255,15 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // ---- epilogue -----------------------------------------------------------------------------------
   // acc[mb][nb][r] of this lane is output pixel p = 32*mb + 8*(r/4) + 4*half + r%4,
   // channel column wn*32*NB + 32*nb + lane%32 of the workgroup's slab.
-  if constexpr (X3) {
+  if constexpr (F2) {
+    const float c0 = f2_unscale(groups.scale) * filt_unscale, c1 = c0 * (1.f / F2_STEP);      // exactly: powers of two between 2^-111 and 2^100
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mb][nb][r] = fmaf(accs[mb][nb][r], c1, acc[mb][nb][r] * c0);
+  } else if constexpr (X3) {
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -1079,6 +1271,65 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[mb][nb][r] += accs[mb][nb][r];
   }
+  // the wave's sums to LDS, where all of them meet behind a barrier
+  auto park = [&]() __attribute__((always_inline)) {
+    float* red = smem + wk * (64 * CO_BLK);
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int p = mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          red[p * CO_BLK + wn * (32 * NB) + nb * 32 + l32] = acc[mb][nb][r];
+      }
+  };
+  auto meet = [&]() __attribute__((always_inline)) {
+    park();
+    if constexpr (F2) {
+      if (groups.misfit() || !filt_fits) s_f2[4] = 1.f;
+    }
+    __syncthreads();
+    if constexpr (F2) {
+      // a group that does not fit: all of it once more, on the fp32 instruction, as plainly as it can be said.  (Every workgroup of 3x3
+      // 256->256 at 33x44: 41 us instead of 13.5, three bf16 terms 17.5; 64->64 at 132x176: 33, 14.3 and 17.6)
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.f;
+        const long long fp32_at = 2LL * a.cin_total * (K * K) * cout;      // (in elements of two bytes: behind the terms)
+        for (int c = c_lo; c < c_hi; ++c) {
+          stage_load(c);
+          __syncthreads();
+          stage_store(0, c, std::false_type());
+          __syncthreads();
+          const TL* const ub = chunk_b(c) + fp32_at;
+#pragma unroll 1
+          for (int u = 0; u < UPC; ++u) {
+            if (unit_tap(u) >= K * K) break;
+            float4 av[2][PL], bv[NB][PL];
+            load_b(ub, u, bv);
+            const int ky = unit_tap(u) / K, kx = unit_tap(u) - ky * K;
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+              for (int q = 0; q < PL; ++q)
+                av[mb][q] = *reinterpret_cast<const float4*>(&sbuf[q * STAGE + swapped(mb, ky) + ky * RP + kx * LS + SUB * unit_sub(u)]);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+              for (int q = 0; q < PL; ++q) mma_unit2(acc[0][nb], acc[1][nb], av[0][q], av[1][q], bv[nb][q], float());
+          }
+        }
+        __syncthreads();
+        park();
+        __syncthreads();
+      }
+    }
+  };
   if constexpr (GRU) {
     // Gate math of a ConvGRU: column 8 * j + e is the update gate of hidden channel 4 * j + e (e < 4) or the candidate of 4 * j + e - 4.
     // An item is a pixel x four adjacent hidden channels: two 16-byte groups in LDS, 16 bytes of either reservoir, 16 (bf16: 8) of
@@ -1094,17 +1345,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       ru[i] = *reinterpret_cast<const float4*>(a.res + at);
       rc[i] = *reinterpret_cast<const float4*>(a.g_cres + at);
     }
-    float* red = smem + wk * (64 * CO_BLK);
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int p = mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          red[p * CO_BLK + wn * (32 * NB) + nb * 32 + l32] = acc[mb][nb][r];
-      }
-    __syncthreads();
+    meet();
 #pragma unroll
     for (int i = 0; i < PERG; ++i) {
       if (!((live_in >> i) & 1u)) continue;
@@ -1148,17 +1389,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       go[i] = pix * a.cout + co0 + 16 * g4;
       conv_gates_load<T>(a, (live_bits >> i) & 1u, (cp_bits >> i) & 1u, ho[i], go[i], item[i]);
     }
-    float* red = smem + wk * (64 * CO_BLK);
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int p = mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          red[p * CO_BLK + wn * (32 * NB) + nb * 32 + l32] = acc[mb][nb][r];
-      }
-    __syncthreads();
+    meet();
 #pragma unroll
     for (int i = 0; i < PERG; ++i) {
       if (!((live_in >> i) & 1u)) continue;
@@ -1178,17 +1409,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   } else {
     // the last barrier of the main loop has retired every read of the staging buffers that is used
     if (!EARLY && !SPLIT) epilogue_fetch(0);      // (ahead of the exchange: bf16 2x200x280 pass 298.8 -> 294.7 us with k_upconv2x's)
-    float* red = smem + wk * (64 * CO_BLK);
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int p = mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          red[p * CO_BLK + wn * (32 * NB) + nb * 32 + l32] = acc[mb][nb][r];
-      }
-    __syncthreads();
+    meet();
     unsigned bad_bits = 0u;                      // groups whose sums are not finite (conv_quad_again)
 #pragma unroll
     for (int h0 = 0; h0 < PER; h0 += PB) {       // the 128-column slabs in two passes of four groups per thread
@@ -1411,6 +1632,14 @@ void launch_split_finish(const ConvArgsT<T>& a, unsigned cap, int parts, hipStre
   hipLaunchKernelGGL((k_conv_split_finish<T, K, S>), dim3(cap, ny), dim3(256), 0, st, a, parts);
 }
 
+// The arguments of an F2 kernel: the filter copy from its fp16 terms on.
+template <typename T>
+ConvArgsT<T> f2_args(const ConvArgsT<T>& a0, int k) {
+  ConvArgsT<T> a = a0;
+  a.filt_mc = (const T*)((const char*)a0.filt_mc + 6LL * a0.cin_total * k * k * a0.cout);
+  return a;
+}
+
 template <typename T, int K, int S>
 bool launch_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   constexpr bool HAS_X3 = sizeof(T) == 4 && (K == 5 || (K == 3 && S == 1));
@@ -1423,12 +1652,15 @@ bool launch_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   const dim3 grid(a.cout / 32 * parts, cap);
   const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
-    if constexpr (HAS_X3) hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true, true>), grid, dim3(256), 0, st, a);
+    if constexpr (HAS_X3) {
+      if (a.x3 == 2) hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true, 2>), grid, dim3(256), 0, st, f2_args(a, K));
+      else hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true, 1>), grid, dim3(256), 0, st, a);
+    }
   } else {
     hipLaunchKernelGGL((k_conv_mfma<T, K, S, 1, 1, false, false, false, true>), grid, dim3(256), 0, st, a);
   }
   if constexpr (HAS_X3 && S == 2) {
-    if (x3) {
+    if (a.x3 == 1) {
       launch_split_finish<T, K, S>(a, cap, parts, st);
       return true;
     }
@@ -1450,8 +1682,11 @@ bool launch_up_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   if constexpr (sizeof(T) == 4) x3 = a.x3 != 0;
   const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
-    if constexpr (sizeof(T) == 4)
-      hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true, true>), dim3(a.cout / 32 * parts, cap), dim3(256), 0, st, a);
+    if constexpr (sizeof(T) == 4) {
+      const dim3 grid(a.cout / 32 * parts, cap);
+      if (a.x3 == 2) hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true, 2>), grid, dim3(256), 0, st, f2_args(a, 5));
+      else hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true, 1>), grid, dim3(256), 0, st, a);
+    }
   } else {
     hipLaunchKernelGGL((k_conv_mfma<T, 5, 1, 1, 1, false, false, true, true>), dim3(a.cout / 32 * parts, cap), dim3(256), 0, st, a);
   }
@@ -1474,8 +1709,11 @@ bool launch_gates_split(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   if constexpr (sizeof(T) == 4) x3 = a.x3 != 0;
   const std::lock_guard<std::mutex> pair(mie_split_launches());
   if (x3) {
-    if constexpr (sizeof(T) == 4)
-      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true, true>), dim3(a.cout / 32 * parts, cap), dim3(256), 0, st, a);
+    if constexpr (sizeof(T) == 4) {
+      const dim3 grid(a.cout / 32 * parts, cap);
+      if (a.x3 == 2) hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true, 2>), grid, dim3(256), 0, st, f2_args(a, 3));
+      else hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true, 1>), grid, dim3(256), 0, st, a);
+    }
   } else {
     hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, false, false, true>), dim3(a.cout / 32 * parts, cap), dim3(256), 0, st, a);
   }
@@ -1577,31 +1815,35 @@ inline bool x3_takes(int k, int s, int c1, int c2, int cout) {
   return (k == 3 || k == 5) && s == 1 && c1 % 32 == 0 && c2 % 32 == 0 && cout % 32 == 0;
 }
 
-template <int K, bool GATES, bool UP, int S = 1>
-bool launch_x3(const ConvArgsT<float>& a0, unsigned cap, hipStream_t st) {
+template <int AR, int K, bool GATES, bool UP, int S>
+bool launch_terms(const ConvArgsT<float>& a0, unsigned cap, hipStream_t st) {
   ConvArgsT<float> a = a0;
   const int cout = a.cout;
   if (!x3_takes(K, S, a.c1, UP ? 0 : a.c2, cout)) return false;
-  if constexpr (S == 2) {
+  if constexpr (S == 2 && AR == 1) {
     // few tiles and a workspace, but too few chunks to split (32->64 at 64x96): the same outputs as from the split form
     if (a.ws != nullptr && !a.refresh && (long long)cap * (cout / 32) <= 128) {
-      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 1, 1, false, GATES, UP, false, true, true>), dim3(xcd_plan(a, cap, cout / 32, K, UP), cout / 32), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 1, 1, false, GATES, UP, false, AR, true>), dim3(xcd_plan(a, cap, cout / 32, K, UP), cout / 32), dim3(256), 0, st, a);
       return true;
     }
   }
   switch (pick_slab_x3(cout, cap, S)) {
     case 128:
-      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 4, 1, false, GATES, UP, false, true>), dim3(xcd_plan(a, cap, cout / 128, K, UP), cout / 128), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 4, 1, false, GATES, UP, false, AR>), dim3(xcd_plan(a, cap, cout / 128, K, UP), cout / 128), dim3(256), 0, st, a);
       return true;
     case 64:
-      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 2, 1, false, GATES, UP, false, true>), dim3(xcd_plan(a, cap, cout / 64, K, UP), cout / 64), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 2, 1, false, GATES, UP, false, AR>), dim3(xcd_plan(a, cap, cout / 64, K, UP), cout / 64), dim3(256), 0, st, a);
       return true;
     case 32:
-      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 1, 1, false, GATES, UP, false, true>), dim3(xcd_plan(a, cap, cout / 32, K, UP), cout / 32), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<float, K, S, 1, 1, false, GATES, UP, false, AR>), dim3(xcd_plan(a, cap, cout / 32, K, UP), cout / 32), dim3(256), 0, st, a);
       return true;
     default:
       return false;
   }
+}
+template <int K, bool GATES, bool UP, int S = 1>
+bool launch_x3(const ConvArgsT<float>& a, unsigned cap, hipStream_t st) {
+  return a.x3 == 2 ? launch_terms<2, K, GATES, UP, S>(f2_args(a, K), cap, st) : launch_terms<1, K, GATES, UP, S>(a, cap, st);
 }
 
 template <typename T, int K, int S, bool HALF>
@@ -1683,26 +1925,31 @@ bool launch_gates(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
 }
 
 // The stacked gates conv of a ConvGRU, gate math in the epilogue.
-template <typename T>
-bool launch_gru(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
-  constexpr bool X3 = sizeof(T) == 4;
-  constexpr int CC = X3 ? 32 : 64;
+template <typename T, int AR>
+bool launch_gru_as(const ConvArgsT<T>& a0, unsigned cap, hipStream_t st) {
   ConvArgsT<T> a = a0;
   const int cout = a.cout;
-  if ((X3 && !a.x3) || a.c1 % CC != 0 || a.c2 % CC != 0 || cout != 2 * a.hid || cout % 32 != 0) return false;
-  switch (X3 ? pick_slab_x3(cout, cap, 1) : pick_slab<3, 1, false>(cout, cap)) {
+  switch (AR != 0 ? pick_slab_x3(cout, cap, 1) : pick_slab<3, 1, false>(cout, cap)) {
     case 128:
-      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 4, 1, false, true, false, false, X3, false, true>), dim3(xcd_plan(a, cap, cout / 128, 3), cout / 128), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 4, 1, false, true, false, false, AR, false, true>), dim3(xcd_plan(a, cap, cout / 128, 3), cout / 128), dim3(256), 0, st, a);
       return true;
     case 64:
-      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 2, 1, false, true, false, false, X3, false, true>), dim3(xcd_plan(a, cap, cout / 64, 3), cout / 64), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 2, 1, false, true, false, false, AR, false, true>), dim3(xcd_plan(a, cap, cout / 64, 3), cout / 64), dim3(256), 0, st, a);
       return true;
     case 32:
-      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, true, false, false, X3, false, true>), dim3(xcd_plan(a, cap, cout / 32, 3), cout / 32), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_conv_mfma<T, 3, 1, 1, 1, false, true, false, false, AR, false, true>), dim3(xcd_plan(a, cap, cout / 32, 3), cout / 32), dim3(256), 0, st, a);
       return true;
     default:
       return false;
   }
+}
+template <typename T>
+bool launch_gru(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
+  constexpr bool X3 = sizeof(T) == 4;
+  constexpr int CC = X3 ? 32 : 64;
+  if ((X3 && !a.x3) || a.c1 % CC != 0 || a.c2 % CC != 0 || a.cout != 2 * a.hid || a.cout % 32 != 0) return false;
+  if constexpr (X3) return a.x3 == 2 ? launch_gru_as<T, 2>(f2_args(a, 3), cap, st) : launch_gru_as<T, 1>(a, cap, st);
+  else return launch_gru_as<T, 0>(a, cap, st);
 }
 
 // Staging depth: the full one when both inputs' channel counts are multiples of it, else

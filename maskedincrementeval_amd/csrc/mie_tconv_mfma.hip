@@ -508,7 +508,7 @@ extern "C" int mie_tconv2x_masked(const void* x, const uint8_t* xmask, int c1, c
                                   int dtype, void* workspace, long long workspace_bytes, void* stream) {
   const char* who = "mie_tconv2x_masked";
   mie_clear_error();
-  const bool x3 = dtype == MIE_DTYPE_F32_BF16X3;
+  const bool x3 = dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2;      // (three terms for both)
   if (x3) dtype = MIE_DTYPE_F32;
   MIE_REQUIRE(dtype == MIE_DTYPE_F32 || dtype == MIE_DTYPE_BF16, MIE_ERR_UNSUPPORTED, "%s: unknown delta dtype %d", who, dtype);
   if (dtype == MIE_DTYPE_BF16)
@@ -526,7 +526,7 @@ extern "C" int mie_tconv2x_refresh(const void* x, int c1, const void* x2, int c2
                                    float* reservoir, int act_kind, float slope, int dtype, void* stream) {
   const char* who = "mie_tconv2x_refresh";
   mie_clear_error();
-  const bool x3 = dtype == MIE_DTYPE_F32_BF16X3;
+  const bool x3 = dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2;      // (three terms for both)
   if (x3) dtype = MIE_DTYPE_F32;
   MIE_REQUIRE(dtype == MIE_DTYPE_F32 || dtype == MIE_DTYPE_BF16, MIE_ERR_UNSUPPORTED, "%s: unknown delta dtype %d", who, dtype);
   if (dtype == MIE_DTYPE_BF16)
@@ -543,7 +543,7 @@ extern "C" int mie_tconv2x_lead_masked(const void* lead, const uint8_t* lead_mas
   const char* who = "mie_tconv2x_lead_masked";
   mie_clear_error();
   MIE_REQUIRE(lead != nullptr, MIE_ERR_INVALID_ARG, "%s: NULL pointer", who);
-  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3, MIE_ERR_UNSUPPORTED, "%s: bf16 or three-term fp32 deltas, not dtype %d", who, dtype);
+  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2, MIE_ERR_UNSUPPORTED, "%s: bf16 deltas or fp32 ones in terms, not dtype %d", who, dtype);
   if (dtype == MIE_DTYPE_BF16)
     return tconv2x_impl<mie_bf16>(who, x, xmask, c1, x2, x2mask, c2, h_in, w_in, filter, filter_mc, cin_total, 3, cout, out, blocks, out_delta,
                                   nullptr, reservoir, act_kind, slope, false, nullptr, nullptr, 0, stream, false, lead, lead_mask, lead_filter);

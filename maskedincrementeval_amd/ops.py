@@ -621,16 +621,23 @@ def build_unplanned_tiles(*args):
         _pass.phase = phase
 
 
-def pack_filter(filt: torch.Tensor, dtype=torch.float32, x3: bool = False) -> torch.Tensor:
+def pack_filter(filt: torch.Tensor, dtype=torch.float32, x3: bool = False, f16x2: bool = False) -> torch.Tensor:
     """Matrix-core copy of a contiguous fp32 [Cin,K,K,Cout] filter in `dtype`, shape
     [Cin/B, K*K, 2, Cout, B/2] with B = 8 (fp32) or 16 (bf16) input channels per block:
     element [b,t,h,co,j] is filt[B*b + (B/2)*h + j, t//K, t%K, co].
     x3=True: the three-term bf16 copy of an fp32 filter (MIE_DTYPE_F32_BF16X3), shape [Cin/16, K*K, 3, 2, Cout, 8]:
-    [b,t,0] + [b,t,1] + [b,t,2] is the fp32 weight, each term rounded to bf16."""
+    [b,t,0] + [b,t,1] + [b,t,2] is the fp32 weight, each term rounded to bf16.
+    f16x2=True: the copy for MIE_DTYPE_F32_F16X2, as bytes: the three bf16 terms as above, two fp16 terms
+    [Cin/16, K*K, 2, 2, Cout, 8], the fp32 weights in the same order (four channels where a term has eight), 1 / scale and whether all
+    weights fit it."""
     if filt.dim() != 4 or filt.shape[1] != filt.shape[2] or not filt.is_contiguous() or filt.dtype != torch.float32:
         raise ValueError("filter must be contiguous fp32 [Cin,K,K,Cout], got %s" % (tuple(filt.shape),))
     _require_gpu(filt, "filter")
     cin, k, _, cout = filt.shape
+    if f16x2:
+        packed = torch.empty(14 * filt.numel() + _lib.F16X2_END_BYTES, dtype=torch.uint8, device=filt.device)
+        check(lib().mie_pack_filter(filt.data_ptr(), cin, k, cout, packed.data_ptr(), _lib.DTYPE_F32_F16X2, _stream(filt)))
+        return packed
     if x3:
         packed = torch.empty((cin // 16, k * k, 3, 2, cout, 8), dtype=torch.bfloat16, device=filt.device)
         check(lib().mie_pack_filter(filt.data_ptr(), cin, k, cout, packed.data_ptr(), _lib.DTYPE_F32_BF16X3, _stream(filt)))
@@ -641,23 +648,34 @@ def pack_filter(filt: torch.Tensor, dtype=torch.float32, x3: bool = False) -> to
     return packed
 
 
-# How the matrix-core kernels multiply fp32 deltas: "bf16x3" = every value as three bf16 terms, six term products
+# How the matrix-core kernels multiply fp32 deltas.
+# "f16x2": every value as two fp16 terms under a scale that follows the data, three term products per multiply on the fp16 matrix-core
+# instruction, where the library has that form (mie_conv_f32x3_takes: 3x3 / 5x5 at stride 1 with channel counts in
+# multiples of 32, 5x5 at stride 2 in multiples of 16; on planes of few tiles 3x3 at stride 2: mie_conv_needs_no_workspace); values that do
+# not fit the scale are multiplied on the fp32 instruction (include/mie.h, MIE_DTYPE_F32_F16X2).  Error against fp64 0.6-0.97 times
+# that of three bf16 terms.
+# "bf16x3": every value as three bf16 terms, six term products
 # per multiply on the bf16 matrix-core instruction (fp32 accuracy: the three dropped products are at most 2^-23 of
 # |x * w|, typically 2^-26, and the measured error against fp64 is 0.6-1.1 times the fp32 instruction's; about twice
-# its rate), where the library has that form (mie_conv_f32x3_takes: 3x3 / 5x5 at stride 1 with channel counts in
-# multiples of 32, 5x5 at stride 2 in multiples of 16; the stride-2 transposed conv in multiples of 64), and on planes of few tiles
-# 3x3 at stride 2 (mie_conv_needs_no_workspace: 64..512 channels there, error against fp64 0.35-0.73 times the fp32
-# instruction's); "native" = v_mfma_f32_32x32x2_f32 everywhere.  Environment variable MIE_F32_MATMUL.
-f32_matmul = os.environ.get("MIE_F32_MATMUL", "bf16x3")
+# its rate), for the same layers and the stride-2 transposed conv in multiples of 64 channels; no scale, whatever the range of the values.
+# "native": v_mfma_f32_32x32x2_f32 everywhere.  Environment variable MIE_F32_MATMUL.
+f32_matmul = os.environ.get("MIE_F32_MATMUL", "f16x2")
+
+
+def f32_in_terms() -> int:
+    """MIE_DTYPE_* code of fp32 deltas multiplied in terms under the current setting, 0 (MIE_DTYPE_F32) for the fp32 instruction."""
+    if f32_matmul == "f16x2":
+        return _lib.DTYPE_F32_F16X2
+    if f32_matmul == "bf16x3":
+        return _lib.DTYPE_F32_BF16X3
+    if f32_matmul != "native":
+        raise ValueError("ops.f32_matmul must be 'f16x2', 'bf16x3' or 'native', not %r" % (f32_matmul,))
+    return _lib.DTYPE_F32
 
 
 def f32x3_takes(k: int, stride: int, c1: int, c2: int, cout: int) -> bool:
-    """Whether a conv of this shape on fp32 deltas runs in the three-term bf16 form under the current setting."""
-    if f32_matmul != "bf16x3":
-        if f32_matmul != "native":
-            raise ValueError("ops.f32_matmul must be 'bf16x3' or 'native', not %r" % (f32_matmul,))
-        return False
-    return bool(lib().mie_conv_f32x3_takes(k, stride, c1, c2, cout))
+    """Whether a conv of this shape on fp32 deltas runs in terms under the current setting."""
+    return f32_in_terms() != _lib.DTYPE_F32 and bool(lib().mie_conv_f32x3_takes(k, stride, c1, c2, cout))
 
 
 class ConvFilter:
@@ -672,12 +690,17 @@ class ConvFilter:
         self._rows = {}
         self._bf16 = None
         self._x3 = None
+        self._f16x2 = None
         self._up2x = {}
 
-    def for_dtype(self, dtype, x3: bool = False):
-        """(plain fp32 tensor, matrix-core copy | None) for deltas of `dtype`; x3: the three-term copy for fp32
+    def for_dtype(self, dtype, x3: bool = False, f16x2: bool = False):
+        """(plain fp32 tensor, matrix-core copy | None) for deltas of `dtype`; x3 / f16x2: the three-term / two-term copy for fp32
         deltas (Cin % 16 == 0), made on first use."""
         if dtype == torch.float32:
+            if f16x2 and self.plain.is_cuda and self.plain.shape[0] % 16 == 0:
+                if self._f16x2 is None:
+                    self._f16x2 = pack_filter(self.plain.contiguous(), f16x2=True)
+                return self.plain, self._f16x2
             if x3 and self.plain.is_cuda and self.plain.shape[0] % 16 == 0:
                 if self._x3 is None:
                     self._x3 = pack_filter(self.plain.contiguous(), x3=True)
@@ -722,16 +745,16 @@ class ConvFilter:
 
 def _filter_args(filt, k, dtype=torch.float32, x3_shape=None, with_code=False, three_term=False):
     """(plain tensor, pointer of the matrix-core copy or None) of a Tensor or ConvFilter; with_code: a third value,
-    the MIE_DTYPE_* code of the call.  x3_shape = (stride, c1, c2, cout): fp32 deltas take the three-term bf16 form
-    (its filter copy, its code) where the setting (f32_matmul) and the library allow it; three_term: so the caller has found."""
+    the MIE_DTYPE_* code of the call.  x3_shape = (stride, c1, c2, cout): fp32 deltas are multiplied in terms
+    (that filter copy, that code) where the setting (f32_matmul) and the library allow it; three_term: so the caller has found."""
     mc = None
     code = _DTYPES.get(dtype)
     if isinstance(filt, ConvFilter):
         x3 = (x3_shape is not None and dtype == torch.float32 and filt.plain.shape[0] % 16 == 0
               and (three_term or f32x3_takes(k, *x3_shape)))
-        filt, mc = filt.for_dtype(dtype, x3)
         if x3:
-            code = _lib.DTYPE_F32_BF16X3
+            code = f32_in_terms()
+        filt, mc = filt.for_dtype(dtype, x3 and code == _lib.DTYPE_F32_BF16X3, x3 and code == _lib.DTYPE_F32_F16X2)
     if filt.dim() != 4 or filt.shape[1] != k or filt.shape[2] != k or not filt.is_contiguous() \
             or filt.dtype != torch.float32:
         raise ValueError("filter must be contiguous fp32 [Cin,%d,%d,Cout], got %s" % (k, k, tuple(filt.shape)))
@@ -810,8 +833,8 @@ def conv_masked(x, xmask, x2, x2mask, filt, k, stride, pad, out_ts: TileMask, ou
     small = k in (3, 5) and out_ts.capacity * (filt.shape[3] // 32) <= 128
     x3_shape = (stride, c1, c2, filt.shape[3]) if path != _lib.PATH_VALU else None
     # (3x3 stride 2 runs on the fp32 instruction but for planes of few tiles)
-    three_term = (k, stride) == (3, 2) and x3_shape is not None and workspace is None and f32_matmul == "bf16x3" and dt == torch.float32 \
-        and bool(lib().mie_conv_needs_no_workspace(k, stride, c1, c2, filt.shape[3], out_ts.capacity, _lib.DTYPE_F32_BF16X3))
+    three_term = (k, stride) == (3, 2) and x3_shape is not None and workspace is None and dt == torch.float32 and f32_in_terms() != _lib.DTYPE_F32 \
+        and bool(lib().mie_conv_needs_no_workspace(k, stride, c1, c2, filt.shape[3], out_ts.capacity, f32_in_terms()))
     filt, mc_ptr, code = _filter_args(filt, k, dt, x3_shape, with_code=True, three_term=three_term)
     cin_total, cout = filt.shape[0], filt.shape[3]
     if tuple(out_delta.shape) != (n, cout, out_ts.h, out_ts.w) or out_ts.n != n:
@@ -894,7 +917,7 @@ def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt, refresh=Fa
     n, c, h, w = a.shape
     chunk = mfma_chunk(a.dtype)
     if not (upconv2x_enabled and isinstance(filt, ConvFilter) and filt.plain.is_cuda and k == 5 and stride == 1 and pad == 2
-            and (a.dtype == torch.bfloat16 or (a.dtype == torch.float32 and f32_matmul == "bf16x3")) and c == filt.shape[0]
+            and (a.dtype == torch.bfloat16 or (a.dtype == torch.float32 and f32_in_terms() != _lib.DTYPE_F32)) and c == filt.shape[0]
             and c % chunk == 0 and cout % 32 == 0 and h >= 2 and w >= 2 and c * cout < 1 << 24
             and n * c * h * w * a.element_size() < 0xffffff00):
         return False
@@ -1075,7 +1098,7 @@ def tconv2x_takes(c1: int, c2: int, cout: int, k: int, stride: int, pad: int, ou
 def tconv2x_takes_lead(lead_c: int, c1: int, c2: int, cout: int, k: int, dtype) -> bool:
     """Whether tconv2x_masked takes a leading part of `lead_c` channels along with a layer of this shape."""
     return (lead_c == 2 and k == 3 and c1 % 64 == 0 and c2 % 64 == 0 and cout % 32 == 0
-            and (dtype == torch.bfloat16 or (dtype == torch.float32 and f32_matmul == "bf16x3")))
+            and (dtype == torch.bfloat16 or (dtype == torch.float32 and f32_in_terms() != _lib.DTYPE_F32)))
 
 
 def _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out, addend, reservoir):
@@ -1085,7 +1108,7 @@ def _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out, addend, reservoir):
         raise ValueError("x2 %s incompatible with x %s" % (tuple(x2.shape), tuple(x.shape)))
     # fp32 deltas in the three-term bf16 form where the setting asks for it and the channel counts are whole chunks of 64
     # (the same conditions under which ConvFilter.for_dtype hands out the three-term copy: else the fp32 copy and code)
-    x3 = (x.dtype == torch.float32 and isinstance(filt, ConvFilter) and f32_matmul == "bf16x3"
+    x3 = (x.dtype == torch.float32 and isinstance(filt, ConvFilter) and f32_in_terms() != _lib.DTYPE_F32
           and c1 % 64 == 0 and c2 % 64 == 0 and filt.shape[3] % 32 == 0
           and filt.plain.is_cuda and filt.plain.shape[0] % 16 == 0)
     if x3:

@@ -1,0 +1,145 @@
+"""The two-term fp16 form of the fp32 matrix-core convs (MIE_DTYPE_F32_F16X2): filter copy, error against fp64 beside three bf16
+terms, and the inputs that do not fit the scale of a workgroup.  No counterpart in the reference, whose convs have one arithmetic."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from maskedincrementeval_amd import _lib, ops
+from maskedincrementeval_amd.masked_types import TileMask
+from maskedincrementeval_amd.synthetic import he_normal_conv_weight
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _dev(t):
+    return ops.as_nhwc(t.to(DEV).contiguous(memory_format=torch.channels_last))
+
+
+def _filt(w_oihw):
+    return ops.ConvFilter(w_oihw.permute(1, 2, 3, 0).contiguous().to(DEV))
+
+
+@pytest.fixture
+def setting():
+    old = ops.f32_matmul
+    yield
+    ops.f32_matmul = old
+
+
+@pytest.mark.parametrize("top,bottom,fits", [(1.0, 1e-8, 1.0), (1e-12, 1e-20, 1.0), (3e10, 100.0, 1.0), (1.0, 1e-9, 0.0), (1e-20, 1e-32, 0.0),
+                                             (float("inf"), 1.0, 0.0), (float("nan"), 1.0, 0.0), (0.0, 0.0, 1.0)])
+def test_filter_copy(top, bottom, fits):
+    cin, k, cout = 32, 3, 40
+    g = torch.Generator().manual_seed(1)
+    w = (torch.rand(cin, k, k, cout, generator=g) + 0.5) * (1.0 if top != 0.0 else 0.0)
+    w = w * (min(top, 3e38) if top == top and top != 0.0 else 1.0) * 0.6
+    w[8:16, 1, 1, 5] = bottom * torch.rand(8, generator=g).clamp_min(0.5)          # a small group
+    w[3, 0, 0, 0], w[16:24, 2, 2, 7] = top, 0.0
+    raw = ops.pack_filter(w.contiguous().to(DEV), f16x2=True).cpu()
+    m = w.numel()
+    assert raw.numel() == 14 * m + _lib.F16X2_END_BYTES
+    three = raw[:6 * m].view(torch.bfloat16).view(cin // 16, k * k, 3, 2, cout, 8).permute(2, 0, 3, 5, 1, 4).reshape(3, cin, k, k, cout)
+    terms = raw[6 * m:10 * m].view(torch.float16).view(cin // 16, k * k, 2, 2, cout, 8).permute(2, 0, 3, 5, 1, 4).reshape(2, cin, k, k, cout).double()
+    values = raw[10 * m:14 * m].view(torch.float32).view(cin // 16, k * k, 2, 2, cout, 4).permute(0, 3, 2, 5, 1, 4).reshape(cin, k, k, cout)
+    end = raw[14 * m:14 * m + 16].view(torch.float32)
+    assert torch.equal(values.nan_to_num(nan=7.0), w.nan_to_num(nan=7.0))
+    assert end[1].item() == fits
+    if fits:
+        assert torch.equal(three.double().sum(0), w.double()) or top < 1e-30
+        back = (terms[0] + terms[1] / 2048) * end[0].double()
+        # 23 bits, and where a value lies far below the largest of its filter what the fp16 subnormals leave
+        assert ((back - w.double()).abs() <= w.double().abs() * 2.0 ** -23 + 2.0 ** -36 * end[0].double()).all()
+        mant = torch.frexp(end[0])[0].item()
+        assert mant == 0.5 and (top == 0.0 or 2.0 ** 14 <= (w.abs().max() / end[0]).item() < 2.0 ** 15)
+
+
+def _conv(x, wt, k, stride, mode, c1=None, xm=None, path=_lib.PATH_MFMA, workspace=None):
+    n, cin, h, w = x.shape
+    c1 = cin if c1 is None else c1
+    ho, wo = ops.conv_out_size(h, w, k, stride, k // 2)
+    ts = TileMask(n, ho, wo, DEV)
+    ops.build_mask_tiles(xm, None, n, h, w, _lib.FOOT_CONV, k, stride, k // 2, ts)
+    out = ops.new_nhwc(n, wt.shape[0], ho, wo, DEV)
+    ops.f32_matmul = mode
+    ops.conv_masked(_dev(x[:, :c1]), xm, None if c1 == cin else _dev(x[:, c1:]), None if c1 == cin else xm, _filt(wt), k, stride, k // 2, ts, out,
+                    path=path, workspace=workspace)
+    torch.cuda.synchronize()
+    return out.cpu().double()
+
+
+# planes of more than 256 slabs of 16 columns, or more channels than the one-launch form: k_conv_mfma, whole and (the last three with a workspace) split
+SHAPES = [(32, 32, 3, 1, 136, 130, None), (64, 64, 3, 1, 70, 75, None), (128, 128, 3, 1, 41, 47, 64), (256, 256, 3, 1, 33, 44, None),
+          (256, 512, 3, 1, 34, 39, 128), (64, 32, 5, 1, 33, 47, None), (128, 128, 5, 1, 34, 42, None), (32, 64, 5, 2, 131, 133, None),
+          (128, 256, 5, 2, 66, 88, None), (1024, 256, 3, 1, 17, 9, None), (256, 32, 5, 1, 16, 16, None), (512, 64, 5, 2, 17, 16, 256)]
+
+
+@pytest.mark.parametrize("cin,cout,k,stride,h,w,c1", SHAPES)
+def test_error_against_fp64_beside_three_terms(cin, cout, k, stride, h, w, c1, setting):
+    g = torch.Generator().manual_seed(cin + h)
+    x = torch.randn(1, cin, h, w, generator=g) * torch.rand(1, 1, h, w, generator=g)
+    wt = he_normal_conv_weight(cout, cin, k, 7)
+    ref = F.conv2d(x.double(), wt.double(), stride=stride, padding=k // 2)
+    bound = F.conv2d(x.double().abs(), wt.double().abs(), stride=stride, padding=k // 2)
+    err = {}
+    for mode in ("bf16x3", "f16x2"):
+        e = (_conv(x, wt, k, stride, mode, c1) - ref).abs()
+        err[mode] = (e.norm() / ref.norm()).item(), (e / bound).max().item()
+    # the norm of the error is that of some thousand outputs at least; a single output's may be either way
+    assert err["f16x2"][0] <= err["bf16x3"][0] and err["f16x2"][1] < 4e-7, err
+
+
+@pytest.mark.parametrize("cin,cout,k,stride,h,w,c1", SHAPES)
+def test_scaled_inputs_give_scaled_outputs(cin, cout, k, stride, h, w, c1, setting):
+    """The scale follows the data: inputs times a power of two, the same bits."""
+    g = torch.Generator().manual_seed(cin)
+    x = torch.randn(1, cin, h, w, generator=g)
+    wt = he_normal_conv_weight(cout, cin, k, 7)
+    one = _conv(x, wt, k, stride, "f16x2", c1)
+    for e in (-27, 30):
+        assert torch.equal(_conv(x * 2.0 ** e, wt * 2.0 ** -e, k, stride, "f16x2", c1), one)
+        assert torch.equal(_conv(x * 2.0 ** e, wt, k, stride, "f16x2", c1), one * 2.0 ** e)
+
+
+@pytest.mark.parametrize("cin,cout,k,stride,h,w,c1", SHAPES)
+@pytest.mark.parametrize("what", ["below", "above", "not finite", "filter", "first chunk zero", "second input only"])
+def test_values_that_do_not_fit_the_scale(cin, cout, k, stride, h, w, c1, what, setting):
+    """Every value of the result within 4e-7 of sum |x||w|, three fp32 roundings, as the fp32 instruction has it; non-finite ones
+    where an fp32 conv has them, and only there."""
+    g = torch.Generator().manual_seed(cin + k)
+    x, wt = torch.randn(1, cin, h, w, generator=g), he_normal_conv_weight(cout, cin, k, 7)
+    if what == "below":
+        x[:, :, h // 2:] *= 1e-13
+    elif what == "above":
+        x[:, cin // 2:] *= 1e6
+    elif what == "filter":
+        wt[:, : cin // 2] *= 1e-10
+    elif what == "first chunk zero":
+        x[:, :32] = 0.0
+        x *= 1e-3
+    elif what == "second input only":
+        x[:, : cin // 2] *= 1e-12
+    else:
+        x[0, 1, 2, 3], x[0, cin - 1, h - 1, w - 1], x[0, 0, h // 2, 0], x[0, cin // 2, h // 2, w - 2] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    got = _conv(x, wt, k, stride, "f16x2", c1)
+    ref = F.conv2d(x.double(), wt.double(), stride=stride, padding=k // 2)
+    bound = F.conv2d(x.double().abs(), wt.double().abs(), stride=stride, padding=k // 2)
+    if what == "not finite":
+        want = F.conv2d(x, wt, stride=stride, padding=k // 2)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+        assert torch.equal(got[torch.isinf(want)].float(), want[torch.isinf(want)])
+        fine = torch.isfinite(want) & torch.isfinite(ref)
+    else:
+        fine = torch.isfinite(ref)
+        assert torch.isfinite(got).all()
+    assert ((got - ref).abs() <= 4e-7 * bound)[fine].all(), ((got - ref).abs() / bound)[fine].max()
+
+
+def test_masked_pixels_do_not_count(setting):
+    """What lies under a cleared mask byte is neither multiplied nor looked at for the scale."""
+    g = torch.Generator().manual_seed(3)
+    x, wt = torch.randn(1, 64, 70, 75, generator=g), he_normal_conv_weight(64, 64, 3, 7)
+    m = (torch.rand(1, 1, 70, 75, generator=g) < 0.5).to(torch.uint8)
+    clean = _conv(x * m, wt, 3, 1, "f16x2", xm=m.to(DEV))
+    junk = torch.where(m.bool().expand_as(x), x, torch.full((), float("inf")))
+    assert torch.equal(_conv(junk, wt, 3, 1, "f16x2", xm=m.to(DEV)), clean)
