@@ -925,7 +925,7 @@ int mie_events_to_frame_bf16(const double* events, int n_events, int kind, int n
  * a + b, one per output phase, with combined filters -- mie_upconv_masked's layer (interpolate_from_module +
  * nnConvIncr.forward, incr_modules/e2depth_incr.py:306-313,429-431) in 16 instead of 25 products per weight.
  *   filter_up : mie_pack_filter_up2x's copy for the dtype
- *   dtype     : MIE_DTYPE_BF16, or MIE_DTYPE_F32_BF16X3 for fp32 deltas; c a multiple of 64 / 32, cout of 32;
+ *   dtype     : MIE_DTYPE_BF16, or MIE_DTYPE_F32_BF16X3 / MIE_DTYPE_F32_F16X2 for fp32 deltas; c a multiple of 64 / 32, cout of 32;
  *               planes of at least 2x2 pixels
  *   the rest as in mie_upconv_masked.  The tile set's flags are read: it must be one of the library's builders'.
  *   Whole blocks of 8 x 8 positions (128 -> 64 channels in bf16 on large planes: 8 x 16) run for any active tile in
@@ -948,7 +948,8 @@ int mie_upconv2x_refresh(const void* a, const void* b, int c, int h_in, int w_in
 /*
  * Combined filters of mie_upconv2x_masked from a plain fp32 [cin][5][5][cout] filter (combined in double, rounded once):
  * `packed` holds 4 * 80 * cin * cout bf16 values (16 taps, and the planes' four sides and corners,
- * per phase) (MIE_DTYPE_BF16) or three times that (MIE_DTYPE_F32_BF16X3).
+ * per phase) (MIE_DTYPE_BF16) or three times that (MIE_DTYPE_F32_BF16X3), or
+ * 8 bytes a value, two fp16 terms and the fp32 one, and MIE_F16X2_END_BYTES (MIE_DTYPE_F32_F16X2).
  * cin a multiple of 16, cout of 32.
  */
 int mie_pack_filter_up2x(const float* filter, int cin, int cout, void* packed, int dtype,

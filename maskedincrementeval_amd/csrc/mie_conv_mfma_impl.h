@@ -259,7 +259,7 @@ __device__ __forceinline__ float f2_wave_max(float m) {
 // The scale for values whose largest is m (anything: what does not fit is found later).
 __device__ __forceinline__ float f2_scale(float m) {
   int e = (__float_as_int(m) >> 23) - 127;
-  e = m == 0.f ? 12 : e < -28 ? -28 : e > 52 ? 52 : e;
+  e = m == 0.f ? 12 : e < -60 ? -60 : e > 52 ? 52 : e;
   return __int_as_float((127 + 12 - e) << 23);
 }
 __device__ __forceinline__ float f2_unscale(float s) { return __int_as_float((254 << 23) - __float_as_int(s)); }      // 1 / s
@@ -1256,7 +1256,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // acc[mb][nb][r] of this lane is output pixel p = 32*mb + 8*(r/4) + 4*half + r%4,
   // channel column wn*32*NB + 32*nb + lane%32 of the workgroup's slab.
   if constexpr (F2) {
-    const float c0 = f2_unscale(groups.scale) * filt_unscale, c1 = c0 * (1.f / F2_STEP);      // exactly: powers of two between 2^-111 and 2^100
+    const float c0 = f2_unscale(groups.scale) * filt_unscale, c1 = c0 * (1.f / F2_STEP);      // exactly: powers of two, 2^-143 at the least
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll

@@ -25,6 +25,7 @@
 // (Flag words are looked up where they are needed: kept in a small array indexed at run time they went to LDS, whose
 // promotion reads the workgroup size from the dispatch packet in host memory -- 7 us at the start of every workgroup.)
 #include "mie_conv_mfma_impl.h"
+#include "mie_pack_terms.h"
 
 namespace {
 
@@ -80,16 +81,8 @@ __device__ void up2x_coef(int q, int row, double (&c)[5]) {
   }
 }
 
-// P[phase][ci/16][unit][term][(ci%16)/8][co][ci%8] in bf16: one term (bf16 deltas) or the three of an fp32 value.
-template <int PL>
-__global__ __launch_bounds__(256) void k_pack_up2x(const float* __restrict__ f, mie_bf16* __restrict__ p, int cin, int cout) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= 4LL * UNITS * cin * cout) return;
-  const int co = (int)(i % cout);
-  long long t = i / cout;
-  const int ci = (int)(t % cin);
-  t /= cin;
-  const int u = (int)(t % UNITS), ph = (int)(t / UNITS);
+// The coefficients of unit u of phase ph's filter, down and across.
+__device__ void up2x_unit(int ph, int u, double (&cv)[5], double (&ch)[5]) {
   int vr, hr;
   double sign = 1.0;
   if (u < U_TOP) {
@@ -102,12 +95,30 @@ __global__ __launch_bounds__(256) void k_pack_up2x(const float* __restrict__ f, 
     const int side = u < U_RIGHT ? 0 : 1, k = u - (side ? U_RIGHT : U_LEFT);
     vr = k & 3; hr = 6 + 3 * side + (k >> 2);
   }
-  double cv[5], ch[5], v = 0.0;
   up2x_coef(ph >> 1, vr, cv);
   up2x_coef(ph & 1, hr, ch);
+  for (int k = 0; k < 5; ++k) cv[k] *= sign;
+}
+__device__ __forceinline__ float up2x_weight(const float* __restrict__ f, const double (&cv)[5], const double (&ch)[5], int ci, int co, int cout) {
+  double v = 0.0;
   for (int ky = 0; ky < 5; ++ky)
     for (int kx = 0; kx < 5; ++kx) v += cv[ky] * ch[kx] * (double)f[((long long)ci * 25 + ky * 5 + kx) * cout + co];
-  const float w = (float)(sign * v);
+  return (float)v;
+}
+
+// P[phase][ci/16][unit][term][(ci%16)/8][co][ci%8] in bf16: one term (bf16 deltas) or the three of an fp32 value.
+template <int PL>
+__global__ __launch_bounds__(256) void k_pack_up2x(const float* __restrict__ f, mie_bf16* __restrict__ p, int cin, int cout) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= 4LL * UNITS * cin * cout) return;
+  const int co = (int)(i % cout);
+  long long t = i / cout;
+  const int ci = (int)(t % cin);
+  t /= cin;
+  const int u = (int)(t % UNITS), ph = (int)(t / UNITS);
+  double cv[5], ch[5];
+  up2x_unit(ph, u, cv, ch);
+  const float w = up2x_weight(f, cv, ch, ci, co, cout);
   const long long o = ((((((long long)ph * (cin / 16) + ci / 16) * UNITS + u) * PL) * 2 + (ci % 16) / 8) * cout + co) * 8 + ci % 8;
   const long long term = 2LL * cout * 8;
   const mie_bf16 hi = (mie_bf16)w;
@@ -118,6 +129,23 @@ __global__ __launch_bounds__(256) void k_pack_up2x(const float* __restrict__ f, 
     p[o + term] = mid;
     p[o + 2 * term] = (mie_bf16)(r1 - (float)mid);
   }
+}
+// The fp32 values of the two-term copy in their places, and the ranges of the blocks (mie_pack_terms.h).
+__global__ __launch_bounds__(256) void k_f2_up2x_values(const float* __restrict__ f, float* __restrict__ values, unsigned* __restrict__ parts,
+                                                        long long groups, int cin, int cout) {
+  unsigned most = 0u, least = ~0u;
+  for (long long g = (long long)blockIdx.x * 256 + threadIdx.x; g < groups; g += (long long)gridDim.x * 256) {
+    const int co = (int)(g % cout), half = (int)((g / cout) & 1);
+    const long long t = g / cout / 2;
+    const int u = (int)(t % UNITS), blk = (int)(t / UNITS % (cin / 16)), ph = (int)(t / UNITS / (cin / 16));
+    double cv[5], ch[5];
+    up2x_unit(ph, u, cv, ch);
+    float v[8];
+#pragma unroll 1
+    for (int j = 0; j < 8; ++j) v[j] = up2x_weight(f, cv, ch, blk * 16 + half * 8 + j, co, cout);
+    f2_put_values(values, t, half, co, cout, v, most, least);
+  }
+  f2_put_parts(parts, most, least);
 }
 
 // A unit of two M blocks in the three-term form, only the product of the leading terms into `acc` and the five smaller ones
@@ -136,11 +164,24 @@ __device__ __forceinline__ void mma_up2x_x3(v16f& acc0, v16f& acc1, v16f& sm0, v
   mma_unit(sm0, a0[0], b[1], mie_bf16()); mma_unit(sm1, a1[0], b[1], mie_bf16());
 }
 
-template <typename T, int WN>
+// The same in two fp16 terms, half as many products (kernel alone, all tiles active, three terms -> two: 256->128 at 33x44 48.0 -> 30.4 us,
+// 128->64 at 66x88 45.6 -> 28.8, at 32x32 15.1 -> 12.3).  The leading products of a chunk's units go in turn into two accumulators: with
+// one the error, relative 2-norm against fp64, would be that of three terms or above (256->128 at 33x44 2.8e-7), this way it is
+// 2.77 -> 2.22e-7, 1.97 -> 1.73e-7 and 1.45 -> 1.43e-7.
+__device__ __forceinline__ void mma_up2x_f2(v16f& acc0, v16f& acc1, v16f& sm0, v16f& sm1, const float4 (&a0)[2], const float4 (&a1)[2],
+                                            const float4 (&b)[2]) {
+  mma_f16(sm0, a0[1], b[0]);  mma_f16(sm1, a1[1], b[0]);
+  mma_f16(acc0, a0[0], b[0]); mma_f16(acc1, a1[0], b[0]);
+  mma_f16(sm0, a0[0], b[1]);  mma_f16(sm1, a1[0], b[1]);
+}
+
+// AR: 0 bf16 deltas, 1 fp32 in three bf16 terms, 2 in two fp16 terms (mie_conv_mfma_impl.h).
+template <typename T, int WN, int AR>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvArgsT<T> a, Up2xOrder od) {
-  constexpr bool X3 = sizeof(T) == 4;
+  static_assert((AR != 0) == (sizeof(T) == 4), "fp32 deltas in terms, bf16 as they are");
+  constexpr bool X3 = AR != 0, F2 = AR == 2;
   typedef mie_bf16 TL;
-  constexpr int PL = X3 ? 3 : 1;
+  constexpr int PL = F2 ? 2 : X3 ? 3 : 1;
   constexpr int GPS = X3 ? 2 : 1;                            // 16-byte global loads per staging slot
   constexpr int NBUF = X3 ? 2 : 1;
   constexpr int EPS = 8, SUB = 16;
@@ -169,6 +210,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   constexpr int SMEM = STAGE_F > RED ? STAGE_F : RED;
   static_assert(SMEM * 4 <= 65536, "LDS budget");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
+  __shared__ float s_f2[F2 ? 5 : 1];                         // F2: largest values of the waves' first slots; whether a group does not fit
   TL* const sbuf = reinterpret_cast<TL*>(smem);
 
   // ---- which positions, phase and slab: each XCD (workgroup index mod 8) takes a contiguous eighth of the order (group of
@@ -301,13 +343,16 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
         rb[i][g] = *reinterpret_cast<const float4*>(x2c + st_off[i] + 16 * g);
       }
   };
-  auto stage_store = [&](int buf) {
+  F2Groups groups;
+  // (terms: in terms, or F2's fp32 form; first: the first chunk, F2's scale from it)
+  auto stage_store = [&](int buf, auto terms, bool first = false) __attribute__((always_inline)) {
+    constexpr bool TERMS = decltype(terms)::value;
     TL* dst = sbuf + buf * (PL * STAGE);
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
+    float v[F2 ? NLD : 1][8];
+    auto sum = [&](int i, float (&f)[8]) __attribute__((always_inline)) {
       const bool k1 = (ok1 >> i) & 1u, k2 = (ok2 >> i) & 1u;
-      float fa[8], fb[8], f[8];
+      float fa[8], fb[8];
       if constexpr (X3) {
         const float4 a0 = k1 ? ra[i][0] : z4, a1 = k1 ? ra[i][1] : z4, b0 = k2 ? rb[i][0] : z4, b1 = k2 ? rb[i][1] : z4;
         const float ta[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
@@ -320,8 +365,38 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) f[e] = fa[e] + fb[e];
+    };
+    if constexpr (F2) {
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) sum(i, v[i]);
+      if (TERMS && first) {
+        float m = 0.f;
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) m = __builtin_elementwise_maximum(m, f2_amax8(v[i]));
+        m = f2_wave_max(m);
+        if (lane == 0) s_f2[wave] = m;
+        if (tid == 0) s_f2[4] = 0.f;
+        __syncthreads();
+        groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(
+            __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[1], s_f2[2]), s_f2[3]))))));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      float f[8];
+      if constexpr (F2) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = v[i][e];
+      } else {
+        sum(i, f);
+      }
       if (tid + 256 * i < n_slots) {
-        if constexpr (X3) {
+        if constexpr (F2) {
+          float4 pl[2] = {make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7])};
+          if constexpr (TERMS) groups.terms(f, pl);
+#pragma unroll
+          for (int q = 0; q < 2; ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
+        } else if constexpr (X3) {
           float4 pl[3];
           split3(f, pl);
 #pragma unroll
@@ -378,14 +453,24 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   };
   auto first_b = [&](int c) { return group_b(c, 0, side == 0 ? 4 * NI * cls : strip_unit(0)); };
 
-  v16f acc[2], sm[X3 ? 2 : 1];
+  v16f acc[2], acc_odd[F2 ? 2 : 1], sm[X3 ? 2 : 1];
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       acc[mb][r] = 0.f;
+      if (F2) acc_odd[mb][r] = 0.f;
       if (X3) sm[mb][r] = 0.f;
     }
+  // F2: the filter's scale and whether it fits, on their way from here on
+  const long long weights = 4LL * UNITS * a.c1 * cout;
+  float filt_unscale = 1.f;
+  bool filt_fits = true;
+  if constexpr (F2) {
+    const float* const end = f2_filter_end(a.filt_mc, weights);
+    filt_unscale = end[0];
+    filt_fits = end[1] != 0.f;
+  }
 
   float4 bring[4][PL];
   seek_b(first_b(0));
@@ -401,7 +486,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
     const int pl = i / (LS / EPS);
     *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (i - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  stage_store(0);
+  const auto in_terms = std::true_type();
+  stage_store(0, in_terms, true);
   __syncthreads();
 
   // All loads of a chunk are unconditional (see k_conv_mfma); behind the last one "the next" is the chunk itself.
@@ -434,7 +520,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
           __builtin_amdgcn_sched_barrier(0);
           const auto& A = av[i & 1];
           const auto& B = bring[i & 3];
-          if constexpr (X3) mma_up2x_x3(acc[0], acc[1], sm[0], sm[1], A[0], A[1], B);
+          if constexpr (F2) {
+            if (i & 1) mma_up2x_f2(acc_odd[0], acc_odd[1], sm[0], sm[1], A[0], A[1], B);
+            else mma_up2x_f2(acc[0], acc[1], sm[0], sm[1], A[0], A[1], B);
+          } else if constexpr (X3) mma_up2x_x3(acc[0], acc[1], sm[0], sm[1], A[0], A[1], B);
           else mma_unit2(acc[0], acc[1], A[0][0], A[1][0], B[0], mie_bf16());
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -471,7 +560,11 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
             const auto& A = av[t & 1];
             const auto& B = bring[t];
             if (t < 3 || !corner) {
-              if constexpr (X3) {
+              if constexpr (F2) {
+                mma_f16(sm[0], A[1], B[0]);
+                mma_f16(t & 1 ? acc_odd[0] : acc[0], A[0], B[0]);
+                mma_f16(sm[0], A[0], B[1]);
+              } else if constexpr (X3) {
                 mma_unit(sm[0], A[2], B[0], mie_bf16()); mma_unit(sm[0], A[1], B[1], mie_bf16());
                 mma_unit(acc[0], A[0], B[0], mie_bf16()); mma_unit(sm[0], A[0], B[2], mie_bf16());
                 mma_unit(sm[0], A[1], B[0], mie_bf16()); mma_unit(sm[0], A[0], B[1], mie_bf16());
@@ -485,12 +578,62 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
         }
       }
       if (NBUF == 1) __syncthreads();
-      if (more) stage_store((c + 1) % NBUF);
+      if (more) stage_store((c + 1) % NBUF, in_terms);
+      if constexpr (F2) {
+        if (!more && (groups.misfit() || !filt_fits)) s_f2[4] = 1.f;
+      }
       __syncthreads();
     }
   };
   if (side == 0) contract(std::true_type());
   else contract(std::false_type());
+  if constexpr (F2) {
+    const float c0 = f2_unscale(groups.scale) * filt_unscale, c1 = c0 * (1.f / F2_STEP);      // exactly: powers of two, 2^-143 at the least
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mb][r] = fmaf(sm[mb][r], c1, (acc[mb][r] + acc_odd[mb][r]) * c0);
+    // a group that does not fit: all of it once more on the fp32 instruction, from the fp32 copy of the filter behind the terms
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mb][r] = 0.f;
+      for (int c = 0; c < nch; ++c) {
+        stage_load(c);
+        __syncthreads();
+        stage_store(0, std::false_type());
+        __syncthreads();
+        auto unit = [&](const TL* gb, int at0, int at1) __attribute__((always_inline)) {
+#pragma unroll
+          for (int q = 0; q < PL; ++q) {
+            const float4 b = *reinterpret_cast<const float4*>(gb + 2 * weights + b_lane + q * (2 * cout * EPS));
+            mma_unit(acc[0], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at0]), b, float());
+            if (side == 0) mma_unit(acc[1], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at1]), b, float());
+          }
+        };
+        for (int qi = 0; qi < NQW; ++qi) {
+          if (side == 0) {
+#pragma unroll 1
+            for (int k = 0; k < 4 * NI; ++k) {
+              const int at = (cls * NI + (k >> 2)) * RP + (k & 3) * LS + SUB * qi;
+              unit(group_b(c, qi, 4 * NI * cls + k), a_lane[0] + at, a_lane[1] + at);
+            }
+          } else {
+#pragma unroll 1
+            for (int g = 0; g < ng; ++g) {
+              const int code = (int)((strip >> (4 * g)) & 15u);
+              const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
+              const int base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF, step = on ? (corner ? RPS : LS) : 0;
+#pragma unroll 1
+              for (int t = 0; t < (corner ? 3 : 4); ++t) unit(group_b(c, qi, strip_unit(g) + t), base + t * step, 0);
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
 
   // ---- epilogue ----------------------------------------------------------------------------------------------------------
   long long off[PB];
@@ -518,7 +661,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
     for (int r = 0; r < 16; ++r) {
       const int p = mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
       float s = acc[mb][r];
-      if (X3) s += sm[mb][r];
+      if (X3 && !F2) s += sm[mb][r];
       red[p * CO_BLK + wn * 32 + l32] = s;
     }
   __syncthreads();
@@ -541,13 +684,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   }
 }
 
-template <typename T, int WN>
+template <typename T, int WN, int AR>
 void launch_one(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
   od.combos = 4 * (a.cout / (32 * WN));
   od.total = a.ts.n * od.items * od.combos;
   // Launch order: the (phase, slab) pairs in `groups` parts.  Every part of the filter then reaches 8 / groups of the eight
   // L2s and the input all of them `groups` times; the split that moves the least is taken.
-  const double filt = 4.0 * 16 * a.c1 * a.cout * (sizeof(T) == 4 ? 6 : 2);
+  const double filt = 4.0 * 16 * a.c1 * a.cout * (AR == 2 ? 4 : AR == 1 ? 6 : 2);
   const double in = (double)a.ts.n * a.h_in * a.w_in * a.c1 * sizeof(T) * (a.x2 ? 2 : 1);
   double best = 8 * filt + in;
   od.groups = 1;
@@ -559,13 +702,14 @@ void launch_one(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
   od.m_cpg = mie_tile_magic(od.per_group, od.cpg);
   od.m_items = mie_tile_magic((long long)a.ts.n * od.items, od.items);
   od.m_bx = od.blocks_x > 0 ? mie_tile_magic(od.items, od.blocks_x) : 0u;
-  hipLaunchKernelGGL((k_upconv2x<T, WN>), dim3(8 * ((od.total + 7) / 8)), dim3(256), 0, st, a, od);
+  hipLaunchKernelGGL((k_upconv2x<T, WN, AR>), dim3(8 * ((od.total + 7) / 8)), dim3(256), 0, st, a, od);
 }
 
 // Slab width, by how many rounds of workgroups it takes.  A 64-column workgroup takes 1.75 times as long as a 32-column one.
 // fp32 (three-term): one workgroup fills a CU's matrix cores (two take twice as long), so a round is 256: 64 columns where they
 // need half the rounds or close to it, which leaves 32 columns up to one round (256->128 at 20x20: 26 us against 39) and in
-// the third (at 42x46, 608 of them: 68 against 78; at 33x44, 480: 48 against 45; at 60x80 134 against 122).  bf16: workgroups
+// the third (at 42x46, 608 of them: 68 against 78; at 33x44, 480: 48 against 45; at 60x80 134 against 122).  In two terms 64 columns
+// from one round on (256->128 at 25x35 29.9 against 27.7, at 42x46 45.4 and 46.5, 128->64 at 80x100 48.3 and 45.1; at 20x20 21.8 against 28.1).  bf16: workgroups
 // are short and three of a CU hide each other's latencies, so 64 columns start where 32 no longer fit one round of
 // 768 (128->64 at 66x74, 656 of them: 15.7 against 17.2; at 66x88, 784: 20.4 against 17.7), 128 columns, which read the
 // input least, where they make more than a round themselves (256->128 at 8x60x80: 246 against 217; at 4x60x80, 1440: 126
@@ -575,19 +719,20 @@ void launch_up2x(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
   const int cout = a.cout;
   const long long wgs = (long long)a.ts.n * od.items * 4 * (cout / 32);
   if constexpr (sizeof(T) == 4) {
-    if (cout % 64 == 0 && wgs > 256 && (wgs <= 512 || wgs > 768)) launch_one<T, 2>(a, od, st);
-    else launch_one<T, 1>(a, od, st);
+    const bool wide = cout % 64 == 0 && wgs > 256 && (wgs <= 512 || wgs > 768 || a.x3 == 2);
+    if (a.x3 == 2) wide ? launch_one<T, 2, 2>(a, od, st) : launch_one<T, 1, 2>(a, od, st);
+    else wide ? launch_one<T, 2, 1>(a, od, st) : launch_one<T, 1, 1>(a, od, st);
   } else {
-    if (cout % 128 == 0 && wgs / 4 >= 1024) launch_one<T, 4>(a, od, st);
-    else if (cout % 64 == 0 && wgs > 768) launch_one<T, 2>(a, od, st);
-    else launch_one<T, 1>(a, od, st);
+    if (cout % 128 == 0 && wgs / 4 >= 1024) launch_one<T, 4, 0>(a, od, st);
+    else if (cout % 64 == 0 && wgs > 768) launch_one<T, 2, 0>(a, od, st);
+    else launch_one<T, 1, 0>(a, od, st);
   }
 }
 
 template <typename T>
 int up2x_impl(const char* who, const void* x, const uint8_t* xm, const void* x2, const uint8_t* x2m, int c, int h, int w,
               const void* filter_up, int cout, const float* bias, const mie_tileset* out, void* out_delta, const void* addend,
-              float* reservoir, int act_kind, float slope, bool refresh, void* stream) {
+              float* reservoir, int act_kind, float slope, bool refresh, int terms, void* stream) {
   const int rc = mie_check_tileset(out, who);
   if (rc != MIE_OK) return rc;
   MIE_REQUIRE(x != nullptr && filter_up != nullptr && out_delta != nullptr, MIE_ERR_INVALID_ARG,
@@ -615,6 +760,7 @@ int up2x_impl(const char* who, const void* x, const uint8_t* xm, const void* x2,
   a.h_in = h; a.w_in = w; a.cin_total = c; a.filt_mc = (const T*)filter_up; a.pad = 2; a.cout = cout;
   a.out = (T*)out_delta; a.res = reservoir; a.act = act_kind; a.slope = slope; a.addend = (const T*)addend;
   a.refresh = refresh ? 1 : 0; a.bias = bias;
+  a.x3 = terms;
   a.ts = mie_dev_tileset(out);
   Up2xOrder od = {};
   od.flags = (const uint32_t*)out->flags;
@@ -641,12 +787,18 @@ extern "C" int mie_pack_filter_up2x(const float* filter, int cin, int cout, void
   mie_clear_error();
   MIE_REQUIRE(filter != nullptr && packed != nullptr && (const void*)filter != packed, MIE_ERR_INVALID_ARG,
               "%s: filter and packed must be given and differ", who);
-  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3, MIE_ERR_UNSUPPORTED, "%s: no combined filter of dtype %d", who, dtype);
+  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2, MIE_ERR_UNSUPPORTED, "%s: no combined filter of dtype %d", who, dtype);
   MIE_REQUIRE(cin > 0 && cout > 0 && cin % 16 == 0 && cout % 32 == 0 && (long long)cin * cout < (1LL << 24), MIE_ERR_UNSUPPORTED,
               "%s: needs cin %% 16 == 0 and cout %% 32 == 0 (cin=%d cout=%d)", who, cin, cout);
   MIE_REQUIRE(mie_aligned(filter, 4) && mie_aligned(packed, 16), MIE_ERR_INVALID_ARG, "%s: packed must be 16-byte aligned", who);
   const dim3 grid((unsigned)((4LL * UNITS * cin * cout + 255) / 256));
-  if (dtype == MIE_DTYPE_BF16)
+  if (dtype == MIE_DTYPE_F32_F16X2) {
+    const long long groups = 4LL * UNITS * (cin / 8) * cout;
+    const int blocks = mie_f2_blocks(groups);
+    hipLaunchKernelGGL(k_f2_up2x_values, dim3(blocks), dim3(256), 0, (hipStream_t)stream, filter, mie_f2_values(packed, groups),
+                       mie_f2_parts(packed, groups), groups, cin, cout);
+    mie_f2_split(packed, groups, blocks, cout, (hipStream_t)stream);
+  } else if (dtype == MIE_DTYPE_BF16)
     hipLaunchKernelGGL(k_pack_up2x<1>, grid, dim3(256), 0, (hipStream_t)stream, filter, (mie_bf16*)packed, cin, cout);
   else
     hipLaunchKernelGGL(k_pack_up2x<3>, grid, dim3(256), 0, (hipStream_t)stream, filter, (mie_bf16*)packed, cin, cout);
@@ -658,12 +810,12 @@ extern "C" int mie_upconv2x_masked(const void* a, const uint8_t* amask, const vo
                                    const void* addend, float* reservoir, int act_kind, float slope, int dtype, void* stream) {
   const char* who = "mie_upconv2x_masked";
   mie_clear_error();
-  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3, MIE_ERR_UNSUPPORTED, "%s: dtype %d not implemented", who, dtype);
+  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2, MIE_ERR_UNSUPPORTED, "%s: dtype %d not implemented", who, dtype);
   if (dtype == MIE_DTYPE_BF16)
     return up2x_impl<mie_bf16>(who, a, amask, b, bmask, c, h_in, w_in, filter_up, cout, nullptr, out, out_delta, addend, reservoir,
-                               act_kind, slope, false, stream);
+                               act_kind, slope, false, 0, stream);
   return up2x_impl<float>(who, a, amask, b, bmask, c, h_in, w_in, filter_up, cout, nullptr, out, out_delta, addend, reservoir,
-                          act_kind, slope, false, stream);
+                          act_kind, slope, false, dtype == MIE_DTYPE_F32_F16X2 ? 2 : 1, stream);
 }
 
 extern "C" int mie_upconv2x_refresh(const void* a, const void* b, int c, int h_in, int w_in, const void* filter_up, int cout,
@@ -671,10 +823,10 @@ extern "C" int mie_upconv2x_refresh(const void* a, const void* b, int c, int h_i
                                     float slope, int dtype, void* stream) {
   const char* who = "mie_upconv2x_refresh";
   mie_clear_error();
-  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3, MIE_ERR_UNSUPPORTED, "%s: dtype %d not implemented", who, dtype);
+  MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2, MIE_ERR_UNSUPPORTED, "%s: dtype %d not implemented", who, dtype);
   if (dtype == MIE_DTYPE_BF16)
     return up2x_impl<mie_bf16>(who, a, nullptr, b, nullptr, c, h_in, w_in, filter_up, cout, bias, out, out_dense, nullptr, reservoir,
-                               act_kind, slope, true, stream);
+                               act_kind, slope, true, 0, stream);
   return up2x_impl<float>(who, a, nullptr, b, nullptr, c, h_in, w_in, filter_up, cout, bias, out, out_dense, nullptr, reservoir,
-                          act_kind, slope, true, stream);
+                          act_kind, slope, true, dtype == MIE_DTYPE_F32_F16X2 ? 2 : 1, stream);
 }

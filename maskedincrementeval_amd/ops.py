@@ -715,14 +715,20 @@ class ConvFilter:
     def up2x(self, dtype) -> torch.Tensor:
         """The combined filters of upconv2x_masked for deltas of `dtype` (a 5x5 filter, Cin % 16 == 0, Cout % 32 == 0), made
         on first use from the fp32 weights."""
-        packed = self._up2x.get(dtype)
+        code = _lib.DTYPE_BF16 if dtype == torch.bfloat16 else _lib.DTYPE_F32_BF16X3
+        return self._up2x_of(code)
+
+    def _up2x_of(self, code: int) -> torch.Tensor:
+        """The same for a MIE_DTYPE_* code (MIE_DTYPE_F32_F16X2: as bytes)."""
+        packed = self._up2x.get(code)
         if packed is None:
             cin, cout = self.plain.shape[0], self.plain.shape[3]
-            terms = 3 if dtype == torch.float32 else 1
-            packed = torch.empty((4, cin // 16, 80, terms, 2, cout, 8), dtype=torch.bfloat16, device=self.plain.device)
-            check(lib().mie_pack_filter_up2x(self.plain.contiguous().data_ptr(), cin, cout, packed.data_ptr(),
-                                             _lib.DTYPE_F32_BF16X3 if terms == 3 else _lib.DTYPE_BF16, _stream(self.plain)))
-            self._up2x[dtype] = packed
+            if code == _lib.DTYPE_F32_F16X2:
+                packed = torch.empty(8 * 320 * cin * cout + _lib.F16X2_END_BYTES, dtype=torch.uint8, device=self.plain.device)
+            else:
+                packed = torch.empty((4, cin // 16, 80, 1 if code == _lib.DTYPE_BF16 else 3, 2, cout, 8), dtype=torch.bfloat16, device=self.plain.device)
+            check(lib().mie_pack_filter_up2x(self.plain.contiguous().data_ptr(), cin, cout, packed.data_ptr(), code, _stream(self.plain)))
+            self._up2x[code] = packed
         return packed
 
     @property
@@ -942,8 +948,13 @@ def _upconv2x_args(a, b, filt, out_ts, out, reservoir, addend):
         if t is not None and t.shape != out.shape:
             raise ValueError("%s shape %s != output %s" % (name, tuple(t.shape), tuple(out.shape)))
     _ready(out_ts)
-    up = replay.keep(filt.up2x(a.dtype))
-    return n, c, h, w, cout, up.data_ptr(), _lib.DTYPE_BF16 if a.dtype == torch.bfloat16 else _lib.DTYPE_F32_BF16X3
+    code = _lib.DTYPE_BF16 if a.dtype == torch.bfloat16 else f32_in_terms()
+    # (the four phases' sums are short: in two fp16 terms layers of 64 and 96 channels would be 1.13 and 1.05 times as far from fp64 as in three
+    # bf16 terms, from 128 on .99 and less: 128->64 1.97 -> 1.73e-7 at 66x88, 256->128 2.77 -> 2.22e-7 at 33x44)
+    if code == _lib.DTYPE_F32_F16X2 and c < 128:
+        code = _lib.DTYPE_F32_BF16X3
+    up = replay.keep(filt._up2x_of(code))
+    return n, c, h, w, cout, up.data_ptr(), code
 
 
 def upconv2x_masked(a, amask, b, bmask, filt: ConvFilter, out_ts: TileMask, out_delta, reservoir=None, act=_lib.ACT_NONE,

@@ -143,3 +143,53 @@ def test_masked_pixels_do_not_count(setting):
     clean = _conv(x * m, wt, 3, 1, "f16x2", xm=m.to(DEV))
     junk = torch.where(m.bool().expand_as(x), x, torch.full((), float("inf")))
     assert torch.equal(_conv(junk, wt, 3, 1, "f16x2", xm=m.to(DEV)), clean)
+
+
+def _up2x(a, b, wt, mode, out=None):
+    n, c, h, w = a.shape
+    ts = TileMask(n, 2 * h, 2 * w, DEV)
+    ops.build_mask_tiles(None, None, n, 2 * h, 2 * w, _lib.FOOT_CONV, 5, 1, 2, ts)
+    out = ops.new_nhwc(n, wt.shape[0], 2 * h, 2 * w, DEV)
+    ops.f32_matmul = mode
+    ops.upconv2x_masked(_dev(a), None, None if b is None else _dev(b), None, _filt(wt), ts, out)
+    torch.cuda.synchronize()
+    return out.cpu().double()
+
+
+# decoders at the resolution of their inputs: 32 columns a workgroup (up to 256 of them) and 64; blocks in part, strips and corners
+@pytest.mark.parametrize("c,cout,h,w,two", [(128, 64, 32, 32, True), (128, 64, 66, 88, True), (256, 128, 33, 44, True), (256, 64, 9, 11, False),
+                                            (160, 32, 21, 37, True), (128, 96, 2, 40, True), (128, 32, 10, 3, False)])
+@pytest.mark.parametrize("what", ["fits", "below", "above", "not finite", "filter"])
+def test_decoders_at_the_resolution_of_their_inputs(c, cout, h, w, two, what, setting):
+    g = torch.Generator().manual_seed(c + h)
+    a = torch.randn(1, c, h, w, generator=g) * torch.rand(1, 1, h, w, generator=g)
+    b = torch.randn(1, c, h, w, generator=g) if two else None
+    wt = he_normal_conv_weight(cout, c, 5, 7)
+    if what == "below":
+        a[:, :, h // 2:] *= 1e-13
+        b = None if b is None else b * (torch.arange(h).view(1, 1, h, 1) < h // 2)
+    elif what == "above":
+        a[:, c // 2:] *= 1e6
+    elif what == "filter":
+        wt[:, : c // 2] *= 1e-10
+    elif what == "not finite":
+        a[0, 1, h // 2, w // 2], a[0, c - 1, 0, 0] = float("inf"), float("nan")
+    up = lambda t: F.interpolate(t.double(), scale_factor=2, mode="bilinear", align_corners=False)      # noqa: E731
+    s = a if b is None else a + b
+    size = a.abs() if b is None else a.abs() + b.abs()
+    ref, bound = F.conv2d(up(s), wt.double(), padding=2), F.conv2d(up(size), wt.double().abs(), padding=2)
+    got = _up2x(a, b, wt, "f16x2")
+    if what == "not finite":
+        # (the phases' windows are the clamped taps': zero coefficients times an infinity make NaN of some outputs beside an fp32 conv's)
+        bad = torch.zeros(1, 1, h, w)
+        bad[0, 0, h // 2, w // 2] = bad[0, 0, 0, 0] = 1.0
+        near = F.max_pool2d(F.interpolate(F.max_pool2d(bad, 5, 1, 2), scale_factor=2), 3, 1, 1).bool().expand_as(got)
+        assert torch.isfinite(got[~near]).all() and not torch.isfinite(got[~torch.isfinite(ref)]).any()
+        fine = ~near
+    else:
+        fine = torch.ones_like(got, dtype=torch.bool)
+    # the combined weights are rounded sums of up to 25, the sum of the inputs is rounded: five fp32 roundings
+    assert ((got - ref).abs() <= 6e-7 * bound + 1e-30)[fine].all(), ((got - ref).abs() / bound)[fine].max()
+    if what == "fits":
+        three = _up2x(a, b, wt, "bf16x3")
+        assert (got - ref).norm() <= (three - ref).norm()
