@@ -37,12 +37,18 @@ __host__ __device__ constexpr int tc_shift(int k, int pad) { return (tc_phase(k,
 // along by a branch; of 128 that costs registers where there are none (364 -> 408; bf16 128->128 from 2x120x160 96.9 us, with the
 // branch 98.3, from 150x170 66.8, 68.1), and they are two forms (with the two channels 79.4, by the branch 81.0; of 64 columns a form of its
 // own was slower, 27.3 -> 30.2).
-template <typename T, int K, int WN, bool SPLIT, bool X3 = false, bool LEAD = false>
-__global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(ConvArgsT<T> a, TileSetDev pts) {
+// ARITH: 0 deltas as they are, 1 X3, 2 fp32 deltas in two fp16 terms (F2 of mie_conv_mfma_impl.h): leading products and cross products in
+// accumulators of their own, 256 of them, which one wave a SIMD has room for (X3 adds all six to one, as it has no room for two in its
+// 128-column form either).  All active, three terms -> two, us, and error against fp64: 64+64->64 from 160x160 38.1 -> 33.7, 1.97 -> 1.19e-7;
+// 512->256 from 40x44 34 -> 28, 2.84 -> 1.49e-7; 5x5 128+64->64 from 66x88 29.0 -> 22.4, 2.71 -> 1.47e-7; 64+64->32 from 128x128, two chunks,
+// bound by its trips to memory, 14.0 -> 13.7, 1.39 -> 1.07e-7.
+template <typename T, int K, int WN, bool SPLIT, int ARITH = 0, bool LEAD = false>
+__global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mfma(ConvArgsT<T> a, TileSetDev pts) {
+  constexpr bool X3 = ARITH != 0, F2 = ARITH == 2;
   static_assert(!X3 || sizeof(T) == 4, "X3: fp32 deltas");
   constexpr bool ANY_LEAD = K == 3 && !SPLIT && (X3 || sizeof(T) == 2) && WN < 4;      // (the types that mie_tconv2x_lead_masked takes)
   using TL = std::conditional_t<X3, mie_bf16, T>;            // element type in LDS and on the matrix cores
-  constexpr int PL = X3 ? 3 : 1;                             // operand planes (terms per value)
+  constexpr int PL = F2 ? 2 : X3 ? 3 : 1;                    // operand planes (terms per value)
   constexpr int GPS = X3 ? 2 : 1;                            // 16-byte global loads per staging slot
   constexpr int PAD = K / 2;
   constexpr int LO = (K == 5) ? 1 : 0;                       // halo above / left of the block (shifts reach -LO .. +1)
@@ -72,6 +78,7 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
   static_assert(SMEM * 4 <= 65536, "LDS budget");
   static_assert(!SPLIT || WN == 1, "the split form is the 32-channel slab kernel");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
+  __shared__ float s_f2[F2 ? 5 : 1];                         // F2: largest values of the waves' first slots; whether a group does not fit
   TL* const sbuf = reinterpret_cast<TL*>(smem);
 
   int n, y0, x0;                                             // block origin in INPUT coordinates
@@ -98,13 +105,25 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
     return;
   }
 
-  v16f acc[4][2];
+  v16f acc[4][2], sm[F2 ? 4 : 1][2];
 #pragma unroll
   for (int ph = 0; ph < 4; ++ph)
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[ph][mb][r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        acc[ph][mb][r] = 0.f;
+        if (F2) sm[F2 ? ph : 0][mb][r] = 0.f;
+      }
+  // F2: the filter's scale and whether it fits, on their way from here on
+  const long long weights = (long long)a.cin_total * (K * K) * cout;
+  float filt_unscale = 1.f;
+  bool filt_fits = true;
+  if constexpr (F2) {
+    const float* const end = f2_filter_end(a.filt_mc, weights);
+    filt_unscale = end[0];
+    filt_fits = end[1] != 0.f;
+  }
 
   // ---- staging plan (as in k_conv_mfma, stride 1) ------------------------------------------------------
   const int iy0 = y0 - LO, ix0 = x0 - LO;
@@ -136,7 +155,8 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
   const int nch = nch1 + (a.x2 != nullptr ? a.c2 / CC : 0);
 
   float4 st_reg[NLD][GPS];
-  auto stage_load = [&](int c) {
+  F2Groups groups;
+  auto stage_load = [&](int c) __attribute__((always_inline)) {
     const bool second = c >= nch1;
     const T* xin = second ? a.x2 : a.x;
     const int cs = second ? a.c2 : a.c1;
@@ -156,12 +176,30 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
       }
     }
   };
-  auto stage_store = [&](int buf) {
+  auto slots_max = [&](const float4 (&regs)[NLD][GPS]) __attribute__((always_inline)) {
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const float4 u = regs[i][0], v = regs[i][GPS - 1];
+      const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+      m = __builtin_elementwise_maximum(m, f2_amax8(f));
+    }
+    return m;
+  };
+  // (terms: in terms, or F2's fp32 form)
+  auto stage_store = [&](int buf, auto terms) __attribute__((always_inline)) {
     TL* dst = sbuf + buf * (PL * STAGE);
 #pragma unroll
     for (int i = 0; i < NLD; ++i)
       if (tid + 256 * i < NSLOT) {
-        if constexpr (X3) {
+        if constexpr (F2) {
+          const float4 u = st_reg[i][0], v = st_reg[i][GPS - 1];
+          const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+          float4 pl[2] = {u, v};
+          if constexpr (decltype(terms)::value) groups.terms(f, pl);
+#pragma unroll
+          for (int q = 0; q < 2; ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
+        } else if constexpr (X3) {
           const float f[8] = {st_reg[i][0].x, st_reg[i][0].y, st_reg[i][0].z, st_reg[i][0].w,
                               st_reg[i][1].x, st_reg[i][1].y, st_reg[i][1].z, st_reg[i][1].w};
           float4 pl[3];
@@ -191,7 +229,7 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
     return reinterpret_cast<const TL*>(a.filt_mc) + ((long long)((fb + ci0) / SUB + q0w) * (K * K) * (PL * 2) * cout + cob0) * EPS;
   };
   float4 bring[RING][PL];
-  auto load_b = [&](const TL* ub, int unit, float4 (&bv)[PL]) {
+  auto load_b = [&](const TL* ub, int unit, float4 (&bv)[PL]) __attribute__((always_inline)) {
     const int tap = unit / NQW, qi = unit % NQW;
 #pragma unroll
     for (int q = 0; q < PL; ++q)
@@ -202,10 +240,28 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
   const int c_hi = SPLIT ? (bz + 1) * nch >> a.xcd_fs : nch;
   const TL* ub_cur = chunk_b(c_lo);
   const TL* ub_next = ub_cur;
+  const auto in_terms = std::true_type();
+  const bool both = F2 && c_lo < nch1 && nch1 < c_hi;      // (F2: the scale is for both inputs)
+  float4 st_two[F2 ? NLD : 1][GPS];
+  if constexpr (F2) {
+    stage_load(both ? nch1 : c_lo);
+#pragma unroll
+    for (int i = 0; i < NLD; ++i)
+#pragma unroll
+      for (int g = 0; g < GPS; ++g) st_two[i][g] = st_reg[i][g];
+  }
   stage_load(c_lo);
 #pragma unroll
   for (int i = 0; i < (PD > 0 ? PD : 1); ++i) load_b(ub_cur, i, bring[i % RING]);
-  stage_store(0);
+  if constexpr (F2) {
+    const float m = f2_wave_max(__builtin_elementwise_maximum(slots_max(st_two), slots_max(st_reg)));
+    if (lane == 0) s_f2[wave] = m;
+    if (tid == 0) s_f2[4] = 0.f;
+    __syncthreads();
+    groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(
+        __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[1], s_f2[2]), s_f2[3]))))));
+  }
+  stage_store(0, in_terms);
   __syncthreads();
 
   for (int c = c_lo; c < c_hi; ++c) {
@@ -239,7 +295,9 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
         const int tap = i / NQW;
         const int ky = tap / K, kx = tap - ky * K;
         const int ph = tc_phase(ky, PAD) * 2 + tc_phase(kx, PAD);      // compile-time after unrolling
-        if constexpr (X3) {
+        if constexpr (F2) {
+          mma_unit2_f2(acc[ph][0], acc[ph][1], sm[ph][0], sm[ph][1], av[i & 1][0], av[i & 1][1], bring[i % RING]);
+        } else if constexpr (X3) {
           // the six significant term products of the unit, the two pixel blocks interleaved (smallest terms first)
           const auto& A = av[i & 1];
           const auto& B = bring[i % RING];
@@ -258,9 +316,49 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
       if (PD == 0) load_b(ub_next, 0, bring[0]);
     }
     if (NBUF == 1) __syncthreads();
-    if (more) stage_store((c - c_lo + 1) % NBUF);
+    if (more) stage_store((c - c_lo + 1) % NBUF, in_terms);
+    if constexpr (F2) {
+      if (!more && (groups.misfit() || !filt_fits)) s_f2[4] = 1.f;
+    }
     __syncthreads();
     ub_cur = ub_next;
+  }
+  float c0 = 1.f;                      // F2: 1 / scales
+  if constexpr (F2) {
+    c0 = f2_unscale(groups.scale) * filt_unscale;      // exactly: powers of two, 2^-143 at the least
+    // a group that does not fit: all of it once more on the fp32 instruction, from the fp32 copy of the filter behind the terms
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
+#pragma unroll
+      for (int ph = 0; ph < 4; ++ph)
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[ph][mb][r] = sm[ph][mb][r] = 0.f;
+      c0 = 1.f;
+      for (int c = c_lo; c < c_hi; ++c) {
+        stage_load(c);
+        __syncthreads();
+        stage_store(0, std::false_type());
+        __syncthreads();
+        const TL* const ub = chunk_b(c) + 2 * weights;
+#pragma unroll
+        for (int tap = 0; tap < K * K; ++tap) {      // (a tap's phase picks the accumulators)
+          const int ky = tap / K, kx = tap - ky * K, ph = tc_phase(ky, PAD) * 2 + tc_phase(kx, PAD);
+          const int at = (tc_shift(ky, PAD) + LO) * RP + (tc_shift(kx, PAD) + LO) * LS;
+#pragma unroll 1
+          for (int qi = 0; qi < NQW; ++qi) {
+            float4 b[PL];
+            load_b(ub, tap * NQW + qi, b);
+#pragma unroll
+            for (int q = 0; q < PL; ++q)
+#pragma unroll
+              for (int mb = 0; mb < 2; ++mb)
+                mma_unit(acc[ph][mb], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + a_lane[mb] + at + SUB * qi]), b[q], float());
+          }
+        }
+      }
+      __syncthreads();
+    }
   }
 
   // ---- epilogue, one phase at a time -----------------------------------------------------------------------
@@ -292,7 +390,7 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int p = mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        red[p * CO_BLK + wn * 32 + l32] = acc[ph][mb][r];
+        red[p * CO_BLK + wn * 32 + l32] = F2 ? fmaf(sm[F2 ? ph : 0][mb][r], c0 * (1.f / F2_STEP), acc[ph][mb][r] * c0) : acc[ph][mb][r];
       }
     __syncthreads();
     long long off[PER];
@@ -380,8 +478,9 @@ __global__ __launch_bounds__(256, !X3 && WN <= 2 ? 2 : 1) void k_tconv_mfma(Conv
   epilogue(std::integral_constant<int, 3>{});
 }
 
-template <typename T, int K, bool X3 = false>
+template <typename T, int K, int ARITH = 0>
 bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st) {
+  constexpr bool X3 = ARITH != 0;
   constexpr int CC = X3 ? 64 : stage_channels(K, 1) * (4 / (int)sizeof(T));
   if (a0.filt_mc == nullptr || a0.c1 % CC != 0 || a0.c2 % CC != 0 || a0.cout % 32 != 0) return false;
   constexpr bool DEEP = K == 3 && (X3 || sizeof(T) == 2);
@@ -391,7 +490,7 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
   // makes up for its second launch.  One launch over split, 2 to 64 slabs: 1280 channels .89 to 1.05, 1408 .88 to 1.11, 1536 .92 to 1.17,
   // 2048 1.04 to 1.31; 128 slabs of four tiles or fewer, 1536 .97 to 1.18, 2048 1.05 to 1.26, of more .75 to .97 (bf16 of 2048: .5 to 1.0).
   const bool split = !DEEP || (X3 && a0.g_cpd == nullptr && a0.c1 + a0.c2 > 1408 && (long long)cap_p * (cout / 16) <= (cap_p <= 4 ? 128 : 64));
-  ConvArgsT<T> a = a0;
+  ConvArgsT<T> a = ARITH == 2 ? f2_args(a0, K) : a0;
   a.xcd_fs = 0; a.xcd_m = 0;
   if constexpr (!DEEP || X3) {
     const unsigned cap_out = (unsigned)(a.ts.n * a.ts.tiles_y * a.ts.tiles_x);
@@ -405,7 +504,7 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
       if (parts >= 2) {
         a.xcd_fs = __builtin_ctz(parts);
         const std::lock_guard<std::mutex> pair(mie_split_launches());
-        hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, true, X3>), dim3(cout / 32 * parts, cap_p), dim3(256), 0, st, a, pts);
+        hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, true, ARITH>), dim3(cout / 32 * parts, cap_p), dim3(256), 0, st, a, pts);
         unsigned ny = (unsigned)((1024 + cap_out - 1) / cap_out);
         if (ny > (unsigned)(cout / 16)) ny = (unsigned)(cout / 16);
         if (ny < 1) ny = 1;
@@ -420,13 +519,13 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
   // form it would spill, so that form stops at 64 columns)
   if (!X3 && cout % 128 == 0 && (long long)cap_p * (cout / 128) >= 400) {
     if (DEEP && a.g_cpd != nullptr)
-      hipLaunchKernelGGL((k_tconv_mfma<T, K, 4, false, false, DEEP && !X3>), dim3(cap_p, cout / 128), dim3(256), 0, st, a, pts);
+      hipLaunchKernelGGL((k_tconv_mfma<T, K, 4, false, 0, DEEP && !X3>), dim3(cap_p, cout / 128), dim3(256), 0, st, a, pts);
     else
-      hipLaunchKernelGGL((k_tconv_mfma<T, K, 4, false, false>), dim3(cap_p, cout / 128), dim3(256), 0, st, a, pts);
+      hipLaunchKernelGGL((k_tconv_mfma<T, K, 4, false>), dim3(cap_p, cout / 128), dim3(256), 0, st, a, pts);
   } else if (cout % 64 == 0 && (long long)cap_p * (cout / 64) >= 400) {
-    hipLaunchKernelGGL((k_tconv_mfma<T, K, 2, false, X3>), dim3(cap_p, cout / 64), dim3(256), 0, st, a, pts);
+    hipLaunchKernelGGL((k_tconv_mfma<T, K, 2, false, ARITH>), dim3(cap_p, cout / 64), dim3(256), 0, st, a, pts);
   } else {
-    hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, false, X3>), dim3(cap_p, cout / 32), dim3(256), 0, st, a, pts);
+    hipLaunchKernelGGL((k_tconv_mfma<T, K, 1, false, ARITH>), dim3(cap_p, cout / 32), dim3(256), 0, st, a, pts);
   }
   return true;
 }
@@ -436,7 +535,7 @@ int tconv2x_impl(const char* who, const void* x, const uint8_t* xmask, int c1, c
                  const uint8_t* x2mask, int c2, int h_in, int w_in, const float* filter, const void* filter_mc,
                  int cin_total, int k, int cout, const mie_tileset* out, const mie_tileset* blocks,
                  void* out_delta, const void* addend, float* reservoir, int act_kind, float slope, bool refresh,
-                 const float* bias, void* workspace, long long workspace_bytes, void* stream, bool x3 = false,
+                 const float* bias, void* workspace, long long workspace_bytes, void* stream, int x3 = 0,
                  const void* lead = nullptr, const uint8_t* lead_mask = nullptr, const float* lead_filter = nullptr) {
   int rc = mie_check_tileset(out, who);
   if (rc != MIE_OK) return rc;
@@ -480,7 +579,7 @@ int tconv2x_impl(const char* who, const void* x, const uint8_t* xmask, int c1, c
   a.pad = k / 2; a.cout = cout; a.out = (T*)out_delta; a.res = reservoir; a.act = act_kind; a.slope = slope;
   a.addend = (const T*)addend; a.refresh = refresh ? 1 : 0; a.bias = bias;
   a.hid = 0; a.g_cpd = nullptr; a.g_cpm = nullptr; a.g_cpres = nullptr; a.g_cres = nullptr; a.g_dh = nullptr; a.g_dc = nullptr;
-  a.ws = (float*)workspace; a.ws_floats = workspace_bytes / 4; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = x3 ? 1 : 0;
+  a.ws = (float*)workspace; a.ws_floats = workspace_bytes / 4; a.ws_plane = 0; a.xcd_fs = 0; a.xcd_m = 0; a.x3 = x3;
   a.ts = mie_dev_tileset(out);
   const TileSetDev pts = mie_dev_tileset(blocks);
   if (lead != nullptr) {
@@ -490,7 +589,8 @@ int tconv2x_impl(const char* who, const void* x, const uint8_t* xmask, int c1, c
   }
   bool ok;
   if constexpr (sizeof(T) == 4) {
-    if (x3) ok = (k == 3) ? launch_tconv<T, 3, true>(a, pts, (hipStream_t)stream) : launch_tconv<T, 5, true>(a, pts, (hipStream_t)stream);
+    if (x3 == 2) ok = (k == 3) ? launch_tconv<T, 3, 2>(a, pts, (hipStream_t)stream) : launch_tconv<T, 5, 2>(a, pts, (hipStream_t)stream);
+    else if (x3) ok = (k == 3) ? launch_tconv<T, 3, 1>(a, pts, (hipStream_t)stream) : launch_tconv<T, 5, 1>(a, pts, (hipStream_t)stream);
     else ok = (k == 3) ? launch_tconv<T, 3>(a, pts, (hipStream_t)stream) : launch_tconv<T, 5>(a, pts, (hipStream_t)stream);
   } else {
     ok = (k == 3) ? launch_tconv<T, 3>(a, pts, (hipStream_t)stream) : launch_tconv<T, 5>(a, pts, (hipStream_t)stream);
@@ -508,7 +608,7 @@ extern "C" int mie_tconv2x_masked(const void* x, const uint8_t* xmask, int c1, c
                                   int dtype, void* workspace, long long workspace_bytes, void* stream) {
   const char* who = "mie_tconv2x_masked";
   mie_clear_error();
-  const bool x3 = dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2;      // (three terms for both)
+  const int x3 = dtype == MIE_DTYPE_F32_BF16X3 ? 1 : dtype == MIE_DTYPE_F32_F16X2 ? 2 : 0;
   if (x3) dtype = MIE_DTYPE_F32;
   MIE_REQUIRE(dtype == MIE_DTYPE_F32 || dtype == MIE_DTYPE_BF16, MIE_ERR_UNSUPPORTED, "%s: unknown delta dtype %d", who, dtype);
   if (dtype == MIE_DTYPE_BF16)
@@ -526,7 +626,7 @@ extern "C" int mie_tconv2x_refresh(const void* x, int c1, const void* x2, int c2
                                    float* reservoir, int act_kind, float slope, int dtype, void* stream) {
   const char* who = "mie_tconv2x_refresh";
   mie_clear_error();
-  const bool x3 = dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2;      // (three terms for both)
+  const int x3 = dtype == MIE_DTYPE_F32_BF16X3 ? 1 : dtype == MIE_DTYPE_F32_F16X2 ? 2 : 0;
   if (x3) dtype = MIE_DTYPE_F32;
   MIE_REQUIRE(dtype == MIE_DTYPE_F32 || dtype == MIE_DTYPE_BF16, MIE_ERR_UNSUPPORTED, "%s: unknown delta dtype %d", who, dtype);
   if (dtype == MIE_DTYPE_BF16)
@@ -546,7 +646,7 @@ extern "C" int mie_tconv2x_lead_masked(const void* lead, const uint8_t* lead_mas
   MIE_REQUIRE(dtype == MIE_DTYPE_BF16 || dtype == MIE_DTYPE_F32_BF16X3 || dtype == MIE_DTYPE_F32_F16X2, MIE_ERR_UNSUPPORTED, "%s: bf16 deltas or fp32 ones in terms, not dtype %d", who, dtype);
   if (dtype == MIE_DTYPE_BF16)
     return tconv2x_impl<mie_bf16>(who, x, xmask, c1, x2, x2mask, c2, h_in, w_in, filter, filter_mc, cin_total, 3, cout, out, blocks, out_delta,
-                                  nullptr, reservoir, act_kind, slope, false, nullptr, nullptr, 0, stream, false, lead, lead_mask, lead_filter);
+                                  nullptr, reservoir, act_kind, slope, false, nullptr, nullptr, 0, stream, 0, lead, lead_mask, lead_filter);
   return tconv2x_impl<float>(who, x, xmask, c1, x2, x2mask, c2, h_in, w_in, filter, filter_mc, cin_total, 3, cout, out, blocks, out_delta, nullptr,
-                             reservoir, act_kind, slope, false, nullptr, nullptr, 0, stream, true, lead, lead_mask, lead_filter);
+                             reservoir, act_kind, slope, false, nullptr, nullptr, 0, stream, dtype == MIE_DTYPE_F32_F16X2 ? 2 : 1, lead, lead_mask, lead_filter);
 }

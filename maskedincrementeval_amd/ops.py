@@ -1117,14 +1117,15 @@ def _tconv2x_args(x, x2, filt, k, out_ts, block_ts, out, addend, reservoir):
     c2 = 0 if x2 is None else x2.shape[1]
     if x2 is not None and (x2.shape[0] != n or x2.shape[2:] != x.shape[2:] or x2.dtype != x.dtype):
         raise ValueError("x2 %s incompatible with x %s" % (tuple(x2.shape), tuple(x.shape)))
-    # fp32 deltas in the three-term bf16 form where the setting asks for it and the channel counts are whole chunks of 64
-    # (the same conditions under which ConvFilter.for_dtype hands out the three-term copy: else the fp32 copy and code)
+    # fp32 deltas in terms where the setting asks for it and the channel counts are whole chunks of 64
+    # (the same conditions under which ConvFilter.for_dtype hands out such a copy: else the fp32 copy and code)
     x3 = (x.dtype == torch.float32 and isinstance(filt, ConvFilter) and f32_in_terms() != _lib.DTYPE_F32
           and c1 % 64 == 0 and c2 % 64 == 0 and filt.shape[3] % 32 == 0
           and filt.plain.is_cuda and filt.plain.shape[0] % 16 == 0)
     if x3:
-        plain, mc = replay.keep(filt.for_dtype(torch.float32, x3=True))
-        mc_ptr, code = mc.data_ptr(), _lib.DTYPE_F32_BF16X3
+        code = f32_in_terms()
+        plain, mc = replay.keep(filt.for_dtype(torch.float32, x3=code == _lib.DTYPE_F32_BF16X3, f16x2=code == _lib.DTYPE_F32_F16X2))
+        mc_ptr = mc.data_ptr()
     else:
         plain, mc_ptr = _filter_args(filt, k, x.dtype)
         code = delta_dtype(x)
@@ -1163,7 +1164,7 @@ def tconv2x_masked(x, xmask, x2, x2mask, filt, k, out_ts: TileMask, block_ts: Ti
             block_ts.ref, nhwc_ptr(out_delta, "out_delta", dtype=dt), nhwc_ptr(reservoir, "reservoir"), act, float(slope), code, _stream(x)))
         return out_delta
     # (3x3 on bf16 deltas and in the three-term form, but for very many channels there: one launch on planes of few blocks)
-    split = k != 3 or code == _lib.DTYPE_F32 or (code == _lib.DTYPE_F32_BF16X3 and c1 + c2 > 1408)
+    split = k != 3 or code == _lib.DTYPE_F32 or (code != _lib.DTYPE_BF16 and c1 + c2 > 1408)
     ws_ptr, ws_bytes = _workspace_args(workspace, block_ts.capacity * (cout // 32) <= 128 and split, x.device)
     check(lib().mie_tconv2x_masked(
         nhwc_ptr(x, "x", dtype=dt), pix_ptr(xmask, n, h, w, "xmask"), c1, nhwc_ptr(x2, "x2", dtype=dt),

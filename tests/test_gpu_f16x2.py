@@ -193,3 +193,43 @@ def test_decoders_at_the_resolution_of_their_inputs(c, cout, h, w, two, what, se
     if what == "fits":
         three = _up2x(a, b, wt, "bf16x3")
         assert (got - ref).norm() <= (three - ref).norm()
+
+
+# transposed convs: 32 and 64 columns a workgroup, planes cut off at both edges, split (more than 1408 channels on few blocks, 5x5)
+@pytest.mark.parametrize("c1,c2,cout,h,w,k", [(64, 64, 32, 127, 131, 3), (128, 0, 64, 132, 176, 3), (64, 64, 64, 160, 159, 3), (1024, 512, 64, 8, 7, 3),
+                                              (64, 64, 32, 90, 93, 5), (256, 64, 32, 9, 8, 5)])
+@pytest.mark.parametrize("what", ["fits", "below", "above", "not finite", "second input only"])
+def test_transposed_convs(c1, c2, cout, h, w, k, what, setting):
+    g = torch.Generator().manual_seed(c1 + h)
+    cin = c1 + c2
+    x = torch.randn(1, cin, h, w, generator=g)
+    wt = torch.randn(cin, cout, k, k, generator=g) * (8.0 / (cin * k * k)) ** 0.5
+    if what == "below":
+        x[:, :, h // 2:] *= 1e-13
+    elif what == "above":
+        x[:, cin // 2:] *= 1e6
+    elif what == "second input only":
+        x[:, :c1] = 0.0
+        x *= 1e-6
+    elif what == "not finite":
+        x[0, 1, h // 2, w // 2], x[0, cin - 1, 0, 0], x[0, 5, h - 1, w - 1] = float("inf"), float("nan"), float("-inf")
+    up = lambda x_, w_: F.conv_transpose2d(x_, w_, stride=2, padding=k // 2, output_padding=1)      # noqa: E731
+    ref, bound = up(x.double(), wt.double()), up(x.double().abs(), wt.double().abs())
+    filt = ops.ConvFilter(wt.permute(0, 2, 3, 1).contiguous().to(DEV))
+    ts, blocks = TileMask(1, 2 * h, 2 * w, DEV), TileMask(1, h, w, DEV)
+    ops.build_mask_tiles(None, None, 1, h, w, _lib.FOOT_TCONV, k, 2, k // 2, ts)
+    ops.build_mask_tiles(ts, None, 1, 2 * h, 2 * w, _lib.FOOT_CONV, 2, 2, 0, blocks)
+    got = {}
+    for mode in ("bf16x3", "f16x2"):
+        ops.f32_matmul = mode
+        out = ops.new_nhwc(1, cout, 2 * h, 2 * w, DEV)
+        ops.tconv2x_masked(_dev(x[:, :c1]), None, _dev(x[:, c1:]) if c2 else None, None, filt, k, ts, blocks, out)
+        torch.cuda.synchronize()
+        got[mode] = out.cpu().double()
+    fine = torch.isfinite(ref)
+    if what == "not finite":
+        want = up(x, wt)
+        assert torch.equal(torch.isnan(got["f16x2"]), torch.isnan(want)) and torch.equal(torch.isinf(got["f16x2"]), torch.isinf(want))
+    assert ((got["f16x2"] - ref).abs() <= 4e-7 * bound)[fine].all(), ((got["f16x2"] - ref).abs() / bound)[fine].max()
+    if what == "fits":
+        assert (got["f16x2"] - ref).norm() <= (got["bf16x3"] - ref).norm()
