@@ -939,6 +939,10 @@ int mie_upconv2x_masked(const void* a, const uint8_t* amask, const void* b,
                         void* out_delta, const void* addend, float* reservoir,
                         int act_kind, float slope, int dtype, void* stream);
 
+/* 1 where MIE_DTYPE_F32_F16X2 is the form of it for fp32 deltas that is nearer to fp64 and faster, 0 where MIE_DTYPE_F32_BF16X3 is (less than
+ * 128 channels on small planes, 32 channels), or there is neither.  Host logic. */
+int mie_f16x2_takes_upconv2x(int n, int h_in, int w_in, int c, int cout);
+
 /* Its dense twin (every tile of `out` active): bias, activation and reservoir fill as in mie_conv_refresh. */
 int mie_upconv2x_refresh(const void* a, const void* b, int c, int h_in, int w_in,
                          const void* filter_up, int cout, const float* bias,

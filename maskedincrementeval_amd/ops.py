@@ -950,8 +950,9 @@ def _upconv2x_args(a, b, filt, out_ts, out, reservoir, addend):
     _ready(out_ts)
     code = _lib.DTYPE_BF16 if a.dtype == torch.bfloat16 else f32_in_terms()
     # (the four phases' sums are short: in two fp16 terms layers of 64 and 96 channels would be 1.13 and 1.05 times as far from fp64 as in three
-    # bf16 terms, from 128 on .99 and less: 128->64 1.97 -> 1.73e-7 at 66x88, 256->128 2.77 -> 2.22e-7 at 33x44)
-    if code == _lib.DTYPE_F32_F16X2 and c < 128:
+    # bf16 terms, from 128 on .99 and less: 128->64 1.97 -> 1.73e-7 at 66x88, 256->128 2.77 -> 2.22e-7 at 33x44; large planes of few channels have
+    # a form of their own, .94)
+    if code == _lib.DTYPE_F32_F16X2 and not lib().mie_f16x2_takes_upconv2x(n, h, w, c, cout):
         code = _lib.DTYPE_F32_BF16X3
     up = replay.keep(filt._up2x_of(code))
     return n, c, h, w, cout, up.data_ptr(), code

@@ -386,6 +386,14 @@ def test_workspace_queries_name_layers_of_the_matrix_cores_only(mie_lib):
     assert u(32, 32, 4, x3) == 1 and u(48, 32, 4, x3) == 0 and u(32, 48, 4, x3) == 0 and u(64, 32, 0, x3) == 0 and u(0, 32, 4, bf) == 0
 
 
+def test_decoders_in_two_terms_are_those_nearer_to_fp64(mie_lib):
+    """mie_f16x2_takes_upconv2x: from 128 channels on, of 64 and 96 where k_upconv2x would make more than 512 workgroups of 32 columns."""
+    q = mie_lib.mie_f16x2_takes_upconv2x
+    assert q(1, 8, 8, 128, 32) == 1 and q(1, 132, 176, 64, 32) == 1 and q(1, 64, 64, 64, 32) == 0 and q(1, 64, 64, 64, 64) == 1
+    assert q(1, 80, 82, 64, 32) == 0 and q(2, 80, 82, 64, 32) == 1          # 4 * (11 * 10 + 6 + 6) = 472 each
+    assert q(1, 2, 4000, 64, 32) == 0 and q(1, 1, 40, 128, 32) == 0 and q(1, 64, 64, 48, 32) == 0 and q(1, 132, 176, 32, 32) == 0 and q(1, 64, 64, 128, 48) == 0 and q(0, 64, 64, 128, 32) == 0
+
+
 def test_workspace_queries_draw_the_line_where_the_split_form_is_faster(mie_lib):
     """One launch up to so many input channels, by kind of layer, type and rows a workgroup (2, 4, 8: slabs of 16 columns x tiles)."""
     bf, x3 = _lib.DTYPE_BF16, _lib.DTYPE_F32_BF16X3

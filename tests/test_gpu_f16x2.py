@@ -156,9 +156,11 @@ def _up2x(a, b, wt, mode, out=None):
     return out.cpu().double()
 
 
-# decoders at the resolution of their inputs: 32 columns a workgroup (up to 256 of them) and 64; blocks in part, strips and corners
+# decoders at the resolution of their inputs: 32 columns a workgroup (up to 256 of them) and 64; blocks in part, strips and corners; 64 and 96
+# channels on many blocks: all phases in a workgroup
 @pytest.mark.parametrize("c,cout,h,w,two", [(128, 64, 32, 32, True), (128, 64, 66, 88, True), (256, 128, 33, 44, True), (256, 64, 9, 11, False),
-                                            (160, 32, 21, 37, True), (128, 96, 2, 40, True), (128, 32, 10, 3, False)])
+                                            (160, 32, 21, 37, True), (128, 96, 2, 40, True), (128, 32, 10, 3, False),
+                                            (64, 32, 72, 123, True), (96, 64, 63, 66, False)])
 @pytest.mark.parametrize("what", ["fits", "below", "above", "not finite", "filter"])
 def test_decoders_at_the_resolution_of_their_inputs(c, cout, h, w, two, what, setting):
     g = torch.Generator().manual_seed(c + h)

@@ -247,3 +247,14 @@ def test_pixels_outside_the_mask_keep_their_reservoir(n, c, cout, h, w, dtype, f
         if res is not None:
             bits = lambda t: t.contiguous().view(torch.int32)
             assert torch.equal(bits(res.cpu())[off], bits(r0)[off])
+
+
+# fp32, 64 or 96 channels, more workgroups than two to a CU: the four phases in one workgroup.  Blocks and strips
+# cut off at both sides, one row of blocks, planes of strips only (which stay with the other form), slabs, samples.
+@pytest.mark.parametrize("n,c,cout,h,w", [(1, 64, 32, 100, 140), (2, 96, 64, 40, 41), (1, 64, 32, 3, 1200), (1, 64, 32, 1200, 3),
+                                          (1, 64, 32, 2, 2200), (9, 64, 96, 17, 10)])
+def test_decoder_conv_of_few_channels_on_many_blocks(n, c, cout, h, w):
+    assert _lib.lib().mie_f16x2_takes_upconv2x(n, h, w, c, cout) == (h > 2)
+    test_decoder_conv_at_input_resolution(n, c, cout, h, w, torch.float32)
+    if n == 1 and h > 2 and c == 64:
+        test_pixels_outside_the_mask_keep_their_reservoir(n, c, cout, h, w, torch.float32, "blocks")
