@@ -19,8 +19,9 @@
 //   * fp32 deltas as three bf16 terms (split3), the products by size in three accumulators, so that the large ones are added up
 //     among themselves: chains of 9 sums a chunk.  Error of the sums against fp64, relative 2-norm, split form -> this:
 //     256->256 1.20e-7 -> 1.07e-7, 512->512 1.90e-7 -> 1.44e-7, 64->64 1.4e-7 -> 0.8e-7.  bf16: three accumulators in turn.
-//     (For MIE_DTYPE_F32_F16X2 too: with two fp16 terms these would be 1.42e-7, 1.77e-7 and 1.15e-7, whose 23 bits a value show where so
-//     little else is rounded.)
+//     (For MIE_DTYPE_F32_F16X2 too, but for the 3x3 convs of many channels: DEEP_F2_FROM.)
+//   * In two fp16 terms (F2) the scale is a pass's, a wave's own with OWN: every DEEP_BL taps the leading products are folded into the total at
+//     its true size, with what that rounds off carried on among the small ones (deep_fold), and chunks of any size add up.
 //   * Up-sampling: the sums of the source pixels in LDS, the window blended from them, as in k_conv_mfma.  fp32 layers of 256 channels are
 //     not taken: 25 taps of filter, 614 KB a workgroup, take as long as the split form (256->128 at 16x24 16.4 us, 14.6).
 // Measured back to back on one plane with all pixels active, the filter another each time, split form -> this, us:
@@ -58,14 +59,38 @@ __device__ __forceinline__ float4 global_ld4(GlobalBytes p) {
   return make_float4(v[0], v[1], v[2], v[3]);
 }
 
+constexpr int DEEP_BL = 3;
 constexpr int DEEP_WAVES = 8, DEEP_COLS = 16, DEEP_THREADS = 64 * DEEP_WAVES, DEEP_WGS = 256;
 enum { DEEP_PLAIN = 0, DEEP_GATES = 1, DEEP_UP = 2, DEEP_GRU = 3 };
 
-// Sizes of a form; NCW: chunks of 32 channels in LDS at a time, ROWS: output rows of a tile.
-template <typename T, int K, int S, int NCW, int ROWS, int KIND>
+__device__ __forceinline__ void mma16_f16(v4acc& acc, const float4& w, const float4& x) {
+  const v4f w4 = {w.x, w.y, w.z, w.w}, x4 = {x.x, x.y, x.z, x.w};
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mie_f16x8, w4), __builtin_bit_cast(mie_f16x8, x4), acc, 0, 0, 0);
+}
+// Four of a lane's eight channels on the fp32 instruction, from fp32 copies laid out as the terms are (the first four in plane 0).
+__device__ __forceinline__ void mma16_f32(v4acc& acc, const float4& w, const float4& x) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, x.x, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, x.y, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.z, x.z, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w.w, x.w, acc, 0, 0, 0);
+}
+// Two terms: the products so far (acc, at the scales that c0 takes off) to the total, what the addition rounds off to the small ones.
+__device__ __forceinline__ void deep_fold(v4acc& tot, v4acc& low, v4acc& acc, float c0) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float t = tot[r], u = fmaf(acc[r], c0, t);
+    low[r] += fmaf(acc[r], c0, t - u);
+    tot[r] = u;
+    acc[r] = 0.f;
+  }
+}
+
+// Sizes of a form; NCW: chunks of 32 channels in LDS at a time, ROWS: output rows of a tile, AR: 0 bf16, 1 fp32 in three bf16 terms, 2 in
+// two fp16 terms.
+template <int AR, int K, int S, int NCW, int ROWS, int KIND>
 struct Deep {
-  static constexpr bool X3 = sizeof(T) == 4;
-  static constexpr int PL = X3 ? 3 : 1, GPS = X3 ? 2 : 1;      // term planes; 16-byte loads of 8 channels
+  static constexpr bool X3 = AR != 0;
+  static constexpr int PL = AR == 2 ? 2 : X3 ? 3 : 1, GPS = X3 ? 2 : 1;      // term planes; 16-byte loads of 8 channels
   static constexpr int CC = 32, EPS = 8, LS = CC + EPS;        // LDS elements per staged pixel of a chunk
   static constexpr int TPC = DEEP_WAVES / NCW, NT = (K * K + TPC - 1) / TPC;
   static constexpr int WX = 7 * S + K, WY = (ROWS - 1) * S + K, NPIX = WX * WY;
@@ -84,17 +109,20 @@ struct Deep {
   static constexpr int BYTES = WIN_B + LO_B > PARK_B ? WIN_B + LO_B : PARK_B;
 };
 
-template <typename T, int K, int S, int NCW, int ROWS, int KIND>
+template <typename T, int AR, int K, int S, int NCW, int ROWS, int KIND>
 __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
-  typedef Deep<T, K, S, NCW, ROWS, KIND> D;
-  constexpr bool X3 = D::X3, UP = D::UP, GATES = KIND == DEEP_GATES, GRU = KIND == DEEP_GRU, AGAIN = X3 && S == 2;
+  typedef Deep<AR, K, S, NCW, ROWS, KIND> D;
+  static_assert((AR != 0) == (sizeof(T) == 4), "fp32 deltas in terms, bf16 as they are");
+  constexpr bool X3 = D::X3, F2 = AR == 2, UP = D::UP, GATES = KIND == DEEP_GATES, GRU = KIND == DEEP_GRU, AGAIN = AR == 1 && S == 2;
   constexpr int PL = D::PL, GPS = D::GPS, CC = D::CC, EPS = D::EPS, LS = D::LS, TPC = D::TPC, NT = D::NT;
   constexpr int WX = D::WX, NPIX = D::NPIX, RP = D::RP, STAGE = D::STAGE, SPP = D::SPP, STEP = D::STEP, NLD = D::NLD;
   constexpr bool OWN = D::OWN;
   constexpr int MB = D::MB, OS = D::OS, NLO = D::NLO, LOS = D::LOS;
   static_assert(D::BYTES <= 160 * 1024, "LDS of a CU");
   static_assert(!UP || (K == 5 && S == 1), "the up-sampling variant is the 5x5 stride-1 conv");
+  static_assert(!F2 || (K == 3 && S == 1 && !UP), "two terms: the 3x3 convs");
   __shared__ __attribute__((aligned(16))) char smem[D::BYTES];
+  __shared__ float s_f2[F2 && !OWN ? DEEP_WAVES + 1 : 1];      // largest values of the waves' slots; whether a group does not fit
   mie_bf16* const win = reinterpret_cast<mie_bf16*>(smem);
   float* const s_lo = reinterpret_cast<float*>(smem + D::WIN_B);
   float* const park = reinterpret_cast<float*>(smem);
@@ -214,8 +242,15 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
     }
   };
   auto kept = [](const float4& v, bool k) { return make_float4(k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f); };
-  auto put = [&](int at, const float (&f)[8]) {
-    if constexpr (X3) {
+  F2Groups groups;
+  bool misfit = false;
+  auto put = [&](int at, const float (&f)[8], auto terms) {
+    if constexpr (F2) {
+      float4 pl[2] = {make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7])};
+      if constexpr (decltype(terms)::value) groups.terms(f, pl);
+#pragma unroll
+      for (int q = 0; q < PL; ++q) *reinterpret_cast<float4*>(win + q * STAGE + at) = pl[q];
+    } else if constexpr (X3) {
       float4 pl[3];
       split3(f, pl);
 #pragma unroll
@@ -226,7 +261,18 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   };
   unsigned ok1 = 0u, ok2 = 0u;
   const int st_c = ck * (PL * STAGE) + q8;      // this thread's place in a staged pixel
-  auto store_x = [&](int pass) {
+  // F2: the scale of a pass, a wave's own (OWN) or the workgroup's
+  auto scale_of = [&](float m) {
+    m = f2_wave_max(m);
+    if constexpr (!OWN) {
+      if (lane == 0) s_f2[wave] = m;
+      __syncthreads();
+      m = f2_wave_max(s_f2[lane & (DEEP_WAVES - 1)]);
+    }
+    groups.start(f2_scale(m));
+  };
+  // (terms: in terms, or F2's fp32 form)
+  auto store_x = [&](int pass, auto terms) {
     const int c = pass * NCW + ck;
     if constexpr (UP) {
 #pragma unroll
@@ -275,10 +321,20 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
             o[e + 3] = conv_up2x_v(lr0, lr1, conv_up2x_h(lq0, lq1, t00.w, t01.w), conv_up2x_h(lq0, lq1, t10.w, t11.w));
           }
         }
-        put(st_c + ly * RP + lx * LS, o);
+        put(st_c + ly * RP + lx * LS, o, terms);
       }
     } else {
       const unsigned ok = c >= nch ? 0u : c >= nch1 ? ok2 : ok1;
+      if constexpr (F2 && decltype(terms)::value) {
+        float m = 0.f;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+          const float4 u = xr[i][0], v = xr[i][GPS - 1];
+          const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+          m = __builtin_elementwise_maximum(m, (ok >> i) & 1u ? f2_amax8(f) : 0.f);
+        }
+        scale_of(m);
+      }
 #pragma unroll
       for (int i = 0; i < NL; ++i) {
         const int pix = p0 + STEP * i, ly = pix / WX, lx = pix - ly * WX;
@@ -288,7 +344,7 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
         if constexpr (X3) {
           const float4 v = kept(xr[i][GPS - 1], k);
           const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-          put(st_c + ly * RP + lx * LS, f);
+          put(st_c + ly * RP + lx * LS, f, terms);
         } else {
           *reinterpret_cast<float4*>(win + st_c + ly * RP + lx * LS) = u;
         }
@@ -328,7 +384,18 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   }
 
   // ---- contraction
-  v4acc acc[MB], sm[MB], sl[MB];      // fp32: products of 1, 2^-8 and 2^-16 of the largest
+  v4acc acc[MB], sm[MB], sl[MB];      // fp32: products of 1, 2^-8 and 2^-16 of the largest; F2: of 1 and 2^-11, and the totals' small part
+  v4acc tot[F2 ? MB : 1];
+  float c0 = 1.f, filt_unscale = 1.f;
+  bool filt_fits = true;
+  const long long weights = (long long)a.cin_total * (K * K) * cout;
+  if constexpr (F2) {
+    const float* const end = f2_filter_end(a.filt_mc, weights);
+    filt_unscale = end[0];
+    filt_fits = end[1] != 0.f;
+#pragma unroll
+    for (int b = 0; b < MB; ++b) tot[b] = v4acc{0.f, 0.f, 0.f, 0.f};
+  }
 #pragma unroll
   for (int b = 0; b < MB; ++b) acc[b] = v4acc{0.f, 0.f, 0.f, 0.f}, sm[b] = sl[b] = v4acc{0.f, 0.f, 0.f, 0.f};
   const mie_bf16* const x_lane = win + cg * (PL * STAGE) + (l16 >> 3) * S * RP + (l16 & 7) * S * LS + EPS * kg;
@@ -344,7 +411,18 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
         for (int b = 0; b < MB; ++b)
 #pragma unroll
           for (int q = 0; q < PL; ++q) xv[b][q] = *reinterpret_cast<const float4*>(x_lane + q * STAGE + (2 * S * b + ky) * RP + kx * LS);
-        if constexpr (X3) {
+        if constexpr (F2) {
+#pragma unroll
+          for (int b = 0; b < MB; ++b) mma16_f16(acc[b], w[i][0], xv[b][0]);
+#pragma unroll
+          for (int b = 0; b < MB; ++b) mma16_f16(sm[b], w[i][0], xv[b][1]);
+#pragma unroll
+          for (int b = 0; b < MB; ++b) mma16_f16(sm[b], w[i][1], xv[b][0]);
+          if (i % DEEP_BL == DEEP_BL - 1 || i == NT - 1) {
+#pragma unroll
+            for (int b = 0; b < MB; ++b) deep_fold(tot[b], sl[b], acc[b], c0);
+          }
+        } else if constexpr (X3) {
           auto term = [&](v4acc (&s)[MB], int tw, int tx) {
 #pragma unroll
             for (int b = 0; b < MB; ++b) mma16(s[b], w[i][tw], xv[b][tx]);
@@ -358,10 +436,23 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
       }
       if constexpr (MORE) load_w(next, i, std::false_type());
     }
+    if constexpr (F2) {      // (the rest of a wave whose last tap is none; the small products at this chunk's scale)
+      const float c1 = c0 * (1.f / F2_STEP);
+#pragma unroll
+      for (int b = 0; b < MB; ++b) {
+        if (TPC > 1) deep_fold(tot[b], sl[b], acc[b], c0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sl[b][r] = fmaf(sm[b][r], c1, sl[b][r]), sm[b][r] = 0.f;
+      }
+    }
   };
   for (int pass = 0, c = cg; pass * NCW < nch; ++pass, c += NCW) {
     if (!OWN && pass > 0) __syncthreads();
-    store_x(pass);
+    store_x(pass, std::true_type());
+    if constexpr (F2) {
+      misfit = misfit || groups.misfit();
+      c0 = f2_unscale(groups.scale) * filt_unscale;
+    }
     if constexpr (OWN) mie_wave_order();
     else __syncthreads();
     if ((pass + 1) * NCW < nch) load_x(pass + 1);
@@ -369,12 +460,49 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
     else if (c < nch) chunk(nullptr, std::false_type());
     if constexpr (OWN) mie_wave_order();
   }
+  if constexpr (F2) {
+    // a group that does not fit: all the sums of the wave (OWN) or the workgroup once more, on the fp32 instruction from the fp32 copy of the
+    // filter behind the terms
+    bool again = __ballot(misfit || !filt_fits) != 0ull;
+    if constexpr (!OWN) {
+      if (tid == 0) s_f2[DEEP_WAVES] = 0.f;
+      __syncthreads();
+      if (again && lane == 0) s_f2[DEEP_WAVES] = 1.f;
+      __syncthreads();
+      again = __builtin_amdgcn_readfirstlane(__float_as_int(s_f2[DEEP_WAVES])) != 0;
+    }
+    if (__builtin_expect(again, 0)) {
+#pragma unroll
+      for (int b = 0; b < MB; ++b) tot[b] = sl[b] = v4acc{0.f, 0.f, 0.f, 0.f};
+      for (int pass = 0, c = cg; pass * NCW < nch; ++pass, c += NCW) {
+        if constexpr (!OWN) __syncthreads();
+        load_x(pass);
+        store_x(pass, std::false_type());
+        if constexpr (OWN) mie_wave_order();
+        else __syncthreads();
+        if (c < nch) {
+          const char* const wp = chunk_w(c) + 4 * weights + w_lane;
+#pragma unroll 1
+          for (int tap = tc; tap < K * K; tap += TPC) {
+            const int ky = tap / K, kx = tap - ky * K;
+#pragma unroll
+            for (int q = 0; q < PL; ++q) {
+              const float4 wv = *reinterpret_cast<const float4*>(wp + ((tap - tc) * PL + q) * w_step);
+#pragma unroll
+              for (int b = 0; b < MB; ++b) mma16_f32(tot[b], wv, *reinterpret_cast<const float4*>(x_lane + q * STAGE + (2 * S * b + ky) * RP + kx * LS));
+            }
+          }
+        }
+        if constexpr (OWN) mie_wave_order();
+      }
+    }
+  }
   if constexpr (!OWN) __syncthreads();
 
   // ---- the waves' sums meet in LDS: pixel 16 * b + l16, channels 4 * kg ...
 #pragma unroll
   for (int b = 0; b < MB; ++b) {
-    const v4acc s = acc[b] + (sm[b] + sl[b]);
+    const v4acc s = F2 ? tot[b < (F2 ? MB : 1) ? b : 0] + sl[b] : acc[b] + (sm[b] + sl[b]);
     *reinterpret_cast<float4*>(park + wave * D::PARK + (16 * b + l16) * OS + 4 * kg) = make_float4(s[0], s[1], s[2], s[3]);
   }
   __syncthreads();
@@ -425,9 +553,23 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   }
 }
 
+// Two terms for MIE_DTYPE_F32_F16X2: 3x3 convs of this many input channels and more.  Their error hardly grows with the channels (1.14 .. 1.19e-7
+// of the output against fp64; a third as many sums between folds would make it 1.05 .. 1.09e-7, and a chunk 7 % longer), that of three
+// terms does: 256 channels 1.07e-7, 512 1.43e-7.  us: 512->512 at 16x16 12.8 -> 11.1, at 8x8 9.0 -> 8.3, gates of 256+256 at 16x16 22.3 -> 19.7, of a
+// ConvGRU of 512 there 22.6 -> 20.3.  (Below: 256->256 at 8x12 6.7 and 6.1, 64->64 at 32x32 4.0 and 4.4; stride 2 of 128 channels at
+// 16x24 8.2 and 9.4, whose waves share their pixels and meet once more over the scale.)
+constexpr int DEEP_F2_FROM = 512;
+
 template <typename T, int K, int S, int NCW, int ROWS, int KIND>
 void launch_form(const ConvArgsT<T>& a, unsigned cap, hipStream_t st) {
-  hipLaunchKernelGGL((k_conv_deep<T, K, S, NCW, ROWS, KIND>), dim3(a.cout / DEEP_COLS, 8 / ROWS * cap), dim3(DEEP_THREADS), 0, st, a);
+  const dim3 grid(a.cout / DEEP_COLS, 8 / ROWS * cap);
+  if constexpr (sizeof(T) == 4 && K == 3 && S == 1 && KIND != DEEP_UP) {
+    if (a.x3 == 2 && a.c1 + a.c2 >= DEEP_F2_FROM) {
+      hipLaunchKernelGGL((k_conv_deep<T, 2, K, S, NCW, ROWS, KIND>), grid, dim3(DEEP_THREADS), 0, st, f2_args(a, K));
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_conv_deep<T, sizeof(T) == 4 ? 1 : 0, K, S, NCW, ROWS, KIND>), grid, dim3(DEEP_THREADS), 0, st, a);
 }
 
 // Chunks in LDS at a time.

@@ -68,10 +68,12 @@ def _conv(x, wt, k, stride, mode, c1=None, xm=None, path=_lib.PATH_MFMA, workspa
     return out.cpu().double()
 
 
-# planes of more than 256 slabs of 16 columns, or more channels than the one-launch form: k_conv_mfma, whole and (the last three with a workspace) split
+# planes of more than 256 slabs of 16 columns, or more channels than the one-launch form: k_conv_mfma, whole and (the three with a workspace) split
 SHAPES = [(32, 32, 3, 1, 136, 130, None), (64, 64, 3, 1, 70, 75, None), (128, 128, 3, 1, 41, 47, 64), (256, 256, 3, 1, 33, 44, None),
           (256, 512, 3, 1, 34, 39, 128), (64, 32, 5, 1, 33, 47, None), (128, 128, 5, 1, 34, 42, None), (32, 64, 5, 2, 131, 133, None),
-          (128, 256, 5, 2, 66, 88, None), (1024, 256, 3, 1, 17, 9, None), (256, 32, 5, 1, 16, 16, None), (512, 64, 5, 2, 17, 16, 256)]
+          (128, 256, 5, 2, 66, 88, None), (1024, 256, 3, 1, 17, 9, None), (256, 32, 5, 1, 16, 16, None), (512, 64, 5, 2, 17, 16, 256),
+          # the one-launch form from 512 channels on: two, four and eight rows a workgroup, waves of two and three chunks
+          (512, 64, 3, 1, 7, 9, None), (512, 64, 3, 1, 16, 24, 192), (576, 128, 3, 1, 24, 20, None), (512, 128, 3, 1, 31, 33, 256)]
 
 
 @pytest.mark.parametrize("cin,cout,k,stride,h,w,c1", SHAPES)
