@@ -942,6 +942,9 @@ int mie_upconv2x_masked(const void* a, const uint8_t* amask, const void* b,
 /* 1 where MIE_DTYPE_F32_F16X2 is the form of it for fp32 deltas that is nearer to fp64 and faster, 0 where MIE_DTYPE_F32_BF16X3 is (less than
  * 128 channels on small planes, 32 channels), or there is neither.  Host logic. */
 int mie_f16x2_takes_upconv2x(int n, int h_in, int w_in, int c, int cout);
+/* 1 where it has the four phases of a block in one workgroup (MIE_DTYPE_F32_F16X2, 64 and 96 channels; MIE_DTYPE_BF16, 64 channels; planes
+ * of many blocks).  Host logic. */
+int mie_all_phases_upconv2x(int n, int h_in, int w_in, int c, int cout, int dtype);
 
 /* Its dense twin (every tile of `out` active): bias, activation and reservoir fill as in mie_conv_refresh. */
 int mie_upconv2x_refresh(const void* a, const void* b, int c, int h_in, int w_in,

@@ -40,7 +40,7 @@ EXPORTS = (
     "mie_convlstm_gates_refresh", "mie_convgru_gates_refresh", "mie_mul_dense", "mie_tconv2x_masked",
     "mie_tconv2x_refresh", "mie_conv_f32x3_takes", "mie_conv_needs_no_workspace", "mie_conv_gates_needs_no_workspace", "mie_upconv_needs_no_workspace", "mie_conv_gru_masked", "mie_tconv2x_lead_masked",
     "mie_build_mask_plan", "mie_build_mask_plan_wgs",
-    "mie_upconv2x_masked", "mie_upconv2x_refresh", "mie_f16x2_takes_upconv2x", "mie_pack_filter_up2x", "mie_call_index", "mie_call_signature", "mie_run_calls",
+    "mie_upconv2x_masked", "mie_upconv2x_refresh", "mie_f16x2_takes_upconv2x", "mie_all_phases_upconv2x", "mie_pack_filter_up2x", "mie_call_index", "mie_call_signature", "mie_run_calls",
 )
 PLAN_MAX_STEPS = 40
 
@@ -198,6 +198,8 @@ def _declare(l):
     l.mie_upconv2x_refresh.argtypes = [vp, vp, ci, ci, ci, vp, ci, vp, tsp, vp, vp, ci, cf, ci, vp]
     l.mie_f16x2_takes_upconv2x.restype = ci
     l.mie_f16x2_takes_upconv2x.argtypes = [ci, ci, ci, ci, ci]
+    l.mie_all_phases_upconv2x.restype = ci
+    l.mie_all_phases_upconv2x.argtypes = [ci, ci, ci, ci, ci, ci]
     l.mie_pack_filter_up2x.restype = ci
     l.mie_pack_filter_up2x.argtypes = [vp, ci, ci, vp, ci, vp]
     l.mie_tconv_refresh.restype = ci

@@ -684,13 +684,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   }
 }
 
-// The same for fp32 deltas in two fp16 terms with all four phases of a block (or strip) in one workgroup, a phase to a wave x 32 output
-// channels: the window (12x12 pixels, 3 rows of 36) is loaded, added up and split once instead of four times, and the waves' sums do not
+// The same with all four phases of a block (or strip) in one workgroup, a phase to a wave x 32 output channels, for fp32 deltas in two fp16
+// terms and for bf16 ones of 64 channels (one chunk: nothing but the loop over its 64 units): the window (12x12 pixels, 3 rows of 36) is loaded, added up and split once instead of four times, and the waves' sums do not
 // have to meet in LDS -- what layers of few channels spend their time on, whose workgroups in k_upconv2x are two or three chunks long
 // between a prologue and an exchange (64->32 at 132x176, all tiles active: 1580 workgroups there, 50 us, of which the matrix cores have
 // work for 19; here 396).
 //
-// Sums.  With all of K in one wave the chain of roundings at the size of the sum would be four times as long, and the fp16 leading terms
+// fp32 sums.  With all of K in one wave the chain of roundings at the size of the sum would be four times as long, and the fp16 leading terms
 // fill the accumulator's 24 bits where bf16 ones do not (in one chain 64 channels are 1.41e-7 from fp64, relative 2-norm, k_upconv2x in
 // three terms 1.10e-7).  So every BL = 4 units start from zero, and are added to the total, under the MFMAs of the next four (two sets of
 // accumulators), with what the addition rounds off carried on in the accumulator of the small products: 1.04e-7 at any number of
@@ -699,21 +699,26 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
 //
 // The next chunk is staged a slot at a time, its loads ten units ahead of its LDS writes (16 registers instead of 48).  What is left
 // above the matrix cores' time (22 us with LDS, filter and input reads taken out): the loads of the next chunk (5), its split (3), A (3).
-__global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2xOrder od) {
+template <typename T>
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(ConvArgsT<T> a, Up2xOrder od) {
+  constexpr bool F2 = sizeof(T) == 4;
   typedef mie_bf16 TL;
-  constexpr int EPS = 8, SUB = 16, IT = 12, CC = 32, LS = CC + EPS, Q4 = CC / EPS;
+  constexpr int PL = F2 ? 2 : 1, GPS = F2 ? 2 : 1;           // operand planes, 16-byte loads of a slot
+  constexpr int NBUF = F2 ? 2 : 1;                           // (bf16: one chunk)
+  constexpr int EPS = 8, SUB = 16, IT = 12, CC = F2 ? 32 : 64, LS = CC + EPS, Q4 = CC / EPS;
   constexpr int NLD = (IT * IT * Q4 + 255) / 256;
   constexpr int RP = row_pitch_dw(IT, LS / 2, 1) * 2;
   constexpr int ZOFF = IT * RP, STAGE = ZOFF + LS;           // the zero pixel behind the tile
   constexpr int SPX = STRIP + 4, RPS = SPX * LS;
   static_assert(3 * SPX <= IT * IT && 3 * RPS <= ZOFF, "a strip stages less than a block");
-  constexpr int NQ = CC / SUB, UPC = 16 * NQ, PD = 3, BL = 4;  // (ring of four units of the filter)
+  constexpr int NQ = CC / SUB, UPC = 16 * NQ, BL = 4;
+  constexpr int RING = F2 ? 4 : 8, PD = RING - 1, AHEAD = F2 ? 2 : 4;      // units of the filter and of LDS in registers
   static_assert(UPC % (2 * BL) == 0, "a chunk ends with a block of the odd accumulators");
   constexpr int CO_BLK = 32, RED = 4 * 64 * CO_BLK;
-  constexpr int STAGE_F = 2 * 2 * STAGE / 2, SMEM = STAGE_F > RED ? STAGE_F : RED;
+  constexpr int STAGE_F = NBUF * PL * STAGE / 2, SMEM = STAGE_F > RED ? STAGE_F : RED;
   static_assert(SMEM * 4 <= 65536, "LDS budget");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
-  __shared__ float s_f2[5];                                  // largest values of the waves' first slots; whether a group does not fit
+  __shared__ float s_f2[F2 ? 5 : 1];                                  // largest values of the waves' first slots; whether a group does not fit
   TL* const sbuf = reinterpret_cast<TL*>(smem);
 
   // the strips first, dealt out to the XCDs one by one: they are the longest of the workgroups; then the blocks as in k_upconv2x
@@ -822,7 +827,7 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
     iy = iy < 0 ? 0 : (iy >= H ? H - 1 : iy);
     ix = ix < 0 ? 0 : (ix >= W ? W - 1 : ix);
     const int po = (n * H + iy) * W + ix;
-    st_off[i] = ((unsigned)po * (unsigned)a.c1 + (unsigned)(EPS * q4)) * 4u;
+    st_off[i] = ((unsigned)po * (unsigned)a.c1 + (unsigned)(EPS * q4)) * (unsigned)sizeof(T);
     st_po[i] = po;
   }
   const uint8_t* const x2m = has2 ? a.x2m : nullptr;
@@ -831,30 +836,43 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
   mie_mask_ask(x2m, a.filt_mc, st_po, b2);
   const int nch = a.c1 / CC;
 
-  float4 ra[2], rb[2];
-  const float* x2p = has2 ? a.x2 : a.x;
+  float4 ra[GPS], rb[GPS];
+  const T* x2p = has2 ? a.x2 : a.x;
   auto load = [&](int i, int c) __attribute__((always_inline)) {
     const char* xc = reinterpret_cast<const char*>(a.x + c * CC);
     const char* x2c = reinterpret_cast<const char*>(x2p + c * CC);
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
+    for (int g = 0; g < GPS; ++g) {
       ra[g] = *reinterpret_cast<const float4*>(xc + st_off[i] + 16 * g);
       rb[g] = *reinterpret_cast<const float4*>(x2c + st_off[i] + 16 * g);
     }
   };
   F2Groups groups;
-  auto sum = [&](int i, const float4 (&u)[2], const float4 (&w)[2], float (&f)[8]) __attribute__((always_inline)) {
+  auto sum = [&](int i, const float4 (&u)[GPS], const float4 (&w)[GPS], float (&f)[8]) __attribute__((always_inline)) {
     const bool k1 = (ok1 >> i) & 1u, k2 = (ok2 >> i) & 1u;
-    const float ta[8] = {u[0].x, u[0].y, u[0].z, u[0].w, u[1].x, u[1].y, u[1].z, u[1].w};
-    const float tb[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
+    if constexpr (F2) {
+      const float ta[8] = {u[0].x, u[0].y, u[0].z, u[0].w, u[1].x, u[1].y, u[1].z, u[1].w};
+      const float tb[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = (k1 ? ta[e] : 0.f) + (k2 ? tb[e] : 0.f);
+      for (int e = 0; e < 8; ++e) f[e] = (k1 ? ta[e] : 0.f) + (k2 ? tb[e] : 0.f);
+    } else {
+      const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+      float fa[8], fb[8];
+      slot_to_f32(k1 ? u[0] : z4, fa, T());
+      slot_to_f32(k2 ? w[0] : z4, fb, T());
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = fa[e] + fb[e];
+    }
   };
   auto put = [&](int i, const float (&f)[8], TL* dst, auto terms) __attribute__((always_inline)) {
-    float4 pl[2] = {make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7])};
-    if constexpr (decltype(terms)::value) groups.terms(f, pl);
+    if constexpr (F2) {
+      float4 pl[2] = {make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7])};
+      if constexpr (decltype(terms)::value) groups.terms(f, pl);
 #pragma unroll
-    for (int q = 0; q < 2; ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
+      for (int q = 0; q < PL; ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
+    } else {
+      *reinterpret_cast<float4*>(dst + st_lds[i]) = f32_to_slot(f, T());
+    }
   };
   auto store = [&](int i, TL* dst, auto terms) __attribute__((always_inline)) {
     float f[8];
@@ -889,7 +907,7 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
   }
   const bool at_first = l32 == 0, at_last = l32 == cols - 1;
   const int b_lane = (half * cout + l32) * EPS;
-  const int unit_sz = 2 * 2 * cout * EPS;
+  const int unit_sz = PL * 2 * cout * EPS;
   const TL* const filt = reinterpret_cast<const TL*>(a.filt_mc) + co0 * EPS;
   auto group_b = [&](int c, int qi, int unit) -> const TL* {
     return filt + ((long long)(phase * od.nci + c * NQ + qi) * UNITS + unit) * unit_sz;
@@ -897,39 +915,43 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
   auto strip_unit = [&](int g) { return u_side + 4 * (int)((strip >> (4 * g)) & 15u); };
   const TL* bp;
   auto seek_b = [&](const TL* gb) { bp = gb + b_lane; };
-  auto load_b = [&](float4 (&bv)[2]) __attribute__((always_inline)) {
+  auto load_b = [&](float4 (&bv)[PL]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < PL; ++q) {
       bv[q] = *reinterpret_cast<const float4*>(bp);
       bp += 2 * cout * EPS;
     }
   };
   auto first_b = [&](int c) { return group_b(c, 0, side == 0 ? 0 : strip_unit(0)); };
 
-  v16f zero, tot[2], acc[2], sm[2];
+  v16f zero, acc[2], tot[F2 ? 2 : 1], odd[F2 ? 2 : 1], sm[F2 ? 2 : 1];
 #pragma unroll
   for (int r = 0; r < 16; ++r) zero[r] = 0.f;
 #pragma unroll
-  for (int mb = 0; mb < 2; ++mb) tot[mb] = zero, acc[mb] = zero, sm[mb] = zero;
+  for (int mb = 0; mb < 2; ++mb) {
+    acc[mb] = zero;
+    if constexpr (F2) tot[mb] = zero, odd[mb] = zero, sm[mb] = zero;
+  }
   const long long weights = 4LL * UNITS * a.c1 * cout;
-  const float* const end = f2_filter_end(a.filt_mc, weights);
-  const float filt_unscale = end[0];
-  const bool filt_fits = end[1] != 0.f;
-
-  v16f odd[2];
-  odd[0] = zero; odd[1] = zero;
-  auto flush = [&](const v16f (&from)[2], int mb, int r) __attribute__((always_inline)) {
+  float filt_unscale = 1.f;
+  bool filt_fits = true;
+  if constexpr (F2) {
+    const float* const end = f2_filter_end(a.filt_mc, weights);
+    filt_unscale = end[0];
+    filt_fits = end[1] != 0.f;
+  }
+  auto flush = [&](const v16f (&from)[2], int mb, int r) __attribute__((always_inline)) {      // (F2)
     const float t = tot[mb][r], x = from[mb][r], u = t + x;
     sm[mb][r] = fmaf(x - (u - t), F2_STEP, sm[mb][r]);      // (exactly what is lost where |x| <= |t|)
     tot[mb][r] = u;
   };
-  float4 bring[4][2];
+  float4 bring[RING][PL];
   seek_b(first_b(0));
-  float4 fa[NLD][2], fb[NLD][2];
+  float4 fa[NLD][GPS], fb[NLD][GPS];
 #pragma unroll
   for (int i = 0; i < NLD; ++i)
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
+    for (int g = 0; g < GPS; ++g) {
       fa[i][g] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.x) + st_off[i] + 16 * g);
       fb[i][g] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(x2p) + st_off[i] + 16 * g);
     }
@@ -939,24 +961,26 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
   ok1 = mie_mask_take(a.xm, b1, ~0u);
   ok2 = mie_mask_take(x2m, b2, has2 ? ~0u : 0u);
   live_bits = mie_mask_take(live_m, live_b, in);
-  for (int i = tid; i < 2 * 2 * (LS / EPS); i += 256) {
+  for (int i = tid; i < NBUF * PL * (LS / EPS); i += 256) {
     const int pl = i / (LS / EPS);
     *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (i - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
   }
   const auto in_terms = std::true_type();
   {
-    float m = 0.f, f[NLD][8];
+    float f[NLD][8];
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      sum(i, fa[i], fb[i], f[i]);
-      m = __builtin_elementwise_maximum(m, f2_amax8(f[i]));
+    for (int i = 0; i < NLD; ++i) sum(i, fa[i], fb[i], f[i]);
+    if constexpr (F2) {
+      float m = 0.f;
+#pragma unroll
+      for (int i = 0; i < NLD; ++i) m = __builtin_elementwise_maximum(m, f2_amax8(f[i]));
+      m = f2_wave_max(m);
+      if (lane == 0) s_f2[phase] = m;
+      if (tid == 0) s_f2[4] = 0.f;
+      __syncthreads();
+      groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(
+          __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[1], s_f2[2]), s_f2[3]))))));
     }
-    m = f2_wave_max(m);
-    if (lane == 0) s_f2[phase] = m;
-    if (tid == 0) s_f2[4] = 0.f;
-    __syncthreads();
-    groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(
-        __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[1], s_f2[2]), s_f2[3]))))));
 #pragma unroll
     for (int i = 0; i < NLD; ++i) put(i, f[i], sbuf, in_terms);
   }
@@ -964,17 +988,18 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
 
   if (side == 0) {
     const TL* sin = sbuf;
-    TL* snext = sbuf + 2 * STAGE;
-    float4 av[2][2][2];
-    auto load_a = [&](const TL* s, int u, float4 (&dst)[2][2]) __attribute__((always_inline)) {
+    TL* snext = sbuf + (NBUF - 1) * PL * STAGE;
+    float4 av[AHEAD][2][PL];
+    auto load_a = [&](const TL* s, int u, float4 (&dst)[2][PL]) __attribute__((always_inline)) {
       const int qi = u / 16, k = u % 16;
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (int q = 0; q < PL; ++q)
           dst[mb][q] = *reinterpret_cast<const float4*>(&s[q * STAGE + a_lane[mb] + (k >> 2) * RP + (k & 3) * LS + SUB * qi]);
     };
-    load_a(sin, 0, av[0]);
+#pragma unroll
+    for (int i = 0; i < AHEAD - 1; ++i) load_a(sin, i, av[i]);
     for (int c = 0; c < nch; ++c) {
       const int cn = c + 1 < nch ? c + 1 : c;
 #pragma unroll
@@ -982,26 +1007,28 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
         const int ip = i + PD;
         if (ip == UPC) seek_b(first_b(cn));
         else if (ip % 16 == 0) seek_b(group_b(c, ip / 16, 0));
-        load_b(bring[ip & 3]);
-        if (i + 1 < UPC) load_a(sin, i + 1, av[(i + 1) & 1]);
+        load_b(bring[ip % RING]);
+        if (i + AHEAD - 1 < UPC) load_a(sin, i + AHEAD - 1, av[(i + AHEAD - 1) % AHEAD]);
         __builtin_amdgcn_sched_barrier(0);
-        const auto& A = av[i & 1];
-        const auto& B = bring[i & 3];
-        v16f (&now)[2] = (i / BL) % 2 ? odd : acc;
-        v16f (&was)[2] = (i / BL) % 2 ? acc : odd;
-        if (i % BL == 0) {
-          now[0] = zero; now[1] = zero;
-        }
-        mma_f16(now[0], A[0][0], B[0]); mma_f16(now[1], A[1][0], B[0]);
-        mma_f16(sm[0], A[0][1], B[0]);  mma_f16(sm[1], A[1][1], B[0]);
-        mma_f16(sm[0], A[0][0], B[1]);  mma_f16(sm[1], A[1][0], B[1]);
+        const auto& A = av[i % AHEAD];
+        const auto& B = bring[i % RING];
+        if constexpr (F2) {
+          v16f (&now)[2] = (i / BL) % 2 ? odd : acc;
+          v16f (&was)[2] = (i / BL) % 2 ? acc : odd;
+          if (i % BL == 0) now[0] = zero, now[1] = zero;
+          mma_f16(now[0], A[0][0], B[0]); mma_f16(now[1], A[1][0], B[0]);
+          mma_f16(sm[0], A[0][1], B[0]);  mma_f16(sm[1], A[1][1], B[0]);
+          mma_f16(sm[0], A[0][0], B[1]);  mma_f16(sm[1], A[1][0], B[1]);
 #pragma unroll
-        for (int e = (32 / BL) * (i % BL); e < (32 / BL) * (i % BL + 1); ++e) flush(was, e / 16, e % 16);
-        static_assert(NLD == 3, "the slots' places in the units");
-        if (i % 10 == 9) store(i / 10, snext, in_terms);
-        if (i % 10 == 0 && i < 30) load(i / 10, cn);
+          for (int e = (32 / BL) * (i % BL); e < (32 / BL) * (i % BL + 1); ++e) flush(was, e / 16, e % 16);
+          static_assert(!F2 || NLD == 3, "the slots' places in the units");
+          if (i % 10 == 9) store(i / 10, snext, in_terms);
+          if (i % 10 == 0 && i < 30) load(i / 10, cn);
+        } else {
+          mma_unit2(acc[0], acc[1], A[0][0], A[1][0], B[0], mie_bf16());
+        }
         __builtin_amdgcn_sched_barrier(0);
-        if (i == UPC - 2) {
+        if (F2 && i == UPC - 2) {
           __syncthreads();
           load_a(snext, 0, av[0]);
           __builtin_amdgcn_sched_barrier(0);
@@ -1011,9 +1038,14 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
       sin = snext;
       snext = t;
     }
+    if constexpr (F2) {
 #pragma unroll
-    for (int e = 0; e < 32; ++e) flush(odd, e / 16, e % 16);
+      for (int e = 0; e < 32; ++e) flush(odd, e / 16, e % 16);
+    } else {
+      __syncthreads();
+    }
   } else {
+    if constexpr (PD > 3) seek_b(first_b(0) + 3 * unit_sz);
     auto lane_of = [&](int g, int qi, int& base, int& step) {
       const int code = (int)((strip >> (4 * g)) & 15u);
       const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
@@ -1023,12 +1055,14 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
     for (int c = 0; c < nch; ++c) {
       const bool more = c + 1 < nch;
       const int cn = more ? c + 1 : c;
-      const TL* sin = sbuf + (c & 1) * (2 * STAGE);
-      if (more) stage(cn, sbuf + ((c + 1) & 1) * (2 * STAGE), in_terms);
-      float4 av[2][2];
-      auto load_a = [&](int at, float4 (&dst)[2]) __attribute__((always_inline)) {
+      const TL* sin = sbuf + c % NBUF * (PL * STAGE);
+      if constexpr (F2) {
+        if (more) stage(cn, sbuf + (c + 1) % NBUF * (PL * STAGE), in_terms);
+      }
+      float4 av[2][PL];
+      auto load_a = [&](int at, float4 (&dst)[PL]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) dst[q] = *reinterpret_cast<const float4*>(&sin[q * STAGE + at]);
+        for (int q = 0; q < PL; ++q) dst[q] = *reinterpret_cast<const float4*>(&sin[q * STAGE + at]);
       };
       int base, step, qi = 0, g = 0;
       lane_of(0, 0, base, step);
@@ -1040,7 +1074,7 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
         const bool corner = ((strip >> (4 * g)) & 15u) >= 3u;
         int base_n, step_n;
         lane_of(gn, qn, base_n, step_n);
-        acc[0] = zero;
+        if (F2) acc[0] = zero;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           if (t == 1) seek_b(gb_next);
@@ -1050,24 +1084,32 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
           const auto& A = av[t & 1];
           const auto& B = bring[t];
           if (t < 3 || !corner) {
-            mma_f16(sm[0], A[1], B[0]);
-            mma_f16(acc[0], A[0], B[0]);
-            mma_f16(sm[0], A[0], B[1]);
+            if constexpr (F2) {
+              mma_f16(sm[0], A[1], B[0]);
+              mma_f16(acc[0], A[0], B[0]);
+              mma_f16(sm[0], A[0], B[1]);
+            } else {
+              mma_unit(acc[0], A[0], B[0], mie_bf16());
+            }
           }
           __builtin_amdgcn_sched_barrier(0);
         }
+        if constexpr (F2) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) flush(acc, 0, r);
+          for (int r = 0; r < 16; ++r) flush(acc, 0, r);
+        }
         base = base_n; step = step_n; g = gn; qi = qn;
       }
       __syncthreads();
     }
   }
-  const float c0 = f2_unscale(groups.scale) * filt_unscale, c1 = c0 * (1.f / F2_STEP);      // exactly: powers of two, 2^-143 at the least
+  if constexpr (F2) {
+    const float c0 = f2_unscale(groups.scale) * filt_unscale, c1 = c0 * (1.f / F2_STEP);      // exactly: powers of two, 2^-143 at the least
 #pragma unroll
-  for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[mb][r] = fmaf(sm[mb][r], c1, tot[mb][r] * c0);
+      for (int r = 0; r < 16; ++r) acc[mb][r] = fmaf(sm[mb][r], c1, tot[mb][r] * c0);
+  }
   float* const red = smem + phase * (64 * CO_BLK);
   auto park = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -1089,54 +1131,58 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
       off[i] = (((long long)n * hout + oy) * wout + ox) * cout + co0 + col;
       co[i] = co0 + col;
     }
-    conv_epilogue_load4<float, PB>(a, off, live, r0, add);
+    conv_epilogue_load4<T, PB>(a, off, live, r0, add);
   };
   fetch(0);
-  if (groups.misfit() || !filt_fits) s_f2[4] = 1.f;
+  if constexpr (F2) {
+    if (groups.misfit() || !filt_fits) s_f2[4] = 1.f;
+  }
   park();
   __syncthreads();
-  if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
-    // a group that does not fit: all of it once more on the fp32 instruction (see k_upconv2x)
+  if constexpr (F2) {
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
+      // a group that does not fit: all of it once more on the fp32 instruction (see k_upconv2x)
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb) acc[mb] = zero;
-    for (int c = 0; c < nch; ++c) {
-      __syncthreads();
-      stage(c, sbuf, std::false_type());
-      if (tid < 2 * (LS / EPS)) {
-        const int pl = tid / (LS / EPS);
-        *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (tid - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int mb = 0; mb < 2; ++mb) acc[mb] = zero;
+      for (int c = 0; c < nch; ++c) {
+        __syncthreads();
+        stage(c, sbuf, std::false_type());
+        if (tid < 2 * (LS / EPS)) {
+          const int pl = tid / (LS / EPS);
+          *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (tid - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        __syncthreads();
+        auto unit = [&](const TL* gb, int at0, int at1) __attribute__((always_inline)) {
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const float4 b = *reinterpret_cast<const float4*>(gb + 2 * weights + b_lane + q * (2 * cout * EPS));
+            mma_unit(acc[0], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at0]), b, float());
+            if (side == 0) mma_unit(acc[1], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at1]), b, float());
+          }
+        };
+        for (int qi = 0; qi < NQ; ++qi) {
+          if (side == 0) {
+#pragma unroll 1
+            for (int k = 0; k < 16; ++k) {
+              const int at = (k >> 2) * RP + (k & 3) * LS + SUB * qi;
+              unit(group_b(c, qi, k), a_lane[0] + at, a_lane[1] + at);
+            }
+          } else {
+#pragma unroll 1
+            for (int g = 0; g < ng; ++g) {
+              const int code = (int)((strip >> (4 * g)) & 15u);
+              const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
+              const int base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF, step = on ? (corner ? RPS : LS) : 0;
+#pragma unroll 1
+              for (int t = 0; t < (corner ? 3 : 4); ++t) unit(group_b(c, qi, strip_unit(g) + t), base + t * step, 0);
+            }
+          }
+        }
       }
       __syncthreads();
-      auto unit = [&](const TL* gb, int at0, int at1) __attribute__((always_inline)) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const float4 b = *reinterpret_cast<const float4*>(gb + 2 * weights + b_lane + q * (2 * cout * EPS));
-          mma_unit(acc[0], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at0]), b, float());
-          if (side == 0) mma_unit(acc[1], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at1]), b, float());
-        }
-      };
-      for (int qi = 0; qi < NQ; ++qi) {
-        if (side == 0) {
-#pragma unroll 1
-          for (int k = 0; k < 16; ++k) {
-            const int at = (k >> 2) * RP + (k & 3) * LS + SUB * qi;
-            unit(group_b(c, qi, k), a_lane[0] + at, a_lane[1] + at);
-          }
-        } else {
-#pragma unroll 1
-          for (int g = 0; g < ng; ++g) {
-            const int code = (int)((strip >> (4 * g)) & 15u);
-            const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
-            const int base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF, step = on ? (corner ? RPS : LS) : 0;
-#pragma unroll 1
-            for (int t = 0; t < (corner ? 3 : 4); ++t) unit(group_b(c, qi, strip_unit(g) + t), base + t * step, 0);
-          }
-        }
-      }
+      park();
+      __syncthreads();
     }
-    __syncthreads();
-    park();
-    __syncthreads();
   }
 #pragma unroll
   for (int h0 = 0; h0 < PER; h0 += PB) {
@@ -1144,7 +1190,7 @@ __global__ __launch_bounds__(256, 2) void k_upconv2x_all(ConvArgsT<float> a, Up2
     float4 s[PB];
 #pragma unroll
     for (int i = 0; i < PB; ++i) s[i] = *reinterpret_cast<const float4*>(&smem[4 * (tid + 256 * (h0 + i))]);
-    conv_epilogue_store4<float, PB>(a, off, co, ok, s, r0, add, live);
+    conv_epilogue_store4<T, PB>(a, off, co, ok, s, r0, add, live);
   }
 }
 
@@ -1170,7 +1216,7 @@ void launch_one(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
   od.m_bx = od.blocks_x > 0 ? mie_tile_magic(od.items, od.blocks_x) : 0u;
   if constexpr (WN == 0) {
     const int strips = a.ts.n * 2 * (od.strips_x + od.strips_y) * od.combos;
-    hipLaunchKernelGGL(k_upconv2x_all, dim3(8 * ((od.total + 7) / 8 + (strips + 7) / 8)), dim3(256), 0, st, a, od);
+    hipLaunchKernelGGL(k_upconv2x_all<T>, dim3(8 * ((od.total + 7) / 8 + (strips + 7) / 8)), dim3(256), 0, st, a, od);
   } else {
     hipLaunchKernelGGL((k_upconv2x<T, WN, AR>), dim3(8 * ((od.total + 7) / 8)), dim3(256), 0, st, a, od);
   }
@@ -1185,13 +1231,19 @@ void launch_one(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
 // 768 (128->64 at 66x74, 656 of them: 15.7 against 17.2; at 66x88, 784: 20.4 against 17.7), 128 columns, which read the
 // input least, where they make more than a round themselves (256->128 at 8x60x80: 246 against 217; at 4x60x80, 1440: 126
 // against 116; at 3x60x80, 1080: 92 either way; at 8x30x40, 832: 76 against 83).
-// k_upconv2x_all or k_upconv2x (wgs: of 32 columns): where the latter needs more workgroups than two to a CU, and the layer has 64 or
-// 96 channels.  64->32 at 80x112 (608 of them) 22.2 -> 19.1 us, at 132x176 (1584) 50 -> 32, at 240x320 137 -> 87; 64->64 at 64x64 (576) 22
-// -> 18.8, 96->32 at 96x96 31 -> 24.4; at 72x80 (400) 15.7 against 18.1.  (Against k_upconv2x in three terms: in two it would be faster, too, but
-// 1.13 and 1.05 times as far from fp64 with 64 and 96 channels.)  From 128 channels on, in two terms either way, a workgroup here is longer than
-// the launch is wide: 128->64 at 66x88 29.3 against 32, at 120x160 78 against 87, 256->128 at 60x80 86 against 96.
-// (In one chunk of 32 channels three terms are as near: 9.94e-8 and 1.00e-7.  Planes of two rows or columns are all strips.)
-bool up2x_all(int c, long long wgs, const Up2xOrder& od) { return c >= 64 && c < 128 && wgs > 512 && od.blocks_y * od.blocks_x > 0; }
+// k_upconv2x_all or k_upconv2x (wgs: of 32 columns, of the latter).
+// fp32: where the latter needs more workgroups than two to a CU, and the layer has 64 or 96 channels.  64->32 at 80x112 (608 of them) 22.2 ->
+// 19.1 us, at 132x176 (1584) 50 -> 32, at 240x320 137 -> 87; 64->64 at 64x64 (576) 22 -> 18.8, 96->32 at 96x96 31 -> 24.4; at 72x80 (400)
+// 15.7 against 18.1.  (Against k_upconv2x in three terms: in two it would be faster, too, but 1.13 and 1.05 times as far from fp64 with 64 and
+// 96 channels.)  From 128 channels on, in two terms either way, a workgroup here is longer than the launch is wide: 128->64 at
+// 66x88 29.3 against 32, at 120x160 78 against 87, 256->128 at 60x80 86 against 96.  In one chunk of 32 channels three terms are as near:
+// 9.94e-8 and 1.00e-7.  Planes of two rows or columns are all strips.
+// bf16: 64 channels, whose other form is the list-driven one (k_conv_mfma<..., UP>, k_upconv64_persist), from more workgroups here than
+// CUs on: 64->32 at 120x140 20.7 -> 17.7, at 2x100x140 27.0 -> 20.6, at 160x160 26.4 -> 19.7, 64->64 at 100x140 26.4 -> 20.6, 64->32 at
+// 8x240x320 374 -> 308; in between (128x128 17.4 and 17.2, 116x132 16.9 and 17.1) and below (96x96 13.3 and 13.6) either way.
+bool up2x_all(int c, long long wgs, const Up2xOrder& od, bool bf) {
+  return (bf ? c == 64 && wgs > 1024 : c >= 64 && c < 128 && wgs > 512) && od.blocks_y * od.blocks_x > 0;
+}
 
 template <typename T>
 void launch_up2x(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
@@ -1199,11 +1251,12 @@ void launch_up2x(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
   const long long wgs = (long long)a.ts.n * od.items * 4 * (cout / 32);
   if constexpr (sizeof(T) == 4) {
     const bool wide = cout % 64 == 0 && wgs > 256 && (wgs <= 512 || wgs > 768 || a.x3 == 2);
-    if (a.x3 == 2 && up2x_all(a.c1, wgs, od)) launch_one<T, 0, 2>(a, od, st);
+    if (a.x3 == 2 && up2x_all(a.c1, wgs, od, false)) launch_one<T, 0, 2>(a, od, st);
     else if (a.x3 == 2) wide ? launch_one<T, 2, 2>(a, od, st) : launch_one<T, 1, 2>(a, od, st);
     else wide ? launch_one<T, 2, 1>(a, od, st) : launch_one<T, 1, 1>(a, od, st);
   } else {
-    if (cout % 128 == 0 && wgs / 4 >= 1024) launch_one<T, 4, 0>(a, od, st);
+    if (up2x_all(a.c1, wgs, od, true)) launch_one<T, 0, 0>(a, od, st);
+    else if (cout % 128 == 0 && wgs / 4 >= 1024) launch_one<T, 4, 0>(a, od, st);
     else if (cout % 64 == 0 && wgs > 768) launch_one<T, 2, 0>(a, od, st);
     else launch_one<T, 1, 0>(a, od, st);
   }
@@ -1315,9 +1368,15 @@ extern "C" int mie_upconv2x_refresh(const void* a, const void* b, int c, int h_i
                           act_kind, slope, true, dtype == MIE_DTYPE_F32_F16X2 ? 2 : 1, stream);
 }
 
-extern "C" int mie_f16x2_takes_upconv2x(int n, int h_in, int w_in, int c, int cout) {
-  if (n <= 0 || h_in < 2 || w_in < 2 || c <= 0 || cout <= 0 || c % 32 != 0 || cout % 32 != 0) return 0;
+extern "C" int mie_all_phases_upconv2x(int n, int h_in, int w_in, int c, int cout, int dtype) {
+  const bool bf = dtype == MIE_DTYPE_BF16;
+  if (n <= 0 || h_in < 2 || w_in < 2 || c <= 0 || cout <= 0 || c % 32 != 0 || cout % 32 != 0 || !(bf || dtype == MIE_DTYPE_F32_F16X2)) return 0;
   Up2xOrder od = {};
   up2x_items(od, h_in, w_in);
-  return c >= 128 || up2x_all(c, (long long)n * od.items * 4 * (cout / 32), od) ? 1 : 0;
+  return up2x_all(c, (long long)n * od.items * 4 * (cout / 32), od, bf) ? 1 : 0;
+}
+
+extern "C" int mie_f16x2_takes_upconv2x(int n, int h_in, int w_in, int c, int cout) {
+  if (n <= 0 || h_in < 2 || w_in < 2 || c <= 0 || cout <= 0 || c % 32 != 0 || cout % 32 != 0) return 0;
+  return c >= 128 || mie_all_phases_upconv2x(n, h_in, w_in, c, cout, MIE_DTYPE_F32_F16X2);
 }

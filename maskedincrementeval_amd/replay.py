@@ -174,7 +174,7 @@ def _idle() -> bool:
 # questions to the library, answered in every phase and never recorded
 PASS_THROUGH = frozenset(("mie_last_error_string", "mie_tile_capacity", "mie_version", "mie_conv_f32x3_takes",
                           "mie_conv_needs_no_workspace", "mie_conv_gates_needs_no_workspace", "mie_upconv_needs_no_workspace",
-                          "mie_f16x2_takes_upconv2x"))
+                          "mie_f16x2_takes_upconv2x", "mie_all_phases_upconv2x"))
 _VIEWS = frozenset(("aten::permute", "aten::detach", "aten::view", "aten::slice", "aten::select", "aten::alias",
                     "aten::as_strided", "aten::t", "aten::transpose", "aten::unsqueeze", "aten::squeeze",
                     "aten::expand", "aten::_reshape_alias", "aten::_unsafe_view", "aten::split", "aten::unbind"))

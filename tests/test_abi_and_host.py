@@ -392,6 +392,9 @@ def test_decoders_in_two_terms_are_those_nearer_to_fp64(mie_lib):
     assert q(1, 8, 8, 128, 32) == 1 and q(1, 132, 176, 64, 32) == 1 and q(1, 64, 64, 64, 32) == 0 and q(1, 64, 64, 64, 64) == 1
     assert q(1, 80, 82, 64, 32) == 0 and q(2, 80, 82, 64, 32) == 1          # 4 * (11 * 10 + 6 + 6) = 472 each
     assert q(1, 2, 4000, 64, 32) == 0 and q(1, 1, 40, 128, 32) == 0 and q(1, 64, 64, 48, 32) == 0 and q(1, 132, 176, 32, 32) == 0 and q(1, 64, 64, 128, 48) == 0 and q(0, 64, 64, 128, 32) == 0
+    a, bf, f2 = mie_lib.mie_all_phases_upconv2x, _lib.DTYPE_BF16, _lib.DTYPE_F32_F16X2
+    assert a(1, 132, 176, 64, 32, f2) == 1 and a(1, 132, 176, 128, 32, f2) == 0 and a(1, 64, 64, 64, 32, f2) == 0 and a(1, 132, 176, 64, 32, _lib.DTYPE_F32_BF16X3) == 0
+    assert a(1, 132, 176, 64, 32, bf) == 1 and a(1, 96, 96, 64, 32, bf) == 0 and a(1, 132, 176, 96, 32, bf) == 0 and a(1, 2, 9000, 64, 32, bf) == 0
 
 
 def test_workspace_queries_draw_the_line_where_the_split_form_is_faster(mie_lib):

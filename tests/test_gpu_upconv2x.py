@@ -258,3 +258,11 @@ def test_decoder_conv_of_few_channels_on_many_blocks(n, c, cout, h, w):
     test_decoder_conv_at_input_resolution(n, c, cout, h, w, torch.float32)
     if n == 1 and h > 2 and c == 64:
         test_pixels_outside_the_mask_keep_their_reservoir(n, c, cout, h, w, torch.float32, "blocks")
+
+
+# bf16, 64 channels, more such workgroups than CUs
+@pytest.mark.parametrize("n,c,cout,h,w", [(2, 64, 32, 100, 140), (1, 64, 96, 75, 74), (5, 64, 32, 34, 90), (1, 64, 32, 2100, 3), (1, 64, 32, 3, 2100)])
+def test_decoder_conv_of_one_chunk_on_many_blocks(n, c, cout, h, w):
+    assert _lib.lib().mie_all_phases_upconv2x(n, h, w, c, cout, _lib.DTYPE_BF16)
+    test_decoder_conv_at_input_resolution(n, c, cout, h, w, torch.bfloat16)
+    test_pixels_outside_the_mask_keep_their_reservoir(n, c, cout, h, w, torch.bfloat16, "blocks")
