@@ -93,7 +93,8 @@ extern "C" {
  * workgroup's input does not lie within fp16's range of its scale -- groups of eight channels of a pixel 2^23 below the largest value
  * or 2^6 above it, infinities, NaN -- it contracts in fp32 instead, as for MIE_DTYPE_F32, from a copy of the filter
  * that the packed one holds too: correct, and slower.  Forms that add up the products of three terms more finely than that -- those
- * without a workspace on planes of few tiles, the transposed convs -- keep the three (the packed copy holds them as well).
+ * without a workspace on planes of few tiles, but for the 3x3 stride-1 convs of 512 channels and more, and the transposed convs on planes
+ * of few blocks -- keep the three (the packed copy holds them as well).
  * Taken, for the same shapes, wherever MIE_DTYPE_F32_BF16X3 is. */
 #define MIE_DTYPE_F32_F16X2 3
 /* bytes behind the weights of a filter copy packed for it (scale, whether all weights fit it, workspace of the packing) */
@@ -247,7 +248,7 @@ int mie_pack_filter(const float* filter, int cin, int k, int cout, void* packed,
                     int dtype, void* stream);
 
 /*
- * 1 if the matrix-core conv takes this shape with dtype MIE_DTYPE_F32_BF16X3 (k = 3 or 5 at stride 1 with
+ * 1 if the matrix-core conv takes this shape with dtype MIE_DTYPE_F32_BF16X3 or MIE_DTYPE_F32_F16X2 (k = 3 or 5 at stride 1 with
  * c1, c2 multiples of 32, or k = 5 at stride 2 with multiples of 16; cout a multiple of 32), else 0: such a call must then be made with MIE_DTYPE_F32 and the
  * fp32 filter copy.  No counterpart in the reference (it has one arithmetic, cuDNN's or its own
  * kernel's fp32: ext/pointops/_C_ext/pointops/ext_conv.cu:74-76).
@@ -256,9 +257,9 @@ int mie_conv_f32x3_takes(int k, int stride, int c1, int c2, int cout);
 
 /*
  * Whether mie_conv_masked, without a workspace, runs a conv of this shape (matrix-core path; `tiles` = mie_tile_capacity of
- * its output, dtype with MIE_DTYPE_F32_BF16X3 where the call has it) in one launch faster than mie_conv_masked_ws runs it with one.
+ * its output, dtype with MIE_DTYPE_F32_BF16X3 or MIE_DTYPE_F32_F16X2 where the call has it) in one launch faster than mie_conv_masked_ws runs it with one.
  * 0 for layers that the matrix-core path does not take, whatever their filter copy.  Host logic only.
- * Where it is 1 with MIE_DTYPE_F32_BF16X3, that call takes a 3x3 conv of stride 2 too (which mie_conv_f32x3_takes does not name:
+ * Where it is 1 with one of these two, that call takes a 3x3 conv of stride 2 too (which mie_conv_f32x3_takes does not name:
  * on planes of more tiles it runs on the fp32 instruction).
  */
 int mie_conv_needs_no_workspace(int k, int stride, int c1, int c2, int cout, int tiles, int dtype);
@@ -567,7 +568,7 @@ int mie_convgru_gates_incr(const void* gates_delta, float* update_res,
 /*
  * The stacked gates conv of a ConvGRU whose state is reset each step (3x3, stride 1, pad 1, cin -> 2*hid channels) with
  * mie_convgru_gates_incr as its epilogue, so that the 2*hid-channel delta is never written to memory.  Matrix-core path only,
- * bf16 deltas or fp32 in the three-term form (MIE_DTYPE_F32_BF16X3): needs filter_mc, cin in whole staging chunks and hid % 16 == 0;
+ * bf16 deltas or fp32 in terms (MIE_DTYPE_F32_BF16X3, MIE_DTYPE_F32_F16X2): needs filter_mc, cin in whole staging chunks and hid % 16 == 0;
  * otherwise MIE_ERR_UNSUPPORTED (use the two calls then).  The filter's columns are interleaved in groups of four: column 8*j + e
  * is the update gate of hidden channel 4*j + e for e < 4, the candidate of hidden channel 4*j + e - 4 for e >= 4.  update_res,
  * cand_res, h_delta as in mie_convgru_gates_incr, plain channel order.
@@ -806,7 +807,7 @@ int mie_tconv_masked(const void* x, const uint8_t* xmask, int cin, int h_in,
  * sub-pixel phases of the output are four stride-1 contractions over disjoint
  * tap subsets of the same staged input, so no product is spent on inserted zeros.
  *   x / x2 : [n,h_in,w_in,c1] / [n,h_in,w_in,c2] deltas with their pixel masks
- *        (x2 optional); c1, c2 multiples of 32 (bf16 and MIE_DTYPE_F32_BF16X3: 64), cout of 32
+ *        (x2 optional); c1, c2 multiples of 32 (bf16, MIE_DTYPE_F32_BF16X3 and MIE_DTYPE_F32_F16X2: 64), cout of 32
  *   filter / filter_mc : [cin_total][k][k][cout] as in mie_tconv_masked and its
  *        matrix-core copy (mie_pack_filter, required); c1 + c2 <= cin_total
  *   out    : output tile set at (2*h_in, 2*w_in), built with MIE_FOOT_TCONV
@@ -817,7 +818,7 @@ int mie_tconv_masked(const void* x, const uint8_t* xmask, int cin, int h_in,
  *        e.g. the contribution of a few more input channels computed by
  *        mie_tconv_masked, covered by `out`)
  *   workspace / workspace_bytes : as in mie_conv_masked_ws (on planes of very few
- *        blocks k = 5, MIE_DTYPE_F32 and MIE_DTYPE_F32_BF16X3 of more than 1408
+ *        blocks k = 5, MIE_DTYPE_F32, and fp32 in terms of more than 1408
  *        channels split their contraction over up to 8 workgroups; k = 3 has no
  *        other use for it); may be NULL
  * Replaces: transposed_conv2d_from_module
@@ -837,7 +838,7 @@ int mie_tconv2x_masked(const void* x, const uint8_t* xmask, int c1,
  * The same for k = 3 with two more input channels in front, a narrow part of the concat (a flow estimate of the scale before):
  *   lead, lead_mask : [n,h_in,w_in,2] delta and its pixel mask (NULL: all), covered by `out`
  *   lead_filter     : [2][3][3][cout] fp32, its rows of the filter (bf16 deltas: the weights rounded to bf16)
- * in place of mie_tconv_masked of the lead and an addend.  MIE_DTYPE_BF16 or MIE_DTYPE_F32_BF16X3 (MIE_ERR_UNSUPPORTED otherwise).
+ * in place of mie_tconv_masked of the lead and an addend.  MIE_DTYPE_BF16 or fp32 in terms (MIE_ERR_UNSUPPORTED otherwise).
  */
 int mie_tconv2x_lead_masked(const void* lead, const uint8_t* lead_mask, const float* lead_filter, const void* x, const uint8_t* xmask, int c1,
                             const void* x2, const uint8_t* x2mask, int c2, int h_in, int w_in, const float* filter, const void* filter_mc,

@@ -561,7 +561,7 @@ class nnConvIncr(replay.Watched, nn.Conv2d, _ConvIncrMixin):
         # is bound by launches and the one-kernel form wins (1.5 % of a 264x352 frame) unless the layer has more
         # than 4 staged chunks (256 channels: the per-chunk blend then costs what the saved launch gains); on
         # large planes the separate up-sampling kernel is cheaper (8x480x640 step +2 % with the one-kernel form).
-        # fp32 in the three-term form: the one-kernel form wins at every size and depth (264x352 frame -0.4 %,
+        # fp32 in terms: the one-kernel form wins at every size and depth (264x352 frame -0.4 %,
         # 8x480x640 step -1.8 %).
         dt = ops.delta_torch_dtype(x)
         tiles = x.shape[0] * ((2 * x.shape[2] + 7) // 8) * ((2 * x.shape[3] + 7) // 8)

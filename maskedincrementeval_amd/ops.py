@@ -864,7 +864,7 @@ def conv_masked(x, xmask, x2, x2mask, filt, k, stride, pad, out_ts: TileMask, ou
 
 
 # Up to which size fp32 decoder layers take the one-kernel form where they run on the fp32 matrix-core instruction
-# (see nnConvIncr.forward_fused_upsampled; in the three-term form they always do).
+# (see nnConvIncr.forward_fused_upsampled; in terms they always do).
 upconv_max_tiles = 2048
 upconv_max_chunks = 4
 
@@ -1163,7 +1163,7 @@ def tconv2x_masked(x, xmask, x2, x2mask, filt, k, out_ts: TileMask, block_ts: Ti
             pix_ptr(x2mask, n, h, w, "x2mask"), c2, h, w, plain.data_ptr(), mc_ptr, cin_total, cout, out_ts.ref,
             block_ts.ref, nhwc_ptr(out_delta, "out_delta", dtype=dt), nhwc_ptr(reservoir, "reservoir"), act, float(slope), code, _stream(x)))
         return out_delta
-    # (3x3 on bf16 deltas and in the three-term form, but for very many channels there: one launch on planes of few blocks)
+    # (3x3 on bf16 deltas and fp32 in terms, but for very many channels there: one launch on planes of few blocks)
     split = k != 3 or code == _lib.DTYPE_F32 or (code != _lib.DTYPE_BF16 and c1 + c2 > 1408)
     ws_ptr, ws_bytes = _workspace_args(workspace, block_ts.capacity * (cout // 32) <= 128 and split, x.device)
     check(lib().mie_tconv2x_masked(
