@@ -457,30 +457,34 @@ __device__ __forceinline__ void split_order(const ConvArgsT<T>& a, int& bx, int&
 // AGAIN (X3 only): outputs whose sum is not finite are computed again in fp32 (conv_quad_again).
 // GRU (with GATES): the gate math of a ConvGRU in place of the ConvLSTM's chain; eight columns, update and candidate, to four
 // hidden channels.
+// WIDE (F2): eight waves and chunks of twice the channels; f2_wide says where.
 template <typename T, int K, int S, int WN, int NB, bool HALF, bool GATES = false, bool UP = false, bool SPLIT = false,
-          int ARITH = 0, bool AGAIN = false, bool GRU = false>
+          int ARITH = 0, bool AGAIN = false, bool GRU = false, bool WIDE = false>
 // (Build with -mllvm -pragma-unroll-threshold=65536: the unit loop of the 128-column 5x5 / 7x7 kernels is 100 / 196
 // positions long, and where the compiler refuses to unroll it the operand ring is indexed at run time and lands in
 // scratch memory -- a factor of three in time.)
-__global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GATES, UP, SPLIT, ARITH != 0)) void k_conv_mfma(ConvArgsT<T> a) {
+__global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K, S, HALF, GATES, UP, SPLIT, ARITH != 0)) void k_conv_mfma(ConvArgsT<T> a) {
   constexpr bool X3 = ARITH != 0, F2 = ARITH == 2;           // values in terms; in two of them
   static_assert(!X3 || (sizeof(T) == 4 && !HALF && (K == 3 || K == 5)), "X3: fp32 deltas, 3x3 / 5x5");
   using TL = std::conditional_t<X3, mie_bf16, T>;            // element type in LDS and on the matrix cores
   constexpr int PL = F2 ? 2 : X3 ? 3 : 1;                    // operand planes (terms per value)
   constexpr int GPS = X3 ? 2 : 1;                            // 16-byte global loads per staging slot
-  constexpr int NBUF = X3 ? ((K == 3 && S == 1) ? 2 : 1) : stage_buffers(S, (int)sizeof(T));
+  constexpr int TH = WIDE ? 512 : 256, WAVES = TH / 64;
+  static_assert(!WIDE || (F2 && !UP && !SPLIT), "eight waves: two terms");
+  constexpr int NBUF = X3 ? (((K == 3 && S == 1) || WIDE) ? 2 : 1) : stage_buffers(S, (int)sizeof(T));
   constexpr int EPS = 16 / (int)sizeof(TL);                  // elements per 16-byte slot (4 / 8)
   constexpr int SUB = 2 * EPS;                               // channels per unit (8 / 16)
-  constexpr int WK = 4 / WN;
+  constexpr int WK = WAVES / WN;
   constexpr int IT = 7 * S + K;                              // input tile edge incl. halo
-  constexpr int CC = X3 ? (S == 2 ? 16 : 32) : stage_channels(K, S, HALF) * (4 / (int)sizeof(T));   // channels per LDS stage
+  constexpr int CC = X3 ? (S == 2 ? 16 : 32) * (WIDE ? 2 : 1) : stage_channels(K, S, HALF) * (4 / (int)sizeof(T));   // channels per LDS stage
   constexpr int LS = CC + EPS;                               // LDS elements per staged pixel
   constexpr int NPIX = IT * IT;
   constexpr int Q4 = CC / EPS;                               // 16-byte slots per pixel
   constexpr int NSLOT = NPIX * Q4;
-  constexpr int NLD = (NSLOT + 255) / 256;                   // staging slots per thread
+  constexpr int NLD = (NSLOT + TH - 1) / TH;                   // staging slots per thread
   constexpr int RP = row_pitch_dw(IT, LS * (int)sizeof(TL) / 4, S) * 4 / (int)sizeof(TL);   // elements per tile row
-  constexpr int STAGE = IT * RP;                             // elements per plane of a staging buffer
+  constexpr bool ROOM = RP - IT * LS >= EPS;                 // a slot fits into the padding of a row
+  constexpr int STAGE = IT * RP + (WIDE && !ROOM ? 4 * EPS : 0);   // elements per plane of a staging buffer
   constexpr int NQ = CC / SUB;                               // sub-chunks (units per tap) per stage
   // k-split: over whole sub-chunks (every wave takes NQW of them, for every tap), or -- more waves than sub-chunks,
   // X3 only -- one sub-chunk and every TP-th tap per wave (the last position of a chunk is then empty for some waves)
@@ -499,9 +503,9 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   static_assert(!UP || (S == 1 && K == 5 && !GATES), "the up-sampling variant is the 5x5 stride-1 conv");
   // the k-split reduction of the epilogue reuses the staging buffers and the source block
   constexpr int SMEM = (STAGE_F + LO_F > RED) ? STAGE_F + LO_F : RED;
-  static_assert(SMEM * 4 <= 65536, "LDS budget");
+  static_assert(SMEM * 4 <= (WIDE ? 160 * 1024 : 65536), "LDS budget");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
-  __shared__ float s_f2[F2 ? 5 : 1];                         // largest values of the waves' first slots; whether a group does not fit
+  __shared__ float s_f2[F2 ? WAVES + 1 : 1];                         // largest values of the waves' first slots; whether a group does not fit
   static_assert(!F2 || !AGAIN, "two terms: what does not fit is contracted in fp32");
   TL* const sbuf = reinterpret_cast<TL*>(smem);
   float* const s_lo = smem + STAGE_F;
@@ -562,7 +566,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   if (SPLIT && tk == 2) return;      // stale tiles are zeroed by k_conv_split_finish
   if (GATES && tk == 2) {  // stale tile: zero the hidden / cell deltas of this workgroup's hidden channels
     constexpr int HG = CO_BLK / (GRU ? 8 : 16);          // groups of four hidden channels
-    for (int idx = tid; idx < 64 * HG; idx += 256) {
+    for (int idx = tid; idx < 64 * HG; idx += TH) {
       const int p = idx / HG, g4 = idx - p * HG;
       const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
       if (oy < hout && ox < wout) {
@@ -574,7 +578,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     return;
   }
   if (tk == 2) {  // stale tile: zero this workgroup's channel slab
-    for (int idx = tid; idx < 16 * CO_BLK; idx += 256) {       // groups of four channels
+    for (int idx = tid; idx < 16 * CO_BLK; idx += TH) {       // groups of four channels
       const int p = idx / (CO_BLK / 4), col = 4 * (idx - p * (CO_BLK / 4));
       const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
       if (oy < hout && ox < wout)
@@ -589,7 +593,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // fp32 kernels the reservoir / addend values are fetched once the mask bytes are there and have the whole contraction to
   // arrive.
   constexpr int QPP = CO_BLK / 4;                            // groups of four channels per pixel
-  constexpr int PER = GATES ? 1 : 64 * QPP / 256;            // groups per thread
+  constexpr int PER = GATES ? 1 : 64 * QPP / TH;            // groups per thread
   constexpr int PB = PER > 4 ? 4 : PER;                      // groups per pass of the epilogue (registers)
   long long e_off[PB];
   int e_co[PB];
@@ -606,7 +610,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   auto epilogue_fetch = [&](int h0) {
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
-      const int idx = tid + 256 * (h0 + i);
+      const int idx = tid + TH * (h0 + i);
       const int p = idx / QPP, col = 4 * (idx - p * QPP);
       const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
       e_ok[i] = oy < hout && ox < wout;
@@ -638,7 +642,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   unsigned inb = 0u;             // slot inside the image
 #pragma unroll
   for (int i = 0; i < NLD; ++i) {
-    const int slot = tid + 256 * i;
+    const int slot = tid + TH * i;
     const int pix = slot / Q4, q4 = slot - pix * Q4;
     const int lrow = pix / IT;
     const int swz = (S == 2) ? ((lrow >> 1) & 1) : 0;
@@ -658,7 +662,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
 
   // UP: the source block.  Rows iy0 .. iy0+11 of the up-sampled image (iy0 even) blend source rows
   // iy0/2 - 1 .. iy0/2 + 6; one 16-byte slot per (source pixel, channel group) and tensor.
-  constexpr int NLO = UP ? (64 * Q4 + 255) / 256 : 1;
+  constexpr int NLO = UP ? (64 * Q4 + TH - 1) / TH : 1;
   const int h_lo = a.h_in >> 1, w_lo = a.w_in >> 1;
   const int lo_y0 = (iy0 >> 1) - 1, lo_x0 = (ix0 >> 1) - 1;
   int lo_po[NLO];
@@ -667,7 +671,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   if (UP) {
 #pragma unroll
     for (int i = 0; i < NLO; ++i) {
-      const int slot = tid + 256 * i;
+      const int slot = tid + TH * i;
       const int lpix = slot / Q4;
       const int ly = lo_y0 + (lpix >> 3), lx = lo_x0 + (lpix & 7);
       lo_po[i] = 0;
@@ -712,7 +716,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       const T* dummy = a.filt_mc;
 #pragma unroll
       for (int i = 0; i < NLO; ++i) {
-        const int q4 = (tid + 256 * i) % Q4;
+        const int q4 = (tid + TH * i) % Q4;
         const long long eo = (long long)lo_po[i] * a.c1 + c * CC + EPS * q4;
         const bool k1 = ((first ? lo_inb : lo_ok1) >> i) & 1u;
         const bool k2 = first ? (a.x2 != nullptr && ((lo_inb >> i) & 1u)) : ((lo_ok2 >> i) & 1u);
@@ -756,7 +760,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     TL* dst = sbuf + buf * (PL * STAGE);
 #pragma unroll
     for (int i = 0; i < NLD; ++i)
-      if (tid + 256 * i < NSLOT) {
+      if (tid + TH * i < NSLOT) {
         float4 r[GPS];
 #pragma unroll
         for (int g = 0; g < GPS; ++g) r[g] = kept(regs[i][g], (ok >> i) & 1u);
@@ -767,10 +771,12 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   auto scale_of = [&](float m) __attribute__((always_inline)) {
     m = f2_wave_max(m);
     if (lane == 0) s_f2[wave] = m;
-    if (tid == 0) s_f2[F2 ? 4 : 0] = 0.f;
+    if (tid == 0) s_f2[F2 ? WAVES : 0] = 0.f;
     __syncthreads();
-    groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(
-        __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[F2 ? 1 : 0], s_f2[F2 ? 2 : 0]), s_f2[F2 ? 3 : 0]))))));
+    float w = s_f2[0];
+#pragma unroll
+    for (int i = 1; i < WAVES; ++i) w = __builtin_elementwise_maximum(w, s_f2[F2 ? i : 0]);
+    groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(w)))));
   };
   auto slots_max = [&](const float4 (&regs)[NLD][GPS], unsigned ok) __attribute__((always_inline)) {
     float m = 0.f;
@@ -792,7 +798,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       float lo_max = 0.f;
 #pragma unroll
       for (int i = 0; i < NLO; ++i) {
-        const int slot = tid + 256 * i;
+        const int slot = tid + TH * i;
         const int lpix = slot / Q4, q4 = slot - lpix * Q4;
         float fa[EPS], fb[EPS];
         const bool k1 = (lo_ok1 >> i) & 1u, k2 = (lo_ok2 >> i) & 1u;
@@ -839,7 +845,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       if (sizeof(T) == 2 || (X3 && WN == 1)) asm volatile("" : "+v"(opaque));
 #pragma unroll
       for (int i = 0; i < NLD; ++i) {
-        const int slot = tid + 256 * i + opaque;
+        const int slot = tid + TH * i + opaque;
         if (slot >= NSLOT) continue;
         const int pix = slot / Q4, q4 = slot - pix * Q4;
         const int hy = iy0 + pix / IT, hx = ix0 + pix % IT;
@@ -888,7 +894,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     } else {
 #pragma unroll
       for (int i = 0; i < NLD; ++i)
-        if (tid + 256 * i < NSLOT) {
+        if (tid + TH * i < NSLOT) {
           float4 r[GPS];
 #pragma unroll
           for (int g = 0; g < GPS; ++g) r[g] = kept(st_reg[i][g], (ok >> i) & 1u);
@@ -959,11 +965,11 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // 1.6 .. 2.0 GHz by their power, and a launch that wastes less time runs at a lower clock.)
   const auto in_terms = std::true_type();
   constexpr bool WOVEN = X3 && NBUF == 2 && !UP && UPC >= NLD + 3;
-  constexpr int TRASH = IT * LS;                             // behind the pixels of row 0: where slots that do not exist go
-  static_assert(!WOVEN || RP - IT * LS >= EPS, "room for a slot in the row padding");
+  constexpr int TRASH = ROOM ? IT * LS : IT * RP;            // behind the pixels of row 0, or behind the rows: where slots that do not exist go
+  static_assert(!WOVEN || TRASH + EPS <= STAGE, "room for a slot");
   int st_at[NLD];
 #pragma unroll
-  for (int i = 0; i < NLD; ++i) st_at[i] = tid + 256 * i < NSLOT ? st_lds[i] : TRASH;
+  for (int i = 0; i < NLD; ++i) st_at[i] = tid + TH * i < NSLOT ? st_lds[i] : TRASH;
   unsigned ok_n = 0u;                                        // which slots of the chunk in st_reg count
   auto load_raw = [&](int c, bool first = false) __attribute__((always_inline)) {
     const bool second = c >= nch1;
@@ -1054,7 +1060,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   // the output pixel mask of this thread's groups (or items of the gate chain, with their previous-cell masks): asked for
   // behind the first loads, taken behind their barrier
   constexpr int HG = CO_BLK / (GRU ? 8 : 16);                // groups of four hidden channels
-  constexpr int PERG = (64 * HG + 255) / 256;                // items per thread (the 32-column slab has 128: half the threads idle)
+  constexpr int PERG = (64 * HG + TH - 1) / TH;                // items per thread (the 32-column slab has 128: half the threads idle)
   constexpr int NLIVE = GATES ? PERG : PER;
   const uint8_t* const live_m = a.refresh ? nullptr : a.ts.pixmask;
   const uint8_t* const cp_m = GATES && !GRU && a.g_cpd != nullptr ? a.g_cpm : nullptr;
@@ -1063,7 +1069,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     int at[NLIVE];
 #pragma unroll
     for (int g = 0; g < NLIVE; ++g) {
-      const int idx = tid + 256 * g, p = GATES ? idx / HG : idx / QPP;
+      const int idx = tid + TH * g, p = GATES ? idx / HG : idx / QPP;
       const int oy = y0 + (p >> 3), ox = x0 + (p & 7);
       const bool k = p < 64 && oy < hout && ox < wout;
       at[g] = k ? (n * hout + oy) * wout + ox : 0;
@@ -1287,13 +1293,13 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
   auto meet = [&]() __attribute__((always_inline)) {
     park();
     if constexpr (F2) {
-      if (groups.misfit() || !filt_fits) s_f2[4] = 1.f;
+      if (groups.misfit() || !filt_fits) s_f2[WAVES] = 1.f;
     }
     __syncthreads();
     if constexpr (F2) {
       // a group that does not fit: all of it once more, on the fp32 instruction, as plainly as it can be said.  (Every workgroup of 3x3
       // 256->256 at 33x44: 41 us instead of 13.5, three bf16 terms 17.5; 64->64 at 132x176: 33, 14.3 and 17.6)
-      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[WAVES])) != 0, 0)) {
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -1339,7 +1345,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     long long ho[PERG];
 #pragma unroll
     for (int i = 0; i < PERG; ++i) {
-      const int idx = tid + 256 * i, p = idx / HG, g4 = idx - p * HG;
+      const int idx = tid + TH * i, p = idx / HG, g4 = idx - p * HG;
       ho[i] = (((long long)n * hout + y0 + (p >> 3)) * wout + x0 + (p & 7)) * a.hid + co0 / 2 + 4 * g4;
       const long long at = ((live_bits >> i) & 1u) ? ho[i] : 0;
       ru[i] = *reinterpret_cast<const float4*>(a.res + at);
@@ -1353,7 +1359,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
         mie_st4(a.g_dh, ho[i], make_float4(0.f, 0.f, 0.f, 0.f));
         continue;
       }
-      const int idx = tid + 256 * i, p = idx / HG, g4 = idx - p * HG;
+      const int idx = tid + TH * i, p = idx / HG, g4 = idx - p * HG;
       float4 dg[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -1383,7 +1389,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     long long ho[PERG], go[PERG];
 #pragma unroll
     for (int i = 0; i < PERG; ++i) {
-      const int idx = tid + 256 * i, p = idx / HG, g4 = idx - p * HG;
+      const int idx = tid + TH * i, p = idx / HG, g4 = idx - p * HG;
       const long long pix = ((long long)n * hout + y0 + (p >> 3)) * wout + x0 + (p & 7);
       ho[i] = pix * a.hid + co0 / 4 + 4 * g4;
       go[i] = pix * a.cout + co0 + 16 * g4;
@@ -1393,7 +1399,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
 #pragma unroll
     for (int i = 0; i < PERG; ++i) {
       if (!((live_in >> i) & 1u)) continue;
-      const int idx = tid + 256 * i, p = idx / HG, g4 = idx - p * HG;
+      const int idx = tid + TH * i, p = idx / HG, g4 = idx - p * HG;
       float4 dg[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -1417,7 +1423,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
       float4 v[PB];
 #pragma unroll
       for (int i = 0; i < PB; ++i) {
-        const int idx = tid + 256 * (h0 + i);      // group idx: pixel idx / QPP, channels 4 * (idx % QPP) ...
+        const int idx = tid + TH * (h0 + i);      // group idx: pixel idx / QPP, channels 4 * (idx % QPP) ...
         float4 sum = *reinterpret_cast<const float4*>(&smem[4 * idx]);
 #pragma unroll
         for (int k2 = 1; k2 < WK; ++k2) {
@@ -1446,7 +1452,7 @@ __global__ __launch_bounds__(256, conv_min_waves((int)sizeof(T), K, S, HALF, GAT
     if constexpr (AGAIN) {
       if (__builtin_expect(__ballot(bad_bits != 0u) != 0ull, 0))
         for (int g = 0; g < PER; ++g) {
-          const int idx = tid + 256 * g, p = idx / QPP, co = co0 + 4 * (idx - p * QPP);
+          const int idx = tid + TH * g, p = idx / QPP, co = co0 + 4 * (idx - p * QPP);
           if ((bad_bits >> g) & 1u) conv_quad_again<T, K, S>(conv_args_again<T>(), n, y0 + (p >> 3), x0 + (p & 7), co);
         }
     }
@@ -1815,6 +1821,18 @@ inline bool x3_takes(int k, int s, int c1, int c2, int cout) {
   return (k == 3 || k == 5) && s == 1 && c1 % 32 == 0 && c2 % 32 == 0 && cout % 32 == 0;
 }
 
+// Two terms: eight waves a workgroup, chunks of twice the channels (WIDE).  Where the workgroups are one round of the chip, one a CU, a CU has one
+// wave a SIMD with four, and nothing runs while it waits.  us, four waves -> eight, every tile active, filters cold: 3x3 256->256 at 33x44
+// (240 workgroups) 12.4 -> 12.05, 256->512 there 17.3 -> 16.7; 5x5 stride 2 (which is then double-buffered, too) 128->256 at 66x88 18.4 -> 15.4,
+// 64->128 at 80x100 11.6 -> 10.5.  (What is left of a 3x3 layer: a third is its head and tail, the rest runs at 0.8 of what the L1 delivers
+// of filter and input.)  Not for fewer channels: 3x3 64->64 at 66x88 6.9 and 7.2.  A second round of such workgroups is no better than
+// two of four waves a CU side by side (5x5 stride 2 64->128 at 132x176, 64 columns wide so that it is one: 15.7 and 14.7 alone, a frame the same);
+// the ConvGRU's gates, likewise, the same.  Frame of 264x352 342 -> 335 us, planned ahead 328 -> 320, refresh 386 -> 378.
+inline bool f2_wide(const ConvArgsT<float>& a, unsigned cap, int slab, int s) {
+  const int chunk = s == 2 ? 32 : 64;
+  return slab != 0 && (long long)cap * (a.cout / slab) <= 256 && a.c1 % chunk == 0 && a.c2 % chunk == 0 && a.c1 + a.c2 >= (s == 2 ? 64 : 256);
+}
+
 template <int AR, int K, bool GATES, bool UP, int S>
 bool launch_terms(const ConvArgsT<float>& a0, unsigned cap, hipStream_t st) {
   ConvArgsT<float> a = a0;
@@ -1827,7 +1845,17 @@ bool launch_terms(const ConvArgsT<float>& a0, unsigned cap, hipStream_t st) {
       return true;
     }
   }
-  switch (pick_slab_x3(cout, cap, S)) {
+  const int slab = pick_slab_x3(cout, cap, S);
+  if constexpr (AR == 2 && !UP && (K == 3 || S == 2)) {
+    if (f2_wide(a, cap, slab, S)) {
+      const dim3 grid(xcd_plan(a, cap, cout / slab, K, UP), cout / slab);
+      if (slab == 128) hipLaunchKernelGGL((k_conv_mfma<float, K, S, 4, 1, false, GATES, UP, false, AR, false, false, true>), grid, dim3(512), 0, st, a);
+      else if (slab == 64) hipLaunchKernelGGL((k_conv_mfma<float, K, S, 2, 1, false, GATES, UP, false, AR, false, false, true>), grid, dim3(512), 0, st, a);
+      else hipLaunchKernelGGL((k_conv_mfma<float, K, S, 1, 1, false, GATES, UP, false, AR, false, false, true>), grid, dim3(512), 0, st, a);
+      return true;
+    }
+  }
+  switch (slab) {
     case 128:
       hipLaunchKernelGGL((k_conv_mfma<float, K, S, 4, 1, false, GATES, UP, false, AR>), dim3(xcd_plan(a, cap, cout / 128, K, UP), cout / 128), dim3(256), 0, st, a);
       return true;

@@ -72,6 +72,8 @@ def _conv(x, wt, k, stride, mode, c1=None, xm=None, path=_lib.PATH_MFMA, workspa
 SHAPES = [(32, 32, 3, 1, 136, 130, None), (64, 64, 3, 1, 70, 75, None), (128, 128, 3, 1, 41, 47, 64), (256, 256, 3, 1, 33, 44, None),
           (256, 512, 3, 1, 34, 39, 128), (64, 32, 5, 1, 33, 47, None), (128, 128, 5, 1, 34, 42, None), (32, 64, 5, 2, 131, 133, None),
           (128, 256, 5, 2, 66, 88, None), (1024, 256, 3, 1, 17, 9, None), (256, 32, 5, 1, 16, 16, None), (512, 64, 5, 2, 17, 16, 256),
+          # eight waves a workgroup (up to 256 of them): slabs of 32, 64 and 128, two and many chunks; inputs that are no whole chunks of it
+          (64, 128, 5, 2, 80, 100, None), (96, 128, 5, 2, 79, 101, 32), (512, 1024, 3, 1, 30, 44, 256), (320, 256, 3, 1, 33, 47, 64), (256, 256, 3, 1, 33, 44, 96),
           # the one-launch form from 512 channels on: two, four and eight rows a workgroup, waves of two and three chunks
           (512, 64, 3, 1, 7, 9, None), (512, 64, 3, 1, 16, 24, 192), (576, 128, 3, 1, 24, 20, None), (512, 128, 3, 1, 31, 33, 256)]
 
