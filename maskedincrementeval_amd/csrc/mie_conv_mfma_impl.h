@@ -1825,12 +1825,13 @@ inline bool x3_takes(int k, int s, int c1, int c2, int cout) {
 // wave a SIMD with four, and nothing runs while it waits.  us, four waves -> eight, every tile active, filters cold: 3x3 256->256 at 33x44
 // (240 workgroups) 12.4 -> 12.05, 256->512 there 17.3 -> 16.7; 5x5 stride 2 (which is then double-buffered, too) 128->256 at 66x88 18.4 -> 15.4,
 // 64->128 at 80x100 11.6 -> 10.5.  (What is left of a 3x3 layer: a third is its head and tail, the rest runs at 0.8 of what the L1 delivers
-// of filter and input.)  Not for fewer channels: 3x3 64->64 at 66x88 6.9 and 7.2.  A second round of such workgroups is no better than
+// of filter and input.)  Not for fewer channels: 3x3 64->64 at 66x88 6.9 and 7.2; nor for slabs of 128
+// columns, whose four waves are busy as they are (gates of 256+256 at 33x44 31 and 33 in a trace, frames the same).  A second round of such workgroups is no better than
 // two of four waves a CU side by side (5x5 stride 2 64->128 at 132x176, 64 columns wide so that it is one: 15.7 and 14.7 alone, a frame the same);
 // the ConvGRU's gates, likewise, the same.  Frame of 264x352 342 -> 335 us, planned ahead 328 -> 320, refresh 386 -> 378.
 inline bool f2_wide(const ConvArgsT<float>& a, unsigned cap, int slab, int s) {
   const int chunk = s == 2 ? 32 : 64;
-  return slab != 0 && (long long)cap * (a.cout / slab) <= 256 && a.c1 % chunk == 0 && a.c2 % chunk == 0 && a.c1 + a.c2 >= (s == 2 ? 64 : 256);
+  return (slab == 32 || slab == 64) && (long long)cap * (a.cout / slab) <= 256 && a.c1 % chunk == 0 && a.c2 % chunk == 0 && a.c1 + a.c2 >= (s == 2 ? 64 : 256);
 }
 
 template <int AR, int K, bool GATES, bool UP, int S>
@@ -1849,8 +1850,7 @@ bool launch_terms(const ConvArgsT<float>& a0, unsigned cap, hipStream_t st) {
   if constexpr (AR == 2 && !UP && (K == 3 || S == 2)) {
     if (f2_wide(a, cap, slab, S)) {
       const dim3 grid(xcd_plan(a, cap, cout / slab, K, UP), cout / slab);
-      if (slab == 128) hipLaunchKernelGGL((k_conv_mfma<float, K, S, 4, 1, false, GATES, UP, false, AR, false, false, true>), grid, dim3(512), 0, st, a);
-      else if (slab == 64) hipLaunchKernelGGL((k_conv_mfma<float, K, S, 2, 1, false, GATES, UP, false, AR, false, false, true>), grid, dim3(512), 0, st, a);
+      if (slab == 64) hipLaunchKernelGGL((k_conv_mfma<float, K, S, 2, 1, false, GATES, UP, false, AR, false, false, true>), grid, dim3(512), 0, st, a);
       else hipLaunchKernelGGL((k_conv_mfma<float, K, S, 1, 1, false, GATES, UP, false, AR, false, false, true>), grid, dim3(512), 0, st, a);
       return true;
     }
