@@ -595,8 +595,16 @@ class NetBench:
         return roofline
 
     def _products(self, layer):
-        """Term products per multiply of a launch that ran in terms (decoders at the resolution of their inputs: six)."""
-        return 6 if self.ops.f32_matmul == "bf16x3" or layer["op"].startswith("upconv2x") else 3
+        """Term products per multiply of a launch that ran in terms (decoders at the resolution of their inputs: three or six)."""
+        import re
+        if self.ops.f32_matmul == "bf16x3":
+            return 6
+        m = re.search(r"(\d+)->(\d+) @(?:(\d+)x)?(\d+)x(\d+)", layer["shape"])
+        if not layer["op"].startswith("upconv2x") or m is None:
+            return 3
+        from maskedincrementeval_amd._lib import lib
+        c, cout, n, h, w = (int(v or 1) for v in m.groups())
+        return 3 if lib().mie_f16x2_takes_upconv2x(n, h // 2, w // 2, c, cout) else 6
 
     def _takes_x3(self, layer):
         """Whether the launch of a per-launch table row ran in terms (its shape string is
