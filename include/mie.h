@@ -90,8 +90,8 @@ extern "C" {
 /* The same with two fp16 terms and three term products: value * scale = hi + lo, the scale a power of two that a
  * workgroup takes from its own input (and mie_pack_filter from the weights), 23 bits of every value.  Half the matrix
  * instructions of MIE_DTYPE_F32_BF16X3, and less error against fp64 (fewer roundings at the size of the sum).  Where a
- * workgroup's input does not lie within fp16's range of its scale -- groups of eight channels of a pixel 2^23 below the largest value
- * or 2^6 above it, infinities, NaN -- it contracts in fp32 instead, as for MIE_DTYPE_F32, from a copy of the filter
+ * workgroup's input does not lie within fp16's range of its scale -- groups of eight channels of a pixel 2^24 below the largest value it was taken from
+ * or eight times that value, infinities, NaN -- it contracts in fp32 instead, as for MIE_DTYPE_F32, from a copy of the filter
  * that the packed one holds too: correct, and slower.  Forms that add up the products of three terms more finely than that -- those
  * without a workspace on planes of few tiles, but for the 3x3 stride-1 convs of 512 channels and more, and the transposed convs on planes
  * of few blocks -- keep the three (the packed copy holds them as well).

@@ -216,8 +216,9 @@ __device__ __forceinline__ void split3(const float (&f)[8], float4 (&pl)[3]) {
 // against fp64, relative 2-norm, of 288 / 1152 / 4608 terms in four chains 1.05 / 1.40 / 2.33e-7, three bf16 terms 1.09 / 1.89 /
 // 3.70e-7.
 // The price is fp16's range.  A workgroup takes s from the largest value of its first chunk (of both inputs'), which goes to [2^12, 2^13),
-// so that a value is held to 2^-23 of itself or 2^-48 of that largest one, whichever is more: within 2^26 of it nothing is lost.  The largest
-// of every eight staged channels of a pixel has to lie below 65000 and not below 2^-24, where 11 bits are left of it, or be zero.
+// so that a value is held to 2^-23 of itself or 2^-48 of that largest one, whichever is more.  The largest of every eight staged channels of a
+// pixel has to lie below 65000 and not below 2^-12, or be zero: outputs that such groups alone make up are then no further from fp64 than three
+// terms (norm of the error of 2304 terms, groups at 2^-12 .. -14: 2.4, 2.6, 3.5e-7, three terms 3.7e-7, far above it 2.3e-7).
 // Where one does not, infinities and NaN included, the workgroup does its contraction over on v_mfma_f32_32x32x2_f32, from the
 // same places of LDS and of a second, fp32, copy of the filter.  Over the networks' steps the largest value of a window was up to 3.5 times
 // its first chunk's, and such groups lay within 2^24 of it but for a few tiles of a recurrent state fed back (within 2^30, 2 tiles of 4767
@@ -275,7 +276,7 @@ struct F2Groups {
     split2(f, scale, pl);
   }
   __device__ __forceinline__ bool misfit() const {      // (the scale's exponent taken off the bounds)
-    const unsigned k = __float_as_uint(scale) - (127u << 23), lo = (127u - 24u) << 23, hi = 0x477de800u;      // 2^-24, 65000
+    const unsigned k = __float_as_uint(scale) - (127u << 23), lo = (127u - 12u) << 23, hi = 0x477de800u;      // 2^-12, 65000
     return most > hi - k || least < lo - k - 1u;
   }
 };

@@ -239,3 +239,70 @@ def test_transposed_convs(c1, c2, cout, h, w, k, what, setting):
     assert ((got["f16x2"] - ref).abs() <= 4e-7 * bound)[fine].all(), ((got["f16x2"] - ref).abs() / bound)[fine].max()
     if what == "fits":
         assert (got["f16x2"] - ref).norm() <= (got["bf16x3"] - ref).norm()
+
+
+def _halves(x, factor):
+    """The lower half of the plane `factor` times the upper one: outputs far enough down see small values only, in workgroups that
+    see the large ones too."""
+    return x * torch.where(torch.arange(x.shape[2]) < x.shape[2] // 2, 1.0, factor).view(1, 1, -1, 1)
+
+
+# (from where the two terms hold all of a value to far behind where they hold nothing; 4e-7, 6e-7 as in the tests above)
+FACTORS = [2.0 ** -22, 2.0 ** -24, 1e-8, 1e-9, 1e-10, 1e-11, 2.0 ** -40]
+
+
+@pytest.mark.parametrize("cin,cout,k,stride,h,w,c1", SHAPES)
+def test_no_digits_lost_below_the_largest_value(cin, cout, k, stride, h, w, c1, setting):
+    g = torch.Generator().manual_seed(cin + w)
+    x0, wt = torch.randn(1, cin, h, w, generator=g), he_normal_conv_weight(cout, cin, k, 7)
+    for factor in FACTORS:
+        x = _halves(x0, factor)
+        ref = F.conv2d(x.double(), wt.double(), stride=stride, padding=k // 2)
+        bound = F.conv2d(x.double().abs(), wt.double().abs(), stride=stride, padding=k // 2)
+        e = (_conv(x, wt, k, stride, "f16x2", c1) - ref).abs()
+        assert (e <= 4e-7 * bound).all(), (factor, (e / bound).max())
+
+
+@pytest.mark.parametrize("c,cout,h,w,two", [(128, 64, 66, 88, True), (256, 128, 33, 44, True), (256, 64, 9, 11, False), (64, 32, 72, 123, True), (96, 64, 63, 66, False)])
+def test_no_digits_lost_below_the_largest_value_decoders(c, cout, h, w, two, setting):
+    g = torch.Generator().manual_seed(c + w)
+    a0, b0, wt = torch.randn(1, c, h, w, generator=g), torch.randn(1, c, h, w, generator=g), he_normal_conv_weight(cout, c, 5, 7)
+    up = lambda t: F.interpolate(t.double(), scale_factor=2, mode="bilinear", align_corners=False)      # noqa: E731
+    for factor in FACTORS:
+        a, b = _halves(a0, factor), _halves(b0, factor)
+        s, size = (a + b, a.abs() + b.abs()) if two else (a, a.abs())
+        ref, bound = F.conv2d(up(s), wt.double(), padding=2), F.conv2d(up(size), wt.double().abs(), padding=2)
+        e = (_up2x(a, b if two else None, wt, "f16x2") - ref).abs()
+        assert (e <= 6e-7 * bound).all(), (factor, (e / bound).max())
+
+
+def _tconv(x, c1, wt, k, mode):
+    (_, cin, h, w), cout = x.shape, wt.shape[1]
+    filt = ops.ConvFilter(wt.permute(0, 2, 3, 1).contiguous().to(DEV))
+    ts, blocks = TileMask(1, 2 * h, 2 * w, DEV), TileMask(1, h, w, DEV)
+    ops.build_mask_tiles(None, None, 1, h, w, _lib.FOOT_TCONV, k, 2, k // 2, ts)
+    ops.build_mask_tiles(ts, None, 1, 2 * h, 2 * w, _lib.FOOT_CONV, 2, 2, 0, blocks)
+    ops.f32_matmul = mode
+    out = ops.new_nhwc(1, cout, 2 * h, 2 * w, DEV)
+    ops.tconv2x_masked(_dev(x[:, :c1]), None, _dev(x[:, c1:]) if c1 < cin else None, None, filt, k, ts, blocks, out)
+    torch.cuda.synchronize()
+    return out.cpu().double()
+
+
+def _tconv_ref(x, wt, k):
+    up = lambda x_, w_: F.conv_transpose2d(x_, w_, stride=2, padding=k // 2, output_padding=1)      # noqa: E731
+    return up(x.double(), wt.double()), up(x.double().abs(), wt.double().abs())
+
+
+TCONVS = [(64, 64, 32, 127, 131, 3), (128, 0, 64, 132, 176, 3), (1024, 512, 64, 8, 7, 3), (64, 64, 32, 90, 93, 5)]
+
+
+@pytest.mark.parametrize("c1,c2,cout,h,w,k", TCONVS)
+def test_no_digits_lost_below_the_largest_value_transposed(c1, c2, cout, h, w, k, setting):
+    g = torch.Generator().manual_seed(c1 + w)
+    x0, wt = torch.randn(1, c1 + c2, h, w, generator=g), torch.randn(c1 + c2, cout, k, k, generator=g) * (8.0 / ((c1 + c2) * k * k)) ** 0.5
+    for factor in FACTORS:
+        x = _halves(x0, factor)
+        ref, bound = _tconv_ref(x, wt, k)
+        e = (_tconv(x, c1, wt, k, "f16x2") - ref).abs()
+        assert (e <= 4e-7 * bound).all(), (factor, (e / bound).max())
