@@ -257,10 +257,12 @@ __device__ __forceinline__ float f2_wave_max(float m) {
   step(std::integral_constant<int, 0x142>()); step(std::integral_constant<int, 0x143>());      // row_bcast 15, 31
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), 63));
 }
-// The scale for values whose largest is m (anything: what does not fit is found later).
+// The scale for values whose largest is m (anything: what does not fit is found later).  Zeros tell nothing of what follows: F2_BLANK, which
+// values above 2^-57 do not fit.
+constexpr float F2_BLANK = 9444732965739290427392.f;      // 2^73
 __device__ __forceinline__ float f2_scale(float m) {
   int e = (__float_as_int(m) >> 23) - 127;
-  e = m == 0.f ? 12 : e < -60 ? -60 : e > 52 ? 52 : e;
+  e = m == 0.f ? -61 : e < -60 ? -60 : e > 52 ? 52 : e;
   return __int_as_float((127 + 12 - e) << 23);
 }
 __device__ __forceinline__ float f2_unscale(float s) { return __int_as_float((254 << 23) - __float_as_int(s)); }      // 1 / s
@@ -1263,7 +1265,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   // acc[mb][nb][r] of this lane is output pixel p = 32*mb + 8*(r/4) + 4*half + r%4,
   // channel column wn*32*NB + 32*nb + lane%32 of the workgroup's slab.
   if constexpr (F2) {
-    const float c0 = f2_unscale(groups.scale) * filt_unscale, c1 = c0 * (1.f / F2_STEP);      // exactly: powers of two, 2^-143 at the least
+    const float c0 = f2_unscale(groups.scale) * filt_unscale, c1 = c0 * (1.f / F2_STEP);      // exactly: powers of two, 2^-143 at the least but for sums of zeros
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll

@@ -325,7 +325,7 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
   }
   float c0 = 1.f;                      // F2: 1 / scales
   if constexpr (F2) {
-    c0 = f2_unscale(groups.scale) * filt_unscale;      // exactly: powers of two, 2^-143 at the least
+    c0 = f2_unscale(groups.scale) * filt_unscale;      // exactly: powers of two, 2^-143 at the least but for sums of zeros
     // a group that does not fit: all of it once more on the fp32 instruction, from the fp32 copy of the filter behind the terms
     if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
 #pragma unroll

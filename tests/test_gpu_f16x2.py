@@ -306,3 +306,46 @@ def test_no_digits_lost_below_the_largest_value_transposed(c1, c2, cout, h, w, k
         ref, bound = _tconv_ref(x, wt, k)
         e = (_tconv(x, c1, wt, k, "f16x2") - ref).abs()
         assert (e <= 4e-7 * bound).all(), (factor, (e / bound).max())
+
+
+def _leading_zero(x, c1, scale):
+    """`scale` times x with the leading channels of each input zero, up to half of them: the chunks that a scale is first taken from."""
+    x = x * scale
+    for lo, hi in ((0, c1), (c1, x.shape[1])):
+        x[:, lo:lo + min(64, (hi - lo) // 2)] = 0.0
+    return x
+
+
+@pytest.mark.parametrize("cin,cout,k,stride,h,w,c1", SHAPES)
+def test_leading_channels_zero(cin, cout, k, stride, h, w, c1, setting):
+    g = torch.Generator().manual_seed(cin + 5)
+    x0, wt = torch.randn(1, cin, h, w, generator=g), he_normal_conv_weight(cout, cin, k, 7)
+    for scale in (1e-4, 1e-5, 1e-6, 1e-7):
+        x = _leading_zero(x0, cin if c1 is None else c1, scale)
+        ref = F.conv2d(x.double(), wt.double(), stride=stride, padding=k // 2)
+        bound = F.conv2d(x.double().abs(), wt.double().abs(), stride=stride, padding=k // 2)
+        e = (_conv(x, wt, k, stride, "f16x2", c1) - ref).abs()
+        assert (e <= 4e-7 * bound).all(), (scale, (e / bound).max())
+
+
+@pytest.mark.parametrize("c,cout,h,w", [(128, 64, 66, 88), (256, 128, 33, 44), (64, 32, 72, 123), (96, 64, 63, 66)])
+def test_leading_channels_zero_decoders(c, cout, h, w, setting):
+    g = torch.Generator().manual_seed(c + 5)
+    a0, wt = torch.randn(1, c, h, w, generator=g), he_normal_conv_weight(cout, c, 5, 7)
+    up = lambda t: F.interpolate(t.double(), scale_factor=2, mode="bilinear", align_corners=False)      # noqa: E731
+    for scale in (1e-4, 1e-5, 1e-6, 1e-7):
+        a = _leading_zero(a0, c, scale)
+        ref, bound = F.conv2d(up(a), wt.double(), padding=2), F.conv2d(up(a.abs()), wt.double().abs(), padding=2)
+        e = (_up2x(a, None, wt, "f16x2") - ref).abs()
+        assert (e <= 6e-7 * bound).all(), (scale, (e / bound).max())
+
+
+@pytest.mark.parametrize("c1,c2,cout,h,w,k", TCONVS)
+def test_leading_channels_zero_transposed(c1, c2, cout, h, w, k, setting):
+    g = torch.Generator().manual_seed(c1 + 5)
+    x0, wt = torch.randn(1, c1 + c2, h, w, generator=g), torch.randn(c1 + c2, cout, k, k, generator=g) * (8.0 / ((c1 + c2) * k * k)) ** 0.5
+    for scale in (1e-4, 1e-5, 1e-6, 1e-7):
+        x = _leading_zero(x0, c1, scale)
+        ref, bound = _tconv_ref(x, wt, k)
+        e = (_tconv(x, c1, wt, k, "f16x2") - ref).abs()
+        assert (e <= 4e-7 * bound).all(), (scale, (e / bound).max())
