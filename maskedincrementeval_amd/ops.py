@@ -914,7 +914,8 @@ upconv2x_enabled = os.environ.get("MIE_UPCONV2X", "1") != "0"      # tuning knob
 def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt, refresh=False) -> bool:
     """Whether a decoder layer over `a` runs at the resolution of its inputs: upconv2x_masked has a kernel for it and is the
     faster form where all tiles are active (nnConvIncr._upconv_forward asks for that first).  It is not on planes so small that upconv_masked splits the contraction (256->128 at 16x16: 25 us against
-    22, at 20x20 26 against 35), for bf16 layers of one staged chunk on planes of few blocks (mie_all_phases_upconv2x: 64->32 at 96x96 13.6 us against 13.3), and where border strips and blocks filled in part undo the fewer taps: 16 for each of the four
+    22, at 20x20 26 against 35), for bf16 layers of one staged chunk, whose a + b upconv_masked holds in 32 bits up to the blend (this form rounds it to
+    bf16; on planes of few blocks it is not the faster one either: 64->32 at 96x96 13.6 us against 13.3), and where border strips and blocks filled in part undo the fewer taps: 16 for each of the four
     phases of an item against 25 for each tile, once that is more than a round of workgroups (256->128 at 8x19x23: 138
     us against 123).  Nor, but for a refresh, where upconv_masked has its form for planes of few tiles (fp32 128->64 at 32x48 15.0 us
     against 11.4, 64->32 at 64x64 10.3 against 7.8; bf16 9.8 against 6.8 and 7.4 against 5.4), in bf16 on all such planes, also where the
@@ -933,7 +934,7 @@ def upconv2x_takes(a, cout: int, k: int, stride: int, pad: int, filt, refresh=Fa
     items = n * (-(-(h - 2) // 8) * -(-(w - 2) // 8) + 2 * -(-w // 32) + 2 * -(-(h - 2) // 32))
     if (c >= 4 * chunk and tiles * slabs <= 64) or (4 * items * slabs > 256 and 4 * 16 * items > 25 * tiles):
         return False
-    return a.dtype != torch.bfloat16 or c > chunk or bool(lib().mie_all_phases_upconv2x(n, h, w, c, cout, _lib.DTYPE_BF16))
+    return not (a.dtype == torch.bfloat16 and c == chunk)
 
 
 def _upconv2x_args(a, b, filt, out_ts, out, reservoir, addend):

@@ -266,3 +266,11 @@ def test_decoder_conv_of_one_chunk_on_many_blocks(n, c, cout, h, w):
     assert _lib.lib().mie_all_phases_upconv2x(n, h, w, c, cout, _lib.DTYPE_BF16)
     test_decoder_conv_at_input_resolution(n, c, cout, h, w, torch.bfloat16)
     test_pixels_outside_the_mask_keep_their_reservoir(n, c, cout, h, w, torch.bfloat16, "blocks")
+
+
+# ... whose layers a network does not take there: upconv_masked holds a + b in 32 bits up to the blend, this form rounds it to bf16
+@pytest.mark.parametrize("n,cout,h,w", [(2, 32, 100, 140), (1, 96, 75, 74), (8, 32, 240, 320)])
+def test_decoders_of_one_chunk_keep_the_sum_of_their_inputs_in_32_bits(n, cout, h, w):
+    filt = ops.ConvFilter(torch.zeros(64, 5, 5, cout, device=DEV))
+    for refresh in (False, True):
+        assert not ops.upconv2x_takes(torch.empty((n, 64, h, w), dtype=torch.bfloat16), cout, 5, 1, 2, filt, refresh)
