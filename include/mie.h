@@ -91,8 +91,10 @@ extern "C" {
  * workgroup takes from its own input (and mie_pack_filter from the weights), 23 bits of every value.  Half the matrix
  * instructions of MIE_DTYPE_F32_BF16X3, and less error against fp64 (fewer roundings at the size of the sum).  Where a
  * workgroup's input does not lie within fp16's range of its scale -- groups of eight channels of a pixel 2^24 below the largest value it was taken from
- * or eight times that value, infinities, NaN -- it contracts in fp32 instead, as for MIE_DTYPE_F32, from a copy of the filter
- * that the packed one holds too: correct, and slower.  Forms that add up the products of three terms more finely than that -- those
+ * or eight times that value -- or the filter's groups of eight do not lie within 2^29 of its largest weight, it goes on in three
+ * bf16 terms from that chunk of channels on, from a copy of the filter that the packed one holds too, in 1.05 to 1.6 times the time of
+ * MIE_DTYPE_F32_BF16X3; from 2^127 on, infinities and NaN, as for MIE_DTYPE_F32.  (Small values beside large ones in their group of eight are
+ * held to 2^-24, weights to 2^-22, of that group's largest.)  Forms that add up the products of three terms more finely than that -- those
  * without a workspace on planes of few tiles, but for the 3x3 stride-1 convs of 512 channels and more, and the transposed convs on planes
  * of few blocks -- keep the three (the packed copy holds them as well).
  * Taken, for the same shapes, wherever MIE_DTYPE_F32_BF16X3 is. */

@@ -122,7 +122,8 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   static_assert(!UP || (K == 5 && S == 1), "the up-sampling variant is the 5x5 stride-1 conv");
   static_assert(!F2 || (K == 3 && S == 1 && !UP), "two terms: the 3x3 convs");
   __shared__ __attribute__((aligned(16))) char smem[D::BYTES];
-  __shared__ float s_f2[F2 && !OWN ? DEEP_WAVES + 1 : 1];      // largest values of the waves' slots; whether a group does not fit
+  __shared__ float s_f2[F2 && !OWN ? DEEP_WAVES + 2 : 1];      // largest values of the waves' slots; whether a group of a pass does not fit, of
+                                                               // every other one in the same place
   mie_bf16* const win = reinterpret_cast<mie_bf16*>(smem);
   float* const s_lo = reinterpret_cast<float*>(smem + D::WIN_B);
   float* const park = reinterpret_cast<float*>(smem);
@@ -243,7 +244,6 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   };
   auto kept = [](const float4& v, bool k) { return make_float4(k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f); };
   F2Groups groups;
-  bool misfit = false;
   auto put = [&](int at, const float (&f)[8], auto terms) {
     if constexpr (F2) {
       float4 pl[2] = {make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7])};
@@ -262,10 +262,11 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   unsigned ok1 = 0u, ok2 = 0u;
   const int st_c = ck * (PL * STAGE) + q8;      // this thread's place in a staged pixel
   // F2: the scale of a pass, a wave's own (OWN) or the workgroup's
-  auto scale_of = [&](float m) {
+  auto scale_of = [&](int pass, float m) {
     m = f2_wave_max(m);
     if constexpr (!OWN) {
       if (lane == 0) s_f2[wave] = m;
+      if (pass == 0 && tid < 2) s_f2[DEEP_WAVES + tid] = 0.f;
       __syncthreads();
       m = f2_wave_max(s_f2[lane & (DEEP_WAVES - 1)]);
     }
@@ -333,7 +334,7 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
           const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
           m = __builtin_elementwise_maximum(m, (ok >> i) & 1u ? f2_amax8(f) : 0.f);
         }
-        scale_of(m);
+        scale_of(pass, m);
       }
 #pragma unroll
       for (int i = 0; i < NL; ++i) {
@@ -387,12 +388,12 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
   v4acc acc[MB], sm[MB], sl[MB];      // fp32: products of 1, 2^-8 and 2^-16 of the largest; F2: of 1 and 2^-11, and the totals' small part
   v4acc tot[F2 ? MB : 1];
   float c0 = 1.f, filt_unscale = 1.f;
-  bool filt_fits = true;
+  bool unfit = false;
   const long long weights = (long long)a.cin_total * (K * K) * cout;
   if constexpr (F2) {
     const float* const end = f2_filter_end(a.filt_mc, weights);
     filt_unscale = end[0];
-    filt_fits = end[1] != 0.f;
+    unfit = end[1] != 1.f;
 #pragma unroll
     for (int b = 0; b < MB; ++b) tot[b] = v4acc{0.f, 0.f, 0.f, 0.f};
   }
@@ -446,55 +447,55 @@ __global__ __launch_bounds__(DEEP_THREADS) void k_conv_deep(ConvArgsT<T> a) {
       }
     }
   };
+  int unfit_pass = unfit ? 0 : nch;      // F2: the first pass that does not fit
   for (int pass = 0, c = cg; pass * NCW < nch; ++pass, c += NCW) {
     if (!OWN && pass > 0) __syncthreads();
     store_x(pass, std::true_type());
     if constexpr (F2) {
-      misfit = misfit || groups.misfit();
+      if constexpr (OWN) unfit_pass = __ballot(groups.misfit()) != 0ull && pass < unfit_pass ? pass : unfit_pass;
+      else if (groups.misfit()) s_f2[DEEP_WAVES + (pass & 1)] = 1.f;
       c0 = f2_unscale(groups.scale) * filt_unscale;
     }
     if constexpr (OWN) mie_wave_order();
     else __syncthreads();
+    if constexpr (F2) {
+      if (!OWN && __builtin_amdgcn_readfirstlane(__float_as_int(s_f2[F2 && !OWN ? DEEP_WAVES + (pass & 1) : 0])) != 0) unfit_pass = pass < unfit_pass ? pass : unfit_pass;
+      if (__builtin_expect(unfit_pass <= pass, 0)) break;
+    }
     if ((pass + 1) * NCW < nch) load_x(pass + 1);
     if (c + NCW < nch) chunk(chunk_w(c + NCW), std::true_type());
     else if (c < nch) chunk(nullptr, std::false_type());
     if constexpr (OWN) mie_wave_order();
   }
   if constexpr (F2) {
-    // a group that does not fit: all the sums of the wave (OWN) or the workgroup once more, on the fp32 instruction from the fp32 copy of the
-    // filter behind the terms
-    bool again = __ballot(misfit || !filt_fits) != 0ull;
-    if constexpr (!OWN) {
-      if (tid == 0) s_f2[DEEP_WAVES] = 0.f;
-      __syncthreads();
-      if (again && lane == 0) s_f2[DEEP_WAVES] = 1.f;
-      __syncthreads();
-      again = __builtin_amdgcn_readfirstlane(__float_as_int(s_f2[DEEP_WAVES])) != 0;
-    }
-    if (__builtin_expect(again, 0)) {
-#pragma unroll
-      for (int b = 0; b < MB; ++b) tot[b] = sl[b] = v4acc{0.f, 0.f, 0.f, 0.f};
-      for (int pass = 0, c = cg; pass * NCW < nch; ++pass, c += NCW) {
-        if constexpr (!OWN) __syncthreads();
+    // from the first pass on that does not fit, of the wave (OWN) or the workgroup: on the fp32 instruction from the fp32 copy of the filter behind
+    // the terms (512->512 at 16x16 10.7 us, no pass fits 19; at 8x8 7.9 and 12.1)
+    if (__builtin_expect(unfit_pass < nch, 0)) {
+      for (int pass = __builtin_amdgcn_readfirstlane(unfit_pass), c = cg + NCW * pass; pass * NCW < nch; ++pass, c += NCW) {
         load_x(pass);
+        if (c < nch)
+#pragma unroll
+          for (int i = 0; i < NT; ++i) load_w(chunk_w(c) + 4 * weights, i, std::false_type());
+        if constexpr (OWN) mie_wave_order();
+        else __syncthreads();
         store_x(pass, std::false_type());
         if constexpr (OWN) mie_wave_order();
         else __syncthreads();
-        if (c < nch) {
-          const char* const wp = chunk_w(c) + 4 * weights + w_lane;
-#pragma unroll 1
-          for (int tap = tc; tap < K * K; tap += TPC) {
+        if (c >= nch) continue;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          const int tap = tc + TPC * i;
+          if (TPC == 1 || TPC * i + TPC <= K * K || tap < K * K) {
             const int ky = tap / K, kx = tap - ky * K;
 #pragma unroll
-            for (int q = 0; q < PL; ++q) {
-              const float4 wv = *reinterpret_cast<const float4*>(wp + ((tap - tc) * PL + q) * w_step);
+            for (int q = 0; q < PL; ++q)
 #pragma unroll
-              for (int b = 0; b < MB; ++b) mma16_f32(tot[b], wv, *reinterpret_cast<const float4*>(x_lane + q * STAGE + (2 * S * b + ky) * RP + kx * LS));
-            }
+              for (int b = 0; b < MB; ++b) mma16_f32(tot[b], w[i][q], *reinterpret_cast<const float4*>(x_lane + q * STAGE + (2 * S * b + ky) * RP + kx * LS));
+            __builtin_amdgcn_sched_barrier(0);
           }
         }
-        if constexpr (OWN) mie_wave_order();
       }
+      if constexpr (OWN) mie_wave_order();
     }
   }
   if constexpr (!OWN) __syncthreads();

@@ -218,12 +218,18 @@ __device__ __forceinline__ void split3(const float (&f)[8], float4 (&pl)[3]) {
 // The price is fp16's range.  A workgroup takes s from the largest value of its first chunk (of both inputs'), which goes to [2^12, 2^13),
 // so that a value is held to 2^-23 of itself or 2^-48 of that largest one, whichever is more.  The largest of every eight staged channels of a
 // pixel has to lie below 65000 and not below 2^-12, or be zero: outputs that such groups alone make up are then no further from fp64 than three
-// terms (norm of the error of 2304 terms, groups at 2^-12 .. -14: 2.4, 2.6, 3.5e-7, three terms 3.7e-7, far above it 2.3e-7).
-// Where one does not, infinities and NaN included, the workgroup does its contraction over on v_mfma_f32_32x32x2_f32, from the
-// same places of LDS and of a second, fp32, copy of the filter.  Over the networks' steps the largest value of a window was up to 3.5 times
-// its first chunk's, and such groups lay within 2^24 of it but for a few tiles of a recurrent state fed back (within 2^30, 2 tiles of 4767
-// 2^36).  The filter's scale takes its largest weight to [2^14, 2^15); a filter one of whose groups of eight input channels lies below 2^-29
-// of it is marked and contracted in fp32 always.
+// terms (norm of the error of 2304 terms, groups at 2^-12 .. -14: 2.4, 2.6, 3.5e-7, three terms 3.7e-7, far above it 2.3e-7).  (So the two terms
+// hold 2^-24 of a group's largest at the least, also for its small values.)
+// Over the networks' steps the largest value of a window was up to 3.5 times its first chunk's, and such groups lay within 2^24 of it but for a few
+// tiles of a recurrent state fed back (within 2^30, 2 tiles of 4767 2^36).  The threads note the chunks that do not fit, and the workgroup leaves
+// its loop in front of the first of these and goes on from there in three bf16 terms: X3's planes of the input, and the terms of the filter split
+// in registers, from an fp32 copy behind its two.  Where a value is too large for these (F2_HUGE: infinities, NaN) all of it is done over on
+// v_mfma_f32_32x32x2_f32.  us where all fit | all but the first chunk's channels 2^8 larger | half the pixels 2^-28 of the others, no chunk fits
+// | three terms: 3x3 256->256 at 33x44 13.6 | 17.5 | 20.6 | 16.6, 64->64 at 132x176 14.4 | 18.1 | 20.8 | 16.8, 5x5 stride 2 128->256 at 66x88 17.3 |
+// 22.1 | 25.9 | 23.5 (both contractions one after the other, the second on the fp32 instruction: 34, 32 and 45).  The look at every chunk costs
+// 0.2-0.3 us a launch; at the end only, it would cost the whole of the two terms' contraction once more.
+// The filter's scale takes its largest weight to [2^14, 2^15); a filter one of whose groups of eight input channels lies below 2^-29
+// of it is marked, and contracted in three terms from the first chunk on.
 typedef _Float16 mie_f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 mie_f16x8 __attribute__((ext_vector_type(8)));
 constexpr float F2_STEP = 2048.f;
@@ -241,6 +247,11 @@ __device__ __forceinline__ void split2(const float (&f)[8], float s, float4 (&pl
   split2_pair(f[4], f[5], s, s_lo, pl[0].z, pl[1].z);
   split2_pair(f[6], f[7], s, s_lo, pl[0].w, pl[1].w);
 }
+// Three bf16 terms of an operand that is there as fp32, its first four channels in the first half.
+__device__ __forceinline__ void split3_raw(const float4 (&raw)[2], float4 (&pl)[3]) {
+  const float f[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
+  split3(f, pl);
+}
 // (NaN if one of them is)
 __device__ __forceinline__ float f2_max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
 __device__ __forceinline__ float f2_amax8(const float (&f)[8]) {
@@ -257,32 +268,36 @@ __device__ __forceinline__ float f2_wave_max(float m) {
   step(std::integral_constant<int, 0x142>()); step(std::integral_constant<int, 0x143>());      // row_bcast 15, 31
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), 63));
 }
-// The scale for values whose largest is m (anything: what does not fit is found later).  Zeros tell nothing of what follows: F2_BLANK, which
+// The scale for values whose largest is m (anything: what does not fit is found later).  Zeros tell nothing of what follows: 2^73, which
 // values above 2^-57 do not fit.
-constexpr float F2_BLANK = 9444732965739290427392.f;      // 2^73
 __device__ __forceinline__ float f2_scale(float m) {
   int e = (__float_as_int(m) >> 23) - 127;
   e = m == 0.f ? -61 : e < -60 ? -60 : e > 52 ? 52 : e;
   return __int_as_float((127 + 12 - e) << 23);
 }
 __device__ __forceinline__ float f2_unscale(float s) { return __int_as_float((254 << 23) - __float_as_int(s)); }      // 1 / s
+constexpr unsigned F2_HUGE = (127u + 127u) << 23;      // bits of 2^127: from here on, infinities and NaN among them, values may have no finite bf16 terms
 // The groups a thread stages: in terms at their scale, and noted.
 struct F2Groups {
   float scale;
   unsigned most, least;                   // bits of the largest, bits less one of the least, zeros left out
   __device__ __forceinline__ void start(float s) { scale = s; most = 0u; least = ~0u; }
-  __device__ __forceinline__ void terms(const float (&f)[8], float4 (&pl)[2]) {
+  __device__ __forceinline__ void note(const float (&f)[8]) {
     const unsigned u = __float_as_uint(f2_amax8(f));
     most = max(most, u);
     least = min(least, u - 1u);
+  }
+  __device__ __forceinline__ void terms(const float (&f)[8], float4 (&pl)[2]) {
+    note(f);
     split2(f, scale, pl);
   }
+  __device__ __forceinline__ bool huge() const { return most >= F2_HUGE; }
   __device__ __forceinline__ bool misfit() const {      // (the scale's exponent taken off the bounds)
     const unsigned k = __float_as_uint(scale) - (127u << 23), lo = (127u - 12u) << 23, hi = 0x477de800u;      // 2^-12, 65000
     return most > hi - k || least < lo - k - 1u;
   }
 };
-// What a filter copy of this form ends with: 1 / (its scale), and whether all of it fits.
+// What a filter copy of this form ends with: 1 / (its scale), whether all of it fits, and whether three bf16 terms do not hold it either.
 template <typename T>
 __device__ __forceinline__ const float* f2_filter_end(const T* filt_mc, long long weights) {
   return reinterpret_cast<const float*>(reinterpret_cast<const char*>(filt_mc) + 8 * weights);
@@ -500,7 +515,8 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   constexpr int PD = RING - 1;                               // prefetch distance in units
   constexpr int CO_BLK = 32 * NB * WN;
   constexpr int RED = WK * 64 * CO_BLK;                      // every wave parks its accumulators here for the epilogue
-  constexpr int STAGE_F = NBUF * PL * STAGE * (int)sizeof(TL) / 4;  // the staging buffers, in floats
+  constexpr int PLANES = F2 && NBUF == 1 ? 3 : NBUF * PL;    // (F2: one buffer of three planes for what does not fit)
+  constexpr int STAGE_F = PLANES * STAGE * (int)sizeof(TL) / 4;     // the staging buffers, in floats
   constexpr int LOS = CC;                                    // floats per source pixel in LDS
   constexpr int LO_F = UP ? 64 * LOS : 0;                    // fp32 sums of the 8x8 source block, CC channels
   static_assert(!UP || (S == 1 && K == 5 && !GATES), "the up-sampling variant is the 5x5 stride-1 conv");
@@ -508,8 +524,9 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   constexpr int SMEM = (STAGE_F + LO_F > RED) ? STAGE_F + LO_F : RED;
   static_assert(SMEM * 4 <= (WIDE ? 160 * 1024 : 65536), "LDS budget");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
-  __shared__ float s_f2[F2 ? WAVES + 1 : 1];                         // largest values of the waves' first slots; whether a group does not fit
-  static_assert(!F2 || !AGAIN, "two terms: what does not fit is contracted in fp32");
+  __shared__ float s_f2[F2 ? WAVES + 3 : 1];                         // largest values of the waves' first slots; whether a group of a chunk does
+                                                                     // not fit, of every other one in the same place: a fast wave may be one ahead
+  static_assert(!F2 || !AGAIN, "two terms: what is not finite is contracted in fp32");
   TL* const sbuf = reinterpret_cast<TL*>(smem);
   float* const s_lo = smem + STAGE_F;
 
@@ -735,7 +752,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   };
   // one staged slot to LDS: as it is, or (X3) its eight fp32 values as three bf16 planes
   F2Groups groups;
-  bool filt_fits = true;                    // F2
+  float filt_form = 1.f;                    // F2: 1 where the filter fits, -1 where not even three terms hold it
   auto store_slot = [&](TL* dst, const float4 (&raw)[GPS]) __attribute__((always_inline)) {
     if constexpr (F2) {
       const float f[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[GPS - 1].x, raw[GPS - 1].y, raw[GPS - 1].z, raw[GPS - 1].w};
@@ -753,10 +770,16 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
       *reinterpret_cast<float4*>(dst) = raw[0];
     }
   };
-  // F2's fp32 form: the first four channels of a slot where the leading terms would be, the others where the rests would
-  auto store_raw = [&](TL* dst, const float4 (&raw)[GPS]) __attribute__((always_inline)) {
+  // F2, what does not fit: in three terms (2), or as it is (0), the first four channels of a slot in one plane, the others in the next
+  auto store_unfit = [&](TL* dst, const float4 (&raw)[GPS], auto form) __attribute__((always_inline)) {
+    if constexpr (F2) {
+      const float f[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[GPS - 1].x, raw[GPS - 1].y, raw[GPS - 1].z, raw[GPS - 1].w};
+      groups.note(f);
+      float4 pl[3] = {raw[0], raw[GPS - 1], raw[0]};
+      if constexpr (decltype(form)::value == 2) split3(f, pl);
 #pragma unroll
-    for (int g = 0; g < GPS; ++g) *reinterpret_cast<float4*>(dst + g * STAGE) = raw[g];
+      for (int q = 0; q < (decltype(form)::value == 2 ? 3 : 2); ++q) *reinterpret_cast<float4*>(dst + q * STAGE) = pl[q];
+    }
   };
   auto kept = [](const float4& v, bool k) __attribute__((always_inline)) { return make_float4(k ? v.x : 0.f, k ? v.y : 0.f, k ? v.z : 0.f, k ? v.w : 0.f); };
   auto store_slots = [&](const float4 (&regs)[NLD][GPS], int buf, unsigned ok) __attribute__((always_inline)) {
@@ -774,7 +797,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   auto scale_of = [&](float m) __attribute__((always_inline)) {
     m = f2_wave_max(m);
     if (lane == 0) s_f2[wave] = m;
-    if (tid == 0) s_f2[F2 ? WAVES : 0] = 0.f;
+    if (tid < 2) s_f2[F2 ? WAVES + tid : 0] = 0.f;
     __syncthreads();
     float w = s_f2[0];
 #pragma unroll
@@ -792,9 +815,9 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
     }
     return m;
   };
-  // (c: the chunk in the registers; terms: in terms, or F2's fp32 form; first: the first chunk, F2's scale from its sums)
+  // (c: the chunk in the registers; terms: 1 in terms, or a form of store_unfit; first: the first chunk, F2's scale from its sums)
   auto stage_store = [&](int buf, int c, auto terms, bool first = false) __attribute__((always_inline)) {
-    constexpr bool TERMS = decltype(terms)::value;
+    constexpr bool TERMS = decltype(terms)::value == 1;
     TL* dst = sbuf + buf * (PL * STAGE);
     if constexpr (UP) {
       // x + x2 of the source block to LDS in fp32 (bit pattern zero = 0 in both element types) ...
@@ -879,7 +902,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
         if constexpr (F2) {
           const float4 raw[GPS] = {make_float4(o[0], o[1], o[2], o[3]), make_float4(o[4], o[5], o[6], o[7])};
           if constexpr (TERMS) store_slot(d, raw);
-          else store_raw(d, raw);
+          else store_unfit(d, raw, terms);
         } else if constexpr (X3) {
           float4 pl[3];
           split3(o, pl);
@@ -901,7 +924,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
           float4 r[GPS];
 #pragma unroll
           for (int g = 0; g < GPS; ++g) r[g] = kept(st_reg[i][g], (ok >> i) & 1u);
-          store_raw(dst + st_lds[i], r);
+          store_unfit(dst + st_lds[i], r, terms);
         }
     }
   };
@@ -966,7 +989,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   // behind them.  (3x3 256->256: a chunk 1.55 -> 1.2 us in a launch of 16 workgroups, 18.3 -> 16.2 us together; at 33x44,
   // 240 workgroups, 20.0 -> 18.6; 512->512 at 8x12, unsplit, 30.7 -> 25.8.  On the full chip the matrix cores are held to
   // 1.6 .. 2.0 GHz by their power, and a launch that wastes less time runs at a lower clock.)
-  const auto in_terms = std::true_type();
+  const auto in_terms = std::integral_constant<int, 1>();
   constexpr bool WOVEN = X3 && NBUF == 2 && !UP && UPC >= NLD + 3;
   constexpr int TRASH = ROOM ? IT * LS : IT * RP;            // behind the pixels of row 0, or behind the rows: where slots that do not exist go
   static_assert(!WOVEN || TRASH + EPS <= STAGE, "room for a slot");
@@ -1016,8 +1039,28 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   if constexpr (F2) {
     const float* const end = f2_filter_end(a.filt_mc, (long long)a.cin_total * (K * K) * cout);
     filt_unscale = end[0];
-    filt_fits = end[1] != 0.f;
+    filt_form = end[1] - end[2];
   }
+  int c_end = c_hi;                         // F2: where the contraction in two terms ends: in front of the first chunk that does not fit
+  auto note_misfit = [&](int c) __attribute__((always_inline)) {      // in front of the barrier behind the stores of chunk c ...
+    if constexpr (F2) {
+      s_f2[groups.misfit() ? WAVES + ((c - c_lo) & 1) : WAVES + 2] = 1.f;      // (without a branch)
+    }
+  };
+  // ... asked behind it whether some thread noted one, and looked at where the chunk begins (true: it does not fit)
+  float stop = 0.f;
+  auto ask_stop = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) stop = s_f2[WAVES + ((c - c_lo) & 1)];
+  };
+  auto stops_at = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) {
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(stop)) != 0, 0)) {
+        c_end = c < c_end ? c : c_end;
+        return true;
+      }
+    }
+    return false;
+  };
   MIE_STAMP(2);
   const bool early = c_hi - c_lo >= 4;      // uniform over the workgroup
   if constexpr (WOVEN) {
@@ -1092,7 +1135,10 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   }
   if constexpr (WOVEN) store_slots(st_first, 0, c_lo >= nch1 ? ok2 : ok1);
   else stage_store(0, c_lo, in_terms, true);
+  note_misfit(c_lo);
   __syncthreads();
+  if (F2 && filt_form != 1.f) c_end = c_lo;
+  ask_stop(c_lo);
   unsigned cp_bits = 0u;
   if (!SPLIT) live_bits = mie_mask_take(live_m, live_b, live_in);
   if (GATES && !GRU) cp_bits = mie_mask_take(cp_m, cp_b, a.g_cpd != nullptr ? live_bits : 0u);
@@ -1142,7 +1188,8 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
     const TL* sin = sbuf;
     TL* snext = sbuf + PL * STAGE;
     load_a(sin, 0, av0);
-    for (int c = c_lo; c < c_hi; ++c) {
+    for (int c = c_lo; c < c_end; ++c) {
+      if (stops_at(c)) break;
 #pragma unroll
       for (int i = 0; i < UPC; ++i) {
         const int ip = i + PD;
@@ -1160,6 +1207,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
         if (i < NLD) {
           store_one(i, snext);
         } else if (i == NLD) {
+          note_misfit(c + 1);      // (well ahead of the barrier, which waits for what was written)
           int cn = __builtin_amdgcn_readfirstlane(c + 2 < c_hi ? c + 2 : c_hi - 1);
           asm volatile("" : "+s"(cn));
           load_raw(cn);
@@ -1176,6 +1224,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
         if (i == UPC - 2) {
           __syncthreads();
           load_a(snext, 0, av0);
+          ask_stop(c + 1);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -1188,10 +1237,11 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
   } else if constexpr (PIPE) {
     float4 av[2][2][PL], av0[2][PL];
     load_a(sbuf, 0, av0);
-    for (int c = c_lo; c < c_hi; ++c) {
+    for (int c = c_lo; c < c_end; ++c) {
       const bool more = c + 1 < c_hi;
       const TL* sin = sbuf + ((c - c_lo) & 1) * (PL * STAGE);
       const TL* sin_next = sbuf + ((c - c_lo + 1) & 1) * (PL * STAGE);
+      if (stops_at(c)) break;
 #pragma unroll
       for (int i = 0; i < UPC; ++i) {
         if (PD > 0) {
@@ -1217,7 +1267,9 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
         }
         if (i == UPC - 2) {
           // every wave has its last operands of this chunk (the wait for them is part of the barrier)
+          note_misfit(c + 1);
           __syncthreads();
+          ask_stop(c + 1);
           load_a(sin_next, 0, av0);       // after the last chunk: read and dropped
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1228,7 +1280,8 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
     // (the epilogue reuses the staging buffers: every read of them that matters was waited for in front of the
     // last barrier; the operand read behind it returns whatever a faster wave has parked there, and is dropped)
   } else {
-    for (int c = c_lo; c < c_hi; ++c) {
+    stops_at(c_lo);
+    for (int c = c_lo; c < c_end; ++c) {
       const bool more = c + 1 < c_hi;
       const int cn = more ? c + 1 : c;      // after the last chunk: redundant re-load, never stored
       ub_next = chunk_b(cn);
@@ -1255,7 +1308,10 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
       }
       if (NBUF == 1 && !UP) __syncthreads();   // every wave is done reading the only buffer (UP: stage_store syncs)
       if (more) stage_store((c - c_lo + 1) % NBUF, c + 1, in_terms);
+      note_misfit(c + 1);
       __syncthreads();
+      ask_stop(c + 1);
+      stops_at(c + 1);
       ub_cur = ub_next;
       MIE_STAMP(4 + (c - c_lo));
     }
@@ -1280,8 +1336,98 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[mb][nb][r] += accs[mb][nb][r];
   }
+  // F2, from the first chunk on that does not fit: three bf16 terms of the input and of the fp32 copy of the filter, as little code as
+  // keeps the matrix cores busy (bound by the filter's 8 bytes a weight); where there are values that these do not hold, all of it on the
+  // fp32 instruction.
+  if constexpr (F2) {
+    if (__builtin_expect(c_end < c_hi, 0)) {
+      const long long fp32_at = 2LL * a.cin_total * (K * K) * cout;      // (in elements of two bytes: behind the terms)
+      constexpr int R = 4;                                               // units of the filter in registers
+      auto plainly = [&](int c_from, auto form) __attribute__((always_inline)) {
+        constexpr bool THREE = decltype(form)::value == 2;
+        constexpr int PA = THREE ? 3 : 2;
+        for (int c = c_from; c < c_hi; ++c) {
+          const TL* const ub = chunk_b(c) + fp32_at;
+          float4 br[R][NB][PL];
+          auto load = [&](int unit, float4 (&bv)[NB][PL]) __attribute__((always_inline)) {
+            const int u = unit < UPC ? unit : UPC - 1, tap = unit_tap(u) < K * K ? unit_tap(u) : K * K - 1;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+              for (int q = 0; q < PL; ++q)
+                bv[nb][q] = *reinterpret_cast<const float4*>(ub + ((long long)(((unit_sub(u) * (K * K) + tap) * PL + q) * 2) * cout + nb * 32) * EPS + b_lane);
+          };
+          stage_load(c);
+#pragma unroll
+          for (int j = 0; j < R - 1; ++j) load(j, br[j]);
+          __syncthreads();
+          stage_store(0, c, form);
+          __syncthreads();
+          float4 av[2][2][PA];
+          auto read = [&](int unit, float4 (&x)[2][PA]) __attribute__((always_inline)) {
+            const int u = unit < UPC ? unit : UPC - 1, tap = unit_tap(u) < K * K ? unit_tap(u) : K * K - 1, ky = tap / K, kx = tap - ky * K;
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+              for (int q = 0; q < PA; ++q)
+                x[mb][q] = *reinterpret_cast<const float4*>(&sbuf[q * STAGE + swapped(mb, ky) + ky * RP + kx * LS + SUB * unit_sub(u)]);
+          };
+          read(0, av[0]);
+#pragma unroll 1
+          for (int u0 = 0; u0 < UPC; u0 += R) {
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+              const int u = u0 + j;
+              load(u + R - 1, br[(j + R - 1) % R]);
+              read(u + 1, av[(j + 1) & 1]);
+              __builtin_amdgcn_sched_barrier(0);
+              if (u >= UPC || unit_tap(u) >= K * K) continue;
+              const auto& x = av[j & 1];
+#pragma unroll
+              for (int nb = 0; nb < NB; ++nb) {
+                if constexpr (THREE) {
+                  float4 b3[3];
+                  split3_raw(br[j][nb], b3);
+                  mma_unit2_x3(acc[0][nb], acc[1][nb], accs[0][nb], accs[1][nb], x[0], x[1], b3);
+                } else {
+#pragma unroll
+                  for (int q = 0; q < PL; ++q) mma_unit2(acc[0][nb], acc[1][nb], x[0][q], x[1][q], br[j][nb][q], float());
+                }
+              }
+            }
+          }
+        }
+      };
+      auto clear = [&](auto& v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[mb][nb][r] = 0.f;
+      };
+      clear(accs);
+      if (filt_form >= 0.f) plainly(c_end, std::integral_constant<int, 2>());
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[mb][nb][r] += accs[mb][nb][r];
+      __syncthreads();
+      if (tid == 0) s_f2[WAVES] = filt_form < 0.f ? 1.f : 0.f;
+      __syncthreads();
+      if (groups.huge()) s_f2[WAVES] = 1.f;
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[WAVES])) != 0) {
+        clear(acc);
+        plainly(c_lo, std::integral_constant<int, 0>());
+        __syncthreads();
+      }
+    }
+  }
   // the wave's sums to LDS, where all of them meet behind a barrier
-  auto park = [&]() __attribute__((always_inline)) {
+  auto meet = [&]() __attribute__((always_inline)) {
     float* red = smem + wk * (64 * CO_BLK);
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
@@ -1292,52 +1438,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
         for (int nb = 0; nb < NB; ++nb)
           red[p * CO_BLK + wn * (32 * NB) + nb * 32 + l32] = acc[mb][nb][r];
       }
-  };
-  auto meet = [&]() __attribute__((always_inline)) {
-    park();
-    if constexpr (F2) {
-      if (groups.misfit() || !filt_fits) s_f2[WAVES] = 1.f;
-    }
     __syncthreads();
-    if constexpr (F2) {
-      // a group that does not fit: all of it once more, on the fp32 instruction, as plainly as it can be said.  (Every workgroup of 3x3
-      // 256->256 at 33x44: 41 us instead of 13.5, three bf16 terms 17.5; 64->64 at 132x176: 33, 14.3 and 17.6)
-      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[WAVES])) != 0, 0)) {
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mb][nb][r] = 0.f;
-        const long long fp32_at = 2LL * a.cin_total * (K * K) * cout;      // (in elements of two bytes: behind the terms)
-        for (int c = c_lo; c < c_hi; ++c) {
-          stage_load(c);
-          __syncthreads();
-          stage_store(0, c, std::false_type());
-          __syncthreads();
-          const TL* const ub = chunk_b(c) + fp32_at;
-#pragma unroll 1
-          for (int u = 0; u < UPC; ++u) {
-            if (unit_tap(u) >= K * K) break;
-            float4 av[2][PL], bv[NB][PL];
-            load_b(ub, u, bv);
-            const int ky = unit_tap(u) / K, kx = unit_tap(u) - ky * K;
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-              for (int q = 0; q < PL; ++q)
-                av[mb][q] = *reinterpret_cast<const float4*>(&sbuf[q * STAGE + swapped(mb, ky) + ky * RP + kx * LS + SUB * unit_sub(u)]);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-              for (int q = 0; q < PL; ++q) mma_unit2(acc[0][nb], acc[1][nb], av[0][q], av[1][q], bv[nb][q], float());
-          }
-        }
-        __syncthreads();
-        park();
-        __syncthreads();
-      }
-    }
   };
   if constexpr (GRU) {
     // Gate math of a ConvGRU: column 8 * j + e is the update gate of hidden channel 4 * j + e (e < 4) or the candidate of 4 * j + e - 4.

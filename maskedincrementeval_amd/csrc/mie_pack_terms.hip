@@ -42,8 +42,9 @@ __global__ __launch_bounds__(256) void k_f2_split(const float* __restrict__ valu
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     end[0] = f2_unscale(scale);
     end[1] = fits ? 1.f : 0.f;
+    end[2] = most >= F2_HUGE ? 1.f : 0.f;
 #pragma unroll
-    for (int i = 2; i < 12; ++i) end[i] = 0.f;
+    for (int i = 3; i < 12; ++i) end[i] = 0.f;
   }
   const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
   if (g >= groups) return;

@@ -28,6 +28,16 @@ namespace {
 __host__ __device__ constexpr int tc_phase(int k, int pad) { return (((k - pad) % 2) + 2) % 2; }
 __host__ __device__ constexpr int tc_shift(int k, int pad) { return (tc_phase(k, pad) + pad - k) / 2; }   // numerator is even
 
+// The six significant term products of a unit, the two pixel blocks interleaved (smallest terms first).
+__device__ __forceinline__ void mma_tconv_x3(v16f (&acc)[2], const float4 (&A)[2][3], const float4 (&B)[3]) {
+  mma_unit(acc[0], A[0][2], B[0], mie_bf16()); mma_unit(acc[1], A[1][2], B[0], mie_bf16());
+  mma_unit(acc[0], A[0][1], B[1], mie_bf16()); mma_unit(acc[1], A[1][1], B[1], mie_bf16());
+  mma_unit(acc[0], A[0][0], B[2], mie_bf16()); mma_unit(acc[1], A[1][0], B[2], mie_bf16());
+  mma_unit(acc[0], A[0][1], B[0], mie_bf16()); mma_unit(acc[1], A[1][1], B[0], mie_bf16());
+  mma_unit(acc[0], A[0][0], B[1], mie_bf16()); mma_unit(acc[1], A[1][0], B[1], mie_bf16());
+  mma_unit(acc[0], A[0][0], B[0], mie_bf16()); mma_unit(acc[1], A[1][0], B[0], mie_bf16());
+}
+
 // X3 (fp32 deltas): the three-term bf16 form of k_conv_mfma -- staged values and weights as hi + mid + lo in bf16, six
 // v_mfma_f32_32x32x16_bf16 products per multiply, fp32 accuracy; chunks of 64 channels (four units per tap, so that the
 // k-split stays over whole sub-chunks and every tap's phase is known at compile time), three bf16 planes in LDS,
@@ -73,12 +83,13 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
   constexpr int PD = RING - 1;
   constexpr int CO_BLK = 32 * WN;
   constexpr int RED = WK * 64 * CO_BLK;                      // the accumulators of one phase, parked for the epilogue
-  constexpr int STAGE_F = NBUF * PL * STAGE * (int)sizeof(TL) / 4;
+  constexpr int STAGE_F = (F2 ? 3 : NBUF * PL) * STAGE * (int)sizeof(TL) / 4;      // (F2: three planes for what does not fit)
   constexpr int SMEM = STAGE_F > RED ? STAGE_F : RED;
   static_assert(SMEM * 4 <= 65536, "LDS budget");
   static_assert(!SPLIT || WN == 1, "the split form is the 32-channel slab kernel");
+  static_assert(!F2 || NBUF == 1, "two terms: one staging buffer");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
-  __shared__ float s_f2[F2 ? 5 : 1];                         // F2: largest values of the waves' first slots; whether a group does not fit
+  __shared__ float s_f2[F2 ? 6 : 1];                         // F2: largest values of the waves' first slots; whether a group of a chunk does not fit
   TL* const sbuf = reinterpret_cast<TL*>(smem);
 
   int n, y0, x0;                                             // block origin in INPUT coordinates
@@ -118,11 +129,11 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
   // F2: the filter's scale and whether it fits, on their way from here on
   const long long weights = (long long)a.cin_total * (K * K) * cout;
   float filt_unscale = 1.f;
-  bool filt_fits = true;
+  float filt_form = 1.f;
   if constexpr (F2) {
     const float* const end = f2_filter_end(a.filt_mc, weights);
     filt_unscale = end[0];
-    filt_fits = end[1] != 0.f;
+    filt_form = end[1] - end[2];
   }
 
   // ---- staging plan (as in k_conv_mfma, stride 1) ------------------------------------------------------
@@ -186,7 +197,7 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
     }
     return m;
   };
-  // (terms: in terms, or F2's fp32 form)
+  // (terms: 1 in terms, F2: 2 in three of them, 0 as it is)
   auto stage_store = [&](int buf, auto terms) __attribute__((always_inline)) {
     TL* dst = sbuf + buf * (PL * STAGE);
 #pragma unroll
@@ -195,10 +206,14 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
         if constexpr (F2) {
           const float4 u = st_reg[i][0], v = st_reg[i][GPS - 1];
           const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-          float4 pl[2] = {u, v};
-          if constexpr (decltype(terms)::value) groups.terms(f, pl);
+          constexpr int FORM = decltype(terms)::value;
+          float4 pl[FORM == 2 ? 3 : 2];
+          pl[0] = u; pl[1] = v;
+          if constexpr (FORM == 1) groups.terms(f, pl);
+          else groups.note(f);
+          if constexpr (FORM == 2) split3(f, pl);
 #pragma unroll
-          for (int q = 0; q < 2; ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
+          for (int q = 0; q < (FORM == 2 ? 3 : 2); ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
         } else if constexpr (X3) {
           const float f[8] = {st_reg[i][0].x, st_reg[i][0].y, st_reg[i][0].z, st_reg[i][0].w,
                               st_reg[i][1].x, st_reg[i][1].y, st_reg[i][1].z, st_reg[i][1].w};
@@ -240,7 +255,27 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
   const int c_hi = SPLIT ? (bz + 1) * nch >> a.xcd_fs : nch;
   const TL* ub_cur = chunk_b(c_lo);
   const TL* ub_next = ub_cur;
-  const auto in_terms = std::true_type();
+  const auto in_terms = std::integral_constant<int, 1>();
+  int c_end = c_hi;                         // F2: where the contraction in two terms ends: in front of the first chunk that does not fit
+  auto note_misfit = [&]() __attribute__((always_inline)) {
+    if constexpr (F2) {
+      s_f2[groups.misfit() ? 4 : 5] = 1.f;      // (without a branch)
+    }
+  };
+  // (asked behind the barrier and looked at where the chunk begins; two barriers a chunk: nobody notes the next one before)
+  float stop = 0.f;
+  auto ask_stop = [&]() __attribute__((always_inline)) {
+    if constexpr (F2) stop = s_f2[4];
+  };
+  auto stops_at = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) {
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(stop)) != 0, 0)) {
+        c_end = c;
+        return true;
+      }
+    }
+    return false;
+  };
   const bool both = F2 && c_lo < nch1 && nch1 < c_hi;      // (F2: the scale is for both inputs)
   float4 st_two[F2 ? NLD : 1][GPS];
   if constexpr (F2) {
@@ -262,9 +297,12 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
         __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[1], s_f2[2]), s_f2[3]))))));
   }
   stage_store(0, in_terms);
+  note_misfit();
   __syncthreads();
+  if (F2 && filt_form != 1.f) c_end = c_lo;
+  ask_stop();
 
-  for (int c = c_lo; c < c_hi; ++c) {
+  for (int c = c_lo; c < c_end; ++c) {
     const bool more = c + 1 < c_hi;
     const int cn = more ? c + 1 : c;
     ub_next = chunk_b(cn);
@@ -282,6 +320,7 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
           dst[mb][q] = *reinterpret_cast<const float4*>(&sin[q * STAGE + a_lane[mb] + dy * RP + dx * LS + SUB * qi]);
     };
     load_a(0, av[0]);
+    if (stops_at(c)) break;
 #pragma unroll
     for (int i = 0; i < UPC; ++i) {
       if (PD > 0) {
@@ -298,15 +337,7 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
         if constexpr (F2) {
           mma_unit2_f2(acc[ph][0], acc[ph][1], sm[ph][0], sm[ph][1], av[i & 1][0], av[i & 1][1], bring[i % RING]);
         } else if constexpr (X3) {
-          // the six significant term products of the unit, the two pixel blocks interleaved (smallest terms first)
-          const auto& A = av[i & 1];
-          const auto& B = bring[i % RING];
-          mma_unit(acc[ph][0], A[0][2], B[0], mie_bf16()); mma_unit(acc[ph][1], A[1][2], B[0], mie_bf16());
-          mma_unit(acc[ph][0], A[0][1], B[1], mie_bf16()); mma_unit(acc[ph][1], A[1][1], B[1], mie_bf16());
-          mma_unit(acc[ph][0], A[0][0], B[2], mie_bf16()); mma_unit(acc[ph][1], A[1][0], B[2], mie_bf16());
-          mma_unit(acc[ph][0], A[0][1], B[0], mie_bf16()); mma_unit(acc[ph][1], A[1][1], B[0], mie_bf16());
-          mma_unit(acc[ph][0], A[0][0], B[1], mie_bf16()); mma_unit(acc[ph][1], A[1][0], B[1], mie_bf16());
-          mma_unit(acc[ph][0], A[0][0], B[0], mie_bf16()); mma_unit(acc[ph][1], A[1][0], B[0], mie_bf16());
+          mma_tconv_x3(acc[ph], av[i & 1], bring[i % RING]);
         } else {
 #pragma unroll
           for (int mb = 0; mb < 2; ++mb) mma_unit(acc[ph][mb], av[i & 1][mb][0], bring[i % RING][0], T());
@@ -317,47 +348,82 @@ __global__ __launch_bounds__(256, ARITH == 0 && WN <= 2 ? 2 : 1) void k_tconv_mf
     }
     if (NBUF == 1) __syncthreads();
     if (more) stage_store((c - c_lo + 1) % NBUF, in_terms);
-    if constexpr (F2) {
-      if (!more && (groups.misfit() || !filt_fits)) s_f2[4] = 1.f;
-    }
+    note_misfit();
     __syncthreads();
+    ask_stop();
     ub_cur = ub_next;
   }
   float c0 = 1.f;                      // F2: 1 / scales
   if constexpr (F2) {
     c0 = f2_unscale(groups.scale) * filt_unscale;      // exactly: powers of two, 2^-143 at the least but for sums of zeros
-    // a group that does not fit: all of it once more on the fp32 instruction, from the fp32 copy of the filter behind the terms
-    if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
+    // a chunk that does not fit: all of it in three bf16 terms of the input and of the fp32 copy of the filter behind the two.  (Not from
+    // this chunk on, as in k_conv_mfma: adding up both sets of sums at its place costs the fast path registers.)  us where all fit | later
+    // channels 1000 times larger | no chunk fits | three terms: 64+64->64 from 160x160 31.2 | 31.4 | 44 | 36.5, 512->256 from 40x44 26.3 | 49 | 41 | 32,
+    // 5x5 128+64->64 from 66x88 20.6 | 20.6 | 33 | 26.5.
+    if (__builtin_expect(c_end < c_hi, 0)) {
+      auto plainly = [&](auto form) __attribute__((always_inline)) {
+        constexpr bool THREE = decltype(form)::value == 2;
+        constexpr int PA = THREE ? 3 : 2;
+        for (int c = c_lo; c < c_hi; ++c) {
+          const TL* ub = chunk_b(c) + 2 * weights;
+          stage_load(c);
 #pragma unroll
-      for (int ph = 0; ph < 4; ++ph)
+          for (int i = 0; i < RING - 1; ++i) load_b(ub, i, bring[i]);
+          __syncthreads();
+          stage_store(0, form);
+          __syncthreads();
+          float4 av[2][2][PA];
+          auto read = [&](int i, float4 (&x)[2][PA]) __attribute__((always_inline)) {
+            const int tap = i / NQW, ky = tap / K, kx = tap - ky * K;
+            const int at = (tc_shift(ky, PAD) + LO) * RP + (tc_shift(kx, PAD) + LO) * LS + SUB * (i % NQW);
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+            for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[ph][mb][r] = sm[ph][mb][r] = 0.f;
-      c0 = 1.f;
-      for (int c = c_lo; c < c_hi; ++c) {
-        stage_load(c);
-        __syncthreads();
-        stage_store(0, std::false_type());
-        __syncthreads();
-        const TL* const ub = chunk_b(c) + 2 * weights;
+              for (int q = 0; q < PA; ++q) x[mb][q] = *reinterpret_cast<const float4*>(&sbuf[q * STAGE + a_lane[mb] + at]);
+          };
+          read(0, av[0]);
 #pragma unroll
-        for (int tap = 0; tap < K * K; ++tap) {      // (a tap's phase picks the accumulators)
-          const int ky = tap / K, kx = tap - ky * K, ph = tc_phase(ky, PAD) * 2 + tc_phase(kx, PAD);
-          const int at = (tc_shift(ky, PAD) + LO) * RP + (tc_shift(kx, PAD) + LO) * LS;
-#pragma unroll 1
-          for (int qi = 0; qi < NQW; ++qi) {
-            float4 b[PL];
-            load_b(ub, tap * NQW + qi, b);
+          for (int i = 0; i < UPC; ++i) {
+            const int tap = i / NQW, ky = tap / K, kx = tap - ky * K, ph = tc_phase(ky, PAD) * 2 + tc_phase(kx, PAD);
+            asm volatile("" : "+s"(ub));      // (or the units' addresses are all kept in registers)
+            if (i + RING - 1 < UPC) load_b(ub, i + RING - 1, bring[(i + RING - 1) % RING]);
+            if (i + 1 < UPC) read(i + 1, av[(i + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            const auto& x = av[i & 1];
+            if constexpr (THREE) {
+              float4 b3[3];
+              split3_raw(bring[i % RING], b3);
+              mma_tconv_x3(acc[ph], x, b3);
+            } else {
 #pragma unroll
-            for (int q = 0; q < PL; ++q)
-#pragma unroll
-              for (int mb = 0; mb < 2; ++mb)
-                mma_unit(acc[ph][mb], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + a_lane[mb] + at + SUB * qi]), b[q], float());
+              for (int q = 0; q < PL; ++q) mma_unit2(acc[ph][0], acc[ph][1], x[0][q], x[1][q], bring[i % RING][q], float());
+            }
+            __builtin_amdgcn_sched_barrier(0);
           }
         }
-      }
+      };
+      auto clear = [&](v16f (&v)[4][2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ph = 0; ph < 4; ++ph)
+#pragma unroll
+          for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[ph][mb][r] = 0.f;
+      };
+      clear(acc);
+      clear(sm);
+      c0 = 1.f;
+      if (filt_form >= 0.f) plainly(std::integral_constant<int, 2>());
       __syncthreads();
+      if (tid == 0) s_f2[4] = filt_form < 0.f ? 1.f : 0.f;
+      __syncthreads();
+      if (groups.huge()) s_f2[4] = 1.f;
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0) {      // values that three bf16 terms do not hold: all of it on the fp32 instruction
+        clear(acc);
+        plainly(std::integral_constant<int, 0>());
+        __syncthreads();
+      }
     }
   }
 

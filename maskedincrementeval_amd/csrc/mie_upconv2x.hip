@@ -210,7 +210,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   constexpr int SMEM = STAGE_F > RED ? STAGE_F : RED;
   static_assert(SMEM * 4 <= 65536, "LDS budget");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
-  __shared__ float s_f2[F2 ? 5 : 1];                         // F2: largest values of the waves' first slots; whether a group does not fit
+  __shared__ float s_f2[F2 ? 7 : 1];                         // F2: largest values of the waves' first slots; whether a group of a chunk does not fit,
+                                                             // of every other one in the same place
   TL* const sbuf = reinterpret_cast<TL*>(smem);
 
   // ---- which positions, phase and slab: each XCD (workgroup index mod 8) takes a contiguous eighth of the order (group of
@@ -344,9 +345,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
       }
   };
   F2Groups groups;
-  // (terms: in terms, or F2's fp32 form; first: the first chunk, F2's scale from it)
+  // (terms: 1 in terms, F2: 2 in three of them, 0 as it is; first: the first chunk, F2's scale from it)
   auto stage_store = [&](int buf, auto terms, bool first = false) __attribute__((always_inline)) {
-    constexpr bool TERMS = decltype(terms)::value;
+    constexpr int FORM = decltype(terms)::value;
     TL* dst = sbuf + buf * (PL * STAGE);
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
     float v[F2 ? NLD : 1][8];
@@ -369,13 +370,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
     if constexpr (F2) {
 #pragma unroll
       for (int i = 0; i < NLD; ++i) sum(i, v[i]);
-      if (TERMS && first) {
+      if (FORM == 1 && first) {
         float m = 0.f;
 #pragma unroll
         for (int i = 0; i < NLD; ++i) m = __builtin_elementwise_maximum(m, f2_amax8(v[i]));
         m = f2_wave_max(m);
         if (lane == 0) s_f2[wave] = m;
-        if (tid == 0) s_f2[4] = 0.f;
+        if (tid < 2) s_f2[4 + tid] = 0.f;
         __syncthreads();
         groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(
             __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[1], s_f2[2]), s_f2[3]))))));
@@ -392,10 +393,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
       }
       if (tid + 256 * i < n_slots) {
         if constexpr (F2) {
-          float4 pl[2] = {make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7])};
-          if constexpr (TERMS) groups.terms(f, pl);
+          float4 pl[FORM == 2 ? 3 : 2];
+          pl[0] = make_float4(f[0], f[1], f[2], f[3]); pl[1] = make_float4(f[4], f[5], f[6], f[7]);
+          if constexpr (FORM == 1) groups.terms(f, pl);
+          else groups.note(f);
+          if constexpr (FORM == 2) split3(f, pl);
 #pragma unroll
-          for (int q = 0; q < 2; ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
+          for (int q = 0; q < (FORM == 2 ? 3 : 2); ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
         } else if constexpr (X3) {
           float4 pl[3];
           split3(f, pl);
@@ -465,12 +469,32 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
   // F2: the filter's scale and whether it fits, on their way from here on
   const long long weights = 4LL * UNITS * a.c1 * cout;
   float filt_unscale = 1.f;
-  bool filt_fits = true;
+  float filt_form = 1.f;
   if constexpr (F2) {
     const float* const end = f2_filter_end(a.filt_mc, weights);
     filt_unscale = end[0];
-    filt_fits = end[1] != 0.f;
+    filt_form = end[1] - end[2];
   }
+  int c_end = nch;                         // F2: where the contraction in two terms ends: in front of the first chunk that does not fit
+  auto note_misfit = [&](int c) __attribute__((always_inline)) {      // in front of the barrier behind the stores of chunk c ...
+    if constexpr (F2) {
+      s_f2[groups.misfit() ? 4 + (c & 1) : 6] = 1.f;      // (without a branch)
+    }
+  };
+  // ... asked behind it whether some thread noted one, and looked at where the chunk begins (true: it does not fit)
+  float stop = 0.f;
+  auto ask_stop = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) stop = s_f2[4 + (c & 1)];
+  };
+  auto stops_at = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) {
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(stop)) != 0, 0)) {
+        c_end = c;
+        return true;
+      }
+    }
+    return false;
+  };
 
   float4 bring[4][PL];
   seek_b(first_b(0));
@@ -486,13 +510,16 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
     const int pl = i / (LS / EPS);
     *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (i - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  const auto in_terms = std::true_type();
+  const auto in_terms = std::integral_constant<int, 1>();
   stage_store(0, in_terms, true);
+  note_misfit(0);
   __syncthreads();
+  if (F2 && filt_form != 1.f) c_end = 0;
+  ask_stop(0);
 
   // All loads of a chunk are unconditional (see k_conv_mfma); behind the last one "the next" is the chunk itself.
   auto contract = [&](auto block) {
-    for (int c = 0; c < nch; ++c) {
+    for (int c = 0; c < c_end; ++c) {
       const bool more = c + 1 < nch;
       const int cn = more ? c + 1 : c;
       const TL* const ub_next = first_b(cn);
@@ -510,6 +537,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
               dst[mb][q] = *reinterpret_cast<const float4*>(&sa[q * STAGE + a_lane[mb] + (k >> 2) * RP + (k & 3) * LS + SUB * qi]);
         };
         load_a(0, av[0]);
+        if (stops_at(c)) break;
 #pragma unroll
         for (int i = 0; i < UPC; ++i) {
           const int ip = i + 3;
@@ -543,6 +571,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
         int base, step, qi = 0, g = 0;
         lane_of(0, 0, base, step);
         load_a(base, av[0]);
+        if (stops_at(c)) break;
         for (int left = NQW * ng; left > 0; --left) {
           const bool end = g + 1 == ng;
           const int gn = end ? 0 : g + 1, qn = left == 1 ? 0 : (end ? qi + 1 : qi);
@@ -579,10 +608,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
       }
       if (NBUF == 1) __syncthreads();
       if (more) stage_store((c + 1) % NBUF, in_terms);
-      if constexpr (F2) {
-        if (!more && (groups.misfit() || !filt_fits)) s_f2[4] = 1.f;
-      }
+      note_misfit(c + 1);
       __syncthreads();
+      ask_stop(c + 1);
     }
   };
   if (side == 0) contract(std::true_type());
@@ -593,45 +621,108 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[mb][r] = fmaf(sm[mb][r], c1, (acc[mb][r] + acc_odd[mb][r]) * c0);
-    // a group that does not fit: all of it once more on the fp32 instruction, from the fp32 copy of the filter behind the terms
-    if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
+    // from the first chunk on that does not fit: three bf16 terms of the input and of the fp32 copy of the filter behind the two, as in k_conv_mfma.
+    // us where all fit | later channels 2^8 larger | no chunk fits | three terms: 256->128 at 33x44 28.9 | 47 | 65 | 42, 128->64 at 66x88 27.6 | 37 | 44 |
+    // 41, and of k_upconv2x_all 64->32 at 132x176 30.8 | 39.5 | 46 | 44.5.
+    if (__builtin_expect(c_end < nch, 0)) {
+      auto plainly = [&](int c_from, auto form) __attribute__((always_inline)) {
+        constexpr bool THREE = decltype(form)::value == 2;
+        constexpr int PA = THREE ? 3 : 2;
+        auto load = [&](const TL* gb, float4 (&b)[PL]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[mb][r] = 0.f;
-      for (int c = 0; c < nch; ++c) {
-        stage_load(c);
-        __syncthreads();
-        stage_store(0, std::false_type());
-        __syncthreads();
-        auto unit = [&](const TL* gb, int at0, int at1) __attribute__((always_inline)) {
-#pragma unroll
-          for (int q = 0; q < PL; ++q) {
-            const float4 b = *reinterpret_cast<const float4*>(gb + 2 * weights + b_lane + q * (2 * cout * EPS));
-            mma_unit(acc[0], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at0]), b, float());
-            if (side == 0) mma_unit(acc[1], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at1]), b, float());
-          }
+          for (int q = 0; q < PL; ++q) b[q] = *reinterpret_cast<const float4*>(gb + 2 * weights + b_lane + q * (2 * cout * EPS));
         };
-        for (int qi = 0; qi < NQW; ++qi) {
-          if (side == 0) {
-#pragma unroll 1
-            for (int k = 0; k < 4 * NI; ++k) {
-              const int at = (cls * NI + (k >> 2)) * RP + (k & 3) * LS + SUB * qi;
-              unit(group_b(c, qi, 4 * NI * cls + k), a_lane[0] + at, a_lane[1] + at);
+        auto read_x = [&](int at, float4 (&x)[PA]) __attribute__((always_inline)) {
+#pragma unroll
+          for (int q = 0; q < PA; ++q) x[q] = *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at]);
+        };
+        auto unit = [&](const float4 (&b)[PL], const float4 (&x0)[PA], const float4 (&x1)[PA], auto block) __attribute__((always_inline)) {
+          if constexpr (THREE) {
+            float4 b3[3];
+            split3_raw(b, b3);
+            if constexpr (decltype(block)::value) {
+              mma_up2x_x3(acc[0], acc[1], sm[0], sm[1], x0, x1, b3);
+            } else {
+              mma_unit(sm[0], x0[2], b3[0], mie_bf16()); mma_unit(sm[0], x0[1], b3[1], mie_bf16());
+              mma_unit(acc[0], x0[0], b3[0], mie_bf16()); mma_unit(sm[0], x0[0], b3[2], mie_bf16());
+              mma_unit(sm[0], x0[1], b3[0], mie_bf16()); mma_unit(sm[0], x0[0], b3[1], mie_bf16());
             }
           } else {
+#pragma unroll
+            for (int q = 0; q < PL; ++q) {
+              mma_unit(acc[0], x0[q], b[q], float());
+              if constexpr (decltype(block)::value) mma_unit(acc[1], x1[q], b[q], float());
+            }
+          }
+        };
+        for (int c = c_from; c < nch; ++c) {
+          stage_load(c);
+          __syncthreads();
+          stage_store(0, form);
+          __syncthreads();
+          for (int qi = 0; qi < NQW; ++qi) {
+            if (side == 0) {
+              const TL* const gb = group_b(c, qi, 4 * NI * cls);
+              float4 br[4][PL];
+#pragma unroll
+              for (int j = 0; j < 3; ++j) load(gb + j * unit_sz, br[j]);
+              float4 xv[2][2][PA];
+#pragma unroll
+              for (int mb = 0; mb < 2; ++mb) read_x(a_lane[mb] + cls * NI * RP + SUB * qi, xv[0][mb]);
 #pragma unroll 1
-            for (int g = 0; g < ng; ++g) {
-              const int code = (int)((strip >> (4 * g)) & 15u);
-              const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
-              const int base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF, step = on ? (corner ? RPS : LS) : 0;
+              for (int ky = 0; ky < NI; ++ky) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                  const int ahead = 4 * ky + j + 3;
+                  load(gb + (ahead < 4 * NI ? ahead : 4 * NI - 1) * unit_sz, br[(j + 3) & 3]);
+                  const int k = 4 * ky + j + 1 < 4 * NI ? 4 * ky + j + 1 : 0, at = (cls * NI + (k >> 2)) * RP + (k & 3) * LS + SUB * qi;
+#pragma unroll
+                  for (int mb = 0; mb < 2; ++mb) read_x(a_lane[mb] + at, xv[(j + 1) & 1][mb]);
+                  __builtin_amdgcn_sched_barrier(0);
+                  unit(br[j], xv[j & 1][0], xv[j & 1][1], std::true_type());
+                }
+              }
+            } else {
 #pragma unroll 1
-              for (int t = 0; t < (corner ? 3 : 4); ++t) unit(group_b(c, qi, strip_unit(g) + t), base + t * step, 0);
+              for (int g = 0; g < ng; ++g) {
+                const int code = (int)((strip >> (4 * g)) & 15u);
+                const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
+                const int base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF, step = on ? (corner ? RPS : LS) : 0;
+#pragma unroll 1
+                for (int t = 0; t < (corner ? 3 : 4); ++t) {
+                  float4 b[PL];
+                  load(group_b(c, qi, strip_unit(g) + t), b);
+                  float4 x[PA];
+                  read_x(base + t * step, x);
+                  unit(b, x, x, std::false_type());
+                }
+              }
             }
           }
         }
-      }
+      };
+      auto clear = [&](v16f (&v)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) v[mb][r] = 0.f;
+      };
+      clear(sm);
+      if (filt_form >= 0.f) plainly(c_end, std::integral_constant<int, 2>());
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mb][r] += sm[mb][r];
       __syncthreads();
+      if (tid == 0) s_f2[4] = filt_form < 0.f ? 1.f : 0.f;
+      __syncthreads();
+      if (groups.huge()) s_f2[4] = 1.f;
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0) {      // values that three bf16 terms do not hold: all of it on the fp32 instruction
+        clear(acc);
+        plainly(0, std::integral_constant<int, 0>());
+        __syncthreads();
+      }
     }
   }
 
@@ -718,7 +809,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
   constexpr int STAGE_F = NBUF * PL * STAGE / 2, SMEM = STAGE_F > RED ? STAGE_F : RED;
   static_assert(SMEM * 4 <= 65536, "LDS budget");
   __shared__ __attribute__((aligned(16))) float smem[SMEM];
-  __shared__ float s_f2[F2 ? 5 : 1];                                  // largest values of the waves' first slots; whether a group does not fit
+  __shared__ float s_f2[F2 ? 7 : 1];                                  // as in k_upconv2x
   TL* const sbuf = reinterpret_cast<TL*>(smem);
 
   // the strips first, dealt out to the XCDs one by one: they are the longest of the workgroups; then the blocks as in k_upconv2x
@@ -866,10 +957,14 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
   };
   auto put = [&](int i, const float (&f)[8], TL* dst, auto terms) __attribute__((always_inline)) {
     if constexpr (F2) {
-      float4 pl[2] = {make_float4(f[0], f[1], f[2], f[3]), make_float4(f[4], f[5], f[6], f[7])};
-      if constexpr (decltype(terms)::value) groups.terms(f, pl);
+      constexpr int FORM = decltype(terms)::value;
+      float4 pl[FORM == 2 ? 3 : 2];
+      pl[0] = make_float4(f[0], f[1], f[2], f[3]); pl[1] = make_float4(f[4], f[5], f[6], f[7]);
+      if constexpr (FORM == 1) groups.terms(f, pl);
+      else groups.note(f);
+      if constexpr (FORM == 2) split3(f, pl);
 #pragma unroll
-      for (int q = 0; q < PL; ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
+      for (int q = 0; q < (FORM == 2 ? 3 : 2); ++q) *reinterpret_cast<float4*>(dst + q * STAGE + st_lds[i]) = pl[q];
     } else {
       *reinterpret_cast<float4*>(dst + st_lds[i]) = f32_to_slot(f, T());
     }
@@ -934,12 +1029,31 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
   }
   const long long weights = 4LL * UNITS * a.c1 * cout;
   float filt_unscale = 1.f;
-  bool filt_fits = true;
+  float filt_form = 1.f;
   if constexpr (F2) {
     const float* const end = f2_filter_end(a.filt_mc, weights);
     filt_unscale = end[0];
-    filt_fits = end[1] != 0.f;
+    filt_form = end[1] - end[2];
   }
+  int c_end = nch;
+  auto note_misfit = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) {
+      s_f2[groups.misfit() ? 4 + (c & 1) : 6] = 1.f;      // (without a branch)
+    }
+  };
+  float stop = 0.f;
+  auto ask_stop = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) stop = s_f2[4 + (c & 1)];
+  };
+  auto stops_at = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) {
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(stop)) != 0, 0)) {
+        c_end = c;
+        return true;
+      }
+    }
+    return false;
+  };
   auto flush = [&](const v16f (&from)[2], int mb, int r) __attribute__((always_inline)) {      // (F2)
     const float t = tot[mb][r], x = from[mb][r], u = t + x;
     sm[mb][r] = fmaf(x - (u - t), F2_STEP, sm[mb][r]);      // (exactly what is lost where |x| <= |t|)
@@ -965,7 +1079,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
     const int pl = i / (LS / EPS);
     *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (i - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  const auto in_terms = std::true_type();
+  const auto in_terms = std::integral_constant<int, 1>();
   {
     float f[NLD][8];
 #pragma unroll
@@ -976,7 +1090,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
       for (int i = 0; i < NLD; ++i) m = __builtin_elementwise_maximum(m, f2_amax8(f[i]));
       m = f2_wave_max(m);
       if (lane == 0) s_f2[phase] = m;
-      if (tid == 0) s_f2[4] = 0.f;
+      if (tid < 2) s_f2[4 + tid] = 0.f;
       __syncthreads();
       groups.start(f2_scale(__int_as_float(__builtin_amdgcn_readfirstlane(
           __float_as_int(__builtin_elementwise_maximum(f2_max3(s_f2[0], s_f2[1], s_f2[2]), s_f2[3]))))));
@@ -984,7 +1098,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
 #pragma unroll
     for (int i = 0; i < NLD; ++i) put(i, f[i], sbuf, in_terms);
   }
+  note_misfit(0);
   __syncthreads();
+  if (F2 && filt_form != 1.f) c_end = 0;
+  ask_stop(0);
 
   if (side == 0) {
     const TL* sin = sbuf;
@@ -1000,8 +1117,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
     };
 #pragma unroll
     for (int i = 0; i < AHEAD - 1; ++i) load_a(sin, i, av[i]);
-    for (int c = 0; c < nch; ++c) {
+    for (int c = 0; c < c_end; ++c) {
       const int cn = c + 1 < nch ? c + 1 : c;
+      if (stops_at(c)) break;
 #pragma unroll
       for (int i = 0; i < UPC; ++i) {
         const int ip = i + PD;
@@ -1029,7 +1147,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
         }
         __builtin_amdgcn_sched_barrier(0);
         if (F2 && i == UPC - 2) {
+          note_misfit(c + 1);
           __syncthreads();
+          ask_stop(c + 1);
           load_a(snext, 0, av[0]);
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1052,10 +1172,11 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
       base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF;
       step = on ? (corner ? RPS : LS) : 0;
     };
-    for (int c = 0; c < nch; ++c) {
+    for (int c = 0; c < c_end; ++c) {
       const bool more = c + 1 < nch;
       const int cn = more ? c + 1 : c;
       const TL* sin = sbuf + c % NBUF * (PL * STAGE);
+      if (stops_at(c)) break;
       if constexpr (F2) {
         if (more) stage(cn, sbuf + (c + 1) % NBUF * (PL * STAGE), in_terms);
       }
@@ -1100,7 +1221,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
         }
         base = base_n; step = step_n; g = gn; qi = qn;
       }
+      note_misfit(c + 1);
       __syncthreads();
+      ask_stop(c + 1);
     }
   }
   if constexpr (F2) {
@@ -1110,13 +1233,107 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[mb][r] = fmaf(sm[mb][r], c1, tot[mb][r] * c0);
   }
+  if constexpr (F2) {
+    // from the first chunk on that does not fit: as in k_upconv2x
+    if (__builtin_expect(c_end < nch, 0)) {
+      auto plainly = [&](int c_from, auto form) __attribute__((always_inline)) {
+        constexpr bool THREE = decltype(form)::value == 2;
+        constexpr int PA = THREE ? 3 : 2;
+        auto read = [&](const TL* gb, float4 (&b)[PL]) __attribute__((always_inline)) {
+#pragma unroll
+          for (int q = 0; q < PL; ++q) b[q] = *reinterpret_cast<const float4*>(gb + 2 * weights + b_lane + q * (2 * cout * EPS));
+        };
+        auto read_x = [&](int at, float4 (&x)[PA]) __attribute__((always_inline)) {
+#pragma unroll
+          for (int q = 0; q < PA; ++q) x[q] = *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at]);
+        };
+        auto unit = [&](const float4 (&b)[PL], const float4 (&x0)[PA], const float4 (&x1)[PA], auto block) __attribute__((always_inline)) {
+          if constexpr (THREE) {
+            float4 b3[3];
+            split3_raw(b, b3);
+            if constexpr (decltype(block)::value) {
+              mma_up2x_x3(acc[0], acc[1], sm[0], sm[1], x0, x1, b3);
+            } else {
+              mma_unit(sm[0], x0[2], b3[0], mie_bf16()); mma_unit(sm[0], x0[1], b3[1], mie_bf16());
+              mma_unit(acc[0], x0[0], b3[0], mie_bf16()); mma_unit(sm[0], x0[0], b3[2], mie_bf16());
+              mma_unit(sm[0], x0[1], b3[0], mie_bf16()); mma_unit(sm[0], x0[0], b3[1], mie_bf16());
+            }
+          } else {
+#pragma unroll
+            for (int q = 0; q < PL; ++q) {
+              mma_unit(acc[0], x0[q], b[q], float());
+              if constexpr (decltype(block)::value) mma_unit(acc[1], x1[q], b[q], float());
+            }
+          }
+        };
+        for (int c = c_from; c < nch; ++c) {
+          __syncthreads();
+          stage(c, sbuf, form);
+          if (tid < PA * (LS / EPS)) {
+            const int pl = tid / (LS / EPS);
+            *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (tid - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
+          }
+          __syncthreads();
+          for (int qi = 0; qi < NQ; ++qi) {
+            if (side == 0) {
+              const TL* const gb = group_b(c, qi, 0);
+              float4 br[4][PL];
+#pragma unroll
+              for (int j = 0; j < 3; ++j) read(gb + j * unit_sz, br[j]);
+              float4 xv[2][2][PA];
+#pragma unroll
+              for (int mb = 0; mb < 2; ++mb) read_x(a_lane[mb] + SUB * qi, xv[0][mb]);
+#pragma unroll 1
+              for (int ky = 0; ky < 4; ++ky) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                  const int ahead = 4 * ky + j + 3;
+                  read(gb + (ahead < 16 ? ahead : 15) * unit_sz, br[(j + 3) & 3]);
+                  const int k = (4 * ky + j + 1) & 15, at = (k >> 2) * RP + (k & 3) * LS + SUB * qi;
+#pragma unroll
+                  for (int mb = 0; mb < 2; ++mb) read_x(a_lane[mb] + at, xv[(j + 1) & 1][mb]);
+                  __builtin_amdgcn_sched_barrier(0);
+                  unit(br[j], xv[j & 1][0], xv[j & 1][1], std::true_type());
+                }
+              }
+            } else {
+#pragma unroll 1
+              for (int g = 0; g < ng; ++g) {
+                const int code = (int)((strip >> (4 * g)) & 15u);
+                const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
+                const int base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF, step = on ? (corner ? RPS : LS) : 0;
+#pragma unroll 1
+                for (int t = 0; t < (corner ? 3 : 4); ++t) {
+                  float4 b[PL];
+                  read(group_b(c, qi, strip_unit(g) + t), b);
+                  float4 x[PA];
+                  read_x(base + t * step, x);
+                  unit(b, x, x, std::false_type());
+                }
+              }
+            }
+          }
+        }
+      };
+      sm[0] = sm[1] = zero;
+      if (filt_form >= 0.f) plainly(c_end, std::integral_constant<int, 2>());
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mb][r] += sm[mb][r];
+      __syncthreads();
+      if (tid == 0) s_f2[4] = filt_form < 0.f ? 1.f : 0.f;
+      __syncthreads();
+      if (groups.huge()) s_f2[4] = 1.f;
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0) {      // values that three bf16 terms do not hold: all of it on the fp32 instruction
+        acc[0] = acc[1] = zero;
+        plainly(0, std::integral_constant<int, 0>());
+        __syncthreads();
+      }
+    }
+  }
   float* const red = smem + phase * (64 * CO_BLK);
-  auto park = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) red[(mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3)) * CO_BLK + l32] = acc[mb][r];
-  };
   // ---- epilogue: as in k_upconv2x, but that every wave parks whole sums ------------------------------------------------------
   long long off[PB];
   int co[PB];
@@ -1134,56 +1351,11 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
     conv_epilogue_load4<T, PB>(a, off, live, r0, add);
   };
   fetch(0);
-  if constexpr (F2) {
-    if (groups.misfit() || !filt_fits) s_f2[4] = 1.f;
-  }
-  park();
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) red[(mb * 32 + 8 * (r >> 2) + 4 * half + (r & 3)) * CO_BLK + l32] = acc[mb][r];
   __syncthreads();
-  if constexpr (F2) {
-    if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(s_f2[4])) != 0, 0)) {
-      // a group that does not fit: all of it once more on the fp32 instruction (see k_upconv2x)
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb) acc[mb] = zero;
-      for (int c = 0; c < nch; ++c) {
-        __syncthreads();
-        stage(c, sbuf, std::false_type());
-        if (tid < 2 * (LS / EPS)) {
-          const int pl = tid / (LS / EPS);
-          *reinterpret_cast<float4*>(sbuf + pl * STAGE + ZOFF + EPS * (tid - pl * (LS / EPS))) = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        __syncthreads();
-        auto unit = [&](const TL* gb, int at0, int at1) __attribute__((always_inline)) {
-#pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            const float4 b = *reinterpret_cast<const float4*>(gb + 2 * weights + b_lane + q * (2 * cout * EPS));
-            mma_unit(acc[0], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at0]), b, float());
-            if (side == 0) mma_unit(acc[1], *reinterpret_cast<const float4*>(&sbuf[q * STAGE + at1]), b, float());
-          }
-        };
-        for (int qi = 0; qi < NQ; ++qi) {
-          if (side == 0) {
-#pragma unroll 1
-            for (int k = 0; k < 16; ++k) {
-              const int at = (k >> 2) * RP + (k & 3) * LS + SUB * qi;
-              unit(group_b(c, qi, k), a_lane[0] + at, a_lane[1] + at);
-            }
-          } else {
-#pragma unroll 1
-            for (int g = 0; g < ng; ++g) {
-              const int code = (int)((strip >> (4 * g)) & 15u);
-              const bool corner = code >= 3, on = !corner || (code == 3 ? at_first : at_last);
-              const int base = on ? a_lane[0] + (corner ? jx * LS : code * RPS) + SUB * qi : ZOFF, step = on ? (corner ? RPS : LS) : 0;
-#pragma unroll 1
-              for (int t = 0; t < (corner ? 3 : 4); ++t) unit(group_b(c, qi, strip_unit(g) + t), base + t * step, 0);
-            }
-          }
-        }
-      }
-      __syncthreads();
-      park();
-      __syncthreads();
-    }
-  }
 #pragma unroll
   for (int h0 = 0; h0 < PER; h0 += PB) {
     if (h0 > 0) fetch(h0);

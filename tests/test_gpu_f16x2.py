@@ -349,3 +349,65 @@ def test_leading_channels_zero_transposed(c1, c2, cout, h, w, k, setting):
         ref, bound = _tconv_ref(x, wt, k)
         e = (_tconv(x, c1, wt, k, "f16x2") - ref).abs()
         assert (e <= 4e-7 * bound).all(), (scale, (e / bound).max())
+
+
+@pytest.mark.parametrize("cin,cout,k,stride,h,w,c1", SHAPES)
+def test_channels_of_many_sizes(cin, cout, k, stride, h, w, c1, setting):
+    """Channels of 1 ... 2^8 and of 1 ... 2^30, growing and falling, which end the contraction in two terms at a chunk in the middle.  Where a few
+    channels make up the sums, all roundings of a chain are at their size: three terms are up to 7.4e-7 of sum |x||w| from fp64, 1.1e-6 of the
+    norm.  So: no further than these, or 4e-7 as above; of the norm, with one rounding more at the size of the sum, where the two sets of
+    sums meet, and the chains of the one-launch form, which three terms of growing channels keep to 0.9e-7: 1.4 times."""
+    g = torch.Generator().manual_seed(cin + 11)
+    x0, wt = torch.randn(1, cin, h, w, generator=g), he_normal_conv_weight(cout, cin, k, 7)
+    for top in (8.0, 30.0):
+        for order in (torch.arange(cin), torch.arange(cin).flip(0), torch.randperm(cin, generator=g)):
+            x = x0 * (2.0 ** (top * order / cin)).view(1, -1, 1, 1)
+            ref = F.conv2d(x.double(), wt.double(), stride=stride, padding=k // 2)
+            bound = F.conv2d(x.double().abs(), wt.double().abs(), stride=stride, padding=k // 2)
+            e, e3 = ((_conv(x, wt, k, stride, mode, c1) - ref).abs() for mode in ("f16x2", "bf16x3"))
+            assert (e / bound).max() <= max(4e-7, (e3 / bound).max()) and e.norm() <= 1.4 * e3.norm(), (top, (e / bound).max(), e.norm() / e3.norm())
+
+
+def _graph_us(f):
+    """us of a call, the least of eight replays of twenty."""
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        f()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            for _ in range(20):
+                f()
+    graph.replay()
+    best = float("inf")
+    for _ in range(8):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        graph.replay()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 50.0)
+    return best
+
+
+@pytest.mark.parametrize("what", ["channels", "pixels", "filter"])
+def test_decoders_that_do_not_fit_take_about_as_long_as_in_three_terms(what, setting):
+    """256->128 at 33x44: 47, 65 and 65 us against 42; as two contractions, the second on the fp32 instruction, 120."""
+    c, cout, h, w = 256, 128, 33, 44
+    g = torch.Generator().manual_seed(3)
+    a, wt = torch.randn(1, c, h, w, generator=g), he_normal_conv_weight(cout, c, 5, 7)
+    if what == "channels":
+        a = a * (2.0 ** (8.0 * torch.arange(c) / c)).view(1, -1, 1, 1)
+    elif what == "pixels":
+        a[:, :, 1::2] *= 2.0 ** -28
+    else:
+        wt[3] *= 1e-12
+    ts_up, ts = TileMask(1, 2 * h, 2 * w, DEV), TileMask(1, 2 * h, 2 * w, DEV)
+    ops.build_mask_tiles(None, None, 1, h, w, _lib.FOOT_UP2X, 0, 0, 0, ts_up)
+    ops.build_mask_tiles(ts_up, None, 1, 2 * h, 2 * w, _lib.FOOT_CONV, 5, 1, 2, ts)
+    out, filt, x = ops.new_nhwc(1, cout, 2 * h, 2 * w, DEV), _filt(wt), _dev(a)
+    us = {}
+    for mode in ("bf16x3", "f16x2"):
+        ops.f32_matmul = mode
+        us[mode] = _graph_us(lambda: ops.upconv2x_masked(x, None, x, None, filt, ts, out))
+    assert us["f16x2"] < 2.0 * us["bf16x3"], us
