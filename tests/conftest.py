@@ -36,8 +36,8 @@ def mie_lib():
 
 @pytest.fixture(autouse=True)
 def _f32_matmul_mode(request):
-    """Tests parametrized over `f32mode` run with ops.f32_matmul set to it: "bf16x3" (fp32 deltas multiplied as three
-    bf16 terms on the bf16 matrix-core instruction, the default) or "native" (the fp32 instruction)."""
+    """Tests parametrized over `f32mode` run with ops.f32_matmul set to it: "f16x2" (fp32 deltas multiplied as two fp16 terms, the default), "bf16x3" (as three
+    bf16 terms) or "native" (the fp32 instruction)."""
     spec = getattr(request.node, "callspec", None)
     mode = spec.params.get("f32mode") if spec is not None else None
     if mode is None:

@@ -174,7 +174,7 @@ def test_config2_activation_chain_50_steps(density):
 
 @pytest.mark.parametrize("fused", [True, False])
 @pytest.mark.parametrize("cin,hid", [(16, 16), (32, 32), (64, 32)])
-@pytest.mark.parametrize("f32mode", ["bf16x3", "native"])
+@pytest.mark.parametrize("f32mode", ["f16x2", "bf16x3", "native"])
 def test_convlstm_module_matches_oracle(fused, cin, hid, f32mode):
     # (32, 32) and (64, 32) take the conv + gate chain kernel when fused, (16, 16) the two-kernel form
     n, h, w = 1, 26, 34
@@ -306,7 +306,7 @@ def test_e2depth_refresh_runs_on_the_library_kernels_and_replays_as_a_graph():
 
 
 @pytest.mark.parametrize("fuse", [True, False])
-@pytest.mark.parametrize("f32mode", ["bf16x3", "native"])
+@pytest.mark.parametrize("f32mode", ["f16x2", "bf16x3", "native"])
 def test_e2depth_incr_small_matches_oracle(fuse, f32mode):
     _run_e2depth(72, 104, steps=4, density=0.05, fuse=fuse)
 
@@ -375,7 +375,7 @@ def test_e2depth_incr_empty_frames_between_active_ones():
 
 
 @pytest.mark.parametrize("cin,hid,h,w", [(128, 128, 16, 8), (64, 64, 12, 20), (256, 256, 8, 8)])
-@pytest.mark.parametrize("f32mode", ["bf16x3", "native"])
+@pytest.mark.parametrize("f32mode", ["f16x2", "bf16x3", "native"])
 @pytest.mark.parametrize("one_launch", [False, True])
 def test_convlstm_on_a_small_plane_splits_the_gates_conv(cin, hid, h, w, f32mode, one_launch):
     # planes of few tiles: the gates conv runs as a split contraction (partial sums in the workspace) and the gate
@@ -415,7 +415,7 @@ def test_convlstm_on_a_small_plane_splits_the_gates_conv(cin, hid, h, w, f32mode
             assert torch.isfinite(dh[0]).all() and torch.isfinite(dc[0]).all()
             _close(dh[0], dh_r, "%s dh %d" % (what, step)), _close(dc[0], dc_r, "%s dc %d" % (what, step))
     plane = n * h * w * 4 * hid
-    if one_launch and f32mode == "bf16x3":
+    if one_launch and f32mode != "native":
         assert not torch.isfinite(ws).any()
     else:
         assert torch.isfinite(ws[:plane]).any() and torch.isfinite(ws[plane:2 * plane]).any()      # the split form ran
