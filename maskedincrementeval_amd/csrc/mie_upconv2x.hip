@@ -860,8 +860,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
   const int* const flags_n = reinterpret_cast<const int*>(od.flags) + (long long)n * a.ts.tiles_y * a.ts.tiles_x;
   // item g of a thread: four channels of phase g / 2 of position 32 * (g % 2) + tid / 8
   constexpr int PER = 8, PB = 4;
+  int item = tid;
   auto pixel = [&](int g, int& oy, int& ox) __attribute__((always_inline)) -> bool {
-    const int p = 32 * (g & 1) + (tid >> 3), dy = pos_y(p), dx = pos_x(p);
+    const int p = 32 * (g & 1) + (item >> 3), dy = pos_y(p), dx = pos_x(p);
     oy = 2 * (y0 + dy) + (g >> 2); ox = 2 * (x0 + dx) + ((g >> 1) & 1);
     return dy < rows && dx < cols;
   };
@@ -1345,11 +1346,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(Co
       int oy, ox;
       ok[i] = pixel(h0 + i, oy, ox);
       live[i] = ((live_bits >> (h0 + i)) & 1u) != 0;
-      off[i] = (((long long)n * hout + oy) * wout + ox) * cout + co0 + col;
-      co[i] = co0 + col;
+      co[i] = co0 + 4 * (item & 7);
+      off[i] = (((long long)n * hout + oy) * wout + ox) * cout + co[i];
     }
     conv_epilogue_load4<T, PB>(a, off, live, r0, add);
   };
+  asm volatile("" : "+v"(item));      // (its places anew: kept from the start they would be spilled across the contraction)
   fetch(0);
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
