@@ -595,16 +595,30 @@ class NetBench:
         return roofline
 
     def _products(self, layer):
-        """Term products per multiply of a launch that ran in terms (decoders at the resolution of their inputs: three or six)."""
+        """Term products per multiply of a launch that ran in terms: three, or six where the library has three terms (decoders at the
+        resolution of their inputs as it says; one-launch forms but for 3x3 of 512 channels and more)."""
         import re
         if self.ops.f32_matmul == "bf16x3":
             return 6
-        m = re.search(r"(\d+)->(\d+) @(?:(\d+)x)?(\d+)x(\d+)", layer["shape"])
-        if not layer["op"].startswith("upconv2x") or m is None:
+        m = re.search(r"(\d)x\d s(\d) (\d+)->(\d+)\S* @(\d+)x(\d+)", layer["shape"])
+        if m is None:
             return 3
-        from maskedincrementeval_amd._lib import lib
-        c, cout, n, h, w = (int(v or 1) for v in m.groups())
-        return 3 if lib().mie_f16x2_takes_upconv2x(n, h // 2, w // 2, c, cout) else 6
+        from maskedincrementeval_amd import _lib
+        lib, code = _lib.lib(), _lib.DTYPE_F32_F16X2
+        k, s_, c, cout, h, w = (int(v) for v in m.groups())
+        tiles, op = layer["tiles"], layer["op"]
+        n = max(1, tiles // _lib.tile_capacity(1, h, w))
+        if op.startswith("upconv2x"):
+            return 3 if lib.mie_f16x2_takes_upconv2x(n, h // 2, w // 2, c, cout) else 6
+        if op.startswith("upconv"):
+            one = lib.mie_upconv_needs_no_workspace(c, cout, tiles, code)
+        elif op.startswith("tconv"):      # (slabs of 16 columns of the blocks of 16x16 pixels)
+            one = k == 3 and c >= 128 and _lib.tile_capacity(n, (h + 1) // 2, (w + 1) // 2) * (cout // 16) <= 256
+        elif op.startswith("conv_gates"):
+            one = lib.mie_conv_gates_needs_no_workspace(c, 0, cout // 4, tiles, code)
+        else:
+            one = lib.mie_conv_needs_no_workspace(k, s_, c, 0, cout, tiles, code)
+        return 6 if one and not (k == 3 and s_ == 1 and c >= 512 and not op.startswith("tconv")) else 3
 
     def _takes_x3(self, layer):
         """Whether the launch of a per-launch table row ran in terms (its shape string is
