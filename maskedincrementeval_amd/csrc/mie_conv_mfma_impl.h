@@ -227,7 +227,7 @@ __device__ __forceinline__ void split3(const float (&f)[8], float4 (&pl)[3]) {
 // v_mfma_f32_32x32x2_f32.  us where all fit | all but the first chunk's channels 2^8 larger | half the pixels 2^-28 of the others, no chunk fits
 // | three terms: 3x3 256->256 at 33x44 13.6 | 17.5 | 20.6 | 16.6, 64->64 at 132x176 14.4 | 18.1 | 20.8 | 16.8, 5x5 stride 2 128->256 at 66x88 17.3 |
 // 22.1 | 25.9 | 23.5 (both contractions one after the other, the second on the fp32 instruction: 34, 32 and 45).  The look at every chunk costs
-// 0.2-0.3 us a launch; at the end only, it would cost the whole of the two terms' contraction once more.
+// 0.1-0.2 us a launch; at the end only, it would cost the whole of the two terms' contraction once more.
 // The filter's scale takes its largest weight to [2^14, 2^15); a filter one of whose groups of eight input channels lies below 2^-29
 // of it is marked, and contracted in three terms from the first chunk on.
 typedef _Float16 mie_f16x2 __attribute__((ext_vector_type(2)));
@@ -1047,19 +1047,14 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
       s_f2[groups.misfit() ? WAVES + ((c - c_lo) & 1) : WAVES + 2] = 1.f;      // (without a branch)
     }
   };
-  // ... asked behind it whether some thread noted one, and looked at where the chunk begins (true: it does not fit)
+  // ... asked behind it whether some thread noted one, and looked at where chunk c would begin.  (As a part of the loop's own condition: a break of
+  // its own costs twice as much, 0.3 us a launch)
   float stop = 0.f;
   auto ask_stop = [&](int c) __attribute__((always_inline)) {
     if constexpr (F2) stop = s_f2[WAVES + ((c - c_lo) & 1)];
   };
-  auto stops_at = [&](int c) __attribute__((always_inline)) {
-    if constexpr (F2) {
-      if (__builtin_expect(__builtin_amdgcn_readfirstlane(__float_as_int(stop)) != 0, 0)) {
-        c_end = c < c_end ? c : c_end;
-        return true;
-      }
-    }
-    return false;
+  auto stop_before = [&](int c) __attribute__((always_inline)) {
+    if constexpr (F2) c_end = __builtin_amdgcn_readfirstlane(__float_as_int(stop)) != 0 && c < c_end ? c : c_end;
   };
   MIE_STAMP(2);
   const bool early = c_hi - c_lo >= 4;      // uniform over the workgroup
@@ -1188,8 +1183,8 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
     const TL* sin = sbuf;
     TL* snext = sbuf + PL * STAGE;
     load_a(sin, 0, av0);
+    stop_before(c_lo);
     for (int c = c_lo; c < c_end; ++c) {
-      if (stops_at(c)) break;
 #pragma unroll
       for (int i = 0; i < UPC; ++i) {
         const int ip = i + PD;
@@ -1232,16 +1227,17 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
       TL* const t = const_cast<TL*>(sin);
       sin = snext;
       snext = t;
+      stop_before(c + 1);
       MIE_STAMP(4 + (c - c_lo));
     }
   } else if constexpr (PIPE) {
     float4 av[2][2][PL], av0[2][PL];
     load_a(sbuf, 0, av0);
+    stop_before(c_lo);
     for (int c = c_lo; c < c_end; ++c) {
       const bool more = c + 1 < c_hi;
       const TL* sin = sbuf + ((c - c_lo) & 1) * (PL * STAGE);
       const TL* sin_next = sbuf + ((c - c_lo + 1) & 1) * (PL * STAGE);
-      if (stops_at(c)) break;
 #pragma unroll
       for (int i = 0; i < UPC; ++i) {
         if (PD > 0) {
@@ -1275,12 +1271,13 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
         }
       }
       ub_cur = ub_next;
+      stop_before(c + 1);
       MIE_STAMP(4 + (c - c_lo));
     }
     // (the epilogue reuses the staging buffers: every read of them that matters was waited for in front of the
     // last barrier; the operand read behind it returns whatever a faster wave has parked there, and is dropped)
   } else {
-    stops_at(c_lo);
+    stop_before(c_lo);
     for (int c = c_lo; c < c_end; ++c) {
       const bool more = c + 1 < c_hi;
       const int cn = more ? c + 1 : c;      // after the last chunk: redundant re-load, never stored
@@ -1311,7 +1308,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, conv_min_waves((int)sizeof(T), K,
       note_misfit(c + 1);
       __syncthreads();
       ask_stop(c + 1);
-      stops_at(c + 1);
+      stop_before(c + 1);
       ub_cur = ub_next;
       MIE_STAMP(4 + (c - c_lo));
     }
