@@ -937,7 +937,11 @@ bool mie_upconv_deep_form(int c, int cout, long long tiles, int dtype) {
 //   5x5 s2        160 .96, 192 1.04  160 .91, 256 1.10  256 .98, 320 1.01  448 .99, 512 1.4    384 .98, 448 1.09   320 .92, 384 1.07
 //   gates         640 .91, 768 1.02  1024 .93, 1536 1.07  512 .76          2048 .94, 2560 1.04  3072 .83           3072 .73
 //   up            128 .84            128 .89            (none)             448 .97, 512 1.28   384 .87, 448 1.01   512 .99, 768 1.07
-// (3x3 fp32 of eight rows: 384 and 512, which fill its passes of four chunks, .98 and 1.01; 448 1.05.)  Far above it, 5x5 stride 2
+// (3x3 fp32 of eight rows: 384 and 512, which fill its passes of four chunks, .98 and 1.01; 448 1.05.)
+// The fp32 lines are of three terms in both forms.  With MIE_DTYPE_F32_F16X2, whose split form runs in two, medians of four layers a cell: 3x3 of
+// two rows 448 .99, 512 and more (in two terms here, too) .87 to 1.01, four 256 .89, 320 1.03, 448 1.04, 512 .89, eight 128 .85, 192 1.05, 256 1.01, 384 1.12,
+// 512 1.15; 5x5 s2 160 .97, 128 .99 and 160 1.04, 96 .99, 128 1.07 and 256 1.25; gates 1024 .97, 1024 1.01, 256 .98, 512 1.04; up 128 .93.  So
+// with it 5x5 s2 and 3x3 of eight rows would go to the split form earlier.  Far above it, 5x5 stride 2
 // of 512 / 1024 channels: fp32 1.6 / 2.1, up to 2.9 times as long, bf16 1.4 / 2.0.
 bool mie_conv_deep_faster(int k, int s, int c1, int c2, int cout, long long tiles, int dtype, bool gates) {
   if (!mie_conv_deep_form(k, s, c1, c2, cout, tiles, dtype)) return false;

@@ -5,9 +5,9 @@
 // with v_mfma_f32_32x32x16_bf16 (fp32 accumulation, fp32 reservoirs).  The two element types share
 // one kernel: every operand access is a 16-byte access, which holds 4 fp32 or 8 bf16 channels, so
 // the bf16 kernel is the fp32 kernel with twice the channels per LDS stage, per unit and per load.
-// The text below gives the fp32 numbers.  A third form, X3, multiplies fp32 deltas on the bf16 instruction at fp32
-// accuracy (three bf16 terms per value, six term products per multiply): it is described at the kernel template and
-// is what fp32 deltas take by default wherever it exists.
+// The text below gives the fp32 numbers.  Two more forms multiply fp32 deltas at fp32 accuracy on the 16-bit instructions: X3 (three
+// bf16 terms per value, six term products per multiply; described at the kernel template) and F2 (two fp16 terms, three products; described
+// beside split2), which is what fp32 deltas take by default wherever it exists.
 //
 // Work decomposition.  One 256-thread workgroup (4 waves) computes one active
 // 8x8 output tile (M = 64 pixels) x CO_BLK output channels as an implicit GEMM
@@ -1897,7 +1897,7 @@ unsigned xcd_plan(ConvArgsT<T>& a, unsigned cap, int nslabs, int k, bool up = fa
 // (129 .. 256): measured on MI355X, one workgroup per CU with twice the columns beats one and a half rounds of the
 // narrow ones (5x5 256->128 at 66x88: 198 workgroups of 64 columns 61-65 us, 396 of 32 columns 71-74 us; 3x3 gates conv
 // 256+256->1024 at 33x44: 240 of 128 columns 53 us, 480 of 64 columns 57 us); at stride 2, whose workgroups are short,
-// it does not (28 vs 29 us).
+// it does not (28 vs 29 us).  (All in three terms; in two the same rule.)
 inline int pick_slab_x3(int cout, unsigned cap, int s) {
   const bool ok128 = cout % 128 == 0, ok64 = cout % 64 == 0, ok32 = cout % 32 == 0;
   const int f = forced_slab();
@@ -1925,8 +1925,7 @@ inline bool x3_takes(int k, int s, int c1, int c2, int cout) {
 // Two terms: eight waves a workgroup, chunks of twice the channels (WIDE).  Where the workgroups are one round of the chip, one a CU, a CU has one
 // wave a SIMD with four, and nothing runs while it waits.  us, four waves -> eight, every tile active, filters cold: 3x3 256->256 at 33x44
 // (240 workgroups) 12.4 -> 12.05, 256->512 there 17.3 -> 16.7; 5x5 stride 2 (which is then double-buffered, too) 128->256 at 66x88 18.4 -> 15.4,
-// 64->128 at 80x100 11.6 -> 10.5.  (What is left of a 3x3 layer: a third is its head and tail, the rest runs at 0.8 of what the L1 delivers
-// of filter and input.)  Not for fewer channels: 3x3 64->64 at 66x88 6.9 and 7.2; nor for slabs of 128
+// 64->128 at 80x100 11.6 -> 10.5.  Not for fewer channels: 3x3 64->64 at 66x88 6.9 and 7.2; nor for slabs of 128
 // columns, whose four waves are busy as they are (gates of 256+256 at 33x44 31 and 33 in a trace, frames the same).  A second round of such workgroups is no better than
 // two of four waves a CU side by side (5x5 stride 2 64->128 at 132x176, 64 columns wide so that it is one: 15.7 and 14.7 alone, a frame the same);
 // the ConvGRU's gates, likewise, the same.  Frame of 264x352 342 -> 335 us, planned ahead 328 -> 320, refresh 386 -> 378.

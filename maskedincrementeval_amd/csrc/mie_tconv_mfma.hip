@@ -553,7 +553,7 @@ bool launch_tconv(const ConvArgsT<T>& a0, const TileSetDev& pts, hipStream_t st)
   const unsigned cap_p = (unsigned)(pts.n * pts.tiles_y * pts.tiles_x);
   const int cout = a0.cout;
   // The one-launch form takes every launch of its types that could be split, but for fp32 of so many channels that the split contraction
-  // makes up for its second launch.  One launch over split, 2 to 64 slabs: 1280 channels .89 to 1.05, 1408 .88 to 1.11, 1536 .92 to 1.17,
+  // makes up for its second launch.  One launch over split, three terms in both, 2 to 64 slabs: 1280 channels .89 to 1.05, 1408 .88 to 1.11, 1536 .92 to 1.17,
   // 2048 1.04 to 1.31; 128 slabs of four tiles or fewer, 1536 .97 to 1.18, 2048 1.05 to 1.26, of more .75 to .97 (bf16 of 2048: .5 to 1.0).
   const bool split = !DEEP || (X3 && a0.g_cpd == nullptr && a0.c1 + a0.c2 > 1408 && (long long)cap_p * (cout / 16) <= (cap_p <= 4 ? 128 : 64));
   ConvArgsT<T> a = ARITH == 2 ? f2_args(a0, K) : a0;

@@ -776,10 +776,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
 }
 
 // The same with all four phases of a block (or strip) in one workgroup, a phase to a wave x 32 output channels, for fp32 deltas in two fp16
-// terms and for bf16 ones of 64 channels (one chunk: nothing but the loop over its 64 units): the window (12x12 pixels, 3 rows of 36) is loaded, added up and split once instead of four times, and the waves' sums do not
-// have to meet in LDS -- what layers of few channels spend their time on, whose workgroups in k_upconv2x are two or three chunks long
-// between a prologue and an exchange (64->32 at 132x176, all tiles active: 1580 workgroups there, 50 us, of which the matrix cores have
-// work for 19; here 396).
+// terms and for bf16 ones of 64 channels (one chunk).  The window (12x12 pixels, 3 rows of 36) is loaded, added up and split once instead of
+// four times, and the waves' sums do not have to meet in LDS: what layers of few channels spend their time on, whose workgroups in k_upconv2x
+// are two or three chunks long between a prologue and an exchange (64->32 at 132x176, all tiles active: 1580 workgroups there, 50 us; here
+// 396, 31 us, 37 with reservoir and activation, of which the matrix cores are busy for a third).
 //
 // fp32 sums.  With all of K in one wave the chain of roundings at the size of the sum would be four times as long, and the fp16 leading terms
 // fill the accumulator's 24 bits where bf16 ones do not (in one chain 64 channels are 1.41e-7 from fp64, relative 2-norm, k_upconv2x in
@@ -788,8 +788,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x(ConvAr
 // channels (BL = 8 1.15e-7, 16 1.35e-7; without the carry 1.28, 1.27 and 1.41e-7).  Four VALU instructions a value, 128 a block, beside
 // 24 MFMAs of 32 cycles.
 //
-// The next chunk is staged a slot at a time, its loads ten units ahead of its LDS writes (16 registers instead of 48).  What is left
-// above the matrix cores' time (22 us with LDS, filter and input reads taken out): the loads of the next chunk (5), its split (3), A (3).
+// The next chunk is staged a slot at a time, its loads ten units ahead of its LDS writes (16 registers instead of 48).
 template <typename T>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 2 : 3) void k_upconv2x_all(ConvArgsT<T> a, Up2xOrder od) {
   constexpr bool F2 = sizeof(T) == 4;
@@ -1396,25 +1395,26 @@ void launch_one(const ConvArgsT<T>& a, Up2xOrder od, hipStream_t st) {
   }
 }
 
-// Slab width, by how many rounds of workgroups it takes.  A 64-column workgroup takes 1.75 times as long as a 32-column one.
-// fp32 (three-term): one workgroup fills a CU's matrix cores (two take twice as long), so a round is 256: 64 columns where they
-// need half the rounds or close to it, which leaves 32 columns up to one round (256->128 at 20x20: 26 us against 39) and in
-// the third (at 42x46, 608 of them: 68 against 78; at 33x44, 480: 48 against 45; at 60x80 134 against 122).  In two terms 64 columns
-// from one round on (256->128 at 25x35 29.9 against 27.7, at 42x46 45.4 and 46.5, 128->64 at 80x100 48.3 and 45.1; at 20x20 21.8 against 28.1).  bf16: workgroups
-// are short and three of a CU hide each other's latencies, so 64 columns start where 32 no longer fit one round of
-// 768 (128->64 at 66x74, 656 of them: 15.7 against 17.2; at 66x88, 784: 20.4 against 17.7), 128 columns, which read the
-// input least, where they make more than a round themselves (256->128 at 8x60x80: 246 against 217; at 4x60x80, 1440: 126
-// against 116; at 3x60x80, 1080: 92 either way; at 8x30x40, 832: 76 against 83).
-// k_upconv2x_all or k_upconv2x (wgs: of 32 columns, of the latter).
-// fp32: where the latter needs more workgroups than two to a CU, and the layer has 64 or 96 channels.  64->32 at 80x112 (608 of them) 22.2 ->
-// 19.1 us, at 132x176 (1584) 50 -> 32, at 240x320 137 -> 87; 64->64 at 64x64 (576) 22 -> 18.8, 96->32 at 96x96 31 -> 24.4; at 72x80 (400)
-// 15.7 against 18.1.  (Against k_upconv2x in three terms: in two it would be faster, too, but 1.13 and 1.05 times as far from fp64 with 64 and
-// 96 channels.)  From 128 channels on, in two terms either way, a workgroup here is longer than the launch is wide: 128->64 at
-// 66x88 29.3 against 32, at 120x160 78 against 87, 256->128 at 60x80 86 against 96.  In one chunk of 32 channels three terms are as near:
-// 9.94e-8 and 1.00e-7.  Planes of two rows or columns are all strips.
-// bf16: 64 channels, whose other form is the list-driven one (k_conv_mfma<..., UP>, k_upconv64_persist), from more workgroups here than
-// CUs on: 64->32 at 120x140 20.7 -> 17.7, at 2x100x140 27.0 -> 20.6, at 160x160 26.4 -> 19.7, 64->64 at 100x140 26.4 -> 20.6, 64->32 at
-// 8x240x320 374 -> 308; in between (128x128 17.4 and 17.2, 116x132 16.9 and 17.1) and below (96x96 13.3 and 13.6) either way.
+// Slab width of k_upconv2x, by how many rounds of workgroups it takes.  A 64-column workgroup takes 1.75 times as long as a 32-column one.
+//   * fp32, three terms: one workgroup fills a CU's matrix cores (two take twice as long), so a round is 256: 64 columns where they need half
+//     the rounds or close to it, which leaves 32 columns up to one round (256->128 at 20x20: 26 us against 39) and in the third (at
+//     42x46, 608 of them: 68 against 78; at 33x44, 480: 48 against 45; at 60x80 134 against 122).
+//   * two terms: 64 columns from one round on (256->128 at 25x35 29.9 against 27.7, at 42x46 45.4 and 46.5, 128->64 at 80x100 48.3 and 45.1;
+//     at 20x20 21.8 against 28.1).
+//   * bf16: workgroups are short and three of a CU hide each other's latencies, so 64 columns start where 32 no longer fit one round of
+//     768 (128->64 at 66x74, 656 of them: 15.7 against 17.2; at 66x88, 784: 20.4 against 17.7), 128 columns, which read the input least,
+//     where they make more than a round themselves (256->128 at 8x60x80: 246 against 217; at 4x60x80, 1440: 126 against 116; at 3x60x80,
+//     1080: 92 either way; at 8x30x40, 832: 76 against 83).
+//
+// k_upconv2x_all or k_upconv2x (wgs: of 32 columns, of the latter):
+//   * fp32: where the latter, in three terms, needs more workgroups than two to a CU, and the layer has 64 or 96 channels.  64->32 at 80x112
+//     (608 of them) 22.2 -> 19.1 us, at 132x176 (1584) 50 -> 31, at 240x320 137 -> 87; 64->64 at 64x64 (576) 22 -> 18.8, 96->32 at 96x96
+//     31 -> 24.4; at 72x80 (400) 15.7 against 18.1.  (k_upconv2x in two terms would be 1.13 and 1.05 times as far from fp64 with 64 and 96
+//     channels.)  From 128 channels on, in two terms either way, a workgroup here is longer than the launch is wide: 128->64 at 66x88
+//     29.3 against 32, at 120x160 78 against 87, 256->128 at 60x80 86 against 96.  In one chunk of 32 channels three terms are as near:
+//     9.94e-8 and 1.00e-7.  Planes of two rows or columns are all strips.
+//   * bf16: 64 channels, from more workgroups here than CUs on.  (For calls of this form; networks keep the list-driven one for these
+//     layers, which holds a + b in 32 bits up to the blend.)
 bool up2x_all(int c, long long wgs, const Up2xOrder& od, bool bf) {
   return (bf ? c == 64 && wgs > 1024 : c >= 64 && c < 128 && wgs > 512) && od.blocks_y * od.blocks_x > 0;
 }

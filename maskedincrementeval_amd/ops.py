@@ -1494,8 +1494,8 @@ def gru_interleave_index(hid: int, device=None) -> torch.Tensor:
 def conv_gru_takes(cin: int, cin_total: int, hid: int, dtype, tiles: int = 0) -> bool:
     """Whether conv_gru_incr has a kernel for the layer and is the faster form (else: conv_masked + convgru_gates_incr): `cin` channels
     of input, a filter of `cin_total`, `tiles` of the plane (0: not asked).  It is not for fp32 layers of many channels on planes so
-    small that conv_masked splits the contraction: in one launch a workgroup has all of it.  One launch over two, medians of 3 to 12
-    layers: up to 128 slabs (16 columns x a tile) 1024 channels .97, 1536 1.18, 2048 1.30; up to 256 slabs, 512 channels .92, 576 1.19, 1024 1.38
+    small that conv_masked splits the contraction: in one launch a workgroup has all of it.  One launch over two, three terms in both, medians of
+    3 to 12 layers: up to 128 slabs (16 columns x a tile) 1024 channels .97, 1536 1.18, 2048 1.30; up to 256 slabs, 512 channels .92, 576 1.19, 1024 1.38
     (bf16: 2048 channels .88 and .95)."""
     slabs = tiles * (hid // 8)
     if dtype == torch.float32 and 0 < slabs <= 256 and cin > (1024 if slabs <= 128 else 512):
