@@ -220,13 +220,14 @@ def test_concat_layers_refuse_the_planning_stream():
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("decoder", ["transposed", "upsample"])
-def test_a_step_planned_under_one_setting_runs_under_another(decoder, dtype, monkeypatch):
+@pytest.mark.parametrize("x3", ["f16x2", "bf16x3"])
+def test_a_step_planned_under_one_setting_runs_under_another(x3, decoder, dtype, monkeypatch):
     # ops.f32_matmul is chosen per call, also between a plan and its step: which tile sets the step needs follows it.  (Deltas are
     # differences of values of order one: sums in another order, all that a plan of the other setting changes, show as some 1e-7)
     h, w = 64, 96
     a, b = (seed_module_(MultiResUNetRecurrentIncr(num_bins=4, decoder=decoder), seed=3).to(DEV).eval() for _ in range(2))
     gen = MovingEdges(h, w, seed=5)
-    x3, native = "bf16x3", "native"
+    native = "native"
     with torch.no_grad():
         x0 = _cl(torch.randn(1, 4, h, w, generator=torch.Generator().manual_seed(1))).to(dtype)
         a.forward_refresh_reservoirs(x0), b.forward_refresh_reservoirs(x0)
